@@ -388,6 +388,23 @@ int32_t krk_group_push(krk_group* g, const krk_optim* o, const uint64_t* ids, co
  * krk_group_push. */
 int32_t krk_group_push_raw(krk_group* g, const krk_optim* o, const uint64_t* ids, const int64_t* offsets,
                            const float* grads, int64_t grad_dim, float lr, uint32_t flags);
+/* Combined requests whose pieces lie where the caller has them (a framework's tensors, one per
+ * table): one krk_part per member in member order instead of concatenated buffers, nothing is
+ * gathered first. KRK_DEVICE_PTRS is required. ids is [n]; rows is the member's output [n, dim] of
+ * a pull, contiguous; of a push its gradient rows, `stride` floats apart (a block of columns of a
+ * wider matrix, or 0 where every position has the same row), only read. Both rules of alignment
+ * (16 bytes where dim is a multiple of 4) hold for every part and for stride. Otherwise as
+ * krk_group_pull and krk_group_push_raw; KRK_NOTE_ROWS / KRK_IDS_AS_PULLED compare the parts' ids
+ * and counts. */
+typedef struct krk_part {
+  const uint64_t* ids;
+  int64_t n;
+  float* rows;
+  int64_t stride;
+} krk_part;
+int32_t krk_group_pull_parts(krk_group* g, const krk_part* parts, uint32_t flags);
+int32_t krk_group_push_raw_parts(krk_group* g, const krk_optim* o, const krk_part* parts, int64_t grad_dim,
+                                 float lr, uint32_t flags);
 /* krk_sparse_set_stream for a group and all its members. */
 int32_t krk_group_set_stream(krk_group* g, void* stream);
 

@@ -1,4 +1,6 @@
-"""Builds kraken_amd/libkraken_hip.so (gfx950) from kraken_amd/csrc with hipcc.
+"""Builds kraken_amd/libkraken_hip.so (gfx950) from kraken_amd/csrc with hipcc, and
+kraken_amd/_torch_native.so (the autograd functions of torch_embedding.py, host code) where torch is
+installed.
 
     python -m kraken_amd.build
 
@@ -6,10 +8,12 @@ The library links only the HIP runtime; it is loaded through its C ABI
 (include/kraken_hip.h). hipcc cross-compiles, so no GPU is needed to build.
 """
 import concurrent.futures
+import importlib.util
 import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -45,11 +49,43 @@ def _compile(src):
     return obj, err
 
 
+TORCH_NATIVE = os.path.join(HERE, "_torch_native.so")
+
+
+def _compile_torch_binding():
+    """-> the object file of the torch module, or None where torch is not installed."""
+    spec = importlib.util.find_spec("torch")
+    if spec is None:
+        return None
+    torch_dir = os.path.dirname(spec.origin)
+    obj = os.path.join(OBJ, "torch_binding.o")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           "-DTORCH_EXTENSION_NAME=_torch_native", "-I" + os.path.join(ROOT, "include")]
+    for d in (os.path.join(torch_dir, "include"), os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
+              os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(hipcc()))), "include"),
+              sysconfig.get_paths()["include"]):
+        cmd += ["-isystem", d]
+    r = subprocess.run(cmd + ["-c", os.path.join(CSRC, "torch_binding.cpp"), "-o", obj], capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed on torch_binding.cpp:\n" + r.stderr)
+    return obj, os.path.join(torch_dir, "lib")
+
+
+def _link_torch_binding(obj, torch_lib):
+    cmd = ["g++", "-shared", "-o", TORCH_NATIVE, obj, "-L" + torch_lib, "-lc10", "-ltorch_cpu", "-ltorch",
+           "-ltorch_python", "-lc10_hip", "-L" + HERE, "-lkraken_hip", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("link of _torch_native.so failed:\n" + r.stderr)
+
+
 def build(verbose=True):
     os.makedirs(OBJ, exist_ok=True)
     srcs = [s for s in SOURCES if os.path.exists(os.path.join(CSRC, s))]
-    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=8) as ex:
+        binding = ex.submit(_compile_torch_binding)
         results = list(ex.map(_compile, srcs))
+        binding = binding.result()
     for obj, err in results:
         if verbose and err.strip():
             print(err, file=sys.stderr)
@@ -57,6 +93,8 @@ def build(verbose=True):
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("link failed:\n" + r.stderr)
+    if binding:
+        _link_torch_binding(*binding)
     if verbose:
         print("built", LIB)
     return LIB

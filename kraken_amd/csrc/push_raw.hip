@@ -339,8 +339,7 @@ __global__ __launch_bounds__(kBlock) void rows_of_ids_kernel(TableView tv, const
 // of the next) holds it; its key is (member << row_bits) | row. A missing id raises the error
 // on its own member.
 __global__ __launch_bounds__(kBlock) void group_rows_of_ids_kernel(const TableDesc* __restrict__ descs,
-                                                                   GroupCall call,
-                                                                   const uint64_t* __restrict__ ids, int64_t n,
+                                                                   GroupCall call, GroupParts parts,
                                                                    int row_bits, uint32_t miss_key,
                                                                    uint32_t* __restrict__ keys,
                                                                    uint32_t* __restrict__ pos) {
@@ -352,12 +351,12 @@ __global__ __launch_bounds__(kBlock) void group_rows_of_ids_kernel(const TableDe
   } else {
     while (m + 1 < call.n_tables && blockIdx.x >= call.block_start[m + 1]) ++m;
   }
-  const int64_t p = call.row_start[m] + (int64_t)(blockIdx.x - call.block_start[m]) * (kBlock / kBucket) +
-                    threadIdx.x / kBucket;
+  const int64_t i = (int64_t)(blockIdx.x - call.block_start[m]) * (kBlock / kBucket) + threadIdx.x / kBucket;
+  const int64_t p = call.row_start[m] + i;
   const int gl = threadIdx.x & (kBucket - 1);
   const bool active = p < call.row_start[m + 1];
   const TableView tv = descs[m].tv;
-  uint32_t r = probe_find(tv, active ? ids[p] : 0, active, gl, kBucket);
+  uint32_t r = probe_find(tv, active ? parts.ids[m][i] : 0, active, gl, kBucket);
   if (!active || gl != 0) return;
   if (r == kEmptyRow) {
     atomicOr(&tv.counters[1], kErrMissingId);
@@ -367,6 +366,17 @@ __global__ __launch_bounds__(kBlock) void group_rows_of_ids_kernel(const TableDe
   }
   keys[p] = r;
   if (pos) pos[p] = (uint32_t)p;
+}
+
+// The gradient rows of a combined request that come in parts, one array after the other.
+__global__ __launch_bounds__(kBlock) void gather_parts_kernel(GroupCall call, GroupParts parts, int dim, int64_t total,
+                                                              float* __restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i >= total) return;
+  const int64_t p = i / dim;
+  int m = 0;
+  while (m + 1 < call.n_tables && p >= call.row_start[m + 1]) ++m;
+  out[i] = parts.rows[m][(p - call.row_start[m]) * (int64_t)parts.stride[m] + (i - p * dim)];
 }
 
 // ---- pooled pushes: from bag offsets to per-position bag numbers ----------------
@@ -893,11 +903,11 @@ struct SortCall {
   int32_t row_bits;                                    // bits of a row number
   uint32_t row_mask;                                   // a key's row (member bits above it)
   uint32_t miss_key;                                   // keys at or above it stand for missing ids
-  // Not null: `keys` are the row notes of the pull of these ids (a member's own row numbers).
+  // `keys` are the row notes of the pull of these ids (a member's own row numbers).
   // A note of kEmptyRow was taken while the row's creator, another wavefront of that pull, had
   // not published the row number yet (further occurrences of an id that the pull inserted):
   // such a position is looked up here.
-  const uint64_t* note_ids;
+  int32_t noted;
   int64_t row_start[kMaxGroupTables + 1];
 };
 
@@ -947,8 +957,8 @@ __device__ __forceinline__ uint32_t sort_block_scan(uint32_t v, uint32_t* wave_t
 // grid: one workgroup per bucket (n_tables << bucket_bits)
 template <int OPT, int VEC, bool GROUPED>
 __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(const TableDesc* __restrict__ descs, TableView tv,
-                                                                 SortCall call, const uint32_t* __restrict__ keys,
-                                                                 const float* __restrict__ grads, int dim,
+                                                                 SortCall call, GroupParts parts,
+                                                                 const uint32_t* __restrict__ keys, int dim,
                                                                  int elems, int group, ApplyArgs args, GroupSrc gs) {
   __shared__ uint32_t skey[kSortMax];                  // row >> bucket_bits
   __shared__ uint16_t spos[kSortMax];
@@ -997,11 +1007,12 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(const TableDesc
       if (i < own) mine[i] = keys[a + (j < all ? j : all - 1)];
     }
   }
-  if (call.note_ids) {
+  if (call.noted) {
+    const uint64_t* ids = parts.ids[m];
 #pragma unroll
     for (int i = 0; i < kSortItems; ++i) {
       const int j = t * own + i;
-      if (i < own && j < all && mine[i] == kEmptyRow) mine[i] = probe_find_alone(tv, call.note_ids[a + j]);
+      if (i < own && j < all && mine[i] == kEmptyRow) mine[i] = probe_find_alone(tv, ids[j]);
     }
   }
   uint32_t take = 0;
@@ -1126,7 +1137,8 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(const TableDesc
   const int lt = t / group;
   const int gl = t & (group - 1);
   const bool lane_on = gl < elems;
-  const float* g_base = grads + a * (int64_t)dim;
+  const float* g_base = parts.rows[m];
+  const uint32_t g_stride = parts.stride[m];
   // Who adds a run up: a lane group (up to kShortRun entries, the reference's order exactly), a
   // wavefront (its lane groups take a stretch each and the stretches' sums are added in order),
   // or the whole workgroup. A lane group walking 64 entries on its own took eight trips to memory
@@ -1153,7 +1165,7 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(const TableDesc
 #pragma unroll
       for (int u = 0; u < kRunAhead; ++u) {
         if (j0 + u < hi && lane_on) {
-          gload<VEC>(g_base + (int64_t)spos[j0 + u] * dim + gl * VEC, v[u]);
+          gload<VEC>(g_base + (int64_t)spos[j0 + u] * g_stride + gl * VEC, v[u]);
         } else {
 #pragma unroll
           for (int c = 0; c < VEC; ++c) v[u][c] = 0.0f;
@@ -1183,7 +1195,7 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(const TableDesc
 #pragma unroll
     for (int u = 0; u < kPairAhead; ++u) {
       if (lo + u < hi && lane_on) {
-        gload<VEC>(g_base + (int64_t)spos[lo + u] * dim + gl * VEC, v[u]);
+        gload<VEC>(g_base + (int64_t)spos[lo + u] * g_stride + gl * VEC, v[u]);
       } else {
 #pragma unroll
         for (int c = 0; c < VEC; ++c) v[u][c] = 0.0f;
@@ -1206,7 +1218,7 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(const TableDesc
 #pragma unroll
       for (int u = 0; u < kRunAhead; ++u) {
         if (j0 + u < hi && lane_on) {
-          gload<VEC>(g_base + (int64_t)spos[j0 + u] * dim + gl * VEC, w[u]);
+          gload<VEC>(g_base + (int64_t)spos[j0 + u] * g_stride + gl * VEC, w[u]);
         } else {
 #pragma unroll
           for (int c = 0; c < VEC; ++c) w[u][c] = 0.0f;
@@ -1319,25 +1331,24 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(const TableDesc
 
 template <int VEC, bool GROUPED>
 static void launch_bucket_push(int opt, unsigned buckets, hipStream_t stream, const TableDesc* descs,
-                               const TableView& tv, const SortCall& call, const uint32_t* keys, const float* grads,
-                               int dim, int elems, int group, const ApplyArgs& args, const GroupSrc& gs) {
+                               const TableView& tv, const SortCall& call, const GroupParts& parts, const uint32_t* keys, int dim, int elems, int group, const ApplyArgs& args, const GroupSrc& gs) {
   const dim3 grid(buckets), block(kSortBlock);
   switch (opt) {
     case KRK_SGD:
-      hipLaunchKernelGGL((bucket_push_kernel<KRK_SGD, VEC, GROUPED>), grid, block, 0, stream, descs, tv, call, keys,
-                         grads, dim, elems, group, args, gs);
+      hipLaunchKernelGGL((bucket_push_kernel<KRK_SGD, VEC, GROUPED>), grid, block, 0, stream, descs, tv, call, parts,
+                         keys, dim, elems, group, args, gs);
       break;
     case KRK_ADAGRAD:
       hipLaunchKernelGGL((bucket_push_kernel<KRK_ADAGRAD, VEC, GROUPED>), grid, block, 0, stream, descs, tv, call,
-                         keys, grads, dim, elems, group, args, gs);
+                         parts, keys, dim, elems, group, args, gs);
       break;
     case KRK_ADAM:
-      hipLaunchKernelGGL((bucket_push_kernel<KRK_ADAM, VEC, GROUPED>), grid, block, 0, stream, descs, tv, call, keys,
-                         grads, dim, elems, group, args, gs);
+      hipLaunchKernelGGL((bucket_push_kernel<KRK_ADAM, VEC, GROUPED>), grid, block, 0, stream, descs, tv, call, parts,
+                         keys, dim, elems, group, args, gs);
       break;
     default:
       hipLaunchKernelGGL((bucket_push_kernel<KRK_RMSPROP, VEC, GROUPED>), grid, block, 0, stream, descs, tv, call,
-                         keys, grads, dim, elems, group, args, gs);
+                         parts, keys, dim, elems, group, args, gs);
       break;
   }
 }
@@ -1916,7 +1927,7 @@ int32_t krk_sparse_push_raw(krk_sparse* t, const krk_optim* o, const uint64_t* i
     while (((int64_t)1 << sc.row_bits) < t->row_cap) ++sc.row_bits;
     sc.row_mask = 0xFFFFFFFFu;
     sc.miss_key = kNoRow;
-    sc.note_ids = nullptr;
+    sc.noted = 0;
     sc.row_start[0] = 0;
     sc.row_start[1] = n;
     ApplyArgs args;
@@ -1940,15 +1951,19 @@ int32_t krk_sparse_push_raw(krk_sparse* t, const krk_optim* o, const uint64_t* i
                          d_ids, n, kNoRow, (const uint32_t*)nullptr, false, found, (uint32_t*)nullptr);
       keys = found;
     } else {
-      sc.note_ids = d_ids;
+      sc.noted = 1;
     }
     const GroupSrc none{nullptr, 0, -1, -1, -1, 0};
+    GroupParts parts;
+    parts.ids[0] = d_ids;
+    parts.rows[0] = const_cast<float*>(d_g);
+    parts.stride[0] = (uint32_t)t->dim;
     if (t->vec == 4) {
-      launch_bucket_push<4, false>(o->type, 1u << sc.bucket_bits, t->stream, nullptr, tv, sc, keys, d_g, (int)t->dim, t->elems,
-                                   t->group, args, none);
+      launch_bucket_push<4, false>(o->type, 1u << sc.bucket_bits, t->stream, nullptr, tv, sc, parts, keys, (int)t->dim,
+                                   t->elems, t->group, args, none);
     } else {
-      launch_bucket_push<1, false>(o->type, 1u << sc.bucket_bits, t->stream, nullptr, tv, sc, keys, d_g, (int)t->dim, t->elems,
-                                   t->group, args, none);
+      launch_bucket_push<1, false>(o->type, 1u << sc.bucket_bits, t->stream, nullptr, tv, sc, parts, keys, (int)t->dim,
+                                   t->elems, t->group, args, none);
     }
     KRK_HIP(hipGetLastError());
     return sparse_finish(t, flags);
@@ -1957,30 +1972,14 @@ int32_t krk_sparse_push_raw(krk_sparse* t, const krk_optim* o, const uint64_t* i
   return sparse_finish(t, flags);
 }
 
-int32_t krk_group_push_raw(krk_group* g, const krk_optim* o, const uint64_t* ids, const int64_t* offsets,
-                           const float* grads, int64_t grad_dim, float lr, uint32_t flags) {
-  if (!g || !offsets) return KRK_E_ARGUMENT;
-  KRK_TRY(ensure_runtime());
-  KRK_TRY(check_flags(flags));
-  if (!o || o->type < KRK_ADAGRAD || o->type > KRK_SGD) {
-    set_error("optimizer type is not supported");
-    return KRK_UNSUPPORTED_OPTIM;
-  }
-  GroupLock lk(g);
-  GroupCall call;
-  int64_t total = 0;
-  KRK_TRY(group_plan(g, offsets, &call, &total));
-  if (total == 0) return group_finish(g, flags);
-  if (!ids || !grads) return KRK_E_ARGUMENT;
-  if (total > ((int64_t)1 << 28)) {
-    set_error("krk_group_push_raw handles at most 2^28 ids per call; split the request");
-    return KRK_E_CAPACITY;
-  }
-  if (grad_dim != g->dim) {
-    set_error("gradient width %lld does not match table dimension %lld", (long long)grad_dim,
-              (long long)g->dim);
-    return KRK_GRADIENT_UNCOMPATIBLE;
-  }
+}  // extern "C"
+
+// A combined push with repeats whose members' ids and gradient rows lie at parts (device
+// addresses); the caller holds the group's lock and has checked the request. contiguous: the
+// gradient rows are one array, member after member, that starts at parts.rows of the first.
+static int32_t group_push_raw_enqueue(krk_group* g, const krk_optim* o, const int64_t* offsets, int64_t total,
+                                      const GroupCall& call, const GroupParts& parts, bool contiguous, float lr,
+                                      uint32_t flags) {
   const uint32_t mask = optim_state_mask(*o);
   for (krk_sparse* t : g->tables) KRK_TRY(sparse_ensure_columns(t, mask));
   KRK_TRY(group_refresh(g));
@@ -2016,10 +2015,6 @@ int32_t krk_group_push_raw(krk_group* g, const krk_optim* o, const uint64_t* ids
   }
   rows_call.block_start[n_tables] = blocks;
   rows_call.even_blocks = even && blocks > 0 ? blocks / (uint32_t)n_tables : 0u;
-  const uint64_t* d_ids;
-  const float* d_g;
-  KRK_TRY(g->input(ids, (size_t)total, flags, 0, &d_ids));
-  KRK_TRY(g->input(grads, (size_t)total * g->dim, flags, 1, &d_g));
   ApplyArgs args;
   args.lr = lr;
   args.k = make_optim_k(*o);
@@ -2035,41 +2030,119 @@ int32_t krk_group_push_raw(krk_group* g, const krk_optim* o, const uint64_t* ids
     sc.row_bits = row_bits;
     sc.row_mask = row_bits >= 32 ? 0xFFFFFFFFu : ((1u << row_bits) - 1u);
     sc.miss_key = miss_key;
-    sc.note_ids = nullptr;
+    sc.noted = 0;
     for (int m = 0; m <= n_tables; ++m) sc.row_start[m] = offsets[m];
     // KRK_IDS_AS_PULLED: the rows of these very ids were noted by the combined pull before (and
     // nothing has moved since): the look-up launch is not needed. A note is a member's own row
     // number, which is all the bucket kernel reads of a key.
-    const uint32_t* keys = noted_rows(g, ids, offsets, flags);
+    const uint32_t* keys = noted_rows(g, parts.ids, offsets, flags);
     const bool noted = keys != nullptr;
     if (!noted) {
       KRK_TRY(g->scratch[0].reserve((size_t)total * sizeof(uint32_t)));
       uint32_t* found = g->scratch[0].as<uint32_t>();
       hipLaunchKernelGGL(group_rows_of_ids_kernel, dim3(rows_call.block_start[n_tables]), dim3(kBlock), 0,
-                         g->stream, g->d_descs, rows_call, d_ids, total, row_bits, miss_key, found,
+                         g->stream, g->d_descs, rows_call, parts, row_bits, miss_key, found,
                          (uint32_t*)nullptr);
       keys = found;
     } else {
-      sc.note_ids = d_ids;
+      sc.noted = 1;
     }
     if (g->vec == 4) {
       launch_bucket_push<4, true>(o->type, (unsigned)n_tables << sc.bucket_bits, g->stream, g->d_descs, TableView{}, sc,
-                                  keys, d_g, (int)g->dim, g->elems, g->group, args, gs);
+                                  parts, keys, (int)g->dim, g->elems, g->group, args, gs);
     } else {
       launch_bucket_push<1, true>(o->type, (unsigned)n_tables << sc.bucket_bits, g->stream, g->d_descs, TableView{}, sc,
-                                  keys, d_g, (int)g->dim, g->elems, g->group, args, gs);
+                                  parts, keys, (int)g->dim, g->elems, g->group, args, gs);
     }
     KRK_HIP(hipGetLastError());
-    return group_finish(g, flags);
+    return KRK_SUCCESS;
+  }
+  const float* d_g = parts.rows[0];
+  if (!contiguous) {
+    KRK_TRY(g->todo.reserve((size_t)total * g->dim * sizeof(float)));
+    float* gathered = g->todo.as<float>();
+    hipLaunchKernelGGL(gather_parts_kernel, dim3(grid_for(total * g->dim, kBlock)), dim3(kBlock), 0, g->stream, call,
+                       parts, (int)g->dim, total * g->dim, gathered);
+    d_g = gathered;
   }
   TableView none{};
   const ReduceShape sh{g->dim, g->vec, g->elems, g->group};
   KRK_TRY(sort_and_reduce(sh, g->stream, g->scratch, none, o->type, total, miss_key, row_bits + member_bits,
                           d_g, args, PooledSrc{nullptr, nullptr}, &gs, [&](uint32_t* keys, uint32_t* pos) {
                             hipLaunchKernelGGL(group_rows_of_ids_kernel, dim3(rows_call.block_start[n_tables]),
-                                               dim3(kBlock), 0, g->stream, g->d_descs, rows_call, d_ids, total,
+                                               dim3(kBlock), 0, g->stream, g->d_descs, rows_call, parts,
                                                row_bits, miss_key, keys, pos);
                           }));
+  return KRK_SUCCESS;
+}
+
+extern "C" {
+
+int32_t krk_group_push_raw(krk_group* g, const krk_optim* o, const uint64_t* ids, const int64_t* offsets,
+                           const float* grads, int64_t grad_dim, float lr, uint32_t flags) {
+  if (!g || !offsets) return KRK_E_ARGUMENT;
+  KRK_TRY(ensure_runtime());
+  KRK_TRY(check_flags(flags));
+  if (!o || o->type < KRK_ADAGRAD || o->type > KRK_SGD) {
+    set_error("optimizer type is not supported");
+    return KRK_UNSUPPORTED_OPTIM;
+  }
+  GroupLock lk(g);
+  GroupCall call;
+  int64_t total = 0;
+  KRK_TRY(group_plan(g, offsets, &call, &total));
+  if (total == 0) return group_finish(g, flags);
+  if (!ids || !grads) return KRK_E_ARGUMENT;
+  if (total > ((int64_t)1 << 28)) {
+    set_error("krk_group_push_raw handles at most 2^28 ids per call; split the request");
+    return KRK_E_CAPACITY;
+  }
+  if (grad_dim != g->dim) {
+    set_error("gradient width %lld does not match table dimension %lld", (long long)grad_dim,
+              (long long)g->dim);
+    return KRK_GRADIENT_UNCOMPATIBLE;
+  }
+  const uint64_t* d_ids;
+  const float* d_g;
+  KRK_TRY(g->input(ids, (size_t)total, flags, 0, &d_ids));
+  KRK_TRY(g->input(grads, (size_t)total * g->dim, flags, 1, &d_g));
+  GroupParts parts;
+  for (int m = 0; m < call.n_tables; ++m) {
+    parts.ids[m] = d_ids + offsets[m];
+    parts.rows[m] = const_cast<float*>(d_g) + offsets[m] * g->dim;
+    parts.stride[m] = (uint32_t)g->dim;
+  }
+  KRK_TRY(group_push_raw_enqueue(g, o, offsets, total, call, parts, true, lr, flags));
+  return group_finish(g, flags);
+}
+
+int32_t krk_group_push_raw_parts(krk_group* g, const krk_optim* o, const krk_part* in, int64_t grad_dim, float lr,
+                                 uint32_t flags) {
+  if (!g || !in || !(flags & KRK_DEVICE_PTRS)) return KRK_E_ARGUMENT;
+  KRK_TRY(ensure_runtime());
+  KRK_TRY(check_flags(flags));
+  if (!o || o->type < KRK_ADAGRAD || o->type > KRK_SGD) {
+    set_error("optimizer type is not supported");
+    return KRK_UNSUPPORTED_OPTIM;
+  }
+  GroupLock lk(g);
+  int64_t offsets[kMaxGroupTables + 1];
+  GroupParts parts;
+  KRK_TRY(group_parts(g, in, true, offsets, &parts));
+  GroupCall call;
+  int64_t total = 0;
+  KRK_TRY(group_plan(g, offsets, &call, &total));
+  if (total == 0) return group_finish(g, flags);
+  if (total > ((int64_t)1 << 28)) {
+    set_error("krk_group_push_raw_parts handles at most 2^28 ids per call; split the request");
+    return KRK_E_CAPACITY;
+  }
+  if (grad_dim != g->dim) {
+    set_error("gradient width %lld does not match table dimension %lld", (long long)grad_dim,
+              (long long)g->dim);
+    return KRK_GRADIENT_UNCOMPATIBLE;
+  }
+  KRK_TRY(group_push_raw_enqueue(g, o, offsets, total, call, parts, false, lr, flags));
   return group_finish(g, flags);
 }
 

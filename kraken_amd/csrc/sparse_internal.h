@@ -459,6 +459,16 @@ struct GroupCall {
   int64_t row_start[kMaxGroupTables + 1];
 };
 
+// Where the members' shares of a combined request lie: one array after the other for the calls
+// that take concatenated buffers, anywhere for the calls that take one part per member.
+// Pulls: rows[m] receives member m's rows, dim floats each. Pushes: rows[m] holds its gradient
+// rows, stride[m] floats apart (a block of columns of a wider matrix is pushed where it lies).
+struct GroupParts {
+  const uint64_t* ids[kMaxGroupTables];
+  float* rows[kMaxGroupTables];
+  uint32_t stride[kMaxGroupTables];
+};
+
 // What a combined pull carries besides when it queues its missing ids (the members' tables are
 // being filled): every member has its own 64 lists, counted by its own table's list counters.
 struct GroupFill {
@@ -478,11 +488,11 @@ struct krk_group : krk::ObjBase {
   int vec = 1, elems = 0, group = 1;
   hipStream_t own_stream = nullptr;    // the stream created with the group
   krk::DeviceBuffer scratch[5];        // push_raw work space
-  // Row notes of one combined pull (see krk_sparse::notes): valid while noted_ids is not null
-  // and every member's layout_version is what it was.
+  // Row notes of one combined pull (see krk_sparse::notes): valid while noted_ids is not
+  // empty and every member's layout_version is what it was.
   krk::DeviceBuffer notes;
   krk::DeviceBuffer todo;              // the lists of a combined pull that queues its missing ids
-  const uint64_t* noted_ids = nullptr;
+  std::vector<const uint64_t*> noted_ids;   // per member; empty: nothing noted
   std::vector<int64_t> noted_offsets;
   std::vector<uint64_t> noted_versions;
 };
@@ -495,12 +505,14 @@ inline const uint32_t* noted_rows(const krk_sparse* t, const uint64_t* ids, int6
                   t->noted_version == t->layout_version;
   return ok ? t->notes.as<uint32_t>() : nullptr;
 }
-inline const uint32_t* noted_rows(const krk_group* g, const uint64_t* ids, const int64_t* offsets, uint32_t flags) {
+inline const uint32_t* noted_rows(const krk_group* g, const uint64_t* const* ids, const int64_t* offsets,
+                                  uint32_t flags) {
   const size_t n = g->tables.size();
-  bool ok = (flags & KRK_IDS_AS_PULLED) && g->noted_ids && g->noted_ids == ids && g->noted_offsets.size() == n + 1 &&
+  bool ok = (flags & KRK_IDS_AS_PULLED) && g->noted_ids.size() == n && g->noted_offsets.size() == n + 1 &&
             g->noted_versions.size() == n;
   for (size_t m = 0; ok && m < n; ++m)
     ok = g->noted_offsets[m] == offsets[m] && g->noted_offsets[m + 1] == offsets[m + 1] &&
+         (offsets[m] == offsets[m + 1] || g->noted_ids[m] == ids[m]) &&
          g->noted_versions[m] == g->tables[m]->layout_version;
   return ok ? g->notes.as<uint32_t>() : nullptr;
 }
@@ -522,6 +534,8 @@ struct GroupLock {
 // Checks the offsets of a combined request and lays its members out over the grid.
 // per_block: positions a workgroup of the launch takes (0: kBlock / the group's lanes per row)
 int32_t group_plan(krk_group* g, const int64_t* offsets, GroupCall* call, int64_t* total, int per_block = 0);
+// Checks a request of one part per member and lists its sizes (offsets[members + 1]) and addresses.
+int32_t group_parts(krk_group* g, const krk_part* in, bool push, int64_t* offsets, GroupParts* parts);
 // Uploads the layouts of members that moved since the last call.
 int32_t group_refresh(krk_group* g);
 // Blocking calls: waits for the group's stream and reports the first member's error.

@@ -856,38 +856,36 @@ __device__ __forceinline__ int find_table(const GroupCall& c) { return find_tabl
 
 template <int VEC>
 __global__ __launch_bounds__(kBlock) void group_pull_kernel(const TableDesc* __restrict__ descs,
-                                                            GroupCall call,
-                                                            const uint64_t* __restrict__ ids,
-                                                            float* __restrict__ out, int dim, int elems,
-                                                            int group, uint32_t* __restrict__ notes) {
+                                                            GroupCall call, GroupParts parts, int dim,
+                                                            int elems, int group,
+                                                            uint32_t* __restrict__ notes) {
   const int t = find_table(call);
   TableView tv = descs[t].tv;
   tv.epoch = call.epoch[t];
   const InitK init = descs[t].init;
   const int per_block = kBlock / group;
-  const int64_t local = (int64_t)(blockIdx.x - call.block_start[t]) * per_block + threadIdx.x / group;
-  const int64_t i = call.row_start[t] + local;
-  pull_body<VEC>(tv, init, ids, i, i < call.row_start[t + 1], threadIdx.x & (group - 1), out, dim,
-                 elems, group, notes, kFillingIdsCombined);
+  const int64_t i = (int64_t)(blockIdx.x - call.block_start[t]) * per_block + threadIdx.x / group;
+  const int64_t a = call.row_start[t];
+  pull_body<VEC>(tv, init, parts.ids[t], i, i < call.row_start[t + 1] - a, threadIdx.x & (group - 1), parts.rows[t],
+                 dim, elems, group, notes ? notes + a : nullptr, kFillingIdsCombined);
 }
 
 // the same for rows 32 to 128 floats wide: a workgroup takes 64 positions of its table
 template <int VEC, int STEPS>
 __global__ __launch_bounds__(kBlock) void group_pull_wide_kernel(const TableDesc* __restrict__ descs,
-                                                                 GroupCall call,
-                                                                 const uint64_t* __restrict__ ids,
-                                                                 float* __restrict__ out, int dim,
+                                                                 GroupCall call, GroupParts parts, int dim,
                                                                  int elems, uint32_t* __restrict__ notes) {
   const int t = find_table(call);
   TableView tv = descs[t].tv;
   tv.epoch = call.epoch[t];
   const InitK init = descs[t].init;
-  const int64_t local = ((int64_t)(blockIdx.x - call.block_start[t]) * (blockDim.x / kWave) + threadIdx.x / kWave) *
+  const int64_t first = ((int64_t)(blockIdx.x - call.block_start[t]) * (blockDim.x / kWave) + threadIdx.x / kWave) *
                         kWideIds;
-  const int64_t first = call.row_start[t] + local;
-  if (first >= call.row_start[t + 1]) return;    // the whole wavefront
-  pull_wide<VEC, true, STEPS>(tv, init, ids, first, call.row_start[t + 1], out, dim, elems, nullptr, 0, notes,
-                              kFillingIdsCombined);
+  const int64_t a = call.row_start[t];
+  const int64_t n = call.row_start[t + 1] - a;
+  if (first >= n) return;                        // the whole wavefront
+  pull_wide<VEC, true, STEPS>(tv, init, parts.ids[t], first, n, parts.rows[t], dim, elems, nullptr, 0,
+                              notes ? notes + a : nullptr, kFillingIdsCombined);
 }
 
 // ---- combined pulls while the members' tables are being filled ---------------------------------
@@ -901,25 +899,22 @@ static_assert(kQueues % kGroupMissPerTable == 0, "every workgroup walks the same
 
 template <int VEC>
 __global__ __launch_bounds__(kBlock) void group_pull_resident_kernel(const TableDesc* __restrict__ descs,
-                                                                     GroupCall call, GroupFill fill,
-                                                                     const uint64_t* __restrict__ ids,
-                                                                     float* __restrict__ out,
+                                                                     GroupCall call, GroupParts parts, GroupFill fill,
                                                                      uint32_t* __restrict__ todo, int dim,
                                                                      int elems, int group,
                                                                      uint32_t* __restrict__ notes) {
   const uint32_t bx = blockIdx.x;
   const int t = find_table(call, bx);
   const int64_t a = call.row_start[t];
-  pull_resident_body<VEC>(descs[t].tv, ids + a, call.row_start[t + 1] - a, out + a * dim,
+  pull_resident_body<VEC>(descs[t].tv, parts.ids[t], call.row_start[t + 1] - a, parts.rows[t],
                           todo + fill.todo_start[t], (int)((fill.parity_bits >> t) & 1u), dim, elems, group,
                           bx - call.block_start[t], notes ? notes + a : nullptr);
 }
 
 template <int VEC, int STEPS>
 __global__ __launch_bounds__(kBlock) void group_pull_resident_wide_kernel(const TableDesc* __restrict__ descs,
-                                                                          GroupCall call, GroupFill fill,
-                                                                          const uint64_t* __restrict__ ids,
-                                                                          float* __restrict__ out,
+                                                                          GroupCall call, GroupParts parts,
+                                                                          GroupFill fill,
                                                                           uint32_t* __restrict__ todo, int dim,
                                                                           int elems, uint32_t* __restrict__ notes) {
   const uint32_t bx = blockIdx.x;
@@ -929,16 +924,15 @@ __global__ __launch_bounds__(kBlock) void group_pull_resident_wide_kernel(const 
   const int64_t first = ((int64_t)(bx - call.block_start[t]) * (blockDim.x / kWave) + threadIdx.x / kWave) * kWideIds;
   if (first >= n) return;                        // the whole wavefront
   InitK none{};
-  pull_wide<VEC, false, STEPS>(descs[t].tv, none, ids + a, first, n, out + a * dim, dim, elems,
+  pull_wide<VEC, false, STEPS>(descs[t].tv, none, parts.ids[t], first, n, parts.rows[t], dim, elems,
                                todo + fill.todo_start[t], (int)((fill.parity_bits >> t) & 1u),
                                notes ? notes + a : nullptr);
 }
 
 template <int VEC>
 __global__ __launch_bounds__(kMissBlock) void group_pull_missing_kernel(const TableDesc* __restrict__ descs,
-                                                                        GroupCall call, GroupFill fill,
-                                                                        const uint64_t* __restrict__ ids,
-                                                                        float* __restrict__ out,
+                                                                        GroupCall call, GroupParts parts,
+                                                                        GroupFill fill,
                                                                         const uint32_t* __restrict__ todo,
                                                                         int per_block, int dim, int elems,
                                                                         int group, uint32_t* __restrict__ notes) {
@@ -974,7 +968,7 @@ __global__ __launch_bounds__(kMissBlock) void group_pull_missing_kernel(const Ta
     for (int i = 0; i + 1 < kMine; ++i) j += k >= upto[i] ? 1 : 0;
     return lists[(int64_t)(w + j * kGroupMissPerTable) * capacity + (k - (j ? upto[j - 1] : 0u))];
   };
-  insert_queued<VEC, kInsertAndCopy>(tv, init, ids + a, out + a * dim, position_of, total, 0u, kMissEntries, dim,
+  insert_queued<VEC, kInsertAndCopy>(tv, init, parts.ids[t], parts.rows[t], position_of, total, 0u, kMissEntries, dim,
                                      elems, group, notes ? notes + a : nullptr);
 }
 
@@ -2794,6 +2788,7 @@ int32_t krk_group_destroy(krk_group* g) {
   if (g->h_descs) (void)hipHostFree(g->h_descs);
   for (auto& b : g->scratch) b.release();
   g->notes.release();
+  g->todo.release();
   g->stream = g->own_stream;
   g->close_stream();
   delete g;
@@ -2909,19 +2904,13 @@ int32_t krk_group_sync(krk_group* g) {
 // (a step at dim 64: 42.7 us with 256 lanes, 41.7 us with 128; rows of 16 and 32 floats lose with 128).
 static int group_wide_block(int group) { return group == 16 ? 128 : kBlock; }
 
-int32_t krk_group_pull(krk_group* g, const uint64_t* ids, const int64_t* offsets, float* out,
-                       uint32_t flags) {
-  if (!g || !offsets) return KRK_E_ARGUMENT;
-  KRK_TRY(ensure_runtime());
-  KRK_TRY(check_flags(flags));
-  GroupLock lk(g);
-  GroupCall call;
-  int64_t total = 0;
-  const bool wide = g->vec == 4 && pull_is_wide(g->group, g->elems);
-  KRK_TRY(group_plan(g, offsets, &call, &total, wide ? (group_wide_block(g->group) / kWave) * kWideIds : 0));
-  if (total == 0) return group_finish(g, flags);
-  if (!ids || !out) return KRK_E_ARGUMENT;
-  if ((flags & KRK_DEVICE_PTRS) && g->vec == 4 && !aligned16(out)) return KRK_E_ARGUMENT;
+}  // extern "C"
+
+// The launches of a combined pull whose members' ids and rows lie at parts (device addresses) and
+// whose sizes are offsets' differences; the caller holds the group's lock. ids: what the caller
+// passed for each member, for KRK_NOTE_ROWS.
+static int32_t group_pull_enqueue(krk_group* g, const int64_t* offsets, GroupCall& call, int64_t total, bool wide,
+                                  const GroupParts& parts, uint32_t flags) {
   for (size_t i = 0; i < g->tables.size(); ++i) {
     krk_sparse* t = g->tables[i];
     const int64_t cnt = offsets[i + 1] - offsets[i];
@@ -2934,15 +2923,11 @@ int32_t krk_group_pull(krk_group* g, const uint64_t* ids, const int64_t* offsets
     call.epoch[i] = t->epoch;
   }
   KRK_TRY(group_refresh(g));
-  const uint64_t* d_ids;
-  float* d_out;
-  KRK_TRY(g->input(ids, (size_t)total, flags, 0, &d_ids));
-  KRK_TRY(g->output(out, (size_t)total * g->dim, flags, 1, &d_out));
   const dim3 grid(call.block_start[call.n_tables]), block(wide ? group_wide_block(g->group) : kBlock);
   // KRK_NOTE_ROWS: the row of every position stays behind
   uint32_t* notes = nullptr;
   if (flags & KRK_NOTE_ROWS) {
-    g->noted_ids = nullptr;
+    g->noted_ids.clear();
     if (flags & KRK_DEVICE_PTRS) {
       KRK_TRY(g->notes.reserve((size_t)total * sizeof(uint32_t)));
       notes = g->notes.as<uint32_t>();
@@ -2970,47 +2955,47 @@ int32_t krk_group_pull(krk_group* g, const uint64_t* ids, const int64_t* offsets
     uint32_t* todo = g->todo.as<uint32_t>();
     const dim3 missing_grid((unsigned)call.n_tables * kGroupMissPerTable), missing_block(kMissBlock);
     if (wide && g->group == 8) {
-      hipLaunchKernelGGL((group_pull_resident_wide_kernel<4, 2>), grid, block, 0, g->stream, g->d_descs, call, fill,
-                         d_ids, d_out, todo, (int)g->dim, g->elems, notes);
+      hipLaunchKernelGGL((group_pull_resident_wide_kernel<4, 2>), grid, block, 0, g->stream, g->d_descs, call, parts,
+                         fill, todo, (int)g->dim, g->elems, notes);
     } else if (wide && g->group == 16) {
-      hipLaunchKernelGGL((group_pull_resident_wide_kernel<4, 4>), grid, block, 0, g->stream, g->d_descs, call, fill,
-                         d_ids, d_out, todo, (int)g->dim, g->elems, notes);
+      hipLaunchKernelGGL((group_pull_resident_wide_kernel<4, 4>), grid, block, 0, g->stream, g->d_descs, call, parts,
+                         fill, todo, (int)g->dim, g->elems, notes);
     } else if (wide) {
-      hipLaunchKernelGGL((group_pull_resident_wide_kernel<4, 8>), grid, block, 0, g->stream, g->d_descs, call, fill,
-                         d_ids, d_out, todo, (int)g->dim, g->elems, notes);
+      hipLaunchKernelGGL((group_pull_resident_wide_kernel<4, 8>), grid, block, 0, g->stream, g->d_descs, call, parts,
+                         fill, todo, (int)g->dim, g->elems, notes);
     } else if (g->vec == 4) {
-      hipLaunchKernelGGL((group_pull_resident_kernel<4>), grid, block, 0, g->stream, g->d_descs, call, fill, d_ids,
-                         d_out, todo, (int)g->dim, g->elems, g->group, notes);
+      hipLaunchKernelGGL((group_pull_resident_kernel<4>), grid, block, 0, g->stream, g->d_descs, call, parts, fill,
+                         todo, (int)g->dim, g->elems, g->group, notes);
     } else {
-      hipLaunchKernelGGL((group_pull_resident_kernel<1>), grid, block, 0, g->stream, g->d_descs, call, fill, d_ids,
-                         d_out, todo, (int)g->dim, g->elems, g->group, notes);
+      hipLaunchKernelGGL((group_pull_resident_kernel<1>), grid, block, 0, g->stream, g->d_descs, call, parts, fill,
+                         todo, (int)g->dim, g->elems, g->group, notes);
     }
     if (g->vec == 4) {
       hipLaunchKernelGGL((group_pull_missing_kernel<4>), missing_grid, missing_block, 0, g->stream, g->d_descs, call,
-                         fill, d_ids, d_out, todo, per_block, (int)g->dim, g->elems, g->group, notes);
+                         parts, fill, todo, per_block, (int)g->dim, g->elems, g->group, notes);
     } else {
       hipLaunchKernelGGL((group_pull_missing_kernel<1>), missing_grid, missing_block, 0, g->stream, g->d_descs, call,
-                         fill, d_ids, d_out, todo, per_block, (int)g->dim, g->elems, g->group, notes);
+                         parts, fill, todo, per_block, (int)g->dim, g->elems, g->group, notes);
     }
   } else if (wide && g->group == 8) {
-    hipLaunchKernelGGL((group_pull_wide_kernel<4, 2>), grid, block, 0, g->stream, g->d_descs, call, d_ids, d_out,
+    hipLaunchKernelGGL((group_pull_wide_kernel<4, 2>), grid, block, 0, g->stream, g->d_descs, call, parts,
                        (int)g->dim, g->elems, notes);
   } else if (wide && g->group == 16) {
-    hipLaunchKernelGGL((group_pull_wide_kernel<4, 4>), grid, block, 0, g->stream, g->d_descs, call, d_ids, d_out,
+    hipLaunchKernelGGL((group_pull_wide_kernel<4, 4>), grid, block, 0, g->stream, g->d_descs, call, parts,
                        (int)g->dim, g->elems, notes);
   } else if (wide) {
-    hipLaunchKernelGGL((group_pull_wide_kernel<4, 8>), grid, block, 0, g->stream, g->d_descs, call, d_ids, d_out,
+    hipLaunchKernelGGL((group_pull_wide_kernel<4, 8>), grid, block, 0, g->stream, g->d_descs, call, parts,
                        (int)g->dim, g->elems, notes);
   } else if (g->vec == 4) {
-    hipLaunchKernelGGL((group_pull_kernel<4>), grid, block, 0, g->stream, g->d_descs, call, d_ids, d_out,
+    hipLaunchKernelGGL((group_pull_kernel<4>), grid, block, 0, g->stream, g->d_descs, call, parts,
                        (int)g->dim, g->elems, g->group, notes);
   } else {
-    hipLaunchKernelGGL((group_pull_kernel<1>), grid, block, 0, g->stream, g->d_descs, call, d_ids, d_out,
+    hipLaunchKernelGGL((group_pull_kernel<1>), grid, block, 0, g->stream, g->d_descs, call, parts,
                        (int)g->dim, g->elems, g->group, notes);
   }
   KRK_HIP(hipGetLastError());
   if (notes) {
-    g->noted_ids = ids;
+    g->noted_ids.assign(parts.ids, parts.ids + call.n_tables);
     g->noted_offsets.assign(offsets, offsets + call.n_tables + 1);
     g->noted_versions.clear();
     for (krk_sparse* t : g->tables) g->noted_versions.push_back(t->layout_version);
@@ -3020,7 +3005,82 @@ int32_t krk_group_pull(krk_group* g, const uint64_t* ids, const int64_t* offsets
     for (krk_sparse* t : g->tables) any = any || sparse_near_full(t);
     if (any) KRK_TRY(sparse_publish(g->tables.data(), (int)g->tables.size(), g->stream));
   }
+  return KRK_SUCCESS;
+}
+
+extern "C" {
+
+int32_t krk_group_pull(krk_group* g, const uint64_t* ids, const int64_t* offsets, float* out,
+                       uint32_t flags) {
+  if (!g || !offsets) return KRK_E_ARGUMENT;
+  KRK_TRY(ensure_runtime());
+  KRK_TRY(check_flags(flags));
+  GroupLock lk(g);
+  GroupCall call;
+  int64_t total = 0;
+  const bool wide = g->vec == 4 && pull_is_wide(g->group, g->elems);
+  KRK_TRY(group_plan(g, offsets, &call, &total, wide ? (group_wide_block(g->group) / kWave) * kWideIds : 0));
+  if (total == 0) return group_finish(g, flags);
+  if (!ids || !out) return KRK_E_ARGUMENT;
+  if ((flags & KRK_DEVICE_PTRS) && g->vec == 4 && !aligned16(out)) return KRK_E_ARGUMENT;
+  const uint64_t* d_ids;
+  float* d_out;
+  KRK_TRY(g->input(ids, (size_t)total, flags, 0, &d_ids));
+  KRK_TRY(g->output(out, (size_t)total * g->dim, flags, 1, &d_out));
+  GroupParts parts;
+  for (int m = 0; m < call.n_tables; ++m) {
+    parts.ids[m] = d_ids + offsets[m];
+    parts.rows[m] = d_out + offsets[m] * g->dim;
+    parts.stride[m] = (uint32_t)g->dim;
+  }
+  KRK_TRY(group_pull_enqueue(g, offsets, call, total, wide, parts, flags));
   KRK_TRY(g->output_back(out, (size_t)total * g->dim, flags, 1));
+  return group_finish(g, flags);
+}
+
+}  // extern "C"
+
+int32_t krk::group_parts(krk_group* g, const krk_part* in, bool push, int64_t* offsets, GroupParts* parts) {
+  offsets[0] = 0;
+  for (size_t m = 0; m < g->tables.size(); ++m) {
+    const krk_part& p = in[m];
+    if (p.n < 0 || (p.n > 0 && (!p.ids || !p.rows))) return KRK_E_ARGUMENT;
+    offsets[m + 1] = offsets[m] + p.n;
+    parts->ids[m] = p.ids;
+    parts->rows[m] = p.rows;
+    parts->stride[m] = (uint32_t)g->dim;
+    if (p.n == 0) continue;
+    if (push) {
+      if (p.stride < 0 || p.stride > (int64_t)1 << 30 || (g->vec == 4 && p.stride % 4 != 0)) {
+        set_error("a part's gradient rows must lie a whole number of 16-byte vectors apart");
+        return KRK_E_ARGUMENT;
+      }
+      parts->stride[m] = (uint32_t)p.stride;
+    }
+    if (g->vec == 4 && !aligned16(p.rows)) {
+      set_error("a part's rows must be 16-byte aligned");
+      return KRK_E_ARGUMENT;
+    }
+  }
+  return KRK_SUCCESS;
+}
+
+extern "C" {
+
+int32_t krk_group_pull_parts(krk_group* g, const krk_part* in, uint32_t flags) {
+  if (!g || !in || !(flags & KRK_DEVICE_PTRS)) return KRK_E_ARGUMENT;
+  KRK_TRY(ensure_runtime());
+  KRK_TRY(check_flags(flags));
+  GroupLock lk(g);
+  int64_t offsets[kMaxGroupTables + 1];
+  GroupParts parts;
+  KRK_TRY(group_parts(g, in, false, offsets, &parts));
+  GroupCall call;
+  int64_t total = 0;
+  const bool wide = g->vec == 4 && pull_is_wide(g->group, g->elems);
+  KRK_TRY(group_plan(g, offsets, &call, &total, wide ? (group_wide_block(g->group) / kWave) * kWideIds : 0));
+  if (total == 0) return group_finish(g, flags);
+  KRK_TRY(group_pull_enqueue(g, offsets, call, total, wide, parts, flags));
   return group_finish(g, flags);
 }
 
@@ -3099,7 +3159,9 @@ int32_t krk_group_push(krk_group* g, const krk_optim* o, const uint64_t* ids, co
   KRK_TRY(g->input(ids, (size_t)total, flags, 0, &d_ids));
   KRK_TRY(g->input(grads, (size_t)total * g->dim, flags, 1, &d_g));
   for (int i = 0; i < call.n_tables; ++i) call.epoch[i] = 0;
-  const uint32_t* notes = noted_rows(g, ids, offsets, flags);   // KRK_IDS_AS_PULLED: no second look-up
+  const uint64_t* member_ids[kMaxGroupTables];
+  for (int i = 0; i < call.n_tables; ++i) member_ids[i] = ids + offsets[i];
+  const uint32_t* notes = noted_rows(g, member_ids, offsets, flags);   // KRK_IDS_AS_PULLED: no second look-up
   if (g->vec == 4) {
     launch_group_push<4>(g, *o, call, d_ids, d_g, lr, wide, notes);
   } else {

@@ -1,0 +1,400 @@
+// The autograd functions behind kraken_amd/torch_embedding.py, over the C ABI.
+//
+// A step of an embedding layer is two or three kernel launches of a few microseconds each, so what
+// the host does around them is what a small or ordinary batch waits for. As
+// torch.autograd.Function classes in Python (pytorch/embedding.py:9-23,
+// pytorch/combine_embedding.py:10-31 in the reference) a forward and a backward of one layer cost
+// 60 to 120 us, most of it interpreter work and the hand-over of the interpreter lock to the
+// engine's thread and back; 26 tables cost 400 us. Here a forward is one call that builds the
+// request from the tensors' addresses, and the backward node runs in the engine's thread without
+// taking the lock.
+//
+// Tensors are used where they lie: the ids of a combined request are not concatenated, and a
+// gradient that is a block of columns of a wider matrix (what torch.cat along the feature dimension
+// hands back) is read in place.
+#include <ATen/ATen.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include <memory>
+#include <vector>
+
+#include "kraken_hip.h"
+
+namespace {
+
+namespace py = pybind11;
+using at::Tensor;
+using torch::autograd::edge_list;
+using torch::autograd::Node;
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+
+constexpr uint32_t kFlags = KRK_DEVICE_PTRS | KRK_ASYNC;
+
+// api.KrakenHipError, as the ctypes calls raise it; usable with and without the interpreter lock.
+[[noreturn]] void fail(int32_t rc, const char* what) {
+  py::gil_scoped_acquire gil;
+  py::object type = py::module_::import("kraken_amd.api").attr("KrakenHipError");
+  py::object err = type(rc, what);
+  PyErr_SetObject(type.ptr(), err.ptr());
+  python_error e;
+  e.persist();
+  throw e;
+}
+#define KRK_CALL(fn, ...)                       \
+  do {                                          \
+    const int32_t rc_ = fn(__VA_ARGS__);        \
+    if (rc_ != KRK_SUCCESS) fail(rc_, #fn);     \
+  } while (0)
+
+void* current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
+
+// int64 ids are the uint64 ids bit for bit (worker/emitter.cc:126 casts the same way)
+Tensor ids_of(const Tensor& t, const char* name = "indices") {
+  if (t.scalar_type() != at::kLong || !t.is_cuda()) {
+    throw py::type_error(std::string(name) + " must be an int64 CUDA tensor");
+  }
+  return t.contiguous();
+}
+const uint64_t* id_ptr(const Tensor& t) { return reinterpret_cast<const uint64_t*>(t.const_data_ptr<int64_t>()); }
+const int64_t* off_ptr(const Tensor& t) { return t.const_data_ptr<int64_t>(); }
+const float* float_ptr(const Tensor& t) { return t.defined() ? t.const_data_ptr<float>() : nullptr; }
+
+Tensor weights_of(const c10::optional<Tensor>& w) {
+  return w.has_value() && w->defined() ? w->detach().contiguous().to(at::kFloat) : Tensor();
+}
+
+Tensor new_rows(at::IntArrayRef sizes, const Tensor& like) {
+  return at::empty(sizes, at::TensorOptions().dtype(at::kFloat).device(like.device()));
+}
+
+// The gradient rows of `g` where they lie, `stride` floats apart, if the kernels can read them there;
+// otherwise of a contiguous float copy, which `keep` then holds.
+struct Rows {
+  Tensor keep;
+  int64_t stride = 0;
+  float* ptr() const { return const_cast<float*>(keep.const_data_ptr<float>()); }
+};
+Rows rows_of(const Tensor& g, int64_t dim) {
+  Rows r;
+  r.stride = dim;
+  if (g.scalar_type() == at::kFloat && g.dim() >= 1 && g.size(-1) == dim && (dim == 1 || g.stride(-1) == 1)) {
+    int64_t stride = -1, span = 0;
+    bool ok = true;
+    for (int64_t i = g.dim() - 2; i >= 0 && ok; --i) {
+      if (g.size(i) == 1) continue;
+      if (stride < 0) {
+        stride = g.stride(i);
+        span = stride * g.size(i);
+      } else {
+        ok = g.stride(i) == span;
+        span *= g.size(i);
+      }
+    }
+    if (stride < 0) stride = dim;
+    const bool vec = dim % 4 == 0;
+    ok = ok && stride < ((int64_t)1 << 30) &&
+         (!vec || (stride % 4 == 0 && (reinterpret_cast<uintptr_t>(g.const_data_ptr<float>()) & 15) == 0));
+    if (ok) {
+      r.keep = g;
+      r.stride = stride;
+      return r;
+    }
+  }
+  r.keep = g.contiguous().to(at::kFloat);
+  return r;
+}
+
+bool recording(const Tensor& param) { return at::GradMode::is_enabled() && param.requires_grad(); }
+
+// The node of a pass over `param` (the empty Parameter that stands for the tables, whose edge is
+// what makes the engine run the node).
+template <typename N>
+std::shared_ptr<N> new_node(const Tensor& param) {
+  auto node = std::shared_ptr<N>(new N(), torch::autograd::deleteNode);
+  node->set_next_edges(torch::autograd::collect_next_edges(param));
+  return node;
+}
+
+// ---- one table --------------------------------------------------------------------------------
+struct Table {
+  krk_sparse* h;
+  const krk_optim* optim;
+  int64_t dim;
+  double lr;
+};
+using TablePtr = std::shared_ptr<Table>;
+
+struct EmbeddingBackward : Node {
+  TablePtr table;
+  SavedVariable ids;
+  variable_list apply(variable_list&& grads) override {
+    const Tensor saved = ids.unpack();
+    const Tensor g = grads[0].contiguous().to(at::kFloat);
+    KRK_CALL(krk_sparse_set_stream, table->h, current_stream());
+    KRK_CALL(krk_sparse_push_raw, table->h, table->optim, id_ptr(saved), saved.numel(), float_ptr(g), table->dim,
+             (float)table->lr, kFlags | KRK_IDS_AS_PULLED);
+    return variable_list(1);
+  }
+  void release_variables() override { ids.reset_data(); }
+  std::string name() const override { return "EmbeddingFunctionBackward"; }
+};
+
+Tensor embedding(const TablePtr& table, const Tensor& param, const Tensor& indices) {
+  const Tensor ids = ids_of(indices);
+  std::vector<int64_t> sizes = indices.sizes().vec();
+  sizes.push_back(table->dim);
+  Tensor out = new_rows(sizes, ids);
+  const bool record = recording(param);
+  KRK_CALL(krk_sparse_set_stream, table->h, current_stream());
+  // the table notes where it found every id: backward pushes gradients for this very tensor
+  // (autograd keeps it alive and unchanged), so its look-up need not be repeated
+  KRK_CALL(krk_sparse_pull, table->h, id_ptr(ids), ids.numel(), out.mutable_data_ptr<float>(),
+           kFlags | (record ? KRK_NOTE_ROWS : 0u));
+  if (record) {
+    auto node = new_node<EmbeddingBackward>(param);
+    node->table = table;
+    node->ids = SavedVariable(ids, false);
+    torch::autograd::set_history(out, node);
+  }
+  return out;
+}
+
+struct JaggedBackward : Node {
+  TablePtr table;
+  int mode = 0;
+  SavedVariable ids, offsets;
+  Tensor weights;
+  variable_list apply(variable_list&& grads) override {
+    const Tensor saved = ids.unpack(), off = offsets.unpack();
+    const Tensor g = grads[0].contiguous().to(at::kFloat);
+    KRK_CALL(krk_sparse_set_stream, table->h, current_stream());
+    KRK_CALL(krk_sparse_push_pooled, table->h, table->optim, id_ptr(saved), saved.numel(), off_ptr(off),
+             off.numel() - 1, float_ptr(weights), mode, float_ptr(g), table->dim, (float)table->lr, kFlags);
+    return variable_list(1);
+  }
+  void release_variables() override {
+    ids.reset_data();
+    offsets.reset_data();
+    weights.reset();
+  }
+  std::string name() const override { return "JaggedEmbeddingFunctionBackward"; }
+};
+
+Tensor jagged(const TablePtr& table, const Tensor& param, const Tensor& indices, const Tensor& offsets_in,
+              const c10::optional<Tensor>& weights_in, int mode, double patch) {
+  const Tensor ids = ids_of(indices);
+  const Tensor off = ids_of(offsets_in, "offsets");
+  const Tensor w = weights_of(weights_in);
+  const int64_t bags = off.numel() - 1;
+  Tensor out = new_rows({bags, table->dim}, ids);
+  KRK_CALL(krk_sparse_set_stream, table->h, current_stream());
+  KRK_CALL(krk_sparse_pull_pooled, table->h, id_ptr(ids), ids.numel(), off_ptr(off), bags, float_ptr(w), mode,
+           (float)patch, out.mutable_data_ptr<float>(), kFlags);
+  if (recording(param)) {
+    auto node = new_node<JaggedBackward>(param);
+    node->table = table;
+    node->mode = mode;
+    node->ids = SavedVariable(ids, false);
+    node->offsets = SavedVariable(off, false);
+    node->weights = w;
+    torch::autograd::set_history(out, node);
+  }
+  return out;
+}
+
+// ---- the tables of a combined request -----------------------------------------------------------
+// Tables of equal dimension form one group of the engine; mixed dimensions give several groups.
+struct Combine {
+  struct Group {
+    krk_group* h;
+    int64_t dim;
+    std::vector<int> members;      // positions of its tables in the request
+  };
+  std::vector<Group> groups;
+  std::vector<krk_sparse*> tables;
+  std::vector<int64_t> dims;
+  const krk_optim* optim;
+  double lr;
+};
+using CombinePtr = std::shared_ptr<Combine>;
+
+// Piece `sizes` of a storage that several outputs share, `at` floats from its start: a tensor of its
+// own (the pieces do not overlap, so none is a view of another).
+Tensor piece_of(const Tensor& whole, int64_t at, at::IntArrayRef sizes) {
+  Tensor t = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(whole.storage()), whole.key_set(), whole.dtype());
+  t.unsafeGetTensorImpl()->set_storage_offset(at);
+  t.unsafeGetTensorImpl()->set_sizes_contiguous(sizes);
+  return t;
+}
+
+struct CombineBackward : Node {
+  CombinePtr c;
+  std::vector<SavedVariable> ids;
+  variable_list apply(variable_list&& grads) override {
+    void* stream = current_stream();
+    Tensor zeros;                  // one row for the outputs the loss never used: every position reads it
+    for (const Combine::Group& g : c->groups) {
+      std::vector<krk_part> parts(g.members.size());
+      std::vector<Tensor> keep;
+      keep.reserve(2 * g.members.size());
+      for (size_t m = 0; m < g.members.size(); ++m) {
+        const int i = g.members[m];
+        Tensor saved = ids[i].unpack();
+        krk_part& p = parts[m];
+        p.ids = id_ptr(saved);
+        p.n = saved.numel();
+        if (grads[i].defined()) {
+          Rows r = rows_of(grads[i], g.dim);
+          p.rows = r.ptr();
+          p.stride = r.stride;
+          keep.push_back(std::move(r.keep));
+        } else {
+          if (!zeros.defined() || zeros.numel() < g.dim)
+            zeros = at::zeros({g.dim}, at::TensorOptions().dtype(at::kFloat).device(saved.device()));
+          p.rows = zeros.mutable_data_ptr<float>();
+          p.stride = 0;
+        }
+        keep.push_back(std::move(saved));
+      }
+      KRK_CALL(krk_group_set_stream, g.h, stream);
+      KRK_CALL(krk_group_push_raw_parts, g.h, c->optim, parts.data(), g.dim, (float)c->lr, kFlags | KRK_IDS_AS_PULLED);
+    }
+    return variable_list(1);
+  }
+  void release_variables() override {
+    for (auto& v : ids) v.reset_data();
+  }
+  std::string name() const override { return "CombineEmbeddingFunctionBackward"; }
+};
+
+std::vector<Tensor> combine(const CombinePtr& c, const Tensor& param, const std::vector<Tensor>& indices) {
+  if (indices.size() != c->dims.size()) throw py::value_error("one index tensor per table");
+  const bool record = recording(param);
+  void* stream = current_stream();
+  std::vector<Tensor> outs(indices.size()), ids(indices.size());
+  std::vector<int64_t> sizes;
+  for (const Combine::Group& g : c->groups) {
+    std::vector<krk_part> parts(g.members.size());
+    int64_t total = 0;
+    for (int i : g.members) {
+      ids[i] = ids_of(indices[i]);
+      total += ids[i].numel();
+    }
+    const Tensor whole = new_rows({total, g.dim}, ids[g.members[0]]);
+    float* base = whole.mutable_data_ptr<float>();
+    int64_t at = 0;
+    for (size_t m = 0; m < g.members.size(); ++m) {
+      const int i = g.members[m];
+      sizes.assign(indices[i].sizes().begin(), indices[i].sizes().end());
+      sizes.push_back(g.dim);
+      outs[i] = piece_of(whole, at, sizes);
+      parts[m] = krk_part{id_ptr(ids[i]), ids[i].numel(), base + at, g.dim};
+      at += ids[i].numel() * g.dim;
+    }
+    KRK_CALL(krk_group_set_stream, g.h, stream);
+    KRK_CALL(krk_group_pull_parts, g.h, parts.data(), kFlags | (record ? KRK_NOTE_ROWS : 0u));
+  }
+  if (record) {
+    auto node = new_node<CombineBackward>(param);
+    node->c = c;
+    node->ids.reserve(ids.size());
+    for (const Tensor& t : ids) node->ids.emplace_back(t, false);
+    for (Tensor& o : outs) torch::autograd::set_history(o, node);
+  }
+  return outs;
+}
+
+struct CombineJaggedBackward : Node {
+  CombinePtr c;
+  std::vector<int> modes;
+  std::vector<SavedVariable> ids, offsets;
+  std::vector<Tensor> weights;
+  variable_list apply(variable_list&& grads) override {
+    void* stream = current_stream();
+    for (const Combine::Group& g : c->groups) KRK_CALL(krk_group_set_stream, g.h, stream);
+    for (size_t i = 0; i < c->tables.size(); ++i) {
+      if (!grads[i].defined()) continue;       // an output the loss never used: nothing to push
+      const Tensor saved = ids[i].unpack(), off = offsets[i].unpack();
+      const Tensor g = grads[i].contiguous().to(at::kFloat);
+      KRK_CALL(krk_sparse_push_pooled, c->tables[i], c->optim, id_ptr(saved), saved.numel(), off_ptr(off),
+               off.numel() - 1, float_ptr(weights[i]), modes[i], float_ptr(g), c->dims[i], (float)c->lr, kFlags);
+    }
+    return variable_list(1);
+  }
+  void release_variables() override {
+    for (auto& v : ids) v.reset_data();
+    for (auto& v : offsets) v.reset_data();
+    weights.clear();
+  }
+  std::string name() const override { return "CombineJaggedEmbeddingFunctionBackward"; }
+};
+
+std::vector<Tensor> combine_jagged(const CombinePtr& c, const Tensor& param, const std::vector<int>& modes,
+                                   const std::vector<double>& patches, const std::vector<Tensor>& values,
+                                   const std::vector<Tensor>& offsets_in,
+                                   const std::vector<c10::optional<Tensor>>& weights_in) {
+  const size_t n = c->tables.size();
+  if (values.size() != n || offsets_in.size() != n || weights_in.size() != n || modes.size() != n ||
+      patches.size() != n)
+    throw py::value_error("one jagged batch per table");
+  void* stream = current_stream();
+  std::vector<Tensor> outs(n), ids(n), offsets(n), weights(n);
+  for (const Combine::Group& g : c->groups) KRK_CALL(krk_group_set_stream, g.h, stream);
+  for (size_t i = 0; i < n; ++i) {
+    ids[i] = ids_of(values[i]);
+    offsets[i] = ids_of(offsets_in[i], "offsets");
+    weights[i] = weights_of(weights_in[i]);
+    const int64_t bags = offsets[i].numel() - 1;
+    outs[i] = new_rows({bags, c->dims[i]}, ids[i]);
+    KRK_CALL(krk_sparse_pull_pooled, c->tables[i], id_ptr(ids[i]), ids[i].numel(), off_ptr(offsets[i]), bags,
+             float_ptr(weights[i]), modes[i], (float)patches[i], outs[i].mutable_data_ptr<float>(), kFlags);
+  }
+  if (recording(param)) {
+    auto node = new_node<CombineJaggedBackward>(param);
+    node->c = c;
+    node->modes = modes;
+    for (const Tensor& t : ids) node->ids.emplace_back(t, false);
+    for (const Tensor& t : offsets) node->offsets.emplace_back(t, false);
+    node->weights = weights;
+    for (Tensor& o : outs) torch::autograd::set_history(o, node);
+  }
+  return outs;
+}
+
+}  // namespace
+
+// The Python side hands over addresses of objects it keeps alive with the Parameter, which every
+// node keeps alive through its edge.
+PYBIND11_MODULE(_torch_native, m) {
+  using release = py::call_guard<py::gil_scoped_release>;
+  py::class_<Table, TablePtr>(m, "Table")
+      .def(py::init([](uintptr_t h, uintptr_t optim, int64_t dim, double lr) {
+        return std::make_shared<Table>(
+            Table{reinterpret_cast<krk_sparse*>(h), reinterpret_cast<const krk_optim*>(optim), dim, lr});
+      }))
+      .def_readwrite("lr", &Table::lr);
+  py::class_<Combine, CombinePtr>(m, "Combine")
+      .def(py::init([](const std::vector<std::tuple<uintptr_t, int64_t, std::vector<int>>>& groups,
+                       const std::vector<uintptr_t>& tables, const std::vector<int64_t>& dims, uintptr_t optim,
+                       double lr) {
+        auto c = std::make_shared<Combine>();
+        for (const auto& [h, dim, members] : groups)
+          c->groups.push_back({reinterpret_cast<krk_group*>(h), dim, members});
+        for (uintptr_t t : tables) c->tables.push_back(reinterpret_cast<krk_sparse*>(t));
+        c->dims = dims;
+        c->optim = reinterpret_cast<const krk_optim*>(optim);
+        c->lr = lr;
+        return c;
+      }))
+      .def_readwrite("lr", &Combine::lr);
+  m.def("embedding", &embedding, release());
+  m.def("jagged", &jagged, release());
+  m.def("combine", &combine, release());
+  m.def("combine_jagged", &combine_jagged, release());
+}

@@ -9,7 +9,8 @@ Nothing is copied to the host and nothing is synchronised: the table enqueues it
 torch's current stream.
 
 PyTorch is plumbing here (it owns the tensors and the stream); the arithmetic is the table
-engine's. Importing this module needs torch; nothing else in the package does.
+engine's. The autograd functions are native (csrc/torch_binding.cpp, built with the library).
+Importing this module needs torch; nothing else in the package does.
 """
 import ctypes as C
 
@@ -18,17 +19,12 @@ import torch
 from . import api
 from .configs import as_initializer, as_optim
 
-
-def _stream_ptr():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
-
-
-def _ids_ptr(indices):
-    """int64 indices are the uint64 ids bit for bit (worker/emitter.cc:126 casts the same way)."""
-    if indices.dtype != torch.int64 or not indices.is_cuda:
-        raise TypeError("indices must be an int64 CUDA tensor")
-    indices = indices.contiguous()
-    return indices, C.c_void_p(indices.data_ptr())
+api.lib()                                       # the native module links against it
+try:
+    from . import _torch_native as _native
+except ImportError as e:
+    raise ImportError("kraken_amd/_torch_native.so is missing or was built against another torch: build it with "
+                      "`python -m kraken_amd.build`") from e
 
 
 class GpuSparseTable(torch.nn.Parameter):
@@ -43,8 +39,16 @@ class GpuSparseTable(torch.nn.Parameter):
         self._table = api.SparseTable(dimension, as_initializer(initializer) or api.Initializer.create(
             api.InitializerType.kNormal, {}), capacity_hint=capacity_hint)
         self._optim = as_optim(optim) or api.Optim.create(api.OptimType.kSGD)
-        self.lr = float(lr)
+        self._native = _native.Table(self._table.h.value, C.addressof(self._optim.raw), self._dimension, float(lr))
         return self
+
+    @property
+    def lr(self):
+        return self._native.lr
+
+    @lr.setter
+    def lr(self, lr):
+        self._native.lr = float(lr)
 
     def dimension(self):
         return self._dimension
@@ -52,39 +56,13 @@ class GpuSparseTable(torch.nn.Parameter):
     def table(self):
         return self._table
 
-    def _on_current_stream(self):
-        api._check(api.lib().krk_sparse_set_stream(self._table.h, _stream_ptr()), "krk_sparse_set_stream")
-        return self._table.h
 
-
-class EmbeddingFunction(torch.autograd.Function):
-    """pytorch/embedding.py:9-23"""
+class EmbeddingFunction:
+    """pytorch/embedding.py:9-23: pulls the rows of `indices`; its backward pushes their gradients."""
 
     @staticmethod
-    def forward(ctx, sparse_table, indices):
-        ids, p_ids = _ids_ptr(indices)
-        dim = sparse_table.dimension()
-        out = torch.empty(tuple(indices.shape) + (dim,), dtype=torch.float32, device=indices.device)
-        h = sparse_table._on_current_stream()
-        # the table notes where it found every id: backward pushes gradients for this very
-        # tensor (autograd keeps it alive and unchanged), so its look-up need not be repeated
-        api._check(api.lib().krk_sparse_pull(h, p_ids, ids.numel(), C.c_void_p(out.data_ptr()),
-                                             api.DEVICE_PTRS | api.ASYNC | api.NOTE_ROWS), "krk_sparse_pull")
-        ctx.table = sparse_table
-        ctx.save_for_backward(ids)
-        return out
-
-    @staticmethod
-    def backward(ctx, grad):
-        (ids,) = ctx.saved_tensors
-        t = ctx.table
-        grad = grad.contiguous().to(torch.float32)
-        h = t._on_current_stream()
-        api._check(api.lib().krk_sparse_push_raw(h, C.byref(t._optim.raw), C.c_void_p(ids.data_ptr()), ids.numel(),
-                                                 C.c_void_p(grad.data_ptr()), t.dimension(), t.lr,
-                                                 api.DEVICE_PTRS | api.ASYNC | api.IDS_AS_PULLED),
-                   "krk_sparse_push_raw")
-        return None, None
+    def apply(sparse_table, indices):
+        return _native.embedding(sparse_table._native, sparse_table, indices)
 
 
 class Embedding(torch.nn.Module):
@@ -145,38 +123,12 @@ class JaggedTensor:
         return JaggedTensor(torch.cat(list_values, dim=0), torch.as_tensor(offsets), weights)
 
 
-class JaggedEmbeddingFunction(torch.autograd.Function):
+class JaggedEmbeddingFunction:
     """pytorch/jagged_embedding_funcs.py over pytorch/py/jagged_ops.cc, fused with the table."""
 
     @staticmethod
-    def forward(ctx, sparse_table, indices, offsets, weights, mode, patch_value):
-        ids, p_ids = _ids_ptr(indices)
-        if offsets.dtype != torch.int64 or not offsets.is_cuda:
-            raise TypeError("offsets must be an int64 CUDA tensor")
-        offsets = offsets.contiguous()
-        w = weights.contiguous().to(torch.float32) if weights is not None else None
-        bags = offsets.numel() - 1
-        out = torch.empty((bags, sparse_table.dimension()), dtype=torch.float32, device=indices.device)
-        h = sparse_table._on_current_stream()
-        api._check(api.lib().krk_sparse_pull_pooled(
-            h, p_ids, ids.numel(), C.c_void_p(offsets.data_ptr()), bags,
-            C.c_void_p(w.data_ptr()) if w is not None else None, mode, patch_value, C.c_void_p(out.data_ptr()),
-            api.DEVICE_PTRS | api.ASYNC), "krk_sparse_pull_pooled")
-        ctx.table, ctx.mode, ctx.weights = sparse_table, mode, w
-        ctx.save_for_backward(ids, offsets)
-        return out
-
-    @staticmethod
-    def backward(ctx, grad):
-        ids, offsets = ctx.saved_tensors
-        t, w = ctx.table, ctx.weights
-        grad = grad.contiguous().to(torch.float32)
-        h = t._on_current_stream()
-        api._check(api.lib().krk_sparse_push_pooled(
-            h, C.byref(t._optim.raw), C.c_void_p(ids.data_ptr()), ids.numel(), C.c_void_p(offsets.data_ptr()),
-            offsets.numel() - 1, C.c_void_p(w.data_ptr()) if w is not None else None, ctx.mode,
-            C.c_void_p(grad.data_ptr()), t.dimension(), t.lr, api.DEVICE_PTRS | api.ASYNC), "krk_sparse_push_pooled")
-        return None, None, None, None, None, None
+    def apply(sparse_table, indices, offsets, weights, mode, patch_value):
+        return _native.jagged(sparse_table._native, sparse_table, indices, offsets, weights, mode, patch_value)
 
 
 class JaggedEmbedding(torch.nn.Module):
@@ -220,8 +172,18 @@ class GpuCombineSparseTable(torch.nn.Parameter):
             self._members.setdefault(d, []).append(i)
         self._groups = {d: api.TableGroup([self._tables[i] for i in idx]) for d, idx in self._members.items()}
         self._optim = as_optim(optim) or api.Optim.create(api.OptimType.kSGD)
-        self.lr = float(lr)
+        self._native = _native.Combine([(self._groups[d].h.value, d, idx) for d, idx in self._members.items()],
+                                       [t.h.value for t in self._tables], self._dimensions,
+                                       C.addressof(self._optim.raw), float(lr))
         return self
+
+    @property
+    def lr(self):
+        return self._native.lr
+
+    @lr.setter
+    def lr(self, lr):
+        self._native.lr = float(lr)
 
     def dimensions(self):
         return self._dimensions
@@ -229,63 +191,15 @@ class GpuCombineSparseTable(torch.nn.Parameter):
     def tables(self):
         return self._tables
 
-    def _on_current_stream(self, dim):
-        g = self._groups[dim]
-        api._check(api.lib().krk_group_set_stream(g.h, _stream_ptr()), "krk_group_set_stream")
-        return g.h
 
-
-def _group_offsets(counts):
-    off = (C.c_int64 * (len(counts) + 1))()
-    for i, c in enumerate(counts):
-        off[i + 1] = off[i] + c
-    return off
-
-
-class CombineEmbeddingFunction(torch.autograd.Function):
+class CombineEmbeddingFunction:
     """pytorch/combine_embedding.py:10-31 over Emitter::CombinePullSparseTable /
     CombinePushSparseTable (worker/emitter.cc:185-283, 552-632): ids may repeat, within a table
     and across tables."""
 
     @staticmethod
-    def forward(ctx, table, *indices):
-        if len(indices) != len(table.dimensions()):
-            raise ValueError("one index tensor per table")
-        outs = [None] * len(indices)
-        saved = []
-        for dim, members in table._members.items():
-            parts = [_ids_ptr(indices[i])[0].reshape(-1) for i in members]
-            ids = torch.cat(parts) if len(parts) > 1 else parts[0]
-            off = _group_offsets([p.numel() for p in parts])
-            out = torch.empty((ids.numel(), dim), dtype=torch.float32, device=ids.device)
-            h = table._on_current_stream(dim)
-            api._check(api.lib().krk_group_pull(h, C.c_void_p(ids.data_ptr()), off, C.c_void_p(out.data_ptr()),
-                                                api.DEVICE_PTRS | api.ASYNC | api.NOTE_ROWS), "krk_group_pull")
-            for k, i in enumerate(members):
-                outs[i] = out[off[k]:off[k + 1]].view(tuple(indices[i].shape) + (dim,))
-            saved.append(ids)
-        ctx.table = table
-        ctx.counts = [x.numel() for x in indices]
-        ctx.save_for_backward(*saved)
-        return tuple(outs)
-
-    @staticmethod
-    def backward(ctx, *grads):
-        t = ctx.table
-        for ids, (dim, members) in zip(ctx.saved_tensors, t._members.items()):
-            counts = [ctx.counts[i] for i in members]
-            # an output the loss never used has no gradient: its rows get zeros
-            parts = [grads[i].reshape(-1, dim).to(torch.float32) if grads[i] is not None
-                     else torch.zeros((c, dim), dtype=torch.float32, device=ids.device)
-                     for i, c in zip(members, counts)]
-            g = (torch.cat(parts) if len(parts) > 1 else parts[0]).contiguous()
-            off = _group_offsets(counts)
-            h = t._on_current_stream(dim)
-            api._check(api.lib().krk_group_push_raw(h, C.byref(t._optim.raw), C.c_void_p(ids.data_ptr()), off,
-                                                    C.c_void_p(g.data_ptr()), dim, t.lr,
-                                                    api.DEVICE_PTRS | api.ASYNC | api.IDS_AS_PULLED),
-                       "krk_group_push_raw")
-        return (None,) * (1 + len(grads))
+    def apply(table, *indices):
+        return _native.combine(table._native, table, indices)
 
 
 class CombineEmbedding(torch.nn.Module):
@@ -299,60 +213,18 @@ class CombineEmbedding(torch.nn.Module):
     def forward(self, indices):
         if len(indices) != len(self.combine_sparse_table.dimensions()):
             raise ValueError("one index tensor per table")
-        return list(CombineEmbeddingFunction.apply(self.combine_sparse_table, *indices))
+        return CombineEmbeddingFunction.apply(self.combine_sparse_table, *indices)
 
 
-class CombineJaggedEmbeddingFunction(torch.autograd.Function):
-    """The pooling of pytorch/combine_jagged_embedding.py:47-80 fused with the tables: per table
-    one pooled pull forward and one pooled push backward, so the [n, dim] rows that the
+class CombineJaggedEmbeddingFunction:
+    """The pooling of pytorch/combine_jagged_embedding.py:47-80 fused with the tables: a
+    pooled pull forward and a pooled push backward, so the [n, dim] rows that the
     reference pulls, scales and then pools (JaggedEmbeddingSum/MeanFunction over
     pytorch/py/jagged_ops.cc) never exist in memory."""
 
     @staticmethod
-    def forward(ctx, table, modes, patch_values, n_tables, *tensors):
-        values = tensors[:n_tables]
-        offsets = tensors[n_tables:2 * n_tables]
-        weights = tensors[2 * n_tables:]
-        outs, saved, ws = [], [], []
-        for dim in table._members:                  # members run on their group's stream
-            table._on_current_stream(dim)
-        for i, t in enumerate(table.tables()):
-            ids, p_ids = _ids_ptr(values[i])
-            off = offsets[i]
-            if off.dtype != torch.int64 or not off.is_cuda:
-                raise TypeError("offsets must be an int64 CUDA tensor")
-            off = off.contiguous()
-            w = weights[i].contiguous().to(torch.float32) if weights[i] is not None else None
-            bags = off.numel() - 1
-            out = torch.empty((bags, table.dimensions()[i]), dtype=torch.float32, device=ids.device)
-            api._check(api.lib().krk_sparse_pull_pooled(
-                t.h, p_ids, ids.numel(), C.c_void_p(off.data_ptr()), bags,
-                C.c_void_p(w.data_ptr()) if w is not None else None, modes[i], patch_values[i],
-                C.c_void_p(out.data_ptr()), api.DEVICE_PTRS | api.ASYNC), "krk_sparse_pull_pooled")
-            outs.append(out)
-            saved += [ids, off]
-            ws.append(w)
-        ctx.table, ctx.modes, ctx.weights = table, modes, ws
-        ctx.save_for_backward(*saved)
-        return tuple(outs)
-
-    @staticmethod
-    def backward(ctx, *grads):
-        table = ctx.table
-        for dim in table._members:
-            table._on_current_stream(dim)
-        for i, t in enumerate(table.tables()):
-            if grads[i] is None:                    # an output the loss never used: nothing to push
-                continue
-            ids, off = ctx.saved_tensors[2 * i], ctx.saved_tensors[2 * i + 1]
-            w = ctx.weights[i]
-            g = grads[i].contiguous().to(torch.float32)
-            api._check(api.lib().krk_sparse_push_pooled(
-                t.h, C.byref(table._optim.raw), C.c_void_p(ids.data_ptr()), ids.numel(), C.c_void_p(off.data_ptr()),
-                off.numel() - 1, C.c_void_p(w.data_ptr()) if w is not None else None, ctx.modes[i],
-                C.c_void_p(g.data_ptr()), table.dimensions()[i], table.lr, api.DEVICE_PTRS | api.ASYNC),
-                "krk_sparse_push_pooled")
-        return (None,) * (4 + 3 * len(table.tables()))
+    def apply(table, modes, patch_values, values, offsets, weights):
+        return _native.combine_jagged(table._native, table, modes, patch_values, values, offsets, weights)
 
 
 class CombineJaggedEmbedding(torch.nn.Module):
@@ -377,7 +249,6 @@ class CombineJaggedEmbedding(torch.nn.Module):
 
     def forward(self, inputs):
         assert len(self._modes) == len(inputs)
-        n = len(inputs)
-        tensors = ([x.values() for x in inputs] + [x.offsets() for x in inputs] + [x.weights() for x in inputs])
-        return list(CombineJaggedEmbeddingFunction.apply(self.combine_sparse_table, self._modes,
-                                                         self._patch_values, n, *tensors))
+        return CombineJaggedEmbeddingFunction.apply(
+            self.combine_sparse_table, self._modes, self._patch_values, [x.values() for x in inputs],
+            [x.offsets() for x in inputs], [x.weights() for x in inputs])
