@@ -43,14 +43,13 @@ extern "C" {
  * the same ids (worker/emitter.cc:131-182 then :510-531; :552-612 for combined requests). The
  * two flags below let the second call reuse what the first one found. Both need
  * KRK_DEVICE_PTRS and are ignored by every other call.
- * KRK_NOTE_ROWS on krk_sparse_pull / krk_group_pull: the table (group) also keeps the row
- * number of every position of this request (4 bytes a position, in memory of its own) until
- * its next pull with the flag; single-table requests of 2^18 ids and more are not noted.
+ * KRK_NOTE_ROWS on krk_sparse_pull / krk_group_pull and their pooled forms: the table (group)
+ * also keeps the row number of every position of this request (4 bytes a position, in memory of
+ * its own) until its next pull with the flag.
  * KRK_IDS_AS_PULLED on krk_sparse_push / krk_sparse_push_raw / krk_group_push /
- * krk_group_push_raw: the caller states that `ids` is the buffer of that pull (same pointer,
- * same counts) with its contents unchanged. The call then skips its own look-up of the ids
- * (push_raw: for requests of at most 8192 ids a table, where the look-up is a launch of its
- * own). It looks the ids up as usual when the pointer or the counts differ from what was
+ * krk_group_push_raw and the pooled pushes: the caller states that `ids` is the buffer of that
+ * pull (same pointer, same counts) with its contents unchanged. The call then skips its own
+ * look-up of the ids. It looks the ids up as usual when the pointer or the counts differ from what was
  * noted, when nothing was noted, or when rows have moved since (krk_sparse_erase, a table that
  * grew or gained optimizer columns). Results are the same either way; ids whose contents did
  * change give the updates of the old ids' rows. */
@@ -405,6 +404,26 @@ typedef struct krk_part {
 int32_t krk_group_pull_parts(krk_group* g, const krk_part* parts, uint32_t flags);
 int32_t krk_group_push_raw_parts(krk_group* g, const krk_optim* o, const krk_part* parts, int64_t grad_dim,
                                  float lr, uint32_t flags);
+/* krk_sparse_pull_pooled and krk_sparse_push_pooled for every member of a group at once: one
+ * krk_pooled_part per member in member order, KRK_DEVICE_PTRS required. rows receives the
+ * member's pooled rows [bags, dim] (contiguous); of a push it holds the bags' gradient rows,
+ * `stride` floats apart, only read. A member without ids or bags in a push is left alone.
+ * KRK_NOTE_ROWS on the pull and KRK_IDS_AS_PULLED on the push as in krk_sparse_pull: the push of
+ * the ids that were pulled last need not look them up again. */
+typedef struct krk_pooled_part {
+  const uint64_t* ids;
+  int64_t n;
+  const int64_t* offsets;
+  int64_t bags;
+  const float* weights;
+  float* rows;
+  int64_t stride;
+  int32_t mode;
+  float patch_value;
+} krk_pooled_part;
+int32_t krk_group_pull_pooled_parts(krk_group* g, const krk_pooled_part* parts, uint32_t flags);
+int32_t krk_group_push_pooled_parts(krk_group* g, const krk_optim* o, const krk_pooled_part* parts,
+                                    int64_t grad_dim, float lr, uint32_t flags);
 /* krk_sparse_set_stream for a group and all its members. */
 int32_t krk_group_set_stream(krk_group* g, void* stream);
 

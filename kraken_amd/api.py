@@ -169,6 +169,9 @@ EXPORTS = {
     "krk_group_pull_parts": (C.c_int32, [C.c_void_p, C.c_void_p, C.c_uint32]),
     "krk_group_push_raw_parts": (C.c_int32, [C.c_void_p, C.POINTER(krk_optim), C.c_void_p, C.c_int64, C.c_float,
                                              C.c_uint32]),
+    "krk_group_pull_pooled_parts": (C.c_int32, [C.c_void_p, C.c_void_p, C.c_uint32]),
+    "krk_group_push_pooled_parts": (C.c_int32, [C.c_void_p, C.POINTER(krk_optim), C.c_void_p, C.c_int64, C.c_float,
+                                                C.c_uint32]),
     "krk_group_set_stream": (C.c_int32, [C.c_void_p, C.c_void_p]),
     "krk_event_elapsed_ms": (C.c_int32, [C.c_void_p, C.c_void_p, C.POINTER(C.c_float)]),
     "krk_dct2_forward": (C.c_int32, [C.c_void_p, C.c_void_p, C.c_int64, C.c_int32, C.c_uint32]),

@@ -12,9 +12,10 @@
 // itself a sorted sequence of (row, partial) and is reduced by the same kernel again until one
 // workgroup is left. Work per group is bounded by the tile size however skewed the ids are, and
 // the order of additions is fixed, so results do not change from run to run.
+#include <algorithm>
 #include <cstring>
 #include <new>
-
+#include <type_traits>
 
 #include "sparse_internal.h"
 
@@ -32,18 +33,7 @@ __device__ __forceinline__ void vload(const float* p, float (&v)[VEC]) {
     v[0] = *p;
   }
 }
-// A row that is read exactly once (the gradient rows a reduction gathers): non-temporal, so the
-// half gigabyte that passes through does not push the table's records out of the caches.
 typedef float vfloat4_t __attribute__((ext_vector_type(4)));
-template <int VEC>
-__device__ __forceinline__ void vload_once(const float* p, float (&v)[VEC]) {
-  if constexpr (VEC == 4) {
-    const vfloat4_t x = __builtin_nontemporal_load(reinterpret_cast<const vfloat4_t*>(p));
-    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
-  } else {
-    v[0] = __builtin_nontemporal_load(p);
-  }
-}
 template <int VEC>
 __device__ __forceinline__ void vstore_once(float* p, const float (&v)[VEC]) {
   if constexpr (VEC == 4) {
@@ -65,6 +55,17 @@ __device__ __forceinline__ void gload(const float* p, float (&v)[VEC]) {
     v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
   } else {
     v[0] = *(const KRK_GLOBAL float*)p;
+  }
+}
+// A row that is read exactly once (the gradient rows a reduction gathers): non-temporal, so the
+// half gigabyte that passes through does not push the table's records out of the caches.
+template <int VEC>
+__device__ __forceinline__ void gload_once(const KRK_GLOBAL float* p, float (&v)[VEC]) {
+  if constexpr (VEC == 4) {
+    const vfloat4_t x = __builtin_nontemporal_load((const KRK_GLOBAL vfloat4_t*)p);
+    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+  } else {
+    v[0] = __builtin_nontemporal_load(p);
   }
 }
 template <int VEC>
@@ -336,11 +337,15 @@ __global__ __launch_bounds__(kBlock) void rows_of_ids_kernel(TableView tv, const
 }
 
 // The same for a combined request: position p belongs to the member whose [row_start, row_start
-// of the next) holds it; its key is (member << row_bits) | row. A missing id raises the error
-// on its own member.
+// of the next) holds it; its key is (member << row_bits) | row, its payload the position inside the
+// member's request. A missing id raises the error on its own member.
+// bag_of (pooled pushes only): as above, a bag counted inside its member; bit m of bag_payload says
+// that member m's payload is the bag.
 __global__ __launch_bounds__(kBlock) void group_rows_of_ids_kernel(const TableDesc* __restrict__ descs,
                                                                    GroupCall call, GroupParts parts,
                                                                    int row_bits, uint32_t miss_key,
+                                                                   const uint32_t* __restrict__ bag_of,
+                                                                   uint32_t bag_payload,
                                                                    uint32_t* __restrict__ keys,
                                                                    uint32_t* __restrict__ pos) {
   // a workgroup serves one member (call.block_start counts workgroups of kBlock / kBucket
@@ -354,29 +359,64 @@ __global__ __launch_bounds__(kBlock) void group_rows_of_ids_kernel(const TableDe
   const int64_t i = (int64_t)(blockIdx.x - call.block_start[m]) * (kBlock / kBucket) + threadIdx.x / kBucket;
   const int64_t p = call.row_start[m] + i;
   const int gl = threadIdx.x & (kBucket - 1);
-  const bool active = p < call.row_start[m + 1];
+  const bool here = p < call.row_start[m + 1];
+  const uint32_t bag = (bag_of && here) ? bag_of[p] : 0u;
+  const bool active = here && bag != kNoBag;
   const TableView tv = descs[m].tv;
   uint32_t r = probe_find(tv, active ? parts.ids[m][i] : 0, active, gl, kBucket);
-  if (!active || gl != 0) return;
-  if (r == kEmptyRow) {
+  if (!here || gl != 0) return;
+  if (!active) {
+    r = miss_key;
+  } else if (r == kEmptyRow) {
     atomicOr(&tv.counters[1], kErrMissingId);
     r = miss_key;
   } else {
     r |= (uint32_t)m << row_bits;
   }
   keys[p] = r;
-  if (pos) pos[p] = (uint32_t)p;
+  if (pos) pos[p] = ((bag_payload >> m) & 1u) ? bag : (uint32_t)i;
 }
 
-// The gradient rows of a combined request that come in parts, one array after the other.
-__global__ __launch_bounds__(kBlock) void gather_parts_kernel(GroupCall call, GroupParts parts, int dim, int64_t total,
-                                                              float* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= total) return;
-  const int64_t p = i / dim;
+// The key of a position whose row the pull of these ids noted (KRK_IDS_AS_PULLED). A note of
+// kEmptyRow was taken while the row's creator, another wavefront of that pull, had not published
+// its number yet: those ids are looked up.
+__device__ __forceinline__ uint32_t noted_key(const TableView& tv, uint32_t row, const uint64_t* __restrict__ id,
+                                              uint32_t member_key, uint32_t miss_key) {
+  if (row == kEmptyRow) {
+    row = probe_find_alone(tv, *id);
+    if (row == kEmptyRow) {
+      atomicOr(&tv.counters[1], kErrMissingId);
+      return miss_key;
+    }
+  }
+  return member_key | row;
+}
+
+// Keys and payloads of a push whose rows were noted: a stream over the notes (12 bytes a position)
+// instead of a look-up of every id (a sector of the index each: 8.5 million ids of a four-million
+// row table 175 us, a million 15 us).
+__global__ __launch_bounds__(kBlock) void noted_keys_kernel(TableView tv, const uint64_t* __restrict__ ids, int64_t n,
+                                                            const uint32_t* __restrict__ notes, uint32_t miss_key,
+                                                            uint32_t* __restrict__ keys, uint32_t* __restrict__ pos) {
+  const int64_t p = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (p >= n) return;
+  keys[p] = noted_key(tv, notes[p], ids + p, 0u, miss_key);
+  pos[p] = (uint32_t)p;
+}
+
+__global__ __launch_bounds__(kBlock) void group_noted_keys_kernel(const TableDesc* __restrict__ descs, GroupCall call,
+                                                                  GroupParts parts, int64_t total, int row_bits,
+                                                                  uint32_t miss_key,
+                                                                  const uint32_t* __restrict__ notes,
+                                                                  uint32_t* __restrict__ keys,
+                                                                  uint32_t* __restrict__ pos) {
+  const int64_t p = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (p >= total) return;
   int m = 0;
   while (m + 1 < call.n_tables && p >= call.row_start[m + 1]) ++m;
-  out[i] = parts.rows[m][(p - call.row_start[m]) * (int64_t)parts.stride[m] + (i - p * dim)];
+  const int64_t i = p - call.row_start[m];
+  keys[p] = noted_key(descs[m].tv, notes[p], parts.ids[m] + i, (uint32_t)m << row_bits, miss_key);
+  pos[p] = (uint32_t)i;
 }
 
 // ---- pooled pushes: from bag offsets to per-position bag numbers ----------------
@@ -387,27 +427,60 @@ __global__ __launch_bounds__(kBlock) void fill_u32_kernel(uint32_t* __restrict__
 
 constexpr int kBagLanes = 8;   // lanes that share one bag's positions
 
-__global__ __launch_bounds__(kBlock) void bag_expand_kernel(const long long* __restrict__ offsets, int64_t bags,
-                                                            int64_t n, uint32_t* __restrict__ bag_of) {
-  const int64_t b = (int64_t)blockIdx.x * (kBlock / kBagLanes) + threadIdx.x / kBagLanes;
+// What the bags of a pooled push leave for the reduction. Always: ratio[bag], where the member's
+// bags are means, is what a mean bag hands on of its gradient (pytorch/py/jagged_ops.cc:303-334:
+// (float)(1.0 / float(len)), once per bag here as there; the reduction multiplies each gradient
+// row it reads, so no scaled copy of the gradients is written and read back: 852k bags of 32 floats
+// took 85 us for that). bag_of[position] = the bag, kNoBag outside every bag.
+// NOTED: the rows of the positions are known from the pull, so the bag also writes its positions'
+// keys and payloads and no other launch looks at them; bag_of is then only written where a member
+// is weighted (its payloads are positions).
+template <bool GROUPED, bool NOTED>
+__global__ __launch_bounds__(kBlock) void bag_expand_kernel(const TableDesc* __restrict__ descs, TableView tv,
+                                                            PooledCall call, int row_bits, uint32_t miss_key,
+                                                            const uint32_t* __restrict__ notes,
+                                                            uint32_t* __restrict__ bag_of, float* __restrict__ ratio,
+                                                            uint32_t* __restrict__ keys, uint32_t* __restrict__ pos) {
+  int m = 0;
+  if (GROUPED) {
+    if (call.even_blocks) {
+      m = (int)(blockIdx.x / call.even_blocks);
+    } else {
+      while (m + 1 < call.n_tables && blockIdx.x >= call.block_start[m + 1]) ++m;
+    }
+    if (NOTED) tv = descs[m].tv;
+  }
+  const int64_t b = (int64_t)(blockIdx.x - call.block_start[m]) * (kBlock / kBagLanes) + threadIdx.x / kBagLanes;
+  const int64_t bags = call.bag_start[m + 1] - call.bag_start[m];
   if (b >= bags) return;
-  long long lo = offsets[b], hi = offsets[b + 1];
-  if (lo < 0) lo = 0;
-  if (hi > n) hi = n;
-  for (long long p = lo + (threadIdx.x & (kBagLanes - 1)); p < hi; p += kBagLanes) bag_of[p] = (uint32_t)b;
-}
-
-// pytorch/py/jagged_ops.cc:303-334 : a mean bag hands every one of its rows grads * ratio,
-// ratio = (float)(1.0 / float(len)); computed once per bag here as there.
-__global__ __launch_bounds__(kBlock) void bag_scale_kernel(const float* __restrict__ grads,
-                                                           const long long* __restrict__ offsets,
-                                                           int64_t bags, int dim, float* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= bags * dim) return;
-  const int64_t b = i / dim;
-  const long long len = offsets[b + 1] - offsets[b];
-  const float ratio = len > 0 ? (float)(1.0 / (double)(float)len) : 0.0f;
-  out[i] = grads[i] * ratio;
+  const int gl = threadIdx.x & (kBagLanes - 1);
+  const int64_t a = call.row_start[m];
+  const int64_t n = call.row_start[m + 1] - a;
+  const long long begin = call.offsets[m][b], end = call.offsets[m][b + 1];
+  if (gl == 0 && ((call.mean_bits >> m) & 1u))
+    ratio[call.bag_start[m] + b] = end > begin ? (float)(1.0 / (double)(float)(end - begin)) : 0.0f;
+  const bool weighted = call.weights[m] != nullptr;
+  const uint32_t member_key = (uint32_t)m << row_bits;
+  const long long lo = begin < 0 ? 0 : begin, hi = end > n ? n : end;
+  for (long long p = lo + gl; p < hi; p += kBagLanes) {
+    if (NOTED) {
+      keys[a + p] = noted_key(tv, notes[a + p], call.ids[m] + p, member_key, miss_key);
+      if (pos) pos[a + p] = weighted ? (uint32_t)p : (uint32_t)b;
+    }
+    if (!NOTED || weighted || !pos) bag_of[a + p] = (uint32_t)b;
+  }
+  // positions before the first bag and behind the last belong to none
+  auto outside = [&](long long from, long long to) {
+    for (long long p = from + gl; p < to; p += kBagLanes) {
+      bag_of[a + p] = kNoBag;
+      if (NOTED) {
+        keys[a + p] = miss_key;
+        if (pos) pos[a + p] = 0u;
+      }
+    }
+  };
+  if (b == 0) outside(0, begin < n ? begin : n);
+  if (b == bags - 1) outside(end > 0 ? end : 0, n);
 }
 
 // ---------------------------------------------------------------------------
@@ -524,11 +597,21 @@ constexpr int kPrefetch = 4;
 constexpr int kPrefetchCarry = 4;
 constexpr int kCarryTile = 4;   // 16, 32 and 64 were measured: 254, 272 and 304 us for a million dim-128 ids against 244
 
-// Weighted bags (level 0 only): the sorted payload is a position p, its gradient row is
-// vals[bag_of[p]] times weight[p]. Both null otherwise: the payload itself names the row.
+// Pooled pushes (level 0 only). Weighted bags: the sorted payload is a position p, its gradient row
+// is that of bag bag_of[p], times weight[p]; otherwise weight is null and the payload itself names
+// the row. ratio (bags that are means, else null): what a bag hands on of its gradient.
 struct PooledSrc {
   const uint32_t* bag_of;
   const float* weight;
+  const float* ratio;
+};
+// The same for a combined push: the gradient rows lie where the members have them, and bag_of,
+// the ratios and the payloads count from the member's first position and bag. bag_of null: not pooled.
+struct GroupPooledSrc {
+  PooledCall call;
+  const uint32_t* bag_of;
+  const float* ratio;
+  int weighted;          // some member is
 };
 
 // Combined pushes (GROUPED): a key is (member number << row_bits) | row, and a closed run takes
@@ -542,10 +625,14 @@ struct GroupSrc {
 };
 
 // LDS of one workgroup, in 32-bit words: partial sums [2 * per_block][group * VEC] first (vector
-// accesses, 16-byte aligned), then partial keys [2 * per_block], the two carry keys, the staged
-// keys [span + 2], payloads [span] and weights [span].
-__host__ __device__ inline size_t segreduce_lds_words(int per_block, int group, int vec, int tile) {
-  return (size_t)2 * per_block * group * vec + 2 * per_block + 2 + 3 * (size_t)per_block * tile + 2;
+// accesses, 16-byte aligned), then at level 0 the staged gradient rows [span] (two words each: their
+// addresses), then partial keys [2 * per_block], the two carry keys, the staged keys [span + 2], and
+// for pooled pushes weights [span] and ratios [span].
+__host__ __device__ inline size_t segreduce_lds_words(int per_block, int group, int vec, int tile, bool level0,
+                                                      bool pooled) {
+  const size_t span = (size_t)per_block * tile;
+  return (size_t)2 * per_block * group * vec + (level0 ? 2 * span : 0) + 2 * per_block + 2 + span + 2 +
+         (pooled ? 2 * span : 0);
 }
 
 template <int OPT, int VEC, bool LEVEL0, bool GROUPED>
@@ -553,23 +640,46 @@ __global__ __launch_bounds__(kBlock) void segreduce_kernel(
     TableView tv, const uint32_t* __restrict__ keys, const uint32_t* __restrict__ pos,
     const float* __restrict__ vals, int64_t cnt, int tile, uint32_t empty_from,
     uint32_t* __restrict__ keys_out, float* __restrict__ vals_out, int dim, int elems, int group,
-    ApplyArgs args, PooledSrc ps, GroupSrc gs) {
-  extern __shared__ uint32_t lds[];
+    ApplyArgs args, std::conditional_t<LEVEL0 && GROUPED, GroupPooledSrc, PooledSrc> ps, GroupSrc gs) {
+  extern __shared__ __align__(16) uint32_t lds[];
   const int per_block = kBlock / group;
   const int span = per_block * tile;                       // entries staged by this workgroup
   const int64_t first = (int64_t)blockIdx.x * span;        // global index of lds_keys[1]
   float* part_val = reinterpret_cast<float*>(lds);         // [2 * per_block][group * VEC]
-  uint32_t* part_key = lds + 2 * per_block * group * VEC;  // [2 * per_block]
+  const KRK_GLOBAL float** lds_src = reinterpret_cast<const KRK_GLOBAL float**>(lds + 2 * per_block * group * VEC);   // [span]
+  uint32_t* part_key = lds + 2 * per_block * group * VEC + (LEVEL0 ? 2 * span : 0);   // [2 * per_block]
   uint32_t* out_key = part_key + 2 * per_block;            // [2]: what this workgroup carries on
   uint32_t* lds_keys = out_key + 2;                        // [span + 2], shifted by one
-  uint32_t* lds_pos = lds_keys + span + 2;                 // [span]
-  float* lds_w = reinterpret_cast<float*>(lds_pos + span); // [span], weighted bags only
+  float* lds_w = reinterpret_cast<float*>(lds_keys + span + 2);   // [span] \ pooled pushes only
+  float* lds_r = lds_w + span;                                    // [span] /
   for (int i = threadIdx.x; i < span + 2; i += kBlock) {
     const int64_t j = first + i - 1;
     lds_keys[i] = (j >= 0 && j < cnt) ? keys[j] : kNoRow;
   }
-  const bool weighted = LEVEL0 && ps.weight != nullptr;
-  if (LEVEL0) {
+  bool weighted = false, scaled = false;
+  if constexpr (LEVEL0 && GROUPED) {
+    weighted = ps.bag_of != nullptr && ps.weighted != 0;
+    scaled = ps.ratio != nullptr;
+    for (int i = threadIdx.x; i < span; i += kBlock) {
+      const int64_t j = first + i;
+      const uint32_t key = j < cnt ? keys[j] : kNoRow;
+      const KRK_GLOBAL float* src = nullptr;
+      if (key < empty_from) {
+        const int m = (int)(key >> gs.row_bits);
+        uint32_t p = pos[j];
+        if (weighted) {
+          const float* w = ps.call.weights[m];
+          lds_w[i] = w ? w[p] : 1.0f;
+          if (w) p = ps.bag_of[ps.call.row_start[m] + p];
+        }
+        if (scaled) lds_r[i] = ((ps.call.mean_bits >> m) & 1u) ? ps.ratio[ps.call.bag_start[m] + p] : 1.0f;
+        src = (const KRK_GLOBAL float*)ps.call.rows[m] + (int64_t)p * ps.call.stride[m];
+      }
+      lds_src[i] = src;
+    }
+  } else if constexpr (LEVEL0) {
+    weighted = ps.weight != nullptr;
+    scaled = ps.ratio != nullptr;
     for (int i = threadIdx.x; i < span; i += kBlock) {
       const int64_t j = first + i;
       uint32_t p = j < cnt ? pos[j] : 0u;
@@ -579,7 +689,11 @@ __global__ __launch_bounds__(kBlock) void segreduce_kernel(
         const uint32_t b = j < cnt ? ps.bag_of[p] : 0u;
         p = b == kNoBag ? 0u : b;
       }
-      lds_pos[i] = p;
+      if (scaled) {
+        if (p == kNoBag) p = 0u;                           // outside every bag: its key is skipped
+        lds_r[i] = ps.ratio[p];
+      }
+      lds_src[i] = (const KRK_GLOBAL float*)vals + (int64_t)p * dim;
     }
   }
   if (threadIdx.x < 2) out_key[threadIdx.x] = kNoRow;
@@ -684,8 +798,16 @@ __global__ __launch_bounds__(kBlock) void segreduce_kernel(
           const int j = j0 + u;
           k[u] = j < lb ? lds_keys[j + 1] : kNoRow;
           if (j < lb && k[u] < empty_from && lane_on) {
-            const float* src = LEVEL0 ? vals + (int64_t)lds_pos[j] * dim : vals + (first + j) * dim;
-            if constexpr (LEVEL0) vload_once<VEC>(src + e * VEC, v[u]); else vload<VEC>(src + e * VEC, v[u]);
+            if constexpr (LEVEL0) {
+              gload_once<VEC>(lds_src[j] + e * VEC, v[u]);
+            } else {
+              vload<VEC>(vals + (first + j) * dim + e * VEC, v[u]);
+            }
+            if (scaled) {
+              const float r = lds_r[j];
+#pragma unroll
+              for (int c = 0; c < VEC; ++c) v[u][c] = v[u][c] * r;
+            }
             if (weighted) {
               const float w = lds_w[j];
 #pragma unroll
@@ -777,18 +899,19 @@ static void launch_segreduce(bool level0, const TableView& tv, const uint32_t* k
                              const float* vals, int64_t cnt, int tile, uint32_t empty_from,
                              uint32_t* keys_out, float* vals_out, const ReduceShape* t,
                              const ApplyArgs& args, const PooledSrc& ps, const GroupSrc* gs,
-                             hipStream_t stream) {
+                             const GroupPooledSrc* gps, hipStream_t stream) {
   const int per_block = kBlock / t->group;
   const int64_t tiles = (cnt + tile - 1) / tile;
   const dim3 grid(grid_for(tiles, per_block)), block(kBlock);
-  const size_t lds_bytes = segreduce_lds_words(per_block, t->group, VEC, tile) * sizeof(uint32_t);
-  const PooledSrc none{nullptr, nullptr};
+  const bool pooled = level0 && (gps ? gps->bag_of || gps->ratio : ps.weight || ps.ratio);
+  const size_t lds_bytes = segreduce_lds_words(per_block, t->group, VEC, tile, level0, pooled) * sizeof(uint32_t);
+  const PooledSrc none{nullptr, nullptr, nullptr};
   if constexpr (OPT != kOptStore) {
     if (gs) {
       if (level0) {
         hipLaunchKernelGGL((segreduce_kernel<OPT, VEC, true, true>), grid, block, lds_bytes, stream, tv, keys,
                            pos, vals, cnt, tile, empty_from, keys_out, vals_out, (int)t->dim, t->elems,
-                           t->group, args, ps, *gs);
+                           t->group, args, *gps, *gs);
       } else {
         hipLaunchKernelGGL((segreduce_kernel<OPT, VEC, false, true>), grid, block, lds_bytes, stream, tv, keys,
                            pos, vals, cnt, tile, empty_from, keys_out, vals_out, (int)t->dim, t->elems,
@@ -814,27 +937,27 @@ static void dispatch_segreduce(int opt, bool level0, const TableView& tv, const 
                                const uint32_t* pos, const float* vals, int64_t cnt, int tile,
                                uint32_t empty_from, uint32_t* keys_out, float* vals_out,
                                const ReduceShape* t, const ApplyArgs& args, const PooledSrc& ps,
-                               const GroupSrc* gs, hipStream_t stream) {
+                               const GroupSrc* gs, const GroupPooledSrc* gps, hipStream_t stream) {
   switch (opt) {
     case kOptStore:
       launch_segreduce<kOptStore, VEC>(level0, tv, keys, pos, vals, cnt, tile, empty_from, keys_out,
-                                       vals_out, t, args, ps, gs, stream);
+                                       vals_out, t, args, ps, gs, gps, stream);
       break;
     case KRK_SGD:
       launch_segreduce<KRK_SGD, VEC>(level0, tv, keys, pos, vals, cnt, tile, empty_from, keys_out,
-                                     vals_out, t, args, ps, gs, stream);
+                                     vals_out, t, args, ps, gs, gps, stream);
       break;
     case KRK_ADAGRAD:
       launch_segreduce<KRK_ADAGRAD, VEC>(level0, tv, keys, pos, vals, cnt, tile, empty_from, keys_out,
-                                         vals_out, t, args, ps, gs, stream);
+                                         vals_out, t, args, ps, gs, gps, stream);
       break;
     case KRK_ADAM:
       launch_segreduce<KRK_ADAM, VEC>(level0, tv, keys, pos, vals, cnt, tile, empty_from, keys_out,
-                                      vals_out, t, args, ps, gs, stream);
+                                      vals_out, t, args, ps, gs, gps, stream);
       break;
     default:
       launch_segreduce<KRK_RMSPROP, VEC>(level0, tv, keys, pos, vals, cnt, tile, empty_from, keys_out,
-                                         vals_out, t, args, ps, gs, stream);
+                                         vals_out, t, args, ps, gs, gps, stream);
       break;
   }
 }
@@ -883,7 +1006,6 @@ static int pick_tile(int64_t cnt) {
 constexpr int kSortBlock = 1024;
 constexpr int kSortItems = 8;
 constexpr int kSortMax = kSortBlock * kSortItems;      // ids per table
-static_assert(kSortMax <= kNotedMax, "row notes are kept for the requests that take this path");
 constexpr int kSortWaves = kSortBlock / kWave;
 constexpr int kMaxBucketBits = 5;                      // up to 32 buckets a table
 constexpr int kDigitBits = 9;
@@ -896,6 +1018,17 @@ constexpr int kRunListMax = kSortMax / (kShortRun + 1) + 1;   // runs above kSho
 constexpr int kPartOffset = (kSortMax + 1 + 2 * kRunListMax + 3) & ~3;   // the partial sums start on 16 bytes
 constexpr int kShortMaxDim = 64;
 static_assert(kSortWaves * kDigits <= kSortMax + 1, "the histogram fits the work space");
+
+// Pooled pushes: spos holds a bag (counted in its member) where the member's bags are not weighted,
+// a position where they are; bag_of and ratio as bag_expand_kernel leaves them.
+struct BucketPooled {
+  const uint32_t* bag_of;
+  const float* ratio;
+  uint32_t mean_bits;
+  int64_t bag_start[kMaxGroupTables];
+  const float* weights[kMaxGroupTables];
+};
+constexpr int64_t kBucketMaxBags = 65536;              // a bag is kept in 16 bits
 
 struct SortCall {
   int32_t n_tables;
@@ -955,11 +1088,11 @@ __device__ __forceinline__ uint32_t sort_block_scan(uint32_t v, uint32_t* wave_t
 }
 
 // grid: one workgroup per bucket (n_tables << bucket_bits)
-template <int OPT, int VEC, bool GROUPED>
-__global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(const TableDesc* __restrict__ descs, TableView tv,
-                                                                 SortCall call, GroupParts parts,
-                                                                 const uint32_t* __restrict__ keys, int dim,
-                                                                 int elems, int group, ApplyArgs args, GroupSrc gs) {
+template <int OPT, int VEC, bool GROUPED, bool POOLED>
+__global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(
+    const TableDesc* __restrict__ descs, TableView tv, SortCall call, GroupParts parts,
+    const uint32_t* __restrict__ keys, int dim, int elems, int group, ApplyArgs args, GroupSrc gs,
+    std::conditional_t<POOLED, BucketPooled, int> pool) {
   __shared__ uint32_t skey[kSortMax];                  // row >> bucket_bits
   __shared__ uint16_t spos[kSortMax];
   // histogram [wave][digit] while sorting; partial sums and their keys while reducing
@@ -1029,6 +1162,9 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(const TableDesc
     if (take & (1u << i)) {
       skey[at] = (mine[i] & call.row_mask) >> bucket_bits;
       spos[at] = (uint16_t)(t * own + i);
+      if constexpr (POOLED) {
+        if (!pool.weights[m]) spos[at] = (uint16_t)pool.bag_of[a + t * own + i];
+      }
       ++at;
     }
   }
@@ -1139,6 +1275,30 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(const TableDesc
   const bool lane_on = gl < elems;
   const float* g_base = parts.rows[m];
   const uint32_t g_stride = parts.stride[m];
+  // the gradient row of entry j of the sorted list
+  auto load_grad = [&](int j, float (&v)[VEC]) {
+    if constexpr (!POOLED) {
+      gload<VEC>(g_base + (int64_t)spos[j] * g_stride + gl * VEC, v);
+    } else {
+      uint32_t b = spos[j];
+      float w = 1.0f;
+      const bool weighted = pool.weights[m] != nullptr;
+      if (weighted) {
+        w = pool.weights[m][b];
+        b = pool.bag_of[a + b];
+      }
+      gload<VEC>(g_base + (int64_t)b * g_stride + gl * VEC, v);
+      if ((pool.mean_bits >> m) & 1u) {
+        const float r = pool.ratio[pool.bag_start[m] + b];
+#pragma unroll
+        for (int c = 0; c < VEC; ++c) v[c] = v[c] * r;
+      }
+      if (weighted) {
+#pragma unroll
+        for (int c = 0; c < VEC; ++c) v[c] = v[c] * w;
+      }
+    }
+  };
   // Who adds a run up: a lane group (up to kShortRun entries, the reference's order exactly), a
   // wavefront (its lane groups take a stretch each and the stretches' sums are added in order),
   // or the whole workgroup. A lane group walking 64 entries on its own took eight trips to memory
@@ -1165,7 +1325,7 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(const TableDesc
 #pragma unroll
       for (int u = 0; u < kRunAhead; ++u) {
         if (j0 + u < hi && lane_on) {
-          gload<VEC>(g_base + (int64_t)spos[j0 + u] * g_stride + gl * VEC, v[u]);
+          load_grad(j0 + u, v[u]);
         } else {
 #pragma unroll
           for (int c = 0; c < VEC; ++c) v[u][c] = 0.0f;
@@ -1195,7 +1355,7 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(const TableDesc
 #pragma unroll
     for (int u = 0; u < kPairAhead; ++u) {
       if (lo + u < hi && lane_on) {
-        gload<VEC>(g_base + (int64_t)spos[lo + u] * g_stride + gl * VEC, v[u]);
+        load_grad(lo + u, v[u]);
       } else {
 #pragma unroll
         for (int c = 0; c < VEC; ++c) v[u][c] = 0.0f;
@@ -1218,7 +1378,7 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(const TableDesc
 #pragma unroll
       for (int u = 0; u < kRunAhead; ++u) {
         if (j0 + u < hi && lane_on) {
-          gload<VEC>(g_base + (int64_t)spos[j0 + u] * g_stride + gl * VEC, w[u]);
+          load_grad(j0 + u, w[u]);
         } else {
 #pragma unroll
           for (int c = 0; c < VEC; ++c) w[u][c] = 0.0f;
@@ -1329,26 +1489,42 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(const TableDesc
   }
 }
 
+template <int OPT, int VEC, bool GROUPED>
+static void launch_bucket_push_opt(unsigned buckets, hipStream_t stream, const TableDesc* descs, const TableView& tv,
+                                   const SortCall& call, const GroupParts& parts, const uint32_t* keys, int dim,
+                                   int elems, int group, const ApplyArgs& args, const GroupSrc& gs,
+                                   const BucketPooled* pool) {
+  const dim3 grid(buckets), block(kSortBlock);
+  if (pool) {
+    hipLaunchKernelGGL((bucket_push_kernel<OPT, VEC, GROUPED, true>), grid, block, 0, stream, descs, tv, call, parts,
+                       keys, dim, elems, group, args, gs, *pool);
+  } else {
+    hipLaunchKernelGGL((bucket_push_kernel<OPT, VEC, GROUPED, false>), grid, block, 0, stream, descs, tv, call, parts,
+                       keys, dim, elems, group, args, gs, 0);
+  }
+}
+
 template <int VEC, bool GROUPED>
 static void launch_bucket_push(int opt, unsigned buckets, hipStream_t stream, const TableDesc* descs,
-                               const TableView& tv, const SortCall& call, const GroupParts& parts, const uint32_t* keys, int dim, int elems, int group, const ApplyArgs& args, const GroupSrc& gs) {
-  const dim3 grid(buckets), block(kSortBlock);
+                               const TableView& tv, const SortCall& call, const GroupParts& parts,
+                               const uint32_t* keys, int dim, int elems, int group, const ApplyArgs& args,
+                               const GroupSrc& gs, const BucketPooled* pool = nullptr) {
   switch (opt) {
     case KRK_SGD:
-      hipLaunchKernelGGL((bucket_push_kernel<KRK_SGD, VEC, GROUPED>), grid, block, 0, stream, descs, tv, call, parts,
-                         keys, dim, elems, group, args, gs);
+      launch_bucket_push_opt<KRK_SGD, VEC, GROUPED>(buckets, stream, descs, tv, call, parts, keys, dim, elems, group,
+                                                    args, gs, pool);
       break;
     case KRK_ADAGRAD:
-      hipLaunchKernelGGL((bucket_push_kernel<KRK_ADAGRAD, VEC, GROUPED>), grid, block, 0, stream, descs, tv, call,
-                         parts, keys, dim, elems, group, args, gs);
+      launch_bucket_push_opt<KRK_ADAGRAD, VEC, GROUPED>(buckets, stream, descs, tv, call, parts, keys, dim, elems,
+                                                        group, args, gs, pool);
       break;
     case KRK_ADAM:
-      hipLaunchKernelGGL((bucket_push_kernel<KRK_ADAM, VEC, GROUPED>), grid, block, 0, stream, descs, tv, call, parts,
-                         keys, dim, elems, group, args, gs);
+      launch_bucket_push_opt<KRK_ADAM, VEC, GROUPED>(buckets, stream, descs, tv, call, parts, keys, dim, elems, group,
+                                                     args, gs, pool);
       break;
     default:
-      hipLaunchKernelGGL((bucket_push_kernel<KRK_RMSPROP, VEC, GROUPED>), grid, block, 0, stream, descs, tv, call,
-                         parts, keys, dim, elems, group, args, gs);
+      launch_bucket_push_opt<KRK_RMSPROP, VEC, GROUPED>(buckets, stream, descs, tv, call, parts, keys, dim, elems,
+                                                        group, args, gs, pool);
       break;
   }
 }
@@ -1370,12 +1546,13 @@ static bool short_push_fits(int64_t longest, int64_t dim, int elems, int group) 
 // Stable sort of (key, payload) by key, then the tiled segmented reduction: every run of equal
 // keys is summed in payload order and handed to apply_row<opt> once. `fill(keys, payload)`
 // enqueues the kernel that writes the n unsorted pairs; keys >= miss_key are skipped. d_vals
-// holds one value row per payload. scratch[0..4] is the caller's work space.
+// holds one value row per payload (combined pushes: gps says where they lie). scratch[0..4] is the
+// caller's work space.
 template <typename Fill>
 static int32_t sort_and_reduce(const ReduceShape& sh, hipStream_t stream, DeviceBuffer* scratch,
                                const TableView& tv, int opt, int64_t n, uint32_t miss_key, int bits,
                                const float* d_vals, const ApplyArgs& args, const PooledSrc& ps,
-                               const GroupSrc* gs, Fill fill) {
+                               const GroupSrc* gs, const GroupPooledSrc* gps, Fill fill) {
   const int tile0 = pick_tile(n);
   const int per_block = kBlock / sh.group;
   const int64_t groups0 = ((n + tile0 - 1) / tile0 + per_block - 1) / per_block;   // workgroups of level 0
@@ -1415,10 +1592,10 @@ static int32_t sort_and_reduce(const ReduceShape& sh, hipStream_t stream, Device
     }
     if (sh.vec == 4) {
       dispatch_segreduce<4>(opt, level0, tv, in_keys, spos, in_vals, cnt, tile, miss_key, okeys, ovals, &sh,
-                            args, ps, gs, stream);
+                            args, ps, gs, gps, stream);
     } else {
       dispatch_segreduce<1>(opt, level0, tv, in_keys, spos, in_vals, cnt, tile, miss_key, okeys, ovals, &sh,
-                            args, ps, gs, stream);
+                            args, ps, gs, gps, stream);
     }
     KRK_HIP(hipGetLastError());
     if (groups <= 1) break;
@@ -1432,19 +1609,7 @@ static int32_t sort_and_reduce(const ReduceShape& sh, hipStream_t stream, Device
   return KRK_SUCCESS;
 }
 
-// Positions -> rows -> sort_and_reduce fused with the optimizer. d_g holds one gradient row per
-// sort payload (per position, or per bag for pooled pushes). The caller holds the table's lock
-// and has made the optimizer's columns exist.
-static int32_t push_sorted(krk_sparse* t, const krk_optim* o, const uint64_t* d_ids, int64_t n,
-                           const float* d_g, float lr, const uint32_t* bag_of, bool payload_is_bag,
-                           const PooledSrc& ps) {
-  // sort key width: rows are < row_cap; one value above them marks a missing id
-  uint32_t miss_key = 1;
-  int bits = 1;
-  while ((int64_t)miss_key < t->row_cap) {
-    miss_key <<= 1;
-    ++bits;
-  }
+static ApplyArgs table_apply_args(krk_sparse* t, const krk_optim* o, float lr) {
   ApplyArgs args;
   args.lr = lr;
   args.k = make_optim_k(*o);
@@ -1454,14 +1619,47 @@ static int32_t push_sorted(krk_sparse* t, const krk_optim* o, const uint64_t* d_
   args.c1 = cols[1];
   args.c2 = cols[2];
   args.meta_off = ((optim_state_mask(*o) >> KRK_ST_STEPS) & 1u) ? t->meta_off : -1;
-  const TableView tv = t->view();
+  return args;
+}
+
+// Sort key width of a table: rows are < row_cap; one value above them marks a missing id.
+static int key_bits(const krk_sparse* t, uint32_t* miss_key) {
+  uint32_t miss = 1;
+  int bits = 1;
+  while ((int64_t)miss < t->row_cap) {
+    miss <<= 1;
+    ++bits;
+  }
+  *miss_key = miss;
+  return bits;
+}
+
+static SortCall table_sort_call(const krk_sparse* t, int64_t n) {
+  SortCall sc;
+  sc.n_tables = 1;
+  sc.bucket_bits = short_bucket_bits(1);
+  sc.row_bits = 1;
+  while (((int64_t)1 << sc.row_bits) < t->row_cap) ++sc.row_bits;
+  sc.row_mask = 0xFFFFFFFFu;
+  sc.miss_key = kNoRow;
+  sc.noted = 0;
+  sc.row_start[0] = 0;
+  sc.row_start[1] = n;
+  return sc;
+}
+
+// sort_and_reduce fused with the optimizer: fill(keys, payload, miss_key) enqueues what turns the
+// request's ids into rows. d_g holds one gradient row per sort payload (per position, or per bag for
+// pooled pushes). The caller holds the table's lock and has made the optimizer's columns exist.
+template <typename Fill>
+static int32_t push_sorted(krk_sparse* t, const krk_optim* o, int64_t n, const float* d_g, float lr,
+                           const PooledSrc& ps, Fill fill) {
+  uint32_t miss_key;
+  const int bits = key_bits(t, &miss_key);
   const ReduceShape sh{t->dim, t->vec, t->elems, t->group};
-  return sort_and_reduce(sh, t->stream, t->scratch, tv, o->type, n, miss_key, bits, d_g, args, ps, nullptr,
-                         [&](uint32_t* keys, uint32_t* pos) {
-                           hipLaunchKernelGGL(rows_of_ids_kernel, dim3(grid_for(n, kBlock / kBucket)),
-                                              dim3(kBlock), 0, t->stream, tv, d_ids, n, miss_key, bag_of,
-                                              payload_is_bag, keys, pos);
-                         });
+  return sort_and_reduce(sh, t->stream, t->scratch, t->view(), o->type, n, miss_key, bits, d_g,
+                         table_apply_args(t, o, lr), ps, nullptr, nullptr,
+                         [&](uint32_t* keys, uint32_t* pos) { fill(keys, pos, miss_key); });
 }
 
 // stand-alone dedup + sum: (unique index, position) pairs for the sort
@@ -1822,7 +2020,7 @@ int32_t krk_dedup_sum(const uint64_t* ids, int64_t n, const float* grads, int64_
   const DSlot* slots = w.slots;
   const uint32_t* slot_of = w.slot_of;
   KRK_TRY(sort_and_reduce(sh, s, g_dedup_reduce, tv, kOptStore, n, miss_key, bits, d_g, args,
-                          PooledSrc{nullptr, nullptr}, nullptr, [&](uint32_t* keys, uint32_t* pos) {
+                          PooledSrc{nullptr, nullptr, nullptr}, nullptr, nullptr, [&](uint32_t* keys, uint32_t* pos) {
                             hipLaunchKernelGGL(dedup_pairs_kernel, dim3(grid_for(n, kBlock)), dim3(kBlock), 0, s,
                                                slots, slot_of, n, keys, pos);
                           }));
@@ -1920,25 +2118,8 @@ int32_t krk_sparse_push_raw(krk_sparse* t, const krk_optim* o, const uint64_t* i
 
   if (short_push_fits(n, t->dim, t->elems, t->group)) {
     // a short request: see bucket_push_kernel
-    SortCall sc;
-    sc.n_tables = 1;
-    sc.bucket_bits = short_bucket_bits(1);
-    sc.row_bits = 1;
-    while (((int64_t)1 << sc.row_bits) < t->row_cap) ++sc.row_bits;
-    sc.row_mask = 0xFFFFFFFFu;
-    sc.miss_key = kNoRow;
-    sc.noted = 0;
-    sc.row_start[0] = 0;
-    sc.row_start[1] = n;
-    ApplyArgs args;
-    args.lr = lr;
-    args.k = make_optim_k(*o);
-    int32_t cols[3];
-    sparse_optim_columns(t, *o, cols);
-    args.c0 = cols[0];
-    args.c1 = cols[1];
-    args.c2 = cols[2];
-    args.meta_off = ((optim_state_mask(*o) >> KRK_ST_STEPS) & 1u) ? t->meta_off : -1;
+    SortCall sc = table_sort_call(t, n);
+    const ApplyArgs args = table_apply_args(t, o, lr);
     const TableView tv = t->view();
     // KRK_IDS_AS_PULLED: the rows of these very ids were noted by the pull before (and nothing
     // has moved since): the look-up launch is not needed
@@ -1968,42 +2149,49 @@ int32_t krk_sparse_push_raw(krk_sparse* t, const krk_optim* o, const uint64_t* i
     KRK_HIP(hipGetLastError());
     return sparse_finish(t, flags);
   }
-  KRK_TRY(push_sorted(t, o, d_ids, n, d_g, lr, nullptr, false, PooledSrc{nullptr, nullptr}));
+  const uint32_t* notes = noted_rows(t, ids, n, flags);
+  KRK_TRY(push_sorted(t, o, n, d_g, lr, PooledSrc{nullptr, nullptr, nullptr},
+                      [&](uint32_t* keys, uint32_t* pos, uint32_t miss_key) {
+                        if (notes) {
+                          hipLaunchKernelGGL(noted_keys_kernel, dim3(grid_for(n, kBlock)), dim3(kBlock), 0, t->stream,
+                                             t->view(), d_ids, n, notes, miss_key, keys, pos);
+                        } else {
+                          hipLaunchKernelGGL(rows_of_ids_kernel, dim3(grid_for(n, kBlock / kBucket)), dim3(kBlock), 0,
+                                             t->stream, t->view(), d_ids, n, miss_key, (const uint32_t*)nullptr, false,
+                                             keys, pos);
+                        }
+                      }));
   return sparse_finish(t, flags);
 }
 
 }  // extern "C"
 
-// A combined push with repeats whose members' ids and gradient rows lie at parts (device
-// addresses); the caller holds the group's lock and has checked the request. contiguous: the
-// gradient rows are one array, member after member, that starts at parts.rows of the first.
-static int32_t group_push_raw_enqueue(krk_group* g, const krk_optim* o, const int64_t* offsets, int64_t total,
-                                      const GroupCall& call, const GroupParts& parts, bool contiguous, float lr,
-                                      uint32_t flags) {
-  const uint32_t mask = optim_state_mask(*o);
-  for (krk_sparse* t : g->tables) KRK_TRY(sparse_ensure_columns(t, mask));
-  KRK_TRY(group_refresh(g));
-  // sort key: member number above the row number; one value above every key marks a missing id
-  int row_bits = 1;
+// Sort keys of a combined push: the member number above the row number; one value above every
+// key marks a missing id.
+struct GroupKeys {
+  int row_bits;
+  int bits;
+  uint32_t miss_key;
+};
+static int32_t group_keys(krk_group* g, GroupKeys* k) {
+  k->row_bits = 1;
   for (krk_sparse* t : g->tables)
-    while (((int64_t)1 << row_bits) < t->row_cap) ++row_bits;
+    while (((int64_t)1 << k->row_bits) < t->row_cap) ++k->row_bits;
   const int n_tables = (int)g->tables.size();
   int member_bits = 1;
   while ((1 << member_bits) <= n_tables) ++member_bits;
-  if (row_bits + member_bits > 32) {
+  k->bits = k->row_bits + member_bits;
+  if (k->bits > 32) {
     set_error("combined push with repeats: %d tables of up to 2^%d rows do not fit a 32-bit sort key",
-              n_tables, row_bits);
+              n_tables, k->row_bits);
     return KRK_E_CAPACITY;
   }
-  const uint32_t miss_key = (uint32_t)n_tables << row_bits;
-  // members of at most 8192 ids each are sorted one workgroup a member
-  bool by_member = true;
-  int64_t longest = 0;
-  for (int m = 0; m < n_tables; ++m) {
-    by_member = by_member && offsets[m + 1] - offsets[m] <= kSortMax;
-    longest = std::max(longest, offsets[m + 1] - offsets[m]);
-  }
-  // the launch that turns ids into rows gives every member whole workgroups of its own
+  k->miss_key = (uint32_t)n_tables << k->row_bits;
+  return KRK_SUCCESS;
+}
+
+// The launch that turns ids into rows gives every member whole workgroups of its own.
+static GroupCall group_rows_layout(const GroupCall& call, const int64_t* offsets, int n_tables) {
   GroupCall rows_call = call;
   uint32_t blocks = 0;
   bool even = true;
@@ -2015,23 +2203,55 @@ static int32_t group_push_raw_enqueue(krk_group* g, const krk_optim* o, const in
   }
   rows_call.block_start[n_tables] = blocks;
   rows_call.even_blocks = even && blocks > 0 ? blocks / (uint32_t)n_tables : 0u;
+  return rows_call;
+}
+
+static ApplyArgs group_apply_args(const krk_optim* o, float lr) {
   ApplyArgs args;
   args.lr = lr;
   args.k = make_optim_k(*o);
   args.c0 = args.c1 = args.c2 = args.meta_off = -1;     // taken per member from its layout
+  return args;
+}
+
+static GroupSrc group_src(krk_group* g, const krk_optim* o, int row_bits) {
   int32_t st[3];
   optim_state_slots(*o, st);
-  const GroupSrc gs{g->d_descs, row_bits, st[0], st[1], st[2], (int)((mask >> KRK_ST_STEPS) & 1u)};
-  if (by_member && short_push_fits(longest, g->dim, g->elems, g->group)) {
+  return GroupSrc{g->d_descs, row_bits, st[0], st[1], st[2], (int)((optim_state_mask(*o) >> KRK_ST_STEPS) & 1u)};
+}
+
+static SortCall group_sort_call(const GroupKeys& gk, int n_tables, const int64_t* offsets) {
+  SortCall sc;
+  sc.n_tables = n_tables;
+  sc.bucket_bits = short_bucket_bits(n_tables);
+  sc.row_bits = gk.row_bits;
+  sc.row_mask = gk.row_bits >= 32 ? 0xFFFFFFFFu : ((1u << gk.row_bits) - 1u);
+  sc.miss_key = gk.miss_key;
+  sc.noted = 0;
+  for (int m = 0; m <= n_tables; ++m) sc.row_start[m] = offsets[m];
+  return sc;
+}
+
+// A combined push with repeats whose members' ids and gradient rows lie at parts (device
+// addresses); the caller holds the group's lock and has checked the request.
+static int32_t group_push_raw_enqueue(krk_group* g, const krk_optim* o, const int64_t* offsets, int64_t total,
+                                      const GroupCall& call, const GroupParts& parts, float lr, uint32_t flags) {
+  for (krk_sparse* t : g->tables) KRK_TRY(sparse_ensure_columns(t, optim_state_mask(*o)));
+  KRK_TRY(group_refresh(g));
+  GroupKeys gk;
+  KRK_TRY(group_keys(g, &gk));
+  const int n_tables = (int)g->tables.size();
+  const uint32_t miss_key = gk.miss_key;
+  const int row_bits = gk.row_bits;
+  // members of at most 8192 ids each are sorted one workgroup a member
+  int64_t longest = 0;
+  for (int m = 0; m < n_tables; ++m) longest = std::max(longest, offsets[m + 1] - offsets[m]);
+  const GroupCall rows_call = group_rows_layout(call, offsets, n_tables);
+  const ApplyArgs args = group_apply_args(o, lr);
+  const GroupSrc gs = group_src(g, o, row_bits);
+  if (short_push_fits(longest, g->dim, g->elems, g->group)) {
     // short members: see bucket_push_kernel
-    SortCall sc;
-    sc.n_tables = n_tables;
-    sc.bucket_bits = short_bucket_bits(n_tables);
-    sc.row_bits = row_bits;
-    sc.row_mask = row_bits >= 32 ? 0xFFFFFFFFu : ((1u << row_bits) - 1u);
-    sc.miss_key = miss_key;
-    sc.noted = 0;
-    for (int m = 0; m <= n_tables; ++m) sc.row_start[m] = offsets[m];
+    SortCall sc = group_sort_call(gk, n_tables, offsets);
     // KRK_IDS_AS_PULLED: the rows of these very ids were noted by the combined pull before (and
     // nothing has moved since): the look-up launch is not needed. A note is a member's own row
     // number, which is all the bucket kernel reads of a key.
@@ -2041,8 +2261,8 @@ static int32_t group_push_raw_enqueue(krk_group* g, const krk_optim* o, const in
       KRK_TRY(g->scratch[0].reserve((size_t)total * sizeof(uint32_t)));
       uint32_t* found = g->scratch[0].as<uint32_t>();
       hipLaunchKernelGGL(group_rows_of_ids_kernel, dim3(rows_call.block_start[n_tables]), dim3(kBlock), 0,
-                         g->stream, g->d_descs, rows_call, parts, row_bits, miss_key, found,
-                         (uint32_t*)nullptr);
+                         g->stream, g->d_descs, rows_call, parts, row_bits, miss_key, (const uint32_t*)nullptr, 0u,
+                         found, (uint32_t*)nullptr);
       keys = found;
     } else {
       sc.noted = 1;
@@ -2057,23 +2277,96 @@ static int32_t group_push_raw_enqueue(krk_group* g, const krk_optim* o, const in
     KRK_HIP(hipGetLastError());
     return KRK_SUCCESS;
   }
-  const float* d_g = parts.rows[0];
-  if (!contiguous) {
-    KRK_TRY(g->todo.reserve((size_t)total * g->dim * sizeof(float)));
-    float* gathered = g->todo.as<float>();
-    hipLaunchKernelGGL(gather_parts_kernel, dim3(grid_for(total * g->dim, kBlock)), dim3(kBlock), 0, g->stream, call,
-                       parts, (int)g->dim, total * g->dim, gathered);
-    d_g = gathered;
-  }
   TableView none{};
   const ReduceShape sh{g->dim, g->vec, g->elems, g->group};
-  KRK_TRY(sort_and_reduce(sh, g->stream, g->scratch, none, o->type, total, miss_key, row_bits + member_bits,
-                          d_g, args, PooledSrc{nullptr, nullptr}, &gs, [&](uint32_t* keys, uint32_t* pos) {
-                            hipLaunchKernelGGL(group_rows_of_ids_kernel, dim3(rows_call.block_start[n_tables]),
-                                               dim3(kBlock), 0, g->stream, g->d_descs, rows_call, parts,
-                                               row_bits, miss_key, keys, pos);
-                          }));
-  return KRK_SUCCESS;
+  GroupPooledSrc src{};                        // not pooled: a payload is a position of its member
+  src.call.n_tables = n_tables;
+  memcpy(src.call.rows, parts.rows, sizeof(src.call.rows));
+  memcpy(src.call.stride, parts.stride, sizeof(src.call.stride));
+  const uint32_t* notes = noted_rows(g, parts.ids, offsets, flags);
+  return sort_and_reduce(sh, g->stream, g->scratch, none, o->type, total, miss_key, gk.bits, nullptr, args,
+                         PooledSrc{nullptr, nullptr, nullptr}, &gs, &src, [&](uint32_t* keys, uint32_t* pos) {
+                           if (notes) {
+                             hipLaunchKernelGGL(group_noted_keys_kernel, dim3(grid_for(total, kBlock)), dim3(kBlock), 0,
+                                                g->stream, g->d_descs, call, parts, total, row_bits, miss_key, notes,
+                                                keys, pos);
+                           } else {
+                             hipLaunchKernelGGL(group_rows_of_ids_kernel, dim3(rows_call.block_start[n_tables]),
+                                                dim3(kBlock), 0, g->stream, g->d_descs, rows_call, parts, row_bits,
+                                                miss_key, (const uint32_t*)nullptr, 0u, keys, pos);
+                           }
+                         });
+}
+
+// Work space of a pooled push: the bag of every position and, for means, the ratio of every bag.
+struct PooledWork {
+  uint32_t* bag_of;      // null: out of memory
+  float* ratio;          // null: no means
+};
+static PooledWork pooled_work(DeviceBuffer& buffer, int64_t n, int64_t bags, bool mean) {
+  const size_t bag_of_bytes = ((size_t)n * sizeof(uint32_t) + 255) & ~(size_t)255;
+  if (buffer.reserve(bag_of_bytes + (mean ? (size_t)bags * sizeof(float) : 0)) != KRK_SUCCESS)
+    return PooledWork{nullptr, nullptr};
+  return PooledWork{buffer.as<uint32_t>(), mean ? reinterpret_cast<float*>(buffer.as<char>() + bag_of_bytes) : nullptr};
+}
+
+// A pooled push on one table, which `call` describes as its only member (device addresses). The caller
+// holds the table's lock and has made the optimizer's columns exist.
+static int32_t push_pooled_enqueue(krk_sparse* t, const krk_optim* o, PooledCall& call, const uint32_t* notes,
+                                   float lr) {
+  const int64_t n = call.row_start[1], bags = call.bag_start[1];
+  const bool mean = call.mean_bits != 0, weighted = call.weights[0] != nullptr;
+  const int64_t blocks = pooled_layout(&call, kBlock / kBagLanes);
+  if (blocks < 0) {
+    set_error("pooled push: too many bags for one launch; split the request");
+    return KRK_E_CAPACITY;
+  }
+  const PooledWork w = pooled_work(t->scratch[5], n, bags, mean);
+  if (!w.bag_of) return KRK_E_DEVICE;
+  const TableView tv = t->view();
+  auto fill = [&](uint32_t* keys, uint32_t* pos, uint32_t miss_key) {
+    if (notes) {
+      hipLaunchKernelGGL((bag_expand_kernel<false, true>), dim3((unsigned)blocks), dim3(kBlock), 0, t->stream, nullptr,
+                         tv, call, 0, miss_key, notes, w.bag_of, w.ratio, keys, pos);
+    } else {
+      hipLaunchKernelGGL((bag_expand_kernel<false, false>), dim3((unsigned)blocks), dim3(kBlock), 0, t->stream, nullptr,
+                         tv, call, 0, miss_key, (const uint32_t*)nullptr, w.bag_of, w.ratio, (uint32_t*)nullptr,
+                         (uint32_t*)nullptr);
+      // Unweighted: the sort carries bag numbers and the reduction reads bag rows directly.
+      // Weighted: it carries positions, which name the weight and (through bag_of) the bag.
+      hipLaunchKernelGGL(rows_of_ids_kernel, dim3(grid_for(n, kBlock / kBucket)), dim3(kBlock), 0, t->stream, tv,
+                         call.ids[0], n, miss_key, (const uint32_t*)w.bag_of, !weighted, keys, pos);
+    }
+  };
+  if (short_push_fits(n, t->dim, t->elems, t->group) && bags <= kBucketMaxBags) {
+    KRK_TRY(t->scratch[0].reserve((size_t)n * sizeof(uint32_t)));
+    uint32_t* keys = t->scratch[0].as<uint32_t>();
+    fill(keys, nullptr, kNoRow);
+    const SortCall sc = table_sort_call(t, n);
+    GroupParts parts;
+    parts.ids[0] = call.ids[0];
+    parts.rows[0] = call.rows[0];
+    parts.stride[0] = call.stride[0];
+    BucketPooled pool;
+    pool.bag_of = w.bag_of;
+    pool.ratio = w.ratio;
+    pool.mean_bits = call.mean_bits;
+    pool.bag_start[0] = 0;
+    pool.weights[0] = call.weights[0];
+    const GroupSrc none{nullptr, 0, -1, -1, -1, 0};
+    const ApplyArgs args = table_apply_args(t, o, lr);
+    if (t->vec == 4) {
+      launch_bucket_push<4, false>(o->type, 1u << sc.bucket_bits, t->stream, nullptr, tv, sc, parts, keys, (int)t->dim,
+                                   t->elems, t->group, args, none, &pool);
+    } else {
+      launch_bucket_push<1, false>(o->type, 1u << sc.bucket_bits, t->stream, nullptr, tv, sc, parts, keys, (int)t->dim,
+                                   t->elems, t->group, args, none, &pool);
+    }
+    KRK_HIP(hipGetLastError());
+    return KRK_SUCCESS;
+  }
+  return push_sorted(t, o, n, call.rows[0], lr,
+                     PooledSrc{weighted ? w.bag_of : nullptr, weighted ? call.weights[0] : nullptr, w.ratio}, fill);
 }
 
 extern "C" {
@@ -2112,7 +2405,7 @@ int32_t krk_group_push_raw(krk_group* g, const krk_optim* o, const uint64_t* ids
     parts.rows[m] = const_cast<float*>(d_g) + offsets[m] * g->dim;
     parts.stride[m] = (uint32_t)g->dim;
   }
-  KRK_TRY(group_push_raw_enqueue(g, o, offsets, total, call, parts, true, lr, flags));
+  KRK_TRY(group_push_raw_enqueue(g, o, offsets, total, call, parts, lr, flags));
   return group_finish(g, flags);
 }
 
@@ -2142,7 +2435,7 @@ int32_t krk_group_push_raw_parts(krk_group* g, const krk_optim* o, const krk_par
               (long long)g->dim);
     return KRK_GRADIENT_UNCOMPATIBLE;
   }
-  KRK_TRY(group_push_raw_enqueue(g, o, offsets, total, call, parts, false, lr, flags));
+  KRK_TRY(group_push_raw_enqueue(g, o, offsets, total, call, parts, lr, flags));
   return group_finish(g, flags);
 }
 
@@ -2189,24 +2482,122 @@ int32_t krk_sparse_push_pooled(krk_sparse* t, const krk_optim* o, const uint64_t
   if (weights) KRK_TRY(t->input(weights, (size_t)n, flags, 2, &d_w));
   KRK_TRY(t->input(bag_grads, (size_t)bags * t->dim, flags, 3, &d_g));
 
-  const size_t bag_of_bytes = ((size_t)n * sizeof(uint32_t) + 255) & ~(size_t)255;
-  const size_t scaled_bytes = mode == KRK_POOL_MEAN ? (size_t)bags * t->dim * sizeof(float) : 0;
-  KRK_TRY(t->scratch[5].reserve(bag_of_bytes + scaled_bytes));
-  uint32_t* bag_of = t->scratch[5].as<uint32_t>();
-  hipLaunchKernelGGL(fill_u32_kernel, dim3(grid_for(n, kBlock)), dim3(kBlock), 0, t->stream, bag_of, n, kNoBag);
-  hipLaunchKernelGGL(bag_expand_kernel, dim3(grid_for(bags, kBlock / kBagLanes)), dim3(kBlock), 0, t->stream,
-                     d_off, bags, n, bag_of);
-  if (mode == KRK_POOL_MEAN) {
-    float* scaled = reinterpret_cast<float*>(t->scratch[5].as<char>() + bag_of_bytes);
-    hipLaunchKernelGGL(bag_scale_kernel, dim3(grid_for(bags * t->dim, kBlock)), dim3(kBlock), 0, t->stream,
-                       d_g, d_off, bags, (int)t->dim, scaled);
-    d_g = scaled;
-  }
-  KRK_HIP(hipGetLastError());
-  // Unweighted: the sort carries bag numbers and the reduction reads bag rows directly.
-  // Weighted: it carries positions, which name the weight and (through bag_of) the bag.
-  KRK_TRY(push_sorted(t, o, d_ids, n, d_g, lr, bag_of, d_w == nullptr, PooledSrc{d_w ? bag_of : nullptr, d_w}));
+  // one member that begins at zero
+  PooledCall call{};
+  call.n_tables = 1;
+  call.bag_start[1] = bags;
+  call.row_start[1] = n;
+  call.ids[0] = d_ids;
+  call.offsets[0] = d_off;
+  call.weights[0] = d_w;
+  call.rows[0] = const_cast<float*>(d_g);
+  call.stride[0] = (uint32_t)t->dim;
+  call.mean_bits = mode == KRK_POOL_MEAN ? 1u : 0u;
+  KRK_TRY(push_pooled_enqueue(t, o, call, noted_rows(t, ids, n, flags), lr));
   return sparse_finish(t, flags);
 }
 
 }  // extern "C"
+
+int32_t krk_group_push_pooled_parts(krk_group* g, const krk_optim* o, const krk_pooled_part* in, int64_t grad_dim,
+                                    float lr, uint32_t flags) {
+  if (!g || !in || !(flags & KRK_DEVICE_PTRS)) return KRK_E_ARGUMENT;
+  KRK_TRY(ensure_runtime());
+  KRK_TRY(check_flags(flags));
+  if (!o || o->type < KRK_ADAGRAD || o->type > KRK_SGD) {
+    set_error("optimizer type is not supported");
+    return KRK_UNSUPPORTED_OPTIM;
+  }
+  GroupLock lk(g);
+  PooledCall call;
+  KRK_TRY(pooled_parts(g, in, true, &call));
+  const int n_tables = call.n_tables;
+  const int64_t total = call.row_start[n_tables], bags = call.bag_start[n_tables];
+  if (total == 0) return group_finish(g, flags);
+  if (grad_dim != g->dim) {
+    set_error("gradient width %lld does not match table dimension %lld", (long long)grad_dim,
+              (long long)g->dim);
+    return KRK_GRADIENT_UNCOMPATIBLE;
+  }
+  if (total > ((int64_t)1 << 28) || bags > ((int64_t)1 << 28)) {
+    set_error("krk_group_push_pooled_parts handles at most 2^28 ids and bags per call; split the request");
+    return KRK_E_CAPACITY;
+  }
+  GroupKeys gk;
+  KRK_TRY(group_keys(g, &gk));
+  for (int m = 0; m < n_tables; ++m)
+    if (call.row_start[m + 1] > call.row_start[m]) KRK_TRY(sparse_ensure_columns(g->tables[m], optim_state_mask(*o)));
+  KRK_TRY(group_refresh(g));
+  const int64_t blocks = pooled_layout(&call, kBlock / kBagLanes);
+  if (blocks < 0) {
+    set_error("combined request too large for one launch; split it");
+    return KRK_E_CAPACITY;
+  }
+  const uint32_t* notes = noted_rows(g, call.ids, call.row_start, flags);
+  int64_t longest = 0, most_bags = 0;
+  uint32_t bag_payload = 0;
+  bool weighted = false;
+  for (int m = 0; m < n_tables; ++m) {
+    longest = std::max(longest, call.row_start[m + 1] - call.row_start[m]);
+    most_bags = std::max(most_bags, call.bag_start[m + 1] - call.bag_start[m]);
+    if (!call.weights[m]) bag_payload |= 1u << m;
+    weighted = weighted || (call.weights[m] && call.row_start[m + 1] > call.row_start[m]);
+  }
+  const PooledWork w = pooled_work(g->todo, total, bags, call.mean_bits != 0);
+  if (!w.bag_of) return KRK_E_DEVICE;
+  const ApplyArgs args = group_apply_args(o, lr);
+  const GroupSrc gs = group_src(g, o, gk.row_bits);
+  GroupParts parts;
+  memcpy(parts.ids, call.ids, sizeof(parts.ids));
+  memcpy(parts.rows, call.rows, sizeof(parts.rows));
+  memcpy(parts.stride, call.stride, sizeof(parts.stride));
+  const GroupCall rows_call = [&] {
+    GroupCall c{};
+    c.n_tables = n_tables;
+    memcpy(c.row_start, call.row_start, sizeof(c.row_start));
+    return group_rows_layout(c, call.row_start, n_tables);
+  }();
+  auto fill = [&](uint32_t* keys, uint32_t* pos) {
+    if (notes) {
+      hipLaunchKernelGGL((bag_expand_kernel<true, true>), dim3((unsigned)blocks), dim3(kBlock), 0, g->stream, g->d_descs,
+                         TableView{}, call, gk.row_bits, gk.miss_key, notes, w.bag_of, w.ratio, keys, pos);
+    } else {
+      hipLaunchKernelGGL((bag_expand_kernel<true, false>), dim3((unsigned)blocks), dim3(kBlock), 0, g->stream,
+                         g->d_descs, TableView{}, call, gk.row_bits, gk.miss_key, (const uint32_t*)nullptr, w.bag_of,
+                         w.ratio, (uint32_t*)nullptr, (uint32_t*)nullptr);
+      hipLaunchKernelGGL(group_rows_of_ids_kernel, dim3(rows_call.block_start[n_tables]), dim3(kBlock), 0, g->stream,
+                         g->d_descs, rows_call, parts, gk.row_bits, gk.miss_key, (const uint32_t*)w.bag_of, bag_payload,
+                         keys, pos);
+    }
+  };
+  if (short_push_fits(longest, g->dim, g->elems, g->group) && most_bags <= kBucketMaxBags) {
+    KRK_TRY(g->scratch[0].reserve((size_t)total * sizeof(uint32_t)));
+    uint32_t* keys = g->scratch[0].as<uint32_t>();
+    fill(keys, nullptr);
+    const SortCall sc = group_sort_call(gk, n_tables, call.row_start);
+    BucketPooled pool;
+    pool.bag_of = w.bag_of;
+    pool.ratio = w.ratio;
+    pool.mean_bits = call.mean_bits;
+    memcpy(pool.bag_start, call.bag_start, sizeof(pool.bag_start));
+    memcpy(pool.weights, call.weights, sizeof(pool.weights));
+    if (g->vec == 4) {
+      launch_bucket_push<4, true>(o->type, (unsigned)n_tables << sc.bucket_bits, g->stream, g->d_descs, TableView{}, sc,
+                                  parts, keys, (int)g->dim, g->elems, g->group, args, gs, &pool);
+    } else {
+      launch_bucket_push<1, true>(o->type, (unsigned)n_tables << sc.bucket_bits, g->stream, g->d_descs, TableView{}, sc,
+                                  parts, keys, (int)g->dim, g->elems, g->group, args, gs, &pool);
+    }
+    KRK_HIP(hipGetLastError());
+    return group_finish(g, flags);
+  }
+  GroupPooledSrc src;
+  src.call = call;
+  src.bag_of = w.bag_of;
+  src.ratio = w.ratio;
+  src.weighted = weighted ? 1 : 0;
+  const ReduceShape sh{g->dim, g->vec, g->elems, g->group};
+  KRK_TRY(sort_and_reduce(sh, g->stream, g->scratch, TableView{}, o->type, total, gk.miss_key, gk.bits, nullptr, args,
+                          PooledSrc{nullptr, nullptr, nullptr}, &gs, &src, fill));
+  return group_finish(g, flags);
+}

@@ -371,12 +371,6 @@ __device__ inline uint32_t probe_find_alone(const TableView& tv, uint64_t id) {
 
 struct krk_group;
 
-namespace krk {
-// Requests of at most this many ids a table keep row notes (KRK_NOTE_ROWS): the pulls that run
-// as one launch.
-constexpr int64_t kNotedMax = (1 << 18) - 1;
-}  // namespace krk
-
 // The handle behind krk_sparse*.
 struct krk_sparse : krk::ObjBase {
   int64_t dim = 0;
@@ -469,6 +463,24 @@ struct GroupParts {
   uint32_t stride[kMaxGroupTables];
 };
 
+// A pooled request of one or several tables: where each member's positions and bags begin in the
+// request, and where its arrays lie. `block_start` lays the bags out over the grid, as in GroupCall
+// (how many bags a workgroup takes is the launch's own affair).
+struct PooledCall {
+  int32_t n_tables;
+  uint32_t even_blocks;
+  uint32_t mean_bits;                     // bit m: member m's bags are means
+  uint32_t block_start[kMaxGroupTables + 1];
+  int64_t bag_start[kMaxGroupTables + 1];
+  int64_t row_start[kMaxGroupTables + 1];
+  const uint64_t* ids[kMaxGroupTables];
+  const long long* offsets[kMaxGroupTables];
+  const float* weights[kMaxGroupTables];  // null: every position weighs 1
+  float* rows[kMaxGroupTables];           // the pooled rows of a pull, the bags' gradient rows of a push
+  uint32_t stride[kMaxGroupTables];       // floats between two of them
+  float patch[kMaxGroupTables];           // what an empty bag of a pull yields
+};
+
 // What a combined pull carries besides when it queues its missing ids (the members' tables are
 // being filled): every member has its own 64 lists, counted by its own table's list counters.
 struct GroupFill {
@@ -536,6 +548,12 @@ struct GroupLock {
 int32_t group_plan(krk_group* g, const int64_t* offsets, GroupCall* call, int64_t* total, int per_block = 0);
 // Checks a request of one part per member and lists its sizes (offsets[members + 1]) and addresses.
 int32_t group_parts(krk_group* g, const krk_part* in, bool push, int64_t* offsets, GroupParts* parts);
+// Checks a pooled request of one part per member and takes it over; the bags are not laid out yet.
+// push: rows are gradients, `stride` floats apart.
+int32_t pooled_parts(krk_group* g, const krk_pooled_part* in, bool push, PooledCall* call);
+// Lays the bags out over the grid, per_block to a workgroup. Returns the number of workgroups, or -1
+// where one launch cannot hold them.
+int64_t pooled_layout(PooledCall* call, int per_block);
 // Uploads the layouts of members that moved since the last call.
 int32_t group_refresh(krk_group* g);
 // Blocking calls: waits for the group's stream and reports the first member's error.

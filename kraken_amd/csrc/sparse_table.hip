@@ -502,11 +502,12 @@ __global__ __launch_bounds__(kMissBlock) void pull_missing_kernel(TableView tv, 
 // ---------------------------------------------------------------------------
 // The first launch while the table is being filled: positions are only looked up, the ones whose
 // id is missing are queued as in pull_resident_kernel and inserted by pull_missing_kernel.
-__global__ __launch_bounds__(kBlock) void pooled_find_kernel(TableView tv, const uint64_t* __restrict__ ids,
-                                                             int64_t n, uint32_t* __restrict__ rows,
-                                                             uint32_t* __restrict__ todo, int parity) {
+// p: the position in the member's request; n: how many it has; bx: the workgroup's number among
+// the member's.
+__device__ __forceinline__ void pooled_find_body(const TableView& tv, const uint64_t* __restrict__ ids, int64_t p,
+                                                 int64_t n, uint32_t bx, uint32_t* __restrict__ rows,
+                                                 uint32_t* __restrict__ todo, int parity) {
   constexpr int per_block = kBlock / kBucket;
-  const int64_t p = (int64_t)blockIdx.x * per_block + threadIdx.x / kBucket;
   const int gl = threadIdx.x & (kBucket - 1);
   const bool active = p < n;
   const uint32_t row = probe_find(tv, active ? ids[p] : 0, active, gl, kBucket);
@@ -515,7 +516,7 @@ __global__ __launch_bounds__(kBlock) void pooled_find_kernel(TableView tv, const
   if (votes) {
     const int lane = wave_lane();
     const int first = __ffsll(votes) - 1;
-    const int q = blockIdx.x & (kQueues - 1);
+    const int q = bx & (kQueues - 1);
     uint32_t base = 0;
     if (lane == first) base = atomicAdd(queue_counter(tv, parity, q), (uint32_t)__popcll(votes));
     base = __shfl(base, first);
@@ -526,16 +527,22 @@ __global__ __launch_bounds__(kBlock) void pooled_find_kernel(TableView tv, const
   if (active && gl == 0) rows[p] = row;
 }
 
-template <int VEC>
-__global__ __launch_bounds__(kBlock) void pooled_probe_kernel(TableView tv, InitK init,
-                                                              const uint64_t* __restrict__ ids, int64_t n,
-                                                              uint32_t* __restrict__ rows, int elems) {
+__global__ __launch_bounds__(kBlock) void pooled_find_kernel(TableView tv, const uint64_t* __restrict__ ids,
+                                                             int64_t n, uint32_t* __restrict__ rows,
+                                                             uint32_t* __restrict__ todo, int parity) {
   const int64_t p = (int64_t)blockIdx.x * (kBlock / kBucket) + threadIdx.x / kBucket;
+  pooled_find_body(tv, ids, p, n, blockIdx.x, rows, todo, parity);
+}
+
+template <int VEC>
+__device__ __forceinline__ void pooled_probe_body(const TableView& tv, const InitK& init,
+                                                  const uint64_t* __restrict__ ids, int64_t p, int64_t n,
+                                                  uint32_t* __restrict__ rows, int elems, int filling_ids) {
   const int gl = threadIdx.x & (kBucket - 1);
   const bool active = p < n;
   const uint64_t id = active ? ids[p] : 0;
   const ProbeResult pr = probe_insert(tv, id, active, gl, kBucket);
-  if (__popcll(__ballot(active && pr.owner && gl == 0)) >= kFillingIds && wave_lane() == 0) note_inserting(tv);
+  if (__popcll(__ballot(active && pr.owner && gl == 0)) >= filling_ids && wave_lane() == 0) note_inserting(tv);
   if (!active) return;
   if (pr.fresh && pr.owner && pr.row != kEmptyRow) {
     float* rec = tv.recs + (int64_t)pr.row * tv.stride;
@@ -548,19 +555,22 @@ __global__ __launch_bounds__(kBlock) void pooled_probe_kernel(TableView tv, Init
   if (gl == 0) rows[p] = pr.row;
 }
 
+template <int VEC>
+__global__ __launch_bounds__(kBlock) void pooled_probe_kernel(TableView tv, InitK init,
+                                                              const uint64_t* __restrict__ ids, int64_t n,
+                                                              uint32_t* __restrict__ rows, int elems) {
+  const int64_t p = (int64_t)blockIdx.x * (kBlock / kBucket) + threadIdx.x / kBucket;
+  pooled_probe_body<VEC>(tv, init, ids, p, n, rows, elems, kFillingIds);
+}
+
 constexpr int kPoolAhead = 4;   // records of one bag requested together
 
 template <int VEC>
-__global__ __launch_bounds__(kBlock) void pooled_sum_kernel(TableView tv, const uint32_t* __restrict__ rows,
-                                                            const uint64_t* __restrict__ ids,
-                                                            int64_t n, const long long* __restrict__ offsets,
-                                                            int64_t bags, const float* __restrict__ weights,
-                                                            int mean, float patch, float* __restrict__ out,
-                                                            int dim, int elems, int group) {
-  const int per_block = kBlock / group;
-  const int64_t bag = (int64_t)blockIdx.x * per_block + threadIdx.x / group;
-  const int gl = threadIdx.x & (group - 1);
-  if (bag >= bags || gl >= elems) return;      // the host only launches this with elems <= group
+__device__ __forceinline__ void pooled_sum_body(const TableView& tv, const uint32_t* __restrict__ rows,
+                                                const uint64_t* __restrict__ ids, int64_t n,
+                                                const long long* __restrict__ offsets, int64_t bag,
+                                                const float* __restrict__ weights, int mean, float patch,
+                                                float* __restrict__ out, int dim, int gl) {
   long long lo = offsets[bag], hi = offsets[bag + 1];
   if (lo < 0) lo = 0;
   if (hi > n) hi = n;
@@ -603,6 +613,20 @@ __global__ __launch_bounds__(kBlock) void pooled_sum_kernel(TableView tv, const 
     for (int c = 0; c < VEC; ++c) acc[c] = acc[c] * ratio;
   }
   vstore_once<VEC>(out + bag * (int64_t)dim + gl * VEC, acc);
+}
+
+template <int VEC>
+__global__ __launch_bounds__(kBlock) void pooled_sum_kernel(TableView tv, const uint32_t* __restrict__ rows,
+                                                            const uint64_t* __restrict__ ids,
+                                                            int64_t n, const long long* __restrict__ offsets,
+                                                            int64_t bags, const float* __restrict__ weights,
+                                                            int mean, float patch, float* __restrict__ out,
+                                                            int dim, int elems, int group) {
+  const int per_block = kBlock / group;
+  const int64_t bag = (int64_t)blockIdx.x * per_block + threadIdx.x / group;
+  const int gl = threadIdx.x & (group - 1);
+  if (bag >= bags || gl >= elems) return;      // the host only launches this with elems <= group
+  pooled_sum_body<VEC>(tv, rows, ids, n, offsets, bag, weights, mean, patch, out, dim, gl);
 }
 
 template <int OPT, int VEC>
@@ -929,7 +953,8 @@ __global__ __launch_bounds__(kBlock) void group_pull_resident_wide_kernel(const 
                                notes ? notes + a : nullptr);
 }
 
-template <int VEC>
+// ROWS_ONLY: as in pull_missing_kernel; `notes` then receives the rows of the queued positions.
+template <int VEC, bool ROWS_ONLY = false>
 __global__ __launch_bounds__(kMissBlock) void group_pull_missing_kernel(const TableDesc* __restrict__ descs,
                                                                         GroupCall call, GroupParts parts,
                                                                         GroupFill fill,
@@ -968,8 +993,56 @@ __global__ __launch_bounds__(kMissBlock) void group_pull_missing_kernel(const Ta
     for (int i = 0; i + 1 < kMine; ++i) j += k >= upto[i] ? 1 : 0;
     return lists[(int64_t)(w + j * kGroupMissPerTable) * capacity + (k - (j ? upto[j - 1] : 0u))];
   };
-  insert_queued<VEC, kInsertAndCopy>(tv, init, parts.ids[t], parts.rows[t], position_of, total, 0u, kMissEntries, dim,
-                                     elems, group, notes ? notes + a : nullptr);
+  insert_queued<VEC, ROWS_ONLY ? kInsertOnly : kInsertAndCopy>(tv, init, parts.ids[t], parts.rows[t], position_of,
+                                                               total, 0u, kMissEntries, dim, elems, group,
+                                                               notes ? notes + a : nullptr);
+}
+
+// ---- pooled pulls of several tables ---------------------------------------------------------------
+// The two launches of a pooled pull with every member's positions (bags) side by side. A request of
+// 26 fields of 2048 bags is 26 x 10k positions: a table at a time its launches leave three quarters
+// of the chip idle and cost the host two launches each (26 tables of dim 16: 340 us a pull that way).
+template <int VEC>
+__global__ __launch_bounds__(kBlock) void group_pooled_probe_kernel(const TableDesc* __restrict__ descs,
+                                                                    GroupCall call, GroupParts parts,
+                                                                    uint32_t* __restrict__ rows, int elems) {
+  const int t = find_table(call);
+  TableView tv = descs[t].tv;
+  tv.epoch = call.epoch[t];
+  const InitK init = descs[t].init;
+  const int64_t p = (int64_t)(blockIdx.x - call.block_start[t]) * (kBlock / kBucket) + threadIdx.x / kBucket;
+  const int64_t a = call.row_start[t];
+  pooled_probe_body<VEC>(tv, init, parts.ids[t], p, call.row_start[t + 1] - a, rows + a, elems, kFillingIdsCombined);
+}
+
+__global__ __launch_bounds__(kBlock) void group_pooled_find_kernel(const TableDesc* __restrict__ descs,
+                                                                   GroupCall call, GroupParts parts, GroupFill fill,
+                                                                   uint32_t* __restrict__ rows,
+                                                                   uint32_t* __restrict__ todo) {
+  const int t = find_table(call);
+  const uint32_t bx = blockIdx.x - call.block_start[t];
+  const int64_t p = (int64_t)bx * (kBlock / kBucket) + threadIdx.x / kBucket;
+  const int64_t a = call.row_start[t];
+  pooled_find_body(descs[t].tv, parts.ids[t], p, call.row_start[t + 1] - a, bx, rows + a, todo + fill.todo_start[t],
+                   (int)((fill.parity_bits >> t) & 1u));
+}
+
+template <int VEC>
+__global__ __launch_bounds__(kBlock) void group_pooled_sum_kernel(const TableDesc* __restrict__ descs, PooledCall call,
+                                                                  const uint32_t* __restrict__ rows, int dim,
+                                                                  int elems, int group) {
+  int m = 0;
+  if (call.even_blocks) {
+    m = (int)(blockIdx.x / call.even_blocks);
+  } else {
+    while (m + 1 < call.n_tables && blockIdx.x >= call.block_start[m + 1]) ++m;
+  }
+  const int64_t bag = (int64_t)(blockIdx.x - call.block_start[m]) * (kBlock / group) + threadIdx.x / group;
+  const int gl = threadIdx.x & (group - 1);
+  if (bag >= call.bag_start[m + 1] - call.bag_start[m] || gl >= elems) return;
+  const int64_t a = call.row_start[m];
+  pooled_sum_body<VEC>(descs[m].tv, rows + a, call.ids[m], call.row_start[m + 1] - a, call.offsets[m], bag,
+                       call.weights[m], (int)((call.mean_bits >> m) & 1u), call.patch[m], call.rows[m], dim, gl);
 }
 
 template <int OPT, int VEC>
@@ -2019,11 +2092,11 @@ int32_t krk_sparse_pull(krk_sparse* t, const uint64_t* ids, int64_t n, float* ou
   float* d_out;
   KRK_TRY(t->input(ids, (size_t)n, flags, 0, &d_ids));
   KRK_TRY(t->output(out, (size_t)n * t->dim, flags, 1, &d_out));
-  // KRK_NOTE_ROWS: requests served by one launch leave the row of every position behind
+  // KRK_NOTE_ROWS: the row of every position stays behind
   uint32_t* notes = nullptr;
   if (flags & KRK_NOTE_ROWS) {
     t->noted_ids = nullptr;
-    if ((flags & KRK_DEVICE_PTRS) && n <= kNotedMax) {
+    if (flags & KRK_DEVICE_PTRS) {
       KRK_TRY(t->notes.reserve((size_t)n * sizeof(uint32_t)));
       notes = t->notes.as<uint32_t>();
     }
@@ -2087,6 +2160,16 @@ int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, co
   KRK_TRY(t->scratch[5].reserve((rows_words + (size_t)kQueues * (size_t)list_capacity) * sizeof(uint32_t)));
   uint32_t* rows = t->scratch[5].as<uint32_t>();
   uint32_t* todo = rows + rows_words;
+  // KRK_NOTE_ROWS: the rows of the positions, which the second launch reads, stay behind
+  bool noting = false;
+  if (flags & KRK_NOTE_ROWS) {
+    t->noted_ids = nullptr;
+    noting = (flags & KRK_DEVICE_PTRS) && n > 0;
+    if (noting) {
+      KRK_TRY(t->notes.reserve((size_t)n * sizeof(uint32_t)));
+      rows = t->notes.as<uint32_t>();
+    }
+  }
   const int per_block = kBlock / t->group;
   const dim3 probe_grid(grid_for(n, kBlock / kBucket)), grid(grid_for(bags, per_block)), block(kBlock);
   const dim3 small(kMissingGrid), missing_block(kMissBlock);
@@ -2117,6 +2200,11 @@ int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, co
                        mean, patch_value, d_out, (int)t->dim, t->elems, t->group);
   }
   KRK_HIP(hipGetLastError());
+  if (noting) {
+    t->noted_ids = ids;
+    t->noted_n = n;
+    t->noted_version = t->layout_version;
+  }
   if ((flags & KRK_ASYNC) && sparse_near_full(t)) KRK_TRY(sparse_publish(&t, 1, t->stream));
   KRK_TRY(t->output_back(out, (size_t)bags * t->dim, flags, 3));
   return sparse_finish(t, flags);
@@ -3081,6 +3169,168 @@ int32_t krk_group_pull_parts(krk_group* g, const krk_part* in, uint32_t flags) {
   KRK_TRY(group_plan(g, offsets, &call, &total, wide ? (group_wide_block(g->group) / kWave) * kWideIds : 0));
   if (total == 0) return group_finish(g, flags);
   KRK_TRY(group_pull_enqueue(g, offsets, call, total, wide, parts, flags));
+  return group_finish(g, flags);
+}
+
+}  // extern "C"
+
+int64_t krk::pooled_layout(PooledCall* call, int per_block) {
+  const int n = call->n_tables;
+  uint64_t blocks = 0, widest = 0;
+  for (int m = 0; m < n; ++m) {
+    const uint64_t mine = (uint64_t)((call->bag_start[m + 1] - call->bag_start[m] + per_block - 1) / per_block);
+    call->block_start[m] = (uint32_t)blocks;
+    blocks += mine;
+    if (mine > widest) widest = mine;
+  }
+  // members of similar size: the same number of workgroups each, as in group_plan
+  call->even_blocks = 0;
+  if (widest > 0 && widest * (uint64_t)n <= blocks + blocks / 4 + (uint64_t)n) {
+    call->even_blocks = (uint32_t)widest;
+    for (int m = 0; m < n; ++m) call->block_start[m] = (uint32_t)(widest * (uint64_t)m);
+    blocks = widest * (uint64_t)n;
+  }
+  if (blocks * (uint64_t)kBlock >= 0x7FFFFFFFull) return -1;
+  call->block_start[n] = (uint32_t)blocks;
+  return (int64_t)blocks;
+}
+
+int32_t krk::pooled_parts(krk_group* g, const krk_pooled_part* in, bool push, PooledCall* call) {
+  const int n = (int)g->tables.size();
+  memset(call, 0, sizeof(*call));
+  call->n_tables = n;
+  for (int m = 0; m < n; ++m) {
+    const krk_pooled_part& p = in[m];
+    if (p.n < 0 || p.bags < 0 || (p.mode != KRK_POOL_SUM && p.mode != KRK_POOL_MEAN) ||
+        (p.bags > 0 && (!p.offsets || !p.rows)) || (p.n > 0 && !p.ids))
+      return KRK_E_ARGUMENT;
+    // a push leaves a member without ids or without bags alone
+    const bool live = push ? p.n > 0 && p.bags > 0 : p.bags > 0;
+    call->bag_start[m + 1] = call->bag_start[m] + (live ? p.bags : 0);
+    call->row_start[m + 1] = call->row_start[m] + (live ? p.n : 0);
+    call->ids[m] = p.ids;
+    call->offsets[m] = reinterpret_cast<const long long*>(p.offsets);
+    call->weights[m] = p.weights;
+    call->rows[m] = p.rows;
+    call->stride[m] = (uint32_t)g->dim;
+    call->patch[m] = p.patch_value;
+    if (p.mode == KRK_POOL_MEAN) call->mean_bits |= 1u << m;
+    if (!live) continue;
+    if (push) {
+      if (p.stride < 0 || p.stride > (int64_t)1 << 30 || (g->vec == 4 && p.stride % 4 != 0)) {
+        set_error("a part's gradient rows must lie a whole number of 16-byte vectors apart");
+        return KRK_E_ARGUMENT;
+      }
+      call->stride[m] = (uint32_t)p.stride;
+    }
+    if (g->vec == 4 && !aligned16(p.rows)) {
+      set_error("a part's rows must be 16-byte aligned");
+      return KRK_E_ARGUMENT;
+    }
+  }
+  return KRK_SUCCESS;
+}
+
+extern "C" {
+
+int32_t krk_group_pull_pooled_parts(krk_group* g, const krk_pooled_part* in, uint32_t flags) {
+  if (!g || !in || !(flags & KRK_DEVICE_PTRS)) return KRK_E_ARGUMENT;
+  KRK_TRY(ensure_runtime());
+  KRK_TRY(check_flags(flags));
+  if (g->elems > g->group) {
+    set_error("pooled pull supports rows of at most %d floats for this layout", 64 * g->vec);
+    return KRK_INTERFACE_UNIMPLEMENTED;
+  }
+  GroupLock lk(g);
+  PooledCall pool;
+  KRK_TRY(pooled_parts(g, in, false, &pool));
+  const int n_tables = pool.n_tables;
+  if (pool.bag_start[n_tables] == 0) return group_finish(g, flags);
+  const int64_t total = pool.row_start[n_tables];
+  const int64_t sum_blocks = pooled_layout(&pool, kBlock / g->group);
+  if (sum_blocks < 0) {
+    set_error("combined request too large for one launch; split it");
+    return KRK_E_CAPACITY;
+  }
+  GroupCall call;
+  GroupParts parts{};
+  memcpy(parts.ids, pool.ids, sizeof(parts.ids));
+  int64_t checked = 0;
+  constexpr int per_block = kBlock / kBucket;
+  KRK_TRY(group_plan(g, pool.row_start, &call, &checked, per_block));
+  for (int m = 0; m < n_tables; ++m) {
+    krk_sparse* t = g->tables[m];
+    const int64_t cnt = pool.row_start[m + 1] - pool.row_start[m];
+    if (cnt > 0) {
+      KRK_TRY(sparse_ensure_room(t, cnt));
+      KRK_TRY(sparse_next_epoch(t, cnt));
+    }
+    call.epoch[m] = t->epoch;
+  }
+  KRK_TRY(group_refresh(g));
+  // the row of every position, in the notes where they are to stay behind
+  const size_t rows_words = ((size_t)(total > 0 ? total : 1) + 63) & ~(size_t)63;
+  DeviceBuffer& row_buffer = (flags & KRK_NOTE_ROWS) ? g->notes : g->scratch[0];
+  if (flags & KRK_NOTE_ROWS) g->noted_ids.clear();
+  KRK_TRY(row_buffer.reserve(rows_words * sizeof(uint32_t)));
+  uint32_t* rows = row_buffer.as<uint32_t>();
+  const dim3 probe_grid(call.block_start[n_tables]), block(kBlock);
+  bool filling = false;
+  for (krk_sparse* t : g->tables)
+    if (t->host_inserted && __atomic_exchange_n(t->host_inserted, 0u, __ATOMIC_RELAXED) != 0u) filling = true;
+  if (filling && total >= kTwoLaunchWhileFilling) {
+    // the members' tables are being filled: see krk_sparse_pull_pooled and group_pull_missing_kernel
+    GroupFill fill{};
+    uint64_t words = 0;
+    for (int m = 0; m < n_tables; ++m) {
+      const int64_t cnt = pool.row_start[m + 1] - pool.row_start[m];
+      fill.todo_start[m] = (uint32_t)words;
+      if (cnt <= 0) continue;
+      words += (uint64_t)kQueues * (uint64_t)queue_capacity(cnt, per_block);
+      if (g->tables[m]->pull_parity) fill.parity_bits |= 1u << m;
+      g->tables[m]->pull_parity ^= 1;
+    }
+    KRK_TRY(g->todo.reserve((size_t)words * sizeof(uint32_t)));
+    uint32_t* todo = g->todo.as<uint32_t>();
+    const dim3 missing_grid((unsigned)n_tables * kGroupMissPerTable), missing_block(kMissBlock);
+    hipLaunchKernelGGL(group_pooled_find_kernel, probe_grid, block, 0, g->stream, g->d_descs, call, parts, fill, rows,
+                       todo);
+    if (g->vec == 4) {
+      hipLaunchKernelGGL((group_pull_missing_kernel<4, true>), missing_grid, missing_block, 0, g->stream, g->d_descs,
+                         call, parts, fill, todo, per_block, (int)g->dim, g->elems, g->group, rows);
+    } else {
+      hipLaunchKernelGGL((group_pull_missing_kernel<1, true>), missing_grid, missing_block, 0, g->stream, g->d_descs,
+                         call, parts, fill, todo, per_block, (int)g->dim, g->elems, g->group, rows);
+    }
+  } else if (total > 0) {
+    if (g->vec == 4) {
+      hipLaunchKernelGGL((group_pooled_probe_kernel<4>), probe_grid, block, 0, g->stream, g->d_descs, call, parts,
+                         rows, g->elems);
+    } else {
+      hipLaunchKernelGGL((group_pooled_probe_kernel<1>), probe_grid, block, 0, g->stream, g->d_descs, call, parts,
+                         rows, g->elems);
+    }
+  }
+  const dim3 sum_grid((unsigned)sum_blocks);
+  if (g->vec == 4) {
+    hipLaunchKernelGGL((group_pooled_sum_kernel<4>), sum_grid, block, 0, g->stream, g->d_descs, pool, rows,
+                       (int)g->dim, g->elems, g->group);
+  } else {
+    hipLaunchKernelGGL((group_pooled_sum_kernel<1>), sum_grid, block, 0, g->stream, g->d_descs, pool, rows,
+                       (int)g->dim, g->elems, g->group);
+  }
+  KRK_HIP(hipGetLastError());
+  if ((flags & KRK_NOTE_ROWS) && total > 0) {
+    g->noted_ids.assign(pool.ids, pool.ids + n_tables);
+    g->noted_offsets.assign(pool.row_start, pool.row_start + n_tables + 1);
+    g->noted_versions.clear();
+    for (krk_sparse* t : g->tables) g->noted_versions.push_back(t->layout_version);
+  }
+  if (flags & KRK_ASYNC) {
+    bool any = false;
+    for (krk_sparse* t : g->tables) any = any || sparse_near_full(t);
+    if (any) KRK_TRY(sparse_publish(g->tables.data(), (int)g->tables.size(), g->stream));
+  }
   return group_finish(g, flags);
 }
 

@@ -20,6 +20,7 @@
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/utils/pybind.h>
 
+#include <algorithm>
 #include <memory>
 #include <vector>
 
@@ -175,7 +176,8 @@ struct JaggedBackward : Node {
     const Tensor g = grads[0].contiguous().to(at::kFloat);
     KRK_CALL(krk_sparse_set_stream, table->h, current_stream());
     KRK_CALL(krk_sparse_push_pooled, table->h, table->optim, id_ptr(saved), saved.numel(), off_ptr(off),
-             off.numel() - 1, float_ptr(weights), mode, float_ptr(g), table->dim, (float)table->lr, kFlags);
+             off.numel() - 1, float_ptr(weights), mode, float_ptr(g), table->dim, (float)table->lr,
+             kFlags | KRK_IDS_AS_PULLED);
     return variable_list(1);
   }
   void release_variables() override {
@@ -193,10 +195,11 @@ Tensor jagged(const TablePtr& table, const Tensor& param, const Tensor& indices,
   const Tensor w = weights_of(weights_in);
   const int64_t bags = off.numel() - 1;
   Tensor out = new_rows({bags, table->dim}, ids);
+  const bool record = recording(param);
   KRK_CALL(krk_sparse_set_stream, table->h, current_stream());
   KRK_CALL(krk_sparse_pull_pooled, table->h, id_ptr(ids), ids.numel(), off_ptr(off), bags, float_ptr(w), mode,
-           (float)patch, out.mutable_data_ptr<float>(), kFlags);
-  if (recording(param)) {
+           (float)patch, out.mutable_data_ptr<float>(), kFlags | (record ? KRK_NOTE_ROWS : 0u));
+  if (record) {
     auto node = new_node<JaggedBackward>(param);
     node->table = table;
     node->mode = mode;
@@ -310,6 +313,9 @@ std::vector<Tensor> combine(const CombinePtr& c, const Tensor& param, const std:
   return outs;
 }
 
+// Groups whose request is larger than this are served a table at a time.
+constexpr int64_t kCombinedMax = (int64_t)1 << 28;
+
 struct CombineJaggedBackward : Node {
   CombinePtr c;
   std::vector<int> modes;
@@ -317,13 +323,47 @@ struct CombineJaggedBackward : Node {
   std::vector<Tensor> weights;
   variable_list apply(variable_list&& grads) override {
     void* stream = current_stream();
-    for (const Combine::Group& g : c->groups) KRK_CALL(krk_group_set_stream, g.h, stream);
-    for (size_t i = 0; i < c->tables.size(); ++i) {
-      if (!grads[i].defined()) continue;       // an output the loss never used: nothing to push
-      const Tensor saved = ids[i].unpack(), off = offsets[i].unpack();
-      const Tensor g = grads[i].contiguous().to(at::kFloat);
-      KRK_CALL(krk_sparse_push_pooled, c->tables[i], c->optim, id_ptr(saved), saved.numel(), off_ptr(off),
-               off.numel() - 1, float_ptr(weights[i]), modes[i], float_ptr(g), c->dims[i], (float)c->lr, kFlags);
+    for (const Combine::Group& g : c->groups) {
+      std::vector<krk_pooled_part> parts(g.members.size());
+      std::vector<Tensor> keep;
+      keep.reserve(3 * g.members.size());
+      int64_t total = 0;
+      for (size_t m = 0; m < g.members.size(); ++m) {
+        const int i = g.members[m];
+        krk_pooled_part& p = parts[m];
+        p = krk_pooled_part{};
+        if (!grads[i].defined()) continue;     // an output the loss never used: nothing to push
+        Tensor saved = ids[i].unpack(), off = offsets[i].unpack();
+        Rows r = rows_of(grads[i], g.dim);
+        p.ids = id_ptr(saved);
+        p.n = saved.numel();
+        p.offsets = off_ptr(off);
+        p.bags = off.numel() - 1;
+        p.weights = float_ptr(weights[i]);
+        p.rows = r.ptr();
+        p.stride = r.stride;
+        p.mode = modes[i];
+        total += std::max(p.n, p.bags);
+        keep.push_back(std::move(saved));
+        keep.push_back(std::move(off));
+        keep.push_back(std::move(r.keep));
+      }
+      KRK_CALL(krk_group_set_stream, g.h, stream);
+      const int32_t rc = total > kCombinedMax
+                             ? KRK_E_CAPACITY
+                             : krk_group_push_pooled_parts(g.h, c->optim, parts.data(), g.dim, (float)c->lr,
+                                                           kFlags | KRK_IDS_AS_PULLED);
+      if (rc == KRK_SUCCESS) continue;
+      if (rc != KRK_E_CAPACITY) fail(rc, "krk_group_push_pooled_parts");
+      // more than one launch can name: a table at a time
+      for (size_t m = 0; m < g.members.size(); ++m) {
+        const krk_pooled_part& p = parts[m];
+        if (p.n == 0 || p.bags == 0) continue;
+        const int i = g.members[m];
+        const Tensor rows = grads[i].contiguous().to(at::kFloat);
+        KRK_CALL(krk_sparse_push_pooled, c->tables[i], c->optim, p.ids, p.n, p.offsets, p.bags, p.weights, p.mode,
+                 float_ptr(rows), g.dim, (float)c->lr, kFlags);
+      }
     }
     return variable_list(1);
   }
@@ -343,19 +383,43 @@ std::vector<Tensor> combine_jagged(const CombinePtr& c, const Tensor& param, con
   if (values.size() != n || offsets_in.size() != n || weights_in.size() != n || modes.size() != n ||
       patches.size() != n)
     throw py::value_error("one jagged batch per table");
+  const bool record = recording(param);
   void* stream = current_stream();
   std::vector<Tensor> outs(n), ids(n), offsets(n), weights(n);
-  for (const Combine::Group& g : c->groups) KRK_CALL(krk_group_set_stream, g.h, stream);
-  for (size_t i = 0; i < n; ++i) {
-    ids[i] = ids_of(values[i]);
-    offsets[i] = ids_of(offsets_in[i], "offsets");
-    weights[i] = weights_of(weights_in[i]);
-    const int64_t bags = offsets[i].numel() - 1;
-    outs[i] = new_rows({bags, c->dims[i]}, ids[i]);
-    KRK_CALL(krk_sparse_pull_pooled, c->tables[i], id_ptr(ids[i]), ids[i].numel(), off_ptr(offsets[i]), bags,
-             float_ptr(weights[i]), modes[i], (float)patches[i], outs[i].mutable_data_ptr<float>(), kFlags);
+  for (const Combine::Group& g : c->groups) {
+    std::vector<krk_pooled_part> parts(g.members.size());
+    int64_t total = 0, bags = 0;
+    for (int i : g.members) {
+      ids[i] = ids_of(values[i]);
+      offsets[i] = ids_of(offsets_in[i], "offsets");
+      weights[i] = weights_of(weights_in[i]);
+      bags += offsets[i].numel() - 1;
+      total += std::max(ids[i].numel(), offsets[i].numel() - 1);
+    }
+    const Tensor whole = new_rows({bags, g.dim}, ids[g.members[0]]);
+    float* base = whole.mutable_data_ptr<float>();
+    int64_t at = 0;
+    for (size_t m = 0; m < g.members.size(); ++m) {
+      const int i = g.members[m];
+      const int64_t mine = offsets[i].numel() - 1;
+      outs[i] = piece_of(whole, at, {mine, g.dim});
+      parts[m] = krk_pooled_part{id_ptr(ids[i]), ids[i].numel(), off_ptr(offsets[i]), mine, float_ptr(weights[i]),
+                                 base + at, g.dim, modes[i], (float)patches[i]};
+      at += mine * g.dim;
+    }
+    KRK_CALL(krk_group_set_stream, g.h, stream);
+    const int32_t rc =
+        total > kCombinedMax ? KRK_E_CAPACITY
+                             : krk_group_pull_pooled_parts(g.h, parts.data(), kFlags | (record ? KRK_NOTE_ROWS : 0u));
+    if (rc == KRK_SUCCESS) continue;
+    if (rc != KRK_E_CAPACITY) fail(rc, "krk_group_pull_pooled_parts");
+    for (size_t m = 0; m < g.members.size(); ++m) {
+      const krk_pooled_part& p = parts[m];
+      KRK_CALL(krk_sparse_pull_pooled, c->tables[g.members[m]], p.ids, p.n, p.offsets, p.bags, p.weights, p.mode,
+               p.patch_value, p.rows, kFlags);
+    }
   }
-  if (recording(param)) {
+  if (record) {
     auto node = new_node<CombineJaggedBackward>(param);
     node->c = c;
     node->modes = modes;

@@ -197,3 +197,75 @@ def test_pooled_push_equals_push_raw_of_the_expanded_gradient(api, oracle):
         moved = np.abs(wb - before).max()
         assert moved > 1e-3                                   # the pushes did something
         assert np.abs(wa - wb).max() <= 1e-6 * max(1.0, moved * 10), (mode, weights is not None)
+
+
+@pytest.mark.parametrize("bags", [[300, 0, 1, 700], [4000, 20, 0, 700]], ids=["short", "long"])
+@pytest.mark.parametrize("dim", [16, 6])
+@pytest.mark.parametrize("noted", [False, True])
+def test_combined_pooled_pull_and_push(api, oracle, bags, dim, noted):
+    """krk_group_pull_pooled_parts / krk_group_push_pooled_parts over members that differ in mode and
+    weights, one of them empty, one with positions outside every bag, gradients that are columns of
+    a wider matrix; requests on both sides of the 8192 ids a member up to which a push is two
+    launches, new ids every step, with and without the row notes of the pull. Binary-grid values:
+    every sum is exact, so the rows are the oracle's bit for bit."""
+    C = api.C
+
+    class Part(C.Structure):
+        _fields_ = [("ids", C.c_void_p), ("n", C.c_int64), ("offsets", C.c_void_p), ("bags", C.c_int64),
+                    ("weights", C.c_void_p), ("rows", C.c_void_p), ("stride", C.c_int64), ("mode", C.c_int32),
+                    ("patch", C.c_float)]
+
+    rng = np.random.default_rng(dim + len(bags) + noted)
+    modes, weighted = ["sum", "mean", "sum", "mean"], [False, False, True, True]
+    pairs = [_tables(api, oracle, dim, seed=70 + k) for k in range(4)]
+    group = api.TableGroup([t for t, _ in pairs])
+    o_ref, o_gpu = make_optims(oracle, api, 3, {})
+    flags = api.DEVICE_PTRS
+    for step in range(3):
+        parts, push, host, keep = (Part * 4)(), (Part * 4)(), [], []
+        wide = (rng.integers(-64, 65, size=(max(bags), 4, dim)) / 512.0).astype(np.float32)
+        d_wide = api.DeviceArray.from_host(wide.reshape(max(bags), 4 * dim))
+        for k in range(4):
+            ids, off = _bags(rng, bags[k], 8, 1500 * (step + 1), pow2=True) if bags[k] else (
+                np.zeros(0, np.uint64), np.zeros(1, np.int64))
+            if k == 3:                                     # two positions ahead of the bags, one behind
+                ids = np.concatenate([ids[:1], ids[-1:], ids, ids[:1]]) + np.uint64(1)
+                off = off + 2
+            w = (2.0 ** rng.integers(-2, 3, size=ids.size)).astype(np.float32) if weighted[k] else None
+            d = [api.DeviceArray.from_host(a) if a is not None and a.size else None for a in (ids, off, w)]
+            out = api.DeviceArray((max(bags[k], 1), dim), np.float32)
+            keep.append((d, out))
+            ptr = [x.ptr if x is not None else None for x in d]
+            mode = 0 if modes[k] == "sum" else 1
+            parts[k] = Part(ptr[0], ids.size, ptr[1], bags[k], ptr[2], out.ptr, dim, mode, 0.25)
+            push[k] = Part(ptr[0], ids.size, ptr[1], bags[k], ptr[2], d_wide.ptr + 4 * dim * k, 4 * dim, mode, 0.0)
+            host.append((ids, off, w, out))
+        api._check(api.lib().krk_group_pull_pooled_parts(group.h, parts, flags | (api.NOTE_ROWS if noted else 0)), "pull")
+        for k, (ids, off, w, out) in enumerate(host):
+            if not bags[k]:
+                continue
+            ref = pairs[k][1]
+            ref.pull(oracle.dedup(ids)[0])                 # rows are made in the order the oracle meets them
+            lo, hi = int(off[0]), int(off[-1])
+            want = _oracle_pooled_pull(oracle, ref, ids[lo:hi], off - lo, modes[k], 0.25, w[lo:hi] if w is not None else None)
+            assert np.array_equal(out.to_host(), want), (step, k)
+        api._check(api.lib().krk_group_push_pooled_parts(group.h, C.byref(o_gpu.raw), push, dim, 0.5,
+                                                         flags | (api.IDS_AS_PULLED if noted else 0)), "push")
+        for k, (ids, off, w, _) in enumerate(host):
+            if not bags[k]:
+                continue
+            lo, hi = int(off[0]), int(off[-1])
+            vg = oracle.jagged_backward(off - lo, np.ascontiguousarray(wide[:bags[k], k]), modes[k])
+            if w is not None:
+                vg = vg * w[lo:hi, None]
+            u, gs = oracle.dedup_sum(ids[lo:hi], vg)
+            assert pairs[k][1].push(o_ref, u, gs, 0.5) == 0
+            every = np.unique(ids)
+            assert np.array_equal(pairs[k][0].Pull(every)[1], pairs[k][1].pull(every)[1]), (step, k)
+            assert len(pairs[k][0]) == len(pairs[k][1])
+    missing = splitmix64(np.arange(10**7, 10**7 + 40, dtype=np.uint64))
+    d_ids, d_off = api.DeviceArray.from_host(missing), api.DeviceArray.from_host(np.array([0, 40], np.int64))
+    one = (Part * 4)()
+    one[0] = Part(d_ids.ptr, 40, d_off.ptr, 1, None, keep[0][1].ptr, dim, 0, 0.0)
+    assert api.lib().krk_group_push_pooled_parts(group.h, C.byref(o_gpu.raw), one, dim, 0.5, flags) == api.SPARSE_ID_NOT_EXIST
+    group.close()

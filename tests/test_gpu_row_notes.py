@@ -279,3 +279,34 @@ def test_group_push_of_unique_ids_with_notes_equals_without(api, dim):
             _same_tables(api, a, b, [api.StateType.kStateSum])
     ga.close()
     gb.close()
+
+
+@pytest.mark.parametrize("n", [8193, 300_000])
+def test_long_pushes_with_notes_equal_those_without(api, n):
+    """push_raw of requests that are sorted (above 8192 ids, and above the size from which a pull runs
+    as two launches), and the pooled pull and push of one table, with and without the flags. Binary-grid
+    gradients: the sums do not depend on how equal rows are grouped."""
+    dim = 8
+    rng = np.random.default_rng(n)
+    o = api.Optim.create(api.OptimType.kAdagrad)
+    a, b = api.SparseTable(dim, _init(api)), api.SparseTable(dim, _init(api))
+    lib, C = api.lib(), api.C
+    off = np.concatenate([[0], np.sort(rng.choice(np.arange(1, n), 2000, replace=False)), [n]]).astype(np.int64)
+    d_off = api.DeviceArray.from_host(off)
+    outs = [api.DeviceArray((off.size - 1, dim), np.float32) for _ in range(2)]
+    for step in range(2):
+        d_ids = api.DeviceArray.from_host(zipf_ids(rng, 1.1, 50000, n) + np.uint64(step * 20000))
+        d_g = api.DeviceArray.from_host((rng.integers(-64, 65, size=(n, dim)) / 4096.0).astype(np.float32))
+        assert a.Pull(d_ids, note_rows=True)[0] == 0 and b.Pull(d_ids)[0] == 0
+        assert a.PushRaw(o, d_ids, d_g, 0.05, as_pulled=True) == 0
+        assert b.PushRaw(o, d_ids, d_g, 0.05) == 0
+        for t, out, note, pulled in ((a, outs[0], api.NOTE_ROWS, api.IDS_AS_PULLED), (b, outs[1], 0, 0)):
+            p = lambda x: C.c_void_p(x.ptr)
+            assert lib.krk_sparse_pull_pooled(t.h, p(d_ids), n, p(d_off), off.size - 1, None, 0, 0.0, p(out),
+                                              api.DEVICE_PTRS | note) == 0
+            assert lib.krk_sparse_push_pooled(t.h, C.byref(o.raw), p(d_ids), n, p(d_off), off.size - 1, None, 0,
+                                              p(d_g), dim, 0.05, api.DEVICE_PTRS | pulled) == 0
+        assert np.array_equal(outs[0].to_host(), outs[1].to_host())
+    _same_tables(api, a, b, [api.StateType.kStateSum])
+    a.close()
+    b.close()
