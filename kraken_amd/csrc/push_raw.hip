@@ -427,19 +427,44 @@ __global__ __launch_bounds__(kBlock) void fill_u32_kernel(uint32_t* __restrict__
 
 constexpr int kBagLanes = 8;   // lanes that share one bag's positions
 
-// What the bags of a pooled push leave for the reduction. Always: ratio[bag], where the member's
-// bags are means, is what a mean bag hands on of its gradient (pytorch/py/jagged_ops.cc:303-334:
-// (float)(1.0 / float(len)), once per bag here as there; the reduction multiplies each gradient
-// row it reads, so no scaled copy of the gradients is written and read back: 852k bags of 32 floats
-// took 85 us for that). bag_of[position] = the bag, kNoBag outside every bag.
+// What a pooled push carries for a position instead of a bag number alone: the bag in the low
+// bag_bits bits and above them the bag's length, as far as it fits (all ones: look it up). A mean bag
+// hands on grads * ratio, ratio = (float)(1.0 / float(len)) (pytorch/py/jagged_ops.cc:303-334), and
+// the length is what the reduction needs for that: a scaled copy of the gradients takes a pass of
+// its own (852k bags of 32 floats: 85 us), and an array of ratios costs the reduction one more
+// random read per entry (8.5 million entries: 585 us instead of 461).
+struct BagWord {
+  int bag_bits;                          // bags < 2^bag_bits, so that no word is kNoBag
+  __host__ __device__ uint32_t bag(uint32_t w) const { return w & ((1u << bag_bits) - 1u); }
+  __host__ __device__ uint32_t longest() const { return (1u << (32 - bag_bits)) - 1u; }
+  __device__ uint32_t pack(uint32_t b, long long len) const {
+    const uint32_t most = longest();
+    return b | ((len < (long long)most ? (uint32_t)(len < 0 ? 0 : len) : most) << bag_bits);
+  }
+};
+static BagWord bag_word(int64_t bags) {
+  BagWord w{1};
+  while (((int64_t)1 << w.bag_bits) <= bags) ++w.bag_bits;
+  return w;
+}
+// 1.0f / x in fp32 is (float)(1.0 / (double)x) for every fp32 x that is a whole number: the quotient
+// of two 24-bit significands is never close enough to the middle of two floats for the
+// intermediate rounding to matter.
+__device__ __forceinline__ float mean_ratio(long long len) { return len > 0 ? 1.0f / (float)len : 0.0f; }
+__device__ __forceinline__ float mean_ratio(const BagWord& words, uint32_t word, const long long* offsets) {
+  const uint32_t len = word >> words.bag_bits, b = words.bag(word);
+  return mean_ratio(len == words.longest() ? offsets[b + 1] - offsets[b] : (long long)len);
+}
+
+// bag_of[position] = the word of its bag, kNoBag outside every bag.
 // NOTED: the rows of the positions are known from the pull, so the bag also writes its positions'
 // keys and payloads and no other launch looks at them; bag_of is then only written where a member
 // is weighted (its payloads are positions).
 template <bool GROUPED, bool NOTED>
 __global__ __launch_bounds__(kBlock) void bag_expand_kernel(const TableDesc* __restrict__ descs, TableView tv,
-                                                            PooledCall call, int row_bits, uint32_t miss_key,
-                                                            const uint32_t* __restrict__ notes,
-                                                            uint32_t* __restrict__ bag_of, float* __restrict__ ratio,
+                                                            PooledCall call, BagWord words, int row_bits,
+                                                            uint32_t miss_key, const uint32_t* __restrict__ notes,
+                                                            uint32_t* __restrict__ bag_of,
                                                             uint32_t* __restrict__ keys, uint32_t* __restrict__ pos) {
   int m = 0;
   if (GROUPED) {
@@ -457,17 +482,16 @@ __global__ __launch_bounds__(kBlock) void bag_expand_kernel(const TableDesc* __r
   const int64_t a = call.row_start[m];
   const int64_t n = call.row_start[m + 1] - a;
   const long long begin = call.offsets[m][b], end = call.offsets[m][b + 1];
-  if (gl == 0 && ((call.mean_bits >> m) & 1u))
-    ratio[call.bag_start[m] + b] = end > begin ? (float)(1.0 / (double)(float)(end - begin)) : 0.0f;
+  const uint32_t word = words.pack((uint32_t)b, end - begin);
   const bool weighted = call.weights[m] != nullptr;
   const uint32_t member_key = (uint32_t)m << row_bits;
   const long long lo = begin < 0 ? 0 : begin, hi = end > n ? n : end;
   for (long long p = lo + gl; p < hi; p += kBagLanes) {
     if (NOTED) {
       keys[a + p] = noted_key(tv, notes[a + p], call.ids[m] + p, member_key, miss_key);
-      if (pos) pos[a + p] = weighted ? (uint32_t)p : (uint32_t)b;
+      if (pos) pos[a + p] = weighted ? (uint32_t)p : word;
     }
-    if (!NOTED || weighted || !pos) bag_of[a + p] = (uint32_t)b;
+    if (!NOTED || weighted || !pos) bag_of[a + p] = word;
   }
   // positions before the first bag and behind the last belong to none
   auto outside = [&](long long from, long long to) {
@@ -599,21 +623,22 @@ constexpr int kCarryTile = 4;   // 16, 32 and 64 were measured: 254, 272 and 304
 
 // Pooled pushes (level 0 only). Weighted bags: the sorted payload is a position p, its gradient row
 // is that of bag bag_of[p], times weight[p]; otherwise weight is null and the payload itself names
-// the row. ratio (bags that are means, else null): what a bag hands on of its gradient.
+// the bag. pooled false: the payload names the gradient row.
 struct PooledSrc {
+  bool pooled, mean;
+  BagWord words;
   const uint32_t* bag_of;
   const float* weight;
-  const float* ratio;
+  const long long* offsets;
 };
-// The same for a combined push: the gradient rows lie where the members have them, and bag_of,
-// the ratios and the payloads count from the member's first position and bag. bag_of null: not pooled.
+// The same for a combined push: the gradient rows lie where the members have them, and payloads
+// and bags count from the member's first.
 struct GroupPooledSrc {
   PooledCall call;
+  BagWord words;
   const uint32_t* bag_of;
-  const float* ratio;
-  int weighted;          // some member is
+  bool pooled, weighted;          // weighted: some member is
 };
-
 // Combined pushes (GROUPED): a key is (member number << row_bits) | row, and a closed run takes
 // its member's record layout from descs. st0..st2 are the state types of the optimizer's three
 // slots (-1 = unused); the column each lives in differs from member to member.
@@ -635,12 +660,17 @@ __host__ __device__ inline size_t segreduce_lds_words(int per_block, int group, 
          (pooled ? 2 * span : 0);
 }
 
-template <int OPT, int VEC, bool LEVEL0, bool GROUPED>
+// What the entries of a sequence are.
+constexpr int kFromCarry = 0;    // partial sums of the level before
+constexpr int kFromRows = 1;     // level 0: gradient rows
+constexpr int kFromBags = 2;     // level 0 of a pooled push: bags' gradient rows, scaled as they are read
+template <int OPT, int VEC, int FROM, bool GROUPED>
 __global__ __launch_bounds__(kBlock) void segreduce_kernel(
     TableView tv, const uint32_t* __restrict__ keys, const uint32_t* __restrict__ pos,
     const float* __restrict__ vals, int64_t cnt, int tile, uint32_t empty_from,
     uint32_t* __restrict__ keys_out, float* __restrict__ vals_out, int dim, int elems, int group,
-    ApplyArgs args, std::conditional_t<LEVEL0 && GROUPED, GroupPooledSrc, PooledSrc> ps, GroupSrc gs) {
+    ApplyArgs args, std::conditional_t<FROM != kFromCarry && GROUPED, GroupPooledSrc, PooledSrc> ps, GroupSrc gs) {
+  constexpr bool LEVEL0 = FROM != kFromCarry, POOLED = FROM == kFromBags;
   extern __shared__ __align__(16) uint32_t lds[];
   const int per_block = kBlock / group;
   const int span = per_block * tile;                       // entries staged by this workgroup
@@ -656,10 +686,9 @@ __global__ __launch_bounds__(kBlock) void segreduce_kernel(
     const int64_t j = first + i - 1;
     lds_keys[i] = (j >= 0 && j < cnt) ? keys[j] : kNoRow;
   }
-  bool weighted = false, scaled = false;
+  bool weighted = false;
   if constexpr (LEVEL0 && GROUPED) {
-    weighted = ps.bag_of != nullptr && ps.weighted != 0;
-    scaled = ps.ratio != nullptr;
+    weighted = POOLED && ps.weighted;
     for (int i = threadIdx.x; i < span; i += kBlock) {
       const int64_t j = first + i;
       const uint32_t key = j < cnt ? keys[j] : kNoRow;
@@ -667,31 +696,31 @@ __global__ __launch_bounds__(kBlock) void segreduce_kernel(
       if (key < empty_from) {
         const int m = (int)(key >> gs.row_bits);
         uint32_t p = pos[j];
-        if (weighted) {
+        if constexpr (POOLED) {
           const float* w = ps.call.weights[m];
-          lds_w[i] = w ? w[p] : 1.0f;
+          if (weighted) lds_w[i] = w ? w[p] : 1.0f;
           if (w) p = ps.bag_of[ps.call.row_start[m] + p];
+          lds_r[i] = ((ps.call.mean_bits >> m) & 1u) ? mean_ratio(ps.words, p, ps.call.offsets[m]) : 1.0f;
+          p = ps.words.bag(p);
         }
-        if (scaled) lds_r[i] = ((ps.call.mean_bits >> m) & 1u) ? ps.ratio[ps.call.bag_start[m] + p] : 1.0f;
         src = (const KRK_GLOBAL float*)ps.call.rows[m] + (int64_t)p * ps.call.stride[m];
       }
       lds_src[i] = src;
     }
   } else if constexpr (LEVEL0) {
-    weighted = ps.weight != nullptr;
-    scaled = ps.ratio != nullptr;
+    weighted = POOLED && ps.weight != nullptr;
     for (int i = threadIdx.x; i < span; i += kBlock) {
       const int64_t j = first + i;
       uint32_t p = j < cnt ? pos[j] : 0u;
-      if (weighted) {
-        // the payload is the position: it names the weight and, through bag_of, the row
-        lds_w[i] = j < cnt ? ps.weight[p] : 0.0f;
-        const uint32_t b = j < cnt ? ps.bag_of[p] : 0u;
-        p = b == kNoBag ? 0u : b;
-      }
-      if (scaled) {
+      if constexpr (POOLED) {
+        if (weighted) {
+          // the payload is the position: it names the weight and, through bag_of, the bag
+          lds_w[i] = j < cnt ? ps.weight[p] : 0.0f;
+          p = j < cnt ? ps.bag_of[p] : 0u;
+        }
         if (p == kNoBag) p = 0u;                           // outside every bag: its key is skipped
-        lds_r[i] = ps.ratio[p];
+        lds_r[i] = ps.mean ? mean_ratio(ps.words, p, ps.offsets) : 1.0f;
+        p = ps.words.bag(p);
       }
       lds_src[i] = (const KRK_GLOBAL float*)vals + (int64_t)p * dim;
     }
@@ -798,20 +827,13 @@ __global__ __launch_bounds__(kBlock) void segreduce_kernel(
           const int j = j0 + u;
           k[u] = j < lb ? lds_keys[j + 1] : kNoRow;
           if (j < lb && k[u] < empty_from && lane_on) {
-            if constexpr (LEVEL0) {
+            // (a bag's row is read once for every id of the bag: through the caches)
+            if constexpr (POOLED) {
+              gload<VEC>((const float*)(lds_src[j] + e * VEC), v[u]);
+            } else if constexpr (LEVEL0) {
               gload_once<VEC>(lds_src[j] + e * VEC, v[u]);
             } else {
               vload<VEC>(vals + (first + j) * dim + e * VEC, v[u]);
-            }
-            if (scaled) {
-              const float r = lds_r[j];
-#pragma unroll
-              for (int c = 0; c < VEC; ++c) v[u][c] = v[u][c] * r;
-            }
-            if (weighted) {
-              const float w = lds_w[j];
-#pragma unroll
-              for (int c = 0; c < VEC; ++c) v[u][c] = v[u][c] * w;
             }
           } else {
 #pragma unroll
@@ -822,6 +844,17 @@ __global__ __launch_bounds__(kBlock) void segreduce_kernel(
         for (int u = 0; u < kAhead; ++u) {
           const int j = j0 + u;
           if (j >= lb) break;
+          // (not where the rows are requested: the next request would wait for this one to arrive)
+          if constexpr (POOLED) {
+            const float r = lds_r[j];
+#pragma unroll
+            for (int c = 0; c < VEC; ++c) v[u][c] = v[u][c] * r;
+            if (weighted) {
+              const float w = lds_w[j];
+#pragma unroll
+              for (int c = 0; c < VEC; ++c) v[u][c] = v[u][c] * w;
+            }
+          }
           if (k[u] != run_key) {
             close_run(j);
             run_key = k[u];
@@ -903,17 +936,21 @@ static void launch_segreduce(bool level0, const TableView& tv, const uint32_t* k
   const int per_block = kBlock / t->group;
   const int64_t tiles = (cnt + tile - 1) / tile;
   const dim3 grid(grid_for(tiles, per_block)), block(kBlock);
-  const bool pooled = level0 && (gps ? gps->bag_of || gps->ratio : ps.weight || ps.ratio);
+  const bool pooled = level0 && (gps ? gps->pooled : ps.pooled);
   const size_t lds_bytes = segreduce_lds_words(per_block, t->group, VEC, tile, level0, pooled) * sizeof(uint32_t);
-  const PooledSrc none{nullptr, nullptr, nullptr};
+  const PooledSrc none{};
   if constexpr (OPT != kOptStore) {
     if (gs) {
-      if (level0) {
-        hipLaunchKernelGGL((segreduce_kernel<OPT, VEC, true, true>), grid, block, lds_bytes, stream, tv, keys,
+      if (pooled) {
+        hipLaunchKernelGGL((segreduce_kernel<OPT, VEC, kFromBags, true>), grid, block, lds_bytes, stream, tv, keys,
+                           pos, vals, cnt, tile, empty_from, keys_out, vals_out, (int)t->dim, t->elems,
+                           t->group, args, *gps, *gs);
+      } else if (level0) {
+        hipLaunchKernelGGL((segreduce_kernel<OPT, VEC, kFromRows, true>), grid, block, lds_bytes, stream, tv, keys,
                            pos, vals, cnt, tile, empty_from, keys_out, vals_out, (int)t->dim, t->elems,
                            t->group, args, *gps, *gs);
       } else {
-        hipLaunchKernelGGL((segreduce_kernel<OPT, VEC, false, true>), grid, block, lds_bytes, stream, tv, keys,
+        hipLaunchKernelGGL((segreduce_kernel<OPT, VEC, kFromCarry, true>), grid, block, lds_bytes, stream, tv, keys,
                            pos, vals, cnt, tile, empty_from, keys_out, vals_out, (int)t->dim, t->elems,
                            t->group, args, none, *gs);
       }
@@ -921,12 +958,20 @@ static void launch_segreduce(bool level0, const TableView& tv, const uint32_t* k
     }
   }
   const GroupSrc plain{nullptr, 0, -1, -1, -1, 0};
+  if constexpr (OPT != kOptStore) {
+    if (pooled) {
+      hipLaunchKernelGGL((segreduce_kernel<OPT, VEC, kFromBags, false>), grid, block, lds_bytes, stream, tv, keys,
+                         pos, vals, cnt, tile, empty_from, keys_out, vals_out, (int)t->dim, t->elems, t->group,
+                         args, ps, plain);
+      return;
+    }
+  }
   if (level0) {
-    hipLaunchKernelGGL((segreduce_kernel<OPT, VEC, true, false>), grid, block, lds_bytes, stream, tv, keys, pos,
+    hipLaunchKernelGGL((segreduce_kernel<OPT, VEC, kFromRows, false>), grid, block, lds_bytes, stream, tv, keys, pos,
                        vals, cnt, tile, empty_from, keys_out, vals_out, (int)t->dim, t->elems, t->group,
-                       args, ps, plain);
+                       args, none, plain);
   } else {
-    hipLaunchKernelGGL((segreduce_kernel<OPT, VEC, false, false>), grid, block, lds_bytes, stream, tv, keys, pos,
+    hipLaunchKernelGGL((segreduce_kernel<OPT, VEC, kFromCarry, false>), grid, block, lds_bytes, stream, tv, keys, pos,
                        vals, cnt, tile, empty_from, keys_out, vals_out, (int)t->dim, t->elems, t->group,
                        args, none, plain);
   }
@@ -1020,13 +1065,13 @@ constexpr int kShortMaxDim = 64;
 static_assert(kSortWaves * kDigits <= kSortMax + 1, "the histogram fits the work space");
 
 // Pooled pushes: spos holds a bag (counted in its member) where the member's bags are not weighted,
-// a position where they are; bag_of and ratio as bag_expand_kernel leaves them.
+// a position where they are; bag_of as bag_expand_kernel leaves it.
 struct BucketPooled {
   const uint32_t* bag_of;
-  const float* ratio;
+  BagWord words;
   uint32_t mean_bits;
-  int64_t bag_start[kMaxGroupTables];
   const float* weights[kMaxGroupTables];
+  const long long* offsets[kMaxGroupTables];
 };
 constexpr int64_t kBucketMaxBags = 65536;              // a bag is kept in 16 bits
 
@@ -1163,7 +1208,7 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(
       skey[at] = (mine[i] & call.row_mask) >> bucket_bits;
       spos[at] = (uint16_t)(t * own + i);
       if constexpr (POOLED) {
-        if (!pool.weights[m]) spos[at] = (uint16_t)pool.bag_of[a + t * own + i];
+        if (!pool.weights[m]) spos[at] = (uint16_t)pool.words.bag(pool.bag_of[a + t * own + i]);
       }
       ++at;
     }
@@ -1285,11 +1330,11 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(
       const bool weighted = pool.weights[m] != nullptr;
       if (weighted) {
         w = pool.weights[m][b];
-        b = pool.bag_of[a + b];
+        b = pool.words.bag(pool.bag_of[a + b]);
       }
       gload<VEC>(g_base + (int64_t)b * g_stride + gl * VEC, v);
       if ((pool.mean_bits >> m) & 1u) {
-        const float r = pool.ratio[pool.bag_start[m] + b];
+        const float r = mean_ratio(pool.offsets[m][b + 1] - pool.offsets[m][b]);
 #pragma unroll
         for (int c = 0; c < VEC; ++c) v[c] = v[c] * r;
       }
@@ -2020,7 +2065,7 @@ int32_t krk_dedup_sum(const uint64_t* ids, int64_t n, const float* grads, int64_
   const DSlot* slots = w.slots;
   const uint32_t* slot_of = w.slot_of;
   KRK_TRY(sort_and_reduce(sh, s, g_dedup_reduce, tv, kOptStore, n, miss_key, bits, d_g, args,
-                          PooledSrc{nullptr, nullptr, nullptr}, nullptr, nullptr, [&](uint32_t* keys, uint32_t* pos) {
+                          PooledSrc{}, nullptr, nullptr, [&](uint32_t* keys, uint32_t* pos) {
                             hipLaunchKernelGGL(dedup_pairs_kernel, dim3(grid_for(n, kBlock)), dim3(kBlock), 0, s,
                                                slots, slot_of, n, keys, pos);
                           }));
@@ -2150,7 +2195,7 @@ int32_t krk_sparse_push_raw(krk_sparse* t, const krk_optim* o, const uint64_t* i
     return sparse_finish(t, flags);
   }
   const uint32_t* notes = noted_rows(t, ids, n, flags);
-  KRK_TRY(push_sorted(t, o, n, d_g, lr, PooledSrc{nullptr, nullptr, nullptr},
+  KRK_TRY(push_sorted(t, o, n, d_g, lr, PooledSrc{},
                       [&](uint32_t* keys, uint32_t* pos, uint32_t miss_key) {
                         if (notes) {
                           hipLaunchKernelGGL(noted_keys_kernel, dim3(grid_for(n, kBlock)), dim3(kBlock), 0, t->stream,
@@ -2285,7 +2330,7 @@ static int32_t group_push_raw_enqueue(krk_group* g, const krk_optim* o, const in
   memcpy(src.call.stride, parts.stride, sizeof(src.call.stride));
   const uint32_t* notes = noted_rows(g, parts.ids, offsets, flags);
   return sort_and_reduce(sh, g->stream, g->scratch, none, o->type, total, miss_key, gk.bits, nullptr, args,
-                         PooledSrc{nullptr, nullptr, nullptr}, &gs, &src, [&](uint32_t* keys, uint32_t* pos) {
+                         PooledSrc{}, &gs, &src, [&](uint32_t* keys, uint32_t* pos) {
                            if (notes) {
                              hipLaunchKernelGGL(group_noted_keys_kernel, dim3(grid_for(total, kBlock)), dim3(kBlock), 0,
                                                 g->stream, g->d_descs, call, parts, total, row_bits, miss_key, notes,
@@ -2298,44 +2343,33 @@ static int32_t group_push_raw_enqueue(krk_group* g, const krk_optim* o, const in
                          });
 }
 
-// Work space of a pooled push: the bag of every position and, for means, the ratio of every bag.
-struct PooledWork {
-  uint32_t* bag_of;      // null: out of memory
-  float* ratio;          // null: no means
-};
-static PooledWork pooled_work(DeviceBuffer& buffer, int64_t n, int64_t bags, bool mean) {
-  const size_t bag_of_bytes = ((size_t)n * sizeof(uint32_t) + 255) & ~(size_t)255;
-  if (buffer.reserve(bag_of_bytes + (mean ? (size_t)bags * sizeof(float) : 0)) != KRK_SUCCESS)
-    return PooledWork{nullptr, nullptr};
-  return PooledWork{buffer.as<uint32_t>(), mean ? reinterpret_cast<float*>(buffer.as<char>() + bag_of_bytes) : nullptr};
-}
-
 // A pooled push on one table, which `call` describes as its only member (device addresses). The caller
 // holds the table's lock and has made the optimizer's columns exist.
 static int32_t push_pooled_enqueue(krk_sparse* t, const krk_optim* o, PooledCall& call, const uint32_t* notes,
                                    float lr) {
   const int64_t n = call.row_start[1], bags = call.bag_start[1];
-  const bool mean = call.mean_bits != 0, weighted = call.weights[0] != nullptr;
+  const bool weighted = call.weights[0] != nullptr;
   const int64_t blocks = pooled_layout(&call, kBlock / kBagLanes);
   if (blocks < 0) {
     set_error("pooled push: too many bags for one launch; split the request");
     return KRK_E_CAPACITY;
   }
-  const PooledWork w = pooled_work(t->scratch[5], n, bags, mean);
-  if (!w.bag_of) return KRK_E_DEVICE;
+  KRK_TRY(t->scratch[5].reserve((size_t)n * sizeof(uint32_t)));
+  uint32_t* bag_of = t->scratch[5].as<uint32_t>();
+  const BagWord words = bag_word(bags);
   const TableView tv = t->view();
   auto fill = [&](uint32_t* keys, uint32_t* pos, uint32_t miss_key) {
     if (notes) {
       hipLaunchKernelGGL((bag_expand_kernel<false, true>), dim3((unsigned)blocks), dim3(kBlock), 0, t->stream, nullptr,
-                         tv, call, 0, miss_key, notes, w.bag_of, w.ratio, keys, pos);
+                         tv, call, words, 0, miss_key, notes, bag_of, keys, pos);
     } else {
       hipLaunchKernelGGL((bag_expand_kernel<false, false>), dim3((unsigned)blocks), dim3(kBlock), 0, t->stream, nullptr,
-                         tv, call, 0, miss_key, (const uint32_t*)nullptr, w.bag_of, w.ratio, (uint32_t*)nullptr,
+                         tv, call, words, 0, miss_key, (const uint32_t*)nullptr, bag_of, (uint32_t*)nullptr,
                          (uint32_t*)nullptr);
       // Unweighted: the sort carries bag numbers and the reduction reads bag rows directly.
       // Weighted: it carries positions, which name the weight and (through bag_of) the bag.
       hipLaunchKernelGGL(rows_of_ids_kernel, dim3(grid_for(n, kBlock / kBucket)), dim3(kBlock), 0, t->stream, tv,
-                         call.ids[0], n, miss_key, (const uint32_t*)w.bag_of, !weighted, keys, pos);
+                         call.ids[0], n, miss_key, (const uint32_t*)bag_of, !weighted, keys, pos);
     }
   };
   if (short_push_fits(n, t->dim, t->elems, t->group) && bags <= kBucketMaxBags) {
@@ -2348,11 +2382,11 @@ static int32_t push_pooled_enqueue(krk_sparse* t, const krk_optim* o, PooledCall
     parts.rows[0] = call.rows[0];
     parts.stride[0] = call.stride[0];
     BucketPooled pool;
-    pool.bag_of = w.bag_of;
-    pool.ratio = w.ratio;
+    pool.bag_of = bag_of;
+    pool.words = words;
     pool.mean_bits = call.mean_bits;
-    pool.bag_start[0] = 0;
     pool.weights[0] = call.weights[0];
+    pool.offsets[0] = call.offsets[0];
     const GroupSrc none{nullptr, 0, -1, -1, -1, 0};
     const ApplyArgs args = table_apply_args(t, o, lr);
     if (t->vec == 4) {
@@ -2366,7 +2400,7 @@ static int32_t push_pooled_enqueue(krk_sparse* t, const krk_optim* o, PooledCall
     return KRK_SUCCESS;
   }
   return push_sorted(t, o, n, call.rows[0], lr,
-                     PooledSrc{weighted ? w.bag_of : nullptr, weighted ? call.weights[0] : nullptr, w.ratio}, fill);
+                     PooledSrc{true, call.mean_bits != 0, words, bag_of, call.weights[0], call.offsets[0]}, fill);
 }
 
 extern "C" {
@@ -2543,8 +2577,9 @@ int32_t krk_group_push_pooled_parts(krk_group* g, const krk_optim* o, const krk_
     if (!call.weights[m]) bag_payload |= 1u << m;
     weighted = weighted || (call.weights[m] && call.row_start[m + 1] > call.row_start[m]);
   }
-  const PooledWork w = pooled_work(g->todo, total, bags, call.mean_bits != 0);
-  if (!w.bag_of) return KRK_E_DEVICE;
+  KRK_TRY(g->todo.reserve((size_t)total * sizeof(uint32_t)));
+  uint32_t* bag_of = g->todo.as<uint32_t>();
+  const BagWord words = bag_word(most_bags);
   const ApplyArgs args = group_apply_args(o, lr);
   const GroupSrc gs = group_src(g, o, gk.row_bits);
   GroupParts parts;
@@ -2560,13 +2595,13 @@ int32_t krk_group_push_pooled_parts(krk_group* g, const krk_optim* o, const krk_
   auto fill = [&](uint32_t* keys, uint32_t* pos) {
     if (notes) {
       hipLaunchKernelGGL((bag_expand_kernel<true, true>), dim3((unsigned)blocks), dim3(kBlock), 0, g->stream, g->d_descs,
-                         TableView{}, call, gk.row_bits, gk.miss_key, notes, w.bag_of, w.ratio, keys, pos);
+                         TableView{}, call, words, gk.row_bits, gk.miss_key, notes, bag_of, keys, pos);
     } else {
       hipLaunchKernelGGL((bag_expand_kernel<true, false>), dim3((unsigned)blocks), dim3(kBlock), 0, g->stream,
-                         g->d_descs, TableView{}, call, gk.row_bits, gk.miss_key, (const uint32_t*)nullptr, w.bag_of,
-                         w.ratio, (uint32_t*)nullptr, (uint32_t*)nullptr);
+                         g->d_descs, TableView{}, call, words, gk.row_bits, gk.miss_key, (const uint32_t*)nullptr,
+                         bag_of, (uint32_t*)nullptr, (uint32_t*)nullptr);
       hipLaunchKernelGGL(group_rows_of_ids_kernel, dim3(rows_call.block_start[n_tables]), dim3(kBlock), 0, g->stream,
-                         g->d_descs, rows_call, parts, gk.row_bits, gk.miss_key, (const uint32_t*)w.bag_of, bag_payload,
+                         g->d_descs, rows_call, parts, gk.row_bits, gk.miss_key, (const uint32_t*)bag_of, bag_payload,
                          keys, pos);
     }
   };
@@ -2576,11 +2611,11 @@ int32_t krk_group_push_pooled_parts(krk_group* g, const krk_optim* o, const krk_
     fill(keys, nullptr);
     const SortCall sc = group_sort_call(gk, n_tables, call.row_start);
     BucketPooled pool;
-    pool.bag_of = w.bag_of;
-    pool.ratio = w.ratio;
+    pool.bag_of = bag_of;
+    pool.words = words;
     pool.mean_bits = call.mean_bits;
-    memcpy(pool.bag_start, call.bag_start, sizeof(pool.bag_start));
     memcpy(pool.weights, call.weights, sizeof(pool.weights));
+    memcpy(pool.offsets, call.offsets, sizeof(pool.offsets));
     if (g->vec == 4) {
       launch_bucket_push<4, true>(o->type, (unsigned)n_tables << sc.bucket_bits, g->stream, g->d_descs, TableView{}, sc,
                                   parts, keys, (int)g->dim, g->elems, g->group, args, gs, &pool);
@@ -2593,11 +2628,12 @@ int32_t krk_group_push_pooled_parts(krk_group* g, const krk_optim* o, const krk_
   }
   GroupPooledSrc src;
   src.call = call;
-  src.bag_of = w.bag_of;
-  src.ratio = w.ratio;
-  src.weighted = weighted ? 1 : 0;
+  src.words = words;
+  src.bag_of = bag_of;
+  src.pooled = true;
+  src.weighted = weighted;
   const ReduceShape sh{g->dim, g->vec, g->elems, g->group};
   KRK_TRY(sort_and_reduce(sh, g->stream, g->scratch, TableView{}, o->type, total, gk.miss_key, gk.bits, nullptr, args,
-                          PooledSrc{nullptr, nullptr, nullptr}, &gs, &src, fill));
+                          PooledSrc{}, &gs, &src, fill));
   return group_finish(g, flags);
 }

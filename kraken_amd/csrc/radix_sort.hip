@@ -6,7 +6,7 @@
 // workgroups:
 //   1. radix_hist_kernel: every workgroup counts the digits of its tile of 4096 keys in LDS and
 //      writes the counts digit-major, hist[digit][tile];
-//   2. radix_scan_kernel: one wavefront per digit turns its row of counts into the number of
+//   2. radix_scan_kernel: one workgroup per digit turns its row of counts into the number of
 //      equal digits in earlier tiles, and notes the digit's total;
 //   3. radix_scatter_kernel: a workgroup scans the 512 totals in LDS (where each digit's output
 //      begins), ranks its tile's keys among equal digits in tile order (every wavefront finds the
@@ -58,7 +58,7 @@ __device__ __forceinline__ unsigned long long same_digit_n(uint32_t digit, int b
 // counter of a digit that many keys share: a request whose hottest row holds a quarter of the
 // ids spent 5.9 us here per pass for a million keys, 11.8 us for two million.)
 __global__ __launch_bounds__(kRsBlock) void radix_hist_kernel(const uint32_t* __restrict__ keys, int64_t n,
-                                                              int shift, int bits, int64_t tiles,
+                                                              int shift, int bits, int64_t pitch,
                                                               uint32_t* __restrict__ hist) {
   __shared__ uint32_t count[kRsDigits];
   const int t = threadIdx.x;
@@ -81,36 +81,73 @@ __global__ __launch_bounds__(kRsBlock) void radix_hist_kernel(const uint32_t* __
     if (live && (same & ((1ull << lane) - 1ull)) == 0ull) atomicAdd(&count[digit], (uint32_t)__popcll(same));
   }
   __syncthreads();
-  if (t <= (int)mask) hist[(int64_t)t * tiles + blockIdx.x] = count[t];
+  if (t <= (int)mask) {
+    uint32_t* row = hist + (int64_t)t * pitch;
+    row[blockIdx.x] = count[t];
+    if (blockIdx.x == gridDim.x - 1)
+      for (int64_t c = (int64_t)gridDim.x; c < pitch; ++c) row[c] = 0u;   // at most seven
+  }
 }
 
-// one wavefront per digit: hist[digit][0..tiles) -> exclusive prefix sums in place, total[digit]
-__global__ __launch_bounds__(256) void radix_scan_kernel(uint32_t* __restrict__ hist, int64_t tiles, int digits,
-                                                         uint32_t* __restrict__ total) {
-  const int digit = blockIdx.x * (256 / kWave) + threadIdx.x / kWave;
-  if (digit >= digits) return;                         // the whole wavefront
+// One workgroup per digit: hist[digit][0..tiles) -> exclusive prefix sums in place, total[digit].
+// A row is a dependent chain of trips to memory, so a trip takes 2048 tiles, eight a lane in two
+// 16-byte loads (rows are `pitch` counts apart, a multiple of eight, and zero behind the last tile);
+// one wavefront taking 64 tiles a trip walked the rows of 8.5 million keys for 20 us.
+constexpr int kScanLanes = 256;
+constexpr int kScanPer = 8;
+__global__ __launch_bounds__(kScanLanes) void radix_scan_kernel(uint32_t* __restrict__ hist, int64_t pitch,
+                                                                uint32_t* __restrict__ total) {
+  __shared__ uint32_t wave_total[kScanLanes / kWave];
   const int lane = threadIdx.x & (kWave - 1);
-  uint32_t* row = hist + (int64_t)digit * tiles;
+  const int wave = threadIdx.x / kWave;
+  uint4* row = reinterpret_cast<uint4*>(hist + (int64_t)blockIdx.x * pitch);
   uint32_t carry = 0;
-  for (int64_t c0 = 0; c0 < tiles; c0 += kWave) {
-    const int64_t c = c0 + lane;
-    const uint32_t v = c < tiles ? row[c] : 0u;
-    uint32_t incl = v;
+  for (int64_t c0 = 0; c0 < pitch; c0 += kScanLanes * kScanPer) {
+    const int64_t c = c0 + threadIdx.x * kScanPer;
+    const bool on = c < pitch;
+    uint32_t v[kScanPer] = {};
+    if (on) {
+      const uint4 x = row[c / 4], y = row[c / 4 + 1];
+      v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+      v[4] = y.x; v[5] = y.y; v[6] = y.z; v[7] = y.w;
+    }
+    uint32_t sum = 0;
+#pragma unroll
+    for (int i = 0; i < kScanPer; ++i) sum += v[i];
+    uint32_t incl = sum;
 #pragma unroll
     for (int d = 1; d < kWave; d <<= 1) {
       const uint32_t y = __shfl_up(incl, d);
       if (lane >= d) incl += y;
     }
-    if (c < tiles) row[c] = carry + incl - v;
-    carry += __shfl(incl, kWave - 1);
+    if (lane == kWave - 1) wave_total[wave] = incl;
+    __syncthreads();
+    uint32_t at = carry + incl - sum;
+#pragma unroll
+    for (int w = 0; w < kScanLanes / kWave; ++w) {
+      const uint32_t x = wave_total[w];
+      if (w < wave) at += x;
+      carry += x;
+    }
+    __syncthreads();                                   // the next trip writes wave_total
+    uint32_t r[kScanPer];
+#pragma unroll
+    for (int i = 0; i < kScanPer; ++i) {
+      r[i] = at;
+      at += v[i];
+    }
+    if (on) {
+      row[c / 4] = uint4{r[0], r[1], r[2], r[3]};
+      row[c / 4 + 1] = uint4{r[4], r[5], r[6], r[7]};
+    }
   }
-  if (lane == 0) total[digit] = carry;
+  if (threadIdx.x == 0) total[blockIdx.x] = carry;
 }
 
 template <int BITS>
 __global__ __launch_bounds__(kRsBlock) void radix_scatter_kernel(const uint32_t* __restrict__ keys,
                                                                  const uint32_t* __restrict__ vals, int64_t n,
-                                                                 int shift, int64_t tiles,
+                                                                 int shift, int64_t pitch,
                                                                  const uint32_t* __restrict__ hist,
                                                                  const uint32_t* __restrict__ total,
                                                                  uint32_t* __restrict__ keys_out,
@@ -154,7 +191,7 @@ __global__ __launch_bounds__(kRsBlock) void radix_scatter_kernel(const uint32_t*
   // where each digit's output begins (scan of the totals), plus what earlier tiles hold of it
   {
     const uint32_t offset = scan_digits(t < kDigits ? total[t] : 0u);   // its barrier: wave_hist is clear, too
-    if (t < kDigits) gbase[t] = offset + hist[(int64_t)t * tiles + blockIdx.x];
+    if (t < kDigits) gbase[t] = offset + hist[(int64_t)t * pitch + blockIdx.x];
   }
 #pragma unroll
   for (int i = 0; i < kRsItems; ++i) {
@@ -213,18 +250,21 @@ __global__ __launch_bounds__(kRsBlock) void radix_scatter_kernel(const uint32_t*
 }
 
 template <int BITS>
-void launch_scatter(const uint32_t* keys, const uint32_t* vals, int64_t n, int shift, int64_t tiles,
+void launch_scatter(const uint32_t* keys, const uint32_t* vals, int64_t n, int shift, int64_t tiles, int64_t pitch,
                     const uint32_t* hist, const uint32_t* total, uint32_t* keys_out, uint32_t* vals_out,
                     hipStream_t stream) {
   hipLaunchKernelGGL((radix_scatter_kernel<BITS>), dim3((unsigned)tiles), dim3(kRsBlock), 0, stream, keys, vals, n,
-                     shift, tiles, hist, total, keys_out, vals_out);
+                     shift, pitch, hist, total, keys_out, vals_out);
 }
+
+// counts between two digits' rows of the histogram
+int64_t hist_pitch(int64_t tiles) { return (tiles + kScanPer - 1) / kScanPer * kScanPer; }
 
 }  // namespace
 
 size_t radix_sort_work_bytes(int64_t n) {
   const int64_t tiles = (n + kRsTile - 1) / kRsTile;
-  return (size_t)(tiles + 1) * kRsDigits * sizeof(uint32_t);
+  return (size_t)(hist_pitch(tiles) + 1) * kRsDigits * sizeof(uint32_t);
 }
 
 int32_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt, int64_t n,
@@ -238,7 +278,8 @@ int32_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uin
     return KRK_E_CAPACITY;
   }
   uint32_t* hist = reinterpret_cast<uint32_t*>(work);
-  uint32_t* total = hist + tiles * kRsDigits;
+  const int64_t pitch = hist_pitch(tiles);
+  uint32_t* total = hist + pitch * kRsDigits;
   const int passes = (bits + kRsMaxBits - 1) / kRsMaxBits;
   const int width = (bits + passes - 1) / passes;      // 8 or 9 bits where that saves nothing else
   uint32_t* src_k = keys;
@@ -250,19 +291,18 @@ int32_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uin
     const int w = bits - shift < width ? bits - shift : width;
     const int digits = 1 << w;
     hipLaunchKernelGGL(radix_hist_kernel, dim3((unsigned)tiles), dim3(kRsBlock), 0, stream, src_k, n, shift, w,
-                       tiles, hist);
-    hipLaunchKernelGGL(radix_scan_kernel, dim3((unsigned)((digits + 3) / 4)), dim3(256), 0, stream, hist, tiles,
-                       digits, total);
+                       pitch, hist);
+    hipLaunchKernelGGL(radix_scan_kernel, dim3((unsigned)digits), dim3(kScanLanes), 0, stream, hist, pitch, total);
     switch (w) {
-      case 1: launch_scatter<1>(src_k, src_v, n, shift, tiles, hist, total, dst_k, dst_v, stream); break;
-      case 2: launch_scatter<2>(src_k, src_v, n, shift, tiles, hist, total, dst_k, dst_v, stream); break;
-      case 3: launch_scatter<3>(src_k, src_v, n, shift, tiles, hist, total, dst_k, dst_v, stream); break;
-      case 4: launch_scatter<4>(src_k, src_v, n, shift, tiles, hist, total, dst_k, dst_v, stream); break;
-      case 5: launch_scatter<5>(src_k, src_v, n, shift, tiles, hist, total, dst_k, dst_v, stream); break;
-      case 6: launch_scatter<6>(src_k, src_v, n, shift, tiles, hist, total, dst_k, dst_v, stream); break;
-      case 7: launch_scatter<7>(src_k, src_v, n, shift, tiles, hist, total, dst_k, dst_v, stream); break;
-      case 8: launch_scatter<8>(src_k, src_v, n, shift, tiles, hist, total, dst_k, dst_v, stream); break;
-      default: launch_scatter<9>(src_k, src_v, n, shift, tiles, hist, total, dst_k, dst_v, stream); break;
+      case 1: launch_scatter<1>(src_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream); break;
+      case 2: launch_scatter<2>(src_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream); break;
+      case 3: launch_scatter<3>(src_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream); break;
+      case 4: launch_scatter<4>(src_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream); break;
+      case 5: launch_scatter<5>(src_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream); break;
+      case 6: launch_scatter<6>(src_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream); break;
+      case 7: launch_scatter<7>(src_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream); break;
+      case 8: launch_scatter<8>(src_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream); break;
+      default: launch_scatter<9>(src_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream); break;
     }
     KRK_HIP(hipGetLastError());
     uint32_t* tk = src_k;
