@@ -8,8 +8,10 @@
 //
 // tau comes from a three-pass radix select over the bit patterns of |f| (non-negative floats
 // order like their bit patterns): 11 + 11 + 10 bits, each pass one LDS histogram per workgroup.
-// The emit step is a count pass, a scan of the per-tile counts and a write pass that recomputes
-// f, so the output order is the input order.
+// The emit step writes the pairs in input order. Where the caller's buffers hold whatever comes it is
+// one pass (emit_single_kernel); where the count decides whether anything may be written at all it is
+// a count pass, a scan of the per-tile counts and a write pass that recomputes f.
+#include <algorithm>
 #include <new>
 
 #include "krk_internal.h"
@@ -23,6 +25,9 @@ struct krk_dct : krk::ObjBase {
   int32_t* tile_counts = nullptr;
   int32_t* tile_offsets = nullptr;
   void* scan_tmp = nullptr;
+  unsigned long long* tile_state = nullptr;   // single-pass emit: what each tile announced
+  uint32_t* tickets = nullptr;   // single-pass emit: [0] next tile, [1] workgroups that are done
+  uint32_t emit_calls = 0;       // tags the announcements of one call
   uint32_t* host_sel = nullptr;  // pinned
   float tau = 0.0f;
   uint64_t step = 0;
@@ -201,128 +206,253 @@ __global__ __launch_bounds__(kCodecBlock) void emit_count_kernel(const float* __
   }
 }
 
-// Writes the kept (index, value) pairs in input order and the new residual. A tile's pairs are
-// first gathered in LDS in output order and then written out by consecutive lanes, so that the
-// index and value arrays are written in whole lines (a lane writing its own few kept elements
-// leaves partly written lines behind).
-__global__ __launch_bounds__(kCodecBlock) void emit_write_kernel(
-    const float* __restrict__ g, const float* __restrict__ e, int64_t n, int64_t tiles, bool vec,
-    const uint32_t* __restrict__ sel, const int32_t* __restrict__ tile_offsets,
-    const int32_t* __restrict__ tile_counts, long long* __restrict__ idx, float* __restrict__ val,
-    float* __restrict__ e_next) {
-  __shared__ int wave_sum[kCodecBlock / 64];
-  __shared__ uint16_t kept_at[kCodecTile];         // element's place inside the tile
-  __shared__ float kept_val[kCodecTile];
-  const uint32_t tau_bits = sel[2];
+// One tile of `ROWS` rows of 256 elements per wavefront: the kept (index, value) pairs in input order
+// and the new residual. announce(kept) is called once the tile's count is known, by every thread;
+// resolve() yields where the tile's pairs go, to every thread, and is asked for last, when everything
+// that does not depend on it is done. A tile's pairs are first gathered in LDS in output order
+// and then written out by consecutive lanes, so that the index and value arrays are written in whole
+// lines (a lane writing its own few kept elements leaves partly written lines behind).
+template <int BLOCK, int ROWS, typename Announce, typename Resolve>
+__device__ __forceinline__ void emit_tile(const float* __restrict__ g, const float* __restrict__ e, int64_t n,
+                                          int64_t tile, bool vec, uint32_t tau_bits, long long* __restrict__ idx,
+                                          float* __restrict__ val, float* __restrict__ e_next, Announce announce,
+                                          Resolve resolve) {
+  constexpr int kWaveElems = 256 * ROWS;
+  constexpr int kWaves = BLOCK / 64;
+  constexpr int kTile = kWaves * kWaveElems;
+  static_assert(kTile <= 65536, "a place inside the tile is kept in 16 bits");
+  __shared__ int wave_sum[kWaves];
+  __shared__ uint16_t kept_at[kTile];              // element's place inside the tile
+  __shared__ float kept_val[kTile];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const unsigned long long below = (1ull << lane) - 1ull;
-  for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-    const int local = wave * (64 * kCodecItems) + lane * 4;
-    const int64_t base = tile * kCodecTile + local;
-    Quad f[kCodecRows];
-    unsigned long long masks[kCodecRows][4];
-    int wave_total = 0;
-    {
-      Quad a[kCodecRows], b[kCodecRows];
+  const int local = wave * kWaveElems + lane * 4;
+  const int64_t base = tile * kTile + local;
+  Quad f[ROWS];
+  unsigned long long masks[ROWS][4];
+  int wave_total = 0;
+  {
+    Quad a[ROWS], b[ROWS];
 #pragma unroll
-      for (int r = 0; r < kCodecRows; ++r) {
-        a[r] = load_quad(g, base + r * 256, n, vec);
-        b[r] = load_quad(e, base + r * 256, n, true);
-      }
-#pragma unroll
-      for (int r = 0; r < kCodecRows; ++r) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          f[r].v[k] = a[r].v[k] + b[r].v[k];
-          masks[r][k] = __ballot(base + r * 256 + k < n && abs_bits(f[r].v[k]) >= tau_bits);
-          wave_total += __popcll(masks[r][k]);
-        }
-      }
+    for (int r = 0; r < ROWS; ++r) {
+      a[r] = load_quad(g, base + r * 256, n, vec);
+      b[r] = load_quad(e, base + r * 256, n, true);
     }
-    if (lane == 0) wave_sum[wave] = wave_total;
-    __syncthreads();
-    int off = 0;                                   // inside the tile's stretch of the output
 #pragma unroll
-    for (int w = 0; w < kCodecBlock / 64; ++w)
-      if (w < wave) off += wave_sum[w];
-#pragma unroll
-    for (int r = 0; r < kCodecRows; ++r) {
-      const int64_t j = base + r * 256;
-      // kept elements of lower lanes, all four components of each
-      int at = off;
-      int row_total = 0;
+    for (int r = 0; r < ROWS; ++r) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        at += __popcll(masks[r][k] & below);
-        row_total += __popcll(masks[r][k]);
+        f[r].v[k] = a[r].v[k] + b[r].v[k];
+        masks[r][k] = __ballot(base + r * 256 + k < n && abs_bits(f[r].v[k]) >= tau_bits);
+        wave_total += __popcll(masks[r][k]);
       }
-      float rest[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const bool keep = (masks[r][k] >> lane) & 1ull;
-        if (keep) {
-          kept_at[at] = (uint16_t)(local + r * 256 + k);
-          kept_val[at] = f[r].v[k];
-          ++at;
-        }
-        rest[k] = keep ? 0.0f : f[r].v[k];         // t/math.cc:1098-1123 : |x| < th keeps x
-      }
-      if (j + 3 < n) {
-        const vfloat4 out = {rest[0], rest[1], rest[2], rest[3]};
-        __builtin_nontemporal_store(out, reinterpret_cast<vfloat4*>(e_next + j));
-      } else {
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-          if (j + k < n) e_next[j + k] = rest[k];
-      }
-      off += row_total;
     }
+  }
+  if (lane == 0) wave_sum[wave] = wave_total;
+  __syncthreads();
+  int off = 0, count = 0;                          // inside the tile's stretch of the output
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    if (w < wave) off += wave_sum[w];
+    count += wave_sum[w];
+  }
+  announce(count);
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) {
+    const int64_t j = base + r * 256;
+    // kept elements of lower lanes, all four components of each
+    int at = off;
+    int row_total = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      at += __popcll(masks[r][k] & below);
+      row_total += __popcll(masks[r][k]);
+    }
+    float rest[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const bool keep = (masks[r][k] >> lane) & 1ull;
+      if (keep) {
+        kept_at[at] = (uint16_t)(local + r * 256 + k);
+        kept_val[at] = f[r].v[k];
+        ++at;
+      }
+      rest[k] = keep ? 0.0f : f[r].v[k];           // t/math.cc:1098-1123 : |x| < th keeps x
+    }
+    if (j + 3 < n) {
+      const vfloat4 out = {rest[0], rest[1], rest[2], rest[3]};
+      __builtin_nontemporal_store(out, reinterpret_cast<vfloat4*>(e_next + j));
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (j + k < n) e_next[j + k] = rest[k];
+    }
+    off += row_total;
+  }
+  const int64_t out0 = resolve(count);             // has a barrier: the pairs are in LDS
+  const int64_t tile_base = tile * kTile;
+  // (counted from a multiple of 64 of the output, so that a wavefront's stores are whole lines)
+  for (int i = (int)threadIdx.x - (int)(out0 & 63); i < count; i += BLOCK) {
+    if (i < 0) continue;
+    __builtin_nontemporal_store((long long)(tile_base + kept_at[i]), idx + out0 + i);
+    __builtin_nontemporal_store(kept_val[i], val + out0 + i);
+  }
+  __syncthreads();                                 // the next tile reuses the LDS arrays
+}
+
+__global__ __launch_bounds__(kCodecBlock) void emit_write_kernel(
+    const float* __restrict__ g, const float* __restrict__ e, int64_t n, int64_t tiles, bool vec,
+    const uint32_t* __restrict__ sel, const int32_t* __restrict__ tile_offsets, long long* __restrict__ idx,
+    float* __restrict__ val, float* __restrict__ e_next) {
+  const uint32_t tau_bits = sel[2];
+  for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x)
+    emit_tile<kCodecBlock, kCodecRows>(g, e, n, tile, vec, tau_bits, idx, val, e_next, [](int) {},
+                          [&](int) -> int64_t {
+                            __syncthreads();
+                            return tile_offsets[tile];
+                          });
+}
+
+// The whole emit step in one pass: gradient and residual are read once (a count pass ahead of the
+// write pass read them twice: 536 MB more for 67 million elements, 95 of 333 us with the scan). Where
+// a tile's pairs go is the number of pairs in the tiles before it, which the workgroups tell one
+// another: tile_state[t] holds what tile t keeps as soon as that is known, and what tiles 0..t keep
+// together once that is. A tile looks back over its predecessors, 64 at a time, as far as the nearest
+// whose total is known.
+// Tiles are handed out by a counter in ascending order, so every predecessor of a tile is held by a
+// workgroup that already runs, and it announces its count before it waits for anything: every wait
+// ends. An announcement carries the number of the call, so the array is never cleared; the last
+// workgroup to leave puts the counter back to zero.
+// Tiles of 8192: the counter serves one workgroup after the other, some 15 ns each, which is what
+// smaller tiles wait for (67 million elements: 427 us in tiles of 2048, 297 us in tiles of 4096).
+constexpr int kSingleBlock = 512;
+constexpr int kSingleRows = 4;
+constexpr int kSingleTile = (kSingleBlock / 64) * 256 * kSingleRows;
+constexpr int kSingleGrid = 512;
+constexpr uint32_t kTileCount = 1u, kTileTotal = 2u;   // what the low word is: the tile's own count, or all up to it
+constexpr uint32_t kMaxEmitCalls = 1u << 30;
+
+__device__ __forceinline__ void tell(unsigned long long* state, uint32_t call, uint32_t what, uint32_t value) {
+  __hip_atomic_store(state, ((unsigned long long)(call << 2 | what) << 32) | value, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ __launch_bounds__(kSingleBlock) void emit_single_kernel(
+    const float* __restrict__ g, const float* __restrict__ e, int64_t n, uint32_t tiles, bool vec,
+    uint32_t* __restrict__ sel, unsigned long long* tile_state, uint32_t* tickets, uint32_t call,
+    long long* __restrict__ idx, float* __restrict__ val, float* __restrict__ e_next,
+    uint32_t* __restrict__ host_sel) {
+  __shared__ uint32_t s_tile, s_before;
+  const uint32_t tau_bits = sel[2];
+  const int lane = threadIdx.x & 63;
+  for (;;) {
+    if (threadIdx.x == 0) s_tile = atomicAdd(&tickets[0], 1u);
     __syncthreads();
-    const int count = tile_counts[tile];
-    const int64_t out0 = tile_offsets[tile];
-    const int64_t tile_base = tile * kCodecTile;
-    for (int i = threadIdx.x; i < count; i += kCodecBlock) {
-      __builtin_nontemporal_store((long long)(tile_base + kept_at[i]), idx + out0 + i);
-      __builtin_nontemporal_store(kept_val[i], val + out0 + i);
-    }
-    __syncthreads();                               // the next tile reuses the LDS arrays
+    const uint32_t tile = s_tile;
+    if (tile >= tiles) break;                      // the whole workgroup
+    emit_tile<kSingleBlock, kSingleRows>(
+        g, e, n, tile, vec, tau_bits, idx, val, e_next,
+        [&](int count) {
+          if (threadIdx.x == 0) tell(&tile_state[tile], call, tile == 0 ? kTileTotal : kTileCount, (uint32_t)count);
+        },
+        [&](int count) -> int64_t {
+          if (threadIdx.x < 64) {
+            uint32_t before = 0;
+            int64_t base = (int64_t)tile - 1;      // lane l looks at tile base - l
+            bool more = tile > 0;
+            while (more) {
+              const int64_t j = base - lane;
+              unsigned long long word = (unsigned long long)(call << 2 | kTileTotal) << 32;   // before the first tile: nothing
+              if (j >= 0) word = __hip_atomic_load(&tile_state[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              const uint32_t tag = (uint32_t)(word >> 32);
+              const unsigned long long known = __ballot(tag == (call << 2 | kTileTotal));
+              const unsigned long long open = __ballot((tag >> 2) != call);
+              const int last = known ? __ffsll(known) - 1 : 63;   // the farthest tile that counts
+              const unsigned long long need = last == 63 ? ~0ull : ((1ull << (last + 1)) - 1ull);
+              if (open & need) {                   // one of them has not announced yet
+                __builtin_amdgcn_s_sleep(1);
+                continue;
+              }
+              uint32_t v = lane <= last ? (uint32_t)word : 0u;
+#pragma unroll
+              for (int d = 32; d > 0; d >>= 1) v += __shfl_down(v, d, 64);
+              before += __shfl(v, 0);
+              more = known == 0ull;
+              base -= 64;
+            }
+            if (threadIdx.x == 0) {
+              if (tile > 0) tell(&tile_state[tile], call, kTileTotal, before + (uint32_t)count);
+              s_before = before;
+              if (tile == tiles - 1) {             // the count and the threshold, where the host reads them
+                sel[3] = before + (uint32_t)count;
+                host_sel[2] = tau_bits;
+                host_sel[3] = before + (uint32_t)count;
+              }
+            }
+          }
+          __syncthreads();
+          return s_before;
+        });
+  }
+  if (threadIdx.x == 0 && atomicAdd(&tickets[1], 1u) == gridDim.x - 1) {
+    __hip_atomic_store(&tickets[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&tickets[1], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
-
 // ---- densify in one pass over the output ------------------------------------------------------
-constexpr int kTileElems = 4096;                 // floats of one output tile: 16 KB of LDS
-constexpr int64_t kTiledFrom = 1 << 22;          // smaller tensors: zero + scatter, two launches are quicker
-constexpr uint32_t kNoStart = 0xFFFFFFFFu;
-
-__global__ __launch_bounds__(kCodecBlock) void coo_tiles_init_kernel(uint32_t* __restrict__ starts, int64_t tiles,
-                                                                     uint32_t* __restrict__ unordered) {
-  const int64_t i = (int64_t)blockIdx.x * kCodecBlock + threadIdx.x;
-  if (i < tiles) starts[i] = kNoStart;
-  if (i == 0) *unordered = 0u;
-}
-
-// starts[T] / ends[T] = the entries whose index lies in tile T (ends is only read where starts is
-// set); *unordered is raised when the indices do not ascend strictly or leave [0, n).
+// Where each tile's entries begin: the first entry of a tile, and the first one behind the empty
+// tiles before it, name themselves. A wavefront takes 256 entries in two rows of 128, a lane two
+// neighbours of each in one 16-byte load (whole lines an access); the entry before a lane's two is
+// its neighbour's second.
 __global__ __launch_bounds__(kCodecBlock) void coo_tiles_bounds_kernel(const long long* __restrict__ idx,
-                                                                       int64_t nnz, int64_t n,
-                                                                       uint32_t* __restrict__ starts,
-                                                                       uint32_t* __restrict__ ends,
-                                                                       uint32_t* __restrict__ unordered) {
-  const int64_t step = (int64_t)gridDim.x * kCodecBlock;
-  for (int64_t j = (int64_t)blockIdx.x * kCodecBlock + threadIdx.x; j < nnz; j += step) {
-    const long long cur = __builtin_nontemporal_load(idx + j);
-    const long long prev = j ? idx[j - 1] : -1;
-    if (cur <= prev || cur >= n) {
-      atomicOr(unordered, 1u);
-    } else {
-      if (prev < 0 || cur / kTileElems != prev / kTileElems) {
-        starts[cur / kTileElems] = (uint32_t)j;
-        if (prev >= 0) ends[prev / kTileElems] = (uint32_t)j;
+                                                                       int64_t nnz, int64_t n, bool vec, CooTiles out) {
+  typedef long long pair __attribute__((ext_vector_type(2)));
+  constexpr int kRows = 2;
+  const int lane = threadIdx.x & 63;
+  const int64_t step = (int64_t)gridDim.x * (kCodecBlock / 64) * (kRows * 128);
+  for (int64_t base = ((int64_t)blockIdx.x * (kCodecBlock / 64) + threadIdx.x / 64) * (kRows * 128); base < nnz;
+       base += step) {                               // a wavefront's lanes stay together
+    pair cur[kRows];
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+      const int64_t j = base + r * 128 + lane * 2;
+      if (vec && j + 1 < nnz) {
+        cur[r] = __builtin_nontemporal_load(reinterpret_cast<const pair*>(idx + j));
+      } else {
+        cur[r][0] = idx[j < nnz ? j : nnz - 1];
+        cur[r][1] = idx[j + 1 < nnz ? j + 1 : nnz - 1];
       }
-      if (j == nnz - 1) ends[cur / kTileElems] = (uint32_t)nnz;
     }
+    long long last = base ? idx[base - 1] : -1;      // the entry before the row
+    bool bad = false;
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+      const int64_t j = base + r * 128 + lane * 2;
+      long long prev = __shfl_up(cur[r][1], 1);
+      if (lane == 0) prev = last;
+      last = __shfl(cur[r][1], 63);
+      // nearly every lane: two more entries of the tile the one before is in
+      if (j + 2 < nnz && prev >= 0 && prev < cur[r][0] && cur[r][0] < cur[r][1] && cur[r][1] < n &&
+          (prev ^ cur[r][1]) < kCooTile)
+        continue;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        if (j + i >= nnz) continue;
+        const long long c = cur[r][i];
+        const bool wrong = c <= prev || c >= n;
+        bad = bad || wrong;
+        if (!wrong) {
+          const int64_t mine = c / kCooTile;
+          for (int64_t t = prev < 0 ? 0 : prev / kCooTile + 1; t <= mine; ++t) out.starts[t] = (uint32_t)(j + i);
+          if (j + i == nnz - 1)
+            for (int64_t t = mine + 1; t <= (int64_t)out.tiles; ++t) out.starts[t] = (uint32_t)nnz;
+        }
+        prev = c;
+      }
+    }
+    if (bad) __hip_atomic_store(out.unordered, out.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -330,42 +460,38 @@ __global__ __launch_bounds__(kCodecBlock) void coo_tiles_bounds_kernel(const lon
 // whose range is known, so their loads do not wait for one another) and leaves in whole lines,
 // past the caches.
 __global__ __launch_bounds__(kCodecBlock) void coo_tiles_write_kernel(const long long* __restrict__ idx,
-                                                                      const float* __restrict__ val, int64_t nnz,
+                                                                      const float* __restrict__ val,
                                                                       float* __restrict__ dense, int64_t n,
-                                                                      const uint32_t* __restrict__ starts,
-                                                                      const uint32_t* __restrict__ ends,
-                                                                      const uint32_t* __restrict__ unordered) {
-  if (*unordered) return;                        // the scatter launches that follow do the work
-  __shared__ __align__(16) float tile[kTileElems];
-  const int64_t base = (int64_t)blockIdx.x * kTileElems;
-  const uint32_t start = starts[blockIdx.x];
-  const uint32_t end = start != kNoStart ? ends[blockIdx.x] : 0u;
-  for (int i = threadIdx.x; i < kTileElems / 4; i += kCodecBlock)
+                                                                      CooTiles tiles) {
+  if (coo_unordered(tiles)) return;              // the scatter launches that follow do the work
+  __shared__ __align__(16) float tile[kCooTile];
+  const int64_t base = (int64_t)blockIdx.x * kCooTile;
+  const uint32_t start = tiles.starts[blockIdx.x];
+  const uint32_t end = tiles.starts[blockIdx.x + 1];
+  for (int i = threadIdx.x; i < kCooTile / 4; i += kCodecBlock)
     reinterpret_cast<float4*>(tile)[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   __syncthreads();
-  if (start != kNoStart) {
-    for (int64_t j0 = (int64_t)start + threadIdx.x; j0 < (int64_t)end; j0 += 4 * kCodecBlock) {
-      long long at[4];
-      float v[4];
+  for (int64_t j0 = (int64_t)start + threadIdx.x; j0 < (int64_t)end; j0 += 4 * kCodecBlock) {
+    long long at[4];
+    float v[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int64_t j = j0 + u * kCodecBlock;
-        if (j < (int64_t)end) {
-          at[u] = __builtin_nontemporal_load(idx + j);
-          v[u] = __builtin_nontemporal_load(val + j);
-        }
+    for (int u = 0; u < 4; ++u) {
+      const int64_t j = j0 + u * kCodecBlock;
+      if (j < (int64_t)end) {
+        at[u] = __builtin_nontemporal_load(idx + j);
+        v[u] = __builtin_nontemporal_load(val + j);
       }
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (j0 + u * kCodecBlock < (int64_t)end) tile[at[u] - base] = v[u];
     }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (j0 + u * kCodecBlock < (int64_t)end) tile[at[u] - base] = v[u];
   }
   __syncthreads();
   const int64_t left = n - base;
-  const int cnt = left < kTileElems ? (int)left : kTileElems;
-  if (cnt == kTileElems && (((uintptr_t)dense) & 15) == 0) {
+  const int cnt = left < kCooTile ? (int)left : kCooTile;
+  if (cnt == kCooTile && (((uintptr_t)dense) & 15) == 0) {
     typedef float tile4 __attribute__((ext_vector_type(4)));
-    for (int i = threadIdx.x; i < kTileElems / 4; i += kCodecBlock)
+    for (int i = threadIdx.x; i < kCooTile / 4; i += kCodecBlock)
       __builtin_nontemporal_store(reinterpret_cast<const tile4*>(tile)[i], reinterpret_cast<tile4*>(dense + base) + i);
   } else {
     for (int i = threadIdx.x; i < cnt; i += kCodecBlock) dense[base + i] = tile[i];
@@ -373,26 +499,23 @@ __global__ __launch_bounds__(kCodecBlock) void coo_tiles_write_kernel(const long
 }
 
 __global__ __launch_bounds__(kCodecBlock) void coo_zero_if_kernel(float* __restrict__ dense, int64_t n,
-                                                                  const uint32_t* __restrict__ unordered) {
-  if (!*unordered) return;
+                                                                  CooTiles tiles) {
+  if (!coo_unordered(tiles)) return;
   const int64_t step = (int64_t)gridDim.x * kCodecBlock;
   for (int64_t i = (int64_t)blockIdx.x * kCodecBlock + threadIdx.x; i < n; i += step) dense[i] = 0.0f;
 }
 
-// dense[idx[j]] += val[j]; repeated indices add up (t/math.cc:1043). unordered null: always.
+// dense[idx[j]] += val[j]; repeated indices add up (t/math.cc:1043), indices outside [0, n) are
+// skipped. IF: only where the tiles were found to be unordered.
+template <bool IF>
 __global__ __launch_bounds__(kCodecBlock) void coo_add_kernel(const long long* __restrict__ idx,
                                                               const float* __restrict__ val, int64_t nnz,
-                                                              float* __restrict__ dense, int64_t n,
-                                                              const uint32_t* __restrict__ unordered,
-                                                              uint32_t* __restrict__ err) {
-  if (unordered && !*unordered) return;
+                                                              float* __restrict__ dense, int64_t n, CooTiles tiles) {
+  if (IF && !coo_unordered(tiles)) return;
   const int64_t step = (int64_t)gridDim.x * kCodecBlock;
   for (int64_t j = (int64_t)blockIdx.x * kCodecBlock + threadIdx.x; j < nnz; j += step) {
     const long long i = idx[j];
-    if (i < 0 || i >= n) {
-      if (err) atomicOr(err, 1u);
-      continue;
-    }
+    if (i < 0 || i >= n) continue;
     unsafeAtomicAdd(&dense[i], val[j]);   // hardware fp32 add, no CAS loop
   }
 }
@@ -404,43 +527,63 @@ static unsigned stream_grid(int64_t n) {
   return (unsigned)blocks;
 }
 
-size_t coo_densify_work_bytes(int64_t n) {
-  return (2 * (size_t)((n + kTileElems - 1) / kTileElems) + 4) * sizeof(uint32_t);
+int32_t coo_find_tiles(CooWork* work, const long long* d_idx, int64_t nnz, int64_t n, CooTiles* out,
+                       hipStream_t stream) {
+  const int64_t tiles = (n + kCooTile - 1) / kCooTile;
+  const size_t before = work->buffer.bytes;
+  KRK_TRY(work->buffer.reserve((size_t)(tiles + 2) * sizeof(uint32_t)));
+  out->unordered = work->buffer.as<uint32_t>();
+  out->starts = out->unordered + 1;
+  out->tiles = (uint32_t)tiles;
+  if (!work->host_unordered) {
+    KRK_HIP(hipHostMalloc((void**)&work->host_unordered, 64, hipHostMallocDefault));
+    *work->host_unordered = 0u;
+  }
+  KRK_HIP(hipHostGetDevicePointer((void**)&out->host_unordered, work->host_unordered, 0));
+  // a fresh buffer holds no tag, and one that says 0 is never handed out
+  if (work->buffer.bytes != before || work->calls == 0xFFFFFFFFu) {
+    KRK_HIP(hipMemsetAsync(out->unordered, 0, sizeof(uint32_t), stream));
+    *work->host_unordered = 0u;
+    work->calls = 0;
+  }
+  out->tag = ++work->calls;
+  const bool vec = ((uintptr_t)d_idx & 15) == 0;
+  hipLaunchKernelGGL(coo_tiles_bounds_kernel, dim3(stream_grid((nnz + 3) / 4)), dim3(kCodecBlock), 0, stream, d_idx,
+                     nnz, n, vec, *out);
+  KRK_HIP(hipGetLastError());
+  return KRK_SUCCESS;
 }
 
-int32_t coo_densify(const long long* d_idx, const float* d_val, int64_t nnz, float* d_dense, int64_t n,
-                    void* work, uint32_t* err, hipStream_t stream) {
+// A few workgroups that stride over the entries: when the tiles did the work they only look at the
+// flag and leave (2048 of them took 4.7 us a launch for that).
+static dim3 rare_grid(int64_t n) { return dim3(std::min(stream_grid(n), 512u)); }
+
+int32_t coo_scatter_if_unordered(const CooTiles& tiles, const long long* d_idx, const float* d_val, int64_t nnz,
+                                 float* d_dense, int64_t n, hipStream_t stream) {
+  const dim3 block(kCodecBlock);
+  hipLaunchKernelGGL(coo_zero_if_kernel, rare_grid(n), block, 0, stream, d_dense, n, tiles);
+  hipLaunchKernelGGL(coo_add_kernel<true>, rare_grid(nnz), block, 0, stream, d_idx, d_val, nnz, d_dense, n, tiles);
+  KRK_HIP(hipGetLastError());
+  return KRK_SUCCESS;
+}
+
+int32_t coo_densify(CooWork* work, const long long* d_idx, const float* d_val, int64_t nnz, float* d_dense, int64_t n,
+                    hipStream_t stream) {
   if (n <= 0) return KRK_SUCCESS;
   const dim3 block(kCodecBlock);
-  const unsigned per_entry = (unsigned)((nnz + kCodecBlock - 1) / kCodecBlock);
-  if (n < kTiledFrom || nnz >= ((int64_t)1 << 31) || !work) {
+  if (!coo_tiled(n, nnz) || nnz == 0) {
     KRK_HIP(hipMemsetAsync(d_dense, 0, (size_t)n * sizeof(float), stream));   // t/math.cc:1066 dense.Zero()
     if (nnz)
-      hipLaunchKernelGGL(coo_add_kernel, dim3(per_entry), block, 0, stream, d_idx, d_val, nnz, d_dense, n,
-                         (const uint32_t*)nullptr, err);
+      hipLaunchKernelGGL(coo_add_kernel<false>, dim3((unsigned)((nnz + kCodecBlock - 1) / kCodecBlock)), block, 0,
+                         stream, d_idx, d_val, nnz, d_dense, n, CooTiles{});
     KRK_HIP(hipGetLastError());
     return KRK_SUCCESS;
   }
-  const int64_t tiles = (n + kTileElems - 1) / kTileElems;
-  uint32_t* starts = reinterpret_cast<uint32_t*>(work);
-  uint32_t* ends = starts + tiles;
-  uint32_t* unordered = ends + tiles;
-  hipLaunchKernelGGL(coo_tiles_init_kernel, dim3((unsigned)((tiles + kCodecBlock - 1) / kCodecBlock)), block, 0,
-                     stream, starts, tiles, unordered);
-  if (nnz)
-    hipLaunchKernelGGL(coo_tiles_bounds_kernel, dim3(stream_grid(nnz)), block, 0, stream, d_idx, nnz, n, starts,
-                       ends, unordered);
-  hipLaunchKernelGGL(coo_tiles_write_kernel, dim3((unsigned)tiles), block, 0, stream, d_idx, d_val, nnz, d_dense,
-                     n, starts, ends, unordered);
-  if (nnz) {
-    hipLaunchKernelGGL(coo_zero_if_kernel, dim3(stream_grid(n)), block, 0, stream, d_dense, n, unordered);
-    // a few workgroups that stride over the entries: when the tiles did the work they only look at
-    // the flag and leave
-    hipLaunchKernelGGL(coo_add_kernel, dim3(stream_grid(nnz)), block, 0, stream, d_idx, d_val, nnz, d_dense, n,
-                       (const uint32_t*)unordered, err);
-  }
+  CooTiles tiles;
+  KRK_TRY(coo_find_tiles(work, d_idx, nnz, n, &tiles, stream));
+  hipLaunchKernelGGL(coo_tiles_write_kernel, dim3(tiles.tiles), block, 0, stream, d_idx, d_val, d_dense, n, tiles);
   KRK_HIP(hipGetLastError());
-  return KRK_SUCCESS;
+  return coo_scatter_if_unordered(tiles, d_idx, d_val, nnz, d_dense, n, stream);
 }
 
 }  // namespace krk
@@ -448,7 +591,7 @@ int32_t coo_densify(const long long* d_idx, const float* d_val, int64_t nnz, flo
 using namespace krk;
 
 static std::mutex g_densify_mu;          // krk_coo_to_dense owns no object: one shared work buffer
-static DeviceBuffer g_densify_work;
+static CooWork g_densify_work;
 
 extern "C" {
 
@@ -470,6 +613,11 @@ int32_t krk_dct_create(int64_t n, krk_dct** out) {
     if (e == hipSuccess) e = hipMalloc((void**)&s->tile_counts, (size_t)s->tiles * sizeof(int32_t));
     if (e == hipSuccess) e = hipMalloc((void**)&s->tile_offsets, (size_t)s->tiles * sizeof(int32_t));
     if (e == hipSuccess) e = hipMalloc(&s->scan_tmp, scan_scratch_bytes(s->tiles));
+    const size_t state_b = (size_t)((n + kSingleTile - 1) / kSingleTile + 1) * sizeof(unsigned long long);
+    if (e == hipSuccess) e = hipMalloc((void**)&s->tile_state, state_b);
+    if (e == hipSuccess) e = hipMalloc((void**)&s->tickets, 64);
+    if (e == hipSuccess) e = hipMemsetAsync(s->tile_state, 0, state_b, s->stream);
+    if (e == hipSuccess) e = hipMemsetAsync(s->tickets, 0, 64, s->stream);
     if (e == hipSuccess) e = hipHostMalloc((void**)&s->host_sel, 64, hipHostMallocDefault);
     if (e == hipSuccess) e = hipMemsetAsync(s->e, 0, nb, s->stream);   // dct_emitter.cc:54 : val.Clone().Zero()
     if (e == hipSuccess) e = hipMemsetAsync(s->sel, 0, 64, s->stream);
@@ -495,6 +643,8 @@ int32_t krk_dct_destroy(krk_dct* s) {
   if (s->tile_counts) (void)hipFree(s->tile_counts);
   if (s->tile_offsets) (void)hipFree(s->tile_offsets);
   if (s->scan_tmp) (void)hipFree(s->scan_tmp);
+  if (s->tile_state) (void)hipFree(s->tile_state);
+  if (s->tickets) (void)hipFree(s->tickets);
   if (s->host_sel) (void)hipHostFree(s->host_sel);
   s->close_stream();
   delete s;
@@ -539,28 +689,33 @@ int32_t krk_dct_compress(krk_dct* s, const float* grad, uint64_t life_span, floa
     KRK_HIP(hipGetLastError());
   }
   const bool vec = ((uintptr_t)d_g & 15) == 0;
-  const unsigned emit_grid = (unsigned)(s->tiles < kCodecGrid ? s->tiles : kCodecGrid);
-  hipLaunchKernelGGL(emit_count_kernel, dim3(emit_grid), dim3(kCodecBlock), 0, s->stream, d_g, s->e, n,
-                     s->tiles, vec, s->sel, s->tile_counts);
-  KRK_HIP(hipGetLastError());
-  KRK_TRY(exclusive_scan_i32(s->tile_counts, s->tile_offsets, s->tiles,
-                             reinterpret_cast<int32_t*>(s->sel + 3), s->scan_tmp, s->stream));
-  const unsigned emit_blocks = emit_grid;
-  // Room for every element and device buffers: nothing can overflow and nothing is staged, so the
-  // write pass follows at once and the count is read back once, at the end.
-  const bool sure = (flags & KRK_DEVICE_PTRS) && capacity >= n;
-  if (sure) {
-    hipLaunchKernelGGL(emit_write_kernel, dim3(emit_blocks), dim3(kCodecBlock), 0, s->stream, d_g, s->e, n,
-                       s->tiles, vec, s->sel, s->tile_offsets, s->tile_counts, reinterpret_cast<long long*>(idx),
-                       val, s->e_next);
+  // Room for every element and device buffers: nothing can overflow and nothing is staged, so one
+  // pass emits and the count comes with it.
+  if ((flags & KRK_DEVICE_PTRS) && capacity >= n) {
+    const int64_t tiles = (n + kSingleTile - 1) / kSingleTile;
+    if (++s->emit_calls == kMaxEmitCalls) {
+      KRK_HIP(hipMemsetAsync(s->tile_state, 0, (size_t)tiles * sizeof(unsigned long long), s->stream));
+      s->emit_calls = 1;
+    }
+    uint32_t* d_host_sel = nullptr;
+    KRK_HIP(hipHostGetDevicePointer((void**)&d_host_sel, s->host_sel, 0));
+    hipLaunchKernelGGL(emit_single_kernel, dim3((unsigned)(tiles < kSingleGrid ? tiles : kSingleGrid)),
+                       dim3(kSingleBlock), 0, s->stream, d_g, s->e, n, (uint32_t)tiles, vec, s->sel, s->tile_state,
+                       s->tickets, s->emit_calls, reinterpret_cast<long long*>(idx), val, s->e_next, d_host_sel);
     KRK_HIP(hipGetLastError());
-  }
-  KRK_HIP(hipMemcpyAsync(s->host_sel, s->sel, 16, hipMemcpyDeviceToHost, s->stream));
-  KRK_HIP(hipStreamSynchronize(s->stream));
-  const int64_t count = (int64_t)s->host_sel[3];
-  const float new_tau = __builtin_bit_cast(float, s->host_sel[2]);
-  *nnz = count;
-  if (!sure) {
+    KRK_HIP(hipStreamSynchronize(s->stream));
+    *nnz = (int64_t)s->host_sel[3];
+  } else {
+    const dim3 emit_grid((unsigned)(s->tiles < kCodecGrid ? s->tiles : kCodecGrid));
+    hipLaunchKernelGGL(emit_count_kernel, emit_grid, dim3(kCodecBlock), 0, s->stream, d_g, s->e, n, s->tiles, vec,
+                       s->sel, s->tile_counts);
+    KRK_HIP(hipGetLastError());
+    KRK_TRY(exclusive_scan_i32(s->tile_counts, s->tile_offsets, s->tiles,
+                               reinterpret_cast<int32_t*>(s->sel + 3), s->scan_tmp, s->stream));
+    KRK_HIP(hipMemcpyAsync(s->host_sel, s->sel, 16, hipMemcpyDeviceToHost, s->stream));
+    KRK_HIP(hipStreamSynchronize(s->stream));
+    const int64_t count = (int64_t)s->host_sel[3];
+    *nnz = count;
     if (count > capacity) {
       // nothing was committed: restore the threshold the next call will see
       if (reselect) {
@@ -576,13 +731,14 @@ int32_t krk_dct_compress(krk_dct* s, const float* grad, uint64_t life_span, floa
     float* d_val;
     KRK_TRY(s->output(reinterpret_cast<long long*>(idx), (size_t)count, flags, 1, &d_idx));
     KRK_TRY(s->output(val, (size_t)count, flags, 2, &d_val));
-    hipLaunchKernelGGL(emit_write_kernel, dim3(emit_blocks), dim3(kCodecBlock), 0, s->stream, d_g, s->e, n,
-                       s->tiles, vec, s->sel, s->tile_offsets, s->tile_counts, d_idx, d_val, s->e_next);
+    hipLaunchKernelGGL(emit_write_kernel, emit_grid, dim3(kCodecBlock), 0, s->stream, d_g, s->e, n,
+                       s->tiles, vec, s->sel, s->tile_offsets, d_idx, d_val, s->e_next);
     KRK_HIP(hipGetLastError());
     KRK_TRY(s->output_back(reinterpret_cast<long long*>(idx), (size_t)count, flags, 1));
     KRK_TRY(s->output_back(val, (size_t)count, flags, 2));
     KRK_HIP(hipStreamSynchronize(s->stream));
   }
+  const float new_tau = __builtin_bit_cast(float, s->host_sel[2]);
   float* tmp = s->e;
   s->e = s->e_next;
   s->e_next = tmp;
@@ -651,10 +807,9 @@ int32_t krk_coo_to_dense(const int64_t* idx, const float* val, int64_t nnz, floa
   hipError_t e = hipSuccess;
   {
     std::lock_guard<std::mutex> lk(g_densify_mu);
-    int32_t rc = g_densify_work.reserve(coo_densify_work_bytes(n));
-    if (rc == KRK_SUCCESS) rc = coo_densify(d_idx, d_val, nnz, d_dense, n, g_densify_work.ptr, nullptr, st);
+    const int32_t rc = coo_densify(&g_densify_work, d_idx, d_val, nnz, d_dense, n, st);
     // the shared work buffer is free for the next caller once this call's launches are done
-    if (rc == KRK_SUCCESS && n >= kTiledFrom) e = hipStreamSynchronize(st);
+    if (rc == KRK_SUCCESS && n >= kCooTiledFrom) e = hipStreamSynchronize(st);
     if (rc != KRK_SUCCESS) {
       if (tmp) (void)hipFree(tmp);
       return rc;

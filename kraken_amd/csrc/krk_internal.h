@@ -346,13 +346,38 @@ __device__ __forceinline__ void optim_element(const OptimK& k, float lr, float g
 // out[i] = sum(in[0..i)), total written to *total_out (device). in/out may alias.
 // CooTensorImpl::ToDense (t/coo_tensor_impl.cc:250-260, t/math.cc:1006-1096) on the device:
 // dense[0, n) = 0, then dense[idx[j]] += val[j]. Large tensors whose indices ascend strictly and
-// lie in range (what ToCoo produces) are written tile by tile in one pass over the output; any
-// other input is zeroed and scattered into, decided on the device inside the same launches.
-// work holds coo_densify_work_bytes(n); err (may be null) gets bit 0 set when an index is out
-// of range.
-size_t coo_densify_work_bytes(int64_t n);
-int32_t coo_densify(const long long* d_idx, const float* d_val, int64_t nnz, float* d_dense, int64_t n,
-                    void* work, uint32_t* err, hipStream_t stream);
+// lie in range (what ToCoo produces) are taken tile by tile: one launch over the indices finds
+// where each tile's entries begin (coo_find_tiles), and whoever walks the tiles puts one together
+// in LDS. Any other input is zeroed and scattered into; which of the two it is is decided on the
+// device, and the launches of the other way look at the flag and leave.
+constexpr int kCooTile = 2048;                   // floats of one tile: 8 KB of LDS
+constexpr int64_t kCooTiledFrom = 1 << 22;       // smaller tensors: zero + scatter, two launches are quicker
+struct CooTiles {
+  uint32_t* starts;       // [tiles + 1]: tile t owns entries [starts[t], starts[t + 1])
+  uint32_t* unordered;    // == tag: the indices do not ascend strictly or leave [0, n)
+  uint32_t tag;
+  uint32_t tiles;
+  uint32_t* host_unordered;   // page-locked copy of the flag, raised by who walks the tiles
+};
+__device__ __forceinline__ bool coo_unordered(const CooTiles& t) { return *t.unordered == t.tag; }
+struct CooWork {          // work space of one caller, kept between calls
+  DeviceBuffer buffer;
+  uint32_t calls = 0;
+  uint32_t* host_unordered = nullptr;
+  void release() {
+    buffer.release();
+    if (host_unordered) (void)hipHostFree(host_unordered);
+    host_unordered = nullptr;
+  }
+};
+inline bool coo_tiled(int64_t n, int64_t nnz) { return n >= kCooTiledFrom && nnz < ((int64_t)1 << 31); }
+int32_t coo_find_tiles(CooWork* work, const long long* d_idx, int64_t nnz, int64_t n, CooTiles* out,
+                       hipStream_t stream);
+// What is left to do where the indices are unordered, and nothing otherwise: dense = the entries' sums.
+int32_t coo_scatter_if_unordered(const CooTiles& tiles, const long long* d_idx, const float* d_val, int64_t nnz,
+                                 float* d_dense, int64_t n, hipStream_t stream);
+int32_t coo_densify(CooWork* work, const long long* d_idx, const float* d_val, int64_t nnz, float* d_dense, int64_t n,
+                    hipStream_t stream);
 
 // Stable radix sort of n (key, payload) pairs by the low `bits` bits of the key (radix_sort.hip).
 // keys / vals are overwritten; keys_alt / vals_alt hold n entries each; work holds

@@ -156,6 +156,46 @@ def test_codec_device_pointers_and_capacity(api, oracle):
     assert np.array_equal(bag.residual, ref.residual)
 
 
+@pytest.mark.parametrize("n", [256, 8191, 8192, 8193, 600_001, 9_000_001])
+@pytest.mark.parametrize("eta", [0.02, 0.75, 0.99])
+def test_codec_single_pass_emit(api, oracle, n, eta):
+    """Device buffers with room for everything: one pass emits. One tile, tiles' edges, more tiles
+    than workgroups, tiles that keep everything or nothing; three steps on one codec (the tiles'
+    announcements of one step must not be taken for the next one's)."""
+    rng = np.random.default_rng(n)
+    bag, ref = api.DenseBag(n), oracle.DctState(n)
+    for step in range(3):
+        g = rng.standard_normal(n).astype(np.float32)
+        d_idx, d_val, nnz = bag.MaybeToCoo(2, eta, api.DeviceArray.from_host(g))
+        ridx, rval = ref.compress(g, life_span=2, eta=eta, exact_select=True)
+        assert nnz == ridx.size, step
+        assert np.array_equal(d_idx.to_host()[:nnz], ridx) and np.array_equal(d_val.to_host()[:nnz], rval), step
+        assert np.array_equal(bag.residual, ref.residual), step
+    bag.close()
+
+
+@pytest.mark.parametrize("case", ["sgd_mom", "adam_amsgrad", "rmsprop_all"])
+@pytest.mark.parametrize("n", [(1 << 22), (1 << 22) + 2049])
+def test_dense_push_coo_tiles(api, oracle, case, n):
+    """The tile-by-tile update with every number of state columns: ascending indices with empty tiles,
+    a single entry, then unordered ones, blocking and asynchronous."""
+    _, type_, conf = next(c for c in OPTIM_CASES if c[0] == case)
+    from util import make_optims
+    rng = np.random.default_rng(n)
+    w0 = rng.standard_normal(n).astype(np.float32)
+    t, r = api.DenseTable(w0), oracle.DenseTable(w0)
+    o_ref, o_gpu = make_optims(oracle, api, type_, conf)
+    ascending = np.sort(rng.choice(n // 2, size=n // 8, replace=False)).astype(np.int64) + n // 4
+    for flags in (api.DEVICE_PTRS, api.DEVICE_PTRS | api.ASYNC):
+        for idx in (ascending, np.array([n - 1], np.int64), ascending[::-1].copy()):
+            val = (rng.integers(1, 65, size=idx.size) / 1024.0).astype(np.float32)
+            d_idx, d_val = api.DeviceArray.from_host(idx), api.DeviceArray.from_host(val)
+            assert api.lib().krk_dense_push_coo(t.h, api.C.byref(o_gpu.raw), api.C.c_void_p(d_idx.ptr),
+                                                api.C.c_void_p(d_val.ptr), idx.size, 0.01, flags) == 0
+            assert r.push_coo(o_ref, idx, val, 0.01) == 0
+            assert_close(t.Pull()[1], r.pull(), "%d entries" % idx.size)
+
+
 @pytest.mark.parametrize("n", [1 << 22, (1 << 22) + 1, 5_000_003])
 def test_coo_to_dense_large_tensors(api, oracle, n):
     """From 2^22 elements on the dense result is written tile by tile when the indices ascend
