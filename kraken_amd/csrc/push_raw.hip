@@ -96,7 +96,7 @@ static inline unsigned grid_for(int64_t items, int per_block) {
 struct DSlot {
   unsigned long long key;
   uint32_t minpos;   // smallest position holding this id
-  uint32_t uidx;     // its index in the unique list
+  uint32_t unused;
 };
 
 // Equal ids are folded inside the workgroup first, through a small hash table in LDS: the lane
@@ -170,36 +170,106 @@ __global__ __launch_bounds__(kDedupBlock) void dedup_claim_kernel(DSlot* slots, 
   if (active) slot_of[p] = lidx[entry];
 }
 
-__global__ __launch_bounds__(kBlock) void dedup_flag_kernel(const DSlot* __restrict__ slots,
-                                                            const uint32_t* __restrict__ slot_of,
-                                                            int64_t n, int32_t* __restrict__ flag) {
-  const int64_t p = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (p >= n) return;
-  flag[p] = slots[slot_of[p]].minpos == (uint32_t)p ? 1 : 0;
+// The ranks of the first occurrences, in two launches and one random read per position. The first
+// one reads the smallest position of every position's id out of the index, leaves it in place of the
+// slot number, and ranks the first occurrences of its 1024 positions among themselves; their
+// counts go to sums[]. The second one (dedup_emit_kernel) adds what earlier tiles hold.
+// Flags, a scan of them in three launches and an emit that read the index again took six launches
+// where this takes two: they are bound by the launches up to a few hundred thousand ids (a blocking
+// krk_dedup of 26,624 ids 57 -> 45 us) and by the random reads beyond.
+constexpr int kRankTile = kDedupBlock;
+
+// Exclusive scan over the 1024 lanes of a workgroup; *all = the sum. Ends behind a barrier.
+__device__ __forceinline__ uint32_t dedup_block_scan(uint32_t v, uint32_t* wave_total, uint32_t* all) {
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  uint32_t incl = v;
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    const uint32_t y = __shfl_up(incl, d);
+    if (lane >= d) incl += y;
+  }
+  if (lane == kWave - 1) wave_total[wave] = incl;
+  __syncthreads();
+  uint32_t before = incl - v, sum = 0;
+#pragma unroll
+  for (int w = 0; w < kDedupBlock / kWave; ++w) {
+    const uint32_t x = wave_total[w];
+    if (w < wave) before += x;
+    sum += x;
+  }
+  __syncthreads();
+  *all = sum;
+  return before;
 }
 
-// Every position learns its id's index in the unique list from the rank of the id's first
-// position, and the first position also writes the id there and leaves the index in the slot
-// (one launch: a second one that read the index out of the slot had to wait for this one).
-__global__ __launch_bounds__(kBlock) void dedup_emit_kernel(DSlot* slots,
-                                                            const uint32_t* __restrict__ slot_of,
-                                                            const int32_t* __restrict__ rank,
-                                                            const uint64_t* __restrict__ ids, int64_t n,
-                                                            uint64_t* __restrict__ uids,
-                                                            long long* __restrict__ inv,
-                                                            const int32_t* __restrict__ total,
-                                                            int32_t* __restrict__ host_total) {
-  const int64_t p = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (p >= n) return;
-  if (p == 0 && host_total) *host_total = *total;      // the count, where a blocking caller reads it
-  DSlot* s = &slots[slot_of[p]];
-  const uint32_t first = s->minpos;
-  const int32_t r = rank[first];
-  if (inv) inv[p] = (long long)r;
-  if (first == (uint32_t)p) {
-    uids[r] = ids[p];
-    s->uidx = (uint32_t)r;
+__global__ __launch_bounds__(kRankTile) void dedup_rank_kernel(const DSlot* __restrict__ slots, uint32_t* slot_of,
+                                                               int64_t n, uint32_t* __restrict__ rank,
+                                                               uint32_t* __restrict__ sums) {
+  __shared__ uint32_t wave_total[kRankTile / kWave];
+  const int64_t p = (int64_t)blockIdx.x * kRankTile + threadIdx.x;
+  const uint32_t first = p < n ? slots[slot_of[p]].minpos : 0xFFFFFFFFu;
+  uint32_t all;
+  const uint32_t before = dedup_block_scan(first == (uint32_t)p ? 1u : 0u, wave_total, &all);
+  if (p < n) {
+    slot_of[p] = first;
+    rank[p] = before;
   }
+  if (threadIdx.x == 0) sums[blockIdx.x] = all;
+}
+
+// sums[0..m) -> exclusive prefix sums, the total behind them
+__global__ __launch_bounds__(kDedupBlock) void dedup_bases_kernel(uint32_t* __restrict__ sums, int64_t m) {
+  __shared__ uint32_t wave_total[kDedupBlock / kWave];
+  uint32_t carry = 0;
+  for (int64_t at = 0; at < m; at += kDedupBlock) {
+    const int64_t j = at + threadIdx.x;
+    uint32_t all;
+    const uint32_t before = dedup_block_scan(j < m ? sums[j] : 0u, wave_total, &all);
+    if (j < m) sums[j] = carry + before;
+    carry += all;
+  }
+  if (threadIdx.x == 0) sums[m] = carry;
+}
+
+// Every position learns its id's index in the unique list from the rank of the id's first position,
+// and the first position also writes the id there. keys / pos (dedup_sum): the index and the position
+// as the pair that is sorted. Up to kEmitScan tiles every workgroup adds the tiles' counts up by
+// itself (4 KB that all of them read); more of them are a launch of their own (SCANNED).
+constexpr int64_t kEmitScan = kDedupBlock;
+template <bool SCANNED>
+__global__ __launch_bounds__(kDedupBlock) void dedup_emit_kernel(const uint32_t* __restrict__ first_of,
+                                                                 const uint32_t* __restrict__ rank,
+                                                                 const uint32_t* __restrict__ sums, int64_t tiles,
+                                                                 const uint64_t* __restrict__ ids, int64_t n,
+                                                                 uint64_t* __restrict__ uids,
+                                                                 long long* __restrict__ inv,
+                                                                 uint32_t* __restrict__ keys,
+                                                                 uint32_t* __restrict__ pos,
+                                                                 int32_t* __restrict__ total,
+                                                                 int32_t* __restrict__ host_total) {
+  __shared__ uint32_t wave_total[kDedupBlock / kWave];
+  __shared__ uint32_t base[kEmitScan];
+  const int64_t p = (int64_t)blockIdx.x * kDedupBlock + threadIdx.x;
+  const uint32_t first = p < n ? first_of[p] : 0u;
+  uint32_t all;
+  if (SCANNED) {
+    all = sums[tiles];
+  } else {
+    base[threadIdx.x] = dedup_block_scan((int64_t)threadIdx.x < tiles ? sums[threadIdx.x] : 0u, wave_total, &all);
+    __syncthreads();
+  }
+  if (p >= n) return;
+  if (p == 0) {
+    *total = (int32_t)all;
+    if (host_total) *host_total = (int32_t)all;        // the count, where a blocking caller reads it
+  }
+  const uint32_t r = (SCANNED ? sums[first / kRankTile] : base[first / kRankTile]) + rank[first];
+  if (inv) inv[p] = (long long)r;
+  if (keys) {
+    keys[p] = r;
+    pos[p] = (uint32_t)p;
+  }
+  if (first == (uint32_t)p) uids[r] = ids[p];
 }
 
 // Requests of at most kDedupSmall ids: the whole dedup in one launch of one workgroup. The ids
@@ -222,6 +292,8 @@ __device__ __forceinline__ int dedup_small_at(int p) { return p + (p >> 3); }
 __global__ __launch_bounds__(kDedupBlock) void dedup_small_kernel(const uint64_t* __restrict__ ids, int n,
                                                                   uint64_t* __restrict__ uids,
                                                                   long long* __restrict__ inv,
+                                                                  uint32_t* __restrict__ keys,
+                                                                  uint32_t* __restrict__ pos,
                                                                   int32_t* __restrict__ total,
                                                                   int32_t* __restrict__ host_total) {
   __shared__ unsigned long long sid[kDedupSmall + kDedupSmall / 8];   // the ids by position, then the unique ids
@@ -301,8 +373,15 @@ __global__ __launch_bounds__(kDedupBlock) void dedup_small_kernel(const uint64_t
   }
   __syncthreads();
   for (int r = t; r < (int)all; r += kDedupBlock) uids[r] = sid[dedup_small_at(r)];
-  if (!inv) return;
-  for (int p = t; p < n; p += kDedupBlock) inv[p] = (long long)tab[slot_of[p]];
+  if (!inv && !keys) return;
+  for (int p = t; p < n; p += kDedupBlock) {
+    const uint32_t r = tab[slot_of[p]];
+    if (inv) inv[p] = (long long)r;
+    if (keys) {
+      keys[p] = r;
+      pos[p] = (uint32_t)p;
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1707,23 +1786,12 @@ static int32_t push_sorted(krk_sparse* t, const krk_optim* o, int64_t n, const f
                          [&](uint32_t* keys, uint32_t* pos) { fill(keys, pos, miss_key); });
 }
 
-// stand-alone dedup + sum: (unique index, position) pairs for the sort
-__global__ __launch_bounds__(kBlock) void dedup_pairs_kernel(const DSlot* __restrict__ slots,
-                                                             const uint32_t* __restrict__ slot_of, int64_t n,
-                                                             uint32_t* __restrict__ keys,
-                                                             uint32_t* __restrict__ pos) {
-  const int64_t p = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (p >= n) return;
-  keys[p] = slots[slot_of[p]].uidx;
-  pos[p] = (uint32_t)p;
-}
-
 // worker/emitter.cc:162-182 : rows of the unique ids back to one row per position
 template <int VEC>
 __global__ __launch_bounds__(kBlock) void expand_rows_kernel(const float* __restrict__ rows,
                                                              const long long* __restrict__ inv, int64_t n,
                                                              int64_t n_rows, float* __restrict__ out, int dim,
-                                                             int elems, uint32_t* __restrict__ err) {
+                                                             int elems, int32_t* __restrict__ err) {
   const int64_t total = n * elems;
   const int64_t step = (int64_t)gridDim.x * kBlock;
   for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < total; i += step) {
@@ -1736,7 +1804,7 @@ __global__ __launch_bounds__(kBlock) void expand_rows_kernel(const float* __rest
     if (u >= 0 && u < n_rows) {
       vload<VEC>(rows + u * dim + e * VEC, v);
     } else if (e == 0) {
-      atomicOr(err, 1u);
+      __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     vstore<VEC>(out + p * dim + e * VEC, v);
   }
@@ -1758,9 +1826,8 @@ struct DedupWork {
   DSlot* slots;
   uint64_t cap;
   uint32_t* slot_of;
-  int32_t* flag;
-  int32_t* rank;
-  void* scan_tmp;
+  uint32_t* rank;
+  uint32_t* sums;   // first occurrences of every tile of positions, and one more
   int32_t* d_total;
   char* extra;   // `extra_bytes` more for the caller (staged host arguments)
 };
@@ -1772,15 +1839,14 @@ static int32_t dedup_layout(int64_t n, size_t extra_bytes, DedupWork* w) {
   while (cap < (uint64_t)n * 2) cap <<= 1;
   const size_t slots_b = (cap + 1) * sizeof(DSlot);
   const size_t n4 = round256((size_t)n * 4);
-  const size_t scan_b = round256(scan_scratch_bytes(n));
-  KRK_TRY(g_dedup_pool.reserve(slots_b + 3 * n4 + scan_b + 256 + extra_bytes));
+  const size_t sums_b = round256((size_t)(n / kRankTile + 2) * 4);
+  KRK_TRY(g_dedup_pool.reserve(slots_b + 2 * n4 + sums_b + 256 + extra_bytes));
   char* cur = g_dedup_pool.as<char>();
   w->slots = reinterpret_cast<DSlot*>(cur); cur += slots_b;
   w->cap = cap;
   w->slot_of = reinterpret_cast<uint32_t*>(cur); cur += n4;
-  w->flag = reinterpret_cast<int32_t*>(cur); cur += n4;
-  w->rank = reinterpret_cast<int32_t*>(cur); cur += n4;
-  w->scan_tmp = cur; cur += scan_b;
+  w->rank = reinterpret_cast<uint32_t*>(cur); cur += n4;
+  w->sums = reinterpret_cast<uint32_t*>(cur); cur += sums_b;
   w->d_total = reinterpret_cast<int32_t*>(cur); cur += 256;
   w->extra = cur;
   return KRK_SUCCESS;
@@ -1813,25 +1879,38 @@ static void launch_dedup_claims(const DedupWork& w, const uint64_t* d_ids, int64
                      n, w.slot_of, head);
 }
 
+// What follows the claims: ranks, the unique list, the inverse and (keys, pos) where they are asked for.
+static int32_t launch_dedup_emit(const DedupWork& w, const uint64_t* d_ids, int64_t n, uint64_t* d_uids,
+                                 long long* d_inv, uint32_t* keys, uint32_t* pos, int32_t* host_total, hipStream_t s) {
+  const int64_t tiles = (n + kRankTile - 1) / kRankTile;
+  const dim3 grid((unsigned)tiles), block(kRankTile);
+  hipLaunchKernelGGL(dedup_rank_kernel, grid, block, 0, s, w.slots, w.slot_of, n, w.rank, w.sums);
+  if (tiles <= kEmitScan) {
+    hipLaunchKernelGGL((dedup_emit_kernel<false>), grid, block, 0, s, w.slot_of, w.rank, w.sums, tiles, d_ids, n, d_uids,
+                       d_inv, keys, pos, w.d_total, host_total);
+  } else {
+    hipLaunchKernelGGL(dedup_bases_kernel, dim3(1), block, 0, s, w.sums, tiles);
+    hipLaunchKernelGGL((dedup_emit_kernel<true>), grid, block, 0, s, w.slot_of, w.rank, w.sums, tiles, d_ids, n, d_uids,
+                       d_inv, keys, pos, w.d_total, host_total);
+  }
+  KRK_HIP(hipGetLastError());
+  return KRK_SUCCESS;
+}
+
 static int32_t dedup_enqueue(const DedupWork& w, const uint64_t* d_ids, int64_t n, uint64_t* d_uids,
                              long long* d_inv, hipStream_t s) {
   const int64_t words = (int64_t)(w.cap + 1) * (int64_t)(sizeof(DSlot) / 4);
   hipLaunchKernelGGL(fill_u32_kernel, dim3(grid_for(words, kBlock)), dim3(kBlock), 0, s,
                      reinterpret_cast<uint32_t*>(w.slots), words, 0xFFFFFFFFu);
-  const dim3 grid(grid_for(n, kBlock)), block(kBlock);
   launch_dedup_claims(w, d_ids, n, s);
-  hipLaunchKernelGGL(dedup_flag_kernel, grid, block, 0, s, w.slots, w.slot_of, n, w.flag);
-  KRK_HIP(hipGetLastError());
-  KRK_TRY(exclusive_scan_i32(w.flag, w.rank, n, w.d_total, w.scan_tmp, s));
-  hipLaunchKernelGGL(dedup_emit_kernel, grid, block, 0, s, w.slots, w.slot_of, w.rank, d_ids, n, d_uids, d_inv,
-                     w.d_total, (int32_t*)nullptr);
-  KRK_HIP(hipGetLastError());
-  return KRK_SUCCESS;
+  return launch_dedup_emit(w, d_ids, n, d_uids, d_inv, nullptr, nullptr, nullptr, s);
 }
 
 // Where a blocking dedup's count lands: page-locked host memory that the kernel which knows the
 // total writes to, so the host waits for the stream once and reads it (no copy in the stream).
+// A word further on is where krk_expand_rows learns of an index outside its rows.
 static int32_t* g_dedup_count = nullptr;
+constexpr int kExpandErr = 8;
 
 static int32_t dedup_count_buffer() {
   if (g_dedup_count) return KRK_SUCCESS;
@@ -1845,19 +1924,19 @@ static int32_t dedup_read_count(hipStream_t s, int32_t* u) {
   return KRK_SUCCESS;
 }
 
-static int32_t dedup_core(const DedupWork& w, const uint64_t* d_ids, int64_t n, uint64_t* d_uids,
-                          long long* d_inv, hipStream_t s, int32_t* u) {
+// Enqueues a whole dedup; its count arrives in g_dedup_count. Small requests take one launch.
+static int32_t dedup_core(const DedupWork& w, const uint64_t* d_ids, int64_t n, uint64_t* d_uids, long long* d_inv,
+                          uint32_t* keys, uint32_t* pos, hipStream_t s) {
   KRK_TRY(dedup_count_buffer());
+  if (n <= kDedupSmall) {
+    hipLaunchKernelGGL(dedup_small_kernel, dim3(1), dim3(kDedupBlock), 0, s, d_ids, (int)n, d_uids, d_inv, keys, pos,
+                       w.d_total, g_dedup_count);
+    KRK_HIP(hipGetLastError());
+    return KRK_SUCCESS;
+  }
   KRK_HIP(hipMemsetAsync(w.slots, 0xFF, (w.cap + 1) * sizeof(DSlot), s));
-  const dim3 grid(grid_for(n, kBlock)), block(kBlock);
   launch_dedup_claims(w, d_ids, n, s);
-  hipLaunchKernelGGL(dedup_flag_kernel, grid, block, 0, s, w.slots, w.slot_of, n, w.flag);
-  KRK_HIP(hipGetLastError());
-  KRK_TRY(exclusive_scan_i32(w.flag, w.rank, n, w.d_total, w.scan_tmp, s));
-  hipLaunchKernelGGL(dedup_emit_kernel, grid, block, 0, s, w.slots, w.slot_of, w.rank, d_ids, n, d_uids, d_inv,
-                     w.d_total, g_dedup_count);
-  KRK_HIP(hipGetLastError());
-  return dedup_read_count(s, u);
+  return launch_dedup_emit(w, d_ids, n, d_uids, d_inv, keys, pos, g_dedup_count, s);
 }
 
 int32_t krk_dedup(const uint64_t* ids, int64_t n, uint64_t* uids, int64_t* inv, int64_t* n_unique,
@@ -1889,21 +1968,13 @@ int32_t krk_dedup(const uint64_t* ids, int64_t n, uint64_t* uids, int64_t* inv, 
   }
   hipStream_t s = nullptr;
   int32_t u = 0;
-  if (n <= kDedupSmall) {
-    KRK_TRY(dedup_count_buffer());
-    hipLaunchKernelGGL(dedup_small_kernel, dim3(1), dim3(kDedupBlock), 0, s, d_ids, (int)n, d_uids,
-                       inv ? d_inv : nullptr, w.d_total, g_dedup_count);
-    KRK_HIP(hipGetLastError());
-    KRK_TRY(dedup_read_count(s, &u));
-  } else {
-    KRK_TRY(dedup_core(w, d_ids, n, d_uids, inv ? d_inv : nullptr, s, &u));
-  }
+  KRK_TRY(dedup_core(w, d_ids, n, d_uids, inv ? d_inv : nullptr, nullptr, nullptr, s));
+  KRK_TRY(dedup_read_count(s, &u));
   *n_unique = u;
   if (host) {
     KRK_HIP(hipMemcpy(uids, d_uids, (size_t)u * 8, hipMemcpyDeviceToHost));
     if (inv) KRK_HIP(hipMemcpy(inv, d_inv, (size_t)n * 8, hipMemcpyDeviceToHost));
   }
-  KRK_HIP(hipStreamSynchronize(s));
   return KRK_SUCCESS;
 }
 
@@ -1916,8 +1987,9 @@ int32_t krk_dedup(const uint64_t* ids, int64_t n, uint64_t* uids, int64_t* inv, 
 constexpr int64_t kNoAllocCap = (int64_t)KRK_DEDUP_NOALLOC_MAX * 2;   // index slots: at most half full
 constexpr size_t kNoAllocSlotsBytes = (((size_t)kNoAllocCap + 1) * sizeof(DSlot) + 255) & ~(size_t)255;
 constexpr size_t kNoAllocN4 = (size_t)KRK_DEDUP_NOALLOC_MAX * 4;
-constexpr size_t kNoAllocScanBytes = 4096;   // one partial sum per 2048 positions: 512 bytes at the maximum
-constexpr size_t kNoAllocBytes = kNoAllocSlotsBytes + 3 * kNoAllocN4 + kNoAllocScanBytes + 256;
+constexpr size_t kNoAllocSumsBytes = 4096;
+static_assert((KRK_DEDUP_NOALLOC_MAX / kRankTile + 2) * 4 <= kNoAllocSumsBytes, "a count per tile of positions");
+constexpr size_t kNoAllocBytes = kNoAllocSlotsBytes + 2 * kNoAllocN4 + kNoAllocSumsBytes + 256;
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
@@ -1983,9 +2055,8 @@ int32_t krk_dedup_noalloc(const uint64_t* ids, int64_t n, uint64_t* uids, int64_
   w.slots = reinterpret_cast<DSlot*>(cur); cur += kNoAllocSlotsBytes;
   w.cap = cap;
   w.slot_of = reinterpret_cast<uint32_t*>(cur); cur += kNoAllocN4;
-  w.flag = reinterpret_cast<int32_t*>(cur); cur += kNoAllocN4;
-  w.rank = reinterpret_cast<int32_t*>(cur); cur += kNoAllocN4;
-  w.scan_tmp = cur; cur += kNoAllocScanBytes;
+  w.rank = reinterpret_cast<uint32_t*>(cur); cur += kNoAllocN4;
+  w.sums = reinterpret_cast<uint32_t*>(cur); cur += kNoAllocSumsBytes;
   w.d_total = reinterpret_cast<int32_t*>(cur);
   w.extra = nullptr;
   if (n == 0) {
@@ -2048,12 +2119,22 @@ int32_t krk_dedup_sum(const uint64_t* ids, int64_t n, const float* grads, int64_
   }
   hipStream_t s = nullptr;
   int32_t u = 0;
-  KRK_TRY(dedup_core(w, d_ids, n, d_uids, inv ? d_inv : nullptr, s, &u));
   // positions sorted by unique index (stable: position order inside a run, as
   // worker/emitter.cc:527-529 adds them), every run summed and stored as row `index` of sums
+  KRK_TRY(g_dedup_reduce[0].reserve(4 * (size_t)n * sizeof(uint32_t)));   // sort_and_reduce's keys and payload
+  uint32_t* keys = g_dedup_reduce[0].as<uint32_t>();
+  KRK_TRY(dedup_core(w, d_ids, n, d_uids, inv ? d_inv : nullptr, keys, keys + n, s));
+  // The sort's width: there are no more unique ids than ids. Up to 2^18 that is two passes at most and
+  // nothing is waited for; beyond it the count may save a pass (22 us of a million ids), which is
+  // what waiting for it costs at most (10 us of launch and wait).
+  int64_t bound = n;
+  if (n > ((int64_t)1 << 18)) {
+    KRK_TRY(dedup_read_count(s, &u));
+    bound = u;
+  }
   uint32_t miss_key = 1;
-  int bits = 1;
-  while ((int64_t)miss_key < (int64_t)u) {
+  int bits = 0;
+  while ((int64_t)miss_key < bound) {
     miss_key <<= 1;
     ++bits;
   }
@@ -2062,20 +2143,15 @@ int32_t krk_dedup_sum(const uint64_t* ids, int64_t n, const float* grads, int64_
   tv.stride = dim;
   ApplyArgs args{};
   args.c0 = args.c1 = args.c2 = args.meta_off = -1;
-  const DSlot* slots = w.slots;
-  const uint32_t* slot_of = w.slot_of;
-  KRK_TRY(sort_and_reduce(sh, s, g_dedup_reduce, tv, kOptStore, n, miss_key, bits, d_g, args,
-                          PooledSrc{}, nullptr, nullptr, [&](uint32_t* keys, uint32_t* pos) {
-                            hipLaunchKernelGGL(dedup_pairs_kernel, dim3(grid_for(n, kBlock)), dim3(kBlock), 0, s,
-                                               slots, slot_of, n, keys, pos);
-                          }));
+  KRK_TRY(sort_and_reduce(sh, s, g_dedup_reduce, tv, kOptStore, n, miss_key, bits, d_g, args, PooledSrc{}, nullptr,
+                          nullptr, [](uint32_t*, uint32_t*) {}));
+  KRK_TRY(dedup_read_count(s, &u));
   *n_unique = u;
   if (host) {
     KRK_HIP(hipMemcpy(uids, d_uids, (size_t)u * 8, hipMemcpyDeviceToHost));
     if (inv) KRK_HIP(hipMemcpy(inv, d_inv, (size_t)n * 8, hipMemcpyDeviceToHost));
     KRK_HIP(hipMemcpy(sums, d_sums, (size_t)u * (size_t)dim * sizeof(float), hipMemcpyDeviceToHost));
   }
-  KRK_HIP(hipStreamSynchronize(s));
   return KRK_SUCCESS;
 }
 
@@ -2096,23 +2172,26 @@ int32_t krk_expand_rows(const float* rows, int64_t n_rows, const int64_t* inv, i
   const size_t inv_b = round256((size_t)n * 8);
   const size_t out_b = round256((size_t)n * (size_t)dim * sizeof(float));
   std::lock_guard<std::mutex> pool_lock(g_dedup_mu);
-  KRK_TRY(g_dedup_pool.reserve(256 + (host ? in_b + inv_b + out_b : 0)));
+  KRK_TRY(dedup_count_buffer());
+  KRK_TRY(g_dedup_pool.reserve(host ? in_b + inv_b + out_b : 0));
   char* base = g_dedup_pool.as<char>();
-  uint32_t* d_err = reinterpret_cast<uint32_t*>(base);
+  int32_t* d_err = g_dedup_count + kExpandErr;
   const float* d_rows = rows;
   const long long* d_inv = reinterpret_cast<const long long*>(inv);
   float* d_out = out;
   hipStream_t s = nullptr;
   if (host) {
-    float* s_rows = reinterpret_cast<float*>(base + 256);
-    long long* s_inv = reinterpret_cast<long long*>(base + 256 + in_b);
-    d_out = reinterpret_cast<float*>(base + 256 + in_b + inv_b);
+    float* s_rows = reinterpret_cast<float*>(base);
+    long long* s_inv = reinterpret_cast<long long*>(base + in_b);
+    d_out = reinterpret_cast<float*>(base + in_b + inv_b);
     KRK_HIP(hipMemcpy(s_rows, rows, (size_t)n_rows * (size_t)dim * sizeof(float), hipMemcpyHostToDevice));
     KRK_HIP(hipMemcpy(s_inv, inv, (size_t)n * 8, hipMemcpyHostToDevice));
     d_rows = s_rows;
     d_inv = s_inv;
   }
-  KRK_HIP(hipMemsetAsync(d_err, 0, 4, s));
+  // the word lies in page-locked memory that the kernel writes to: neither a launch that clears it nor
+  // a copy that fetches it (three launches and two waits, 30 us, for what takes one of each, 18 us)
+  *static_cast<volatile int32_t*>(d_err) = 0;
   int64_t blocks = (n * elems + kBlock - 1) / kBlock;
   if (blocks > 256 * 64) blocks = 256 * 64;   // grid-stride beyond that
   if (vec == 4) {
@@ -2123,11 +2202,9 @@ int32_t krk_expand_rows(const float* rows, int64_t n_rows, const int64_t* inv, i
                        n_rows, d_out, (int)dim, elems, d_err);
   }
   KRK_HIP(hipGetLastError());
-  uint32_t err = 0;
-  KRK_HIP(hipMemcpy(&err, d_err, 4, hipMemcpyDeviceToHost));
-  if (host) KRK_HIP(hipMemcpy(out, d_out, (size_t)n * (size_t)dim * sizeof(float), hipMemcpyDeviceToHost));
   KRK_HIP(hipStreamSynchronize(s));
-  if (err) {
+  if (host) KRK_HIP(hipMemcpy(out, d_out, (size_t)n * (size_t)dim * sizeof(float), hipMemcpyDeviceToHost));
+  if (*static_cast<volatile int32_t*>(d_err)) {
     set_error("an index lies outside the %lld rows", (long long)n_rows);
     return KRK_E_ARGUMENT;
   }

@@ -1341,23 +1341,20 @@ __global__ __launch_bounds__(kBlock) void route_rank_kernel(const uint64_t* __re
   if ((int)threadIdx.x < nodes) block_counts[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = hist[threadIdx.x];
 }
 
+// perm[where node k's ids begin + ids of node k in earlier workgroups + earlier in this one] = p:
+// a stable partition of the positions by owner.
 // node_count[k] = ids of node k, read off the scanned per-workgroup counts: where node k + 1's
 // ids begin minus where node k's do (thousands of workgroups adding to the same few counters
 // in memory cost more than the rest of the routing together).
-__global__ __launch_bounds__(kRouteMaxNodes) void route_counts_kernel(const int32_t* __restrict__ block_base,
-                                                                      int64_t blocks, int nodes, int32_t n,
-                                                                      int32_t* __restrict__ node_count) {
-  const int k = threadIdx.x;
-  if (k >= nodes) return;
-  const int32_t end = k + 1 < nodes ? block_base[(int64_t)(k + 1) * blocks] : n;
-  node_count[k] = end - block_base[(int64_t)k * blocks];
-}
-
-// perm[where node k's ids begin + ids of node k in earlier workgroups + earlier in this one] = p:
-// a stable partition of the positions by owner.
 __global__ __launch_bounds__(kBlock) void route_scatter_kernel(const uint8_t* __restrict__ rank8, int64_t n,
-                                                               const int32_t* __restrict__ block_base,
-                                                               long long* __restrict__ perm) {
+                                                               const int32_t* __restrict__ block_base, int nodes,
+                                                               long long* __restrict__ perm,
+                                                               int32_t* __restrict__ node_count) {
+  if (blockIdx.x == 0 && (int)threadIdx.x < nodes) {
+    const int64_t k = threadIdx.x, blocks = gridDim.x;
+    const int32_t end = k + 1 < nodes ? block_base[(k + 1) * blocks] : (int32_t)n;
+    node_count[k] = end - block_base[k * blocks];
+  }
   __shared__ int32_t wave_count[kBlock / kWave][kRouteMaxNodes];
   for (int i = threadIdx.x; i < (kBlock / kWave) * kRouteMaxNodes; i += kBlock) (&wave_count[0][0])[i] = 0;
   __syncthreads();
@@ -2800,9 +2797,8 @@ int32_t krk_route_ids(uint64_t table_id, const uint64_t* ring_hash, const uint64
                      (int)m, d_owner, d_rank8, d_bc);
   KRK_HIP(hipGetLastError());
   KRK_TRY(exclusive_scan_i32(d_bc, d_bc, m * blocks, d_total, d_scan, st));
-  hipLaunchKernelGGL(route_counts_kernel, dim3(1), dim3(kRouteMaxNodes), 0, st, d_bc, blocks, (int)m, (int32_t)n,
-                     d_count);
-  hipLaunchKernelGGL(route_scatter_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, st, d_rank8, n, d_bc, d_perm);
+  hipLaunchKernelGGL(route_scatter_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, st, d_rank8, n, d_bc, (int)m,
+                     d_perm, d_count);
   KRK_HIP(hipGetLastError());
   if (host) {
     if (owner) KRK_HIP(hipMemcpy(owner, d_owner, (size_t)n * 8, hipMemcpyDeviceToHost));

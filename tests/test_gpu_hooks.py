@@ -253,3 +253,19 @@ def test_route_ids_partitions_a_request_like_the_worker(api, oracle):
                                  api._ptr(np.zeros(1, np.int64)), api._ptr(one), api._ptr(np.zeros(1, np.int64)), 1,
                                  C.byref(m), 0)
     assert rc == api.E_CAPACITY and m.value == len(set(n for _, n in ring))
+
+
+# seven nodes: 4681 workgroups' counts are scanned by one workgroup (32767 of them), 4682 by three launches
+@pytest.mark.parametrize("n", [1, 256, 4681 * 256, 4681 * 256 + 1])
+def test_route_ids_scan_sizes(api, oracle, n):
+    rng = np.random.default_rng(n)
+    hashes = np.sort(rng.integers(0, 2**63, 7 * 32, dtype=np.uint64) * np.uint64(2))
+    ring = [(int(h), 10 + i % 7) for i, h in enumerate(hashes)]
+    ids = splitmix64(np.arange(n, dtype=np.uint64))
+    want = oracle.route_owners(ring, 3, ids)
+    node_ids, counts, owner, perm = api.route_ids(3, ring, api.DeviceArray.from_host(ids))
+    rank = np.searchsorted(node_ids, want)
+    assert np.array_equal(owner.to_host()[:n], want)
+    assert np.array_equal(perm.to_host()[:n], np.argsort(rank, kind="stable"))
+    assert counts.tolist() == np.bincount(rank, minlength=7).tolist()
+

@@ -81,6 +81,29 @@ def test_dedup_zipf_exact(api, oracle, n, s, space):
     assert np.array_equal(du.to_host()[:cnt], ru) and np.array_equal(dinv.to_host(), rinv)
 
 
+# around the tile of positions whose first occurrences are ranked together (1024), the number of
+# tiles whose counts every workgroup adds up by itself (1024 of them) and the size up to which
+# dedup_sum takes its sort's width from the request (2^18)
+@pytest.mark.parametrize("n", [9 * 1024 - 1, 9 * 1024, 9 * 1024 + 1, 2**18, 2**18 + 1, 2**20, 2**20 + 1])
+@pytest.mark.parametrize("kind", ["zipf", "distinct", "same"])
+def test_dedup_rank_tiles(api, oracle, n, kind):
+    rng = np.random.default_rng(n)
+    if kind == "zipf":
+        ids = zipf_ids(rng, 1.1, 10**6, n)
+    elif kind == "distinct":
+        ids = rng.permutation(n).astype(np.uint64) * np.uint64(0x9E3779B97F4A7C15)
+    else:
+        ids = np.full(n, 2**64 - 1, np.uint64)
+    g = _dyadic_grads(rng, (n, 4))
+    ru, rinv = oracle.dedup(ids)
+    du, dinv, cnt = api.dedup(api.DeviceArray.from_host(ids))
+    assert cnt == ru.size
+    assert np.array_equal(du.to_host()[:cnt], ru) and np.array_equal(dinv.to_host(), rinv)
+    u, inv, sums = api.dedup_sum(ids, g)
+    assert np.array_equal(u, ru) and np.array_equal(inv, rinv)
+    assert np.array_equal(sums, oracle.dedup_sum(ids, g)[1])
+
+
 def _dyadic_grads(rng, shape):
     """Gradients on a coarse binary grid: any order of fp32 additions gives the same bits, so
     the comparison isolates dedup + update from the (order-dependent) rounding of the sums."""
