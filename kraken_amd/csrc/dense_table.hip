@@ -326,8 +326,11 @@ __global__ __launch_bounds__(kDenseBlock) void dense_copy_kernel(const float* __
 // launch makes a model with dozens of small tensors pay a launch per tensor. Here the members'
 // values (and, for the push, gradients) are one concatenated array in member order and a launch
 // takes up to kDenseGroupChunk members: workgroups [block_start[m], block_start[m + 1]) belong to
-// member m.
-constexpr int kDenseGroupChunk = 32;
+// member m. 56 members and the other arguments come to just under the 4096 bytes a launch may carry;
+// a request of dozens of small tensors is bound by its launches (40 tensors of 434k parameters,
+// push + pull: 14.1 us as two launches each of 32 members at most, 9 us as one each).
+constexpr int kDenseGroupChunk = 56;
+static_assert(kDenseGroupChunk <= kWave, "a lane looks at each member");
 
 struct DenseGroupArgs {
   int32_t members;
@@ -335,10 +338,12 @@ struct DenseGroupArgs {
   DenseMember m[kDenseGroupChunk];
 };
 
+// The member of this workgroup: a lane per member and one vote (block_start ascends; walking it takes
+// a chain of scalar loads as long as the list).
 __device__ __forceinline__ int dense_member_of_block(const DenseGroupArgs& a) {
-  int m = 0;
-  while (m + 1 < a.members && blockIdx.x >= a.block_start[m + 1]) ++m;
-  return m;
+  const int lane = threadIdx.x & (kWave - 1);
+  const bool begun = lane < a.members && blockIdx.x >= a.block_start[lane < a.members ? lane : 0];
+  return __builtin_amdgcn_readfirstlane(__popcll(__ballot(begun)) - 1);
 }
 
 __global__ __launch_bounds__(kDenseBlock) void dense_group_pull_kernel(DenseGroupArgs a, float* __restrict__ out) {
@@ -353,6 +358,8 @@ __global__ __launch_bounds__(kDenseBlock) void dense_group_pull_kernel(DenseGrou
     __builtin_nontemporal_store(dense_load(m.w, i), reinterpret_cast<dfloat4*>(dst) + i);
   for (int64_t i = (n4 << 2) + lane; i < m.n; i += stride) dst[i] = m.w[i];
 }
+
+static_assert(sizeof(DenseGroupArgs) + sizeof(OptimK) + 32 <= 4096, "the arguments of one launch");
 
 template <int OPT>
 __global__ __launch_bounds__(kDenseBlock) void dense_group_update_kernel(DenseGroupArgs a,
