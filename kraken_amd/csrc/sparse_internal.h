@@ -390,6 +390,7 @@ struct krk_sparse : krk::ObjBase {
   uint32_t* host_counters = nullptr;  // pinned
   int64_t size_ub = 0;                // upper bound of rows used, exact after a blocking call
   unsigned long long* host_pub = nullptr;   // pinned, written by the device (publish_kernel)
+  uint32_t pub_epoch = 0;                   // launch number of the last publish that was enqueued
   uint32_t* host_inserted = nullptr;        // pinned, behind host_pub: set by pulls that insert
   int64_t last_request = 0;           // size of the last inserting request
   uint64_t enq_total = 0;             // ids handed to inserting launches so far
