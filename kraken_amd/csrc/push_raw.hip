@@ -1128,7 +1128,7 @@ static int pick_tile(int64_t cnt) {
 // the bucket that holds the hottest id has fewer lane groups to share its run out to.
 // ---------------------------------------------------------------------------
 constexpr int kSortBlock = 1024;
-constexpr int kSortItems = 8;
+constexpr int kSortItems = 12;
 constexpr int kSortMax = kSortBlock * kSortItems;      // ids per table
 constexpr int kSortWaves = kSortBlock / kWave;
 constexpr int kMaxBucketBits = 5;                      // up to 32 buckets a table
@@ -1245,17 +1245,18 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(
   const int wave = t / kWave;
 
   // ---- a. the bucket's positions, in position order -------------------------------------------
-  // a lane looks at four or eight consecutive positions, read straight from global memory with
+  // a lane looks at four, eight or twelve consecutive positions, read straight from global memory with
   // 16-byte loads where the member's keys begin on 16 bytes (as eight 4-byte loads, each of
   // them fetched a 32-byte piece of a line for four bytes: 3-4 us of the kernel's 20)
-  const int own = all > 4 * kSortBlock ? kSortItems : 4;
+  const int own = (all + 4 * kSortBlock - 1) / (4 * kSortBlock) * 4;   // 4, 8 or 12
   uint32_t mine[kSortItems];
   if ((reinterpret_cast<uintptr_t>(keys + a) & 15) == 0 && (t + 1) * own <= all) {
-    const uint4 x = *reinterpret_cast<const uint4*>(keys + a + t * own);
-    mine[0] = x.x; mine[1] = x.y; mine[2] = x.z; mine[3] = x.w;
-    if (own == kSortItems) {
-      const uint4 y = *reinterpret_cast<const uint4*>(keys + a + t * own + 4);
-      mine[4] = y.x; mine[5] = y.y; mine[6] = y.z; mine[7] = y.w;
+#pragma unroll
+    for (int i = 0; i < kSortItems; i += 4) {
+      if (i < own) {
+        const uint4 x = *reinterpret_cast<const uint4*>(keys + a + t * own + i);
+        mine[i] = x.x; mine[i + 1] = x.y; mine[i + 2] = x.z; mine[i + 3] = x.w;
+      }
     }
   } else {
 #pragma unroll
@@ -1294,7 +1295,7 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(
   }
   const int len = (int)total;
   if (len == 0) return;                                // uniform
-  const int per_lane = (len + kSortBlock - 1) / kSortBlock;   // 1..8
+  const int per_lane = (len + kSortBlock - 1) / kSortBlock;   // 1..12
   const int padded = per_lane * kSortBlock;
   for (int j = len + t; j < padded; j += kSortBlock) {   // beyond what the lanes above wrote
 

@@ -255,6 +255,32 @@ def test_dedup_sum_random_gradients_and_device_arrays(api, oracle):
     assert rc == api.E_ARGUMENT
 
 
+# a lane of the short path looks at 4, 8 or 12 positions; 12288 of them are the most a table may bring
+@pytest.mark.parametrize("n", [4096, 4097, 8193, 12287, 12288, 12289])
+@pytest.mark.parametrize("shape", ["one_id", "one_bucket", "zipf"])
+def test_push_raw_short_path_sizes(api, oracle, n, shape):
+    """The sizes at which the short path's lanes take more positions and where it ends, with a bucket
+    that holds everything (one id; distinct rows of one bucket) and an ordinary request. Dyadic
+    gradients and plain SGD: exact whatever the order of additions."""
+    dim = 16
+    rng = np.random.default_rng(n)
+    t = api.SparseTable(dim, api.Initializer.create(api.InitializerType.kConstant, {"value": "1"}))
+    if shape == "one_id":
+        ids = np.full(n, 4242, np.uint64)
+    elif shape == "one_bucket":
+        pool = splitmix64(np.arange(450_000, dtype=np.uint64))
+        t.Pull(pool)
+        ids = rng.permutation(pool[t.lookup(pool) % 32 == 0])[:n]
+        assert ids.size == n
+    else:
+        ids = zipf_ids(rng, 1.05, 10**5, n)
+    t.Pull(ids)
+    grads = _dyadic_grads(rng, (n, dim))
+    assert t.PushRaw(api.Optim.create(api.OptimType.kSGD), ids, grads, 0.5) == 0
+    u, gs = oracle.dedup_sum(ids, grads)
+    assert np.array_equal(t.Pull(u)[1], np.float32(1.0) - np.float32(0.5) * gs)
+
+
 @pytest.mark.parametrize("dim", [5, 16, 64])
 @pytest.mark.parametrize("shape", ["one_id", "one_bucket", "long_and_short", "boundary"])
 def test_push_raw_short_path_extremes(api, oracle, dim, shape):
