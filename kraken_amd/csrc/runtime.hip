@@ -85,6 +85,23 @@ int32_t DeviceBuffer::reserve(size_t want) {
   return KRK_SUCCESS;
 }
 
+int32_t HostBuffer::reserve(size_t want) {
+  if (want <= bytes) return KRK_SUCCESS;
+  want = (want + want / 2 + 4095) & ~(size_t)4095;
+  if (ptr) KRK_HIP(hipHostFree(ptr));
+  ptr = nullptr;
+  bytes = 0;
+  KRK_HIP(hipHostMalloc(&ptr, want, hipHostMallocDefault));
+  bytes = want;
+  return KRK_SUCCESS;
+}
+
+void HostBuffer::release() {
+  if (ptr) (void)hipHostFree(ptr);
+  ptr = nullptr;
+  bytes = 0;
+}
+
 void DeviceBuffer::release() {
   if (ptr) (void)hipFree(ptr);
   ptr = nullptr;
@@ -496,6 +513,7 @@ void ObjBase::close_stream() {
     stream = nullptr;
   }
   for (auto& b : stage) b.release();
+  for (auto& b : bounce) b.release();
 }
 }  // namespace krk
 

@@ -564,6 +564,9 @@ int32_t group_finish(krk_group* g, uint32_t flags);
 int32_t sparse_ensure_room(krk_sparse* t, int64_t extra_rows);
 int32_t sparse_ensure_columns(krk_sparse* t, uint32_t state_mask);
 int32_t sparse_finish(krk_sparse* t, uint32_t flags);
+// The two halves of it, for calls that bring host data back in between: one wait then covers both.
+int32_t sparse_finish_begin(krk_sparse* t, uint32_t flags);
+int32_t sparse_finish_end(krk_sparse* t, uint32_t flags);
 // A new launch number for a launch that may insert up to n rows into t; call right before it.
 int32_t sparse_next_epoch(krk_sparse* t, int64_t n);
 // True when only a few more requests like the last one fit under the current row bound.

@@ -1843,11 +1843,18 @@ int32_t collect_counters(krk_sparse* t) {
 }
 
 // End of an API call: blocking calls wait, refresh the row count and surface device-side errors.
-int32_t sparse_finish(krk_sparse* t, uint32_t flags) {
+int32_t sparse_finish_begin(krk_sparse* t, uint32_t flags) {
   if (flags & KRK_ASYNC) return KRK_SUCCESS;
-  KRK_TRY(enqueue_counters(&t, 1, t->stream));
+  return enqueue_counters(&t, 1, t->stream);
+}
+int32_t sparse_finish_end(krk_sparse* t, uint32_t flags) {
+  if (flags & KRK_ASYNC) return KRK_SUCCESS;
   KRK_HIP(hipStreamSynchronize(t->stream));
   return collect_counters(t);
+}
+int32_t sparse_finish(krk_sparse* t, uint32_t flags) {
+  KRK_TRY(sparse_finish_begin(t, flags));
+  return sparse_finish_end(t, flags);
 }
 
 static InitK make_init_k(const krk_init& in, int64_t dim) {
@@ -2152,8 +2159,9 @@ int32_t krk_sparse_pull(krk_sparse* t, const uint64_t* ids, int64_t n, float* ou
     t->noted_version = t->layout_version;
   }
   if ((flags & KRK_ASYNC) && sparse_near_full(t)) KRK_TRY(sparse_publish(&t, 1, t->stream));
+  KRK_TRY(sparse_finish_begin(t, flags));
   KRK_TRY(t->output_back(out, (size_t)n * t->dim, flags, 1));
-  return sparse_finish(t, flags);
+  return sparse_finish_end(t, flags);
 }
 
 int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, const int64_t* offsets,
@@ -2250,8 +2258,9 @@ int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, co
     t->noted_version = t->layout_version;
   }
   if ((flags & KRK_ASYNC) && sparse_near_full(t)) KRK_TRY(sparse_publish(&t, 1, t->stream));
+  KRK_TRY(sparse_finish_begin(t, flags));
   KRK_TRY(t->output_back(out, (size_t)bags * t->dim, flags, 3));
-  return sparse_finish(t, flags);
+  return sparse_finish_end(t, flags);
 }
 
 int32_t krk_sparse_push(krk_sparse* t, const krk_optim* o, const uint64_t* ids, int64_t n,
@@ -2326,8 +2335,9 @@ int32_t krk_sparse_pull_wire(krk_sparse* t, const uint64_t* ids, int64_t n, void
   hipLaunchKernelGGL(rows_to_wire_kernel, dim3(strided_grid((int64_t)(bytes / 2))), dim3(kBlock), 0, t->stream,
                      d_rows, n, (int)t->dim, reinterpret_cast<uint16_t*>(d_reply));
   KRK_HIP(hipGetLastError());
+  KRK_TRY(sparse_finish_begin(t, 0));
   KRK_TRY(t->output_back(reinterpret_cast<uint8_t*>(reply), bytes, 0, 1));
-  return sparse_finish(t, 0);
+  return sparse_finish_end(t, 0);
 }
 
 int32_t krk_sparse_push_wire(krk_sparse* t, const krk_optim* o, const uint64_t* ids, int64_t n,
@@ -3006,10 +3016,14 @@ int32_t krk::group_plan(krk_group* g, const int64_t* offsets, GroupCall* call, i
   return KRK_SUCCESS;
 }
 
-int32_t krk::group_finish(krk_group* g, uint32_t flags) {
+static int32_t group_finish_begin(krk_group* g, uint32_t flags) {
   if (flags & KRK_ASYNC) return KRK_SUCCESS;
-  // one wait for all members: they share the group's stream
-  KRK_TRY(krk::enqueue_counters(g->tables.data(), (int)g->tables.size(), g->stream));
+  return krk::enqueue_counters(g->tables.data(), (int)g->tables.size(), g->stream);
+}
+
+// one wait for all members: they share the group's stream
+static int32_t group_finish_end(krk_group* g, uint32_t flags) {
+  if (flags & KRK_ASYNC) return KRK_SUCCESS;
   KRK_HIP(hipStreamSynchronize(g->stream));
   int32_t first = KRK_SUCCESS;
   for (krk_sparse* t : g->tables) {
@@ -3017,6 +3031,11 @@ int32_t krk::group_finish(krk_group* g, uint32_t flags) {
     if (rc != KRK_SUCCESS && first == KRK_SUCCESS) first = rc;
   }
   return first;
+}
+
+int32_t krk::group_finish(krk_group* g, uint32_t flags) {
+  KRK_TRY(group_finish_begin(g, flags));
+  return group_finish_end(g, flags);
 }
 
 extern "C" {
@@ -3164,8 +3183,9 @@ int32_t krk_group_pull(krk_group* g, const uint64_t* ids, const int64_t* offsets
     parts.stride[m] = (uint32_t)g->dim;
   }
   KRK_TRY(group_pull_enqueue(g, offsets, call, total, wide, parts, flags));
+  KRK_TRY(group_finish_begin(g, flags));
   KRK_TRY(g->output_back(out, (size_t)total * g->dim, flags, 1));
-  return group_finish(g, flags);
+  return group_finish_end(g, flags);
 }
 
 }  // extern "C"

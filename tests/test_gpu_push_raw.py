@@ -255,6 +255,21 @@ def test_dedup_sum_random_gradients_and_device_arrays(api, oracle):
     assert rc == api.E_ARGUMENT
 
 
+# 32 tiles of 4096 keys: up to there a sort's scatter adds the tiles' counts up by itself
+@pytest.mark.parametrize("n", [12289, 31 * 4096 + 1, 32 * 4096, 32 * 4096 + 1])
+@pytest.mark.parametrize("kind", ["distinct", "zipf", "one_id"])
+def test_push_raw_sort_tiles(api, oracle, n, kind):
+    rng = np.random.default_rng(n)
+    ids = {"distinct": splitmix64(np.arange(n, dtype=np.uint64)), "zipf": zipf_ids(rng, 1.2, 10**5, n),
+           "one_id": np.full(n, 9, np.uint64)}[kind]
+    t = api.SparseTable(8, api.Initializer.create(api.InitializerType.kConstant, {"value": "1"}))
+    t.Pull(ids)
+    grads = _dyadic_grads(rng, (n, 8))                  # sums stay below 2^11 in steps of 2^-12: exact
+    assert t.PushRaw(api.Optim.create(api.OptimType.kSGD), ids, grads, 0.5) == 0
+    u, gs = oracle.dedup_sum(ids, grads)
+    assert np.array_equal(t.Pull(u)[1], np.float32(1.0) - np.float32(0.5) * gs)
+
+
 # a lane of the short path looks at 4, 8 or 12 positions; 12288 of them are the most a table may bring
 @pytest.mark.parametrize("n", [4096, 4097, 8193, 12287, 12288, 12289])
 @pytest.mark.parametrize("shape", ["one_id", "one_bucket", "zipf"])

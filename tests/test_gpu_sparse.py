@@ -543,3 +543,27 @@ def test_wide_rows_group_push_ragged_members(api, oracle, name, type_, conf, dim
     for i, (t, r) in enumerate(zip(tables, refs)):
         assert_close(t.Pull(pool)[1], r.pull(pool)[1], "%s dim %d member %d" % (name, dim, i))
     grp.close()
+
+
+# rows of 64 bytes: 16384 of them are the 1 MB up to which host arguments pass through page-locked
+# memory; a request of another size before and behind each, so that kept buffers are reused
+@pytest.mark.parametrize("n", [1, 7, 16383, 16384, 16385])
+def test_host_arguments_around_the_bounce_limit(api, n):
+    rng = np.random.default_rng(n)
+    init = api.Initializer.create(api.InitializerType.kNormal, {"stddev": "0.01", "seed": "5"})
+    ids = rng.permutation(40_000)[:n].astype(np.uint64)
+    grads = rng.standard_normal((n, 16)).astype(np.float32)
+    other = np.arange(50_000, 50_300, dtype=np.uint64)
+    opt = api.Optim.create(api.OptimType.kAdagrad, {})
+    host, dev = api.SparseTable(16, init), api.SparseTable(16, init)
+    for k in range(2):
+        assert host.Pull(other[:100 * (k + 1)])[0] == 0 and dev.Pull(other[:100 * (k + 1)])[0] == 0
+        d_ids = api.DeviceArray.from_host(ids)
+        want = dev.Pull(d_ids)[1].to_host()
+        rc, got = host.Pull(ids)
+        assert rc == 0 and np.array_equal(got, want)
+        assert host.Push(opt, ids, grads, 0.1) == 0
+        assert dev.Push(opt, d_ids, api.DeviceArray.from_host(grads), 0.1) == 0
+    assert np.array_equal(host.Pull(ids)[1], dev.Pull(ids)[1])
+    missing = np.array([10**9], np.uint64)
+    assert host.Push(opt, missing, grads[:1], 0.1) == api.SPARSE_ID_NOT_EXIST
