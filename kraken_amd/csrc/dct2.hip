@@ -11,18 +11,18 @@
 // Shape of the work: Y[M, N] = X[M, K] * Basis[K, N] with M = n / 256 blocks (forward: K = 256,
 // N = keep; inverse: K = keep, N = 256), (1) folded in half by the basis' mirror symmetry and
 // (2) multiplied as six bf16 products per fp32 product on v_mfma_f32_32x32x16_bf16, both below.
-// A workgroup keeps its basis tile resident in LDS and walks over row tiles of 512 blocks; each
-// of its sixteen wavefronts owns 32 rows and holds their X values in registers.
+// A workgroup keeps its basis tile resident in LDS and walks over row tiles of 256 blocks (128 for
+// short requests); each of its wavefronts owns 32 rows and holds their X values in registers.
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 
 #include "krk_internal.h"
 
 namespace krk {
 
 constexpr int kDctB = 256;      // block length
-constexpr int kThreads = 1024;  // sixteen wavefronts, four per SIMD
-constexpr int kTileM = 512;     // rows (blocks) per output tile: 32 per wavefront
+constexpr int kWaveRows = 32;   // rows (blocks) of an output tile per wavefront
 
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -35,7 +35,7 @@ typedef float v2f __attribute__((ext_vector_type(2)));
 // the multiplies of the plain product, at one more fp32 rounding per input pair (forward) or
 // output pair (inverse).
 //
-// Shape of the work per workgroup: 512 blocks (rows) by 32 * NT folded columns, each folded
+// Shape of the work per workgroup: 256 blocks (rows) by 32 * NT folded columns, each folded
 // column carrying two results (forward: coefficients 2c and 2c + 1; inverse: positions j and
 // 255 - j), so a wavefront owns 32 rows and 2 * NT accumulator tiles, the first NT fed with the
 // first operand of a pair (sum, or even coefficient), the others with the second (difference,
@@ -44,9 +44,9 @@ typedef float v2f __attribute__((ext_vector_type(2)));
 // depends on h only, and the order in which the reduction indices are consumed is free as long
 // as the basis follows it. So lane (r, h) holds the operands of 8 or 16 consecutive folded
 // indices per slice (two or four float4 from the row and as many from its mirror image).
-// Sixteen wavefronts a workgroup (four per SIMD, 128 registers each): wavefronts never wait on
-// each other inside the loop, the next slice's loads are in flight while this one multiplies,
-// and what the wavefronts of a SIMD lose while one of them stores its tile, the other three fill in.
+// Eight wavefronts a workgroup (two per SIMD): wavefronts never wait on each other inside the loop,
+// the next slice's loads are in flight while this one multiplies, and what a wavefront of a SIMD
+// loses while it stores its tile, the other fills in.
 //
 // Measured on fp32 [4096, 16384], forward / inverse, microseconds:
 //                                                        keep 64      keep 128     keep 256
@@ -175,12 +175,14 @@ __global__ void dct2_basis3_kernel(__bf16* __restrict__ fwd3, __bf16* __restrict
   }
 }
 
-template <int NT, bool FWD>
-__global__ __launch_bounds__(kThreads) void dct2_split_kernel(const float* __restrict__ X, int64_t ldx,
+template <int NT, bool FWD, int WAVES>
+__global__ __launch_bounds__(WAVES * kWave) void dct2_split_kernel(const float* __restrict__ X, int64_t ldx,
                                                               const __bf16* __restrict__ B3,
                                                               float* __restrict__ Y, int64_t ldy,
                                                               int64_t M, int KF) {
   constexpr int NT2 = 2 * NT;
+  constexpr int kThreads = WAVES * kWave;
+  constexpr int kTileM = WAVES * kWaveRows;
   // Folded indices a lane holds per slice: one group of 8, or two where the accumulators leave
   // the registers for it (a row's loads are then whole 64-byte pieces, which memory serves
   // better; the narrow tiles are the ones that wait for memory). Either way the groups are taken
@@ -332,6 +334,15 @@ static int32_t ensure_basis(hipStream_t s) {
   return KRK_SUCCESS;
 }
 
+// Wavefronts of a workgroup. Eight, a row tile of 256 blocks: a workgroup more or less a compute unit
+// owns one whatever the width (the basis fills up to 98 KB of its LDS), and with sixteen a
+// request of a few thousand blocks kept only a few units busy while the largest was no faster
+// (forward + inverse as blocking calls, sixteen / eight, us: 10,000 blocks keep 64 56 / 42, keep 256
+// 72 / 51; 262,144 blocks 155 / 150 and 304 / 295). Four for requests so small that tiles of
+// 128 blocks still leave units idle (eight / four: 4000 blocks 42 / 38 and 50 / 48; 10,000 blocks
+// keep 256 51 / 60: a workgroup of four takes longer to lay its basis out).
+constexpr int64_t kFewRows = 4096;
+
 static int32_t dct2_run(const float* in, float* out, int64_t n, int32_t keep, uint32_t flags, bool forward) {
   KRK_TRY(ensure_runtime());
   KRK_TRY(check_flags(flags));
@@ -369,12 +380,13 @@ static int32_t dct2_run(const float* in, float* out, int64_t n, int32_t keep, ui
   const int nt = (NF % 64 == 0) ? 2 : 1;          // 64 folded columns a wavefront where the width allows
   const int gy = NF / (32 * nt);
   const size_t lds_bytes = (size_t)(KF / 8) * 3 * 2 * nt * 32 * 16;   // [KF / 8][3][2 nt][32] x 16 bytes
-  const int64_t tiles = (M + kTileM - 1) / kTileM;
+  const int waves = M <= kFewRows ? 4 : 8;
+  const int64_t tiles = (M + waves * kWaveRows - 1) / (waves * kWaveRows);
   int64_t gx = 256 / gy;                           // one workgroup a compute unit
   if (gx > tiles) gx = tiles;
   if (gx < 1) gx = 1;
   const __bf16* basis = forward ? g_basis3_fwd : g_basis3_inv;
-  const dim3 grid((unsigned)gx, (unsigned)gy), block(kThreads);
+  const dim3 grid((unsigned)gx, (unsigned)gy), block((unsigned)(waves * kWave));
   const int64_t ldx = forward ? kDctB : keep, ldy = forward ? keep : kDctB;
   hipError_t e = hipSuccess;
   auto launch = [&](auto kernel) {
@@ -384,12 +396,20 @@ static int32_t dct2_run(const float* in, float* out, int64_t n, int32_t keep, ui
     hipLaunchKernelGGL(kernel, grid, block, lds_bytes, s, d_in, ldx, basis, d_out, ldy, M, KF);
     e = hipGetLastError();
   };
-  if (!forward) {
-    launch(dct2_split_kernel<2, false>);
-  } else if (nt == 2) {
-    launch(dct2_split_kernel<2, true>);            // keep 128 and 256
+  auto launch_waves = [&](auto w) {
+    constexpr int WAVES = decltype(w)::value;
+    if (!forward) {
+      launch(dct2_split_kernel<2, false, WAVES>);
+    } else if (nt == 2) {
+      launch(dct2_split_kernel<2, true, WAVES>);   // keep 128 and 256
+    } else {
+      launch(dct2_split_kernel<1, true, WAVES>);   // keep 64 and 192
+    }
+  };
+  if (waves == 8) {
+    launch_waves(std::integral_constant<int, 8>{});
   } else {
-    launch(dct2_split_kernel<1, true>);            // keep 64 and 192
+    launch_waves(std::integral_constant<int, 4>{});
   }
   if (e == hipSuccess && host)
     e = hipMemcpy(out, d_out, sizeof(float) * (size_t)out_count, hipMemcpyDeviceToHost);

@@ -35,6 +35,23 @@ def test_forward_matches_scipy(dct2, blocks, keep):
     assert (np.abs(got - want) <= 1e-5 * scale + 1e-7).all()
 
 
+# row tiles of 128 blocks up to 4096 blocks, of 256 beyond: a last tile of one row, a full one, and
+# requests of more tiles than there are workgroups
+@pytest.mark.parametrize("blocks", [127, 129, 4096, 4097, 4353, 66_000])
+@pytest.mark.parametrize("keep", [64, 192, 256])
+def test_row_tiles(dct2, blocks, keep):
+    rng = np.random.default_rng(blocks + keep)
+    x = rng.standard_normal(blocks * 256).astype(np.float32)
+    scale = np.linalg.norm(x.reshape(-1, 256), axis=1, keepdims=True)
+    got = dct2.forward(x, keep)
+    assert (np.abs(got - _ref(x, keep)) <= 1e-6 * scale).all()
+    fft = pytest.importorskip("scipy.fft")
+    full = np.zeros((blocks, 256))
+    full[:, :keep] = got
+    want = fft.idct(full, type=2, norm="ortho", axis=1)
+    assert (np.abs(dct2.inverse(got, blocks * 256, keep).reshape(blocks, 256) - want) <= 1e-6 * scale).all()
+
+
 def test_known_vectors(dct2):
     """Closed forms: a constant block has only the k = 0 coefficient (= c * sqrt(256));
     a single cosine of the basis maps to a single coefficient."""
