@@ -90,7 +90,9 @@ __device__ __forceinline__ void store_tile(const v16f (&acc)[2 * NT], float* __r
           __builtin_nontemporal_store(v4f{acc[0][i], acc[2][i], acc[1][i], acc[3][i]},
                                       reinterpret_cast<v4f*>(row + lane_off));
         } else {
-          __builtin_nontemporal_store(v2f{acc[0][i], acc[1][i]}, reinterpret_cast<v2f*>(row + lane_off));
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+            __builtin_nontemporal_store(v2f{acc[t][i], acc[NT + t][i]}, reinterpret_cast<v2f*>(row + lane_off + 2 * t));
         }
       } else {
         if constexpr (NT == 2) {
@@ -342,6 +344,7 @@ static int32_t ensure_basis(hipStream_t s) {
 // 128 blocks still leave units idle (eight / four: 4000 blocks 42 / 38 and 50 / 48; 10,000 blocks
 // keep 256 51 / 60: a workgroup of four takes longer to lay its basis out).
 constexpr int64_t kFewRows = 4096;
+constexpr int64_t kWholeRows = 2 * 256 * 8 * kWaveRows;
 
 static int32_t dct2_run(const float* in, float* out, int64_t n, int32_t keep, uint32_t flags, bool forward) {
   KRK_TRY(ensure_runtime());
@@ -377,10 +380,14 @@ static int32_t dct2_run(const float* in, float* out, int64_t n, int32_t keep, ui
   // pairs (inverse), the columns over keep / 2 coefficient pairs (forward) or 128 position pairs
   const int KF = forward ? kFoldB : keep / 2;
   const int NF = forward ? keep / 2 : kFoldB;
-  const int nt = (NF % 64 == 0) ? 2 : 1;          // 64 folded columns a wavefront where the width allows
+  const int waves = M <= kFewRows ? 4 : 8;
+  // 64 folded columns a wavefront where the width allows. Forward keep 192 takes all of its 96 in one
+  // workgroup from two row tiles a workgroup on, so that X is read once instead of three times
+  // (forward + inverse: 262,144 blocks 285 -> 260 us, 160,000 187 -> 170; 80,000 116 either way,
+  // 10,000 47 -> 56: 147 KB of basis to lay out in a third of the workgroups).
+  const int nt = (NF % 64 == 0) ? 2 : (NF == 96 && M >= kWholeRows ? 3 : 1);
   const int gy = NF / (32 * nt);
   const size_t lds_bytes = (size_t)(KF / 8) * 3 * 2 * nt * 32 * 16;   // [KF / 8][3][2 nt][32] x 16 bytes
-  const int waves = M <= kFewRows ? 4 : 8;
   const int64_t tiles = (M + waves * kWaveRows - 1) / (waves * kWaveRows);
   int64_t gx = 256 / gy;                           // one workgroup a compute unit
   if (gx > tiles) gx = tiles;
@@ -402,6 +409,8 @@ static int32_t dct2_run(const float* in, float* out, int64_t n, int32_t keep, ui
       launch(dct2_split_kernel<2, false, WAVES>);
     } else if (nt == 2) {
       launch(dct2_split_kernel<2, true, WAVES>);   // keep 128 and 256
+    } else if (nt == 3) {
+      if constexpr (WAVES == 8) launch(dct2_split_kernel<3, true, WAVES>);   // keep 192
     } else {
       launch(dct2_split_kernel<1, true, WAVES>);   // keep 64 and 192
     }

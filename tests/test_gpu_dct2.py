@@ -37,8 +37,9 @@ def test_forward_matches_scipy(dct2, blocks, keep):
 
 # row tiles of 128 blocks up to 4096 blocks, of 256 beyond: a last tile of one row, a full one, and
 # requests of more tiles than there are workgroups
-@pytest.mark.parametrize("blocks", [127, 129, 4096, 4097, 4353, 66_000])
-@pytest.mark.parametrize("keep", [64, 192, 256])
+# (131,072 blocks: keep 192 in one column group)
+@pytest.mark.parametrize("blocks,keep", [(b, k) for b in (127, 129, 4096, 4097, 4353, 66_000) for k in (64, 192, 256)] +
+                         [(131_071, 192), (131_072, 192), (131_073, 192)])
 def test_row_tiles(dct2, blocks, keep):
     rng = np.random.default_rng(blocks + keep)
     x = rng.standard_normal(blocks * 256).astype(np.float32)
