@@ -1100,7 +1100,7 @@ static int pick_tile(int64_t cnt) {
 // take is six to nine launches: an embedding step of 10,000 ids of 16 floats, forward, backward,
 // forward, 61 us with it and 39 us with this): two launches, no carry levels, no global sort.
 //   1. ids -> rows for every position, over the whole chip (rows_of_ids / group_rows_of_ids).
-//   2. bucket_push_kernel, one workgroup of 1024 lanes for each of a table's 8 to 32 buckets
+//   2. bucket_push_kernel, one workgroup of 1024 lanes for each of a table's 8 to 128 buckets
 //      (bucket = row mod the number of buckets; as many as keep the request at about one
 //      workgroup per compute unit), so that both one table and 26 tables use much of the chip:
 //      a. the workgroup reads its table's row numbers and keeps the positions of its bucket, in
@@ -1134,7 +1134,11 @@ constexpr int kSortBlock = 1024;
 constexpr int kSortItems = 12;
 constexpr int kSortMax = kSortBlock * kSortItems;      // ids per table
 constexpr int kSortWaves = kSortBlock / kWave;
-constexpr int kMaxBucketBits = 5;                      // up to 32 buckets a table
+// Up to 128 buckets a table. With 32 a request of one table kept 32 compute units busy, and where the
+// rows are wide or the request long their lane groups took several rounds of runs (enqueued back to
+// back, 32 / 128 buckets, us: 8192 ids of 64 floats, Adam, 30.8 / 24.4; 12,000 of them 33.0 / 26.6;
+// 4000 ids of 16 floats, Zipf 1.3, 20.8 / 18.7; 8192 of 16 20.7 / 19.8; 100 of 8 15.8 / 16.1).
+constexpr int kMaxBucketBits = 7;
 constexpr int kDigitBits = 9;
 constexpr int kDigits = 1 << kDigitBits;
 constexpr int kRunAhead = 8;                           // gradient rows requested ahead of the sums

@@ -283,9 +283,10 @@ def test_push_raw_short_path_sizes(api, oracle, n, shape):
     if shape == "one_id":
         ids = np.full(n, 4242, np.uint64)
     elif shape == "one_bucket":
-        pool = splitmix64(np.arange(450_000, dtype=np.uint64))
-        t.Pull(pool)
-        ids = rng.permutation(pool[t.lookup(pool) % 32 == 0])[:n]
+        pool = splitmix64(np.arange(1_650_000, dtype=np.uint64))
+        for part in np.array_split(pool, 8):
+            t.Pull(part)
+        ids = rng.permutation(pool[t.lookup(pool) % 128 == 0])[:n]      # the buckets are row mod 8..128
         assert ids.size == n
     else:
         ids = zipf_ids(rng, 1.05, 10**5, n)
