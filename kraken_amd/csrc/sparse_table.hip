@@ -1670,12 +1670,12 @@ static void await_published(krk_sparse* t, int64_t extra_rows) {
   for (;;) {
     tighten_bound(t);
     const int64_t need = t->size_ub + extra_rows;
-    if (need <= t->row_cap && (uint64_t)need * 2 <= t->slot_cap) return;
-    if ((uint32_t)(__atomic_load_n(t->host_pub, __ATOMIC_ACQUIRE) >> 32) == t->epoch) return;
+    if (need <= t->row_cap && (uint64_t)need * 2 <= t->slot_cap) break;
+    if ((uint32_t)(__atomic_load_n(t->host_pub, __ATOMIC_ACQUIRE) >> 32) == t->epoch) break;
     if (hipStreamQuery(t->stream) != hipErrorNotReady) break;
     std::this_thread::yield();
   }
-  (void)hipGetLastError();   // "not ready" is no failure of a later call
+  if (hipPeekAtLastError() == hipErrorNotReady) (void)hipGetLastError();   // no failure of a later call
 }
 
 // Room for `extra_rows` more rows: records, row keys, and an index at most half full.
