@@ -74,8 +74,12 @@ Tensor new_rows(at::IntArrayRef sizes, const Tensor& like) {
   return at::empty(sizes, at::TensorOptions().dtype(at::kFloat).device(like.device()));
 }
 
+Tensor new_zeros(at::IntArrayRef sizes, const Tensor& like) {
+  return at::zeros(sizes, at::TensorOptions().dtype(at::kFloat).device(like.device()));
+}
+
 // The gradient rows of `g` where they lie, `stride` floats apart, if the kernels can read them there;
-// otherwise of a contiguous float copy, which `keep` then holds.
+// otherwise of a contiguous float copy. `keep` holds whichever it is.
 struct Rows {
   Tensor keep;
   int64_t stride = 0;
@@ -108,6 +112,14 @@ Rows rows_of(const Tensor& g, int64_t dim) {
     }
   }
   r.keep = g.contiguous().to(at::kFloat);
+  return r;
+}
+
+// The gradient rows of an output the loss never used: one row of zeros that every position reads. The
+// rows still take their step with it (moments decay, counters advance, weights decay).
+Rows zero_rows(const Tensor& like, int64_t dim) {
+  Rows r;
+  r.keep = new_zeros({dim}, like);
   return r;
 }
 
@@ -241,11 +253,11 @@ struct CombineBackward : Node {
   std::vector<SavedVariable> ids;
   variable_list apply(variable_list&& grads) override {
     void* stream = current_stream();
-    Tensor zeros;                  // one row for the outputs the loss never used: every position reads it
     for (const Combine::Group& g : c->groups) {
       std::vector<krk_part> parts(g.members.size());
       std::vector<Tensor> keep;
       keep.reserve(2 * g.members.size());
+      Rows zeros;
       for (size_t m = 0; m < g.members.size(); ++m) {
         const int i = g.members[m];
         Tensor saved = ids[i].unpack();
@@ -258,10 +270,9 @@ struct CombineBackward : Node {
           p.stride = r.stride;
           keep.push_back(std::move(r.keep));
         } else {
-          if (!zeros.defined() || zeros.numel() < g.dim)
-            zeros = at::zeros({g.dim}, at::TensorOptions().dtype(at::kFloat).device(saved.device()));
-          p.rows = zeros.mutable_data_ptr<float>();
-          p.stride = 0;
+          if (!zeros.keep.defined()) zeros = zero_rows(saved, g.dim);
+          p.rows = zeros.ptr();
+          p.stride = zeros.stride;
         }
         keep.push_back(std::move(saved));
       }
@@ -327,26 +338,32 @@ struct CombineJaggedBackward : Node {
       std::vector<krk_pooled_part> parts(g.members.size());
       std::vector<Tensor> keep;
       keep.reserve(3 * g.members.size());
+      Rows zeros;
       int64_t total = 0;
       for (size_t m = 0; m < g.members.size(); ++m) {
         const int i = g.members[m];
         krk_pooled_part& p = parts[m];
         p = krk_pooled_part{};
-        if (!grads[i].defined()) continue;     // an output the loss never used: nothing to push
         Tensor saved = ids[i].unpack(), off = offsets[i].unpack();
-        Rows r = rows_of(grads[i], g.dim);
         p.ids = id_ptr(saved);
         p.n = saved.numel();
         p.offsets = off_ptr(off);
         p.bags = off.numel() - 1;
         p.weights = float_ptr(weights[i]);
-        p.rows = r.ptr();
-        p.stride = r.stride;
         p.mode = modes[i];
+        if (grads[i].defined()) {
+          Rows r = rows_of(grads[i], g.dim);
+          p.rows = r.ptr();
+          p.stride = r.stride;
+          keep.push_back(std::move(r.keep));
+        } else {
+          if (!zeros.keep.defined()) zeros = zero_rows(saved, g.dim);
+          p.rows = zeros.ptr();
+          p.stride = zeros.stride;
+        }
         total += std::max(p.n, p.bags);
         keep.push_back(std::move(saved));
         keep.push_back(std::move(off));
-        keep.push_back(std::move(r.keep));
       }
       KRK_CALL(krk_group_set_stream, g.h, stream);
       const int32_t rc = total > kCombinedMax
@@ -360,7 +377,10 @@ struct CombineJaggedBackward : Node {
         const krk_pooled_part& p = parts[m];
         if (p.n == 0 || p.bags == 0) continue;
         const int i = g.members[m];
-        const Tensor rows = grads[i].contiguous().to(at::kFloat);
+        // a call of its own takes a row a bag
+        const Tensor rows = grads[i].defined()
+                                ? grads[i].contiguous().to(at::kFloat)
+                                : new_zeros({p.bags, g.dim}, zeros.keep);
         KRK_CALL(krk_sparse_push_pooled, c->tables[i], c->optim, p.ids, p.n, p.offsets, p.bags, p.weights, p.mode,
                  float_ptr(rows), g.dim, (float)c->lr, kFlags);
       }

@@ -1,0 +1,128 @@
+"""The gradients that autograd hands to the embedding modules in all the forms it has: none at all,
+zeros that were never made, blocks of a wider matrix that start anywhere, one value expanded over
+the batch. Whatever the form, the tables end as the oracle's, pushed with the same gradients in plain
+arrays (an output without a gradient pushes zeros, pytorch/combine_embedding.py:22-31)."""
+import numpy as np
+import pytest
+
+from util import assert_close, make_optims
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+KINDS = ["embedding", "jagged", "combine", "combine_jagged"]
+DIM = 16
+LR = 0.5
+
+
+@pytest.fixture(scope="module")
+def mods():
+    if not torch.cuda.is_available():
+        pytest.skip("torch sees no GPU")
+    from kraken_amd import api, torch_embedding
+    api.lib()
+    return api, torch_embedding
+
+
+class Pair:
+    """A module of `kind` over the oracle's tables with the same rows and optimizer."""
+
+    def __init__(self, mods, oracle, kind, optim=(1, {}), seed=40):
+        self.api, self.te = mods
+        self.oracle, self.kind = oracle, kind
+        self.jagged = "jagged" in kind
+        self.tables = 2 if kind.startswith("combine") else 1
+        api, te = mods
+        inits = [api.Initializer.create(api.InitializerType.kNormal, {"stddev": "0.01", "seed": str(seed + i)})
+                 for i in range(self.tables)]
+        self.refs = [oracle.SparseTable(DIM, oracle.init(oracle.INIT_NORMAL, 0.0, 0.01, seed=seed + i))
+                     for i in range(self.tables)]
+        self.o_ref, self.o_gpu = make_optims(oracle, api, *optim)
+        if kind == "embedding":
+            self.mod = te.Embedding(DIM, inits[0], self.o_gpu, LR)
+        elif kind == "jagged":
+            self.mod = te.JaggedEmbedding(DIM, inits[0], self.o_gpu, LR, mode="sum")
+        elif kind == "combine":
+            self.mod = te.CombineEmbedding([DIM] * 2, inits, self.o_gpu, LR)
+        else:
+            self.mod = te.CombineJaggedEmbedding([DIM] * 2, inits, ["sum", "mean"], None, self.o_gpu, LR)
+        self.param = self.mod.sparse_table if self.tables == 1 else self.mod.combine_sparse_table
+        self.modes = ["sum", "mean"]
+
+    def draw(self, rng, rows, span=200):
+        """-> per table (ids, offsets or None): `rows` output rows each"""
+        batch = []
+        for _ in range(self.tables):
+            if self.jagged:
+                off = np.concatenate([[0], np.cumsum(rng.choice([1, 2, 4], size=rows))]).astype(np.int64)
+                batch.append((rng.integers(0, span, size=int(off[-1])).astype(np.uint64), off))
+            else:
+                batch.append((rng.integers(0, span, size=rows).astype(np.uint64), None))
+        return batch
+
+    def tensors(self, batch):
+        return [(torch.from_numpy(ids.astype(np.int64)).cuda(), None if off is None else torch.from_numpy(off).cuda())
+                for ids, off in batch]
+
+    def forward(self, batch, tensors=None):
+        """-> the module's outputs as a list, checked against the oracle's rows"""
+        t = tensors or self.tensors(batch)
+        if self.kind == "embedding":
+            outs = [self.mod(t[0][0])]
+        elif self.kind == "jagged":
+            outs = [self.mod(*t[0])]
+        elif self.kind == "combine":
+            outs = self.mod([ids for ids, _ in t])
+        else:
+            outs = self.mod([self.te.JaggedTensor(ids, off) for ids, off in t])
+        for i, (ids, off) in enumerate(batch):
+            u, inv = self.oracle.dedup(ids)
+            rows = self.refs[i].pull(u)[1][inv]
+            want = rows if off is None else self.oracle.jagged_forward(rows, off, self.modes[i], 0.0)
+            assert_close(outs[i].detach().cpu().numpy(), want, "forward of table %d" % i, rtol=1e-5, atol=1e-6)
+        return outs
+
+    def push(self, batch, grads):
+        """the oracle's update; grads: an array per table, [its output rows, DIM]"""
+        for i, ((ids, off), g) in enumerate(zip(batch, grads)):
+            vg = g if off is None else self.oracle.jagged_backward(off, g, self.modes[i])
+            u, sums = self.oracle.dedup_sum(ids, vg)
+            assert self.refs[i].push(self.o_ref, u, sums, LR) == 0
+
+    def check(self, what):
+        torch.cuda.synchronize()
+        tables = [self.param.table()] if self.tables == 1 else self.param.tables()
+        for i, (t, r) in enumerate(zip(tables, self.refs)):
+            rid, rval, _, _ = r.export()
+            assert len(t) == len(r)
+            assert_close(t.Pull(rid)[1], rval, "%s: rows of table %d" % (what, i), rtol=1e-5, atol=1e-6)
+
+
+def _coef(rng, rows, n):
+    return [(rng.integers(-8, 9, size=(rows, DIM)) / 16.0).astype(np.float32) for _ in range(n)]
+
+
+def _loss(outs, coefs):
+    return sum((o * torch.from_numpy(c).cuda()).sum() for o, c in zip(outs, coefs) if c is not None)
+
+
+# optimizers for which a gradient of zeros still moves the row, its state or its counter
+MOVING = [("adam", 1, {}), ("momentum", 3, {"momentum": 0.9}), ("sgd_decay", 3, {"weight_decay": 0.05}),
+          ("rmsprop", 2, {"momentum": 0.7})]
+
+
+@pytest.mark.parametrize("optim", MOVING, ids=[m[0] for m in MOVING])
+@pytest.mark.parametrize("kind", ["combine", "combine_jagged"])
+def test_output_without_gradient_pushes_zeros(mods, oracle, kind, optim):
+    """A loss that uses one of two outputs: the rows of the other take their step with zeros."""
+    p = Pair(mods, oracle, kind, optim[1:])
+    rng = np.random.default_rng(1)
+    for step in range(3):
+        batch = p.draw(rng, 96)
+        outs = p.forward(batch)
+        coefs = _coef(rng, 96, 2)
+        used = [coefs[0], None if step == 1 else coefs[1]]
+        _loss(outs, used).backward()
+        p.push(batch, [np.zeros_like(c) if u is None else c for c, u in zip(coefs, used)])
+    p.check("after a step without the second output")
