@@ -346,6 +346,17 @@ def _flags(*arrays, extra=0):
     return extra
 
 
+def _take_handle(obj):
+    """The handle that obj.h held, which obj no longer has. The c_void_p itself says so too: native code
+    that keeps it (torch_embedding) passes a null handle from here on."""
+    h = getattr(obj, "h", None)
+    obj.h = None
+    if not h:
+        return None
+    raw, h.value = h.value, None
+    return raw
+
+
 class SparseTable:
     """ps/sparse_table.h. Pull/Push return the reference's int32 error code."""
 
@@ -357,9 +368,9 @@ class SparseTable:
         self.h = h
 
     def close(self):
-        if getattr(self, "h", None):
-            lib().krk_sparse_destroy(self.h)
-            self.h = None
+        h = _take_handle(self)
+        if h:
+            lib().krk_sparse_destroy(h)
 
     __del__ = close
 
@@ -573,9 +584,9 @@ class TableGroup:
         self.h = h
 
     def close(self):
-        if getattr(self, "h", None):
-            lib().krk_group_destroy(self.h)
-            self.h = None
+        h = _take_handle(self)
+        if h:
+            lib().krk_group_destroy(h)
 
     __del__ = close
 

@@ -22,6 +22,7 @@
 
 #include <algorithm>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "kraken_hip.h"
@@ -134,10 +135,50 @@ std::shared_ptr<N> new_node(const Tensor& param) {
   return node;
 }
 
+// ---- what the Python side owns ------------------------------------------------------------------
+// A value inside a ctypes object (a handle's c_void_p, an optimizer's struct). The object is kept as
+// long as it is bound, so the address stays good whatever becomes of the Python objects around it;
+// its owner may change the value, or bind another object, at any time (api.SparseTable.close() stores
+// a null handle, which the C ABI answers with an error). Reading takes no interpreter lock: the
+// value is copied under a lock of its own.
+template <typename T>
+class Bound {
+ public:
+  explicit Bound(const py::object& o) : object_(o), value_(address(o)) {}
+  ~Bound() {
+    if (!Py_IsInitialized()) {
+      (void)object_.release();
+      return;
+    }
+    py::gil_scoped_acquire gil;      // the last node of a graph dies in the engine's thread
+    object_ = py::object();
+  }
+  Bound(const Bound&) = delete;
+  Bound& operator=(const Bound&) = delete;
+  T get() const {
+    std::lock_guard<std::mutex> lk(mu_);
+    return *value_;
+  }
+  void bind(py::object o) {          // the caller holds the interpreter lock; `o` leaves with the old object
+    T* value = address(o);
+    std::lock_guard<std::mutex> lk(mu_);
+    std::swap(object_, o);
+    value_ = value;
+  }
+
+ private:
+  static T* address(const py::object& o) {
+    return reinterpret_cast<T*>(py::module_::import("ctypes").attr("addressof")(o).cast<uintptr_t>());
+  }
+  mutable std::mutex mu_;
+  py::object object_;
+  T* value_;
+};
+
 // ---- one table --------------------------------------------------------------------------------
 struct Table {
-  krk_sparse* h;
-  const krk_optim* optim;
+  Bound<krk_sparse*> h;
+  Bound<krk_optim> optim;
   int64_t dim;
   double lr;
 };
@@ -149,8 +190,10 @@ struct EmbeddingBackward : Node {
   variable_list apply(variable_list&& grads) override {
     const Tensor saved = ids.unpack();
     const Tensor g = grads[0].contiguous().to(at::kFloat);
-    KRK_CALL(krk_sparse_set_stream, table->h, current_stream());
-    KRK_CALL(krk_sparse_push_raw, table->h, table->optim, id_ptr(saved), saved.numel(), float_ptr(g), table->dim,
+    krk_sparse* h = table->h.get();
+    const krk_optim optim = table->optim.get();
+    KRK_CALL(krk_sparse_set_stream, h, current_stream());
+    KRK_CALL(krk_sparse_push_raw, h, &optim, id_ptr(saved), saved.numel(), float_ptr(g), table->dim,
              (float)table->lr, kFlags | KRK_IDS_AS_PULLED);
     return variable_list(1);
   }
@@ -164,10 +207,11 @@ Tensor embedding(const TablePtr& table, const Tensor& param, const Tensor& indic
   sizes.push_back(table->dim);
   Tensor out = new_rows(sizes, ids);
   const bool record = recording(param);
-  KRK_CALL(krk_sparse_set_stream, table->h, current_stream());
+  krk_sparse* h = table->h.get();
+  KRK_CALL(krk_sparse_set_stream, h, current_stream());
   // the table notes where it found every id: backward pushes gradients for this very tensor
   // (autograd keeps it alive and unchanged), so its look-up need not be repeated
-  KRK_CALL(krk_sparse_pull, table->h, id_ptr(ids), ids.numel(), out.mutable_data_ptr<float>(),
+  KRK_CALL(krk_sparse_pull, h, id_ptr(ids), ids.numel(), out.mutable_data_ptr<float>(),
            kFlags | (record ? KRK_NOTE_ROWS : 0u));
   if (record) {
     auto node = new_node<EmbeddingBackward>(param);
@@ -186,8 +230,10 @@ struct JaggedBackward : Node {
   variable_list apply(variable_list&& grads) override {
     const Tensor saved = ids.unpack(), off = offsets.unpack();
     const Tensor g = grads[0].contiguous().to(at::kFloat);
-    KRK_CALL(krk_sparse_set_stream, table->h, current_stream());
-    KRK_CALL(krk_sparse_push_pooled, table->h, table->optim, id_ptr(saved), saved.numel(), off_ptr(off),
+    krk_sparse* h = table->h.get();
+    const krk_optim optim = table->optim.get();
+    KRK_CALL(krk_sparse_set_stream, h, current_stream());
+    KRK_CALL(krk_sparse_push_pooled, h, &optim, id_ptr(saved), saved.numel(), off_ptr(off),
              off.numel() - 1, float_ptr(weights), mode, float_ptr(g), table->dim, (float)table->lr,
              kFlags | KRK_IDS_AS_PULLED);
     return variable_list(1);
@@ -208,8 +254,9 @@ Tensor jagged(const TablePtr& table, const Tensor& param, const Tensor& indices,
   const int64_t bags = off.numel() - 1;
   Tensor out = new_rows({bags, table->dim}, ids);
   const bool record = recording(param);
-  KRK_CALL(krk_sparse_set_stream, table->h, current_stream());
-  KRK_CALL(krk_sparse_pull_pooled, table->h, id_ptr(ids), ids.numel(), off_ptr(off), bags, float_ptr(w), mode,
+  krk_sparse* h = table->h.get();
+  KRK_CALL(krk_sparse_set_stream, h, current_stream());
+  KRK_CALL(krk_sparse_pull_pooled, h, id_ptr(ids), ids.numel(), off_ptr(off), bags, float_ptr(w), mode,
            (float)patch, out.mutable_data_ptr<float>(), kFlags | (record ? KRK_NOTE_ROWS : 0u));
   if (record) {
     auto node = new_node<JaggedBackward>(param);
@@ -227,14 +274,14 @@ Tensor jagged(const TablePtr& table, const Tensor& param, const Tensor& indices,
 // Tables of equal dimension form one group of the engine; mixed dimensions give several groups.
 struct Combine {
   struct Group {
-    krk_group* h;
+    std::unique_ptr<Bound<krk_group*>> h;
     int64_t dim;
     std::vector<int> members;      // positions of its tables in the request
   };
   std::vector<Group> groups;
-  std::vector<krk_sparse*> tables;
+  std::vector<std::unique_ptr<Bound<krk_sparse*>>> tables;
   std::vector<int64_t> dims;
-  const krk_optim* optim;
+  Bound<krk_optim> optim;
   double lr;
 };
 using CombinePtr = std::shared_ptr<Combine>;
@@ -253,7 +300,9 @@ struct CombineBackward : Node {
   std::vector<SavedVariable> ids;
   variable_list apply(variable_list&& grads) override {
     void* stream = current_stream();
+    const krk_optim optim = c->optim.get();
     for (const Combine::Group& g : c->groups) {
+      krk_group* h = g.h->get();
       std::vector<krk_part> parts(g.members.size());
       std::vector<Tensor> keep;
       keep.reserve(2 * g.members.size());
@@ -276,8 +325,8 @@ struct CombineBackward : Node {
         }
         keep.push_back(std::move(saved));
       }
-      KRK_CALL(krk_group_set_stream, g.h, stream);
-      KRK_CALL(krk_group_push_raw_parts, g.h, c->optim, parts.data(), g.dim, (float)c->lr, kFlags | KRK_IDS_AS_PULLED);
+      KRK_CALL(krk_group_set_stream, h, stream);
+      KRK_CALL(krk_group_push_raw_parts, h, &optim, parts.data(), g.dim, (float)c->lr, kFlags | KRK_IDS_AS_PULLED);
     }
     return variable_list(1);
   }
@@ -311,8 +360,9 @@ std::vector<Tensor> combine(const CombinePtr& c, const Tensor& param, const std:
       parts[m] = krk_part{id_ptr(ids[i]), ids[i].numel(), base + at, g.dim};
       at += ids[i].numel() * g.dim;
     }
-    KRK_CALL(krk_group_set_stream, g.h, stream);
-    KRK_CALL(krk_group_pull_parts, g.h, parts.data(), kFlags | (record ? KRK_NOTE_ROWS : 0u));
+    krk_group* h = g.h->get();
+    KRK_CALL(krk_group_set_stream, h, stream);
+    KRK_CALL(krk_group_pull_parts, h, parts.data(), kFlags | (record ? KRK_NOTE_ROWS : 0u));
   }
   if (record) {
     auto node = new_node<CombineBackward>(param);
@@ -327,6 +377,13 @@ std::vector<Tensor> combine(const CombinePtr& c, const Tensor& param, const std:
 // Groups whose request is larger than this are served a table at a time.
 constexpr int64_t kCombinedMax = (int64_t)1 << 28;
 
+// A pooled request is made of the tables' own calls: one whose table was closed is refused, also where
+// the group still holds the table.
+void check_open(const Combine& c) {
+  for (const auto& t : c.tables)
+    if (!t->get()) KRK_CALL(krk_sparse_sync, nullptr);
+}
+
 struct CombineJaggedBackward : Node {
   CombinePtr c;
   std::vector<int> modes;
@@ -334,7 +391,10 @@ struct CombineJaggedBackward : Node {
   std::vector<Tensor> weights;
   variable_list apply(variable_list&& grads) override {
     void* stream = current_stream();
+    const krk_optim optim = c->optim.get();
+    check_open(*c);
     for (const Combine::Group& g : c->groups) {
+      krk_group* h = g.h->get();
       std::vector<krk_pooled_part> parts(g.members.size());
       std::vector<Tensor> keep;
       keep.reserve(3 * g.members.size());
@@ -365,10 +425,10 @@ struct CombineJaggedBackward : Node {
         keep.push_back(std::move(saved));
         keep.push_back(std::move(off));
       }
-      KRK_CALL(krk_group_set_stream, g.h, stream);
+      KRK_CALL(krk_group_set_stream, h, stream);
       const int32_t rc = total > kCombinedMax
                              ? KRK_E_CAPACITY
-                             : krk_group_push_pooled_parts(g.h, c->optim, parts.data(), g.dim, (float)c->lr,
+                             : krk_group_push_pooled_parts(h, &optim, parts.data(), g.dim, (float)c->lr,
                                                            kFlags | KRK_IDS_AS_PULLED);
       if (rc == KRK_SUCCESS) continue;
       if (rc != KRK_E_CAPACITY) fail(rc, "krk_group_push_pooled_parts");
@@ -381,8 +441,8 @@ struct CombineJaggedBackward : Node {
         const Tensor rows = grads[i].defined()
                                 ? grads[i].contiguous().to(at::kFloat)
                                 : new_zeros({p.bags, g.dim}, zeros.keep);
-        KRK_CALL(krk_sparse_push_pooled, c->tables[i], c->optim, p.ids, p.n, p.offsets, p.bags, p.weights, p.mode,
-                 float_ptr(rows), g.dim, (float)c->lr, kFlags);
+        KRK_CALL(krk_sparse_push_pooled, c->tables[i]->get(), &optim, p.ids, p.n, p.offsets, p.bags, p.weights,
+                 p.mode, float_ptr(rows), g.dim, (float)c->lr, kFlags);
       }
     }
     return variable_list(1);
@@ -405,6 +465,7 @@ std::vector<Tensor> combine_jagged(const CombinePtr& c, const Tensor& param, con
     throw py::value_error("one jagged batch per table");
   const bool record = recording(param);
   void* stream = current_stream();
+  check_open(*c);
   std::vector<Tensor> outs(n), ids(n), offsets(n), weights(n);
   for (const Combine::Group& g : c->groups) {
     std::vector<krk_pooled_part> parts(g.members.size());
@@ -427,16 +488,17 @@ std::vector<Tensor> combine_jagged(const CombinePtr& c, const Tensor& param, con
                                  base + at, g.dim, modes[i], (float)patches[i]};
       at += mine * g.dim;
     }
-    KRK_CALL(krk_group_set_stream, g.h, stream);
+    krk_group* h = g.h->get();
+    KRK_CALL(krk_group_set_stream, h, stream);
     const int32_t rc =
         total > kCombinedMax ? KRK_E_CAPACITY
-                             : krk_group_pull_pooled_parts(g.h, parts.data(), kFlags | (record ? KRK_NOTE_ROWS : 0u));
+                             : krk_group_pull_pooled_parts(h, parts.data(), kFlags | (record ? KRK_NOTE_ROWS : 0u));
     if (rc == KRK_SUCCESS) continue;
     if (rc != KRK_E_CAPACITY) fail(rc, "krk_group_pull_pooled_parts");
     for (size_t m = 0; m < g.members.size(); ++m) {
       const krk_pooled_part& p = parts[m];
-      KRK_CALL(krk_sparse_pull_pooled, c->tables[g.members[m]], p.ids, p.n, p.offsets, p.bags, p.weights, p.mode,
-               p.patch_value, p.rows, kFlags);
+      KRK_CALL(krk_sparse_pull_pooled, c->tables[g.members[m]]->get(), p.ids, p.n, p.offsets, p.bags, p.weights,
+               p.mode, p.patch_value, p.rows, kFlags);
     }
   }
   if (record) {
@@ -453,29 +515,27 @@ std::vector<Tensor> combine_jagged(const CombinePtr& c, const Tensor& param, con
 
 }  // namespace
 
-// The Python side hands over addresses of objects it keeps alive with the Parameter, which every
-// node keeps alive through its edge.
+// Handles and optimizers come as the ctypes objects that hold them (see Bound).
 PYBIND11_MODULE(_torch_native, m) {
   using release = py::call_guard<py::gil_scoped_release>;
   py::class_<Table, TablePtr>(m, "Table")
-      .def(py::init([](uintptr_t h, uintptr_t optim, int64_t dim, double lr) {
-        return std::make_shared<Table>(
-            Table{reinterpret_cast<krk_sparse*>(h), reinterpret_cast<const krk_optim*>(optim), dim, lr});
+      .def(py::init([](const py::object& h, const py::object& optim, int64_t dim, double lr) {
+        return std::shared_ptr<Table>(new Table{Bound<krk_sparse*>(h), Bound<krk_optim>(optim), dim, lr});
       }))
+      .def("bind_table", [](Table& t, const py::object& h) { t.h.bind(h); })
+      .def("bind_optim", [](Table& t, const py::object& optim) { t.optim.bind(optim); })
       .def_readwrite("lr", &Table::lr);
   py::class_<Combine, CombinePtr>(m, "Combine")
-      .def(py::init([](const std::vector<std::tuple<uintptr_t, int64_t, std::vector<int>>>& groups,
-                       const std::vector<uintptr_t>& tables, const std::vector<int64_t>& dims, uintptr_t optim,
-                       double lr) {
-        auto c = std::make_shared<Combine>();
+      .def(py::init([](const std::vector<std::tuple<py::object, int64_t, std::vector<int>>>& groups,
+                       const std::vector<py::object>& tables, const std::vector<int64_t>& dims,
+                       const py::object& optim, double lr) {
+        std::shared_ptr<Combine> c(new Combine{{}, {}, dims, Bound<krk_optim>(optim), lr});
         for (const auto& [h, dim, members] : groups)
-          c->groups.push_back({reinterpret_cast<krk_group*>(h), dim, members});
-        for (uintptr_t t : tables) c->tables.push_back(reinterpret_cast<krk_sparse*>(t));
-        c->dims = dims;
-        c->optim = reinterpret_cast<const krk_optim*>(optim);
-        c->lr = lr;
+          c->groups.push_back({std::make_unique<Bound<krk_group*>>(h), dim, members});
+        for (const py::object& t : tables) c->tables.push_back(std::make_unique<Bound<krk_sparse*>>(t));
         return c;
       }))
+      .def("bind_optim", [](Combine& c, const py::object& optim) { c.optim.bind(optim); })
       .def_readwrite("lr", &Combine::lr);
   m.def("embedding", &embedding, release());
   m.def("jagged", &jagged, release());

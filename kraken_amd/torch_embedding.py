@@ -12,8 +12,6 @@ PyTorch is plumbing here (it owns the tensors and the stream); the arithmetic is
 engine's. The autograd functions are native (csrc/torch_binding.cpp, built with the library).
 Importing this module needs torch; nothing else in the package does.
 """
-import ctypes as C
-
 import torch
 
 from . import api
@@ -36,11 +34,30 @@ class GpuSparseTable(torch.nn.Parameter):
     def __new__(cls, dimension, initializer=None, optim=None, lr=0.01, capacity_hint=0):
         self = super().__new__(cls, torch.empty(0), requires_grad=True)
         self._dimension = int(dimension)
-        self._table = api.SparseTable(dimension, as_initializer(initializer) or api.Initializer.create(
+        self._bound_table = api.SparseTable(dimension, as_initializer(initializer) or api.Initializer.create(
             api.InitializerType.kNormal, {}), capacity_hint=capacity_hint)
-        self._optim = as_optim(optim) or api.Optim.create(api.OptimType.kSGD)
-        self._native = _native.Table(self._table.h.value, C.addressof(self._optim.raw), self._dimension, float(lr))
+        self._bound_optim = as_optim(optim) or api.Optim.create(api.OptimType.kSGD)
+        self._native = _native.Table(self._bound_table.h, self._bound_optim.raw, self._dimension, float(lr))
         return self
+
+    # the native side reads the handle and the optimizer of these objects: another one is bound there too
+    @property
+    def _table(self):
+        return self._bound_table
+
+    @_table.setter
+    def _table(self, table):
+        self._native.bind_table(table.h)
+        self._bound_table = table
+
+    @property
+    def _optim(self):
+        return self._bound_optim
+
+    @_optim.setter
+    def _optim(self, optim):
+        self._native.bind_optim(optim.raw)
+        self._bound_optim = optim
 
     @property
     def lr(self):
@@ -171,11 +188,20 @@ class GpuCombineSparseTable(torch.nn.Parameter):
         for i, d in enumerate(self._dimensions):
             self._members.setdefault(d, []).append(i)
         self._groups = {d: api.TableGroup([self._tables[i] for i in idx]) for d, idx in self._members.items()}
-        self._optim = as_optim(optim) or api.Optim.create(api.OptimType.kSGD)
-        self._native = _native.Combine([(self._groups[d].h.value, d, idx) for d, idx in self._members.items()],
-                                       [t.h.value for t in self._tables], self._dimensions,
-                                       C.addressof(self._optim.raw), float(lr))
+        self._bound_optim = as_optim(optim) or api.Optim.create(api.OptimType.kSGD)
+        self._native = _native.Combine([(self._groups[d].h, d, idx) for d, idx in self._members.items()],
+                                       [t.h for t in self._tables], self._dimensions, self._bound_optim.raw,
+                                       float(lr))
         return self
+
+    @property
+    def _optim(self):
+        return self._bound_optim
+
+    @_optim.setter
+    def _optim(self, optim):
+        self._native.bind_optim(optim.raw)
+        self._bound_optim = optim
 
     @property
     def lr(self):

@@ -2,6 +2,8 @@
 zeros that were never made, blocks of a wider matrix that start anywhere, one value expanded over
 the batch. Whatever the form, the tables end as the oracle's, pushed with the same gradients in plain
 arrays (an output without a gradient pushes zeros, pytorch/combine_embedding.py:22-31)."""
+import gc
+
 import numpy as np
 import pytest
 
@@ -48,6 +50,7 @@ class Pair:
         else:
             self.mod = te.CombineJaggedEmbedding([DIM] * 2, inits, ["sum", "mean"], None, self.o_gpu, LR)
         self.param = self.mod.sparse_table if self.tables == 1 else self.mod.combine_sparse_table
+        self.held = [self.param.table()] if self.tables == 1 else self.param.tables()
         self.modes = ["sum", "mean"]
 
     def draw(self, rng, rows, span=200):
@@ -92,8 +95,7 @@ class Pair:
 
     def check(self, what):
         torch.cuda.synchronize()
-        tables = [self.param.table()] if self.tables == 1 else self.param.tables()
-        for i, (t, r) in enumerate(zip(tables, self.refs)):
+        for i, (t, r) in enumerate(zip(self.held, self.refs)):
             rid, rval, _, _ = r.export()
             assert len(t) == len(r)
             assert_close(t.Pull(rid)[1], rval, "%s: rows of table %d" % (what, i), rtol=1e-5, atol=1e-6)
@@ -126,3 +128,56 @@ def test_output_without_gradient_pushes_zeros(mods, oracle, kind, optim):
         _loss(outs, used).backward()
         p.push(batch, [np.zeros_like(c) if u is None else c for c, u in zip(coefs, used)])
     p.check("after a step without the second output")
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_closed_table_is_refused(mods, oracle, kind):
+    """After close() a forward, and the backward of an earlier forward (in autograd's thread), raise."""
+    p = Pair(mods, oracle, kind)
+    rng = np.random.default_rng(7)
+    batch = p.draw(rng, 32)
+    outs = p.forward(batch)
+    if kind == "combine":
+        for group in p.param._groups.values():
+            group.close()
+    p.held[-1].close()                           # of a pooled request, one table is enough
+    gc.collect()
+    with pytest.raises(p.api.KrakenHipError):
+        _loss(outs, _coef(rng, 32, p.tables)).backward()
+    with pytest.raises(p.api.KrakenHipError):
+        p.forward(batch)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_another_optimizer_between_forward_and_backward(mods, oracle, kind):
+    """The optimizer that a table has when backward runs is the one that counts, replaced or changed."""
+    p = Pair(mods, oracle, kind, (3, {}))
+    rng = np.random.default_rng(8)
+    for step in range(3):
+        batch = p.draw(rng, 48)
+        outs = p.forward(batch)
+        if step == 1:
+            p.o_ref, p.param._optim = make_optims(oracle, p.api, 0, {"eps": 1e-6})
+            p.o_gpu = None
+            gc.collect()
+        elif step == 2:
+            p.o_ref, _ = make_optims(oracle, p.api, 0, {"eps": 0.125})
+            p.param._optim.raw.eps = 0.125
+        coefs = _coef(rng, 48, p.tables)
+        _loss(outs, coefs).backward()
+        p.push(batch, coefs)
+    p.check("after changes of the optimizer")
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_backward_after_the_module_is_gone(mods, oracle, kind):
+    p = Pair(mods, oracle, kind)
+    rng = np.random.default_rng(9)
+    batch = p.draw(rng, 48)
+    coefs = _coef(rng, 48, p.tables)
+    loss = _loss(p.forward(batch), coefs)
+    p.mod = p.param = p.o_gpu = None
+    gc.collect()
+    loss.backward()
+    p.push(batch, coefs)
+    p.check("after a backward without its module")
