@@ -79,8 +79,18 @@ Tensor new_zeros(at::IntArrayRef sizes, const Tensor& like) {
   return at::zeros(sizes, at::TensorOptions().dtype(at::kFloat).device(like.device()));
 }
 
+// `g` as whole rows of `dim` floats one after the other, where the kernels' 16-byte loads may take
+// them. A contiguous tensor need not start on 16 bytes: a row that torch.cat hands back behind 13
+// dense features lies 52 bytes into theirs, and contiguous() returns it as it is.
+Tensor dense_rows(const Tensor& g, int64_t dim) {
+  Tensor rows = g.contiguous().to(at::kFloat);
+  const bool vec = dim % 4 == 0;
+  if (vec && (reinterpret_cast<uintptr_t>(rows.const_data_ptr<float>()) & 15) != 0) rows = rows.clone();
+  return rows;
+}
+
 // The gradient rows of `g` where they lie, `stride` floats apart, if the kernels can read them there;
-// otherwise of a contiguous float copy. `keep` holds whichever it is.
+// otherwise of a dense float copy. `keep` holds whichever it is.
 struct Rows {
   Tensor keep;
   int64_t stride = 0;
@@ -112,7 +122,7 @@ Rows rows_of(const Tensor& g, int64_t dim) {
       return r;
     }
   }
-  r.keep = g.contiguous().to(at::kFloat);
+  r.keep = dense_rows(g, dim);
   return r;
 }
 
@@ -189,7 +199,7 @@ struct EmbeddingBackward : Node {
   SavedVariable ids;
   variable_list apply(variable_list&& grads) override {
     const Tensor saved = ids.unpack();
-    const Tensor g = grads[0].contiguous().to(at::kFloat);
+    const Tensor g = dense_rows(grads[0], table->dim);
     krk_sparse* h = table->h.get();
     const krk_optim optim = table->optim.get();
     KRK_CALL(krk_sparse_set_stream, h, current_stream());
@@ -229,7 +239,7 @@ struct JaggedBackward : Node {
   Tensor weights;
   variable_list apply(variable_list&& grads) override {
     const Tensor saved = ids.unpack(), off = offsets.unpack();
-    const Tensor g = grads[0].contiguous().to(at::kFloat);
+    const Tensor g = dense_rows(grads[0], table->dim);
     krk_sparse* h = table->h.get();
     const krk_optim optim = table->optim.get();
     KRK_CALL(krk_sparse_set_stream, h, current_stream());
@@ -439,7 +449,7 @@ struct CombineJaggedBackward : Node {
         const int i = g.members[m];
         // a call of its own takes a row a bag
         const Tensor rows = grads[i].defined()
-                                ? grads[i].contiguous().to(at::kFloat)
+                                ? dense_rows(grads[i], g.dim)
                                 : new_zeros({p.bags, g.dim}, zeros.keep);
         KRK_CALL(krk_sparse_push_pooled, c->tables[i]->get(), &optim, p.ids, p.n, p.offsets, p.bags, p.weights,
                  p.mode, float_ptr(rows), g.dim, (float)c->lr, kFlags);

@@ -181,3 +181,23 @@ def test_backward_after_the_module_is_gone(mods, oracle, kind):
     loss.backward()
     p.push(batch, coefs)
     p.check("after a backward without its module")
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_contiguous_gradient_off_its_alignment(mods, oracle, kind):
+    """A batch of one behind 13 dense features: what torch.cat hands back for an embedding is one row
+    that starts 13 floats into the matrix, contiguous and not on a 16-byte boundary."""
+    p = Pair(mods, oracle, kind)
+    rng = np.random.default_rng(3)
+    for _ in range(2):
+        batch = p.draw(rng, 1)
+        outs = p.forward(batch)
+        seen = []
+        for o in outs:
+            o.register_hook(lambda g: seen.append((g.is_contiguous(), g.data_ptr() % 16)))
+        dense = torch.ones((1, 13), device="cuda")
+        coef = (rng.integers(-8, 9, size=(1, 13 + DIM * len(outs))) / 16.0).astype(np.float32)
+        (torch.cat([dense] + list(outs), dim=1) * torch.from_numpy(coef).cuda()).sum().backward()
+        assert seen and all(c and off for c, off in seen)       # the form this test is about
+        p.push(batch, [coef[:, 13 + DIM * i:13 + DIM * (i + 1)] for i in range(len(outs))])
+    p.check("after gradients at odd addresses")
