@@ -79,10 +79,11 @@ Tensor new_zeros(at::IntArrayRef sizes, const Tensor& like) {
   return at::zeros(sizes, at::TensorOptions().dtype(at::kFloat).device(like.device()));
 }
 
-// `g` as whole rows of `dim` floats one after the other, where the kernels' 16-byte loads may take
-// them. A contiguous tensor need not start on 16 bytes: a row that torch.cat hands back behind 13
+// `g` as `n` whole rows of `dim` floats one after the other, where the kernels' 16-byte loads may take
+// them; zeros where a function behind the output had no gradient to hand on. A contiguous tensor need not start on 16 bytes: a row that torch.cat hands back behind 13
 // dense features lies 52 bytes into theirs, and contiguous() returns it as it is.
-Tensor dense_rows(const Tensor& g, int64_t dim) {
+Tensor dense_rows(const Tensor& g, int64_t n, int64_t dim, const Tensor& like) {
+  if (!g.defined()) return new_zeros({n, dim}, like);
   Tensor rows = g.contiguous().to(at::kFloat);
   const bool vec = dim % 4 == 0;
   if (vec && (reinterpret_cast<uintptr_t>(rows.const_data_ptr<float>()) & 15) != 0) rows = rows.clone();
@@ -122,7 +123,7 @@ Rows rows_of(const Tensor& g, int64_t dim) {
       return r;
     }
   }
-  r.keep = dense_rows(g, dim);
+  r.keep = dense_rows(g, g.numel() / dim, dim, g);
   return r;
 }
 
@@ -199,7 +200,7 @@ struct EmbeddingBackward : Node {
   SavedVariable ids;
   variable_list apply(variable_list&& grads) override {
     const Tensor saved = ids.unpack();
-    const Tensor g = dense_rows(grads[0], table->dim);
+    const Tensor g = dense_rows(grads[0], saved.numel(), table->dim, saved);
     krk_sparse* h = table->h.get();
     const krk_optim optim = table->optim.get();
     KRK_CALL(krk_sparse_set_stream, h, current_stream());
@@ -239,7 +240,7 @@ struct JaggedBackward : Node {
   Tensor weights;
   variable_list apply(variable_list&& grads) override {
     const Tensor saved = ids.unpack(), off = offsets.unpack();
-    const Tensor g = dense_rows(grads[0], table->dim);
+    const Tensor g = dense_rows(grads[0], off.numel() - 1, table->dim, saved);
     krk_sparse* h = table->h.get();
     const krk_optim optim = table->optim.get();
     KRK_CALL(krk_sparse_set_stream, h, current_stream());
@@ -448,9 +449,7 @@ struct CombineJaggedBackward : Node {
         if (p.n == 0 || p.bags == 0) continue;
         const int i = g.members[m];
         // a call of its own takes a row a bag
-        const Tensor rows = grads[i].defined()
-                                ? dense_rows(grads[i], g.dim)
-                                : new_zeros({p.bags, g.dim}, zeros.keep);
+        const Tensor rows = dense_rows(grads[i], p.bags, g.dim, keep[0]);
         KRK_CALL(krk_sparse_push_pooled, c->tables[i]->get(), &optim, p.ids, p.n, p.offsets, p.bags, p.weights,
                  p.mode, float_ptr(rows), g.dim, (float)c->lr, kFlags);
       }

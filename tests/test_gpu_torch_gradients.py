@@ -201,3 +201,32 @@ def test_contiguous_gradient_off_its_alignment(mods, oracle, kind):
         assert seen and all(c and off for c, off in seen)       # the form this test is about
         p.push(batch, [coef[:, 13 + DIM * i:13 + DIM * (i + 1)] for i in range(len(outs))])
     p.check("after gradients at odd addresses")
+
+
+class _NoGradient(torch.autograd.Function):
+    """A function whose backward has no gradient to hand on."""
+
+    @staticmethod
+    def forward(ctx, x):
+        return x.clone()
+
+    @staticmethod
+    def backward(ctx, grad):
+        return None
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_undefined_gradient_pushes_zeros(mods, oracle, kind):
+    p = Pair(mods, oracle, kind)
+    rng = np.random.default_rng(2)
+    for step in range(3):
+        batch = p.draw(rng, 64)
+        outs = p.forward(batch)
+        coefs = _coef(rng, 64, p.tables)
+        if step == 1:
+            sum(_NoGradient.apply(o).sum() for o in outs).backward()
+            coefs = [np.zeros_like(c) for c in coefs]
+        else:
+            _loss(outs, coefs).backward()
+        p.push(batch, coefs)
+    p.check("after a step without gradients")
