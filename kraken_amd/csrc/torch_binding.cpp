@@ -135,6 +135,16 @@ Rows zero_rows(const Tensor& like, int64_t dim) {
   return r;
 }
 
+// Whether a backward may use the rows that its forward's pull noted: it pushes for the very buffer that
+// was pulled from. Saved-tensor hooks hand back a tensor of their own, and one that offloads may bring
+// the ids of one pass to where the ids of a later pass were noted.
+uint32_t as_pulled(const SavedVariable& ids) { return ids.has_hooks() ? 0u : KRK_IDS_AS_PULLED; }
+uint32_t as_pulled(const std::vector<SavedVariable>& ids) {
+  for (const SavedVariable& v : ids)
+    if (v.has_hooks()) return 0u;
+  return KRK_IDS_AS_PULLED;
+}
+
 bool recording(const Tensor& param) { return at::GradMode::is_enabled() && param.requires_grad(); }
 
 // The node of a pass over `param` (the empty Parameter that stands for the tables, whose edge is
@@ -205,7 +215,7 @@ struct EmbeddingBackward : Node {
     const krk_optim optim = table->optim.get();
     KRK_CALL(krk_sparse_set_stream, h, current_stream());
     KRK_CALL(krk_sparse_push_raw, h, &optim, id_ptr(saved), saved.numel(), float_ptr(g), table->dim,
-             (float)table->lr, kFlags | KRK_IDS_AS_PULLED);
+             (float)table->lr, kFlags | as_pulled(ids));
     return variable_list(1);
   }
   void release_variables() override { ids.reset_data(); }
@@ -246,7 +256,7 @@ struct JaggedBackward : Node {
     KRK_CALL(krk_sparse_set_stream, h, current_stream());
     KRK_CALL(krk_sparse_push_pooled, h, &optim, id_ptr(saved), saved.numel(), off_ptr(off),
              off.numel() - 1, float_ptr(weights), mode, float_ptr(g), table->dim, (float)table->lr,
-             kFlags | KRK_IDS_AS_PULLED);
+             kFlags | as_pulled(ids));
     return variable_list(1);
   }
   void release_variables() override {
@@ -312,6 +322,7 @@ struct CombineBackward : Node {
   variable_list apply(variable_list&& grads) override {
     void* stream = current_stream();
     const krk_optim optim = c->optim.get();
+    const uint32_t noted = as_pulled(ids);
     for (const Combine::Group& g : c->groups) {
       krk_group* h = g.h->get();
       std::vector<krk_part> parts(g.members.size());
@@ -337,7 +348,7 @@ struct CombineBackward : Node {
         keep.push_back(std::move(saved));
       }
       KRK_CALL(krk_group_set_stream, h, stream);
-      KRK_CALL(krk_group_push_raw_parts, h, &optim, parts.data(), g.dim, (float)c->lr, kFlags | KRK_IDS_AS_PULLED);
+      KRK_CALL(krk_group_push_raw_parts, h, &optim, parts.data(), g.dim, (float)c->lr, kFlags | noted);
     }
     return variable_list(1);
   }
@@ -397,12 +408,14 @@ void check_open(const Combine& c) {
 
 struct CombineJaggedBackward : Node {
   CombinePtr c;
+  bool combined = true;            // every group's pull was one request, which noted its rows
   std::vector<int> modes;
   std::vector<SavedVariable> ids, offsets;
   std::vector<Tensor> weights;
   variable_list apply(variable_list&& grads) override {
     void* stream = current_stream();
     const krk_optim optim = c->optim.get();
+    const uint32_t noted = combined ? as_pulled(ids) : 0u;
     check_open(*c);
     for (const Combine::Group& g : c->groups) {
       krk_group* h = g.h->get();
@@ -440,7 +453,7 @@ struct CombineJaggedBackward : Node {
       const int32_t rc = total > kCombinedMax
                              ? KRK_E_CAPACITY
                              : krk_group_push_pooled_parts(h, &optim, parts.data(), g.dim, (float)c->lr,
-                                                           kFlags | KRK_IDS_AS_PULLED);
+                                                           kFlags | noted);
       if (rc == KRK_SUCCESS) continue;
       if (rc != KRK_E_CAPACITY) fail(rc, "krk_group_push_pooled_parts");
       // more than one launch can name: a table at a time
@@ -475,6 +488,7 @@ std::vector<Tensor> combine_jagged(const CombinePtr& c, const Tensor& param, con
   const bool record = recording(param);
   void* stream = current_stream();
   check_open(*c);
+  bool combined = true;
   std::vector<Tensor> outs(n), ids(n), offsets(n), weights(n);
   for (const Combine::Group& g : c->groups) {
     std::vector<krk_pooled_part> parts(g.members.size());
@@ -504,6 +518,7 @@ std::vector<Tensor> combine_jagged(const CombinePtr& c, const Tensor& param, con
                              : krk_group_pull_pooled_parts(h, parts.data(), kFlags | (record ? KRK_NOTE_ROWS : 0u));
     if (rc == KRK_SUCCESS) continue;
     if (rc != KRK_E_CAPACITY) fail(rc, "krk_group_pull_pooled_parts");
+    combined = false;
     for (size_t m = 0; m < g.members.size(); ++m) {
       const krk_pooled_part& p = parts[m];
       KRK_CALL(krk_sparse_pull_pooled, c->tables[g.members[m]]->get(), p.ids, p.n, p.offsets, p.bags, p.weights,
@@ -513,6 +528,7 @@ std::vector<Tensor> combine_jagged(const CombinePtr& c, const Tensor& param, con
   if (record) {
     auto node = new_node<CombineJaggedBackward>(param);
     node->c = c;
+    node->combined = combined;
     node->modes = modes;
     for (const Tensor& t : ids) node->ids.emplace_back(t, false);
     for (const Tensor& t : offsets) node->offsets.emplace_back(t, false);

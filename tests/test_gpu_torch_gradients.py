@@ -230,3 +230,41 @@ def test_undefined_gradient_pushes_zeros(mods, oracle, kind):
             _loss(outs, coefs).backward()
         p.push(batch, coefs)
     p.check("after a step without gradients")
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_ids_unpacked_by_hooks_are_looked_up_again(mods, oracle, kind):
+    """Saved-tensor hooks that offload to the host and bring every tensor back into one buffer per
+    shape: the first backward gets its ids at the address, and in the number, that the second forward
+    pulled from."""
+    p = Pair(mods, oracle, kind, (3, {}))
+    rng = np.random.default_rng(6)
+    first = p.draw(rng, 64, span=100)
+    # the same bags, other ids
+    second = [((ids + np.uint64(100)), off) for ids, off in first]
+    own, shared = p.tensors(first), p.tensors(second)
+    buffers = [t for pair in shared for t in pair if t is not None]
+    packed = []
+
+    def pack(t):
+        packed.append(t)
+        i = (len(packed) - 1) % len(order)
+        return order[i], t.cpu()
+
+    def unpack(x):
+        b = buffers[x[0]]
+        b.copy_(x[1])
+        return b
+
+    # modules save ids (and offsets) of all tables in one order: all ids, then all offsets
+    order = list(range(len(buffers))) if p.tables == 1 or not p.jagged else [0, 2, 1, 3]
+    with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+        outs_a = p.forward(first, own)
+        outs_b = p.forward(second, shared)
+    assert len(packed) == 2 * len(order)
+    ca, cb = _coef(rng, 64, p.tables), _coef(rng, 64, p.tables)
+    _loss(outs_a, ca).backward()
+    _loss(outs_b, cb).backward()
+    p.push(first, ca)
+    p.push(second, cb)
+    p.check("after two backward passes through one buffer")
