@@ -17,12 +17,22 @@ import torch
 from . import api
 from .configs import as_initializer, as_optim
 
-api.lib()                                       # the native module links against it
-try:
-    from . import _torch_native as _native
-except ImportError as e:
-    raise ImportError("kraken_amd/_torch_native.so is missing or was built against another torch: build it with "
-                      "`python -m kraken_amd.build`") from e
+_native = None
+
+
+def _load_native():
+    """The native autograd functions; loaded with the first table, so that the module (JaggedTensor, the
+    classes) can be imported where nothing is built."""
+    global _native
+    if _native is None:
+        api.lib()                               # the native module links against it
+        try:
+            from . import _torch_native
+        except ImportError as e:
+            raise ImportError("kraken_amd/_torch_native.so is missing or was built against another torch: build it "
+                              "with `python -m kraken_amd.build`") from e
+        _native = _torch_native
+    return _native
 
 
 class GpuSparseTable(torch.nn.Parameter):
@@ -37,7 +47,7 @@ class GpuSparseTable(torch.nn.Parameter):
         self._bound_table = api.SparseTable(dimension, as_initializer(initializer) or api.Initializer.create(
             api.InitializerType.kNormal, {}), capacity_hint=capacity_hint)
         self._bound_optim = as_optim(optim) or api.Optim.create(api.OptimType.kSGD)
-        self._native = _native.Table(self._bound_table.h, self._bound_optim.raw, self._dimension, float(lr))
+        self._native = _load_native().Table(self._bound_table.h, self._bound_optim.raw, self._dimension, float(lr))
         return self
 
     # the native side reads the handle and the optimizer of these objects: another one is bound there too
@@ -189,9 +199,9 @@ class GpuCombineSparseTable(torch.nn.Parameter):
             self._members.setdefault(d, []).append(i)
         self._groups = {d: api.TableGroup([self._tables[i] for i in idx]) for d, idx in self._members.items()}
         self._bound_optim = as_optim(optim) or api.Optim.create(api.OptimType.kSGD)
-        self._native = _native.Combine([(self._groups[d].h, d, idx) for d, idx in self._members.items()],
-                                       [t.h for t in self._tables], self._dimensions, self._bound_optim.raw,
-                                       float(lr))
+        self._native = _load_native().Combine(
+            [(self._groups[d].h, d, idx) for d, idx in self._members.items()], [t.h for t in self._tables],
+            self._dimensions, self._bound_optim.raw, float(lr))
         return self
 
     @property
