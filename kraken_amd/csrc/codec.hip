@@ -665,9 +665,10 @@ int32_t krk_dct_compress(krk_dct* s, const float* grad, uint64_t life_span, floa
     return KRK_SUCCESS;
   }
   if (!grad || (capacity > 0 && (!idx || !val))) return KRK_E_ARGUMENT;
-  const float* d_g;
-  KRK_TRY(s->input(grad, (size_t)n, flags, 0, &d_g));
   const bool reselect = s->step % life_span == 0;   // :25
+  const float* d_g;
+  // the gradient of a call on host memory is counted, then written; a selection reads it three times before
+  KRK_TRY(s->input(grad, (size_t)n, flags, 0, &d_g, host_reads(reselect ? 5 : 2, n * 4)));
   if (reselect) {
     const int64_t k = (int64_t)((double)n * (1.0 - (double)eta));   // :27
     if (k < 1 || k > n) {

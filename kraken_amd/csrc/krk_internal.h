@@ -70,8 +70,6 @@ struct DeviceGuard {
 // memory is pageable or not aligned to `align` bytes.
 void* direct_host_pointer(const void* p, size_t align);
 
-// Every API object starts with this: its own stream, the host lock that serialises
-// calls on it, and the staging buffers used when the caller hands over host pointers.
 // Page-locked host memory that grows and is kept.
 struct HostBuffer {
   void* ptr = nullptr;
@@ -83,10 +81,31 @@ struct HostBuffer {
 // Host arguments of up to this size pass through page-locked memory that the kernels read and write
 // themselves; beyond it they are staged on the device by copies. A call's copies cost more than
 // the kernel as long as the data is small: 4001 ids and rows of 16 floats (256 KB), push and
-// pull, 101 us with copies, 61 us this way; 20,000 of them 216 and 187 us. Data that the kernels read at 40 GB/s in place of
-// 8 TB/s, and what an object may keep locked (four such buffers), set the limit.
+// pull, 101 us with copies, 61 us this way; 20,000 of them 216 and 187 us. Data that the kernels
+// read at 40 GB/s in place of 8 TB/s, and what an object may keep locked (four such buffers of up
+// to 1.5 MB), set the limit.
 constexpr size_t kBounceMax = (size_t)1 << 20;
 
+// That holds for what is read once, front to back. An argument that the kernels read several times
+// over, or row by row in an order of their own, crosses PCIe again with each read, and in pieces of
+// at least kHostPiece bytes: a pooled push reads a bag's gradient row once for every id of the bag.
+// Where the reads come to kReadAgainMin bytes more than the argument has, it is copied to the device
+// by a kernel first. Blocking calls on pageable memory, us, everything copied to the device by the
+// runtime / everything read in place / by this rule: pooled pushes of 10,000 bags of 16 floats, ten
+// ids each, 164 / 233 / 144, 2048 bags of 64 floats, 40 weighted ids each, 186 / 260 / 151, 256
+// bags of 16 floats, four ids each (read in place) 91 / 41 / 41; push_raw of 16,000 ids of 8 floats
+// 110 / 117 / 96; a codec step that selects over 260,000 values 352 / 421 / 341.
+constexpr size_t kHostPiece = 128;
+constexpr size_t kReadAgainMin = (size_t)128 << 10;
+// bytes that `reads` reads of `bytes` each take across PCIe
+inline size_t host_reads(int64_t reads, int64_t bytes) {
+  return (size_t)reads * (bytes < (int64_t)kHostPiece ? kHostPiece : (size_t)bytes);
+}
+// Copies host memory that kernels can address to device memory (both on 16 bytes; whole words).
+int32_t copy_from_host(void* dst, const void* src, size_t bytes, hipStream_t stream);
+
+// Every API object starts with this: its own stream, the host lock that serialises
+// calls on it, and the staging buffers used when the caller hands over host pointers.
 struct ObjBase {
   hipStream_t stream = nullptr;
   std::mutex mu;
@@ -96,26 +115,33 @@ struct ObjBase {
   bool direct[4] = {false, false, false, false};   // output slot is the caller's own page-locked buffer
   int32_t open_stream();
   void close_stream();
-  // Copies a host array into staging buffer `slot` (or passes a device pointer through).
+  // Where kernels find a host array: the caller's page-locked memory, page-locked buffer `slot` or
+  // staging buffer `slot` (a device pointer is passed through). read: the bytes the call's kernels
+  // read of it, if that is not each byte once in order (host_reads).
   template <typename T>
-  int32_t input(const T* p, size_t count, uint32_t flags, int slot, const T** dev) {
+  int32_t input(const T* p, size_t count, uint32_t flags, int slot, const T** dev, size_t read = 0) {
     if (flags & KRK_DEVICE_PTRS) {
       *dev = p;
       return KRK_SUCCESS;
     }
+    const size_t bytes = count * sizeof(T);
     if (void* d = direct_host_pointer(p, 16)) {
       *dev = reinterpret_cast<const T*>(d);
       return KRK_SUCCESS;
     }
-    if (count * sizeof(T) <= kBounceMax) {
+    if (bytes <= kBounceMax) {
       // host pointers make a call blocking: what an earlier call put here has been read
-      KRK_TRY(bounce[slot].reserve(count * sizeof(T) + 16));
-      std::memcpy(bounce[slot].ptr, p, count * sizeof(T));
+      KRK_TRY(bounce[slot].reserve(bytes + 16));
+      std::memcpy(bounce[slot].ptr, p, bytes);
       *dev = reinterpret_cast<const T*>(bounce[slot].ptr);
+      if (read < bytes + kReadAgainMin) return KRK_SUCCESS;
+      KRK_TRY(stage[slot].reserve(bytes + 16));
+      KRK_TRY(copy_from_host(stage[slot].ptr, bounce[slot].ptr, bytes, stream));
+      *dev = stage[slot].as<T>();
       return KRK_SUCCESS;
     }
-    KRK_TRY(stage[slot].reserve(count * sizeof(T) + 16));
-    if (count) KRK_HIP(hipMemcpyAsync(stage[slot].ptr, p, count * sizeof(T), hipMemcpyHostToDevice, stream));
+    KRK_TRY(stage[slot].reserve(bytes + 16));
+    KRK_HIP(hipMemcpyAsync(stage[slot].ptr, p, bytes, hipMemcpyHostToDevice, stream));
     *dev = stage[slot].as<T>();
     return KRK_SUCCESS;
   }

@@ -2244,7 +2244,8 @@ int32_t krk_sparse_push_raw(krk_sparse* t, const krk_optim* o, const uint64_t* i
   const uint64_t* d_ids;
   const float* d_g;
   KRK_TRY(t->input(ids, (size_t)n, flags, 0, &d_ids));
-  KRK_TRY(t->input(grads, (size_t)n * t->dim, flags, 1, &d_g));
+  // the rows are read in the order of the sorted ids
+  KRK_TRY(t->input(grads, (size_t)n * t->dim, flags, 1, &d_g, host_reads(n, t->dim * 4)));
 
   if (short_push_fits(n, t->dim, t->elems, t->group)) {
     // a short request: see bucket_push_kernel
@@ -2516,7 +2517,7 @@ int32_t krk_group_push_raw(krk_group* g, const krk_optim* o, const uint64_t* ids
   const uint64_t* d_ids;
   const float* d_g;
   KRK_TRY(g->input(ids, (size_t)total, flags, 0, &d_ids));
-  KRK_TRY(g->input(grads, (size_t)total * g->dim, flags, 1, &d_g));
+  KRK_TRY(g->input(grads, (size_t)total * g->dim, flags, 1, &d_g, host_reads(total, g->dim * 4)));
   GroupParts parts;
   for (int m = 0; m < call.n_tables; ++m) {
     parts.ids[m] = d_ids + offsets[m];
@@ -2596,9 +2597,11 @@ int32_t krk_sparse_push_pooled(krk_sparse* t, const krk_optim* o, const uint64_t
   const float* d_w = nullptr;
   const float* d_g;
   KRK_TRY(t->input(ids, (size_t)n, flags, 0, &d_ids));
-  KRK_TRY(t->input(reinterpret_cast<const long long*>(offsets), (size_t)bags + 1, flags, 1, &d_off));
-  if (weights) KRK_TRY(t->input(weights, (size_t)n, flags, 2, &d_w));
-  KRK_TRY(t->input(bag_grads, (size_t)bags * t->dim, flags, 3, &d_g));
+  // the reduction reads, for every id, its weight, its bag's gradient row and, for a mean, the bag's ends
+  KRK_TRY(t->input(reinterpret_cast<const long long*>(offsets), (size_t)bags + 1, flags, 1, &d_off,
+                   mode == KRK_POOL_MEAN ? host_reads(n, 16) : 0));
+  if (weights) KRK_TRY(t->input(weights, (size_t)n, flags, 2, &d_w, host_reads(n, 4)));
+  KRK_TRY(t->input(bag_grads, (size_t)bags * t->dim, flags, 3, &d_g, host_reads(n, t->dim * 4)));
 
   // one member that begins at zero
   PooledCall call{};

@@ -108,6 +108,26 @@ void DeviceBuffer::release() {
   bytes = 0;
 }
 
+__global__ __launch_bounds__(256) void host_copy_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst,
+                                                        uint32_t words) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (4 * i + 3 < words) {
+    dst[i] = src[i];
+  } else {
+    for (uint32_t w = 4 * i; w < words; ++w)
+      reinterpret_cast<uint32_t*>(dst)[w] = reinterpret_cast<const uint32_t*>(src)[w];
+  }
+}
+
+int32_t copy_from_host(void* dst, const void* src, size_t bytes, hipStream_t stream) {
+  const uint32_t words = (uint32_t)(bytes / 4);      // at most kBounceMax bytes
+  if (words == 0) return KRK_SUCCESS;
+  hipLaunchKernelGGL(host_copy_kernel, dim3((words + 1023) / 1024), dim3(256), 0, stream,
+                     reinterpret_cast<const uint4*>(src), reinterpret_cast<uint4*>(dst), words);
+  KRK_HIP(hipGetLastError());
+  return KRK_SUCCESS;
+}
+
 OptimK make_optim_k(const krk_optim& o) {
   OptimK k;
   k.type = o.type;
