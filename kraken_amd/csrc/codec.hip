@@ -441,7 +441,7 @@ __global__ __launch_bounds__(kCodecBlock) void coo_tiles_bounds_kernel(const lon
       for (int i = 0; i < 2; ++i) {
         if (j + i >= nnz) continue;
         const long long c = cur[r][i];
-        const bool wrong = c <= prev || c >= n;
+        const bool wrong = c < 0 || c <= prev || c >= n;   // prev may be negative, and wrong, itself
         bad = bad || wrong;
         if (!wrong) {
           const int64_t mine = c / kCooTile;

@@ -238,6 +238,28 @@ def test_coo_to_dense_large_tensors(api, oracle, n):
     assert np.array_equal(out.to_host(), want)
 
 
+@pytest.mark.parametrize("idx", [[-6000, -5000], [-(1 << 40), -(1 << 39), 3], [-3, -2, -1, 0, 2047, 2048],
+                                 [5, 1 << 22, (1 << 22) + 1], [1 << 40, (1 << 40) + 1], [-1, (1 << 22) - 1]],
+                         ids=["below", "far_below", "around_zero", "around_n", "far_above", "ends"])
+def test_coo_indices_outside_a_large_tensor(api, oracle, idx):
+    """Entries outside [0, n) are skipped, also where they ascend, and nothing is written for them: not
+    the tiles' starts either, which a negative entry behind another one named before the array."""
+    n = 1 << 22
+    idx = np.array(idx, np.int64)
+    val = np.arange(1, idx.size + 1, dtype=np.float32)
+    want = np.zeros(n, np.float32)
+    inside = (idx >= 0) & (idx < n)
+    want[idx[inside]] = val[inside]
+    assert np.array_equal(api.coo_to_dense(idx, val, n), want)
+    w0 = np.ones(n, np.float32)
+    t = api.DenseTable(w0)
+    opt = api.Optim.create(api.OptimType.kSGD)
+    for _ in range(2):
+        assert t.PushCoo(opt, idx, val, 0.5) == 0
+        w0 = w0 - np.float32(0.5) * want
+        assert np.array_equal(t.Pull()[1], w0)
+
+
 def test_dense_push_coo_large(api, oracle):
     n = (1 << 22) + 77
     rng = np.random.default_rng(4)
