@@ -260,6 +260,24 @@ def test_coo_indices_outside_a_large_tensor(api, oracle, idx):
         assert np.array_equal(t.Pull()[1], w0)
 
 
+def test_coo_gaps_of_every_length(api, oracle):
+    """Empty tiles before, between and behind the entries: gaps that a lane fills alone, that it just no
+    longer does and that take a wavefront several rounds, several of them in one wavefront."""
+    n, tile = (1 << 23) + 5, 2048
+    tiles = -(-n // tile)
+    gaps = [0, 1, 7, 8, 9, 10, 63, 64, 65, 129, 0, 0, 8, 9]
+    starts = np.cumsum(gaps)
+    cases = [[0], [n - 1], [0, n - 1], [7 * tile], [8 * tile], [9 * tile], list(starts * tile + 3),
+             list(range(300)), list(range(n - 300, n)), list(range(40 * tile, 40 * tile + 129)),
+             [(tiles - 9) * tile - 1], [(tiles - 8) * tile - 1], [(tiles - 10) * tile]]
+    for entries in cases:
+        idx = np.unique(np.array(entries, np.int64))
+        val = np.arange(1, idx.size + 1, dtype=np.float32)
+        want = np.zeros(n, np.float32)
+        want[idx] = val
+        assert np.array_equal(api.coo_to_dense(idx, val, n), want), entries[:4]
+
+
 def test_dense_push_coo_large(api, oracle):
     n = (1 << 22) + 77
     rng = np.random.default_rng(4)
