@@ -408,8 +408,9 @@ struct krk_sparse : krk::ObjBase {
 
   krk::DeviceBuffer scratch[6];       // push_raw work space
 
-  // Row notes (KRK_NOTE_ROWS): the row of every position of one pull, kept for a push_raw of the
-  // same ids. Valid while noted_ids is not null and noted_version == layout_version.
+  // Row notes (KRK_NOTE_ROWS): the row of every position of one pull, 4 bytes each whatever the size
+  // of the request, kept for a push of the same ids. Valid while noted_ids is not null and
+  // noted_version == layout_version.
   krk::DeviceBuffer notes;
   const uint64_t* noted_ids = nullptr;
   int64_t noted_n = 0;
@@ -511,6 +512,14 @@ struct krk_group : krk::ObjBase {
 };
 
 namespace krk {
+// Room for the notes of n positions, or null where the device has none: the pull then leaves no notes
+// behind, and the push that follows looks its ids up.
+inline uint32_t* note_room(DeviceBuffer* notes, int64_t n) {
+  if (notes->reserve((size_t)n * sizeof(uint32_t)) == KRK_SUCCESS) return notes->as<uint32_t>();
+  (void)hipGetLastError();   // no failure of the call
+  return nullptr;
+}
+
 // KRK_IDS_AS_PULLED: the row notes of the pull of these very ids, or null when they do not apply
 // (another buffer or count, nothing noted, rows moved since). The caller holds the lock(s).
 inline const uint32_t* noted_rows(const krk_sparse* t, const uint64_t* ids, int64_t n, uint32_t flags) {

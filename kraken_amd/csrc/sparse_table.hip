@@ -2147,10 +2147,7 @@ int32_t krk_sparse_pull(krk_sparse* t, const uint64_t* ids, int64_t n, float* ou
   uint32_t* notes = nullptr;
   if (flags & KRK_NOTE_ROWS) {
     t->noted_ids = nullptr;
-    if (flags & KRK_DEVICE_PTRS) {
-      KRK_TRY(t->notes.reserve((size_t)n * sizeof(uint32_t)));
-      notes = t->notes.as<uint32_t>();
-    }
+    if (flags & KRK_DEVICE_PTRS) notes = note_room(&t->notes, n);
   }
   KRK_TRY(pull_enqueue(t, d_ids, n, d_out, notes));
   if (notes) {
@@ -2208,20 +2205,16 @@ int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, co
   const bool filling = t->host_inserted && __atomic_exchange_n(t->host_inserted, 0u, __ATOMIC_RELAXED) != 0u;
   const bool queued = filling && n >= kTwoLaunchWhileFilling;
   const int64_t list_capacity = queued ? queue_capacity(n, kBlock / kBucket) : 0;
-  const size_t rows_words = ((size_t)(n > 0 ? n : 1) + 63) & ~(size_t)63;
-  KRK_TRY(t->scratch[5].reserve((rows_words + (size_t)kQueues * (size_t)list_capacity) * sizeof(uint32_t)));
-  uint32_t* rows = t->scratch[5].as<uint32_t>();
-  uint32_t* todo = rows + rows_words;
-  // KRK_NOTE_ROWS: the rows of the positions, which the second launch reads, stay behind
-  bool noting = false;
+  // KRK_NOTE_ROWS: the rows of the positions, which the last launch reads, stay behind
+  uint32_t* notes = nullptr;
   if (flags & KRK_NOTE_ROWS) {
     t->noted_ids = nullptr;
-    noting = (flags & KRK_DEVICE_PTRS) && n > 0;
-    if (noting) {
-      KRK_TRY(t->notes.reserve((size_t)n * sizeof(uint32_t)));
-      rows = t->notes.as<uint32_t>();
-    }
+    if ((flags & KRK_DEVICE_PTRS) && n > 0) notes = note_room(&t->notes, n);
   }
+  const size_t rows_words = notes ? 0 : ((size_t)(n > 0 ? n : 1) + 63) & ~(size_t)63;
+  KRK_TRY(t->scratch[5].reserve((rows_words + (size_t)kQueues * (size_t)list_capacity) * sizeof(uint32_t)));
+  uint32_t* rows = notes ? notes : t->scratch[5].as<uint32_t>();
+  uint32_t* todo = t->scratch[5].as<uint32_t>() + rows_words;
   const int per_block = kBlock / t->group;
   const dim3 probe_grid(grid_for(n, kBlock / kBucket)), grid(grid_for(bags, per_block)), block(kBlock);
   const dim3 small(kMissingGrid), missing_block(kMissBlock);
@@ -2252,7 +2245,7 @@ int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, co
                        mean, patch_value, d_out, (int)t->dim, t->elems, t->group);
   }
   KRK_HIP(hipGetLastError());
-  if (noting) {
+  if (notes) {
     t->noted_ids = ids;
     t->noted_n = n;
     t->noted_version = t->layout_version;
@@ -3077,10 +3070,7 @@ static int32_t group_pull_enqueue(krk_group* g, const int64_t* offsets, GroupCal
   uint32_t* notes = nullptr;
   if (flags & KRK_NOTE_ROWS) {
     g->noted_ids.clear();
-    if (flags & KRK_DEVICE_PTRS) {
-      KRK_TRY(g->notes.reserve((size_t)total * sizeof(uint32_t)));
-      notes = g->notes.as<uint32_t>();
-    }
+    if (flags & KRK_DEVICE_PTRS) notes = note_room(&g->notes, total);
   }
   // While the members' tables are being filled (see pull_enqueue) the request takes the two
   // launches of a large pull, member by member.
@@ -3332,10 +3322,13 @@ int32_t krk_group_pull_pooled_parts(krk_group* g, const krk_pooled_part* in, uin
   KRK_TRY(group_refresh(g));
   // the row of every position, in the notes where they are to stay behind
   const size_t rows_words = ((size_t)(total > 0 ? total : 1) + 63) & ~(size_t)63;
-  DeviceBuffer& row_buffer = (flags & KRK_NOTE_ROWS) ? g->notes : g->scratch[0];
-  if (flags & KRK_NOTE_ROWS) g->noted_ids.clear();
-  KRK_TRY(row_buffer.reserve(rows_words * sizeof(uint32_t)));
-  uint32_t* rows = row_buffer.as<uint32_t>();
+  uint32_t* notes = nullptr;
+  if (flags & KRK_NOTE_ROWS) {
+    g->noted_ids.clear();
+    if (total > 0) notes = note_room(&g->notes, total);
+  }
+  if (!notes) KRK_TRY(g->scratch[0].reserve(rows_words * sizeof(uint32_t)));
+  uint32_t* rows = notes ? notes : g->scratch[0].as<uint32_t>();
   const dim3 probe_grid(call.block_start[n_tables]), block(kBlock);
   bool filling = false;
   for (krk_sparse* t : g->tables)
@@ -3382,7 +3375,7 @@ int32_t krk_group_pull_pooled_parts(krk_group* g, const krk_pooled_part* in, uin
                        (int)g->dim, g->elems, g->group);
   }
   KRK_HIP(hipGetLastError());
-  if ((flags & KRK_NOTE_ROWS) && total > 0) {
+  if (notes) {
     g->noted_ids.assign(pool.ids, pool.ids + n_tables);
     g->noted_offsets.assign(pool.row_start, pool.row_start + n_tables + 1);
     g->noted_versions.clear();
