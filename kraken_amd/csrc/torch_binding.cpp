@@ -304,6 +304,7 @@ struct Combine {
   std::vector<int64_t> dims;
   Bound<krk_optim> optim;
   double lr;
+  int64_t combined_max = (int64_t)1 << 28;   // groups whose pooled request is larger are served a table at a time
 };
 using CombinePtr = std::shared_ptr<Combine>;
 
@@ -396,9 +397,6 @@ std::vector<Tensor> combine(const CombinePtr& c, const Tensor& param, const std:
   return outs;
 }
 
-// Groups whose request is larger than this are served a table at a time.
-constexpr int64_t kCombinedMax = (int64_t)1 << 28;
-
 // A pooled request is made of the tables' own calls: one whose table was closed is refused, also where
 // the group still holds the table.
 void check_open(const Combine& c) {
@@ -450,7 +448,7 @@ struct CombineJaggedBackward : Node {
         keep.push_back(std::move(off));
       }
       KRK_CALL(krk_group_set_stream, h, stream);
-      const int32_t rc = total > kCombinedMax
+      const int32_t rc = total > c->combined_max
                              ? KRK_E_CAPACITY
                              : krk_group_push_pooled_parts(h, &optim, parts.data(), g.dim, (float)c->lr,
                                                            kFlags | noted);
@@ -514,8 +512,9 @@ std::vector<Tensor> combine_jagged(const CombinePtr& c, const Tensor& param, con
     krk_group* h = g.h->get();
     KRK_CALL(krk_group_set_stream, h, stream);
     const int32_t rc =
-        total > kCombinedMax ? KRK_E_CAPACITY
-                             : krk_group_pull_pooled_parts(h, parts.data(), kFlags | (record ? KRK_NOTE_ROWS : 0u));
+        total > c->combined_max
+            ? KRK_E_CAPACITY
+            : krk_group_pull_pooled_parts(h, parts.data(), kFlags | (record ? KRK_NOTE_ROWS : 0u));
     if (rc == KRK_SUCCESS) continue;
     if (rc != KRK_E_CAPACITY) fail(rc, "krk_group_pull_pooled_parts");
     combined = false;
@@ -561,7 +560,8 @@ PYBIND11_MODULE(_torch_native, m) {
         return c;
       }))
       .def("bind_optim", [](Combine& c, const py::object& optim) { c.optim.bind(optim); })
-      .def_readwrite("lr", &Combine::lr);
+      .def_readwrite("lr", &Combine::lr)
+      .def_readwrite("combined_max", &Combine::combined_max);
   m.def("embedding", &embedding, release());
   m.def("jagged", &jagged, release());
   m.def("combine", &combine, release());

@@ -256,12 +256,12 @@ def test_group_push_raw_errors(api):
     grp.close()
 
 
-@pytest.mark.parametrize("filler", [5, 9000])
+@pytest.mark.parametrize("filler", [5, 9000, 14_000])
 def test_group_push_raw_adds_repeats_in_position_order(api, filler):
     """worker/emitter.cc:563-606 adds the gradients of a repeated (table, id) in the order the
     request lists them. 1e8 + 1 - 1e8 is 0 in that order and 1 in the other two, so the sort
-    has to be stable: members of few ids take the one-workgroup-a-member sort, a member above
-    8192 ids the radix sort over the whole request."""
+    has to be stable: members of up to 12288 ids take the bucket kernel's sort, a request with a
+    longer member the radix sort over the whole request."""
     dim = 4
     gi = api.Initializer.create(api.InitializerType.kConstant, {"value": "0.5"})
     a, b = api.SparseTable(dim, gi), api.SparseTable(dim, gi)

@@ -199,13 +199,13 @@ def test_pooled_push_equals_push_raw_of_the_expanded_gradient(api, oracle):
         assert np.abs(wa - wb).max() <= 1e-6 * max(1.0, moved * 10), (mode, weights is not None)
 
 
-@pytest.mark.parametrize("bags", [[300, 0, 1, 700], [4000, 20, 0, 700]], ids=["short", "long"])
+@pytest.mark.parametrize("bags", [[300, 0, 1, 700], [6000, 20, 0, 700]], ids=["short", "long"])
 @pytest.mark.parametrize("dim", [16, 6])
 @pytest.mark.parametrize("noted", [False, True])
 def test_combined_pooled_pull_and_push(api, oracle, bags, dim, noted):
     """krk_group_pull_pooled_parts / krk_group_push_pooled_parts over members that differ in mode and
     weights, one of them empty, one with positions outside every bag, gradients that are columns of
-    a wider matrix; requests on both sides of the 8192 ids a member up to which a push is two
+    a wider matrix; requests on both sides of the 12288 ids a member up to which a push is two
     launches, new ids every step, with and without the row notes of the pull. Binary-grid values:
     every sum is exact, so the rows are the oracle's bit for bit."""
     C = api.C

@@ -300,11 +300,11 @@ def test_push_raw_short_path_sizes(api, oracle, n, shape):
 @pytest.mark.parametrize("dim", [5, 16, 64])
 @pytest.mark.parametrize("shape", ["one_id", "one_bucket", "long_and_short", "boundary"])
 def test_push_raw_short_path_extremes(api, oracle, dim, shape):
-    """Requests of at most 8192 ids take the two-launch path (one workgroup per bucket of rows, LDS
-    sort, runs above 64 positions shared out over the workgroup). Its corners, against the oracle's
+    """Requests of at most 12288 ids take the two-launch path (one workgroup per bucket of rows, LDS
+    sort, long runs shared out over the workgroup). Its corners, against the oracle's
     dedup + sum + push: 8192 copies of one id (one run that fills the bucket), 8192 distinct rows that
     all fall into one bucket (the workgroup's arrays at their fullest), long runs next to short ones
-    at an odd row width, and the same ids as a request of 8192 and of 8193 (the second takes the
+    at an odd row width, and the same ids as a request of 12288 and of 12289 (the second takes the
     path of large requests). Dyadic gradients: exact whatever the order of additions. Random
     gradients: the long runs are added as per-lane-group stretches combined in a fixed tree, not
     strictly in position order, so they are held to the float64 sum."""
@@ -316,11 +316,11 @@ def test_push_raw_short_path_extremes(api, oracle, dim, shape):
     if shape == "one_id":
         requests = [np.full(8192, 4242, np.uint64)]
     elif shape == "one_bucket":
-        pool = splitmix64(np.arange(300_000, dtype=np.uint64))
-        t.Pull(pool)
-        r.pull(pool)
+        pool = splitmix64(np.arange(1_100_000, dtype=np.uint64))
+        for part in np.array_split(pool, 8):
+            t.Pull(part)
         rows = t.lookup(pool)
-        same = pool[rows % 32 == 0][:8192]                    # the short path's buckets are row mod 8..32
+        same = pool[rows % 128 == 0][:8192]                   # the short path's buckets are row mod 8..128
         assert same.size == 8192
         requests = [same]
     elif shape == "long_and_short":
@@ -328,8 +328,8 @@ def test_push_raw_short_path_extremes(api, oracle, dim, shape):
         ids = np.concatenate([np.repeat(hot, [3000, 900, 65, 64, 63]), splitmix64(np.arange(100, 4200, dtype=np.uint64))])
         requests = [ids[rng.permutation(ids.size)]]
     else:
-        base = zipf_ids(rng, 1.05, 10**5, 8193)
-        requests = [base[:8192], base]
+        base = zipf_ids(rng, 1.05, 10**5, 12289)
+        requests = [base[:12288], base]
     for ids in requests:
         t.Pull(ids)
         r.pull(ids)

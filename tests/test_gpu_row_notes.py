@@ -100,7 +100,7 @@ def test_notes_are_what_the_flagged_push_reads(api):
 
 
 def test_notes_are_dropped_when_they_do_not_apply(api):
-    """Another buffer, another count, an erase in between, a pull above 8192 ids, a later flagged
+    """Another buffer, another count, an erase in between, a pull whose push sorts, a later flagged
     pull of other ids: each time the flagged push_raw must act on the ids it is given."""
     dim = 16
     o = api.Optim.create(api.OptimType.kSGD)
@@ -154,7 +154,7 @@ def test_notes_are_dropped_when_they_do_not_apply(api):
     rc = t.Push(o, d_x, d_g, float(lr), raw=True, as_pulled=True)
     assert rc == 12
     t.Pull(x[:500])
-    big = np.arange(300000, 300000 + 9000, dtype=np.uint64)
+    big = np.arange(300000, 300000 + 13_000, dtype=np.uint64)
     d_big = api.DeviceArray.from_host(big)
     d_gbig = api.DeviceArray.from_host(np.ones((big.size, dim), np.float32))
     assert t.Pull(d_big, note_rows=True)[0] == 0         # noted, but a push_raw this long sorts by itself
@@ -204,6 +204,48 @@ def test_group_with_notes_equals_without(api, dim):
     counts2 = [3000, 0, 1, 8192 - 5, 777 + 5]
     off2 = ga._offsets(counts2)
     assert ga.CombinePushRaw(o, d_ids, off2, d_g, 0.05, as_pulled=True) in (0, 12)
+    ga.close()
+    gb.close()
+
+
+@pytest.mark.parametrize("dim,longest", [(16, 14_000), (5, 14_000), (128, 700)])
+def test_group_sorted_push_with_notes_equals_without(api, dim, longest):
+    """A combined push with repeats that sorts over the whole request (a member above 12288 ids, or rows
+    above 64 floats) takes its keys from the notes: against the same calls without the flags, and
+    with the buffer overwritten after the pull, where the rows of the pulled ids move and the others'
+    do not. Binary-grid gradients: the sums do not depend on the numbers of the rows."""
+    rng = np.random.default_rng(dim + longest)
+    o = api.Optim.create(api.OptimType.kAdagrad)
+    counts = [3000, 0, 1, longest, 777]
+    ta = [api.SparseTable(dim, _init(api)) for _ in counts]
+    tb = [api.SparseTable(dim, _init(api)) for _ in counts]
+    ga, gb = api.TableGroup(ta), api.TableGroup(tb)
+    off = ga._offsets(counts)
+    total = int(off[-1])
+    d_ids = api.DeviceArray(total, np.uint64)
+    d_g = api.DeviceArray((total, dim), np.float32)
+    for step in range(3):
+        per = [zipf_ids(rng, 1.05, 30000, c) + np.uint64(step * 7000) for c in counts]
+        _h2d(api, d_ids, np.concatenate(per))
+        _h2d(api, d_g, (rng.integers(-64, 65, size=(total, dim)) / 4096.0).astype(np.float32))
+        assert ga.CombinePull(d_ids, off, note_rows=True)[0] == 0
+        assert gb.CombinePull(d_ids, off)[0] == 0
+        assert ga.CombinePushRaw(o, d_ids, off, d_g, 0.05, as_pulled=True) == 0
+        assert gb.CombinePushRaw(o, d_ids, off, d_g, 0.05) == 0
+    for a, b, c in zip(ta, tb, counts):
+        if c:
+            _same_tables(api, a, b, [api.StateType.kStateSum])
+    sgd = api.Optim.create(api.OptimType.kSGD)
+    x = [np.arange(1, c + 1, dtype=np.uint64) + np.uint64(10**6) for c in counts]
+    y = [i + np.uint64(10**6) for i in x]
+    _h2d(api, d_g, np.ones((total, dim), np.float32))
+    before = [(t.Pull(i)[1], t.Pull(j)[1]) for t, i, j in zip(ta, x, y)]
+    _h2d(api, d_ids, np.concatenate(x))
+    assert ga.CombinePull(d_ids, off, note_rows=True)[0] == 0
+    _h2d(api, d_ids, np.concatenate(y))
+    assert ga.CombinePushRaw(sgd, d_ids, off, d_g, 0.5, as_pulled=True) == 0
+    for t, i, j, (bx, by) in zip(ta, x, y, before):
+        assert np.array_equal(t.Pull(i)[1], bx - np.float32(0.5)) and np.array_equal(t.Pull(j)[1], by)
     ga.close()
     gb.close()
 
@@ -281,10 +323,10 @@ def test_group_push_of_unique_ids_with_notes_equals_without(api, dim):
     gb.close()
 
 
-@pytest.mark.parametrize("n", [8193, 300_000])
+@pytest.mark.parametrize("n", [8193, 20_000, 300_000])
 def test_long_pushes_with_notes_equal_those_without(api, n):
-    """push_raw of requests that are sorted (above 8192 ids, and above the size from which a pull runs
-    as two launches), and the pooled pull and push of one table, with and without the flags. Binary-grid
+    """push_raw of a request below the 12288 ids from which it is sorted, of one above them whose pull is
+    still one launch, and of one whose pull runs as two, and the pooled pull and push of one table, with and without the flags. Binary-grid
     gradients: the sums do not depend on how equal rows are grouped."""
     dim = 8
     rng = np.random.default_rng(n)

@@ -268,3 +268,100 @@ def test_ids_unpacked_by_hooks_are_looked_up_again(mods, oracle, kind):
     p.push(first, ca)
     p.push(second, cb)
     p.check("after two backward passes through one buffer")
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_expanded_gradient(mods, oracle, kind):
+    """The gradient of a plain sum is one value expanded over the output; that of a sum over the batch is
+    one row, read by every position."""
+    p = Pair(mods, oracle, kind)
+    rng = np.random.default_rng(10)
+    row = (np.arange(DIM, dtype=np.float32) - 8) / 16
+    for step in range(4):
+        batch = p.draw(rng, 40)
+        outs = p.forward(batch)
+        seen = []
+        for o in outs:
+            o.register_hook(lambda g: seen.append(g.stride()[0]))
+        if step % 2:
+            sum(o.sum() for o in outs).backward()
+            want = np.ones((40, DIM), np.float32)
+        else:
+            sum((o.sum(dim=0) * torch.from_numpy(row).cuda()).sum() for o in outs).backward()
+            want = np.tile(row, (40, 1))
+        assert seen == [0] * len(outs)
+        p.push(batch, [want] * len(outs))
+    p.check("after expanded gradients")
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_backward_twice_over_a_retained_graph(mods, oracle, kind):
+    """Every backward pushes; without retain_graph a second one is refused."""
+    p = Pair(mods, oracle, kind)
+    rng = np.random.default_rng(11)
+    batch = p.draw(rng, 48)
+    coefs = _coef(rng, 48, p.tables)
+    loss = _loss(p.forward(batch), coefs)
+    loss.backward(retain_graph=True)
+    p.push(batch, coefs)
+    loss.backward()
+    p.push(batch, coefs)
+    with pytest.raises(RuntimeError, match="second time"):
+        loss.backward()
+    p.check("after two backward passes")
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_saved_tensors_on_the_host(mods, oracle, kind):
+    p = Pair(mods, oracle, kind)
+    rng = np.random.default_rng(12)
+    for _ in range(2):
+        batch = p.draw(rng, 48)
+        coefs = _coef(rng, 48, p.tables)
+        with torch.autograd.graph.save_on_cpu():
+            loss = _loss(p.forward(batch), coefs)
+        loss.backward()
+        p.push(batch, coefs)
+    p.check("after backward passes over saved tensors from the host")
+
+
+def test_pooled_request_a_table_at_a_time(mods, oracle):
+    """A request above what one combined call takes goes through the tables' own calls, forward and
+    backward, with an output that has no gradient among them, and may change from step to step."""
+    p = Pair(mods, oracle, "combine_jagged", (1, {}))
+    rng = np.random.default_rng(13)
+    limit = p.param._native.combined_max
+    for step in range(4):
+        p.param._native.combined_max = 50 if step in (1, 2) else limit
+        batch = p.draw(rng, 64)
+        outs = p.forward(batch)
+        coefs = _coef(rng, 64, 2)
+        _loss(outs, [coefs[0], None if step == 2 else coefs[1]]).backward()
+        p.push(batch, [coefs[0], np.zeros_like(coefs[1]) if step == 2 else coefs[1]])
+    p.check("after requests of both kinds")
+
+
+def test_pooled_push_whose_keys_do_not_fit_goes_a_table_at_a_time(mods, oracle):
+    """32 tables of which one has room for more than 2^26 rows: member and row number take 33 bits, and
+    the combined push answers that it cannot (KRK_E_CAPACITY)."""
+    api, te = mods
+    n_tables, dim = 32, 4
+    init = api.Initializer.create(api.InitializerType.kConstant, {"value": "1"})
+    emb = te.CombineJaggedEmbedding([dim] * n_tables, [init] * n_tables, optim=api.Optim.create(api.OptimType.kSGD),
+                                    lr=0.5)
+    emb.combine_sparse_table.tables()[3].reserve((1 << 26) + 1)
+    rng = np.random.default_rng(14)
+    ids = [rng.integers(0, 50, size=60) for _ in range(n_tables)]
+    off = torch.arange(0, 61, 3).cuda()                  # 20 bags of three
+    outs = emb([te.JaggedTensor(torch.from_numpy(i).cuda(), off) for i in ids])
+    assert all(torch.equal(o, torch.full((20, dim), 3.0, device="cuda")) for o in outs)
+    group = emb.combine_sparse_table._groups[dim]
+    assert group.CombinePushRaw(emb.combine_sparse_table._optim, np.concatenate(ids).astype(np.uint64),
+                                np.arange(0, 60 * n_tables + 1, 60), np.zeros((60 * n_tables, dim), np.float32),
+                                0.5) == api.E_CAPACITY
+    sum(o.sum() for o in outs).backward()
+    torch.cuda.synchronize()
+    for i, t in zip(ids, emb.combine_sparse_table.tables()):
+        u, count = np.unique(i, return_counts=True)
+        want = 1.0 - 0.5 * count.astype(np.float32)
+        assert np.array_equal(t.Pull(u.astype(np.uint64))[1], np.repeat(want[:, None], dim, axis=1))
