@@ -45,7 +45,8 @@ extern "C" {
  * KRK_DEVICE_PTRS and are ignored by every other call.
  * KRK_NOTE_ROWS on krk_sparse_pull / krk_group_pull and their pooled forms: the table (group)
  * also keeps the row number of every position of this request (4 bytes a position, in memory of
- * its own) until its next pull with the flag.
+ * its own) until its next pull with the flag. Where the device has no room for them the pull goes on
+ * without.
  * KRK_IDS_AS_PULLED on krk_sparse_push / krk_sparse_push_raw / krk_group_push /
  * krk_group_push_raw and the pooled pushes: the caller states that `ids` is the buffer of that
  * pull (same pointer, same counts) with its contents unchanged. The call then skips its own

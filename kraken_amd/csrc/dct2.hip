@@ -339,8 +339,9 @@ static int32_t ensure_basis(hipStream_t s) {
 // Wavefronts of a workgroup. Eight, a row tile of 256 blocks: a workgroup more or less a compute unit
 // owns one whatever the width (the basis fills up to 98 KB of its LDS), and with sixteen a
 // request of a few thousand blocks kept only a few units busy while the largest was no faster
-// (forward + inverse as blocking calls, sixteen / eight, us: 10,000 blocks keep 64 56 / 42, keep 256
-// 72 / 51; 262,144 blocks 155 / 150 and 304 / 295). Four for requests so small that tiles of
+// (forward + inverse as blocking calls, sixteen / eight, us: 10,000 blocks keep 64 57 / 42, keep 256
+// 73 / 51; 100,000 blocks 88 / 81 and 147 / 145; 262,144 blocks 154 / 152 and 305 / 304, no
+// difference beyond that between two runs of one side). Four for requests so small that tiles of
 // 128 blocks still leave units idle (eight / four: 4000 blocks 42 / 38 and 50 / 48; 10,000 blocks
 // keep 256 51 / 60: a workgroup of four takes longer to lay its basis out).
 constexpr int64_t kFewRows = 4096;

@@ -1226,7 +1226,6 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(
     std::conditional_t<POOLED, BucketPooled, int> pool) {
   __shared__ uint32_t skey[kSortMax];                  // row >> bucket_bits
   __shared__ uint16_t spos[kSortMax];
-  // histogram [wave][digit] while sorting; partial sums and their keys while reducing
   // histogram [wave][digit] while sorting; then run starts, the list of long runs, and the
   // wavefronts' partial sums of a long run
   __shared__ __align__(16) uint32_t work[kPartOffset + kSortWaves * kWave * 4];
@@ -1305,7 +1304,6 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(
   const int per_lane = (len + kSortBlock - 1) / kSortBlock;   // 1..12
   const int padded = per_lane * kSortBlock;
   for (int j = len + t; j < padded; j += kSortBlock) {   // beyond what the lanes above wrote
-
     skey[j] = 0xFFFFFFFFu;                             // padding sorts behind everything
     spos[j] = 0;
   }
@@ -1662,7 +1660,7 @@ static void launch_bucket_push(int opt, unsigned buckets, hipStream_t stream, co
 }
 
 // Workgroups per table: as many as keep the request within about one workgroup per compute unit
-// (a workgroup's LDS leaves room for one per unit), between 8 and 32.
+// (a workgroup's LDS leaves room for one per unit), between 8 and 128.
 static int short_bucket_bits(int n_tables) {
   int bits = kMaxBucketBits;
   while (bits > 3 && (n_tables << bits) > 256) --bits;
