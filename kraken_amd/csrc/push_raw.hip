@@ -561,10 +561,16 @@ __global__ __launch_bounds__(kBlock) void bag_expand_kernel(const TableDesc* __r
   const int64_t a = call.row_start[m];
   const int64_t n = call.row_start[m + 1] - a;
   const long long begin = call.offsets[m][b], end = call.offsets[m][b + 1];
+  const long long first = call.offsets[m][0], past = call.offsets[m][bags];
   const uint32_t word = words.pack((uint32_t)b, end - begin);
   const bool weighted = call.weights[m] != nullptr;
   const uint32_t member_key = (uint32_t)m << row_bits;
-  const long long lo = begin < 0 ? 0 : begin, hi = end > n ? n : end;
+  // Offsets on the device are not checked. Whatever they hold, a position in [first, past) lies in some
+  // bag (the one at which the offsets step over it) and the others in none, so that every position is
+  // written; a bag that reaches beyond, as offsets that descend let it, must not write where
+  // `outside` does: a position with its key from the one and its bag from the other would be read
+  // from a gradient row that does not exist.
+  const long long lo = max(begin, max(first, 0ll)), hi = min(end, min(past, (long long)n));
   for (long long p = lo + gl; p < hi; p += kBagLanes) {
     if (NOTED) {
       keys[a + p] = noted_key(tv, notes[a + p], call.ids[m] + p, member_key, miss_key);
@@ -582,8 +588,8 @@ __global__ __launch_bounds__(kBlock) void bag_expand_kernel(const TableDesc* __r
       }
     }
   };
-  if (b == 0) outside(0, begin < n ? begin : n);
-  if (b == bags - 1) outside(end > 0 ? end : 0, n);
+  if (b == 0) outside(0, first < n ? first : n);
+  if (b == bags - 1) outside(past > 0 ? past : 0, n);
 }
 
 // ---------------------------------------------------------------------------

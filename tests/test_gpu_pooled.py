@@ -269,3 +269,56 @@ def test_combined_pooled_pull_and_push(api, oracle, bags, dim, noted):
     one[0] = Part(d_ids.ptr, 40, d_off.ptr, 1, None, keep[0][1].ptr, dim, 0, 0.0)
     assert api.lib().krk_group_push_pooled_parts(group.h, C.byref(o_gpu.raw), one, dim, 0.5, flags) == api.SPARSE_ID_NOT_EXIST
     group.close()
+
+
+@pytest.mark.parametrize("filler", [0, 14_000], ids=["short", "long"])
+@pytest.mark.parametrize("noted", [False, True])
+@pytest.mark.parametrize("weighted", [False, True])
+@pytest.mark.parametrize("grouped", [False, True])
+def test_offsets_that_descend_stay_inside_the_request(api, filler, noted, weighted, grouped):
+    """Offsets on the device are not read back to be checked. Where they descend, a position between the
+    first and the last offset belongs to a bag that the offsets step over it with, every other position to
+    none, whatever bags reach over it; nothing outside the arrays is read. Bags that overlap have the
+    same gradient row here, so that it does not matter which of them a position is given to."""
+    C, dim, n = api.C, 4, 40 + filler
+    gi = api.Initializer.create(api.InitializerType.kConstant, {"value": "1"})
+    t = api.SparseTable(dim, gi)
+    group = api.TableGroup([t]) if grouped else None
+    sgd = api.Optim.create(api.OptimType.kSGD)
+    ids = splitmix64(np.arange(n, dtype=np.uint64))
+    d_ids = api.DeviceArray.from_host(ids)
+    w = np.full(n, 0.5, np.float32) if weighted else None
+    d_w = api.DeviceArray.from_host(w) if weighted else None
+    p = lambda x: C.c_void_p(x.ptr) if x is not None else None
+    top = n - 10
+    for off in ([5, 2, 8, 8, 20, 11, top], [top, 30, 5], [0, n + 7, -3, n], [-(1 << 40), 7, 1 << 40], [12, 12, 12],
+                [n + 100, 3, 9, n + 200], [3, -1, -9]):
+        off = np.array(off, np.int64)
+        bags = off.size - 1
+        d_off = api.DeviceArray.from_host(off)
+        d_g = api.DeviceArray.from_host(np.ones((bags, dim), np.float32))
+        out = api.DeviceArray((bags, dim), np.float32)
+        before = t.Pull(ids)[1]
+        flags = api.DEVICE_PTRS
+        note, pulled = (api.NOTE_ROWS, api.IDS_AS_PULLED) if noted else (0, 0)
+        if grouped:
+            class Part(C.Structure):
+                _fields_ = [("ids", C.c_void_p), ("n", C.c_int64), ("offsets", C.c_void_p), ("bags", C.c_int64),
+                            ("weights", C.c_void_p), ("rows", C.c_void_p), ("stride", C.c_int64), ("mode", C.c_int32),
+                            ("patch", C.c_float)]
+            part = lambda rows: (Part * 1)(Part(d_ids.ptr, n, d_off.ptr, bags, d_w.ptr if weighted else None, rows.ptr,
+                                                dim, 0, 0.0))
+            assert api.lib().krk_group_pull_pooled_parts(group.h, part(out), flags | note) == 0
+            assert api.lib().krk_group_push_pooled_parts(group.h, C.byref(sgd.raw), part(d_g), dim, 0.5,
+                                                         flags | pulled) == 0
+        else:
+            assert api.lib().krk_sparse_pull_pooled(t.h, p(d_ids), n, p(d_off), bags, p(d_w), 0, 0.0, p(out),
+                                                    flags | note) == 0
+            assert api.lib().krk_sparse_push_pooled(t.h, C.byref(sgd.raw), p(d_ids), n, p(d_off), bags, p(d_w), 0,
+                                                    p(d_g), dim, 0.5, flags | pulled) == 0
+        at = np.arange(n)
+        moved = (at >= off[0]) & (at < off[-1])
+        want = before - np.float32(0.25 if weighted else 0.5) * moved[:, None].astype(np.float32)
+        assert np.array_equal(t.Pull(ids)[1], want), off[:3]
+    if group:
+        group.close()
