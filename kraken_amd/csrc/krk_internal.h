@@ -94,7 +94,7 @@ constexpr size_t kBounceMax = (size_t)1 << 20;
 // runtime / everything read in place / by this rule: pooled pushes of 10,000 bags of 16 floats, ten
 // ids each, 164 / 233 / 144, 2048 bags of 64 floats, 40 weighted ids each, 186 / 260 / 151, 256
 // bags of 16 floats, four ids each (read in place) 91 / 41 / 41; push_raw of 16,000 ids of 8 floats
-// 110 / 117 / 96; a codec step that selects over 260,000 values 352 / 421 / 341.
+// 110 / 117 / 96; a codec step that selects over 260,000 values 168 / 228 / 145.
 constexpr size_t kHostPiece = 128;
 constexpr size_t kReadAgainMin = (size_t)128 << 10;
 // bytes that `reads` reads of `bytes` each take across PCIe

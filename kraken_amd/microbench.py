@@ -315,6 +315,74 @@ def host():
     grp.close()
     for t in tables:
         t.close()
+    host_arguments(init)
+
+
+def host_arguments(init):
+    """Blocking calls whose pageable arguments the kernels read several times over or out of order, and
+    the first calls of a table."""
+    import time
+    rng = np.random.default_rng(1)
+    o = api.Optim.create(api.OptimType.kAdagrad)
+
+    def median(fn, n=40):
+        times = []
+        for _ in range(n + 5):
+            t0 = time.perf_counter()
+            fn()
+            times.append(time.perf_counter() - t0)
+        return float(np.median(times[5:])) * 1e6
+
+    resident = np.arange(100_000, dtype=np.uint64)
+    for dim, bags, each in ((16, 256, 4), (16, 10_000, 10), (64, 4096, 2), (64, 2048, 40)):
+        t = api.SparseTable(dim, init, capacity_hint=200_000)
+        t.Pull(resident)
+        ids = rng.integers(0, resident.size, bags * each).astype(np.uint64)
+        off = np.arange(bags + 1, dtype=np.int64) * each
+        g = rng.standard_normal((bags, dim)).astype(np.float32)
+        w = rng.random(ids.size).astype(np.float32)
+        print("pooled push, pageable, %5d bags of %2d ids, dim %2d | sum %7.1f us | weighted mean %7.1f us" % (
+            bags, each, dim, median(lambda: t.PushPooled(o, ids, off, g, 0.01)),
+            median(lambda: t.PushPooled(o, ids, off, g, 0.01, mode="mean", weights=w))), flush=True)
+        t.close()
+    for dim, n in ((16, 4000), (8, 16_000)):
+        t = api.SparseTable(dim, init, capacity_hint=200_000)
+        t.Pull(resident)
+        ids = rng.integers(0, resident.size, n).astype(np.uint64)
+        g = rng.standard_normal((n, dim)).astype(np.float32)
+        print("push_raw, pageable, %5d ids, dim %2d              | %7.1f us" % (
+            n, dim, median(lambda: t.PushRaw(o, ids, g, 0.01))), flush=True)
+        t.close()
+    n = 260_000
+    bag = api.DenseBag(n)
+    g, idx, val = rng.standard_normal(n).astype(np.float32), np.zeros(n, np.int64), np.zeros(n, np.float32)
+    nnz = api.C.c_int64()
+    print("codec, pageable, %d values, a selection each step | %7.1f us" % (n, median(
+        lambda: api.lib().krk_dct_compress(bag.h, api._ptr(g), 1, 0.75, api._ptr(idx), api._ptr(val), n,
+                                           api.C.byref(nnz), 0))), flush=True)
+    bag.close()
+    d = api.DenseTable(np.zeros(1 << 26, np.float32))
+    val = rng.standard_normal(100).astype(np.float32)
+    front = np.arange(100, dtype=np.int64)
+    for name, idx in (("spread", front * ((1 << 26) // 100)), ("at the front", front)):
+        print("sparse push, 100 entries into %d, %-12s | %7.1f us" % (1 << 26, name, median(
+            lambda: d.PushCoo(o, idx, val, 0.01), 15)), flush=True)
+    d.close()
+    first = []
+    ids = rng.integers(0, resident.size, 4000).astype(np.uint64)
+    g = rng.standard_normal((4000, 16)).astype(np.float32)
+    for _ in range(10):
+        t = api.SparseTable(16, init, capacity_hint=200_000)
+        api.synchronize()
+        at = [time.perf_counter()]
+        for fn in (lambda: t.Pull(ids), lambda: t.PushRaw(o, ids, g, 0.01), lambda: t.Pull(ids),
+                   lambda: t.PushRaw(o, ids, g, 0.01)):
+            fn()
+            at.append(time.perf_counter())
+        first.append(np.diff(at) * 1e6)
+        t.close()
+    print("first calls of a table, pageable, 4000 ids, dim 16 | pull %.0f, push_raw %.0f, pull %.0f, push_raw %.0f us" %
+          tuple(np.median(first, axis=0)), flush=True)
 
 
 def pooled():
