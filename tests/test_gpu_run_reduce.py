@@ -1,0 +1,132 @@
+"""Pushes of more than 12288 ids and krk_dedup_sum up to 2^20 ids: pairs grouped by bucket, every bucket
+sorted and added up by one workgroup, buckets that hold more pairs than a workgroup takes cut into
+chunks and merged. Gradients lie on a binary grid, so that every order of additions gives the same
+bits: sums are compared exactly.
+"""
+import numpy as np
+import pytest
+
+from util import splitmix64, zipf_ids
+
+pytestmark = pytest.mark.gpu
+
+MULT = 0x9E3779B1                                       # of the keys' hash
+
+
+@pytest.fixture(scope="module")
+def api():
+    from kraken_amd import api as a
+    a.lib()
+    return a
+
+
+def _grid(rng, shape):
+    return (rng.integers(-64, 65, size=shape) / 4096.0).astype(np.float32)
+
+
+def _sums(inv, grads, n):
+    """Exact while they stay below 2^11."""
+    return np.stack([np.bincount(inv, weights=grads[:, c].astype(np.float64), minlength=n) for c in range(grads.shape[1])],
+                    1).astype(np.float32)
+
+
+def _bucket(keys, bits, bucket_bits=10):
+    return ((keys.astype(np.uint64) * np.uint64(MULT)) & np.uint64((1 << bits) - 1)) >> np.uint64(bits - bucket_bits)
+
+
+def _crowded(rng, n, unique, bits, rows):
+    """n keys below `unique`, every key once, the others taken in turn from `rows` keys of one bucket: its
+    chunks hold more short runs than the merge takes at once."""
+    keys = np.arange(unique)
+    bucket = _bucket(keys, bits)
+    fullest = np.bincount(bucket.astype(np.int64)).argmax()
+    crowd = keys[bucket == fullest][:rows]
+    assert crowd.size == rows
+    return np.concatenate([keys, np.resize(rng.permutation(crowd), n - unique)])
+
+
+# 128 pairs a bucket: more buckets from 32769 and 65537 pairs on; other tiles from 65537, the counts' scan
+# a launch of its own from 262145, longer chunks too; sorted from 2^20 + 1
+@pytest.mark.parametrize("n", [1, 8193, 32768, 32769, 65536, 65537, 2**18, 2**18 + 1, 2**20, 2**20 + 1])
+@pytest.mark.parametrize("kind", ["distinct", "same", "zipf"])
+def test_dedup_sum_sizes(api, n, kind):
+    rng = np.random.default_rng(n)
+    ids = {"distinct": splitmix64(np.arange(n, dtype=np.uint64)), "same": np.full(n, 7, np.uint64),
+           "zipf": zipf_ids(rng, 1.2, 10**5, n)}[kind]
+    grads = _grid(rng, (n, 4))
+    u, inv, sums = api.dedup_sum(ids, grads)
+    assert np.array_equal(u[inv], ids)
+    assert np.array_equal(sums, _sums(inv, grads, u.size))
+
+
+# 39 rows of one bucket 1000 times each: lists of some 5000 entries are taken by ranges of keys; two rows of
+# one bucket, the second of which leaves three entries in each of a thousand chunks, more than the
+# 2048 that fit at once: window by window. dim 300: a row is more than a wavefront holds
+@pytest.mark.parametrize("n", [80_000, 2**20])
+@pytest.mark.parametrize("dim", [3, 8, 300])
+def test_dedup_sum_crowded_bucket(api, n, dim):
+    rng = np.random.default_rng(n + dim)
+    if n == 80_000:
+        keys = _crowded(rng, n, 40_000, 17, 39)
+    else:
+        keys = _crowded(rng, n, 2048, 20, 2)
+        hot, other = keys[2048], keys[2049]
+        keys[2048:] = np.where(np.arange(n - 2048) % 342 == 0, other, hot)
+    grads = _grid(rng, (n, dim))
+    u, inv, sums = api.dedup_sum(splitmix64(keys.astype(np.uint64)), grads)
+    assert np.array_equal(inv, keys)
+    assert np.array_equal(sums, _sums(keys, grads, u.size))
+
+
+@pytest.mark.parametrize("dim", [4, 6, 260])
+@pytest.mark.parametrize("noted", [False, True])
+@pytest.mark.parametrize("shape", ["zipf", "crowded"])
+def test_push_raw_and_pooled(api, dim, noted, shape):
+    """A table alone, two tables together, bags with weights and means: the same sums."""
+    rows, n = 1 << 15, 70_000
+    rng = np.random.default_rng(dim + noted)
+    names = splitmix64(np.arange(rows, dtype=np.uint64))
+    make = lambda: api.SparseTable(dim, api.Initializer.create(api.InitializerType.kConstant, {"value": "1"}),
+                                   capacity_hint=1 << 17)
+    tables = [make() for _ in range(3)]
+    for t in tables:
+        t.Pull(names)
+    order = np.argsort(tables[0].lookup(names))         # ids by row number
+    if shape == "zipf":
+        ids = zipf_ids(rng, 1.3, rows, n)
+        assert np.isin(ids, names).all()
+    else:
+        ids = names[order][_crowded(rng, n, rows, 17, 30)]   # 2^17 rows of room
+    sgd = api.Optim.create(api.OptimType.kSGD)
+    grads = _grid(rng, (n, dim))
+    u, inv = np.unique(ids, return_inverse=True)
+    d = lambda a: api.DeviceArray.from_host(a)
+    d_ids, d_grads, out = d(ids), d(grads), api.DeviceArray((n, dim), np.float32)
+    t = tables[0]
+    assert t.Pull(d_ids, out=out, note_rows=noted)[0] == 0
+    assert t.PushRaw(sgd, d_ids, d_grads, 0.5, as_pulled=noted) == 0
+    assert np.array_equal(t.Pull(u)[1], np.float32(1) - np.float32(0.5) * _sums(inv, grads, u.size))
+    # together: the second member is the short one
+    group = api.TableGroup(tables[1:])
+    counts = [n, 500]
+    both, g2 = np.concatenate([ids, ids[:500]]), np.concatenate([grads, grads[:500]])
+    d_ids, d_grads, out = d(both), d(g2), api.DeviceArray((n + 500, dim), np.float32)
+    offsets = group._offsets(counts)
+    assert group.CombinePull(d_ids, offsets, out=out, note_rows=noted)[0] == 0
+    assert group.CombinePushRaw(sgd, d_ids, offsets, d_grads, 0.5, as_pulled=noted) == 0
+    assert np.array_equal(tables[1].Pull(u)[1], np.float32(1) - np.float32(0.5) * _sums(inv, grads, u.size))
+    few, back = np.unique(ids[:500], return_inverse=True)
+    assert np.array_equal(tables[2].Pull(few)[1], np.float32(1) - np.float32(0.5) * _sums(back, grads[:500], few.size))
+    group.close()
+    # bags of eight: a mean's ratio is 1/8, weights are powers of two
+    bags = n // 8
+    bag_grads = _grid(rng, (bags, dim))
+    weights = (2.0 ** rng.integers(-1, 2, size=bags * 8)).astype(np.float32)
+    for mode, w in (("sum", None), ("mean", None), ("mean", weights)):
+        before = t.Pull(u)[1]
+        assert t.PushPooled(sgd, ids[:bags * 8], np.arange(bags + 1) * 8, bag_grads, 0.5, mode=mode, weights=w) == 0
+        each = np.repeat(bag_grads, 8, 0) * np.float32(1 if mode == "sum" else 0.125)
+        if w is not None:
+            each = each * w[:, None]
+        want = before - np.float32(0.5) * _sums(inv[:bags * 8], each, u.size)
+        assert np.array_equal(t.Pull(u)[1], want), mode
