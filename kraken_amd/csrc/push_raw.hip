@@ -116,12 +116,7 @@ constexpr int kRankTile = kDedupBlock;
 // Exclusive scan over the 1024 lanes of a workgroup; *all = the sum. Ends behind a barrier.
 __device__ __forceinline__ uint32_t dedup_block_scan(uint32_t v, uint32_t* wave_total, uint32_t* all) {
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  uint32_t incl = v;
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const uint32_t y = __shfl_up(incl, d);
-    if (lane >= d) incl += y;
-  }
+  const uint32_t incl = wave_inclusive_sum(v);
   if (lane == kWave - 1) wave_total[wave] = incl;
   __syncthreads();
   uint32_t before = incl - v, sum = 0;
@@ -279,12 +274,7 @@ __global__ __launch_bounds__(kDedupBlock) void dedup_small_kernel(const uint64_t
   // exclusive scan of the counts over the workgroup
   const int lane = t & (kWave - 1), wave = t / kWave;
   const uint32_t mine = (uint32_t)__popc(first);
-  uint32_t incl = mine;
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const uint32_t y = __shfl_up(incl, d);
-    if (lane >= d) incl += y;
-  }
+  const uint32_t incl = wave_inclusive_sum(mine);
   if (lane == kWave - 1) wave_total[wave] = incl;
   __syncthreads();                                     // also: every first occurrence has been read from the table
   uint32_t rank = incl - mine, all = 0;
@@ -864,7 +854,7 @@ static void dispatch_segreduce(int opt, bool level0, const TableView& tv, const 
 constexpr int kLevel0Tile = 16;
 
 // ---------------------------------------------------------------------------
-// Requests of at most 12288 ids per table (twelve positions a lane: what the LDS of a compute unit holds
+// Requests of 2049 to 12288 ids per table (shorter ones: pick_runs; twelve positions a lane: what the LDS of a compute unit holds
 // besides the run lists, one workgroup a unit as with eight; the global sort that longer requests
 // take is six to nine launches: an embedding step of 10,000 ids of 16 floats, forward, backward,
 // forward, 61 us with it and 39 us with this): two launches, no carry levels, no global sort.
@@ -874,8 +864,8 @@ constexpr int kLevel0Tile = 16;
 //      workgroup per compute unit), so that both one table and 26 tables use much of the chip:
 //      a. the workgroup reads its table's row numbers and keeps the positions of its bucket, in
 //         position order (one scan over the workgroup);
-//      b. the (row, position) pairs are sorted by row in LDS with a stable radix sort, nine bits
-//         a pass (two passes for tables of up to two million rows). Every wavefront ranks its own
+//      b. the (row, position) pairs are sorted by row in LDS: up to 256 of them by counting
+//         (rank_list, 0.4-2.4 us), more with a stable radix sort, nine bits a pass (two passes for tables of up to two million rows). Every wavefront ranks its own
 //         elements with wave-wide votes (lanes holding the same digit find each other through
 //         nine ballots), a per-wavefront histogram in LDS turns into offsets by one scan over
 //         (digit, wavefront), and the pairs are scattered through LDS;
@@ -960,12 +950,7 @@ __device__ __forceinline__ unsigned long long match_digit(uint32_t digit) {
 __device__ __forceinline__ uint32_t sort_block_scan(uint32_t v, uint32_t* wave_total, uint32_t& total) {
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
-  uint32_t incl = v;
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const uint32_t y = __shfl_up(incl, d);
-    if (lane >= d) incl += y;
-  }
+  const uint32_t incl = wave_inclusive_sum(v);
   lds_barrier();                                     // wave_total may still be read from a previous scan
   if (lane == kWave - 1) wave_total[wave] = incl;
   lds_barrier();
@@ -1072,7 +1057,9 @@ __global__ __launch_bounds__(kSortBlock) void bucket_push_kernel(
   lds_barrier();
 
   // ---- b. stable sort by row -----------------------------------------------------------------
-  {
+  if (len <= kRankMax) {
+    rank_list(skey, spos, len, 0xFFFFFFFFu);
+  } else {
     // element i of lane l in wavefront w is pair w * 64 * per_lane + i * 64 + l: a wavefront's
     // elements are consecutive, and taking i in ascending order visits them in list order
     uint32_t* hist = work;                             // [kSortWaves][kDigits]
@@ -1938,8 +1925,13 @@ int32_t krk_dedup_sum(const uint64_t* ids, int64_t n, const float* grads, int64_
   tv.stride = dim;
   ApplyArgs args{};
   args.c0 = args.c1 = args.c2 = args.meta_off = -1;
-  KRK_TRY(fill_and_reduce(sh, s, g_dedup_reduce, tv, kOptStore, n, miss_key, bits, d_g, args, PooledSrc{}, nullptr,
-                          nullptr, NotedRows{}, [](uint32_t*, uint32_t*) {}));
+  if (n <= kPickMax) {
+    KRK_TRY(pick_runs(sh, s, tv, kOptStore, keys, miss_key, bits, 0xFFFFFFFFu, nullptr, false, n, n, d_g, args,
+                      PooledSrc{}, nullptr, nullptr));
+  } else {
+    KRK_TRY(fill_and_reduce(sh, s, g_dedup_reduce, tv, kOptStore, n, miss_key, bits, d_g, args, PooledSrc{}, nullptr,
+                            nullptr, NotedRows{}, [](uint32_t*, uint32_t*) {}));
+  }
   KRK_TRY(dedup_read_count(s, &u));
   *n_unique = u;
   if (host) {
@@ -2034,8 +2026,8 @@ int32_t krk_sparse_push_raw(krk_sparse* t, const krk_optim* o, const uint64_t* i
   // the rows are read in the order of the sorted ids
   KRK_TRY(t->input(grads, (size_t)n * t->dim, flags, 1, &d_g, host_reads(n, t->dim * 4)));
 
-  if (short_push_fits(n, t->dim, t->elems, t->group)) {
-    // a short request: see bucket_push_kernel
+  if (n <= kPickMax || short_push_fits(n, t->dim, t->elems, t->group)) {
+    // a short request: see pick_runs and bucket_push_kernel
     SortCall sc = table_sort_call(t, n);
     const ApplyArgs args = table_apply_args(t, o, lr);
     const TableView tv = t->view();
@@ -2051,6 +2043,12 @@ int32_t krk_sparse_push_raw(krk_sparse* t, const krk_optim* o, const uint64_t* i
       keys = found;
     } else {
       sc.noted = 1;
+    }
+    if (n <= kPickMax) {
+      const ReduceShape sh{t->dim, t->vec, t->elems, t->group};
+      KRK_TRY(pick_runs(sh, t->stream, tv, o->type, keys, sc.miss_key, sc.row_bits, sc.row_mask, d_ids, noted, n, n, d_g,
+                        args, PooledSrc{}, nullptr, nullptr));
+      return sparse_finish(t, flags);
     }
     const GroupSrc none{nullptr, 0, -1, -1, -1, 0};
     GroupParts parts;
@@ -2166,8 +2164,13 @@ static int32_t group_push_raw_enqueue(krk_group* g, const krk_optim* o, const in
   const GroupCall rows_call = group_rows_layout(call, offsets, n_tables);
   const ApplyArgs args = group_apply_args(o, lr);
   const GroupSrc gs = group_src(g, o, row_bits);
-  if (short_push_fits(longest, g->dim, g->elems, g->group)) {
-    // short members: see bucket_push_kernel
+  const ReduceShape sh{g->dim, g->vec, g->elems, g->group};
+  GroupPooledSrc src{};                        // not pooled: a payload is a position of its member
+  src.call.n_tables = n_tables;
+  memcpy(src.call.rows, parts.rows, sizeof(src.call.rows));
+  memcpy(src.call.stride, parts.stride, sizeof(src.call.stride));
+  if (longest <= kPickMax || short_push_fits(longest, g->dim, g->elems, g->group)) {
+    // short members: see pick_runs and bucket_push_kernel
     SortCall sc = group_sort_call(gk, n_tables, offsets);
     // KRK_IDS_AS_PULLED: the rows of these very ids were noted by the combined pull before (and
     // nothing has moved since): the look-up launch is not needed. A note is a member's own row
@@ -2184,6 +2187,12 @@ static int32_t group_push_raw_enqueue(krk_group* g, const krk_optim* o, const in
     } else {
       sc.noted = 1;
     }
+    if (longest <= kPickMax) {
+      memcpy(src.call.ids, parts.ids, sizeof(src.call.ids));
+      for (int m = 0; m <= n_tables; ++m) src.call.row_start[m] = offsets[m];
+      return pick_runs(sh, g->stream, TableView{}, o->type, keys, miss_key, row_bits, sc.row_mask, nullptr, noted, total,
+                       longest, nullptr, args, PooledSrc{}, &gs, &src);
+    }
     if (g->vec == 4) {
       launch_bucket_push<4, true>(o->type, (unsigned)n_tables << sc.bucket_bits, g->stream, g->d_descs, TableView{}, sc,
                                   parts, keys, (int)g->dim, g->elems, g->group, args, gs);
@@ -2194,14 +2203,8 @@ static int32_t group_push_raw_enqueue(krk_group* g, const krk_optim* o, const in
     KRK_HIP(hipGetLastError());
     return KRK_SUCCESS;
   }
-  TableView none{};
-  const ReduceShape sh{g->dim, g->vec, g->elems, g->group};
-  GroupPooledSrc src{};                        // not pooled: a payload is a position of its member
-  src.call.n_tables = n_tables;
-  memcpy(src.call.rows, parts.rows, sizeof(src.call.rows));
-  memcpy(src.call.stride, parts.stride, sizeof(src.call.stride));
   const uint32_t* notes = noted_rows(g, parts.ids, offsets, flags);
-  return fill_and_reduce(sh, g->stream, g->scratch, none, o->type, total, miss_key, gk.bits, nullptr, args,
+  return fill_and_reduce(sh, g->stream, g->scratch, TableView{}, o->type, total, miss_key, gk.bits, nullptr, args,
                          PooledSrc{}, &gs, &src, NotedRows{}, [&](uint32_t* keys, uint32_t* pos) {
                            if (notes) {
                              hipLaunchKernelGGL(group_noted_keys_kernel, dim3(grid_for(total, kBlock)), dim3(kBlock), 0,
@@ -2244,11 +2247,17 @@ static int32_t push_pooled_enqueue(krk_sparse* t, const krk_optim* o, PooledCall
                          call.ids[0], n, miss_key, (const uint32_t*)bag_of, !weighted, keys, pos);
     }
   };
-  if (short_push_fits(n, t->dim, t->elems, t->group) && bags <= kBucketMaxBags) {
+  const PooledSrc src{true, call.mean_bits != 0, words, bag_of, call.weights[0], call.offsets[0]};
+  if (n <= kPickMax || (short_push_fits(n, t->dim, t->elems, t->group) && bags <= kBucketMaxBags)) {
     KRK_TRY(t->scratch[0].reserve((size_t)n * sizeof(uint32_t)));
     uint32_t* keys = t->scratch[0].as<uint32_t>();
     fill(keys, nullptr, kNoRow);
     const SortCall sc = table_sort_call(t, n);
+    if (n <= kPickMax) {
+      const ReduceShape sh{t->dim, t->vec, t->elems, t->group};
+      return pick_runs(sh, t->stream, tv, o->type, keys, sc.miss_key, sc.row_bits, sc.row_mask, nullptr, false, n, n,
+                       call.rows[0], table_apply_args(t, o, lr), src, nullptr, nullptr);
+    }
     GroupParts parts;
     parts.ids[0] = call.ids[0];
     parts.rows[0] = call.rows[0];
@@ -2271,8 +2280,7 @@ static int32_t push_pooled_enqueue(krk_sparse* t, const krk_optim* o, PooledCall
     KRK_HIP(hipGetLastError());
     return KRK_SUCCESS;
   }
-  return push_sorted(t, o, n, call.rows[0], lr,
-                     PooledSrc{true, call.mean_bits != 0, words, bag_of, call.weights[0], call.offsets[0]}, NotedRows{}, fill);
+  return push_sorted(t, o, n, call.rows[0], lr, src, NotedRows{}, fill);
 }
 
 extern "C" {
@@ -2479,11 +2487,23 @@ int32_t krk_group_push_pooled_parts(krk_group* g, const krk_optim* o, const krk_
                          keys, pos);
     }
   };
-  if (short_push_fits(longest, g->dim, g->elems, g->group) && most_bags <= kBucketMaxBags) {
+  GroupPooledSrc src;
+  src.call = call;
+  src.words = words;
+  src.bag_of = bag_of;
+  src.pooled = true;
+  src.weighted = weighted;
+  const ReduceShape sh{g->dim, g->vec, g->elems, g->group};
+  if (longest <= kPickMax || (short_push_fits(longest, g->dim, g->elems, g->group) && most_bags <= kBucketMaxBags)) {
     KRK_TRY(g->scratch[0].reserve((size_t)total * sizeof(uint32_t)));
     uint32_t* keys = g->scratch[0].as<uint32_t>();
     fill(keys, nullptr);
     const SortCall sc = group_sort_call(gk, n_tables, call.row_start);
+    if (longest <= kPickMax) {
+      KRK_TRY(pick_runs(sh, g->stream, TableView{}, o->type, keys, gk.miss_key, gk.row_bits, sc.row_mask, nullptr, false,
+                        total, longest, nullptr, args, PooledSrc{}, &gs, &src));
+      return group_finish(g, flags);
+    }
     BucketPooled pool;
     pool.bag_of = bag_of;
     pool.words = words;
@@ -2500,13 +2520,6 @@ int32_t krk_group_push_pooled_parts(krk_group* g, const krk_optim* o, const krk_
     KRK_HIP(hipGetLastError());
     return group_finish(g, flags);
   }
-  GroupPooledSrc src;
-  src.call = call;
-  src.words = words;
-  src.bag_of = bag_of;
-  src.pooled = true;
-  src.weighted = weighted;
-  const ReduceShape sh{g->dim, g->vec, g->elems, g->group};
   KRK_TRY(fill_and_reduce(sh, g->stream, g->scratch, TableView{}, o->type, total, gk.miss_key, gk.bits, nullptr, args,
                           PooledSrc{}, &gs, &src, NotedRows{}, fill));
   return group_finish(g, flags);

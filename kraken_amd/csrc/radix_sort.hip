@@ -111,12 +111,7 @@ __global__ __launch_bounds__(kScanLanes) void radix_scan_kernel(uint32_t* __rest
     uint32_t sum = 0;
 #pragma unroll
     for (int i = 0; i < kScanPer; ++i) sum += v[i];
-    uint32_t incl = sum;
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-      const uint32_t y = __shfl_up(incl, d);
-      if (lane >= d) incl += y;
-    }
+    const uint32_t incl = wave_inclusive_sum(sum);
     if (lane == kWave - 1) wave_total[wave] = incl;
     __syncthreads();
     uint32_t at = carry + incl - sum;
@@ -173,12 +168,7 @@ __global__ __launch_bounds__(kRsBlock) void radix_scatter_kernel(const uint32_t*
   for (int i = t; i < kRsWaves * kDigits; i += kRsBlock) wave_hist[i] = 0u;
   // an exclusive scan over the workgroup's first kDigits lanes (one value each), through wave_total
   auto scan_digits = [&](uint32_t v) -> uint32_t {
-    uint32_t incl = v;
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-      const uint32_t y = __shfl_up(incl, d);
-      if (lane >= d) incl += y;
-    }
+    const uint32_t incl = wave_inclusive_sum(v);
     if (lane == kWave - 1) wave_total[wave] = incl;
     __syncthreads();
     uint32_t offset = incl - v;

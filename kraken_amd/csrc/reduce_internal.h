@@ -347,4 +347,15 @@ int32_t reduce_runs(const ReduceShape& sh, hipStream_t stream, DeviceBuffer* scr
                     int64_t n, uint32_t miss_key, const NotedRows& noted, const float* vals, const ApplyArgs& args,
                     const PooledSrc& ps, const GroupSrc* gs, const GroupPooledSrc* gps);
 
+// Requests of at most this many ids a table need no partition: every bucket's workgroup picks its pairs out
+// of the member's keys.
+constexpr int64_t kPickMax = 2048;
+// keys: n rows (combined requests: members' numbers above their row_bits bits, or noted rows); payloads are
+// positions, or bags where bag_of says so (PooledSrc). noted: the keys are row notes (NotedRows, with
+// the ids of a single table; combined requests have theirs in gps). longest: ids of the longest member.
+int32_t pick_runs(const ReduceShape& sh, hipStream_t stream, const TableView& tv, int opt, const uint32_t* keys,
+                  uint32_t miss_key, int row_bits, uint32_t row_mask, const uint64_t* noted_ids, bool noted, int64_t n,
+                  int64_t longest, const float* vals, const ApplyArgs& args, const PooledSrc& ps, const GroupSrc* gs,
+                  const GroupPooledSrc* gps);
+
 }  // namespace krk

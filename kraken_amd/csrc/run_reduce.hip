@@ -234,11 +234,12 @@ struct Reducer {
   uint32_t bucket;
   int low;                       // bits of a key's place inside its bucket
   uint32_t low_mask;
+  uint32_t member_key;           // what the hash does not cover of a key: the workgroup's member
 
   // the key of entry j: row, and above it the member
   __device__ __forceinline__ uint32_t key_of(int j) const {
     const uint32_t h = (bucket << low) | (s.key[j] & low_mask);
-    return (h * a.hash.inverse) & a.hash.mask;
+    return ((h * a.hash.inverse) & a.hash.mask) | member_key;
   }
   __device__ __forceinline__ uint32_t row_of(uint32_t key) const {
     return GROUPED ? key & ((1u << row_bits) - 1u) : key;
@@ -759,7 +760,7 @@ __global__ __launch_bounds__(kLanes) void reduce_kernel(RunArgs a, TableView tv,
   }
   sort_list(s, len, low);
   const Reducer<OPT, VEC, FROM, GROUPED, false> r{
-      s, a, GROUPED ? lds_members : &one, args, weights, ps.words, weighted, gs.row_bits, cut.bucket, low, low_mask};
+      s, a, GROUPED ? lds_members : &one, args, weights, ps.words, weighted, gs.row_bits, cut.bucket, low, low_mask, 0u};
   const uint32_t runs = r.find_runs(len);
   if (is_cut) {
     // the list: the shortest runs as they are, one entry for any other
@@ -814,13 +815,126 @@ __global__ __launch_bounds__(kLanes) void reduce_kernel(RunArgs a, TableView tv,
   __syncthreads();
   if (!s.last) return;
   const Reducer<OPT, VEC, FROM, GROUPED, true> m{
-      s, a, GROUPED ? lds_members : &one, args, weights, ps.words, weighted, gs.row_bits, cut.bucket, low, low_mask};
+      s, a, GROUPED ? lds_members : &one, args, weights, ps.words, weighted, gs.row_bits, cut.bucket, low, low_mask, 0u};
   merge_lists<OPT, VEC, FROM, GROUPED>(m, a, cut, weights, bag_of);
 }
 
+// ---- requests of at most kPickMax ids a table: no partition ------------------------------------
+// One launch, a workgroup per (member, bucket), that reads the member's keys (at most eight a lane) and
+// keeps those of its bucket. What bounds it are latencies: the keys, then records and gradient rows,
+// and some 3 us of LDS phases, which is why the workgroup has four wavefronts: a barrier among
+// sixteen, of which a few dozen entries need one, is 0.2 us (bucket_push_kernel on 100 ids of 8
+// floats, keys 1.1, picking 2.1, sort 0.4, runs 1.8, updates 1.6 us).
+struct PickArgs {
+  const uint32_t* keys;          // rows, members' numbers above them, or noted rows
+  uint32_t miss_key, row_mask;
+  bool noted;                    // (kEmptyRow: look the id up, see NotedRows)
+  const uint64_t* ids;           // of a single table
+  int n;
+};
+
 template <int OPT, int VEC, int FROM, bool GROUPED>
-int32_t launch_reduce(const RunArgs& a, const TableView& tv, const ApplyArgs& args, const float* vals,
-                      const Source<GROUPED>& ps, const GroupSrc& gs, hipStream_t stream) {
+__global__ __launch_bounds__(kLanes) void pick_kernel(RunArgs a, PickArgs p, TableView tv, ApplyArgs args,
+                                                      const float* __restrict__ vals, Source<GROUPED> ps, GroupSrc gs) {
+  __shared__ RunLds s;
+  __shared__ Member lds_members[GROUPED ? kMaxGroupTables : 1];
+  __shared__ float weights[FROM == kBags ? kListMax : 1];
+  const int t = threadIdx.x;
+  const int lane = t & (kWave - 1);
+  const int wave = t / kWave;
+  const int low = a.hash.bits - a.hash.bucket_bits;
+  const uint32_t low_mask = (1u << low) - 1u;
+  const int m = GROUPED ? (int)(blockIdx.x >> a.hash.bucket_bits) : 0;
+  const uint32_t bucket = blockIdx.x & ((1u << a.hash.bucket_bits) - 1u);
+  int64_t first = 0;
+  int all = p.n;
+  const uint64_t* ids = p.ids;
+  bool weighted = false, positions = false;            // positions: payloads of this member are positions
+  const uint32_t* bag_of = nullptr;
+  if constexpr (GROUPED) {
+    first = ps.call.row_start[m];
+    all = (int)(ps.call.row_start[m + 1] - first);
+    ids = ps.call.ids[m];
+    tv = gs.descs[m].tv;
+    if constexpr (FROM == kBags) positions = weighted = ps.call.weights[m] != nullptr;
+  } else if constexpr (FROM == kBags) {
+    positions = weighted = ps.weight != nullptr;
+  }
+  if constexpr (FROM == kBags) bag_of = ps.bag_of;
+  if (all <= 0) return;                                // uniform for the workgroup
+  // item i of lane l in wavefront w is position (w * own + i) * 64 + l: taking i in ascending order visits
+  // a wavefront's positions in order
+  const int own = (all + kLanes - 1) / kLanes;         // 1..kListItems
+  const int base = wave * own * kWave + lane;
+  uint32_t key[kListItems], ref[kListItems];
+#pragma unroll
+  for (int i = 0; i < kListItems; ++i) {
+    const int j = base + i * kWave;
+    key[i] = i < own && j < all ? p.keys[first + j] : 0xFFFFFFFFu;
+    ref[i] = (uint32_t)j;
+    if constexpr (FROM == kBags) {
+      if (!positions && i < own && j < all) ref[i] = bag_of[first + j];
+    }
+  }
+  Member one;
+  load_members<GROUPED>(GROUPED ? lds_members : &one, a, tv, args, vals, ps, gs);
+  if (p.noted) {
+#pragma unroll
+    for (int i = 0; i < kListItems; ++i) {
+      const int j = base + i * kWave;
+      if (i < own && j < all && key[i] == kEmptyRow) key[i] = probe_find_alone(tv, ids[j]);
+    }
+  }
+  // the bucket's positions, in order
+  unsigned long long take[kListItems];
+  uint32_t mine = 0;
+#pragma unroll
+  for (int i = 0; i < kListItems; ++i) {
+    const bool live = i < own && key[i] < p.miss_key;
+    key[i] = ((key[i] & p.row_mask) * a.hash.mult) & a.hash.mask;
+    take[i] = __ballot(live && key[i] >> low == bucket);
+    mine += (uint32_t)__popcll(take[i]);
+  }
+  if (lane == 0) s.wave_total[wave] = mine;
+  lds_barrier();
+  uint32_t at = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    const uint32_t x = s.wave_total[w];
+    if (w < wave) at += x;
+    total += x;
+  }
+  const int len = (int)total;
+  if (len == 0) return;                                // uniform
+#pragma unroll
+  for (int i = 0; i < kListItems; ++i) {
+    if (take[i] & (1ull << lane)) {
+      const uint32_t to = at + (uint32_t)__popcll(take[i] & ((1ull << lane) - 1ull));
+      s.key[to] = key[i] & low_mask;
+      s.ref[to] = ref[i];
+    }
+    at += (uint32_t)__popcll(take[i]);
+  }
+  sort_list(s, len, low);
+  const Reducer<OPT, VEC, FROM, GROUPED, false> r{
+      s, a, GROUPED ? lds_members : &one, args, weights, ps.words, weighted, gs.row_bits, bucket, low, low_mask,
+      GROUPED ? (uint32_t)m << gs.row_bits : 0u};
+  const uint32_t runs = r.find_runs(len);
+  r.resolve_weights(len, weights, bag_of);
+  r.reduce(runs, false, 0u);
+}
+
+template <int OPT, int VEC, int FROM, bool GROUPED>
+int32_t launch_reduce(const RunArgs& a, const PickArgs* pick, const TableView& tv, const ApplyArgs& args,
+                      const float* vals, const Source<GROUPED>& ps, const GroupSrc& gs, hipStream_t stream) {
+  if (pick) {
+    unsigned members = 1;
+    if constexpr (GROUPED) members = (unsigned)ps.call.n_tables;
+    hipLaunchKernelGGL((pick_kernel<OPT, VEC, FROM, GROUPED>), dim3(members << a.hash.bucket_bits), dim3(kLanes), 0,
+                       stream, a, *pick, tv, args, vals, ps, gs);
+    KRK_HIP(hipGetLastError());
+    return KRK_SUCCESS;
+  }
   hipLaunchKernelGGL((reduce_kernel<OPT, VEC, FROM, GROUPED>), dim3(a.max_chunks + (1u << a.hash.bucket_bits)),
                      dim3(kLanes), 0, stream, a, tv, args, vals, ps, gs);
   KRK_HIP(hipGetLastError());
@@ -828,28 +942,28 @@ int32_t launch_reduce(const RunArgs& a, const TableView& tv, const ApplyArgs& ar
 }
 
 template <int OPT, int VEC>
-int32_t launch_source(const RunArgs& a, const TableView& tv, const ApplyArgs& args, const float* vals,
+int32_t launch_source(const RunArgs& a, const PickArgs* pick, const TableView& tv, const ApplyArgs& args, const float* vals,
                       const PooledSrc& ps, const GroupSrc* gs, const GroupPooledSrc* gps, hipStream_t stream) {
   const GroupSrc plain{nullptr, 0, -1, -1, -1, 0};
   if constexpr (OPT != kOptStore) {
     if (gs) {
-      return gps->pooled ? launch_reduce<OPT, VEC, kBags, true>(a, tv, args, vals, *gps, *gs, stream)
-                         : launch_reduce<OPT, VEC, kRows, true>(a, tv, args, vals, *gps, *gs, stream);
+      return gps->pooled ? launch_reduce<OPT, VEC, kBags, true>(a, pick, tv, args, vals, *gps, *gs, stream)
+                         : launch_reduce<OPT, VEC, kRows, true>(a, pick, tv, args, vals, *gps, *gs, stream);
     }
-    if (ps.pooled) return launch_reduce<OPT, VEC, kBags, false>(a, tv, args, vals, ps, plain, stream);
+    if (ps.pooled) return launch_reduce<OPT, VEC, kBags, false>(a, pick, tv, args, vals, ps, plain, stream);
   }
-  return launch_reduce<OPT, VEC, kRows, false>(a, tv, args, vals, ps, plain, stream);
+  return launch_reduce<OPT, VEC, kRows, false>(a, pick, tv, args, vals, ps, plain, stream);
 }
 
 template <int VEC>
-int32_t launch_opt(int opt, const RunArgs& a, const TableView& tv, const ApplyArgs& args, const float* vals,
+int32_t launch_opt(int opt, const RunArgs& a, const PickArgs* pick, const TableView& tv, const ApplyArgs& args, const float* vals,
                    const PooledSrc& ps, const GroupSrc* gs, const GroupPooledSrc* gps, hipStream_t stream) {
   switch (opt) {
-    case kOptStore: return launch_source<kOptStore, VEC>(a, tv, args, vals, ps, gs, gps, stream);
-    case KRK_SGD: return launch_source<KRK_SGD, VEC>(a, tv, args, vals, ps, gs, gps, stream);
-    case KRK_ADAGRAD: return launch_source<KRK_ADAGRAD, VEC>(a, tv, args, vals, ps, gs, gps, stream);
-    case KRK_ADAM: return launch_source<KRK_ADAM, VEC>(a, tv, args, vals, ps, gs, gps, stream);
-    default: return launch_source<KRK_RMSPROP, VEC>(a, tv, args, vals, ps, gs, gps, stream);
+    case kOptStore: return launch_source<kOptStore, VEC>(a, pick, tv, args, vals, ps, gs, gps, stream);
+    case KRK_SGD: return launch_source<KRK_SGD, VEC>(a, pick, tv, args, vals, ps, gs, gps, stream);
+    case KRK_ADAGRAD: return launch_source<KRK_ADAGRAD, VEC>(a, pick, tv, args, vals, ps, gs, gps, stream);
+    case KRK_ADAM: return launch_source<KRK_ADAM, VEC>(a, pick, tv, args, vals, ps, gs, gps, stream);
+    default: return launch_source<KRK_RMSPROP, VEC>(a, pick, tv, args, vals, ps, gs, gps, stream);
   }
 }
 
@@ -865,6 +979,19 @@ int bucket_bits_for(int64_t n) {
 // 2048 pairs, us: 50,000 ids of 100 floats 39 / 49 / 69, 300,000 of 32 38 / 38 / 47, a million of 16
 // 107 / 74 / 76, of 128 (Zipf 1.3) 186 / 150 / 170.
 int chunk_for(int64_t n) { return n > ((int64_t)1 << 18) ? kListMax / 2 : kListMax / 4; }
+
+// Places of keys below `keys`.
+RunHash make_hash(int bucket_bits, uint64_t keys) {
+  RunHash h;
+  h.bucket_bits = bucket_bits;
+  h.bits = bucket_bits + 1;
+  while (h.bits < 32 && ((uint64_t)1 << h.bits) < keys) ++h.bits;
+  h.mask = h.bits >= 32 ? 0xFFFFFFFFu : (1u << h.bits) - 1u;
+  h.mult = 0x9E3779B1u;
+  h.inverse = h.mult;                                  // Newton's iteration: right to 3, 6, 12, 24, 48 bits
+  for (int i = 0; i < 4; ++i) h.inverse *= 2u - h.mult * h.inverse;
+  return h;
+}
 
 // Buckets and chunks of a request, and where its work space lies.
 struct RunShape {
@@ -894,14 +1021,7 @@ int32_t reduce_runs(const ReduceShape& sh, hipStream_t stream, DeviceBuffer* scr
                     const PooledSrc& ps, const GroupSrc* gs, const GroupPooledSrc* gps) {
   const RunShape shape(n);
   RunArgs a{};
-  a.hash.bucket_bits = shape.bucket_bits;
-  a.hash.bits = a.hash.bucket_bits + 1;
-  while (a.hash.bits < 32 && ((uint64_t)1 << a.hash.bits) < miss_key) ++a.hash.bits;
-  a.hash.mask = a.hash.bits >= 32 ? 0xFFFFFFFFu : (1u << a.hash.bits) - 1u;
-  a.hash.mult = 0x9E3779B1u;
-  uint32_t inverse = a.hash.mult;                      // Newton's iteration: right to 3, 6, 12, 24, 48 bits
-  for (int i = 0; i < 4; ++i) inverse *= 2u - a.hash.mult * inverse;
-  a.hash.inverse = inverse;
+  a.hash = make_hash(shape.bucket_bits, miss_key);
   a.chunk = shape.chunk;
   a.max_chunks = (uint32_t)shape.chunks;
   a.dim = (int)sh.dim;
@@ -926,8 +1046,27 @@ int32_t reduce_runs(const ReduceShape& sh, hipStream_t stream, DeviceBuffer* scr
   a.refs = h + n;
   a.list_h = pairs;                                    // the partition's input has been read
   a.list_refs = pairs + n;
-  if (sh.vec == 4) return launch_opt<4>(opt, a, tv, args, vals, ps, gs, gps, stream);
-  return launch_opt<1>(opt, a, tv, args, vals, ps, gs, gps, stream);
+  if (sh.vec == 4) return launch_opt<4>(opt, a, nullptr, tv, args, vals, ps, gs, gps, stream);
+  return launch_opt<1>(opt, a, nullptr, tv, args, vals, ps, gs, gps, stream);
+}
+
+int32_t pick_runs(const ReduceShape& sh, hipStream_t stream, const TableView& tv, int opt, const uint32_t* keys,
+                  uint32_t miss_key, int row_bits, uint32_t row_mask, const uint64_t* noted_ids, bool noted, int64_t n,
+                  int64_t longest, const float* vals, const ApplyArgs& args, const PooledSrc& ps, const GroupSrc* gs,
+                  const GroupPooledSrc* gps) {
+  const int members = gps ? gps->call.n_tables : 1;
+  // sixteen pairs a bucket, as long as that is two workgroups a compute unit at most (8 and 32 pairs, and
+  // twice the workgroups, are within 5 % of it)
+  int bits = 3;
+  while (bits < 8 && ((int64_t)16 << bits) < longest && (members << (bits + 1)) <= 512) ++bits;
+  RunArgs a{};
+  a.hash = make_hash(bits, (uint64_t)1 << row_bits);
+  a.dim = (int)sh.dim;
+  a.elems = sh.elems;
+  a.group = sh.group;
+  const PickArgs pick{keys, miss_key, row_mask, noted, noted_ids, (int)n};
+  if (sh.vec == 4) return launch_opt<4>(opt, a, &pick, tv, args, vals, ps, gs, gps, stream);
+  return launch_opt<1>(opt, a, &pick, tv, args, vals, ps, gs, gps, stream);
 }
 
 }  // namespace krk

@@ -186,12 +186,7 @@ __device__ inline int block_exclusive_scan(int v, int* lds, int& block_total) {
   // wave-level inclusive scan, then combine the wave totals through LDS
   int lane = threadIdx.x & 63;
   int wave = threadIdx.x >> 6;
-  int x = v;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    int y = __shfl_up(x, d, 64);
-    if (lane >= d) x += y;
-  }
+  const int x = (int)wave_inclusive_sum((uint32_t)v);
   if (lane == 63) lds[wave] = x;
   __syncthreads();
   int base = 0;

@@ -1,4 +1,4 @@
-"""Pushes of more than 12288 ids and krk_dedup_sum up to 2^20 ids: pairs grouped by bucket, every bucket
+"""Pushes of up to 2048 and of more than 12288 ids and krk_dedup_sum up to 2^20 ids: pairs grouped by bucket, every bucket
 sorted and added up by one workgroup, buckets that hold more pairs than a workgroup takes cut into
 chunks and merged. Gradients lie on a binary grid, so that every order of additions gives the same
 bits: sums are compared exactly.
@@ -76,6 +76,33 @@ def test_dedup_sum_crowded_bucket(api, n, dim):
     u, inv, sums = api.dedup_sum(splitmix64(keys.astype(np.uint64)), grads)
     assert np.array_equal(inv, keys)
     assert np.array_equal(sums, _sums(keys, grads, u.size))
+
+
+# up to 2048 ids a table every bucket's workgroup picks its pairs out of the request, one to eight a lane; a
+# list of up to 256 pairs is sorted by counting
+@pytest.mark.parametrize("n", [1, 64, 255, 256, 257, 513, 2047, 2048, 2049])
+@pytest.mark.parametrize("dim", [5, 16, 300])
+def test_short_requests(api, n, dim):
+    rng = np.random.default_rng(n + dim)
+    sgd = api.Optim.create(api.OptimType.kSGD)
+    tables = [api.SparseTable(dim, api.Initializer.create(api.InitializerType.kConstant, {"value": "1"})) for _ in range(3)]
+    group = api.TableGroup(tables[1:])
+    for ids in (np.full(n, 3, np.uint64), splitmix64(np.arange(n, dtype=np.uint64)), zipf_ids(rng, 1.3, 5000, n)):
+        grads = _grid(rng, (n, dim))
+        u, inv = np.unique(ids, return_inverse=True)
+        want = np.float32(0.5) * _sums(inv, grads, u.size)
+        before = tables[0].Pull(u)[1]
+        assert tables[0].PushRaw(sgd, ids, grads, 0.5) == 0
+        assert np.array_equal(tables[0].Pull(u)[1], before - want)
+        offsets = group._offsets([n // 2, n - n // 2])
+        group.CombinePull(ids, offsets)
+        before = [t.Pull(u)[1] for t in tables[1:]]
+        assert group.CombinePushRaw(sgd, ids, offsets, grads, 0.5) == 0
+        for t, b, part in zip(tables[1:], before, (slice(0, n // 2), slice(n // 2, n))):
+            assert np.array_equal(t.Pull(u)[1], b - np.float32(0.5) * _sums(inv[part], grads[part], u.size))
+        got = api.dedup_sum(ids, grads)
+        assert np.array_equal(got[2][np.argsort(got[0])], _sums(inv, grads, u.size))
+    group.close()
 
 
 @pytest.mark.parametrize("dim", [4, 6, 260])
