@@ -392,7 +392,8 @@ struct krk_sparse : krk::ObjBase {
   unsigned long long* host_pub = nullptr;   // pinned, written by the device (publish_kernel)
   uint32_t pub_epoch = 0;                   // launch number of the last publish that was enqueued
   uint32_t* host_inserted = nullptr;        // pinned, behind host_pub: set by pulls that insert
-  int64_t last_request = 0;           // size of the last inserting request
+  int64_t last_request = 0;           // size of the latest large inserting requests
+  int64_t pub_rows = 0;               // rows at the last published count that was looked at
   uint64_t enq_total = 0;             // ids handed to inserting launches so far
   uint64_t enq_at[256] = {};          // enq_total right after the launch with number e (mod 256)
   uint32_t epoch = 0;                 // number of the last launch that could insert
@@ -579,7 +580,7 @@ int32_t sparse_finish_end(krk_sparse* t, uint32_t flags);
 // A new launch number for a launch that may insert up to n rows into t; call right before it.
 int32_t sparse_next_epoch(krk_sparse* t, int64_t n);
 // True when only a few more requests like the last one fit under the current row bound.
-bool sparse_near_full(const krk_sparse* t);
+bool sparse_wants_publish(const krk_sparse* t);
 // Enqueues the kernel that publishes {rows used, launch number} of each table to the host.
 int32_t sparse_publish(krk_sparse* const* tables, int n, hipStream_t stream);
 // Host ids -> each row's stored 64-bit word (counter and momentum flag), blocking.

@@ -1589,7 +1589,7 @@ static int32_t enqueue_counters(krk_sparse* const* tables, int n, hipStream_t st
 static int32_t refresh_rows(krk_sparse* t) {
   KRK_TRY(enqueue_counters(&t, 1, t->stream));
   KRK_HIP(hipStreamSynchronize(t->stream));
-  t->size_ub = t->host_counters[0];
+  t->size_ub = t->pub_rows = t->host_counters[0];
   return KRK_SUCCESS;
 }
 
@@ -1650,13 +1650,19 @@ static uint64_t pow2_at_least(uint64_t x) {
   return c;
 }
 
+// Rows a table has room for beyond its bound.
+static int64_t room_left(const krk_sparse* t) {
+  return std::min<int64_t>(t->row_cap, (int64_t)(t->slot_cap / 2)) - t->size_ub;
+}
+
 // Lowers the row bound with the count the device published last: exact as of that launch,
 // plus everything enqueued after it.
 static void tighten_bound(krk_sparse* t) {
   const unsigned long long pub = __atomic_load_n(t->host_pub, __ATOMIC_ACQUIRE);
   const uint32_t ep = (uint32_t)(pub >> 32);
   if (ep == 0 || ep > t->epoch || t->epoch - ep >= 256) return;
-  const int64_t cand = (int64_t)(uint32_t)pub + (int64_t)(t->enq_total - t->enq_at[ep & 255]);
+  t->pub_rows = (int64_t)(uint32_t)pub;
+  const int64_t cand = t->pub_rows + (int64_t)(t->enq_total - t->enq_at[ep & 255]);
   if (cand < t->size_ub) t->size_ub = cand;
 }
 
@@ -1664,14 +1670,14 @@ static void tighten_bound(krk_sparse* t) {
 // push behind it is still running, and waiting for the whole stream would leave the GPU idle until
 // the next request is there (8.5 million pooled ids over 4 million rows, forward, backward and
 // forward: 1455 us with two waits of that kind). Returns when the bound allows `need_for` more rows,
-// the count of the last request has arrived, or the stream has nothing left to run.
+// the last count that was to be published has arrived, or the stream has nothing left to run.
 static void await_published(krk_sparse* t, int64_t extra_rows) {
-  if (t->pub_epoch != t->epoch || t->epoch == 0) return;
+  if (t->pub_epoch == 0) return;
   for (;;) {
     tighten_bound(t);
     const int64_t need = t->size_ub + extra_rows;
     if (need <= t->row_cap && (uint64_t)need * 2 <= t->slot_cap) break;
-    if ((uint32_t)(__atomic_load_n(t->host_pub, __ATOMIC_ACQUIRE) >> 32) == t->epoch) break;
+    if ((uint32_t)(__atomic_load_n(t->host_pub, __ATOMIC_ACQUIRE) >> 32) == t->pub_epoch) break;
     if (hipStreamQuery(t->stream) != hipErrorNotReady) break;
     std::this_thread::yield();
   }
@@ -1680,6 +1686,7 @@ static void await_published(krk_sparse* t, int64_t extra_rows) {
 
 // Room for `extra_rows` more rows: records, row keys, and an index at most half full.
 int32_t sparse_ensure_room(krk_sparse* t, int64_t extra_rows) {
+  if (room_left(t) < 2 * t->last_request) tighten_bound(t);
   int64_t need = t->size_ub + extra_rows;
   if (need > t->row_cap || (uint64_t)need * 2 > t->slot_cap) {
     await_published(t, extra_rows);
@@ -1718,13 +1725,22 @@ int32_t sparse_next_epoch(krk_sparse* t, int64_t n) {
   t->enq_total += (uint64_t)n;
   t->enq_at[t->epoch & 255] = t->enq_total;
   t->size_ub += n;
-  t->last_request = n;
+  t->last_request = std::max(n, t->last_request / 2);
   return KRK_SUCCESS;
 }
 
-bool sparse_near_full(const krk_sparse* t) {
-  const int64_t room = std::min<int64_t>(t->row_cap, (int64_t)(t->slot_cap / 2)) - t->size_ub;
-  return room < 4 * t->last_request;
+// Whether the pull that has just been enqueued should publish its count: where the bound leaves less than
+// two requests (of the size of the latest large ones), unless the count that is on its way already,
+// when it has arrived, leaves that much. A table that is nearly full, as a trained one is, published in
+// every pull, a launch of 2-5 us on the device and 3 us of the host; with room for five more
+// requests one pull in four does. (Rows that were made since the last count are not in the estimate:
+// then the bound is refreshed by waiting, once.)
+bool sparse_wants_publish(const krk_sparse* t) {
+  const int64_t room = room_left(t);
+  if (room >= 2 * t->last_request) return false;
+  if (t->pub_epoch == 0 || t->epoch - t->pub_epoch >= 256) return true;
+  const int64_t since = (int64_t)(t->enq_total - t->enq_at[t->pub_epoch & 255]);
+  return t->pub_rows + since + 2 * t->last_request > room + t->size_ub;
 }
 
 int32_t sparse_publish(krk_sparse* const* tables, int n, hipStream_t stream) {
@@ -2155,7 +2171,7 @@ int32_t krk_sparse_pull(krk_sparse* t, const uint64_t* ids, int64_t n, float* ou
     t->noted_n = n;
     t->noted_version = t->layout_version;
   }
-  if ((flags & KRK_ASYNC) && sparse_near_full(t)) KRK_TRY(sparse_publish(&t, 1, t->stream));
+  if ((flags & KRK_ASYNC) && sparse_wants_publish(t)) KRK_TRY(sparse_publish(&t, 1, t->stream));
   KRK_TRY(sparse_finish_begin(t, flags));
   KRK_TRY(t->output_back(out, (size_t)n * t->dim, flags, 1));
   return sparse_finish_end(t, flags);
@@ -2250,7 +2266,7 @@ int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, co
     t->noted_n = n;
     t->noted_version = t->layout_version;
   }
-  if ((flags & KRK_ASYNC) && sparse_near_full(t)) KRK_TRY(sparse_publish(&t, 1, t->stream));
+  if ((flags & KRK_ASYNC) && sparse_wants_publish(t)) KRK_TRY(sparse_publish(&t, 1, t->stream));
   KRK_TRY(sparse_finish_begin(t, flags));
   KRK_TRY(t->output_back(out, (size_t)bags * t->dim, flags, 3));
   return sparse_finish_end(t, flags);
@@ -2437,7 +2453,7 @@ int32_t krk_sparse_import(krk_sparse* t, const uint64_t* ids, int64_t n, const f
                        (int)t->dim, t->elems, t->group);
   }
   KRK_HIP(hipGetLastError());
-  if ((flags & KRK_ASYNC) && sparse_near_full(t)) KRK_TRY(sparse_publish(&t, 1, t->stream));
+  if ((flags & KRK_ASYNC) && sparse_wants_publish(t)) KRK_TRY(sparse_publish(&t, 1, t->stream));
   return sparse_finish(t, flags);
 }
 
@@ -3141,7 +3157,7 @@ static int32_t group_pull_enqueue(krk_group* g, const int64_t* offsets, GroupCal
   }
   if (flags & KRK_ASYNC) {
     bool any = false;
-    for (krk_sparse* t : g->tables) any = any || sparse_near_full(t);
+    for (krk_sparse* t : g->tables) any = any || sparse_wants_publish(t);
     if (any) KRK_TRY(sparse_publish(g->tables.data(), (int)g->tables.size(), g->stream));
   }
   return KRK_SUCCESS;
@@ -3383,7 +3399,7 @@ int32_t krk_group_pull_pooled_parts(krk_group* g, const krk_pooled_part* in, uin
   }
   if (flags & KRK_ASYNC) {
     bool any = false;
-    for (krk_sparse* t : g->tables) any = any || sparse_near_full(t);
+    for (krk_sparse* t : g->tables) any = any || sparse_wants_publish(t);
     if (any) KRK_TRY(sparse_publish(g->tables.data(), (int)g->tables.size(), g->stream));
   }
   return group_finish(g, flags);
