@@ -11,11 +11,11 @@
 // Shape of the work: Y[M, N] = X[M, K] * Basis[K, N] with M = n / 256 blocks (forward: K = 256,
 // N = keep; inverse: K = keep, N = 256), (1) folded in half by the basis' mirror symmetry and
 // (2) multiplied as six bf16 products per fp32 product on v_mfma_f32_32x32x16_bf16, both below.
-// A workgroup keeps its basis tile resident in LDS and walks over row tiles of 256 blocks (128 for
-// short requests); each of its wavefronts owns 32 rows and holds their X values in registers.
+// A workgroup keeps its basis tile resident in LDS and walks over row tiles of 256 blocks; each of its
+// wavefronts owns 32 rows and holds their X values in registers. Requests of few blocks have a
+// kernel of their own (dct2_few_kernel).
 #include <cmath>
 #include <mutex>
-#include <type_traits>
 
 #include "krk_internal.h"
 
@@ -23,6 +23,10 @@ namespace krk {
 
 constexpr int kDctB = 256;      // block length
 constexpr int kWaveRows = 32;   // rows (blocks) of an output tile per wavefront
+// Wavefronts of a workgroup, a row tile of 256 blocks: a workgroup more or less a compute unit
+// owns one whatever the width (the basis fills up to 98 KB of its LDS), and sixteen are no faster
+// (262,144 blocks 154 / 152 us at keep 64, 305 / 304 at keep 256).
+constexpr int kWaves = 8;
 
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -177,14 +181,56 @@ __global__ void dct2_basis3_kernel(__bf16* __restrict__ fwd3, __bf16* __restrict
   }
 }
 
-template <int NT, bool FWD, int WAVES>
-__global__ __launch_bounds__(WAVES * kWave) void dct2_split_kernel(const float* __restrict__ X, int64_t ldx,
+// A slice of a lane's row, E folded indices: V = E / 2 float4, forward the values and then their mirror
+// images, inverse even and odd coefficients interleaved -> the two operands of every pair, in pieces.
+template <bool FWD, int E>
+__device__ __forceinline__ void fold_slice(const float4 (&cur)[E / 2], Split3 (&piece)[E / 8][2]) {
+  float v[2 * E];
+#pragma unroll
+  for (int q = 0; q < E / 2; ++q) {
+    v[4 * q] = cur[q].x;
+    v[4 * q + 1] = cur[q].y;
+    v[4 * q + 2] = cur[q].z;
+    v[4 * q + 3] = cur[q].w;
+  }
+  float one[E], two[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    one[e] = FWD ? v[e] + v[2 * E - 1 - e] : v[2 * e];
+    two[e] = FWD ? v[e] - v[2 * E - 1 - e] : v[2 * e + 1];
+  }
+#pragma unroll
+  for (int g = 0; g < E / 8; ++g) {
+    float x8[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x8[e] = one[8 * g + e];
+    piece[g][0] = split3(x8);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x8[e] = two[8 * g + e];
+    piece[g][1] = split3(x8);
+  }
+}
+
+// acc += a * b in six products, the small pieces first; u: the basis' pieces.
+__device__ __forceinline__ void multiply(v16f& acc, const Split3& a, const uint4& u0, const uint4& u1, const uint4& u2) {
+  const bf16x8 b0 = __builtin_bit_cast(bf16x8, u0), b1 = __builtin_bit_cast(bf16x8, u1),
+               b2 = __builtin_bit_cast(bf16x8, u2);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p2, b0, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p0, b2, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p1, b1, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p1, b0, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p0, b1, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p0, b0, acc, 0, 0, 0);
+}
+
+template <int NT, bool FWD>
+__global__ __launch_bounds__(kWaves * kWave) void dct2_split_kernel(const float* __restrict__ X, int64_t ldx,
                                                               const __bf16* __restrict__ B3,
                                                               float* __restrict__ Y, int64_t ldy,
                                                               int64_t M, int KF) {
   constexpr int NT2 = 2 * NT;
-  constexpr int kThreads = WAVES * kWave;
-  constexpr int kTileM = WAVES * kWaveRows;
+  constexpr int kThreads = kWaves * kWave;
+  constexpr int kTileM = kWaves * kWaveRows;
   // Folded indices a lane holds per slice: one group of 8, or two where the accumulators leave
   // the registers for it (a row's loads are then whole 64-byte pieces, which memory serves
   // better; the narrow tiles are the ones that wait for memory). Either way the groups are taken
@@ -253,32 +299,8 @@ __global__ __launch_bounds__(WAVES * kWave) void dct2_split_kernel(const float* 
     for (int t = 0; t < NT2; ++t) acc[t] = v16f{0};
 #pragma unroll 1
     for (int s = 0; s < slices; ++s) {
-      float v[2 * E];
-#pragma unroll
-      for (int q = 0; q < V; ++q) {
-        v[4 * q] = cur[q].x;
-        v[4 * q + 1] = cur[q].y;
-        v[4 * q + 2] = cur[q].z;
-        v[4 * q + 3] = cur[q].w;
-      }
-      // forward: the values, then their mirror images; inverse: even and odd coefficients interleaved
-      float one[E], two[E];
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        one[e] = FWD ? v[e] + v[2 * E - 1 - e] : v[2 * e];
-        two[e] = FWD ? v[e] - v[2 * E - 1 - e] : v[2 * e + 1];
-      }
       Split3 piece[E / 8][2];
-#pragma unroll
-      for (int g = 0; g < E / 8; ++g) {
-        float x8[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x8[e] = one[8 * g + e];
-        piece[g][0] = split3(x8);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x8[e] = two[8 * g + e];
-        piece[g][1] = split3(x8);
-      }
+      fold_slice<FWD, E>(cur, piece);
       // the slice's values are used up: the next slice's take their registers
       if (s + 1 < slices) {
         load_slice(tile, lrow, s + 1, cur);
@@ -292,20 +314,10 @@ __global__ __launch_bounds__(WAVES * kWave) void dct2_split_kernel(const float* 
         const uint4* bg = bl + (size_t)((first(s) + 8 * g + kHalf * h) >> 3) * (3 * NT2 * 32);
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
-          const Split3& a = piece[g][half];
 #pragma unroll
           for (int tt = 0; tt < NT; ++tt) {
             const int t = half * NT + tt;
-            const uint4 u0 = bg[(0 * NT2 + t) * 32], u1 = bg[(1 * NT2 + t) * 32], u2 = bg[(2 * NT2 + t) * 32];
-            const bf16x8 b0 = __builtin_bit_cast(bf16x8, u0), b1 = __builtin_bit_cast(bf16x8, u1),
-                         b2 = __builtin_bit_cast(bf16x8, u2);
-            // the small pieces first
-            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p2, b0, acc[t], 0, 0, 0);
-            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p0, b2, acc[t], 0, 0, 0);
-            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p1, b1, acc[t], 0, 0, 0);
-            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p1, b0, acc[t], 0, 0, 0);
-            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p0, b1, acc[t], 0, 0, 0);
-            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p0, b0, acc[t], 0, 0, 0);
+            multiply(acc[t], piece[g][half], bg[(0 * NT2 + t) * 32], bg[(1 * NT2 + t) * 32], bg[(2 * NT2 + t) * 32]);
           }
         }
       }
@@ -315,6 +327,76 @@ __global__ __launch_bounds__(WAVES * kWave) void dct2_split_kernel(const float* 
       store_tile<NT, FWD>(acc, Y + row0 * ldy, (int)ldy, M - row0, h, c0 + NT * r);
     }
   }
+}
+
+// The same for requests of few blocks: one wavefront a workgroup, 32 blocks by 32 folded columns, the basis
+// read where it is used. Nothing is read twice there, so laying the basis out in LDS first, by a
+// workgroup that then multiplies once, is only a longer way (100 blocks, keep 256: 12 us a
+// transform, two workgroups busy, against 6-7). The products are added in the other kernel's order.
+template <bool FWD>
+__global__ __launch_bounds__(kWave) void dct2_few_kernel(const float* __restrict__ X, int64_t ldx,
+                                                         const __bf16* __restrict__ B3, float* __restrict__ Y,
+                                                         int64_t ldy, int64_t M, int KF) {
+  constexpr int E = FWD ? 16 : 8, kSliceK = 2 * E, kHalf = FWD ? 16 : 8;
+  const int r = threadIdx.x & 31;
+  const int h = threadIdx.x >> 5;
+  const int cl = blockIdx.y * 32 + r;
+  const int64_t row0 = (int64_t)blockIdx.x * kWaveRows;
+  const float* x = X + (row0 + r < M ? row0 + r : M - 1) * ldx;
+  const uint4* src = reinterpret_cast<const uint4*>(B3);
+  auto load_x = [&](int s, float4 (&v)[E / 2]) {
+    const int at = kSliceK * s;
+#pragma unroll
+    for (int q = 0; q < E / 2; ++q) {
+      if (FWD) {
+        const int j = q < E / 4 ? at + kHalf * h + 4 * q : kDctB - E - at - kHalf * h + 4 * (q - E / 4);
+        v[q] = *reinterpret_cast<const float4*>(x + j);
+      } else {
+        v[q] = *reinterpret_cast<const float4*>(x + 2 * at + 2 * kHalf * h + 4 * q);
+      }
+    }
+  };
+  auto load_b = [&](int s, uint4 (&u)[E / 8][2][3]) {
+#pragma unroll
+    for (int g = 0; g < E / 8; ++g) {
+      const int group = (kSliceK * s + 8 * g + kHalf * h) >> 3;
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+          u[g][half][p] = FWD ? src[(group * 3 + p) * kDctB + 2 * cl + half]
+                              : src[((half * 16 + group) * 3 + p) * kFoldB + cl];
+      }
+    }
+  };
+  const int slices = KF / kSliceK;
+  float4 cur[E / 2];
+  uint4 basis[E / 8][2][3];
+  load_x(0, cur);
+  load_b(0, basis);
+  v16f acc[2] = {v16f{0}, v16f{0}};
+#pragma unroll 1
+  for (int s = 0; s < slices; ++s) {
+    Split3 piece[E / 8][2];
+    fold_slice<FWD, E>(cur, piece);
+    uint4 now[E / 8][2][3];
+#pragma unroll
+    for (int g = 0; g < E / 8; ++g)
+#pragma unroll
+      for (int half = 0; half < 2; ++half)
+#pragma unroll
+        for (int p = 0; p < 3; ++p) now[g][half][p] = basis[g][half][p];
+    if (s + 1 < slices) {
+      load_x(s + 1, cur);
+      load_b(s + 1, basis);
+    }
+#pragma unroll
+    for (int g = 0; g < E / 8; ++g)
+#pragma unroll
+      for (int half = 0; half < 2; ++half)
+        multiply(acc[half], piece[g][half], now[g][half][0], now[g][half][1], now[g][half][2]);
+  }
+  store_tile<1, FWD>(acc, Y + row0 * ldy, (int)ldy, M - row0, h, cl);
 }
 
 static std::mutex g_basis_mu;
@@ -336,15 +418,12 @@ static int32_t ensure_basis(hipStream_t s) {
   return KRK_SUCCESS;
 }
 
-// Wavefronts of a workgroup. Eight, a row tile of 256 blocks: a workgroup more or less a compute unit
-// owns one whatever the width (the basis fills up to 98 KB of its LDS), and with sixteen a
-// request of a few thousand blocks kept only a few units busy while the largest was no faster
-// (forward + inverse as blocking calls, sixteen / eight, us: 10,000 blocks keep 64 57 / 42, keep 256
-// 73 / 51; 100,000 blocks 88 / 81 and 147 / 145; 262,144 blocks 154 / 152 and 305 / 304, no
-// difference beyond that between two runs of one side). Four for requests so small that tiles of
-// 128 blocks still leave units idle (eight / four: 4000 blocks 42 / 38 and 50 / 48; 10,000 blocks
-// keep 256 51 / 60: a workgroup of four takes longer to lay its basis out).
-constexpr int64_t kFewRows = 4096;
+// Up to this many coefficients, 16384 blocks at keep 256, a request is one of few blocks (forward + inverse
+// as blocking calls, us, basis in LDS / read where it is used: one block 34 / 30 at keep 64, 45 / 33 at
+// keep 256; 4096 blocks 38 / 33 and 48 / 37; 16,000 44 / 39 and 59 / 55; 24,000 46 / 42 and
+// 63 / 70; 40,000 54 / 50 and 87 / 95; keep 128, 16,000 / 24,000 / 40,000 blocks 53 / 44, 54 / 51, 65 / 68;
+// keep 64 130,000 blocks 88 / 100).
+constexpr int64_t kFewCoefficients = (int64_t)1 << 22;
 constexpr int64_t kWholeRows = 2 * 256 * 8 * kWaveRows;
 
 static int32_t dct2_run(const float* in, float* out, int64_t n, int32_t keep, uint32_t flags, bool forward) {
@@ -381,7 +460,6 @@ static int32_t dct2_run(const float* in, float* out, int64_t n, int32_t keep, ui
   // pairs (inverse), the columns over keep / 2 coefficient pairs (forward) or 128 position pairs
   const int KF = forward ? kFoldB : keep / 2;
   const int NF = forward ? keep / 2 : kFoldB;
-  const int waves = M <= kFewRows ? 4 : 8;
   // 64 folded columns a wavefront where the width allows. Forward keep 192 takes all of its 96 in one
   // workgroup from two row tiles a workgroup on, so that X is read once instead of three times
   // (forward + inverse: 262,144 blocks 285 -> 260 us, 160,000 187 -> 170; 80,000 116 either way,
@@ -389,12 +467,12 @@ static int32_t dct2_run(const float* in, float* out, int64_t n, int32_t keep, ui
   const int nt = (NF % 64 == 0) ? 2 : (NF == 96 && M >= kWholeRows ? 3 : 1);
   const int gy = NF / (32 * nt);
   const size_t lds_bytes = (size_t)(KF / 8) * 3 * 2 * nt * 32 * 16;   // [KF / 8][3][2 nt][32] x 16 bytes
-  const int64_t tiles = (M + waves * kWaveRows - 1) / (waves * kWaveRows);
+  const int64_t tiles = (M + kWaves * kWaveRows - 1) / (kWaves * kWaveRows);
   int64_t gx = 256 / gy;                           // one workgroup a compute unit
   if (gx > tiles) gx = tiles;
   if (gx < 1) gx = 1;
   const __bf16* basis = forward ? g_basis3_fwd : g_basis3_inv;
-  const dim3 grid((unsigned)gx, (unsigned)gy), block((unsigned)(waves * kWave));
+  const dim3 grid((unsigned)gx, (unsigned)gy), block(kWaves * kWave);
   const int64_t ldx = forward ? kDctB : keep, ldy = forward ? keep : kDctB;
   hipError_t e = hipSuccess;
   auto launch = [&](auto kernel) {
@@ -404,22 +482,22 @@ static int32_t dct2_run(const float* in, float* out, int64_t n, int32_t keep, ui
     hipLaunchKernelGGL(kernel, grid, block, lds_bytes, s, d_in, ldx, basis, d_out, ldy, M, KF);
     e = hipGetLastError();
   };
-  auto launch_waves = [&](auto w) {
-    constexpr int WAVES = decltype(w)::value;
-    if (!forward) {
-      launch(dct2_split_kernel<2, false, WAVES>);
-    } else if (nt == 2) {
-      launch(dct2_split_kernel<2, true, WAVES>);   // keep 128 and 256
-    } else if (nt == 3) {
-      if constexpr (WAVES == 8) launch(dct2_split_kernel<3, true, WAVES>);   // keep 192
+  if (M * keep <= kFewCoefficients) {
+    const dim3 few((unsigned)((M + kWaveRows - 1) / kWaveRows), (unsigned)(NF / 32));
+    if (forward) {
+      hipLaunchKernelGGL(dct2_few_kernel<true>, few, dim3(kWave), 0, s, d_in, ldx, basis, d_out, ldy, M, KF);
     } else {
-      launch(dct2_split_kernel<1, true, WAVES>);   // keep 64 and 192
+      hipLaunchKernelGGL(dct2_few_kernel<false>, few, dim3(kWave), 0, s, d_in, ldx, basis, d_out, ldy, M, KF);
     }
-  };
-  if (waves == 8) {
-    launch_waves(std::integral_constant<int, 8>{});
+    e = hipGetLastError();
+  } else if (!forward) {
+    launch(dct2_split_kernel<2, false>);
+  } else if (nt == 2) {
+    launch(dct2_split_kernel<2, true>);   // keep 128 and 256
+  } else if (nt == 3) {
+    launch(dct2_split_kernel<3, true>);   // keep 192
   } else {
-    launch_waves(std::integral_constant<int, 4>{});
+    launch(dct2_split_kernel<1, true>);   // keep 64 and 192
   }
   if (e == hipSuccess && host)
     e = hipMemcpy(out, d_out, sizeof(float) * (size_t)out_count, hipMemcpyDeviceToHost);

@@ -53,6 +53,16 @@ def test_row_tiles(dct2, blocks, keep):
     assert (np.abs(dct2.inverse(got, blocks * 256, keep).reshape(blocks, 256) - want) <= 1e-6 * scale).all()
 
 
+# 2^22 coefficients are the most that the kernel for few blocks takes
+@pytest.mark.parametrize("keep,blocks", [(64, 65536), (128, 32768), (192, 21845), (256, 16384)])
+def test_few_blocks_and_many_agree(dct2, keep, blocks):
+    """One block more goes to the kernel that keeps the basis in LDS: the same products in the same order."""
+    x = np.random.default_rng(keep).standard_normal((blocks + 1) * 256).astype(np.float32)
+    few, many = dct2.forward(x[:-256], keep), dct2.forward(x, keep)
+    assert np.array_equal(few, many[:-1])
+    assert np.array_equal(dct2.inverse(few, blocks * 256, keep), dct2.inverse(many, x.size, keep)[:-256])
+
+
 def test_known_vectors(dct2):
     """Closed forms: a constant block has only the k = 0 coefficient (= c * sqrt(256));
     a single cosine of the basis maps to a single coefficient."""
