@@ -22,7 +22,6 @@ __device__ __forceinline__ void vload(const float* p, float (&v)[VEC]) {
     v[0] = *p;
   }
 }
-typedef float vfloat4_t __attribute__((ext_vector_type(4)));
 template <int VEC>
 __device__ __forceinline__ void vstore_once(float* p, const float (&v)[VEC]) {
   if constexpr (VEC == 4) {
@@ -30,20 +29,6 @@ __device__ __forceinline__ void vstore_once(float* p, const float (&v)[VEC]) {
     __builtin_nontemporal_store(x, reinterpret_cast<vfloat4_t*>(p));
   } else {
     __builtin_nontemporal_store(v[0], p);
-  }
-}
-// The same accesses through pointers the compiler is told lie in global memory. A table's record
-// pointer that a kernel reads out of a descriptor is a generic pointer to the compiler, which
-// then uses flat instructions; those count as LDS operations too, so every wait for an LDS read
-// (the sorted positions, the run starts) would also wait for the records requested before it.
-#define KRK_GLOBAL __attribute__((address_space(1)))
-template <int VEC>
-__device__ __forceinline__ void gload(const float* p, float (&v)[VEC]) {
-  if constexpr (VEC == 4) {
-    const vfloat4_t x = *(const KRK_GLOBAL vfloat4_t*)p;
-    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
-  } else {
-    v[0] = *(const KRK_GLOBAL float*)p;
   }
 }
 // A row that is read exactly once (the gradient rows a reduction gathers): non-temporal, so the

@@ -51,6 +51,22 @@ struct TableView {
   uint32_t* inserted;   // pinned host word: a pull that makes rows sets it (see pull_enqueue)
 };
 
+typedef float vfloat4_t __attribute__((ext_vector_type(4)));
+// Accesses through pointers the compiler is told lie in global memory. A table's record
+// pointer that a kernel reads out of a descriptor is a generic pointer to the compiler, which
+// then uses flat instructions; those count as LDS operations too, so every wait for an LDS read
+// (the sorted positions, the run starts) would also wait for the records requested before it.
+#define KRK_GLOBAL __attribute__((address_space(1)))
+template <int VEC>
+__device__ __forceinline__ void gload(const float* p, float (&v)[VEC]) {
+  if constexpr (VEC == 4) {
+    const vfloat4_t x = *(const KRK_GLOBAL vfloat4_t*)p;
+    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+  } else {
+    v[0] = *(const KRK_GLOBAL float*)p;
+  }
+}
+
 constexpr int kBucket = 4;   // slots per bucket: one aligned 64-byte sector
 
 // The 64-bit word a record keeps when an optimizer needs it: the low 63 bits count Adam's
@@ -344,6 +360,64 @@ __device__ inline ProbeResult probe_insert(const TableView& tv, uint64_t id, boo
   Slot* slot = nullptr;
   int src = 0;
   return probe_insert_impl<false>(tv, id, active, gl, group, won, slot, src);
+}
+
+// The same search for 64 ids of a wavefront at a time, one per lane: every lane hashes its own id once, and
+// then four lanes each read the buckets of sixteen ids, four times over, all of them requested before
+// the first is looked at. With four lanes that all hash the same id a look-up costs 70 to 108 vector
+// instructions per sixteen ids, more than half of the time a large one takes (8.5 million pooled ids
+// 164 us, this way 96-108; four million 75 and 49; a hundred 3.1 and 2.7).
+// hit(lane, row, launch) is called by a lane that found the id of lane `lane`. Returns the lanes whose id
+// was not found (or is the one that equals the empty marker: the caller searches for that one).
+template <typename Hit>
+__device__ __forceinline__ unsigned long long find_many(const TableView& tv, uint64_t id, bool active, Hit hit) {
+  const int lane = wave_lane();
+  const int quad = lane / kBucket, gl = lane & (kBucket - 1);
+  const uint32_t nb_mask = (uint32_t)(tv.mask >> 2);   // rows are numbered in 32 bits, so there are fewer buckets
+  const uint32_t id_lo = (uint32_t)id, id_hi = (uint32_t)(id >> 32);
+  uint32_t b = (uint32_t)mix64(id) & nb_mask;
+  unsigned long long missing = __ballot(active && id == kEmptyKey);
+  unsigned long long open = __ballot(active && id != kEmptyKey);
+  constexpr int kRounds = kWave / (kWave / kBucket);   // of sixteen ids
+  // one bit per lane -> one bit per group of four: whether any of them is set
+  auto quads = [](unsigned long long m) -> unsigned long long {
+    m |= m >> 1;
+    m = (m | m >> 2) & 0x1111111111111111ull;
+    m = (m | m >> 3) & 0x0303030303030303ull;
+    m = (m | m >> 6) & 0x000F000F000F000Full;
+    m = (m | m >> 12) & 0x000000FF000000FFull;
+    return (m | m >> 24) & 0xFFFFull;
+  };
+  for (uint32_t tried = 0; open; ++tried) {
+    if (tried > nb_mask) return missing | open;        // every bucket has been looked at
+    uint4 raw[kRounds];
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+      const uint32_t part = (uint32_t)(open >> (16 * r)) & 0xFFFFu;   // uniform
+      if (part) {
+        const uint32_t at = (uint32_t)__shfl((int)b, 16 * r + quad);
+        if ((part >> quad) & 1u) raw[r] = *reinterpret_cast<const uint4*>(&tv.slots[(uint64_t)at * kBucket + gl]);
+      }
+    }
+    unsigned long long next = 0;
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+      const uint32_t part = (uint32_t)(open >> (16 * r)) & 0xFFFFu;
+      if (part) {
+        const uint32_t lo = (uint32_t)__shfl((int)id_lo, 16 * r + quad), hi = (uint32_t)__shfl((int)id_hi, 16 * r + quad);
+        const bool on = (part >> quad) & 1u;
+        const bool match = on && raw[r].x == lo && raw[r].y == hi;
+        const bool empty = on && (raw[r].x & raw[r].y) == 0xFFFFFFFFu;
+        if (match) hit(16 * r + quad, raw[r].z, raw[r].w);
+        const unsigned long long found = quads(__ballot(match)), ends = quads(__ballot(empty));
+        missing |= (ends & ~found) << (16 * r);
+        next |= (part & ~found & ~ends) << (16 * r);
+      }
+    }
+    open = next;
+    b = (b + 1u) & nb_mask;
+  }
+  return missing;
 }
 
 // One lane looking an id up by itself (no votes): the rare second look of pooled_sum_kernel.

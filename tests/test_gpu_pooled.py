@@ -322,3 +322,28 @@ def test_offsets_that_descend_stay_inside_the_request(api, filler, noted, weight
         assert np.array_equal(t.Pull(ids)[1], want), off[:3]
     if group:
         group.close()
+
+
+# a wavefront looks 64 ids up together; the last of the table's buckets are chained where it is half full
+@pytest.mark.parametrize("n", [1, 15, 16, 63, 64, 65, 255, 257, 5000])
+@pytest.mark.parametrize("dim", [4, 6, 32])
+def test_pooled_pulls_find_every_id(api, n, dim):
+    """Resident ids, ids that are made by the call, repeats of both, and the id that equals the index's
+    empty marker, in one pull; the rows against a plain pull's, added in position order."""
+    rng = np.random.default_rng(n + dim)
+    t = api.SparseTable(dim, api.Initializer.create(api.InitializerType.kNormal, {"stddev": "1", "seed": "5"}),
+                        capacity_hint=4096)
+    t.Pull(splitmix64(np.arange(3500, dtype=np.uint64)))
+    ids = splitmix64(rng.integers(0, 4000, n).astype(np.uint64))
+    ids[rng.integers(0, n, max(1, n // 20))] = np.uint64(2**64 - 1)
+    cuts = np.sort(rng.integers(0, n + 1, max(1, n // 4)))
+    offsets = np.concatenate([[0], cuts, [n]]).astype(np.int64)
+    rc, got = t.PullPooled(ids, offsets)
+    assert rc == 0
+    rows = t.Pull(ids)[1]
+    want = np.zeros((offsets.size - 1, dim), np.float32)
+    for b in range(offsets.size - 1):
+        for j in range(offsets[b], offsets[b + 1]):
+            want[b] = rows[j] if j == offsets[b] else want[b] + rows[j]
+    assert np.array_equal(got, want)
+    assert len(t) == np.union1d(ids, splitmix64(np.arange(3500, dtype=np.uint64))).size
