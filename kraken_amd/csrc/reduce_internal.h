@@ -150,9 +150,8 @@ __device__ __forceinline__ void finish_row(const TableView& tv, uint32_t row, co
       steps |= kHasMomentumBit;
     }
     if (OPT == KRK_ADAM) {
-      const float count = (float)(steps & ~kHasMomentumBit);
-      bc1 = (float)(1.0 - (double)powf(a.k.beta1, count));
-      bc2 = (float)(1.0 - (double)powf(a.k.beta2, count));
+      bc1 = one_minus_power(a.k.log2_beta1, a.k.beta1, steps & ~kHasMomentumBit);
+      bc2 = one_minus_power(a.k.log2_beta2, a.k.beta2, steps & ~kHasMomentumBit);
     }
   }
   if (lane_on) {
@@ -175,7 +174,7 @@ __device__ __forceinline__ void finish_row(const TableView& tv, uint32_t row, co
 }
 
 // The lane's slice of the record is requested before the 64-bit word is looked at: the bias
-// corrections (two powf) then overlap with the loads instead of preceding them.
+// corrections then overlap with the loads instead of preceding them.
 template <int OPT, int VEC>
 __device__ __forceinline__ void apply_row(const TableView& tv, uint32_t row, const float (&gsum)[VEC],
                                           int e, bool lane_on, int gl, bool last_chunk, int dim,

@@ -147,6 +147,8 @@ OptimK make_optim_k(const krk_optim& o) {
   k.alpha = o.alpha;
   k.one_minus_alpha = (float)(1.0 - (double)o.alpha);
   k.acc0 = o.initial_accumulator;
+  k.log2_beta1 = std::log2(std::fabs((double)o.beta1));
+  k.log2_beta2 = std::log2(std::fabs((double)o.beta2));
   return k;
 }
 

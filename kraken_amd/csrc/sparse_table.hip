@@ -217,7 +217,7 @@ __device__ __forceinline__ void push_body(const TableView& tv, const uint64_t* _
   float* rec = tv.recs + (int64_t)row * tv.stride;
 
   // The lane's first slice of the record is requested before the 64-bit word is looked at: the
-  // bias corrections (two powf) then overlap with the loads instead of preceding them.
+  // bias corrections then overlap with the loads instead of preceding them.
   float w[VEC], s0[VEC], s1[VEC], s2[VEC];
   if (gl < elems) {
     vload<VEC>(rec + gl * VEC, w);
@@ -239,9 +239,8 @@ __device__ __forceinline__ void push_body(const TableView& tv, const uint64_t* _
     }
     if (OPT == KRK_ADAM) {
       // ps/optim/adam.cc:61-64 : per-row step counter, float pow, double subtraction
-      const float count = (float)(steps & ~kHasMomentumBit);
-      bc1 = (float)(1.0 - (double)powf(k.beta1, count));
-      bc2 = (float)(1.0 - (double)powf(k.beta2, count));
+      bc1 = one_minus_power(k.log2_beta1, k.beta1, steps & ~kHasMomentumBit);
+      bc2 = one_minus_power(k.log2_beta2, k.beta2, steps & ~kHasMomentumBit);
     }
   }
   for (int e = gl; e < elems; e += group) {
@@ -839,9 +838,8 @@ __device__ __forceinline__ void push_wide(const TableView& tv, const uint64_t* _
       if (OPT == KRK_ADAM) {
         // ps/optim/adam.cc:61-64 : per-row step counter, float pow, double subtraction
         steps += 1;                                 // the flag bit rides along untouched
-        const float count = (float)(steps & ~kHasMomentumBit);
-        bc1 = (float)(1.0 - (double)powf(k.beta1, count));
-        bc2 = (float)(1.0 - (double)powf(k.beta2, count));
+        bc1 = one_minus_power(k.log2_beta1, k.beta1, steps & ~kHasMomentumBit);
+        bc2 = one_minus_power(k.log2_beta2, k.beta2, steps & ~kHasMomentumBit);
       } else {
         first_update = (steps & kHasMomentumBit) == 0;
         steps |= kHasMomentumBit;

@@ -297,6 +297,42 @@ def test_adam_amsgrad_impulse_closed_form(api, oracle):
     assert sorted(steps.tolist()) == [3, 5, 6]
 
 
+@pytest.mark.parametrize("raw", [False, True], ids=["push", "push_raw"])
+@pytest.mark.parametrize("beta1,beta2", [(0.9, 0.999), (0.0, 0.5), (0.99999, 0.9999999), (-0.5, 0.25)])
+def test_adam_bias_corrections_over_many_steps(api, beta1, beta2, raw):
+    """ps/optim/adam.cc:57-78 over 400 updates of a row, against the same float operations in numpy with
+    corrections from the power in extended precision. The sums, products and quotients are rounded alike
+    on both sides; a correction may be off by one unit in its last place, which moves mt / sqrt(vt) by at
+    most 2 units of 2^-24 and its own two roundings by as many again: 4 * 2^-24 of each step's size."""
+    dim, lr, steps = 8, 0.125, 400
+    f32, ld = np.float32, np.longdouble
+    rng = np.random.default_rng(5)
+    t = api.SparseTable(dim, api.Initializer.create(api.InitializerType.kConstant, {"value": "0"}))
+    ids = np.array([9], np.uint64)
+    assert t.Pull(ids)[0] == 0
+    o = api.Optim.create(api.OptimType.kAdam, {"beta1": str(beta1), "beta2": str(beta2), "eps": "1e-3"})
+    b1, b2, eps = f32(beta1), f32(beta2), f32(1e-3)
+    r1, r2 = f32(1.0 - float(b1)), f32(1.0 - float(b2))
+    m = np.zeros(dim, f32)
+    v = np.zeros(dim, f32)
+    w = np.zeros(dim, np.float64)
+    moved = np.zeros(dim)
+    for k in range(1, steps + 1):
+        g = rng.standard_normal(dim).astype(f32)
+        assert (t.PushRaw if raw else t.Push)(o, ids, g[None], lr) == 0
+        m = b1 * m + r1 * g
+        v = b2 * v + r2 * (g * g)
+        c1 = f32(1.0 - float(f32(ld(b1) ** k)))
+        c2 = f32(1.0 - float(f32(ld(b2) ** k)))
+        step = (f32(lr) * (m / c1)) / (np.sqrt(v / c2) + eps)
+        w -= step
+        moved += np.abs(step)
+        if k in (1, 2, 3, 10, 100, steps):
+            got = t.Pull(ids)[1][0]
+            # a weight is rounded once a step as well, to a unit of at most the path's length
+            assert np.all(np.abs(got - w) <= (4 + k) * 2.0 ** -24 * moved), k
+
+
 @pytest.mark.parametrize("dim", [20, 32, 36, 64, 100, 124, 128])
 def test_wide_rows_pull_every_path(api, oracle, dim):
     """Rows of 32 to 128 floats are pulled by kernels of their own (sixteen ids looked up per
