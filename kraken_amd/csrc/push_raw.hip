@@ -854,10 +854,11 @@ static void dispatch_segreduce(int opt, bool level0, const TableView& tv, const 
 constexpr int kLevel0Tile = 16;
 
 // ---------------------------------------------------------------------------
-// Requests of 2049 to 12288 ids per table (shorter ones: pick_runs; twelve positions a lane: what the LDS of a compute unit holds
-// besides the run lists, one workgroup a unit as with eight; the global sort that longer requests
-// take is six to nine launches: an embedding step of 10,000 ids of 16 floats, forward, backward,
-// forward, 61 us with it and 39 us with this): two launches, no carry levels, no global sort.
+// Requests of 2049 to 12288 ids per table whose rows have at most 64 floats (shorter ones: pick_runs;
+// longer ones: partition_pairs and reduce_runs. Twelve positions a lane are what the LDS of a compute unit
+// holds besides the run lists, one workgroup a unit as with eight. An embedding step of 10,000 ids of 16
+// floats, forward, backward, forward: 39 us with this, 61 with a sort of all positions, six to nine
+// launches): two launches, one where the rows come from a pull's notes, no carry levels.
 //   1. ids -> rows for every position, over the whole chip (rows_of_ids / group_rows_of_ids).
 //   2. bucket_push_kernel, one workgroup of 1024 lanes for each of a table's 8 to 128 buckets
 //      (bucket = row mod the number of buckets; as many as keep the request at about one
@@ -865,9 +866,10 @@ constexpr int kLevel0Tile = 16;
 //      a. the workgroup reads its table's row numbers and keeps the positions of its bucket, in
 //         position order (one scan over the workgroup);
 //      b. the (row, position) pairs are sorted by row in LDS: up to 256 of them by counting
-//         (rank_list, 0.4-2.4 us), more with a stable radix sort, nine bits a pass (two passes for tables of up to two million rows). Every wavefront ranks its own
-//         elements with wave-wide votes (lanes holding the same digit find each other through
-//         nine ballots), a per-wavefront histogram in LDS turns into offsets by one scan over
+//         (rank_list, 0.4-2.4 us), more with a stable radix sort, nine bits a pass (two passes for
+//         tables of up to two million rows). Every wavefront ranks its own elements with wave-wide
+//         votes (lanes holding the same digit find each other through nine ballots), a
+//         per-wavefront histogram in LDS turns into offsets by one scan over
 //         (digit, wavefront), and the pairs are scattered through LDS;
 //      c. every run of equal rows is summed in position order (worker/emitter.cc:527-529) and
 //         applied once. Who adds a run up depends on its length: a lane group (up to 16
