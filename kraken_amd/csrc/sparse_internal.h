@@ -473,6 +473,7 @@ struct krk_sparse : krk::ObjBase {
   uint32_t epoch = 0;                 // number of the last launch that could insert
   uint64_t layout_version = 0;        // bumped whenever slots, records or columns move
   int pull_parity = 0;                // which set of list counters the next two-launch pull queues into
+  int few_pulls = 0;                  // pooled pulls that still expect many new ids
 
   int32_t col_off[KRK_ST_COUNT];      // float offset of each state column in a record, -1 = absent
   int32_t meta_off = -1;              // float offset of the step counter (two u32), -1 = absent
@@ -581,6 +582,7 @@ struct krk_group : krk::ObjBase {
   // empty and every member's layout_version is what it was.
   krk::DeviceBuffer notes;
   krk::DeviceBuffer todo;              // the lists of a combined pull that queues its missing ids
+  int few_pulls = 0;                   // as in krk_sparse
   std::vector<const uint64_t*> noted_ids;   // per member; empty: nothing noted
   std::vector<int64_t> noted_offsets;
   std::vector<uint64_t> noted_versions;

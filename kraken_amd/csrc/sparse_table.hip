@@ -15,10 +15,17 @@
 #include <cmath>
 #include <new>
 #include <thread>
+#include <type_traits>
 
 #include "sparse_internal.h"
 
 namespace krk {
+
+// f(std::true_type) or f(std::false_type)
+template <typename F>
+static void with_bool(bool b, F f) {
+  if (b) f(std::true_type()); else f(std::false_type());
+}
 
 constexpr int kBlock = 256;
 constexpr int64_t kTwoLaunchPull = 1 << 18;   // ids from which a pull runs as two launches
@@ -34,6 +41,10 @@ constexpr int kFillingIds = 3;
 // 15 us more than its fused kernel where nothing is new: over 26 tables they pay from one new id
 // in five on (98.6k ids, one in ten new: 21 us fused, 27 us in two launches; all new: 64 and 34).
 constexpr int kFillingIdsCombined = 8;
+// The same for a wavefront of a pooled pull that looks 64 ids up: four, or sixteen, of them are new as often
+// in a request with one new id in 250, or ten.
+constexpr int kFilling64 = 4;
+constexpr int kFilling64Combined = 16;
 constexpr int kMissingGrid = 512;             // workgroups (of 1024 lanes) of the launch that inserts missing ids
 // The positions whose id is missing are queued in kQueues lists, each with a counter on a line
 // of its own: workgroup b of the first launch appends to list b mod kQueues. One counter for the
@@ -533,49 +544,77 @@ __global__ __launch_bounds__(kBlock) void pooled_find_kernel(TableView tv, const
   pooled_find_body(tv, ids, p, n, blockIdx.x, rows, todo, parity);
 }
 
-// p0: the wavefront's first position; it takes 64.
+// Makes the rows of sixteen ids of a wavefront, four lanes each (`mine`: the four have one, `p` is its
+// position). Returns how many rows are new.
+template <int VEC>
+__device__ __forceinline__ int pooled_insert(const TableView& tv, const InitK& init, uint64_t id, bool mine, int64_t p,
+                                             uint32_t* __restrict__ rows, int elems) {
+  const int gl = threadIdx.x & (kBucket - 1);
+  const ProbeResult pr = probe_insert(tv, id, mine, gl, kBucket);
+  const int made = __popcll(__ballot(mine && pr.owner && gl == 0));
+  if (!mine) return made;
+  if (pr.fresh && pr.owner && pr.row != kEmptyRow) {
+    float* rec = tv.recs + (int64_t)pr.row * tv.stride;
+    for (int e = gl; e < elems; e += kBucket) {
+      float v[VEC];
+      init_vec<VEC>(init, id, (int64_t)e * VEC, v);
+      vstore<VEC>(rec + e * VEC, v);
+    }
+  }
+  if (gl == 0) rows[p] = pr.row;
+  return made;
+}
+
+// p0: the wavefront's first position. It takes 64, or sixteen where `few` says so (pooled_few): a wavefront
+// makes sixteen rows at a time, one chain of trips to memory (and, for random initial values, their
+// arithmetic) after the other. A pull of 4000 ids over rows of 64 floats, us, none / 2 % / a fifth / all of them
+// new: with sixteen 12.3 / 28 / 25 / 24-36, with 64 11 / 55 / 63 / 56 while the new ones stayed in four
+// rounds by position, and 11 / 29 / 26 / 37 with those of the wavefront moved together.
 template <int VEC>
 __device__ __forceinline__ void pooled_probe_body(const TableView& tv, const InitK& init,
                                                   const uint64_t* __restrict__ ids, int64_t p0, int64_t n,
-                                                  uint32_t* __restrict__ rows, int elems, int filling_ids) {
+                                                  uint32_t* __restrict__ rows, int elems, int filling_ids, bool few) {
   const int lane = wave_lane();
+  const int quad = lane / kBucket;
+  if (few) {                                           // uniform
+    const int64_t p = p0 + quad;
+    const bool active = p < n;
+    const int made = pooled_insert<VEC>(tv, init, active ? ids[p] : 0, active, p, rows, elems);
+    if (made >= filling_ids && lane == 0) note_inserting(tv);
+    return;
+  }
   const bool active = p0 + lane < n;
   const uint64_t id = active ? ids[p0 + lane] : 0;
   const unsigned long long missing =
       find_many(tv, id, active, [&](int l, uint32_t row, uint32_t) { rows[p0 + l] = row; });
   if (missing == 0ull) return;                         // uniform
-  // the ids that are not there, sixteen at a time as in pull_body
-  const int quad = lane / kBucket, gl = lane & (kBucket - 1);
-  for (int r = 0; r < kBucket; ++r) {
-    const uint32_t part = (uint32_t)(missing >> (16 * r)) & 0xFFFFu;
-    if (part == 0u) continue;                          // uniform
-    const int src = 16 * r + quad;
+  // The ids that are not there, moved together: the lane of the k-th of them goes to lane k (the other lanes
+  // send theirs behind), so that up to sixteen are one round.
+  const int count = __popcll(missing);
+  const unsigned long long below = (1ull << lane) - 1ull;
+  const bool gone = (missing >> lane) & 1ull;
+  const int to = gone ? __popcll(missing & below) : count + __popcll(~missing & below);
+  const int order = __builtin_amdgcn_ds_permute(to * 4, lane);
+  int made = 0;
+  for (int k0 = 0; k0 < count; k0 += kWave / kBucket) {
+    const bool mine = k0 + quad < count;
+    const int src = __shfl(order, k0 + quad);          // (k0 + quad < 64)
     const uint64_t its = (uint64_t)(uint32_t)__shfl((int)(uint32_t)id, src) |
                          ((uint64_t)(uint32_t)__shfl((int)(uint32_t)(id >> 32), src) << 32);
-    const bool mine = (part >> quad) & 1u;
-    const ProbeResult pr = probe_insert(tv, its, mine, gl, kBucket);
-    if (__popcll(__ballot(mine && pr.owner && gl == 0)) >= filling_ids && lane == 0) note_inserting(tv);
-    if (!mine) continue;
-    if (pr.fresh && pr.owner && pr.row != kEmptyRow) {
-      float* rec = tv.recs + (int64_t)pr.row * tv.stride;
-      for (int e = gl; e < elems; e += kBucket) {
-        float v[VEC];
-        init_vec<VEC>(init, its, (int64_t)e * VEC, v);
-        vstore<VEC>(rec + e * VEC, v);
-      }
-    }
-    if (gl == 0) rows[p0 + src] = pr.row;
+    made += pooled_insert<VEC>(tv, init, its, mine, p0 + src, rows, elems);
   }
+  if (made >= filling_ids && lane == 0) note_inserting(tv);
 }
 
 // (Eight wavefronts a SIMD: the path that inserts would take nine registers too many for that and gets by
 // with three words of scratch memory; 8.5 million ids 108 -> 96 us.)
-template <int VEC>
-__global__ __launch_bounds__(kBlock, 8) void pooled_probe_kernel(TableView tv, InitK init,
+template <int VEC, bool FEW>
+__global__ __launch_bounds__(kBlock, FEW ? 1 : 8) void pooled_probe_kernel(TableView tv, InitK init,
                                                               const uint64_t* __restrict__ ids, int64_t n,
                                                               uint32_t* __restrict__ rows, int elems) {
-  const int64_t p0 = (int64_t)blockIdx.x * kBlock + threadIdx.x / kWave * kWave;
-  pooled_probe_body<VEC>(tv, init, ids, p0, n, rows, elems, kFillingIds);
+  constexpr int kTake = FEW ? kWave / kBucket : kWave;
+  const int64_t p0 = ((int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave) * kTake;
+  pooled_probe_body<VEC>(tv, init, ids, p0, n, rows, elems, FEW ? kFillingIds : kFilling64, FEW);
 }
 
 // Records of one bag requested together. Eight take registers of which two wavefronts a SIMD live (852k bags
@@ -1036,7 +1075,7 @@ __global__ __launch_bounds__(kMissBlock) void group_pull_missing_kernel(const Ta
 // The two launches of a pooled pull with every member's positions (bags) side by side. A request of
 // 26 fields of 2048 bags is 26 x 10k positions: a table at a time its launches leave three quarters
 // of the chip idle and cost the host two launches each (26 tables of dim 16: 340 us a pull that way).
-template <int VEC>
+template <int VEC, bool FEW>
 __global__ __launch_bounds__(kBlock) void group_pooled_probe_kernel(const TableDesc* __restrict__ descs,
                                                                     GroupCall call, GroupParts parts,
                                                                     uint32_t* __restrict__ rows, int elems) {
@@ -1044,9 +1083,11 @@ __global__ __launch_bounds__(kBlock) void group_pooled_probe_kernel(const TableD
   TableView tv = descs[t].tv;
   tv.epoch = call.epoch[t];
   const InitK init = descs[t].init;
-  const int64_t p0 = (int64_t)(blockIdx.x - call.block_start[t]) * kBlock + threadIdx.x / kWave * kWave;
+  constexpr int kTake = FEW ? kWave / kBucket : kWave;
+  const int64_t p0 = ((int64_t)(blockIdx.x - call.block_start[t]) * (kBlock / kWave) + threadIdx.x / kWave) * kTake;
   const int64_t a = call.row_start[t];
-  pooled_probe_body<VEC>(tv, init, parts.ids[t], p0, call.row_start[t + 1] - a, rows + a, elems, kFillingIdsCombined);
+  pooled_probe_body<VEC>(tv, init, parts.ids[t], p0, call.row_start[t + 1] - a, rows + a, elems,
+                         FEW ? kFillingIdsCombined : kFilling64Combined, FEW);
 }
 
 __global__ __launch_bounds__(kBlock) void group_pooled_find_kernel(const TableDesc* __restrict__ descs,
@@ -2106,6 +2147,18 @@ int32_t krk_sparse_sync(krk_sparse* t) {
   return sparse_finish(t, 0);
 }
 
+// Whether the wavefronts of a pooled pull of n ids that inserts as it looks up take sixteen ids each or 64:
+// sixteen where many are expected to be new and the request is too short to queue them (longer ones
+// are not faster with it: 50,000 ids of 16 floats, all new, 75 us with 64, 130-200 with sixteen). The device's
+// word lags behind the host, which may be several pulls ahead, and a form that is wrong for a few pulls
+// costs a microsecond each where nothing is new, so once said it holds for eight pulls (4000 ids a pull,
+// all new, 64 floats: 37 us where every pull asked afresh, 30-33 this way).
+constexpr int kFewPulls = 8;
+static bool pooled_few(bool filling, int64_t n, int* left) {
+  if (filling) *left = kFewPulls;
+  return *left > 0 && (*left)-- > 0 && n < kTwoLaunchWhileFilling;
+}
+
 // The launches of one pull of n > 0 ids into d_out [n, dim]; the caller holds the table's lock
 // and has made room for n more rows.
 static int32_t pull_enqueue(krk_sparse* t, const uint64_t* d_ids, int64_t n, float* d_out,
@@ -2253,6 +2306,7 @@ int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, co
   // which one in ten is new cost it half a million additions, served one after the other.
   const bool filling = t->host_inserted && __atomic_exchange_n(t->host_inserted, 0u, __ATOMIC_RELAXED) != 0u;
   const bool queued = filling && n >= kTwoLaunchWhileFilling;
+  const bool few = pooled_few(filling, n, &t->few_pulls);
   const int64_t list_capacity = queued ? queue_capacity(n, kBlock / kBucket) : 0;
   // KRK_NOTE_ROWS: the rows of the positions, which the last launch reads, stay behind
   uint32_t* notes = nullptr;
@@ -2265,8 +2319,12 @@ int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, co
   uint32_t* rows = notes ? notes : t->scratch[5].as<uint32_t>();
   uint32_t* todo = t->scratch[5].as<uint32_t>() + rows_words;
   const int per_block = kBlock / t->group;
-  // a lane looks up an id of its own, or four lanes one where the missing ones are queued
-  const dim3 probe_grid(grid_for(n, queued ? kBlock / kBucket : kBlock)), grid(grid_for(bags, per_block)), block(kBlock);
+  // a lane looks up an id of its own, or four lanes one where many are to be inserted
+  const dim3 probe_grid(grid_for(n, few || queued ? kBlock / kBucket : kBlock)), grid(grid_for(bags, per_block)), block(kBlock);
+  const auto probe = [&](auto vec, auto few) {
+    hipLaunchKernelGGL((pooled_probe_kernel<vec.value, few.value>), probe_grid, block, 0, t->stream, t->view(), t->initk,
+                       d_ids, n, rows, t->elems);
+  };
   const dim3 small(kMissingGrid), missing_block(kMissBlock);
   const int mean = mode == KRK_POOL_MEAN;
   int parity = 0;
@@ -2280,8 +2338,7 @@ int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, co
       hipLaunchKernelGGL((pull_missing_kernel<4, true>), small, missing_block, 0, t->stream, t->view(), t->initk,
                          d_ids, nullptr, todo, parity, list_capacity, (int)t->dim, t->elems, t->group, rows);
     else if (n > 0)
-      hipLaunchKernelGGL((pooled_probe_kernel<4>), probe_grid, block, 0, t->stream, t->view(), t->initk, d_ids,
-                         n, rows, t->elems);
+      with_bool(few, [&](auto few16) { probe(std::integral_constant<int, 4>(), few16); });
     hipLaunchKernelGGL((pooled_sum_kernel<4>), grid, block, 0, t->stream, t->view(), rows, d_ids, n, d_off, bags, d_w,
                        mean, patch_value, d_out, (int)t->dim, t->elems, t->group);
   } else {
@@ -2289,8 +2346,7 @@ int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, co
       hipLaunchKernelGGL((pull_missing_kernel<1, true>), small, missing_block, 0, t->stream, t->view(), t->initk,
                          d_ids, nullptr, todo, parity, list_capacity, (int)t->dim, t->elems, t->group, rows);
     else if (n > 0)
-      hipLaunchKernelGGL((pooled_probe_kernel<1>), probe_grid, block, 0, t->stream, t->view(), t->initk, d_ids,
-                         n, rows, t->elems);
+      with_bool(few, [&](auto few16) { probe(std::integral_constant<int, 1>(), few16); });
     hipLaunchKernelGGL((pooled_sum_kernel<1>), grid, block, 0, t->stream, t->view(), rows, d_ids, n, d_off, bags, d_w,
                        mean, patch_value, d_out, (int)t->dim, t->elems, t->group);
   }
@@ -3362,8 +3418,9 @@ int32_t krk_group_pull_pooled_parts(krk_group* g, const krk_pooled_part* in, uin
   for (krk_sparse* t : g->tables)
     if (t->host_inserted && __atomic_exchange_n(t->host_inserted, 0u, __ATOMIC_RELAXED) != 0u) filling = true;
   const bool queued = filling && total >= kTwoLaunchWhileFilling;
-  // a lane looks up an id of its own, or four lanes one where the missing ones are queued
-  const int per_block = queued ? kBlock / kBucket : kBlock;
+  const bool few = pooled_few(filling, total, &g->few_pulls);
+  // a lane looks up an id of its own, or four lanes one where many are to be inserted
+  const int per_block = few || queued ? kBlock / kBucket : kBlock;
   KRK_TRY(group_plan(g, pool.row_start, &call, &checked, per_block));
   for (int m = 0; m < n_tables; ++m) {
     krk_sparse* t = g->tables[m];
@@ -3410,13 +3467,15 @@ int32_t krk_group_pull_pooled_parts(krk_group* g, const krk_pooled_part* in, uin
                          call, parts, fill, todo, per_block, (int)g->dim, g->elems, g->group, rows);
     }
   } else if (total > 0) {
-    if (g->vec == 4) {
-      hipLaunchKernelGGL((group_pooled_probe_kernel<4>), probe_grid, block, 0, g->stream, g->d_descs, call, parts,
-                         rows, g->elems);
-    } else {
-      hipLaunchKernelGGL((group_pooled_probe_kernel<1>), probe_grid, block, 0, g->stream, g->d_descs, call, parts,
-                         rows, g->elems);
-    }
+    with_bool(few, [&](auto few16) {
+      if (g->vec == 4) {
+        hipLaunchKernelGGL((group_pooled_probe_kernel<4, few16.value>), probe_grid, block, 0, g->stream, g->d_descs,
+                           call, parts, rows, g->elems);
+      } else {
+        hipLaunchKernelGGL((group_pooled_probe_kernel<1, few16.value>), probe_grid, block, 0, g->stream, g->d_descs,
+                           call, parts, rows, g->elems);
+      }
+    });
   }
   const dim3 sum_grid((unsigned)sum_blocks);
   if (g->vec == 4) {

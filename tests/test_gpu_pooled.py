@@ -347,3 +347,45 @@ def test_pooled_pulls_find_every_id(api, n, dim):
             want[b] = rows[j] if j == offsets[b] else want[b] + rows[j]
     assert np.array_equal(got, want)
     assert len(t) == np.union1d(ids, splitmix64(np.arange(3500, dtype=np.uint64))).size
+
+
+# A pull below 8192 ids takes sixteen ids a wavefront while many are new, and for eight pulls after, 64
+# otherwise, whose missing ids are moved together sixteen at a time; from 8192 on new ids are queued.
+@pytest.mark.parametrize("n", [17, 64, 65, 1000, 8191, 8192])
+@pytest.mark.parametrize("dim", [6, 32])
+@pytest.mark.parametrize("combined", [False, True])
+def test_pooled_pulls_make_rows(api, n, dim, combined):
+    """Pulls with no, few and only new ids in turn, more than eight with none between them; bags of one
+    id, so that a bag is its row: against a plain pull of the same ids."""
+    C = api.C
+
+    class Part(C.Structure):
+        _fields_ = [("ids", C.c_void_p), ("n", C.c_int64), ("offsets", C.c_void_p), ("bags", C.c_int64),
+                    ("weights", C.c_void_p), ("rows", C.c_void_p), ("stride", C.c_int64), ("mode", C.c_int32),
+                    ("patch", C.c_float)]
+
+    rng = np.random.default_rng(n + dim)
+    gi = api.Initializer.create(api.InitializerType.kNormal, {"stddev": "1", "seed": "5"})
+    tables = [api.SparseTable(dim, gi, capacity_hint=64) for _ in range(2 if combined else 1)]
+    group = api.TableGroup(tables) if combined else None
+    offsets = api.DeviceArray.from_host(np.arange(n + 1, dtype=np.int64))
+    made = 0
+    for step, share in enumerate([1.0, 0.3, 0.0, 1.0] + [0.0] * 10 + [0.02, 0.3, 1.0, 0.02]):
+        fresh = np.arange(made, made + int(np.ceil(n * share)), dtype=np.uint64)
+        made += fresh.size
+        ids, outs = [], []
+        for _ in tables:
+            old = rng.integers(0, made, n - fresh.size).astype(np.uint64)
+            ids.append(splitmix64(np.concatenate([fresh, old])[rng.permutation(n)]))
+            outs.append(api.DeviceArray((n, dim), np.float32))
+        d_ids = [api.DeviceArray.from_host(i) for i in ids]
+        if group:
+            parts = (Part * 2)(*[Part(d.ptr, n, offsets.ptr, n, None, o.ptr, dim, 0, 0.0) for d, o in zip(d_ids, outs)])
+            assert api.lib().krk_group_pull_pooled_parts(group.h, parts, api.DEVICE_PTRS) == 0
+        else:
+            assert tables[0].PullPooled(d_ids[0], offsets, out=outs[0])[0] == 0
+        for t, i, o in zip(tables, ids, outs):
+            assert len(t) == made, (step, len(t))
+            assert np.array_equal(o.to_host(), t.Pull(i)[1]), step
+    if group:
+        group.close()
