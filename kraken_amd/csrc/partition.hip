@@ -149,7 +149,7 @@ template <int BITS, int LANES, bool NOTED>
 __global__ __launch_bounds__(LANES) void scatter_kernel(Input in, const uint32_t* __restrict__ hist,
                                                         const uint32_t* __restrict__ total, int tiles,
                                                         uint32_t* __restrict__ out_h, uint32_t* __restrict__ out_refs,
-                                                        int chunk, RunPlan plan) {
+                                                        RunCut cut, RunPlan plan) {
   constexpr int kBuckets = 1 << BITS;
   constexpr int kWaves = LANES / kWave;
   constexpr int kTile = LANES * kItems;
@@ -215,7 +215,7 @@ __global__ __launch_bounds__(LANES) void scatter_kernel(Input in, const uint32_t
       uint32_t sum = 0;                                // chunks of cut buckets, and above them how many are cut
 #pragma unroll
       for (int k = 0; k < kPer; ++k)
-        if (all[k] > (uint32_t)chunk) sum += ((all[k] + (uint32_t)chunk - 1u) / (uint32_t)chunk) + (1u << 16);
+        if (all[k] > cut.whole) sum += cut.pieces(all[k]) + (1u << 16);
       uint32_t whole;
       uint32_t before = block_scan<LANES>(sum, wave_total, whole);
       at = begin;
@@ -223,11 +223,11 @@ __global__ __launch_bounds__(LANES) void scatter_kernel(Input in, const uint32_t
 #pragma unroll
         for (int k = 0; k < kPer; ++k) {
           plan.begin[first + k] = at;
-          if (all[k] > (uint32_t)chunk) {
+          if (all[k] > cut.whole) {
             const uint32_t c = before >> 16;
             plan.cut[c] = CutBucket{(uint32_t)(first + k), before & 0xFFFFu, at, all[k]};
             plan.done[c] = 0u;
-            before += ((all[k] + (uint32_t)chunk - 1u) / (uint32_t)chunk) + (1u << 16);
+            before += cut.pieces(all[k]) + (1u << 16);
           }
           at += all[k];
         }
@@ -321,7 +321,7 @@ struct Launch {
   Input in;
   int tiles;
   uint32_t *hist, *total, *out_h, *out_refs;
-  int chunk;
+  RunCut cut;
   RunPlan plan;
   hipStream_t stream;
 };
@@ -329,7 +329,7 @@ struct Launch {
 template <int BITS, int LANES, bool NOTED>
 void launch_scatter(const Launch& l) {
   hipLaunchKernelGGL((scatter_kernel<BITS, LANES, NOTED>), dim3((unsigned)l.tiles), dim3(LANES), 0, l.stream, l.in,
-                     l.hist, l.total, l.tiles <= kScatterScans ? l.tiles : 0, l.out_h, l.out_refs, l.chunk, l.plan);
+                     l.hist, l.total, l.tiles <= kScatterScans ? l.tiles : 0, l.out_h, l.out_refs, l.cut, l.plan);
 }
 
 template <int LANES, bool NOTED>
@@ -356,7 +356,7 @@ size_t partition_work_bytes(int64_t n, int bucket_bits) {
 
 int32_t partition_pairs(const uint32_t* keys, const uint32_t* refs, const NotedRows& noted, const TableView& tv,
                         int64_t n, uint32_t miss_key, const RunHash& hash, uint32_t* out_h, uint32_t* out_refs,
-                        int chunk, const RunPlan& plan, void* work, hipStream_t stream) {
+                        const RunCut& cut, const RunPlan& plan, void* work, hipStream_t stream) {
   if (n > kRunsMax || hash.bucket_bits < kMinBits || hash.bucket_bits > kMaxBits) {
     set_error("partition_pairs: %lld pairs into 2^%d buckets", (long long)n, hash.bucket_bits);
     return KRK_E_CAPACITY;
@@ -368,7 +368,7 @@ int32_t partition_pairs(const uint32_t* keys, const uint32_t* refs, const NotedR
   l.total = l.hist + ((size_t)l.tiles << hash.bucket_bits);
   l.out_h = out_h;
   l.out_refs = out_refs;
-  l.chunk = chunk;
+  l.cut = cut;
   l.plan = plan;
   l.stream = stream;
   if (lanes_for(n) == kSmallLanes) return noted.rows ? run<kSmallLanes, true>(l) : run<kSmallLanes, false>(l);

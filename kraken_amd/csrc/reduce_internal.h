@@ -290,7 +290,11 @@ __device__ __forceinline__ uint32_t noted_key(const TableView& tv, uint32_t row,
 
 // ---- partition.hip -----------------------------------------------------------------------------
 // Which workgroup of the reduction takes what: the pairs of a bucket lie side by side, and a bucket
-// of more than `chunk` pairs is cut into chunks.
+// of more than `whole` pairs is cut into chunks of `chunk`.
+struct RunCut {
+  uint32_t whole, chunk;
+  __host__ __device__ uint32_t pieces(uint32_t len) const { return (len + chunk - 1u) / chunk; }
+};
 struct CutBucket {
   uint32_t bucket;
   uint32_t base;       // chunks of the cut buckets before this one
@@ -315,10 +319,10 @@ constexpr int64_t kRunsMax = (int64_t)1 << 20;
 size_t partition_work_bytes(int64_t n, int bucket_bits);
 // Groups n (key, payload) pairs by bucket, in their order inside one; pairs whose key is miss_key or
 // above are left out, and keys become their h. noted: the rows of the pairs' positions in place of
-// keys and payloads. chunk and plan: see RunPlan.
+// keys and payloads.
 int32_t partition_pairs(const uint32_t* keys, const uint32_t* refs, const NotedRows& noted, const TableView& tv,
                         int64_t n, uint32_t miss_key, const RunHash& hash, uint32_t* out_h, uint32_t* out_refs,
-                        int chunk, const RunPlan& plan, void* work, hipStream_t stream);
+                        const RunCut& cut, const RunPlan& plan, void* work, hipStream_t stream);
 
 // ---- run_reduce.hip ----------------------------------------------------------------------------
 // Work space for n pairs: scratch[0] holds the n keys, then the n payloads, and as much again;

@@ -81,7 +81,8 @@ struct RunArgs {
   RunPlan plan;
   RunHash hash;
   uint32_t max_chunks;           // workgroups for chunks of cut buckets, in front of the buckets'
-  int chunk, dim, elems, group;
+  RunCut cut;
+  int dim, elems, group;
 };
 
 // exclusive prefix sum of one value per lane over the workgroup; total to all
@@ -602,7 +603,7 @@ __device__ __forceinline__ void merge_lists(const Reducer<OPT, VEC, FROM, GROUPE
   RunLds& s = r.s;
   const int t = threadIdx.x;
   const uint32_t low_mask = r.low_mask, range = low_mask + 1u;
-  const uint32_t pieces = (cut.len + (uint32_t)a.chunk - 1u) / (uint32_t)a.chunk;
+  const uint32_t pieces = a.cut.pieces(cut.len);
   uint32_t* offs = s.work;
 
   // Brings the lists' entries with places in [from, from + width) into LDS, in list order: those from
@@ -639,7 +640,7 @@ __device__ __forceinline__ void merge_lists(const Reducer<OPT, VEC, FROM, GROUPE
               const uint32_t mid = (c + hi) / 2;
               if (offs[mid] <= e) c = mid; else hi = mid;
             }
-            const uint32_t idx = cut.begin + (c0 + c) * (uint32_t)a.chunk + (e - offs[c]);
+            const uint32_t idx = cut.begin + (c0 + c) * a.cut.chunk + (e - offs[c]);
             key[k] = shared_word(a.list_h + idx);
             ref[k] = shared_word(a.list_refs + idx);
           }
@@ -737,13 +738,13 @@ __global__ __launch_bounds__(kLanes) void reduce_kernel(RunArgs a, TableView tv,
     }
     cut = a.plan.cut[--which];
     piece = blockIdx.x - cut.base;
-    lo = cut.begin + piece * (uint32_t)a.chunk;
-    len = (int)min((uint32_t)a.chunk, cut.len - piece * (uint32_t)a.chunk);
+    lo = cut.begin + piece * a.cut.chunk;
+    len = (int)min(a.cut.chunk, cut.len - piece * a.cut.chunk);
   } else {
     cut.bucket = blockIdx.x - a.max_chunks;
     lo = a.plan.begin[cut.bucket];
     const uint32_t n = a.plan.begin[cut.bucket + 1] - lo;
-    if (n == 0u || n > (uint32_t)a.chunk) return;      // uniform for the workgroup, as the returns above
+    if (n == 0u || n > a.cut.whole) return;      // uniform for the workgroup, as the returns above
     len = (int)n;
   }
   for (int j = t; j < len; j += kLanes) {
@@ -808,7 +809,7 @@ __global__ __launch_bounds__(kLanes) void reduce_kernel(RunArgs a, TableView tv,
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // this wavefront's part of the list and sums is out
   __syncthreads();
   if (t == 0) {
-    const uint32_t pieces = (cut.len + (uint32_t)a.chunk - 1u) / (uint32_t)a.chunk;
+    const uint32_t pieces = a.cut.pieces(cut.len);
     const uint32_t before = __hip_atomic_fetch_add(a.plan.done + which, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     s.last = before + 1u == pieces ? 1u : 0u;
   }
@@ -978,7 +979,16 @@ int bucket_bits_for(int64_t n) {
 // shorter than a bucket commonly is, though, most buckets are cut. Reduction with chunks of 512 / 1024 /
 // 2048 pairs, us: 50,000 ids of 100 floats 39 / 49 / 69, 300,000 of 32 38 / 38 / 47, a million of 16
 // 107 / 74 / 76, of 128 (Zipf 1.3) 186 / 150 / 170.
-int chunk_for(int64_t n) { return n > ((int64_t)1 << 18) ? kListMax / 2 : kListMax / 4; }
+uint32_t chunk_for(int64_t n) { return n > ((int64_t)1 << 18) ? kListMax / 2 : kListMax / 4; }
+// Nor may buckets be cut because they hold many pairs on average: a bucket stays whole up to a quarter more
+// than that (distinct rows vary by a twentieth, rows at even distances by up to a third). A push of 2^20
+// ids, us, cut from a chunk on / by this rule / sorted: distinct rows of 16 floats 186 / 131 / 164, of
+// 128 768 / 624 / 638; consecutive ones of 128 757 / 608 / 609; Zipf 1.05 and 1.3, of 128, 277 / 278 / 324 and
+// 187 / 185 / 236 (277-287 and 191 with whole buckets of up to two chunks).
+uint32_t whole_for(int64_t n, int bucket_bits) {
+  return std::max(chunk_for(n), (uint32_t)((n >> bucket_bits) * 5 / 4));
+}
+static_assert((kRunsMax >> 10) * 5 / 4 <= kListMax, "a whole bucket is one workgroup's");
 
 // Places of keys below `keys`.
 RunHash make_hash(int bucket_bits, uint64_t keys) {
@@ -995,14 +1005,15 @@ RunHash make_hash(int bucket_bits, uint64_t keys) {
 
 // Buckets and chunks of a request, and where its work space lies.
 struct RunShape {
-  int bucket_bits, chunk;
+  int bucket_bits;
+  RunCut cut;
   size_t buckets, cuts, chunks;
   RunShape(int64_t n) {
     bucket_bits = bucket_bits_for(n);
-    chunk = chunk_for(n);
+    cut = RunCut{whole_for(n, bucket_bits), chunk_for(n)};
     buckets = (size_t)1 << bucket_bits;
-    cuts = (size_t)(n / chunk);          // a cut bucket holds more pairs than a chunk
-    chunks = (size_t)(2 * n / chunk);
+    cuts = (size_t)(n / cut.whole);      // a cut bucket holds more than that
+    chunks = (size_t)(n / cut.chunk) + cuts;
   }
 };
 
@@ -1022,7 +1033,7 @@ int32_t reduce_runs(const ReduceShape& sh, hipStream_t stream, DeviceBuffer* scr
   const RunShape shape(n);
   RunArgs a{};
   a.hash = make_hash(shape.bucket_bits, miss_key);
-  a.chunk = shape.chunk;
+  a.cut = shape.cut;
   a.max_chunks = (uint32_t)shape.chunks;
   a.dim = (int)sh.dim;
   a.elems = sh.elems;
@@ -1040,7 +1051,7 @@ int32_t reduce_runs(const ReduceShape& sh, hipStream_t stream, DeviceBuffer* scr
   a.sums = scratch[3].as<float>();
   uint32_t* pairs = scratch[0].as<uint32_t>();
   uint32_t* h = pairs + 2 * n;
-  KRK_TRY(partition_pairs(pairs, pairs + n, noted, tv, n, miss_key, a.hash, h, h + n, a.chunk, a.plan, scratch[1].ptr,
+  KRK_TRY(partition_pairs(pairs, pairs + n, noted, tv, n, miss_key, a.hash, h, h + n, a.cut, a.plan, scratch[1].ptr,
                           stream));
   a.h = h;
   a.refs = h + n;

@@ -59,6 +59,24 @@ def test_dedup_sum_sizes(api, n, kind):
     assert np.array_equal(sums, _sums(inv, grads, u.size))
 
 
+# 2^20 pairs in 1024 buckets: up to 1280 of them are a bucket's one workgroup's, more are cut into chunks of 1024
+def test_dedup_sum_whole_and_cut_buckets(api):
+    rng = np.random.default_rng(1)
+    n, unique = 2**20, 2**19
+    keys = np.arange(unique)
+    bucket = _bucket(keys, 20).astype(np.int64)
+    want = np.full(1024, 1024)
+    edges = [1023, 1025, 1279, 1280, 1281, 2047, 2048, 2049]
+    want[:len(edges)] = edges
+    want[100:340] -= 16                                 # what the edges have more than 1024 each: 3840
+    more = [np.resize(keys[bucket == b][:40], want[b] - (bucket == b).sum()) for b in range(1024)]
+    keys = np.concatenate([keys, np.concatenate(more)[rng.permutation(n - unique)]])
+    grads = _grid(rng, (n, 4))
+    u, inv, sums = api.dedup_sum(splitmix64(keys.astype(np.uint64)), grads)
+    assert np.array_equal(inv, keys)
+    assert np.array_equal(sums, _sums(keys, grads, u.size))
+
+
 # 39 rows of one bucket 1000 times each: lists of some 5000 entries are taken by ranges of keys; two rows of
 # one bucket, the second of which leaves three entries in each of a thousand chunks, more than the
 # 2048 that fit at once: window by window. dim 300: a row is more than a wavefront holds
