@@ -7,8 +7,8 @@
 // go on in the next chunk: it adds its runs up and leaves a list, one entry for a run's sum, the pairs
 // themselves for the shortest runs. The workgroup that is through last with a cut bucket
 // merges: the chunks' lists, in order, are what the bucket's pairs were before, with few entries.
-// Lists that do not fit into LDS at once (buckets of many cold rows) are taken by ranges of keys,
-// and a single row whose entries do not fit in windows. No workgroup waits for another.
+// Lists that do not fit into LDS at once (buckets of many cold rows) are sorted in memory, over the pairs,
+// and taken a window at a time. No workgroup waits for another.
 //
 // Who adds a run up depends on its length: a lane group (up to 16 entries, the reference's order
 // exactly), a wavefront, or the whole workgroup, whose lane groups add a stretch each and the
@@ -36,8 +36,8 @@ constexpr int kRunBits = 8;                            // of a digit of the sort
 constexpr int kShortest = 16;                          // runs up to this length: one lane group each
 // What a chunk of a cut bucket adds up before the merge: runs of this many entries on. A row that is not
 // the hottest of its bucket may have a few entries in each of hundreds of chunks; passed on one by
-// one, a row with 16 of them in 256 chunks did not fit into the merge's LDS, and taking the lists by
-// ranges of keys then made a reduction of 155 us one of 674. Fewer than four cost little to pass on,
+// one, a row with 16 of them in 256 chunks did not fit into the merge's LDS, which made a
+// reduction of 155 us one of 674. Fewer than four cost little to pass on,
 // and every one of them less would take more room for sums (a row for this many pairs).
 constexpr int kCutSum = 4;
 constexpr int kPerGroup = 16;                          // a wavefront takes runs of up to this many entries per lane group
@@ -53,7 +53,7 @@ struct RunLds {
   uint32_t ref[kListMax];
   // the sort's histogram [wave][digit], then a long run's partial sums [wave][up to 256 floats]
   alignas(16) uint32_t work[kWaves << kRunBits];
-  uint16_t start[kListMax + 2];                        // first entry of every run
+  alignas(4) uint16_t start[kListMax + 2];             // first entry of every run
   uint16_t long_run[kLong], wave_run[kLong];
   uint32_t wave_total[kWaves];
   uint32_t n_long, n_wave, last;
@@ -73,8 +73,8 @@ struct Member {
 };
 
 struct RunArgs {
-  const uint32_t* h;             // pairs in bucket order
-  const uint32_t* refs;
+  uint32_t* h;                   // pairs in bucket order
+  uint32_t* refs;
   uint32_t* list_h;              // the lists of cut buckets' chunks, each where its pairs lie
   uint32_t* list_refs;
   float* sums;                   // sums of long runs of cut buckets
@@ -104,13 +104,13 @@ __device__ __forceinline__ uint32_t run_scan(uint32_t v, uint32_t* wave_total, u
   return offset;
 }
 
-// Stable sort of the first len pairs by the low `bits` bits of the key. (All lanes; the pairs
+// Stable sort of the first len pairs by `bits` bits of the key from bit `from` on. (All lanes; the pairs
 // need not be visible yet.)
-__device__ __forceinline__ void sort_list(RunLds& s, int len, int bits) {
+__device__ __forceinline__ void sort_list(RunLds& s, int len, int bits, int from = 0) {
   const int t = threadIdx.x;
   const int lane = t & (kWave - 1);
   const int wave = t / kWave;
-  const uint32_t key_mask = (1u << bits) - 1u;         // (bits: fewer than 32)
+  const uint32_t key_mask = ((1u << bits) - 1u) << from;   // (from + bits: fewer than 32)
   const int per_lane = (len + kLanes - 1) / kLanes;    // 1..kListItems
   for (int j = len + t; j < per_lane * kLanes; j += kLanes) {
     s.key[j] = 0xFFFFFFFFu;                            // padding: the largest digit of every pass, behind its equals
@@ -129,7 +129,7 @@ __device__ __forceinline__ void sort_list(RunLds& s, int len, int bits) {
   uint32_t* hist = s.work;                             // [kWaves][digits]
   const int wbase = wave * kWave * per_lane + lane;
   for (int pass = 0; pass < passes; ++pass) {
-    const int shift = pass * width;
+    const int shift = from + pass * width;
     uint32_t key[kListItems], ref[kListItems], rank[kListItems];
 #pragma unroll
     for (int i = 0; i < kListItems; ++i) {
@@ -596,119 +596,217 @@ __device__ __forceinline__ void load_members(Member* lds, const RunArgs& a, cons
 
 constexpr int kOffsets = kWaves << kRunBits;           // lists whose offsets are held at a time, in `work`
 
+// Sorts `n` entries by the low `bits` bits of their keys, where they do not fit into LDS: a digit at a time,
+// from (h, refs) to (list_h, list_refs) and back, stable. Tiles of kListMax entries are sorted by the
+// digit in LDS and appended to their digits' stretches. One workgroup, which is the only one that
+// touches these entries by now. Returns whether the result lies in (list_h, list_refs).
+__device__ __forceinline__ bool sort_far(RunLds& s, const RunArgs& a, uint32_t begin, uint32_t n, int bits) {
+  const int t = threadIdx.x;
+  const int passes = (bits + kRunBits - 1) / kRunBits;
+  const int width = (bits + passes - 1) / passes;
+  const uint32_t digit_mask = (1u << width) - 1u;
+  static_assert((1 << kRunBits) == kLanes && sizeof(s.start) >= 2 * kLanes * sizeof(uint32_t), "a digit a lane");
+  uint32_t* next = reinterpret_cast<uint32_t*>(s.start);   // where a digit's next entry goes
+  uint32_t* first = next + kLanes;                         // where its entries begin in the tile
+  for (int pass = 0; pass < passes; ++pass) {
+    const int shift = pass * width;
+    const bool back = pass & 1;
+    const uint32_t* src_h = (back ? a.list_h : a.h) + begin;
+    const uint32_t* src_refs = (back ? a.list_refs : a.refs) + begin;
+    uint32_t* dst_h = (back ? a.h : a.list_h) + begin;
+    uint32_t* dst_refs = (back ? a.refs : a.list_refs) + begin;
+    s.work[t] = 0u;
+    lds_barrier();
+    for (uint32_t j = (uint32_t)t; j < n; j += kLanes) atomicAdd(&s.work[(src_h[j] >> shift) & digit_mask], 1u);
+    lds_barrier();
+    uint32_t all;
+    const uint32_t at = run_scan(s.work[t], s.wave_total, all);
+    next[t] = at;
+    for (uint32_t j0 = 0; j0 < n; j0 += kListMax) {
+      const int len = (int)min((uint32_t)kListMax, n - j0);
+      for (int j = t; j < len; j += kLanes) {
+        s.key[j] = src_h[j0 + j];
+        s.ref[j] = src_refs[j0 + j];
+      }
+      sort_list(s, len, width, shift);
+      for (int j = t; j < len; j += kLanes) {
+        const uint32_t d = (s.key[j] >> shift) & digit_mask;
+        if (j == 0 || ((s.key[j - 1] >> shift) & digit_mask) != d) first[d] = (uint32_t)j;
+      }
+      lds_barrier();
+      for (int j = t; j < len; j += kLanes) {
+        const uint32_t d = (s.key[j] >> shift) & digit_mask;
+        const uint32_t to = next[d] + (uint32_t)j - first[d];
+        dst_h[to] = s.key[j];
+        dst_refs[to] = s.ref[j];
+      }
+      lds_barrier();
+      for (int j = t; j < len; j += kLanes) {
+        const uint32_t d = (s.key[j] >> shift) & digit_mask;
+        if (j == len - 1 || ((s.key[j + 1] >> shift) & digit_mask) != d) next[d] += (uint32_t)j + 1u - first[d];
+      }
+      lds_barrier();                                      // the next tile overwrites the entries
+    }
+    __syncthreads();                                      // the entries are where the next pass reads them
+  }
+  return passes & 1;
+}
+
 // Merges the lists of a cut bucket. weights: LDS for the entries' weights (pooled requests).
+// Entries that do not fit into LDS are sorted in memory and taken a window at a time; every step is linear
+// in the entries, whatever rows they are of. Gathering the lists again for every range of keys that fits
+// walked all of them each time: pushes of 16,384 and of 65,536 pairs, all of one bucket's 16,384 rows of
+// four floats, took 1.4 and 18 ms and take 0.53 and 1.5; of 2^20 pairs 24-34. The sort of such a
+// request takes 0.05 to 0.16, but only rows as far apart as the multiplier's inverse share a bucket like
+// this: of rows 1 to 4096 apart, in tables of 2^16 to 2^25 rows, none holds more than 2.1 times the average.
 template <int OPT, int VEC, int FROM, bool GROUPED>
 __device__ __forceinline__ void merge_lists(const Reducer<OPT, VEC, FROM, GROUPED, true>& r, const RunArgs& a,
                                             const CutBucket& cut, float* weights, const uint32_t* bag_of) {
   RunLds& s = r.s;
   const int t = threadIdx.x;
-  const uint32_t low_mask = r.low_mask, range = low_mask + 1u;
   const uint32_t pieces = a.cut.pieces(cut.len);
   uint32_t* offs = s.work;
+  constexpr int kOwn = kOffsets / kLanes;
 
-  // Brings the lists' entries with places in [from, from + width) into LDS, in list order: those from
-  // number `skip` on, as many as fit. Returns how many there are.
-  auto gather = [&](uint32_t from, uint32_t width, uint32_t skip) -> uint32_t {
-    uint32_t seen = 0;
-    for (uint32_t c0 = 0; c0 < pieces; c0 += kOffsets) {
-      const uint32_t here = min((uint32_t)kOffsets, pieces - c0);
-      constexpr int kOwn = kOffsets / kLanes;
-      const int own = (int)((here + kLanes - 1) / kLanes);   // 1..kOwn
-      uint32_t n[kOwn], sum = 0, total;
+  // Where lists [c0, c0 + kOffsets) begin among these lists' entries, into offs; how many entries they are.
+  auto offsets = [&](uint32_t c0) -> uint32_t {
+    const uint32_t here = min((uint32_t)kOffsets, pieces - c0);
+    const int own = (int)((here + kLanes - 1) / kLanes);   // 1..kOwn
+    uint32_t n[kOwn], sum = 0, total;
 #pragma unroll
-      for (int k = 0; k < kOwn; ++k) {
-        const uint32_t c = (uint32_t)(t * own + k);
-        n[k] = k < own && c < here ? shared_word(a.plan.count + cut.base + c0 + c) : 0u;
-        sum += n[k];
-      }
-      uint32_t at = run_scan(sum, s.wave_total, total);
-#pragma unroll
-      for (int k = 0; k < kOwn; ++k) {
-        if (k < own) offs[t * own + k] = at;
-        at += n[k];
-      }
-      lds_barrier();
-      constexpr int kTake = 4;                         // entries a lane takes a trip, side by side
-      for (uint32_t e0 = 0; e0 < total; e0 += kLanes * kTake) {
-        uint32_t key[kTake], ref[kTake], in = 0;
-#pragma unroll
-        for (int k = 0; k < kTake; ++k) {
-          const uint32_t e = e0 + (uint32_t)(t * kTake + k);
-          if (e < total) {
-            uint32_t c = 0, hi = here;                 // the last list that begins at or before e
-            while (hi - c > 1) {
-              const uint32_t mid = (c + hi) / 2;
-              if (offs[mid] <= e) c = mid; else hi = mid;
-            }
-            const uint32_t idx = cut.begin + (c0 + c) * a.cut.chunk + (e - offs[c]);
-            key[k] = shared_word(a.list_h + idx);
-            ref[k] = shared_word(a.list_refs + idx);
-          }
-        }
-#pragma unroll
-        for (int k = 0; k < kTake; ++k)
-          if (e0 + (uint32_t)(t * kTake + k) < total && (key[k] & low_mask) - from < width) in |= 1u << k;
-        uint32_t got;
-        uint32_t p = seen + run_scan((uint32_t)__popc(in), s.wave_total, got);
-#pragma unroll
-        for (int k = 0; k < kTake; ++k) {
-          if (in & (1u << k)) {
-            if (p >= skip && p - skip < (uint32_t)kListMax) {
-              s.key[p - skip] = key[k];
-              s.ref[p - skip] = ref[k];
-            }
-            ++p;
-          }
-        }
-        seen += got;
-      }
-      lds_barrier();                                      // the offsets have been read
+    for (int k = 0; k < kOwn; ++k) {
+      const uint32_t c = (uint32_t)(t * own + k);
+      n[k] = k < own && c < here ? shared_word(a.plan.count + cut.base + c0 + c) : 0u;
+      sum += n[k];
     }
-    return seen;
+    uint32_t at = run_scan(sum, s.wave_total, total);
+#pragma unroll
+    for (int k = 0; k < kOwn; ++k) {
+      if (k < own) offs[t * own + k] = at;
+      at += n[k];
+    }
+    lds_barrier();
+    return total;
   };
-
-  uint32_t from = 0, width = range;
-  while (from < range) {                               // uniform
-    const uint32_t entries = gather(from, width, 0u);
-    if (entries > (uint32_t)kListMax && width > 1u) {
-      width >>= 1;
+  uint32_t entries = 0;
+  for (uint32_t c0 = 0; c0 < pieces; c0 += kOffsets) {
+    entries += offsets(c0);
+    lds_barrier();
+  }
+  const bool fits = entries <= (uint32_t)kListMax;     // uniform
+  // the lists' entries, in list order, into LDS or over the bucket's pairs, which have been read
+  for (uint32_t c0 = 0, before = 0; c0 < pieces; c0 += kOffsets) {
+    const uint32_t here = min((uint32_t)kOffsets, pieces - c0);
+    const uint32_t total = offsets(c0);
+    constexpr int kTake = 4;                           // entries a lane takes a trip
+    for (uint32_t e0 = 0; e0 < total; e0 += kLanes * kTake) {
+      uint32_t key[kTake], ref[kTake];
+#pragma unroll
+      for (int k = 0; k < kTake; ++k) {
+        const uint32_t e = e0 + (uint32_t)(k * kLanes + t);
+        if (e < total) {
+          uint32_t c = 0, hi = here;                   // the last list that begins at or before e
+          while (hi - c > 1) {
+            const uint32_t mid = (c + hi) / 2;
+            if (offs[mid] <= e) c = mid; else hi = mid;
+          }
+          const uint32_t idx = cut.begin + (c0 + c) * a.cut.chunk + (e - offs[c]);
+          key[k] = shared_word(a.list_h + idx);
+          ref[k] = shared_word(a.list_refs + idx);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < kTake; ++k) {
+        const uint32_t e = e0 + (uint32_t)(k * kLanes + t);
+        if (e < total) {
+          if (fits) {
+            s.key[before + e] = key[k];
+            s.ref[before + e] = ref[k];
+          } else {
+            a.h[cut.begin + before + e] = key[k];
+            a.refs[cut.begin + before + e] = ref[k];
+          }
+        }
+      }
+    }
+    before += total;
+    lds_barrier();                                        // the offsets have been read
+  }
+  if (fits) {
+    sort_list(s, (int)entries, r.low);
+    const uint32_t runs = r.find_runs((int)entries);
+    r.resolve_weights((int)entries, weights, bag_of);
+    r.reduce(runs, false, 0u);
+    return;
+  }
+  __syncthreads();                                        // the entries are in memory
+  const bool in_lists = sort_far(s, a, cut.begin, entries, r.low);
+  const uint32_t* sorted_h = (in_lists ? a.list_h : a.h) + cut.begin;
+  const uint32_t* sorted_refs = (in_lists ? a.list_refs : a.refs) + cut.begin;
+  auto window = [&](uint32_t from) -> int {
+    const int len = (int)min((uint32_t)kListMax, entries - from);
+    for (int j = t; j < len; j += kLanes) {
+      s.key[j] = sorted_h[from + j];
+      s.ref[j] = sorted_refs[from + j];
+    }
+    lds_barrier();
+    return len;
+  };
+  for (uint32_t from = 0; from < entries;) {           // uniform
+    int len = window(from);
+    uint32_t runs = r.find_runs(len);
+    bool whole_window = false;                         // of one row, which may go on behind it
+    if (from + (uint32_t)len < entries) {
+      if (runs > 1u) {                                 // the last row may go on: the next window's first
+        len = s.start[runs - 1u];
+        lds_barrier();
+        runs = r.find_runs(len);
+      } else {
+        whole_window = true;
+      }
+    }
+    if (!whole_window) {
+      r.resolve_weights(len, weights, bag_of);
+      r.reduce(runs, false, 0u);
+      lds_barrier();                                      // the next window overwrites the entries
+      from += (uint32_t)len;
       continue;
     }
-    if (entries > (uint32_t)kListMax) {
-      // one row: window by window, the first lane group keeps the sum
-      const int gl = t & (a.group - 1);
-      for (int e0 = 0; e0 < a.elems; e0 += a.group) {
-        const int e = e0 + gl;
-        const bool on = e < a.elems;
-        float sum[VEC] = {};
-        uint32_t of = 0;
-        for (uint32_t skip = 0; skip < entries; skip += kListMax) {
-          gather(from, width, skip);
-          const int len = (int)min((uint32_t)kListMax, entries - skip);
-          r.resolve_weights(len, weights, bag_of);
-          of = r.key_of(0);
-          float acc[VEC];
-          r.sum_block(of, 0, len, e, on, gl, acc);
-#pragma unroll
-          for (int c = 0; c < VEC; ++c) sum[c] = skip == 0 ? acc[c] : sum[c] + acc[c];
-          lds_barrier();                                  // the next window overwrites the entries
-        }
-        if (t < a.group) {
-          RowRegs<VEC> rec{};
-          r.load(of, e, on, rec);
-          r.finish(of, sum, e, on, gl, e0 + a.group >= a.elems, rec);
-        }
-      }
-    } else if (entries > 0) {
-      sort_list(s, (int)entries, r.low);
-      const uint32_t runs = r.find_runs((int)entries);
-      r.resolve_weights((int)entries, weights, bag_of);
-      r.reduce(runs, false, 0u);
-      lds_barrier();                                      // the next range overwrites the entries
+    const uint32_t of_place = s.key[0] & r.low_mask;
+    uint32_t end = from + (uint32_t)len;               // of the row's entries
+    while (end < entries) {
+      lds_barrier();
+      len = window(end);
+      runs = r.find_runs(len);
+      const uint32_t more = (s.key[0] & r.low_mask) != of_place ? 0u : runs > 1u ? (uint32_t)s.start[1] : (uint32_t)len;
+      end += more;
+      if (more < (uint32_t)len) break;                 // uniform
     }
-    // ranges are the nodes of a binary tree over the places: the largest that begins here comes next
-    from += width;
-    width = from & (0u - from);
+    // window by window, the first lane group keeps the sum
+    const int gl = t & (a.group - 1);
+    for (int e0 = 0; e0 < a.elems; e0 += a.group) {
+      const int e = e0 + gl;
+      const bool on = e < a.elems;
+      float sum[VEC] = {};
+      uint32_t of = 0;
+      for (uint32_t at = from; at < end; at += kListMax) {
+        lds_barrier();                                    // the last window has been read
+        len = min(window(at), (int)(end - at));
+        r.resolve_weights(len, weights, bag_of);
+        of = r.key_of(0);
+        float acc[VEC];
+        r.sum_block(of, 0, len, e, on, gl, acc);
+#pragma unroll
+        for (int c = 0; c < VEC; ++c) sum[c] = at == from ? acc[c] : sum[c] + acc[c];
+      }
+      if (t < a.group) {
+        RowRegs<VEC> rec{};
+        r.load(of, e, on, rec);
+        r.finish(of, sum, e, on, gl, e0 + a.group >= a.elems, rec);
+      }
+    }
+    lds_barrier();
+    from = end;
   }
 }
 

@@ -77,7 +77,7 @@ def test_dedup_sum_whole_and_cut_buckets(api):
     assert np.array_equal(sums, _sums(keys, grads, u.size))
 
 
-# 39 rows of one bucket 1000 times each: lists of some 5000 entries are taken by ranges of keys; two rows of
+# 39 rows of one bucket 1000 times each: lists of some 5000 entries are sorted in memory; two rows of
 # one bucket, the second of which leaves three entries in each of a thousand chunks, more than the
 # 2048 that fit at once: window by window. dim 300: a row is more than a wavefront holds
 @pytest.mark.parametrize("n", [80_000, 2**20])
@@ -94,6 +94,26 @@ def test_dedup_sum_crowded_bucket(api, n, dim):
     u, inv, sums = api.dedup_sum(splitmix64(keys.astype(np.uint64)), grads)
     assert np.array_equal(inv, keys)
     assert np.array_equal(sums, _sums(keys, grads, u.size))
+
+
+# rows whose hash is the same in its upper eight bits: every chunk's list is as long as the chunk, and their
+# 13,000 entries, or 4096 with a few to a row's run, are sorted in memory by three digits (2^25 rows of room)
+@pytest.mark.parametrize("rows", [2049, 26])
+def test_rows_of_one_bucket(api, rows):
+    rng = np.random.default_rng(rows)
+    t = api.SparseTable(4, api.Initializer.create(api.InitializerType.kConstant, {"value": "1"}))
+    t.reserve((1 << 25) - 64)
+    names = splitmix64(np.arange(700_000, dtype=np.uint64))
+    t.Pull(names)
+    bucket = _bucket(t.lookup(names), 25, 8)
+    names = names[bucket == np.bincount(bucket.astype(np.int64)).argmax()][:rows]
+    assert names.size == rows
+    for n in (13_000, 30_000):
+        inv = rng.permutation(np.arange(n) % rows)
+        grads = _grid(rng, (n, 4))
+        before = t.Pull(names)[1]
+        assert t.PushRaw(api.Optim.create(api.OptimType.kSGD), names[inv], grads, 0.5) == 0
+        assert np.array_equal(t.Pull(names)[1], before - np.float32(0.5) * _sums(inv, grads, rows))
 
 
 # up to 2048 ids a table every bucket's workgroup picks its pairs out of the request, one to eight a lane; a
