@@ -468,6 +468,7 @@ struct krk_sparse : krk::ObjBase {
   uint32_t* host_inserted = nullptr;        // pinned, behind host_pub: set by pulls that insert
   int64_t last_request = 0;           // size of the latest large inserting requests
   int64_t pub_rows = 0;               // rows at the last published count that was looked at
+  int behind_for = 0;                 // requests for which the host still counts as ahead of the device
   uint64_t enq_total = 0;             // ids handed to inserting launches so far
   uint64_t enq_at[256] = {};          // enq_total right after the launch with number e (mod 256)
   uint32_t epoch = 0;                 // number of the last launch that could insert
@@ -655,7 +656,7 @@ int32_t sparse_finish_begin(krk_sparse* t, uint32_t flags);
 int32_t sparse_finish_end(krk_sparse* t, uint32_t flags);
 // A new launch number for a launch that may insert up to n rows into t; call right before it.
 int32_t sparse_next_epoch(krk_sparse* t, int64_t n);
-// True when only a few more requests like the last one fit under the current row bound.
+// Whether the pull that has just been enqueued should publish the table's row count.
 bool sparse_wants_publish(const krk_sparse* t);
 // Enqueues the kernel that publishes {rows used, launch number} of each table to the host.
 int32_t sparse_publish(krk_sparse* const* tables, int n, hipStream_t stream);

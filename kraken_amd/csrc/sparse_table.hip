@@ -1724,6 +1724,15 @@ static uint64_t pow2_at_least(uint64_t x) {
   return c;
 }
 
+// Requests that should still fit when a count is asked for: two, or three while the host is ahead of the
+// device, which it is for the next kBehindFor requests after it had to wait for a count. With three, two
+// requests are still in the stream when the host waits for the third, and the stream does not run dry;
+// a host that is the slower one never waits, and a count more often is a launch. 16,384 ids of 128
+// floats a pull, nothing else, with room for 3.2 / 4.2 / 9.2 requests, us: always two 12.7 / 10.7 / 8.1,
+// three 8.4 / 7.6 / 6.7, in every pull below four 8.2 / 8.1 / 7.7; pull and push of 2048 ids of 16 floats, bound by
+// the host, room for 3.2: 12.0 / 14.4 / 14.
+constexpr int kBehindFor = 32;
+static int64_t publish_lead(const krk_sparse* t) { return t->behind_for > 0 ? 3 : 2; }
 // Rows a table has room for beyond its bound.
 static int64_t room_left(const krk_sparse* t) {
   return std::min<int64_t>(t->row_cap, (int64_t)(t->slot_cap / 2)) - t->size_ub;
@@ -1752,6 +1761,7 @@ static void await_published(krk_sparse* t, int64_t extra_rows) {
     const int64_t need = t->size_ub + extra_rows;
     if (need <= t->row_cap && (uint64_t)need * 2 <= t->slot_cap) break;
     if ((uint32_t)(__atomic_load_n(t->host_pub, __ATOMIC_ACQUIRE) >> 32) == t->pub_epoch) break;
+    t->behind_for = kBehindFor;
     if (hipStreamQuery(t->stream) != hipErrorNotReady) break;
     std::this_thread::yield();
   }
@@ -1760,7 +1770,8 @@ static void await_published(krk_sparse* t, int64_t extra_rows) {
 
 // Room for `extra_rows` more rows: records, row keys, and an index at most half full.
 int32_t sparse_ensure_room(krk_sparse* t, int64_t extra_rows) {
-  if (room_left(t) < 2 * t->last_request) tighten_bound(t);
+  if (t->behind_for > 0) --t->behind_for;
+  if (room_left(t) < publish_lead(t) * t->last_request) tighten_bound(t);
   int64_t need = t->size_ub + extra_rows;
   if (need > t->row_cap || (uint64_t)need * 2 > t->slot_cap) {
     await_published(t, extra_rows);
@@ -1804,17 +1815,17 @@ int32_t sparse_next_epoch(krk_sparse* t, int64_t n) {
 }
 
 // Whether the pull that has just been enqueued should publish its count: where the bound leaves less than
-// two requests (of the size of the latest large ones), unless the count that is on its way already,
+// publish_lead requests (of the size of the latest large ones), unless the count that is on its way already,
 // when it has arrived, leaves that much. A table that is nearly full, as a trained one is, published in
 // every pull, a launch of 2-5 us on the device and 3 us of the host; with room for five more
 // requests one pull in four does. (Rows that were made since the last count are not in the estimate:
 // then the bound is refreshed by waiting, once.)
 bool sparse_wants_publish(const krk_sparse* t) {
   const int64_t room = room_left(t);
-  if (room >= 2 * t->last_request) return false;
+  if (room >= publish_lead(t) * t->last_request) return false;
   if (t->pub_epoch == 0 || t->epoch - t->pub_epoch >= 256) return true;
   const int64_t since = (int64_t)(t->enq_total - t->enq_at[t->pub_epoch & 255]);
-  return t->pub_rows + since + 2 * t->last_request > room + t->size_ub;
+  return t->pub_rows + since + publish_lead(t) * t->last_request > room + t->size_ub;
 }
 
 int32_t sparse_publish(krk_sparse* const* tables, int n, hipStream_t stream) {

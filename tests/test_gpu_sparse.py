@@ -603,3 +603,33 @@ def test_host_arguments_around_the_bounce_limit(api, n):
     assert np.array_equal(host.Pull(ids)[1], dev.Pull(ids)[1])
     missing = np.array([10**9], np.uint64)
     assert host.Push(opt, missing, grads[:1], 0.1) == api.SPARSE_ID_NOT_EXIST
+
+
+# The host learns a nearly full table's row count from its pulls, asked for with two requests to go, or three
+# while the host has had to wait; 1 to 6 requests fit behind the rows.
+@pytest.mark.parametrize("room", [1.2, 2.2, 3.2, 6.2])
+@pytest.mark.parametrize("n", [64, 3000])
+def test_pulls_without_waiting_from_a_nearly_full_table(api, room, n):
+    rows, dim = 20 * n, 16
+    gi = api.Initializer.create(api.InitializerType.kNormal, {"stddev": "1", "seed": "3"})
+    t = api.SparseTable(dim, gi)
+    t.reserve(rows + int(room * n))
+    for lo in range(0, rows, n):
+        assert t.Pull(splitmix64(np.arange(lo, lo + n, dtype=np.uint64)))[0] == 0
+    rng = np.random.default_rng(n)
+    batches, made = [], rows
+    for step in range(120):
+        ids = rng.integers(0, made, n).astype(np.uint64)
+        if step % 7 == 0:                                  # a few new rows; the last steps outgrow the table
+            fresh = max(1, n // 8) if step > 100 else 1
+            ids[:fresh] = np.arange(made, made + fresh)
+            made += fresh
+        batches.append(splitmix64(ids))
+    d = [api.DeviceArray.from_host(b) for b in batches]
+    outs = [api.DeviceArray((n, dim), np.float32) for _ in batches]
+    for i, o in zip(d, outs):
+        assert t.Pull(i, out=o, async_=True)[0] == 0
+    assert t.sync() == 0
+    assert len(t) == made
+    for b, o in zip(batches, outs):
+        assert np.array_equal(o.to_host(), t.Pull(b)[1])
