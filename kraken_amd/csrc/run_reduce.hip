@@ -1101,7 +1101,7 @@ RunHash make_hash(int bucket_bits, uint64_t keys) {
   return h;
 }
 
-// Buckets and chunks of a request, and where its work space lies.
+// Buckets and chunks of a request, and what its plan takes.
 struct RunShape {
   int bucket_bits;
   RunCut cut;
@@ -1110,18 +1110,33 @@ struct RunShape {
     bucket_bits = bucket_bits_for(n);
     cut = RunCut{whole_for(n, bucket_bits), chunk_for(n)};
     buckets = (size_t)1 << bucket_bits;
-    cuts = (size_t)(n / cut.whole);      // a cut bucket holds more than that
-    chunks = (size_t)(n / cut.chunk) + cuts;
+    cuts = (size_t)(n / cut.chunk);      // a cut bucket holds more than that, in at most twice as many chunks
+    chunks = 2 * cuts;
   }
+  size_t plan_words() const { return 4 * cuts + 4 + (buckets + 1) + cuts + chunks; }
 };
+// The longest requests of a form that takes more work space than the next one does: small tiles of the
+// partition, short chunks.
+constexpr int64_t kShapeEdges[] = {(int64_t)1 << 16, (int64_t)1 << 18};
 
 }  // namespace
 
 int32_t reserve_runs(const ReduceShape& sh, DeviceBuffer* scratch, int64_t n) {
   const RunShape r(n);
+  size_t partition = partition_work_bytes(n, r.bucket_bits), plan = r.plan_words();
+  for (const int64_t edge : kShapeEdges) {
+    if (edge >= n) break;
+    // so that a shorter request that follows finds its room there: freeing waits for the device
+    const RunShape shorter(edge);
+    partition = std::max(partition, partition_work_bytes(edge, shorter.bucket_bits));
+    plan = std::max(plan, shorter.plan_words());
+  }
   KRK_TRY(scratch[0].reserve(4 * (size_t)n * sizeof(uint32_t)));   // keys, payload, and as much again
-  KRK_TRY(scratch[1].reserve(partition_work_bytes(n, r.bucket_bits)));
-  KRK_TRY(scratch[2].reserve((4 * r.cuts + 4 + (r.buckets + 1) + r.cuts + r.chunks) * sizeof(uint32_t)));
+  KRK_TRY(scratch[1].reserve(partition));
+  KRK_TRY(scratch[2].reserve(plan * sizeof(uint32_t)));
+  // The sum of a run of kCutSum entries lies where the run's first pair does, divided by kCutSum: which
+  // buckets are cut is known on the device only, so there is room for all (134 MB for 2^20 pairs of 128 floats,
+  // a quarter of their gradient rows).
   return scratch[3].reserve(r.cuts ? (size_t)(n / kCutSum + 1) * (size_t)sh.dim * sizeof(float) : 0);
 }
 
