@@ -22,12 +22,21 @@ struct krk_dense : krk::ObjBase {
   bool sgd_started = false;          // momentum buffer exists (first update copies the gradient)
   hipStream_t own_stream = nullptr;  // the stream created with the table (a group lends its own)
   krk_dense_group* member_of = nullptr;
+  float** group_state = nullptr;     // where the group's descriptor of this table keeps `state` (device)
 };
+
+namespace krk {
+struct DenseDesc;
+struct DenseBlock;
+}
 
 // The dense tables of one combined request: they share one stream, and one launch serves all.
 struct krk_dense_group : krk::ObjBase {
   std::vector<krk_dense*> tables;
   std::vector<int64_t> start;        // where each member begins in the concatenated arrays
+  std::vector<uint32_t> block_start; // the members' workgroups of a launch over all of them, and their number
+  krk::DenseDesc* descs = nullptr;   // device: a descriptor per member
+  const krk::DenseBlock* blocks = nullptr;   // behind them: one per workgroup
   int64_t total = 0;
   hipStream_t own_stream = nullptr;
 };
@@ -95,63 +104,128 @@ static unsigned dense_grid(int64_t n) {
   return (unsigned)blocks;
 }
 
-static int32_t ensure_state(krk_dense* t, int st) {
+// State columns that were created, to be entered in the descriptors of a group (in the order of its stream).
+// A launch takes many: the first push of 40 tables under Adam creates 80.
+constexpr int kEntries = 200;
+struct StateEntries {
+  float** at[kEntries];
+  float* value[kEntries];
+};
+static_assert(sizeof(StateEntries) + 16 <= 4096, "the arguments of one launch");
+__global__ void enter_states_kernel(StateEntries e, int n) {
+  const int i = threadIdx.x;
+  if (i < n) *e.at[i] = e.value[i];
+}
+struct StateList {
+  hipStream_t stream = nullptr;
+  int n = 0;
+  StateEntries e;
+  int32_t flush() {
+    if (n == 0) return KRK_SUCCESS;
+    hipLaunchKernelGGL(enter_states_kernel, dim3(1), dim3(256), 0, stream, e, n);
+    KRK_HIP(hipGetLastError());
+    n = 0;
+    return KRK_SUCCESS;
+  }
+};
+
+static int32_t ensure_state(krk_dense* t, int st, StateList* list) {
   if (t->state[st]) return KRK_SUCCESS;
   DeviceGuard guard;
   KRK_HIP(hipMalloc(&guard.p, (size_t)(t->n ? t->n : 1) * sizeof(float)));
   KRK_HIP(hipMemsetAsync(guard.p, 0, (size_t)t->n * sizeof(float), t->stream));
+  if (t->group_state) {   // (a member's stream is the group's)
+    if (list->n == kEntries) KRK_TRY(list->flush());
+    list->e.at[list->n] = t->group_state + st;
+    list->e.value[list->n++] = reinterpret_cast<float*>(guard.p);
+  }
   t->state[st] = guard.release<float>();   // only a zeroed column counts as present
   return KRK_SUCCESS;
 }
 
+// The states an optimizer's three slots stand for (krk_internal.h), -1 = unused.
+static void dense_slots(const krk_optim& o, int32_t st[3]) {
+  st[0] = st[1] = st[2] = -1;
+  switch (o.type) {
+    case KRK_SGD:
+      if (o.has_momentum) st[0] = KRK_ST_MOMENTUM_BUFFER;
+      break;
+    case KRK_ADAGRAD:
+      st[0] = KRK_ST_STATE_SUM;
+      break;
+    case KRK_ADAM:
+      st[0] = KRK_ST_FIRST_MOMENT;
+      st[1] = KRK_ST_SECOND_MOMENT;
+      if (o.amsgrad) st[2] = KRK_ST_SECOND_MOMENT_MAX;
+      break;
+    default:
+      st[0] = KRK_ST_SQUARE_AVERAGE;
+      if (o.centered) st[1] = KRK_ST_G_AVE;
+      if (o.has_momentum) st[2] = KRK_ST_MOMENTUM_BUFFER;
+      break;
+  }
+}
+
+// Creates the columns of the states st (-1: none) that n tables of one stream, those with elements, lack. What could be created
+// is entered also where a later one could not.
+static int32_t ensure_states(krk_dense* const* tables, size_t n, const int32_t* st, int n_st, hipStream_t stream) {
+  int32_t rc = KRK_SUCCESS;
+  StateList list;
+  list.stream = stream;
+  for (size_t i = 0; i < n && rc == KRK_SUCCESS; ++i)
+    for (int k = 0; k < n_st && rc == KRK_SUCCESS; ++k)
+      if (st[k] >= 0 && tables[i]->n > 0 && !tables[i]->state[st[k]]) rc = ensure_state(tables[i], st[k], &list);
+  const int32_t entered = list.flush();
+  return rc != KRK_SUCCESS ? rc : entered;
+}
+
+// Adam's bias corrections of a step (ps/optim/adam.cc:61-64) and SGD's first momentum update.
+struct DenseStep {
+  float bc1, bc2;
+  bool first;        // SGD with momentum: the buffer does not exist yet
+};
+
+// The host's bookkeeping of one Optim::Update of table t: Adam's counter advanced, SGD's first momentum
+// step noted. last: the step of a table before, whose powers serve this one if the counts are the same.
+struct StepMemo {
+  int64_t steps = -1;
+  float bc1 = 1.0f, bc2 = 1.0f;
+};
+static DenseStep dense_step(krk_dense* t, const krk_optim& o, StepMemo* last) {
+  DenseStep s{1.0f, 1.0f, false};
+  if (o.type == KRK_SGD && o.has_momentum) {
+    s.first = !t->sgd_started;
+    t->sgd_started = true;
+  } else if (o.type == KRK_ADAM) {
+    const int64_t steps = ++t->steps;
+    if (steps != last->steps) {
+      last->steps = steps;
+      last->bc1 = (float)(1.0 - (double)std::pow(o.beta1, (float)steps));
+      last->bc2 = (float)(1.0 - (double)std::pow(o.beta2, (float)steps));
+    }
+    s.bc1 = last->bc1;
+    s.bc2 = last->bc2;
+  }
+  return s;
+}
+
+// What an update of one table reads and writes.
 struct DenseMember {
   float* w;
   float* s0;
   float* s1;
   float* s2;
   int64_t n;
-  int64_t start;     // first element in the concatenated arrays of a combined request
-  float bc1, bc2;    // Adam's bias corrections of this member's step
-  int32_t first;     // SGD with momentum: the buffer does not exist yet
+  DenseStep step;
 };
 
-// What one Optim::Update of table t reads and writes, with the host-side bookkeeping
-// of the update (state columns created, Adam's counter advanced, SGD's first momentum step noted).
 static int32_t dense_member(krk_dense* t, const krk_optim& o, DenseMember* m) {
-  const uint32_t mask = optim_state_mask(o);
-  for (int st = 1; st < KRK_ST_COUNT; ++st)
-    if (mask & (1u << st)) KRK_TRY(ensure_state(t, st));
-  m->w = t->w;
-  m->s0 = m->s1 = m->s2 = nullptr;
-  m->n = t->n;
-  m->bc1 = m->bc2 = 1.0f;
-  m->first = 0;
-  switch (o.type) {
-    case KRK_SGD:
-      if (o.has_momentum) {
-        m->s0 = t->state[KRK_ST_MOMENTUM_BUFFER];
-        m->first = t->sgd_started ? 0 : 1;
-        t->sgd_started = true;
-      }
-      break;
-    case KRK_ADAGRAD:
-      m->s0 = t->state[KRK_ST_STATE_SUM];
-      break;
-    case KRK_ADAM: {
-      m->s0 = t->state[KRK_ST_FIRST_MOMENT];
-      m->s1 = t->state[KRK_ST_SECOND_MOMENT];
-      if (o.amsgrad) m->s2 = t->state[KRK_ST_SECOND_MOMENT_MAX];
-      const int64_t steps = ++t->steps;   // ps/optim/adam.cc:61
-      m->bc1 = (float)(1.0 - (double)std::pow(o.beta1, (float)steps));
-      m->bc2 = (float)(1.0 - (double)std::pow(o.beta2, (float)steps));
-      break;
-    }
-    default:
-      m->s0 = t->state[KRK_ST_SQUARE_AVERAGE];
-      if (o.centered) m->s1 = t->state[KRK_ST_G_AVE];
-      if (o.has_momentum) m->s2 = t->state[KRK_ST_MOMENTUM_BUFFER];
-      break;
-  }
+  int32_t st[3];
+  dense_slots(o, st);
+  KRK_TRY(ensure_states(&t, 1, st, 3, t->stream));
+  StepMemo none;
+  const auto column = [&](int i) { return st[i] >= 0 ? t->state[st[i]] : nullptr; };
+  *m = DenseMember{t->w, column(0), column(1), column(2), t->n, dense_step(t, o, &none)};
   return KRK_SUCCESS;
 }
 
@@ -173,7 +247,7 @@ static int32_t dense_apply(krk_dense* t, const krk_optim& o, const float* d_grad
   const OptimK k = make_optim_k(o);
   with_optim(o.type, [&](auto opt) {
     hipLaunchKernelGGL((dense_update_kernel<opt.value>), dim3(dense_grid(t->n)), dim3(kDenseBlock), 0, t->stream, m.w,
-                       m.s0, m.s1, m.s2, d_grad, t->n, lr, k, m.first != 0, m.bc1, m.bc2, no_tiles());
+                       m.s0, m.s1, m.s2, d_grad, t->n, lr, k, m.step.first, m.step.bc1, m.step.bc2, no_tiles());
   });
   KRK_HIP(hipGetLastError());
   return KRK_SUCCESS;
@@ -238,7 +312,7 @@ __global__ __launch_bounds__(kDenseBlock) void coo_update_kernel(DenseMember m, 
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           ww[j] = w4[i][j]; a[j] = a4[i][j]; b[j] = b4[i][j]; c[j] = c4[i][j];
-          optim_element<OPT>(k, lr, g4[j], ww[j], a[j], b[j], c[j], m.first != 0, m.bc1, m.bc2);
+          optim_element<OPT>(k, lr, g4[j], ww[j], a[j], b[j], c[j], m.step.first, m.step.bc1, m.step.bc2);
         }
         dense_store(m.w, q, (dfloat4){ww[0], ww[1], ww[2], ww[3]});
         if (m.s0) dense_store(m.s0, q, (dfloat4){a[0], a[1], a[2], a[3]});
@@ -249,7 +323,7 @@ __global__ __launch_bounds__(kDenseBlock) void coo_update_kernel(DenseMember m, 
       for (int64_t i = base + threadIdx.x; i < m.n; i += kDenseBlock) {
         float ww = m.w[i];
         float a = m.s0 ? m.s0[i] : 0.0f, b = m.s1 ? m.s1[i] : 0.0f, c = m.s2 ? m.s2[i] : 0.0f;
-        optim_element<OPT>(k, lr, grad[i - base], ww, a, b, c, m.first != 0, m.bc1, m.bc2);
+        optim_element<OPT>(k, lr, grad[i - base], ww, a, b, c, m.step.first, m.step.bc1, m.step.bc2);
         m.w[i] = ww;
         if (m.s0) m.s0[i] = a;
         if (m.s1) m.s1[i] = b;
@@ -291,7 +365,7 @@ static int32_t dense_apply_coo(krk_dense* t, const krk_optim& o, const long long
   KRK_TRY(coo_scatter_if_unordered(tiles, d_idx, d_val, nnz, t->coo_grad, t->n, t->stream));
   with_optim(o.type, [&](auto opt) {
     hipLaunchKernelGGL((dense_update_kernel<opt.value>), dim3(dense_grid(t->n)), block, 0, t->stream, m.w, m.s0, m.s1,
-                       m.s2, t->coo_grad, t->n, lr, k, m.first != 0, m.bc1, m.bc2, tiles);
+                       m.s2, t->coo_grad, t->n, lr, k, m.step.first, m.step.bc1, m.step.bc2, tiles);
   });
   KRK_HIP(hipGetLastError());
   return KRK_SUCCESS;
@@ -324,59 +398,75 @@ __global__ __launch_bounds__(kDenseBlock) void dense_copy_kernel(const float* __
 // Ps::CombinePullDenseTable (ps/ps_op.cc:177-252) pulls every dense parameter of the model in one
 // request, and the worker does that after every step (pytorch/optimizer.py:151-173); one table per
 // launch makes a model with dozens of small tensors pay a launch per tensor. Here the members'
-// values (and, for the push, gradients) are one concatenated array in member order and a launch
-// takes up to kDenseGroupChunk members: workgroups [block_start[m], block_start[m + 1]) belong to
-// member m. 56 members and the other arguments come to just under the 4096 bytes a launch may carry;
-// a request of dozens of small tensors is bound by its launches (40 tensors of 434k parameters,
-// push + pull: 14.1 us as two launches each of 32 members at most, 9 us as one each).
-constexpr int kDenseGroupChunk = 56;
-static_assert(kDenseGroupChunk <= kWave, "a lane looks at each member");
-
-struct DenseGroupArgs {
-  int32_t members;
-  uint32_t block_start[kDenseGroupChunk + 1];
-  DenseMember m[kDenseGroupChunk];
+// values (and, for the push, gradients) are one concatenated array in member order, and a launch
+// serves all members that have elements.
+//
+// A request of dozens of small tensors is bound by the host's calls and by the trips to memory before a
+// workgroup knows what to load. What does not change from call to call lies on the device with the
+// group: a record per workgroup, which names its member, and a descriptor per member, in which a state
+// column is entered when it is created. As arguments of the launch (3.8 KB, put together and copied on
+// every call) they made a push and a pull of 40 tensors of 434k parameters take 11 us of the host, 6.2 and
+// 5.0, and take 8.6 now, 4.9 and 3.9 (a pull also takes its members' locks no longer, a push computes the
+// powers of equal step counts once).
+struct DenseDesc {
+  float* w;
+  float* state[KRK_ST_COUNT];
+  int64_t n;
+  int64_t start;     // first element in the concatenated arrays of a combined request
+};
+struct DenseBlock {
+  uint32_t member;
+  uint32_t at, of;   // which of the member's workgroups this is
+  uint32_t unused;
 };
 
-// The member of this workgroup: a lane per member and one vote (block_start ascends; walking it takes
-// a chain of scalar loads as long as the list).
-__device__ __forceinline__ int dense_member_of_block(const DenseGroupArgs& a) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const bool begun = lane < a.members && blockIdx.x >= a.block_start[lane < a.members ? lane : 0];
-  return __builtin_amdgcn_readfirstlane(__popcll(__ballot(begun)) - 1);
-}
+// What changes with every push: the members' steps, for the members of one launch.
+constexpr int kDenseGroupChunk = 64;
+struct DenseSteps {
+  float bc1[kDenseGroupChunk], bc2[kDenseGroupChunk];
+  unsigned long long first;
+};
 
-__global__ __launch_bounds__(kDenseBlock) void dense_group_pull_kernel(DenseGroupArgs a, float* __restrict__ out) {
-  const int mi = dense_member_of_block(a);
-  const DenseMember& m = a.m[mi];
-  const int64_t lane = (int64_t)(blockIdx.x - a.block_start[mi]) * kDenseBlock + threadIdx.x;
-  const int64_t stride = (int64_t)(a.block_start[mi + 1] - a.block_start[mi]) * kDenseBlock;
+__global__ __launch_bounds__(kDenseBlock) void dense_group_pull_kernel(const DenseBlock* __restrict__ blocks,
+                                                                       const DenseDesc* __restrict__ descs,
+                                                                       float* __restrict__ out) {
+  const DenseBlock b = blocks[blockIdx.x];
+  const DenseDesc& m = descs[b.member];
+  const int64_t lane = (int64_t)b.at * kDenseBlock + threadIdx.x;
+  const int64_t stride = (int64_t)b.of * kDenseBlock;
   float* dst = out + m.start;
+  const float* w = m.w;
+  const int64_t n = m.n;
   // 16-byte accesses where the member begins on a 16-byte boundary of the output
-  const int64_t n4 = (m.start & 3) == 0 ? m.n >> 2 : 0;
+  const int64_t n4 = (m.start & 3) == 0 ? n >> 2 : 0;
   for (int64_t i = lane; i < n4; i += stride)
-    __builtin_nontemporal_store(dense_load(m.w, i), reinterpret_cast<dfloat4*>(dst) + i);
-  for (int64_t i = (n4 << 2) + lane; i < m.n; i += stride) dst[i] = m.w[i];
+    __builtin_nontemporal_store(dense_load(w, i), reinterpret_cast<dfloat4*>(dst) + i);
+  for (int64_t i = (n4 << 2) + lane; i < n; i += stride) dst[i] = w[i];
 }
 
-static_assert(sizeof(DenseGroupArgs) + sizeof(OptimK) + 32 <= 4096, "the arguments of one launch");
-
+// member0: the launch's first member
 template <int OPT>
-__global__ __launch_bounds__(kDenseBlock) void dense_group_update_kernel(DenseGroupArgs a,
-                                                                         const float* __restrict__ grads,
-                                                                         float lr, OptimK k) {
-  const int mi = dense_member_of_block(a);
-  const DenseMember& m = a.m[mi];
-  const int64_t lane = (int64_t)(blockIdx.x - a.block_start[mi]) * kDenseBlock + threadIdx.x;
-  const int64_t stride = (int64_t)(a.block_start[mi + 1] - a.block_start[mi]) * kDenseBlock;
+__global__ __launch_bounds__(kDenseBlock) void dense_group_update_kernel(const DenseBlock* __restrict__ blocks,
+                                                                         const DenseDesc* __restrict__ descs,
+                                                                         uint32_t member0, DenseSteps steps, int st0,
+                                                                         int st1, int st2,
+                                                                         const float* __restrict__ grads, float lr,
+                                                                         OptimK k) {
+  const DenseBlock b = blocks[blockIdx.x];
+  const DenseDesc& m = descs[b.member];
+  const uint32_t mi = b.member - member0;
+  const int64_t lane = (int64_t)b.at * kDenseBlock + threadIdx.x;
+  const int64_t stride = (int64_t)b.of * kDenseBlock;
   const float* grad = grads + m.start;
   float* w = m.w;
-  float* s0 = m.s0;
-  float* s1 = m.s1;
-  float* s2 = m.s2;
-  const bool first = m.first != 0;
+  float* s0 = st0 >= 0 ? m.state[st0] : nullptr;
+  float* s1 = st1 >= 0 ? m.state[st1] : nullptr;
+  float* s2 = st2 >= 0 ? m.state[st2] : nullptr;
+  const bool first = (steps.first >> mi) & 1u;
+  const float bc1 = steps.bc1[mi], bc2 = steps.bc2[mi];
   const dfloat4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-  const int64_t n4 = (m.start & 3) == 0 ? m.n >> 2 : 0;
+  const int64_t n = m.n;
+  const int64_t n4 = (m.start & 3) == 0 ? n >> 2 : 0;
   for (int64_t i = lane; i < n4; i += stride) {
     const dfloat4 g4 = __builtin_nontemporal_load(reinterpret_cast<const dfloat4*>(grad) + i);
     const dfloat4 w4 = dense_load(w, i);
@@ -387,17 +477,17 @@ __global__ __launch_bounds__(kDenseBlock) void dense_group_update_kernel(DenseGr
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       ww[j] = w4[j]; sa[j] = a4[j]; sb[j] = b4[j]; sc[j] = c4[j];
-      optim_element<OPT>(k, lr, g4[j], ww[j], sa[j], sb[j], sc[j], first, m.bc1, m.bc2);
+      optim_element<OPT>(k, lr, g4[j], ww[j], sa[j], sb[j], sc[j], first, bc1, bc2);
     }
     dense_store(w, i, (dfloat4){ww[0], ww[1], ww[2], ww[3]});
     if (s0) dense_store(s0, i, (dfloat4){sa[0], sa[1], sa[2], sa[3]});
     if (s1) dense_store(s1, i, (dfloat4){sb[0], sb[1], sb[2], sb[3]});
     if (s2) dense_store(s2, i, (dfloat4){sc[0], sc[1], sc[2], sc[3]});
   }
-  for (int64_t i = (n4 << 2) + lane; i < m.n; i += stride) {
+  for (int64_t i = (n4 << 2) + lane; i < n; i += stride) {
     float g = grad[i], ww = w[i];
     float sa = s0 ? s0[i] : 0.0f, sb = s1 ? s1[i] : 0.0f, sc = s2 ? s2[i] : 0.0f;
-    optim_element<OPT>(k, lr, g, ww, sa, sb, sc, first, m.bc1, m.bc2);
+    optim_element<OPT>(k, lr, g, ww, sa, sb, sc, first, bc1, bc2);
     w[i] = ww;
     if (s0) s0[i] = sa;
     if (s1) s1[i] = sb;
@@ -406,11 +496,33 @@ __global__ __launch_bounds__(kDenseBlock) void dense_group_update_kernel(DenseGr
 }
 
 // Workgroups a member of n elements gets in a combined launch.
-static unsigned dense_member_blocks(int64_t n) {
-  int64_t blocks = (n / 4 + kDenseBlock - 1) / kDenseBlock;
-  if (blocks < 1) blocks = 1;
-  if (blocks > 512) blocks = 512;
-  return (unsigned)blocks;
+static unsigned dense_member_blocks(int64_t n) { return n > 0 ? dense_grid(n) : 0u; }
+
+// Puts the group's records and descriptors on the device. The members' streams have been waited for.
+static int32_t dense_group_describe(krk_dense_group* g) {
+  std::vector<DenseDesc> descs(g->tables.size());
+  std::vector<DenseBlock> blocks;
+  g->block_start.assign(1, 0u);
+  for (size_t i = 0; i < g->tables.size(); ++i) {
+    const krk_dense* t = g->tables[i];
+    DenseDesc& d = descs[i];
+    d.w = t->w;
+    for (int st = 0; st < KRK_ST_COUNT; ++st) d.state[st] = t->state[st];
+    d.n = t->n;
+    d.start = g->start[i];
+    const uint32_t of = dense_member_blocks(t->n);
+    for (uint32_t b = 0; b < of; ++b) blocks.push_back(DenseBlock{(uint32_t)i, b, of, 0u});
+    g->block_start.push_back((uint32_t)blocks.size());
+  }
+  const size_t desc_bytes = (descs.size() * sizeof(DenseDesc) + 255) & ~(size_t)255;
+  std::vector<char> both(desc_bytes + blocks.size() * sizeof(DenseBlock));
+  memcpy(both.data(), descs.data(), descs.size() * sizeof(DenseDesc));
+  if (!blocks.empty()) memcpy(both.data() + desc_bytes, blocks.data(), blocks.size() * sizeof(DenseBlock));
+  KRK_HIP(hipMalloc((void**)&g->descs, both.size()));
+  g->blocks = reinterpret_cast<const DenseBlock*>(reinterpret_cast<const char*>(g->descs) + desc_bytes);
+  KRK_HIP(hipMemcpyAsync(g->descs, both.data(), both.size(), hipMemcpyHostToDevice, g->stream));
+  KRK_HIP(hipStreamSynchronize(g->stream));
+  return KRK_SUCCESS;
 }
 
 // Takes the group's lock and then every member's, in member order.
@@ -598,7 +710,7 @@ int32_t krk_dense_import_state(krk_dense* t, int32_t state_type, const float* st
   if (state && (state_type < 1 || state_type >= KRK_ST_COUNT)) return KRK_E_ARGUMENT;
   std::lock_guard<std::mutex> lk(t->mu);
   if (state && t->n > 0) {
-    KRK_TRY(ensure_state(t, state_type));
+    KRK_TRY(ensure_states(&t, 1, &state_type, 1, t->stream));
     KRK_HIP(hipMemcpyAsync(t->state[state_type], state, (size_t)t->n * sizeof(float),
                            (flags & KRK_DEVICE_PTRS) ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice,
                            t->stream));
@@ -638,6 +750,19 @@ int32_t krk_dense_group_create(krk_dense** tables, int32_t n, krk_dense_group** 
     g->start.push_back(g->total);
     g->total += t->n;
   }
+  // (from here on the members' own calls may be creating columns: they are described under their locks)
+  int32_t described;
+  {
+    DenseGroupLock lk(g);
+    (void)hipStreamSynchronize(g->stream);
+    described = dense_group_describe(g);
+    for (size_t i = 0; i < g->tables.size() && described == KRK_SUCCESS; ++i)
+      g->tables[i]->group_state = g->descs[i].state;
+  }
+  if (described != KRK_SUCCESS) {
+    krk_dense_group_destroy(g);
+    return described;
+  }
   *out = g;
   return KRK_SUCCESS;
 }
@@ -649,8 +774,10 @@ int32_t krk_dense_group_destroy(krk_dense_group* g) {
     std::lock_guard<std::mutex> lk(t->mu);
     t->stream = t->own_stream;
     t->member_of = nullptr;
+    t->group_state = nullptr;
   }
   g->stream = g->own_stream;
+  if (g->descs) (void)hipFree(g->descs);
   g->close_stream();
   delete g;
   return KRK_SUCCESS;
@@ -675,25 +802,13 @@ int32_t krk_dense_group_pull(krk_dense_group* g, float* out, uint32_t flags) {
   KRK_TRY(ensure_runtime());
   KRK_TRY(check_flags(flags));
   if (g->total > 0 && !out) return KRK_E_ARGUMENT;
-  DenseGroupLock lk(g);
+  std::lock_guard<std::mutex> lk(g->mu);   // nothing of the members' host side is looked at
   if (g->total == 0) return KRK_SUCCESS;
   float* d_out;
   KRK_TRY(g->output(out, (size_t)g->total, flags, 0, &d_out));
-  for (size_t i = 0; i < g->tables.size();) {
-    DenseGroupArgs a;
-    a.members = 0;
-    uint32_t blocks = 0;
-    for (; i < g->tables.size() && a.members < kDenseGroupChunk; ++i) {
-      krk_dense* t = g->tables[i];
-      DenseMember& m = a.m[a.members];
-      m = DenseMember{t->w, nullptr, nullptr, nullptr, t->n, g->start[i], 1.0f, 1.0f, 0};
-      a.block_start[a.members++] = blocks;
-      blocks += dense_member_blocks(t->n);
-    }
-    a.block_start[a.members] = blocks;
-    hipLaunchKernelGGL(dense_group_pull_kernel, dim3(blocks), dim3(kDenseBlock), 0, g->stream, a, d_out);
-    KRK_HIP(hipGetLastError());
-  }
+  hipLaunchKernelGGL(dense_group_pull_kernel, dim3(g->block_start.back()), dim3(kDenseBlock), 0, g->stream, g->blocks,
+                     g->descs, d_out);
+  KRK_HIP(hipGetLastError());
   KRK_TRY(g->output_back(out, (size_t)g->total, flags, 0));
   if (!(flags & KRK_ASYNC)) KRK_HIP(hipStreamSynchronize(g->stream));
   return KRK_SUCCESS;
@@ -719,24 +834,27 @@ int32_t krk_dense_group_push(krk_dense_group* g, const krk_optim* o, const float
   const float* d_grads;
   KRK_TRY(g->input(grads, (size_t)n, flags, 0, &d_grads));
   const OptimK k = make_optim_k(*o);
+  int32_t st[3];
+  dense_slots(*o, st);
+  KRK_TRY(ensure_states(g->tables.data(), g->tables.size(), st, 3, g->stream));
+  StepMemo memo;
   for (size_t i = 0; i < g->tables.size();) {
-    DenseGroupArgs a;
-    a.members = 0;
-    uint32_t blocks = 0;
-    for (; i < g->tables.size() && a.members < kDenseGroupChunk; ++i) {
+    const size_t member0 = i;
+    DenseSteps steps;
+    steps.first = 0;
+    for (; i < g->tables.size() && i < member0 + kDenseGroupChunk; ++i) {
       krk_dense* t = g->tables[i];
       if (t->n == 0) continue;
-      DenseMember& m = a.m[a.members];
-      KRK_TRY(dense_member(t, *o, &m));
-      m.start = g->start[i];
-      a.block_start[a.members++] = blocks;
-      blocks += dense_member_blocks(t->n);
+      const DenseStep s = dense_step(t, *o, &memo);
+      steps.bc1[i - member0] = s.bc1;
+      steps.bc2[i - member0] = s.bc2;
+      if (s.first) steps.first |= 1ull << (i - member0);
     }
-    if (a.members == 0) continue;
-    a.block_start[a.members] = blocks;
+    const uint32_t block0 = g->block_start[member0], blocks = g->block_start[i] - block0;
+    if (blocks == 0) continue;
     with_optim(o->type, [&](auto opt) {
-      hipLaunchKernelGGL((dense_group_update_kernel<opt.value>), dim3(blocks), dim3(kDenseBlock), 0, g->stream, a,
-                         d_grads, lr, k);
+      hipLaunchKernelGGL((dense_group_update_kernel<opt.value>), dim3(blocks), dim3(kDenseBlock), 0, g->stream,
+                         g->blocks + block0, g->descs, (uint32_t)member0, steps, st[0], st[1], st[2], d_grads, lr, k);
     });
     KRK_HIP(hipGetLastError());
   }

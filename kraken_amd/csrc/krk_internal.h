@@ -351,7 +351,10 @@ struct OptimK {
   float alpha;
   float one_minus_alpha;
   float acc0;
-  double log2_beta1;       // base-two logarithms of |beta1| and |beta2|, for one_minus_power
+};
+// The same for rows that count their own steps.
+struct RowOptimK : OptimK {
+  double log2_beta1;       // base-two logarithms of |beta1| and |beta2|, for one_minus_power (Adam)
   double log2_beta2;
 };
 
@@ -383,6 +386,7 @@ __device__ __forceinline__ float one_minus_power(double log2_beta, float beta, u
 }
 
 OptimK make_optim_k(const krk_optim& o);
+RowOptimK make_row_optim_k(const krk_optim& o);
 // Which state columns (bit per KRK_ST_*) and whether a step counter this optimizer touches.
 uint32_t optim_state_mask(const krk_optim& o);
 

@@ -1527,7 +1527,7 @@ static int32_t fill_and_reduce(const ReduceShape& sh, hipStream_t stream, Device
 static ApplyArgs table_apply_args(krk_sparse* t, const krk_optim* o, float lr) {
   ApplyArgs args;
   args.lr = lr;
-  args.k = make_optim_k(*o);
+  args.k = make_row_optim_k(*o);
   int32_t cols[3];
   sparse_optim_columns(t, *o, cols);
   args.c0 = cols[0];
@@ -2131,7 +2131,7 @@ static GroupCall group_rows_layout(const GroupCall& call, const int64_t* offsets
 static ApplyArgs group_apply_args(const krk_optim* o, float lr) {
   ApplyArgs args;
   args.lr = lr;
-  args.k = make_optim_k(*o);
+  args.k = make_row_optim_k(*o);
   args.c0 = args.c1 = args.c2 = args.meta_off = -1;     // taken per member from its layout
   return args;
 }

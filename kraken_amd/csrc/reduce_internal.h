@@ -98,7 +98,7 @@ __device__ __forceinline__ float mean_ratio(const BagWord& words, uint32_t word,
 
 struct ApplyArgs {
   float lr;
-  OptimK k;
+  RowOptimK k;
   int c0, c1, c2, meta_off;
 };
 

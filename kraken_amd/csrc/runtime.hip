@@ -147,8 +147,15 @@ OptimK make_optim_k(const krk_optim& o) {
   k.alpha = o.alpha;
   k.one_minus_alpha = (float)(1.0 - (double)o.alpha);
   k.acc0 = o.initial_accumulator;
-  k.log2_beta1 = std::log2(std::fabs((double)o.beta1));
-  k.log2_beta2 = std::log2(std::fabs((double)o.beta2));
+  return k;
+}
+
+RowOptimK make_row_optim_k(const krk_optim& o) {
+  RowOptimK k{make_optim_k(o), 0.0, 0.0};
+  if (o.type == KRK_ADAM) {
+    k.log2_beta1 = std::log2(std::fabs((double)o.beta1));
+    k.log2_beta2 = std::log2(std::fabs((double)o.beta2));
+  }
   return k;
 }
 

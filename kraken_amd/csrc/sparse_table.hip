@@ -210,7 +210,7 @@ template <int OPT, int VEC>
 __device__ __forceinline__ void push_body(const TableView& tv, const uint64_t* __restrict__ ids,
                                           int64_t i, bool active, int gl,
                                           const float* __restrict__ grads, int dim, int elems,
-                                          int group, float lr, const OptimK& k, const PushCols& pc,
+                                          int group, float lr, const RowOptimK& k, const PushCols& pc,
                                           const uint32_t* __restrict__ notes = nullptr) {
   // The gradient row does not depend on the index: its first slice is requested before the
   // probe so that it travels while the probe waits for its bucket.
@@ -707,7 +707,7 @@ template <int OPT, int VEC>
 __global__ __launch_bounds__(kBlock) void push_kernel(TableView tv, const uint64_t* __restrict__ ids,
                                                       int64_t n, const float* __restrict__ grads,
                                                       int dim, int elems, int group, float lr,
-                                                      OptimK k, PushCols pc,
+                                                      RowOptimK k, PushCols pc,
                                                       const uint32_t* __restrict__ notes) {
   const int per_block = kBlock / group;
   const int64_t i = (int64_t)blockIdx.x * per_block + threadIdx.x / group;
@@ -830,7 +830,7 @@ __host__ __device__ inline bool pull_is_wide(int group, int elems) {
 template <int OPT, int STEPS>
 __device__ __forceinline__ void push_wide(const TableView& tv, const uint64_t* __restrict__ ids,
                                           int64_t first, int64_t end, const float* __restrict__ grads,
-                                          int dim, int elems, float lr, const OptimK& k,
+                                          int dim, int elems, float lr, const RowOptimK& k,
                                           const PushCols& pc, const uint32_t* __restrict__ notes = nullptr) {
   constexpr int VEC = 4;
   constexpr int rows_per_step = kWideIds / STEPS;   // 8, 4 or 2
@@ -910,7 +910,7 @@ __host__ __device__ inline bool push_is_wide(int vec, int group, int elems) {
 template <int OPT, int STEPS>
 __global__ __launch_bounds__(kBlock) void push_wide_kernel(TableView tv, const uint64_t* __restrict__ ids,
                                                            int64_t n, const float* __restrict__ grads,
-                                                           int dim, int elems, float lr, OptimK k,
+                                                           int dim, int elems, float lr, RowOptimK k,
                                                            PushCols pc, const uint32_t* __restrict__ notes) {
   const int64_t first = ((int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave) * kWideIds;
   if (first >= n) return;                        // the whole wavefront
@@ -1125,7 +1125,7 @@ __global__ __launch_bounds__(kBlock) void group_push_kernel(const TableDesc* __r
                                                             GroupCall call,
                                                             const uint64_t* __restrict__ ids,
                                                             const float* __restrict__ grads, int dim,
-                                                            int elems, int group, float lr, OptimK k,
+                                                            int elems, int group, float lr, RowOptimK k,
                                                             int st0, int st1, int st2, int use_meta,
                                                             const uint32_t* __restrict__ notes) {
   const uint32_t bx = blockIdx.x;
@@ -1149,7 +1149,7 @@ __global__ __launch_bounds__(kBlock) void group_push_wide_kernel(const TableDesc
                                                                  GroupCall call,
                                                                  const uint64_t* __restrict__ ids,
                                                                  const float* __restrict__ grads, int dim,
-                                                                 int elems, float lr, OptimK k, int st0,
+                                                                 int elems, float lr, RowOptimK k, int st0,
                                                                  int st1, int st2, int use_meta,
                                                                  const uint32_t* __restrict__ notes) {
   const uint32_t bx = blockIdx.x;
@@ -1985,7 +1985,7 @@ static InitK make_init_k(const krk_init& in, int64_t dim) {
 // Enqueues push_kernel or, for whole rows of 32 to 128 floats, push_wide_kernel.
 template <int OPT, int VEC>
 static void launch_push_opt(krk_sparse* t, const uint64_t* ids, int64_t n, const float* grads, float lr,
-                            const OptimK& k, const PushCols& pc, const uint32_t* notes) {
+                            const RowOptimK& k, const PushCols& pc, const uint32_t* notes) {
   const TableView tv = t->view();
   const int dim = (int)t->dim;
   const dim3 block(kBlock);
@@ -2010,7 +2010,7 @@ static void launch_push_opt(krk_sparse* t, const uint64_t* ids, int64_t n, const
 template <int VEC>
 static void launch_push(krk_sparse* t, const krk_optim& o, const uint64_t* ids, int64_t n,
                         const float* grads, float lr, const uint32_t* notes = nullptr) {
-  const OptimK k = make_optim_k(o);
+  const RowOptimK k = make_row_optim_k(o);
   int32_t cols[3];
   sparse_optim_columns(t, o, cols);
   const bool needs_meta = (optim_state_mask(o) >> KRK_ST_STEPS) & 1u;
@@ -3515,7 +3515,7 @@ int32_t krk_group_pull_pooled_parts(krk_group* g, const krk_pooled_part* in, uin
 
 template <int OPT, int VEC>
 static void launch_group_push_opt(krk_group* g, const GroupCall& call, const uint64_t* ids,
-                                  const float* grads, float lr, const OptimK& k, const int32_t st[3],
+                                  const float* grads, float lr, const RowOptimK& k, const int32_t st[3],
                                   int use_meta, bool wide, const uint32_t* notes) {
   const dim3 grid(call.block_start[call.n_tables]), block(wide ? group_wide_block(g->group) : kBlock);
   const int dim = (int)g->dim;
@@ -3540,7 +3540,7 @@ template <int VEC>
 static void launch_group_push(krk_group* g, const krk_optim& o, const GroupCall& call,
                               const uint64_t* ids, const float* grads, float lr, bool wide,
                               const uint32_t* notes) {
-  const OptimK k = make_optim_k(o);
+  const RowOptimK k = make_row_optim_k(o);
   int32_t st[3];
   optim_state_slots(o, st);
   const int use_meta = (optim_state_mask(o) >> KRK_ST_STEPS) & 1u;

@@ -350,3 +350,41 @@ def test_dense_group_matches_the_per_table_loop(api, oracle, name, type_, conf):
     assert np.array_equal(d_out.to_host(), got)
     grp.close()
     assert tables[0].Pull()[0] == 0       # members work on their own again
+
+
+# a push takes 64 members a launch; columns are created by the group's push (200 a launch enter its
+# descriptors), by a member's own while the group is there, and before the group
+@pytest.mark.parametrize("members", [1, 64, 65, 130])
+def test_dense_group_members_and_columns(api, oracle, members):
+    rng = np.random.default_rng(members)
+    sizes = [int(x) for x in rng.integers(1, 1500, size=members)]
+    sizes[members // 2] = sizes[-1] = 0
+    if members == 1:
+        sizes = [1031]
+    w0 = [rng.standard_normal(n).astype(np.float32) for n in sizes]
+    tables, refs = [api.DenseTable(w) for w in w0], [oracle.DenseTable(w) for w in w0]
+    own = 0
+    for optims in (("adagrad", "adam"), ("sgd_mom", "adam")):
+        grp = api.DenseGroup(tables)
+        for name in optims:
+            type_, conf = next(c[1:] for c in OPTIM_CASES if c[0] == name)
+            o_ref, o_gpu = make_optims(oracle, api, type_, conf)
+            g = (rng.standard_normal(sizes[own]) * 1e-2).astype(np.float32)
+            assert tables[own].Push(o_gpu, g, 0.01) == 0 and refs[own].push(o_ref, g, 0.01) == 0
+            for _ in range(2):
+                grads = (rng.standard_normal(grp.n) * 1e-2).astype(np.float32)
+                assert grp.CombinePush(o_gpu, grads, 0.01) == 0
+                at = 0
+                for r, n in zip(refs, sizes):
+                    if n:
+                        assert r.push(o_ref, grads[at:at + n], 0.01) == 0
+                    at += n
+            rc, got = grp.CombinePull()
+            assert rc == 0
+            assert_close(got, np.concatenate([r.pull() for r in refs]), "%d members, %s" % (members, name))
+            for t, r, n in zip(tables, refs, sizes):
+                for st in STATE_OF[type_] if n else []:
+                    ws = r.state(st)
+                    assert_close(t.state(st), ws if ws is not None else np.zeros(n, np.float32), "%s state %d" % (name, st))
+        grp.close()
+        own = members - 2 if members > 1 else 0
