@@ -605,6 +605,29 @@ def test_host_arguments_around_the_bounce_limit(api, n):
     assert host.Push(opt, missing, grads[:1], 0.1) == api.SPARSE_ID_NOT_EXIST
 
 
+@pytest.mark.parametrize("beta", [0.1, 0.3, 0.5, 0.7, 0.8, 0.9, 0.95, 0.99, 0.999, 0.9999, 0.99999, 0.9999999])
+def test_adam_powers_are_correctly_rounded(api, beta):
+    """Both bias corrections at every step count to 200,000: rows that have counted t - 1 steps take one with a
+    gradient of one. Every operation after the powers is a correctly rounded one, so with the powers rounded
+    from extended precision numpy has the same bits."""
+    f32, ld = np.float32, np.longdouble
+    n = 200_000
+    t = api.SparseTable(1, api.Initializer.create(api.InitializerType.kConstant, {"value": "0"}), capacity_hint=n)
+    ids = splitmix64(np.arange(n, dtype=np.uint64))
+    assert t.Pull(ids)[0] == 0
+    assert t.load_state(ids, steps=np.arange(n, dtype=np.int64)) == 0
+    other = 1.0 - beta if 0.05 < beta < 0.95 else 0.6
+    b1, b2 = f32(beta), f32(other)
+    o = api.Optim.create(api.OptimType.kAdam, {"beta1": repr(beta), "beta2": repr(other), "eps": "1e-3"})
+    assert t.Push(o, ids, np.ones((n, 1), f32), 0.125) == 0
+    count = np.arange(1, n + 1)
+    c1, c2 = ((1.0 - np.power(ld(b), count).astype(f32).astype(np.float64)).astype(f32) for b in (b1, b2))
+    r1, r2 = f32(1.0 - float(b1)), f32(1.0 - float(b2))
+    with np.errstate(under="ignore"):
+        want = f32(0) - (f32(0.125) * (r1 / c1)) / (np.sqrt(r2 / c2) + f32(1e-3))
+    assert np.array_equal(t.Pull(ids)[1][:, 0], want)
+
+
 # The host learns a nearly full table's row count from its pulls, asked for with two requests to go, or three
 # while the host has had to wait; 1 to 6 requests fit behind the rows.
 @pytest.mark.parametrize("room", [1.2, 2.2, 3.2, 6.2])
