@@ -307,7 +307,7 @@ def test_dense_group_matches_the_per_table_loop(api, oracle, name, type_, conf):
     """Ps::CombinePullDenseTable (ps/ps_op.cc:177-252) and a step's PushDenseTable calls for every
     dense parameter of a model, as one launch each: against the oracle's loop over the tables.
     Member sizes put some members off the 16-byte grid of the concatenated arrays (the scalar
-    path), one member is empty, 40 members take two launches, and a member that was updated on its
+    path), one member is empty, and a member that was updated on its
     own before joining keeps its own Adam step count."""
     rng = np.random.default_rng(type_ + 40)
     sizes = [64, 1, 150_000, 4099, 0, 7, 1024, 333] + [int(x) for x in rng.integers(1, 3000, size=32)]
