@@ -469,6 +469,7 @@ struct krk_sparse : krk::ObjBase {
   int64_t last_request = 0;           // size of the latest large inserting requests
   int64_t pub_rows = 0;               // rows at the last published count that was looked at
   int behind_for = 0;                 // requests for which the host still counts as ahead of the device
+  bool pushed = false;                // since the last request that could insert
   uint64_t enq_total = 0;             // ids handed to inserting launches so far
   uint64_t enq_at[256] = {};          // enq_total right after the launch with number e (mod 256)
   uint32_t epoch = 0;                 // number of the last launch that could insert

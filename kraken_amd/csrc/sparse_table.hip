@@ -1724,14 +1724,16 @@ static uint64_t pow2_at_least(uint64_t x) {
   return c;
 }
 
-// Requests that should still fit when a count is asked for: two, or three while the host is ahead of the
-// device, which it is for the next kBehindFor requests after it had to wait for a count. With three, two
-// requests are still in the stream when the host waits for the third, and the stream does not run dry;
-// a host that is the slower one never waits, and a count more often is a launch. 16,384 ids of 128
-// floats a pull, nothing else, with room for 3.2 / 4.2 / 9.2 requests, us: always two 12.7 / 10.7 / 8.1,
-// three 8.4 / 7.6 / 6.7, in every pull below four 8.2 / 8.1 / 7.7; pull and push of 2048 ids of 16 floats, bound by
-// the host, room for 3.2: 12.0 / 14.4 / 14.
+// Requests that should still fit when a count is asked for: two, or three for the next kBehindFor requests
+// after the host had to wait for a count among short pulls with nothing between them. With three, two of
+// them are still in the stream when the host waits for the third, and the stream does not run dry.
+// Pulls of 16,384 and of 32,768 ids of 128 floats, nothing else, with room for 3.2 / 4.2 / 9.2 requests, us:
+// always two 10.5-12.7 / 9.5-11 / 7.3-8.1 and 11.3-13.4 / 10.3-11.3 / 8.1-8.4, three 8.4 / 7.6 / 6.8 and
+// 10.1 / 8.9 / 8.0. A count is a launch, so two are better where the stream holds enough: a pull of 65,536 14.9 /
+// 14.0 / 13.2 and 15.5 / 14.6 / 13.3, a pull and a push of 32,768 28.6 / 27.7 / 26.7 and 31.0 / 28.6 / 26.8, and where
+// the host is the slower side and never waits.
 constexpr int kBehindFor = 32;
+constexpr int64_t kShortPullBytes = (int64_t)24 << 20;   // of rows
 static int64_t publish_lead(const krk_sparse* t) { return t->behind_for > 0 ? 3 : 2; }
 // Rows a table has room for beyond its bound.
 static int64_t room_left(const krk_sparse* t) {
@@ -1754,14 +1756,14 @@ static void tighten_bound(krk_sparse* t) {
 // the next request is there (8.5 million pooled ids over 4 million rows, forward, backward and
 // forward: 1455 us with two waits of that kind). Returns when the bound allows `need_for` more rows,
 // the last count that was to be published has arrived, or the stream has nothing left to run.
-static void await_published(krk_sparse* t, int64_t extra_rows) {
+static void await_published(krk_sparse* t, int64_t extra_rows, bool short_pulls) {
   if (t->pub_epoch == 0) return;
   for (;;) {
     tighten_bound(t);
     const int64_t need = t->size_ub + extra_rows;
     if (need <= t->row_cap && (uint64_t)need * 2 <= t->slot_cap) break;
     if ((uint32_t)(__atomic_load_n(t->host_pub, __ATOMIC_ACQUIRE) >> 32) == t->pub_epoch) break;
-    t->behind_for = kBehindFor;
+    if (short_pulls) t->behind_for = kBehindFor;
     if (hipStreamQuery(t->stream) != hipErrorNotReady) break;
     std::this_thread::yield();
   }
@@ -1770,11 +1772,13 @@ static void await_published(krk_sparse* t, int64_t extra_rows) {
 
 // Room for `extra_rows` more rows: records, row keys, and an index at most half full.
 int32_t sparse_ensure_room(krk_sparse* t, int64_t extra_rows) {
-  if (t->behind_for > 0) --t->behind_for;
+  const bool short_pulls = !t->pushed && extra_rows * t->dim * (int64_t)sizeof(float) <= kShortPullBytes;
+  t->pushed = false;
+  t->behind_for = short_pulls ? std::max(t->behind_for - 1, 0) : 0;
   if (room_left(t) < publish_lead(t) * t->last_request) tighten_bound(t);
   int64_t need = t->size_ub + extra_rows;
   if (need > t->row_cap || (uint64_t)need * 2 > t->slot_cap) {
-    await_published(t, extra_rows);
+    await_published(t, extra_rows, short_pulls);
     tighten_bound(t);
     need = t->size_ub + extra_rows;
   }
@@ -1844,6 +1848,7 @@ int32_t sparse_publish(krk_sparse* const* tables, int n, hipStream_t stream) {
 
 // Adds the state columns an optimizer needs; existing records are re-strided once.
 int32_t sparse_ensure_columns(krk_sparse* t, uint32_t mask) {
+  t->pushed = true;
   bool change = false;
   int32_t col_off[KRK_ST_COUNT];
   memcpy(col_off, t->col_off, sizeof(col_off));
