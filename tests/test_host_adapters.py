@@ -26,6 +26,18 @@ def _build():
                            "-lkraken_hip", "-Wl,-rpath," + lib_dir, "-Wl,-rpath,/opt/rocm/lib"])
 
 
+REFUSED = os.path.join(ROOT, "tests", "host", "refused_allocation_test")
+
+
+def _build_refused():
+    lib_dir = os.path.join(ROOT, "kraken_amd")
+    if os.path.exists(REFUSED) and os.path.getmtime(REFUSED) > os.path.getmtime(REFUSED + ".cc"):
+        return
+    subprocess.check_call(["g++", "-std=c++17", "-O2", "-Wall", "-I" + os.path.join(ROOT, "include"), REFUSED + ".cc", "-o",
+                           REFUSED, "-L" + lib_dir, "-lkraken_hip", "-ldl", "-Wl,-rpath," + lib_dir,
+                           "-Wl,-rpath,/opt/rocm/lib"])
+
+
 def _have_gpu():
     try:
         n = C.c_int()
@@ -49,3 +61,16 @@ def test_adapters_on_gpu():
     r = subprocess.run([EXE], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
     assert "table interface ok" in r.stdout
+
+
+def test_refused_allocation_builds():
+    _build_refused()
+
+
+@pytest.mark.gpu
+def test_push_without_room_for_its_sums():
+    """A push whose work space hipMalloc refuses is sorted, with the same result."""
+    _build_refused()
+    r = subprocess.run([REFUSED], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert "refused allocation ok" in r.stdout
