@@ -114,34 +114,42 @@ struct StateEntries {
 static_assert(sizeof(StateEntries) + 16 <= 4096, "the arguments of one launch");
 __global__ void enter_states_kernel(StateEntries e, int n) {
   const int i = threadIdx.x;
-  if (i < n) *e.at[i] = e.value[i];
+  if (i < n && e.at[i]) *e.at[i] = e.value[i];
 }
+// Columns on their way: a table has one when it is zeroed and, for a member of a group, entered.
 struct StateList {
   hipStream_t stream = nullptr;
   int n = 0;
+  bool grouped = false;
+  krk_dense* table[kEntries];
+  int state[kEntries];
   StateEntries e;
+  ~StateList() {
+    for (int i = 0; i < n; ++i) (void)hipFree(e.value[i]);   // given up on the way
+  }
+  int32_t add(krk_dense* t, int st) {
+    if (n == kEntries) KRK_TRY(flush());
+    DeviceGuard guard;
+    KRK_HIP(hipMalloc(&guard.p, (size_t)t->n * sizeof(float)));
+    KRK_HIP(hipMemsetAsync(guard.p, 0, (size_t)t->n * sizeof(float), t->stream));
+    table[n] = t;
+    state[n] = st;
+    e.at[n] = t->group_state ? t->group_state + st : nullptr;
+    e.value[n++] = guard.release<float>();
+    grouped = grouped || t->group_state;
+    return KRK_SUCCESS;
+  }
   int32_t flush() {
-    if (n == 0) return KRK_SUCCESS;
-    hipLaunchKernelGGL(enter_states_kernel, dim3(1), dim3(256), 0, stream, e, n);
-    KRK_HIP(hipGetLastError());
+    if (grouped) {   // (the members' stream is the group's)
+      hipLaunchKernelGGL(enter_states_kernel, dim3(1), dim3(256), 0, stream, e, n);
+      KRK_HIP(hipGetLastError());
+    }
+    for (int i = 0; i < n; ++i) table[i]->state[state[i]] = e.value[i];
     n = 0;
+    grouped = false;
     return KRK_SUCCESS;
   }
 };
-
-static int32_t ensure_state(krk_dense* t, int st, StateList* list) {
-  if (t->state[st]) return KRK_SUCCESS;
-  DeviceGuard guard;
-  KRK_HIP(hipMalloc(&guard.p, (size_t)(t->n ? t->n : 1) * sizeof(float)));
-  KRK_HIP(hipMemsetAsync(guard.p, 0, (size_t)t->n * sizeof(float), t->stream));
-  if (t->group_state) {   // (a member's stream is the group's)
-    if (list->n == kEntries) KRK_TRY(list->flush());
-    list->e.at[list->n] = t->group_state + st;
-    list->e.value[list->n++] = reinterpret_cast<float*>(guard.p);
-  }
-  t->state[st] = guard.release<float>();   // only a zeroed column counts as present
-  return KRK_SUCCESS;
-}
 
 // The states an optimizer's three slots stand for (krk_internal.h), -1 = unused.
 static void dense_slots(const krk_optim& o, int32_t st[3]) {
@@ -166,17 +174,14 @@ static void dense_slots(const krk_optim& o, int32_t st[3]) {
   }
 }
 
-// Creates the columns of the states st (-1: none) that n tables of one stream, those with elements, lack. What could be created
-// is entered also where a later one could not.
+// Creates the columns of the states st (-1: none) that n tables of one stream, those with elements, lack.
 static int32_t ensure_states(krk_dense* const* tables, size_t n, const int32_t* st, int n_st, hipStream_t stream) {
-  int32_t rc = KRK_SUCCESS;
   StateList list;
   list.stream = stream;
-  for (size_t i = 0; i < n && rc == KRK_SUCCESS; ++i)
-    for (int k = 0; k < n_st && rc == KRK_SUCCESS; ++k)
-      if (st[k] >= 0 && tables[i]->n > 0 && !tables[i]->state[st[k]]) rc = ensure_state(tables[i], st[k], &list);
-  const int32_t entered = list.flush();
-  return rc != KRK_SUCCESS ? rc : entered;
+  for (size_t i = 0; i < n; ++i)
+    for (int k = 0; k < n_st; ++k)
+      if (st[k] >= 0 && tables[i]->n > 0 && !tables[i]->state[st[k]]) KRK_TRY(list.add(tables[i], st[k]));
+  return list.n > 0 ? list.flush() : KRK_SUCCESS;
 }
 
 // Adam's bias corrections of a step (ps/optim/adam.cc:61-64) and SGD's first momentum update.

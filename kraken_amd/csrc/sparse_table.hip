@@ -1770,7 +1770,10 @@ static void await_published(krk_sparse* t, int64_t extra_rows, bool short_pulls)
   if (hipPeekAtLastError() == hipErrorNotReady) (void)hipGetLastError();   // no failure of a later call
 }
 
-// Room for `extra_rows` more rows: records, row keys, and an index at most half full.
+// Room for `extra_rows` more rows: records, row keys, and an index at most half full. All ids of a request
+// count as new until it has been looked up, so the first pull of a table that is as full as it was made for
+// doubles it: 1.3 ms for a million rows of 32 floats and a state, or 7.4 in a process that has allocated and
+// freed some 100 GB of device memory before.
 int32_t sparse_ensure_room(krk_sparse* t, int64_t extra_rows) {
   const bool short_pulls = !t->pushed && extra_rows * t->dim * (int64_t)sizeof(float) <= kShortPullBytes;
   t->pushed = false;
