@@ -591,10 +591,14 @@ struct krk_group : krk::ObjBase {
 };
 
 namespace krk {
+// Words that the arrays of row numbers of a request have behind the last one: pooled_add reads four numbers at a
+// time, from a position of a bag and from four behind it.
+constexpr int kRowsAhead = 16;
+
 // Room for the notes of n positions, or null where the device has none: the pull then leaves no notes
 // behind, and the push that follows looks its ids up.
 inline uint32_t* note_room(DeviceBuffer* notes, int64_t n) {
-  if (notes->reserve((size_t)n * sizeof(uint32_t)) == KRK_SUCCESS) return notes->as<uint32_t>();
+  if (notes->reserve(((size_t)n + kRowsAhead) * sizeof(uint32_t)) == KRK_SUCCESS) return notes->as<uint32_t>();
   (void)hipGetLastError();   // no failure of the call
   return nullptr;
 }

@@ -617,90 +617,177 @@ __global__ __launch_bounds__(kBlock, FEW ? 1 : 8) void pooled_probe_kernel(Table
   pooled_probe_body<VEC>(tv, init, ids, p0, n, rows, elems, FEW ? kFillingIds : kFilling64, FEW);
 }
 
-// Records of one bag requested together. Eight take registers of which two wavefronts a SIMD live (852k bags
-// of 32 floats, ten ids each, 180 us, with four 135).
+// Records of one bag requested together; also the row numbers that one load brings.
 constexpr int kPoolAhead = 4;
+typedef uint32_t vrows_t __attribute__((ext_vector_type(4), aligned(4)));   // row numbers lie on four bytes
 
-// The row numbers of the next records are requested with the present ones, so that a bag of ten ids waits
-// for memory four times, not six times (148 -> 135 us; 188 with every address and bound in 64 bits and
-// a test for weights at every id).
-template <int VEC, bool WEIGHTED>
-__device__ __forceinline__ void pooled_add(const TableView& tv, const uint32_t* __restrict__ rows,
-                                           const uint64_t* __restrict__ ids, int count,
-                                           const float* __restrict__ weights, int gl, float (&acc)[VEC]) {
-  uint32_t row[kPoolAhead];
+// A wavefront takes `bags` <= 64 bags, the first of which is `first`; lane i knows where bag i begins and how long it
+// is. Its lane groups work on a bag each, four records at a time, and where there are more bags than groups (MORE)
+// a group whose bag ends takes the next one that nobody has: with a bag per group and wavefront, groups waited for the
+// longest of their bags (0 to 20 ids each: 44 % of the lanes idle). 852k bags of 32 floats, ten ids each:
+// 138 us with a bag per group, where branches and 64-bit addresses made 110 vector instructions for four
+// records, 120 with as many as now, 109 with 64 bags a wavefront. What is left is lines: 6.1 million requests from
+// the compute units' caches to L2, at 62 a nanosecond the most that random lines have reached. Measured and not
+// kept: half the lanes a row with two slices each (123: a line is then asked for twice), eight records at a time
+// (136), the next four requested before the present ones are added (129: 91 registers).
+template <int VEC, bool WEIGHTED, bool MORE>
+__device__ __forceinline__ void pooled_sum_wave(const TableView& tv, const uint32_t* __restrict__ rows,
+                                                const uint64_t* __restrict__ ids, int64_t n,
+                                                const long long* __restrict__ offsets, int64_t first, int bags,
+                                                const float* __restrict__ weights, int mean, float patch,
+                                                float* __restrict__ out, int dim, int elems, int shift) {
+  const int lane = wave_lane();
+  const int gl = lane & ((1 << shift) - 1);
+  const int sub = lane >> shift;
+  const bool part = gl < elems;
+  int my_at = 0, my_count = 0;
+  if (lane < bags) {
+    long long lo = offsets[first + lane], hi = offsets[first + lane + 1];
+    if (lo < 0) lo = 0;
+    if (hi > n) hi = n;
+    if (hi > lo) {                                     // (a request has fewer than 2^31 positions)
+      my_at = (int)lo;
+      my_count = (int)(hi - lo);
+    }
+  }
+  // jagged_ops.cc:219
+  const float my_ratio = mean && my_count > 0 ? (float)(1.0 / (double)(float)my_count) : 1.0f;
+  const float* base = tv.recs + (part ? gl * VEC : 0);
+  const uint32_t stride = (uint32_t)tv.stride * (uint32_t)sizeof(float);
+  const auto record = [&](uint32_t row) {
+    return reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + (uint64_t)row * stride);
+  };
+  const auto numbers = [&](int at) { return *reinterpret_cast<const KRK_GLOBAL vrows_t*>((uintptr_t)(rows + at)); };
+  const unsigned long long groups_below = (1ull << (sub << shift)) - 1ull;   // the lanes of the groups before this one
+  int bag = sub, taken = kWave >> shift;               // this group's bag; how many bags have been taken
+  bool have = bag < bags;
+  int at = __shfl(my_at, bag), left = __shfl(my_count, bag);
+  vrows_t next = {0u, 0u, 0u, 0u};
+  if (left > 0) next = numbers(at);
+  float acc[VEC];
 #pragma unroll
-  for (int u = 0; u < kPoolAhead; ++u) row[u] = u < count ? rows[u] : 0u;
-  for (int j0 = 0; j0 < count; j0 += kPoolAhead) {
-    float v[kPoolAhead][VEC], w[kPoolAhead];
-#pragma unroll
-    for (int u = 0; u < kPoolAhead; ++u) {
-      if (j0 + u < count) {
-        // A position that met its id while another position's group was still creating the row could not
-        // learn the row number in the first launch; by now it is in the index.
-        if (row[u] == kEmptyRow) row[u] = probe_find_alone(tv, ids[j0 + u]);
-        if (row[u] != kEmptyRow) {
-          gload<VEC>(tv.recs + (int64_t)row[u] * tv.stride + gl * VEC, v[u]);
-        } else {
-#pragma unroll
-          for (int c = 0; c < VEC; ++c) v[u][c] = 0.0f;
-        }
-        if (WEIGHTED) w[u] = weights[j0 + u];
+  for (int c = 0; c < VEC; ++c) acc[c] = -0.0f;        // to which every first record adds as itself
+  for (;;) {
+    // what comes after these records: the bag's next ones, or another bag
+    const bool last = left <= kPoolAhead;
+    const float ratio = mean ? __shfl(my_ratio, bag & (kWave - 1)) : 1.0f;
+    bool next_have = have && !last;
+    int next_bag = bag, next_at = at + kPoolAhead, next_left = next_have ? left - kPoolAhead : 0;
+    if constexpr (MORE) {
+      const unsigned long long ends = __ballot(have && last && gl == 0);
+      const int another = taken + __popcll(ends & groups_below);
+      taken += __popcll(ends);
+      const int other_at = __shfl(my_at, another & (kWave - 1));
+      const int other_count = __shfl(my_count, another & (kWave - 1));
+      if (have && last && another < bags) {
+        next_have = true;
+        next_bag = another;
+        next_at = other_at;
+        next_left = other_count;
       }
     }
-#pragma unroll
-    for (int u = 0; u < kPoolAhead; ++u) row[u] = j0 + kPoolAhead + u < count ? rows[j0 + kPoolAhead + u] : 0u;
+    // The positions past the bag's end are not branched around: they read the record again that the lane
+    // has just asked for, and only their addition is masked.
+    uint32_t row[kPoolAhead];
+    bool open = false;
 #pragma unroll
     for (int u = 0; u < kPoolAhead; ++u) {
-      if (j0 + u >= count) break;
+      row[u] = u < left ? next[u] : next[0];
+      open |= row[u] == kEmptyRow;
+    }
+    if (next_left > 0) next = numbers(next_at);
+    // A position that met its id while another position's group was still creating the row could not
+    // learn the row number in the first launch; by now it is in the index (or the table is full).
+    if (__any(open && left > 0)) {
+#pragma unroll 1
+      for (int u = 0; u < kPoolAhead && u < left; ++u) {
+        uint32_t r = row[0];
+#pragma unroll
+        for (int k = 1; k < kPoolAhead; ++k) r = u == k ? row[k] : r;
+        if (r == kEmptyRow) r = probe_find_alone(tv, ids[at + u]);
+        float v[VEC];
+#pragma unroll
+        for (int c = 0; c < VEC; ++c) v[c] = 0.0f;
+        if (r != kEmptyRow) gload<VEC>(record(r), v);
+#pragma unroll
+        for (int c = 0; c < VEC; ++c) acc[c] = acc[c] + (WEIGHTED ? v[c] * weights[at + u] : v[c]);
+      }
+    } else if (left > 0) {
+      float v[kPoolAhead][VEC], w[kPoolAhead];
+#pragma unroll
+      for (int u = 0; u < kPoolAhead; ++u) {
+        gload<VEC>(record(row[u]), v[u]);
+        if (WEIGHTED) w[u] = weights[u < left ? at + u : at];
+      }
+      // all of them are requested by here: a load that only the masked addition used would move behind its mask
+#pragma unroll
+      for (int u = 0; u < kPoolAhead; ++u) {
+#pragma unroll
+        for (int c = 0; c < VEC; ++c) asm volatile("" : "+v"(v[u][c]));
+      }
+#pragma unroll
+      for (int u = 0; u < kPoolAhead; ++u) {
+        if (u == 0 || u < left) {
+          asm volatile("");                            // a mask, not a selection per value
+#pragma unroll
+          for (int c = 0; c < VEC; ++c) {
+            // pytorch/jagged_embedding.py:41-45 scales the rows before pooling
+            acc[c] = acc[c] + (WEIGHTED ? v[u][c] * w[u] : v[u][c]);
+          }
+        }
+      }
+    }
+    if (have && last) {
 #pragma unroll
       for (int c = 0; c < VEC; ++c) {
-        // pytorch/jagged_embedding.py:41-45 scales the rows before pooling
-        const float x = WEIGHTED ? v[u][c] * w[u] : v[u][c];
-        acc[c] = j0 + u == 0 ? x : acc[c] + x;
+        const float x = mean ? acc[c] * ratio : acc[c];
+        acc[c] = left > 0 ? x : patch;                 // (left is 0 here for an empty bag only)
       }
+      if (part) vstore_once<VEC>(out + (first + bag) * (int64_t)dim + gl * VEC, acc);
+#pragma unroll
+      for (int c = 0; c < VEC; ++c) acc[c] = -0.0f;
     }
+    have = next_have;
+    bag = next_bag;
+    at = next_at;
+    left = next_left;
+    if (!__any(have)) break;
   }
 }
 
 template <int VEC>
 __device__ __forceinline__ void pooled_sum_body(const TableView& tv, const uint32_t* __restrict__ rows,
                                                 const uint64_t* __restrict__ ids, int64_t n,
-                                                const long long* __restrict__ offsets, int64_t bag,
-                                                const float* __restrict__ weights, int mean, float patch,
-                                                float* __restrict__ out, int dim, int gl) {
-  long long lo = offsets[bag], hi = offsets[bag + 1];
-  if (lo < 0) lo = 0;
-  if (hi > n) hi = n;
-  float acc[VEC];
-#pragma unroll
-  for (int c = 0; c < VEC; ++c) acc[c] = patch;
-  const int count = hi > lo ? (int)(hi - lo) : 0;       // (a request has fewer than 2^31 positions)
-  if (weights) {
-    pooled_add<VEC, true>(tv, rows + lo, ids + lo, count, weights + lo, gl, acc);
+                                                const long long* __restrict__ offsets, int64_t first, int64_t bags,
+                                                int take, const float* __restrict__ weights, int mean, float patch,
+                                                float* __restrict__ out, int dim, int elems, int group) {
+  if (first >= bags) return;                           // the whole wavefront
+  const int here = bags - first < take ? (int)(bags - first) : take;
+  const int shift = __builtin_ctz(group);              // a power of two
+  const auto run = [&](auto weighted, auto more) {
+    pooled_sum_wave<VEC, weighted.value, more.value>(tv, rows, ids, n, offsets, first, here, weights, mean, patch, out,
+                                                     dim, elems, shift);
+  };
+  const std::true_type yes;
+  const std::false_type no;
+  if (take > kWave >> shift) {
+    if (weights) run(yes, yes); else run(no, yes);
   } else {
-    pooled_add<VEC, false>(tv, rows + lo, ids + lo, count, nullptr, gl, acc);
+    if (weights) run(yes, no); else run(no, no);
   }
-  if (mean && hi > lo) {
-    const float ratio = (float)(1.0 / (double)(float)(hi - lo));   // jagged_ops.cc:219
-#pragma unroll
-    for (int c = 0; c < VEC; ++c) acc[c] = acc[c] * ratio;
-  }
-  vstore_once<VEC>(out + bag * (int64_t)dim + gl * VEC, acc);
 }
 
+// take: the bags of a wavefront (pooled_take)
 template <int VEC>
 __global__ __launch_bounds__(kBlock) void pooled_sum_kernel(TableView tv, const uint32_t* __restrict__ rows,
                                                             const uint64_t* __restrict__ ids,
                                                             int64_t n, const long long* __restrict__ offsets,
                                                             int64_t bags, const float* __restrict__ weights,
                                                             int mean, float patch, float* __restrict__ out,
-                                                            int dim, int elems, int group) {
-  const int per_block = kBlock / group;
-  const int64_t bag = (int64_t)blockIdx.x * per_block + threadIdx.x / group;
-  const int gl = threadIdx.x & (group - 1);
-  if (bag >= bags || gl >= elems) return;      // the host only launches this with elems <= group
-  pooled_sum_body<VEC>(tv, rows, ids, n, offsets, bag, weights, mean, patch, out, dim, gl);
+                                                            int dim, int elems, int group, int take) {
+  // the host only launches this with elems <= group
+  const int64_t first = ((int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave) * take;
+  pooled_sum_body<VEC>(tv, rows, ids, n, offsets, first, bags, take, weights, mean, patch, out, dim, elems, group);
 }
 
 template <int OPT, int VEC>
@@ -1105,19 +1192,18 @@ __global__ __launch_bounds__(kBlock) void group_pooled_find_kernel(const TableDe
 template <int VEC>
 __global__ __launch_bounds__(kBlock) void group_pooled_sum_kernel(const TableDesc* __restrict__ descs, PooledCall call,
                                                                   const uint32_t* __restrict__ rows, int dim,
-                                                                  int elems, int group) {
+                                                                  int elems, int group, int take) {
   int m = 0;
   if (call.even_blocks) {
     m = (int)(blockIdx.x / call.even_blocks);
   } else {
     while (m + 1 < call.n_tables && blockIdx.x >= call.block_start[m + 1]) ++m;
   }
-  const int64_t bag = (int64_t)(blockIdx.x - call.block_start[m]) * (kBlock / group) + threadIdx.x / group;
-  const int gl = threadIdx.x & (group - 1);
-  if (bag >= call.bag_start[m + 1] - call.bag_start[m] || gl >= elems) return;
+  const int64_t first = ((int64_t)(blockIdx.x - call.block_start[m]) * (kBlock / kWave) + threadIdx.x / kWave) * take;
   const int64_t a = call.row_start[m];
-  pooled_sum_body<VEC>(descs[m].tv, rows + a, call.ids[m], call.row_start[m + 1] - a, call.offsets[m], bag,
-                       call.weights[m], (int)((call.mean_bits >> m) & 1u), call.patch[m], call.rows[m], dim, gl);
+  pooled_sum_body<VEC>(descs[m].tv, rows + a, call.ids[m], call.row_start[m + 1] - a, call.offsets[m], first,
+                       call.bag_start[m + 1] - call.bag_start[m], take, call.weights[m],
+                       (int)((call.mean_bits >> m) & 1u), call.patch[m], call.rows[m], dim, elems, group);
 }
 
 template <int OPT, int VEC>
@@ -2178,6 +2264,15 @@ static bool pooled_few(bool filling, int64_t n, int* left) {
   return *left > 0 && (*left)-- > 0 && n < kTwoLaunchWhileFilling;
 }
 
+// Bags that a wavefront of a pooled sum takes: as many as it has lane groups while that leaves the chip (8192
+// wavefronts at a time) room, and up to 64 of a larger request, so that the groups' bags even out (see
+// pooled_sum_wave; 852k bags of 32 floats with 8 / 16 / 32 / 64 a wavefront 142 / 123 / 113 / 109 us).
+static int pooled_take(int64_t bags, int group) {
+  int take = kWave / group;
+  while (take < kWave && bags >= (int64_t)8192 * 2 * take) take *= 2;
+  return take;
+}
+
 // The launches of one pull of n > 0 ids into d_out [n, dim]; the caller holds the table's lock
 // and has made room for n more rows.
 static int32_t pull_enqueue(krk_sparse* t, const uint64_t* d_ids, int64_t n, float* d_out,
@@ -2333,13 +2428,13 @@ int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, co
     t->noted_ids = nullptr;
     if ((flags & KRK_DEVICE_PTRS) && n > 0) notes = note_room(&t->notes, n);
   }
-  const size_t rows_words = notes ? 0 : ((size_t)(n > 0 ? n : 1) + 63) & ~(size_t)63;
+  const size_t rows_words = notes ? 0 : ((size_t)n + kRowsAhead + 63) & ~(size_t)63;
   KRK_TRY(t->scratch[5].reserve((rows_words + (size_t)kQueues * (size_t)list_capacity) * sizeof(uint32_t)));
   uint32_t* rows = notes ? notes : t->scratch[5].as<uint32_t>();
   uint32_t* todo = t->scratch[5].as<uint32_t>() + rows_words;
-  const int per_block = kBlock / t->group;
+  const int take = pooled_take(bags, t->group);
   // a lane looks up an id of its own, or four lanes one where many are to be inserted
-  const dim3 probe_grid(grid_for(n, few || queued ? kBlock / kBucket : kBlock)), grid(grid_for(bags, per_block)), block(kBlock);
+  const dim3 probe_grid(grid_for(n, few || queued ? kBlock / kBucket : kBlock)), grid(grid_for(bags, take * (kBlock / kWave))), block(kBlock);
   const auto probe = [&](auto vec, auto few) {
     hipLaunchKernelGGL((pooled_probe_kernel<vec.value, few.value>), probe_grid, block, 0, t->stream, t->view(), t->initk,
                        d_ids, n, rows, t->elems);
@@ -2359,7 +2454,7 @@ int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, co
     else if (n > 0)
       with_bool(few, [&](auto few16) { probe(std::integral_constant<int, 4>(), few16); });
     hipLaunchKernelGGL((pooled_sum_kernel<4>), grid, block, 0, t->stream, t->view(), rows, d_ids, n, d_off, bags, d_w,
-                       mean, patch_value, d_out, (int)t->dim, t->elems, t->group);
+                       mean, patch_value, d_out, (int)t->dim, t->elems, t->group, take);
   } else {
     if (queued)
       hipLaunchKernelGGL((pull_missing_kernel<1, true>), small, missing_block, 0, t->stream, t->view(), t->initk,
@@ -2367,7 +2462,7 @@ int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, co
     else if (n > 0)
       with_bool(few, [&](auto few16) { probe(std::integral_constant<int, 1>(), few16); });
     hipLaunchKernelGGL((pooled_sum_kernel<1>), grid, block, 0, t->stream, t->view(), rows, d_ids, n, d_off, bags, d_w,
-                       mean, patch_value, d_out, (int)t->dim, t->elems, t->group);
+                       mean, patch_value, d_out, (int)t->dim, t->elems, t->group, take);
   }
   KRK_HIP(hipGetLastError());
   if (notes) {
@@ -3424,7 +3519,8 @@ int32_t krk_group_pull_pooled_parts(krk_group* g, const krk_pooled_part* in, uin
   const int n_tables = pool.n_tables;
   if (pool.bag_start[n_tables] == 0) return group_finish(g, flags);
   const int64_t total = pool.row_start[n_tables];
-  const int64_t sum_blocks = pooled_layout(&pool, kBlock / g->group);
+  const int take = pooled_take(pool.bag_start[n_tables], g->group);
+  const int64_t sum_blocks = pooled_layout(&pool, take * (kBlock / kWave));
   if (sum_blocks < 0) {
     set_error("combined request too large for one launch; split it");
     return KRK_E_CAPACITY;
@@ -3452,7 +3548,7 @@ int32_t krk_group_pull_pooled_parts(krk_group* g, const krk_pooled_part* in, uin
   }
   KRK_TRY(group_refresh(g));
   // the row of every position, in the notes where they are to stay behind
-  const size_t rows_words = ((size_t)(total > 0 ? total : 1) + 63) & ~(size_t)63;
+  const size_t rows_words = ((size_t)total + kRowsAhead + 63) & ~(size_t)63;
   uint32_t* notes = nullptr;
   if (flags & KRK_NOTE_ROWS) {
     g->noted_ids.clear();
@@ -3499,10 +3595,10 @@ int32_t krk_group_pull_pooled_parts(krk_group* g, const krk_pooled_part* in, uin
   const dim3 sum_grid((unsigned)sum_blocks);
   if (g->vec == 4) {
     hipLaunchKernelGGL((group_pooled_sum_kernel<4>), sum_grid, block, 0, g->stream, g->d_descs, pool, rows,
-                       (int)g->dim, g->elems, g->group);
+                       (int)g->dim, g->elems, g->group, take);
   } else {
     hipLaunchKernelGGL((group_pooled_sum_kernel<1>), sum_grid, block, 0, g->stream, g->d_descs, pool, rows,
-                       (int)g->dim, g->elems, g->group);
+                       (int)g->dim, g->elems, g->group, take);
   }
   KRK_HIP(hipGetLastError());
   if (notes) {

@@ -389,3 +389,36 @@ def test_pooled_pulls_make_rows(api, n, dim, combined):
             assert np.array_equal(o.to_host(), t.Pull(i)[1]), step
     if group:
         group.close()
+
+
+@pytest.mark.parametrize("dim,groups", [(8, 16), (32, 8), (128, 2), (10, 4)])
+@pytest.mark.parametrize("per_wavefront", [1, 2, 32])
+def test_pooled_pulls_of_many_bags(api, dim, groups, per_wavefront):
+    """Requests from whose number of bags on a wavefront takes more of them than it has lane groups (twice and up
+    to 64 as many), with a last wavefront that is not full; sums in position order, bit for bit."""
+    bags = min(8192 * groups * per_wavefront, 8192 * 64) + 5
+    rng = np.random.default_rng(dim + per_wavefront)
+    t = api.SparseTable(dim, api.Initializer.create(api.InitializerType.kNormal, {"stddev": "0.01", "seed": "4"}))
+    every = splitmix64(np.arange(500, dtype=np.uint64))
+    rc, rows = t.Pull(every)
+    assert rc == 0
+    lengths = rng.choice([0, 1, 2, 4, 5, 9], size=bags, p=[.3, .3, .2, .1, .05, .05])
+    off = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int64)
+    pick = rng.integers(0, every.size, size=int(off[-1]))
+    w = rng.standard_normal(pick.size).astype(np.float32)
+    want = np.full((bags, dim), -0.75, np.float32)
+    weighted = want.copy()
+    for u in range(int(lengths.max())):
+        on = np.flatnonzero(lengths > u)
+        at = off[:-1][on] + u
+        row = rows[pick[at]]
+        want[on] = row if u == 0 else want[on] + row
+        row = row * w[at][:, None]
+        weighted[on] = row if u == 0 else weighted[on] + row
+    d_ids, d_off = api.DeviceArray.from_host(every[pick]), api.DeviceArray.from_host(off)
+    rc, got = t.PullPooled(d_ids, d_off, "sum", patch_value=-0.75)
+    assert rc == 0 and np.array_equal(got.to_host(), want)
+    rc, got = t.PullPooled(d_ids, d_off, "mean", patch_value=-0.75, weights=api.DeviceArray.from_host(w))
+    some = lengths > 0
+    weighted[some] *= (1.0 / lengths[some]).astype(np.float32)[:, None]
+    assert rc == 0 and np.array_equal(got.to_host(), weighted)
