@@ -197,6 +197,14 @@ inline int32_t check_flags(uint32_t flags) {
 
 constexpr int kWave = 64;
 
+// Workgroup b of a launch of n runs on XCD b mod 8, and the XCDs' L2 caches are separate. Tiles that write
+// next to each other are therefore given to one XCD: it takes a stretch of consecutive tiles.
+constexpr uint32_t kXcds = 8;
+__device__ __forceinline__ uint32_t xcd_tile(uint32_t b, uint32_t n) {
+  const uint32_t xcd = b % kXcds, each = n / kXcds, more = n % kXcds;
+  return xcd * each + (xcd < more ? xcd : more) + b / kXcds;
+}
+
 // Inclusive prefix sum over a wavefront, all of whose lanes call it. Data-parallel moves inside rows of
 // 16 lanes, then the rows' last lanes broadcast to the rows behind them: a tenth of the cycles of
 // six shuffles through LDS, each of which waits for the one before.

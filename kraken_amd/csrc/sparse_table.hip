@@ -1021,7 +1021,10 @@ __global__ __launch_bounds__(kBlock) void pull_resident_wide_kernel(TableView tv
                                                                     uint32_t* __restrict__ todo, int parity,
                                                                     int dim, int elems,
                                                                     uint32_t* __restrict__ notes) {
-  const int64_t first = ((int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave) * kWideIds;
+  // Rows of 65 to 128 floats: the XCDs write a stretch of the output each (a million Zipf 1.3 ids over rows of
+  // 128 floats 101 -> 93 us; the output alone takes 82 at the rate of a fill). Narrower rows are the same either way.
+  const uint32_t bx = STEPS == 8 ? xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
+  const int64_t first = ((int64_t)bx * (kBlock / kWave) + threadIdx.x / kWave) * kWideIds;
   if (first >= n) return;
   InitK none{};
   pull_wide<VEC, false, STEPS>(tv, none, ids, first, n, out, dim, elems, todo, parity, notes);
