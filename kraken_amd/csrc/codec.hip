@@ -559,7 +559,7 @@ int32_t coo_find_tiles(CooWork* work, const long long* d_idx, int64_t nnz, int64
   out->starts = out->unordered + 1;
   out->tiles = (uint32_t)tiles;
   if (!work->host_unordered) {
-    KRK_HIP(hipHostMalloc((void**)&work->host_unordered, 64, hipHostMallocDefault));
+    KRK_HIP(hipHostMalloc((void**)&work->host_unordered, 64, hipHostMallocCoherent));
     *work->host_unordered = 0u;
   }
   KRK_HIP(hipHostGetDevicePointer((void**)&out->host_unordered, work->host_unordered, 0));
@@ -641,7 +641,7 @@ int32_t krk_dct_create(int64_t n, krk_dct** out) {
     if (e == hipSuccess) e = hipMalloc((void**)&s->tickets, 64);
     if (e == hipSuccess) e = hipMemsetAsync(s->tile_state, 0, state_b, s->stream);
     if (e == hipSuccess) e = hipMemsetAsync(s->tickets, 0, 64, s->stream);
-    if (e == hipSuccess) e = hipHostMalloc((void**)&s->host_sel, 64, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipHostMalloc((void**)&s->host_sel, 64, hipHostMallocCoherent);
     if (e == hipSuccess) e = hipMemsetAsync(s->e, 0, nb, s->stream);   // dct_emitter.cc:54 : val.Clone().Zero()
     if (e == hipSuccess) e = hipMemsetAsync(s->sel, 0, 64, s->stream);
     if (e == hipSuccess) e = hipMemsetAsync(s->hist, 0, kBins * sizeof(uint32_t), s->stream);
@@ -727,7 +727,7 @@ int32_t krk_dct_compress(krk_dct* s, const float* grad, uint64_t life_span, floa
                        dim3(kSingleBlock), 0, s->stream, d_g, s->e, n, (uint32_t)tiles, vec, s->sel, s->tile_state,
                        s->tickets, s->emit_calls, reinterpret_cast<long long*>(idx), val, s->e_next, d_host_sel);
     KRK_HIP(hipGetLastError());
-    KRK_HIP(hipStreamSynchronize(s->stream));
+    KRK_TRY(wait_stream(s->stream));
     *nnz = (int64_t)s->host_sel[3];
   } else {
     const dim3 emit_grid((unsigned)(s->tiles < kCodecGrid ? s->tiles : kCodecGrid));

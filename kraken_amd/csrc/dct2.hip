@@ -501,10 +501,9 @@ static int32_t dct2_run(const float* in, float* out, int64_t n, int32_t keep, ui
   }
   if (e == hipSuccess && host)
     e = hipMemcpy(out, d_out, sizeof(float) * (size_t)out_count, hipMemcpyDeviceToHost);
-  if (e == hipSuccess && !(flags & KRK_ASYNC)) e = hipStreamSynchronize(s);
   if (tmp) (void)hipFree(tmp);
   if (e != hipSuccess) return hip_fail(e, "dct2", __FILE__, __LINE__);
-  return KRK_SUCCESS;
+  return host || (flags & KRK_ASYNC) ? KRK_SUCCESS : wait_stream(s);   // (the copy of a host output has waited)
 }
 
 }  // namespace krk

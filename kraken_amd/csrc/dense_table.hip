@@ -344,9 +344,10 @@ constexpr unsigned kCooGrid = 512;
 // One Optim::Update with a sparse gradient of nnz > 0 entries (device addresses); entries whose
 // index lies outside [0, n) are skipped. wait: the caller waits for the update anyway, so it can be
 // waited for here, and the launches for unordered indices follow only where there are any (three
-// launches that look at a flag and leave: 13 us).
+// launches that look at a flag and leave: 13 us). *waited: nothing is left to wait for.
 static int32_t dense_apply_coo(krk_dense* t, const krk_optim& o, const long long* d_idx, const float* d_val,
-                               int64_t nnz, float lr, bool wait) {
+                               int64_t nnz, float lr, bool wait, bool* waited) {
+  *waited = false;
   if (!t->coo_grad) KRK_HIP(hipMalloc((void**)&t->coo_grad, (size_t)t->n * sizeof(float) + 16));
   if (!coo_tiled(t->n, nnz)) {
     KRK_TRY(coo_densify(&t->coo_work, d_idx, d_val, nnz, t->coo_grad, t->n, t->stream));
@@ -364,8 +365,9 @@ static int32_t dense_apply_coo(krk_dense* t, const krk_optim& o, const long long
   });
   KRK_HIP(hipGetLastError());
   if (wait) {
-    KRK_HIP(hipStreamSynchronize(t->stream));
-    if (__atomic_load_n(t->coo_work.host_unordered, __ATOMIC_RELAXED) != tiles.tag) return KRK_SUCCESS;
+    KRK_TRY(wait_stream(t->stream));
+    *waited = __atomic_load_n(t->coo_work.host_unordered, __ATOMIC_RELAXED) != tiles.tag;
+    if (*waited) return KRK_SUCCESS;
   }
   KRK_TRY(coo_scatter_if_unordered(tiles, d_idx, d_val, nnz, t->coo_grad, t->n, t->stream));
   with_optim(o.type, [&](auto opt) {
@@ -547,6 +549,7 @@ struct DenseGroupLock {
 
 static int32_t dense_finish(krk_dense* t, uint32_t flags) {
   if (flags & KRK_ASYNC) return KRK_SUCCESS;
+  if (flags & KRK_DEVICE_PTRS) return wait_stream(t->stream);
   KRK_HIP(hipStreamSynchronize(t->stream));
   return KRK_SUCCESS;
 }
@@ -668,8 +671,10 @@ int32_t krk_dense_push_coo(krk_dense* t, const krk_optim* o, const int64_t* idx,
   const float* d_val;
   KRK_TRY(t->input(idx, (size_t)nnz, flags, 0, &d_idx));
   KRK_TRY(t->input(val, (size_t)nnz, flags, 1, &d_val));
-  KRK_TRY(dense_apply_coo(t, *o, reinterpret_cast<const long long*>(d_idx), d_val, nnz, lr, !(flags & KRK_ASYNC)));
-  return dense_finish(t, flags);
+  bool waited = false;
+  KRK_TRY(dense_apply_coo(t, *o, reinterpret_cast<const long long*>(d_idx), d_val, nnz, lr, !(flags & KRK_ASYNC),
+                          &waited));
+  return waited ? KRK_SUCCESS : dense_finish(t, flags);
 }
 
 int32_t krk_dense_state(krk_dense* t, int32_t state_type, float* out, uint32_t flags) {
@@ -815,6 +820,7 @@ int32_t krk_dense_group_pull(krk_dense_group* g, float* out, uint32_t flags) {
                      g->descs, d_out);
   KRK_HIP(hipGetLastError());
   KRK_TRY(g->output_back(out, (size_t)g->total, flags, 0));
+  if ((flags & KRK_DEVICE_PTRS) && !(flags & KRK_ASYNC)) return wait_stream(g->stream);
   if (!(flags & KRK_ASYNC)) KRK_HIP(hipStreamSynchronize(g->stream));
   return KRK_SUCCESS;
 }
@@ -863,7 +869,9 @@ int32_t krk_dense_group_push(krk_dense_group* g, const krk_optim* o, const float
     });
     KRK_HIP(hipGetLastError());
   }
-  if (!(flags & KRK_ASYNC)) KRK_HIP(hipStreamSynchronize(g->stream));
+  if (flags & KRK_ASYNC) return KRK_SUCCESS;
+  if (flags & KRK_DEVICE_PTRS) return wait_stream(g->stream);
+  KRK_HIP(hipStreamSynchronize(g->stream));
   return KRK_SUCCESS;
 }
 

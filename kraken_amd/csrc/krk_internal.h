@@ -67,8 +67,9 @@ struct DeviceGuard {
 // A host pointer that HIP knows as page-locked (hipHostMalloc, krk_host_malloc, a framework's
 // pinned tensors) can be handed to kernels as it is: they read and write it across PCIe, which
 // saves the staging copy and its launch. Returns the address kernels use, or null when the
-// memory is pageable or not aligned to `align` bytes.
-void* direct_host_pointer(const void* p, size_t align);
+// memory is pageable or not aligned to `align` bytes. coherent: whether the host is sure to see what
+// kernels write there as soon as they have ended (allocated as coherent, which krk_host_malloc does).
+void* direct_host_pointer(const void* p, size_t align, bool* coherent = nullptr);
 
 // Page-locked host memory that grows and is kept.
 struct HostBuffer {
@@ -101,6 +102,34 @@ constexpr size_t kReadAgainMin = (size_t)128 << 10;
 inline size_t host_reads(int64_t reads, int64_t bytes) {
   return (size_t)reads * (bytes < (int64_t)kHostPiece ? kHostPiece : (size_t)bytes);
 }
+// Waiting for the end of a call. hipStreamSynchronize puts a packet of its own into the queue and sleeps on its
+// signal: the host goes on 9.4 us after the launch of an empty kernel and 15 after those of a short kernel and one that
+// writes a word. A host that looks at that word itself goes on after 6.0 and 10.0. So the last launch of a blocking
+// call writes a number into a page-locked word and the host waits for the number to appear. What lies ahead
+// of that launch in its stream has ended by then, and its writes are where kernels that start later, and
+// the host in coherent memory, find them.
+struct StreamWait {
+  uint32_t* word = nullptr;   // null: not open
+  uint32_t ticket = 0;
+  StreamWait() = default;
+  StreamWait(const StreamWait&) = delete;
+  StreamWait& operator=(const StreamWait&) = delete;
+  ~StreamWait() { close(); }
+  static void prepare();   // the memory of the words, with the runtime
+  bool open();    // takes a free word; false where there is none: the call then synchronises with the stream
+  void close();   // gives it back
+};
+// Waits until the word of an open wait holds its number, and closes it. A stream that takes longer than a millisecond,
+// has failed or is being captured is left to hipStreamSynchronize.
+int32_t wait_for(StreamWait* w, hipStream_t stream);
+// The same for a stream whose last launch writes no word: puts a launch behind it that does.
+int32_t wait_stream(hipStream_t stream);
+// Called by the one wavefront of that launch.
+__device__ __forceinline__ void signal_host(uint32_t* word, uint32_t ticket) {
+  __threadfence_system();
+  if (threadIdx.x == 0) __hip_atomic_store(word, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Copies host memory that kernels can address to device memory (both on 16 bytes; whole words).
 int32_t copy_from_host(void* dst, const void* src, size_t bytes, hipStream_t stream);
 
@@ -113,6 +142,17 @@ struct ObjBase {
   HostBuffer bounce[4];
   bool bounced[4] = {false, false, false, false};  // output slot lies in `bounce`
   bool direct[4] = {false, false, false, false};   // output slot is the caller's own page-locked buffer
+  // The end of a blocking call whose last launch writes `waiting`'s word (sparse_finish_begin): whether it has been
+  // waited for, and whether the call has to synchronise after all (an output lies in memory of the caller's that is
+  // not known to be coherent)
+  StreamWait waiting;
+  bool waited = false, incoherent = false;
+  int32_t finish_wait() {
+    if (!waiting.word) KRK_HIP(hipStreamSynchronize(stream));
+    else KRK_TRY(wait_for(&waiting, stream));
+    waited = true;
+    return KRK_SUCCESS;
+  }
   int32_t open_stream();
   void close_stream();
   // Where kernels find a host array: the caller's page-locked memory, page-locked buffer `slot` or
@@ -141,6 +181,7 @@ struct ObjBase {
       return KRK_SUCCESS;
     }
     KRK_TRY(stage[slot].reserve(bytes + 16));
+    incoherent = true;   // the runtime may hold on to the caller's pages until it is asked to synchronise
     KRK_HIP(hipMemcpyAsync(stage[slot].ptr, p, bytes, hipMemcpyHostToDevice, stream));
     *dev = stage[slot].as<T>();
     return KRK_SUCCESS;
@@ -153,8 +194,10 @@ struct ObjBase {
       return KRK_SUCCESS;
     }
     direct[slot] = bounced[slot] = false;
-    if (void* d = direct_host_pointer(p, 16)) {
+    bool coherent = false;
+    if (void* d = direct_host_pointer(p, 16, &coherent)) {
       direct[slot] = true;
+      if (!coherent) incoherent = true;
       *dev = reinterpret_cast<T*>(d);
       return KRK_SUCCESS;
     }
@@ -174,10 +217,11 @@ struct ObjBase {
   int32_t output_back(T* p, size_t count, uint32_t flags, int slot) {
     if ((flags & KRK_DEVICE_PTRS) || !count || direct[slot]) return KRK_SUCCESS;
     if (bounced[slot]) {
-      KRK_HIP(hipStreamSynchronize(stream));
+      KRK_TRY(finish_wait());
       std::memcpy(p, bounce[slot].ptr, count * sizeof(T));
       return KRK_SUCCESS;
     }
+    waiting.close();   // the copy lies behind the launch that writes its word
     KRK_HIP(hipMemcpyAsync(p, stage[slot].ptr, count * sizeof(T), hipMemcpyDeviceToHost, stream));
     return KRK_SUCCESS;
   }

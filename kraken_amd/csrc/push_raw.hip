@@ -1702,12 +1702,12 @@ constexpr int kExpandErr = 8;
 
 static int32_t dedup_count_buffer() {
   if (g_dedup_count) return KRK_SUCCESS;
-  KRK_HIP(hipHostMalloc((void**)&g_dedup_count, 64, hipHostMallocDefault));
+  KRK_HIP(hipHostMalloc((void**)&g_dedup_count, 64, hipHostMallocCoherent));
   return KRK_SUCCESS;
 }
 
 static int32_t dedup_read_count(hipStream_t s, int32_t* u) {
-  KRK_HIP(hipStreamSynchronize(s));
+  KRK_TRY(wait_stream(s));
   *u = *static_cast<volatile int32_t*>(g_dedup_count);
   return KRK_SUCCESS;
 }
@@ -1995,7 +1995,7 @@ int32_t krk_expand_rows(const float* rows, int64_t n_rows, const int64_t* inv, i
                        n_rows, d_out, (int)dim, elems, d_err);
   }
   KRK_HIP(hipGetLastError());
-  KRK_HIP(hipStreamSynchronize(s));
+  KRK_TRY(wait_stream(s));
   if (host) KRK_HIP(hipMemcpy(out, d_out, (size_t)n * (size_t)dim * sizeof(float), hipMemcpyDeviceToHost));
   if (*static_cast<volatile int32_t*>(d_err)) {
     set_error("an index lies outside the %lld rows", (long long)n_rows);

@@ -1,5 +1,7 @@
 // Runtime plumbing of the table engine: error strings, device selection, harness
 // memory helpers, conf parsing, events and the device-wide scan primitive.
+#include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdlib>
 #include <string>
@@ -48,6 +50,7 @@ static int32_t init_device(int device) {
   KRK_HIP(hipSetDevice(device));
   g_device = device;
   KRK_TRY(noalloc_prepare());
+  StreamWait::prepare();
   g_ready = true;
   return KRK_SUCCESS;
 }
@@ -60,7 +63,7 @@ int32_t ensure_runtime() {
   return KRK_SUCCESS;
 }
 
-void* direct_host_pointer(const void* p, size_t align) {
+void* direct_host_pointer(const void* p, size_t align, bool* coherent) {
   if (!p || ((uintptr_t)p & (align - 1))) return nullptr;
   hipPointerAttribute_t attr;
   const hipError_t e = hipPointerGetAttributes(&attr, p);
@@ -69,7 +72,78 @@ void* direct_host_pointer(const void* p, size_t align) {
     return nullptr;
   }
   if (attr.type != hipMemoryTypeHost) return nullptr;
+  if (coherent) *coherent = (attr.allocationFlags & hipHostMallocCoherent) != 0;
   return attr.devicePointer;
+}
+
+// The words that waiting calls have open, a cache line each. A word that is given back while a launch that writes it
+// is still under way (a call that failed in between) may receive an old number over a new one; whoever waits
+// for the new one then finds out from hipStreamSynchronize.
+constexpr int kWaitWords = 64;
+constexpr int kWaitStride = 16;                  // 32-bit words between two of them
+static std::atomic<uint32_t*> g_wait_page{nullptr};
+static std::atomic<uint64_t> g_wait_free{~0ull};
+static std::atomic<uint32_t> g_wait_ticket{0};
+
+void StreamWait::prepare() {
+  if (g_wait_page.load(std::memory_order_acquire)) return;
+  uint32_t* page = nullptr;
+  if (hipHostMalloc((void**)&page, kWaitWords * kWaitStride * sizeof(uint32_t),
+                    hipHostMallocCoherent | hipHostMallocPortable) != hipSuccess) {
+    (void)hipGetLastError();                     // calls synchronise with their streams then
+    return;
+  }
+  std::memset(page, 0, kWaitWords * kWaitStride * sizeof(uint32_t));
+  g_wait_page.store(page, std::memory_order_release);   // (under the runtime's lock) kept for the life of the process
+}
+
+bool StreamWait::open() {
+  close();
+  uint32_t* page = g_wait_page.load(std::memory_order_acquire);
+  if (!page) return false;
+  uint64_t open_words = g_wait_free.load(std::memory_order_relaxed);
+  do {
+    if (open_words == 0) return false;
+  } while (!g_wait_free.compare_exchange_weak(open_words, open_words & (open_words - 1), std::memory_order_acquire));
+  word = page + (size_t)__builtin_ctzll(open_words) * kWaitStride;
+  do {
+    ticket = g_wait_ticket.fetch_add(1, std::memory_order_relaxed) + 1;
+  } while (ticket == 0);
+  return true;
+}
+
+void StreamWait::close() {
+  if (!word) return;
+  const size_t at = (size_t)(word - g_wait_page.load(std::memory_order_relaxed)) / kWaitStride;
+  g_wait_free.fetch_or(1ull << at, std::memory_order_release);
+  word = nullptr;
+}
+
+int32_t wait_for(StreamWait* w, hipStream_t stream) {
+  using clock = std::chrono::steady_clock;
+  const clock::time_point until = clock::now() + std::chrono::milliseconds(1);
+  bool there = false;
+  for (int looks = 0;; ++looks) {
+    there = __atomic_load_n(w->word, __ATOMIC_ACQUIRE) == w->ticket;
+    if (there || ((looks & 63) == 63 && clock::now() > until)) break;
+    __builtin_ia32_pause();
+  }
+  w->close();
+  if (!there) KRK_HIP(hipStreamSynchronize(stream));
+  return KRK_SUCCESS;
+}
+
+__global__ void signal_kernel(uint32_t* word, uint32_t ticket) { signal_host(word, ticket); }
+
+int32_t wait_stream(hipStream_t stream) {
+  StreamWait w;
+  if (!w.open()) {
+    KRK_HIP(hipStreamSynchronize(stream));
+    return KRK_SUCCESS;
+  }
+  hipLaunchKernelGGL(signal_kernel, dim3(1), dim3(1), 0, stream, w.word, w.ticket);
+  KRK_HIP(hipGetLastError());
+  return wait_for(&w, stream);
 }
 
 int32_t DeviceBuffer::reserve(size_t want) {
@@ -91,7 +165,7 @@ int32_t HostBuffer::reserve(size_t want) {
   if (ptr) KRK_HIP(hipHostFree(ptr));
   ptr = nullptr;
   bytes = 0;
-  KRK_HIP(hipHostMalloc(&ptr, want, hipHostMallocDefault));
+  KRK_HIP(hipHostMalloc(&ptr, want, hipHostMallocCoherent));
   bytes = want;
   return KRK_SUCCESS;
 }
@@ -485,7 +559,7 @@ int32_t krk_free(void* dptr) {
 int32_t krk_host_malloc(void** hptr, size_t bytes) {
   if (!hptr) return KRK_E_ARGUMENT;
   KRK_TRY(ensure_runtime());
-  KRK_HIP(hipHostMalloc(hptr, bytes ? bytes : 1, hipHostMallocDefault));
+  KRK_HIP(hipHostMalloc(hptr, bytes ? bytes : 1, hipHostMallocCoherent));
   return KRK_SUCCESS;
 }
 int32_t krk_host_free(void* hptr) {

@@ -1300,12 +1300,20 @@ __global__ void publish_kernel(PublishArgs a) {
 // of its own of, cost 6 us each (160 us for a combined request of 26 tables).
 struct CountersArgs {
   int32_t n;
+  uint32_t* word;      // where the call waits, once the counters are there (null: it synchronises)
+  uint32_t ticket;
   const uint32_t* counters[kMaxGroupTables];
   uint32_t* host[kMaxGroupTables];
 };
-__global__ void counters_kernel(CountersArgs a) {
-  const int i = threadIdx.x / 4, w = threadIdx.x & 3;
-  if (i < a.n) __hip_atomic_store(a.host[i] + w, a.counters[i][w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+__global__ __launch_bounds__(kWave) void counters_kernel(CountersArgs a) {
+  static_assert(2 * kMaxGroupTables == kWave, "two lanes a table");
+  const int i = threadIdx.x / 2, w = 2 * (threadIdx.x & 1);
+  if (i < a.n) {
+    const unsigned long long two = *reinterpret_cast<const unsigned long long*>(a.counters[i] + w);
+    __hip_atomic_store(reinterpret_cast<unsigned long long*>(a.host[i] + w), two, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  if (a.word) signal_host(a.word, a.ticket);
 }
 
 // export: rows in insertion order
@@ -1737,14 +1745,16 @@ static int32_t alloc_slots(uint64_t cap, Slot** out, hipStream_t s) {
 }
 
 // Enqueues what brings the tables' counters to the host.
-static int32_t enqueue_counters(krk_sparse* const* tables, int n, hipStream_t stream) {
+static int32_t enqueue_counters(krk_sparse* const* tables, int n, hipStream_t stream, const StreamWait* wait = nullptr) {
   CountersArgs a;
   a.n = n;
+  a.word = wait ? wait->word : nullptr;
+  a.ticket = wait ? wait->ticket : 0u;
   for (int i = 0; i < n; ++i) {
     a.counters[i] = tables[i]->counters;
     a.host[i] = tables[i]->host_counters;
   }
-  hipLaunchKernelGGL(counters_kernel, dim3(1), dim3(4 * kMaxGroupTables), 0, stream, a);
+  hipLaunchKernelGGL(counters_kernel, dim3(1), dim3(kWave), 0, stream, a);
   KRK_HIP(hipGetLastError());
   return KRK_SUCCESS;
 }
@@ -2041,12 +2051,27 @@ int32_t collect_counters(krk_sparse* t) {
 }
 
 // End of an API call: blocking calls wait, refresh the row count and surface device-side errors.
+// the counters of an object's tables, and the word that its call waits for
+static int32_t enqueue_finish(ObjBase* o, krk_sparse* const* tables, int n) {
+  o->waiting.close();
+  o->waited = false;
+  if (!o->incoherent) o->waiting.open();
+  o->incoherent = false;
+  const int32_t rc = enqueue_counters(tables, n, o->stream, &o->waiting);
+  if (rc != KRK_SUCCESS) o->waiting.close();
+  return rc;
+}
 int32_t sparse_finish_begin(krk_sparse* t, uint32_t flags) {
   if (flags & KRK_ASYNC) return KRK_SUCCESS;
-  return enqueue_counters(&t, 1, t->stream);
+  return enqueue_finish(t, &t, 1);
 }
 int32_t sparse_finish_end(krk_sparse* t, uint32_t flags) {
   if (flags & KRK_ASYNC) return KRK_SUCCESS;
+  if (!t->waited) KRK_TRY(t->finish_wait());
+  return collect_counters(t);
+}
+static int32_t sparse_drain(krk_sparse* t) {
+  KRK_TRY(enqueue_counters(&t, 1, t->stream));
   KRK_HIP(hipStreamSynchronize(t->stream));
   return collect_counters(t);
 }
@@ -2169,7 +2194,7 @@ int32_t krk_sparse_create(int64_t dim, const krk_init* init, int64_t capacity_hi
   if (rc == KRK_SUCCESS) {
     hipError_t e = hipMalloc((void**)&t->counters, kCounterWords * sizeof(uint32_t));
     if (e == hipSuccess) e = hipMemsetAsync(t->counters, 0, kCounterWords * sizeof(uint32_t), t->stream);
-    if (e == hipSuccess) e = hipHostMalloc((void**)&t->host_counters, 16, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipHostMalloc((void**)&t->host_counters, 16, hipHostMallocCoherent);
     if (e == hipSuccess) e = hipHostMalloc((void**)&t->host_pub, 16, hipHostMallocCoherent);
     if (e == hipSuccess) {
       *t->host_pub = 0ull;
@@ -2221,7 +2246,7 @@ int32_t krk_sparse_set_stream(krk_sparse* t, void* stream) {
   hipStream_t next = stream == KRK_OWN_STREAM ? t->own_stream : reinterpret_cast<hipStream_t>(stream);
   if (next == t->stream) return KRK_SUCCESS;
   // what is enqueued on the old stream must be complete before work on the new one may follow
-  KRK_TRY(sparse_finish(t, 0));
+  KRK_TRY(sparse_drain(t));
   t->stream = next;
   return KRK_SUCCESS;
 }
@@ -2252,7 +2277,7 @@ int32_t krk_sparse_reserve(krk_sparse* t, int64_t rows) {
 int32_t krk_sparse_sync(krk_sparse* t) {
   KRK_TRY(check_table(t));
   std::lock_guard<std::mutex> lk(t->mu);
-  return sparse_finish(t, 0);
+  return sparse_drain(t);
 }
 
 // Whether the wavefronts of a pooled pull of n ids that inserts as it looks up take sixteen ids each or 64:
@@ -3046,7 +3071,7 @@ int32_t krk_route_ids(uint64_t table_id, const uint64_t* ring_hash, const uint64
     g_route_pinned = nullptr;
     g_route_pinned_bytes = 0;
     g_route_on_device = nullptr;
-    KRK_HIP(hipHostMalloc((void**)&g_route_pinned, 2 * (up_b + count_b), hipHostMallocDefault));
+    KRK_HIP(hipHostMalloc((void**)&g_route_pinned, 2 * (up_b + count_b), hipHostMallocCoherent));
     g_route_pinned_bytes = 2 * (up_b + count_b);
   }
   const bool same_ring = g_route_on_device == (const void*)d_ring_hash && g_route_last.size() == up_b &&
@@ -3077,7 +3102,7 @@ int32_t krk_route_ids(uint64_t table_id, const uint64_t* ring_hash, const uint64
     if (owner) KRK_HIP(hipMemcpy(owner, d_owner, (size_t)n * 8, hipMemcpyDeviceToHost));
     KRK_HIP(hipMemcpy(perm, d_perm, (size_t)n * 8, hipMemcpyDeviceToHost));
   }
-  KRK_HIP(hipStreamSynchronize(st));
+  KRK_TRY(wait_stream(st));
   g_route_on_device = d_ring_hash;   // only now: a call that failed above leaves the ring to be sent again
   for (int64_t k = 0; k < m; ++k) counts[k] = h_count[k];
   return KRK_SUCCESS;
@@ -3234,13 +3259,13 @@ int32_t krk::group_plan(krk_group* g, const int64_t* offsets, GroupCall* call, i
 
 static int32_t group_finish_begin(krk_group* g, uint32_t flags) {
   if (flags & KRK_ASYNC) return KRK_SUCCESS;
-  return krk::enqueue_counters(g->tables.data(), (int)g->tables.size(), g->stream);
+  return krk::enqueue_finish(g, g->tables.data(), (int)g->tables.size());
 }
 
 // one wait for all members: they share the group's stream
 static int32_t group_finish_end(krk_group* g, uint32_t flags) {
   if (flags & KRK_ASYNC) return KRK_SUCCESS;
-  KRK_HIP(hipStreamSynchronize(g->stream));
+  if (!g->waited) KRK_TRY(g->finish_wait());
   int32_t first = KRK_SUCCESS;
   for (krk_sparse* t : g->tables) {
     const int32_t rc = krk::collect_counters(t);
@@ -3260,6 +3285,7 @@ int32_t krk_group_sync(krk_group* g) {
   if (!g) return KRK_E_ARGUMENT;
   KRK_TRY(ensure_runtime());
   GroupLock lk(g);
+  KRK_HIP(hipStreamSynchronize(g->stream));
   return group_finish(g, 0);
 }
 

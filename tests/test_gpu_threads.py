@@ -169,3 +169,47 @@ def test_group_calls_and_member_calls_from_several_threads(api, oracle):
         assert np.array_equal(gid[og], rid[orr])
         assert np.array_equal(gval[og], rval[orr])
     grp.close()
+
+
+def test_more_blocking_calls_at_once_than_there_are_words_to_wait_on(api):
+    """72 threads, a table each: every call returns after its own work, with its own rows, whichever of
+    the 64 words its wait got, or none."""
+    n_threads, dim = 72, 8
+    tables = [api.SparseTable(dim, api.Initializer.create(api.InitializerType.kConstant, {"value": str(k)}))
+              for k in range(n_threads)]
+    start, errors = threading.Barrier(n_threads), []
+
+    def worker(k):
+        try:
+            rng = np.random.default_rng(k)
+            start.wait()
+            for n in (1, 300, 4000):
+                ids = splitmix64(rng.integers(0, 1 << 40, size=n, dtype=np.uint64))
+                rc, rows = tables[k].Pull(ids)
+                assert rc == 0 and (rows == np.float32(k)).all()
+                assert tables[k].Push(api.Optim.create(api.OptimType.kSGD), np.unique(ids),
+                                      np.zeros((np.unique(ids).size, dim), np.float32), 0.5) == 0
+        except Exception as e:
+            errors.append(e)
+
+    threads = [threading.Thread(target=worker, args=(k,)) for k in range(n_threads)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    assert not errors, errors
+
+
+def test_a_blocking_call_behind_work_that_takes_longer_than_its_wait_looks(api):
+    """The host looks at its word for a millisecond and then synchronises: the call returns only once what it
+    enqueued behind some 20 ms of other work has run."""
+    n = 1 << 26
+    t = api.DenseTable(np.zeros(n, np.float32))
+    g, out = api.DeviceArray.from_host(np.ones(n, np.float32)), api.DeviceArray(n, np.float32)
+    sgd = api.Optim.create(api.OptimType.kSGD)
+    for k in range(1, 3):
+        for _ in range(100):
+            assert t.Push(sgd, g, 1.0, async_=True) == 0
+        assert t.Pull(out=out)[0] == 0
+        got = out.to_host()
+        assert (got == -100.0 * k).all()
