@@ -617,6 +617,16 @@ __global__ __launch_bounds__(kBlock, FEW ? 1 : 8) void pooled_probe_kernel(Table
   pooled_probe_body<VEC>(tv, init, ids, p0, n, rows, elems, FEW ? kFillingIds : kFilling64, FEW);
 }
 
+__device__ __forceinline__ void publish_rows(unsigned long long* host_pub, const uint32_t* counters, uint32_t epoch) {
+  __hip_atomic_store(host_pub, (unsigned long long)counters[0] | ((unsigned long long)epoch << 32), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// the members' counts of a combined request
+struct GroupPublish {
+  uint32_t on;
+  uint32_t epoch[kMaxGroupTables];
+};
+
 // Records of one bag requested together; also the row numbers that one load brings.
 constexpr int kPoolAhead = 4;
 typedef uint32_t vrows_t __attribute__((ext_vector_type(4), aligned(4)));   // row numbers lie on four bytes
@@ -777,14 +787,17 @@ __device__ __forceinline__ void pooled_sum_body(const TableView& tv, const uint3
   }
 }
 
-// take: the bags of a wavefront (pooled_take)
+// take: the bags of a wavefront (pooled_take). publish: where the number of the table's rows goes besides, or null
+// (publish_kernel's work, by a lane of the launch that follows the one that makes rows: 4.4 us and a gap less).
 template <int VEC>
 __global__ __launch_bounds__(kBlock) void pooled_sum_kernel(TableView tv, const uint32_t* __restrict__ rows,
                                                             const uint64_t* __restrict__ ids,
                                                             int64_t n, const long long* __restrict__ offsets,
                                                             int64_t bags, const float* __restrict__ weights,
                                                             int mean, float patch, float* __restrict__ out,
-                                                            int dim, int elems, int group, int take) {
+                                                            int dim, int elems, int group, int take,
+                                                            unsigned long long* publish) {
+  if (publish && blockIdx.x == 0 && threadIdx.x == 0) publish_rows(publish, tv.counters, tv.epoch);
   // the host only launches this with elems <= group
   const int64_t first = ((int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave) * take;
   pooled_sum_body<VEC>(tv, rows, ids, n, offsets, first, bags, take, weights, mean, patch, out, dim, elems, group);
@@ -1195,7 +1208,11 @@ __global__ __launch_bounds__(kBlock) void group_pooled_find_kernel(const TableDe
 template <int VEC>
 __global__ __launch_bounds__(kBlock) void group_pooled_sum_kernel(const TableDesc* __restrict__ descs, PooledCall call,
                                                                   const uint32_t* __restrict__ rows, int dim,
-                                                                  int elems, int group, int take) {
+                                                                  int elems, int group, int take, GroupPublish publish) {
+  if (publish.on && blockIdx.x == 0 && threadIdx.x < call.n_tables) {
+    const TableView& tv = descs[threadIdx.x].tv;       // (a table's page-locked words: its count, and `inserted`)
+    publish_rows(reinterpret_cast<unsigned long long*>(tv.inserted) - 1, tv.counters, publish.epoch[threadIdx.x]);
+  }
   int m = 0;
   if (call.even_blocks) {
     m = (int)(blockIdx.x / call.even_blocks);
@@ -1290,9 +1307,7 @@ struct PublishArgs {
 __global__ void publish_kernel(PublishArgs a) {
   const int i = threadIdx.x;
   if (i >= a.n) return;
-  const uint32_t rows = a.counters[i][0];
-  __hip_atomic_store(a.host_pub[i], (unsigned long long)rows | ((unsigned long long)a.epoch[i] << 32),
-                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  publish_rows(a.host_pub[i], a.counters[i], a.epoch[i]);
 }
 
 // A table's four counters -> its host_counters (pinned), for up to 32 tables: what a blocking call
@@ -2469,6 +2484,8 @@ int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, co
   };
   const dim3 small(kMissingGrid), missing_block(kMissBlock);
   const int mean = mode == KRK_POOL_MEAN;
+  unsigned long long* publish = (flags & KRK_ASYNC) && sparse_wants_publish(t) ? t->host_pub : nullptr;
+  if (publish) t->pub_epoch = t->epoch;
   int parity = 0;
   if (queued) {
     parity = t->pull_parity;
@@ -2482,7 +2499,7 @@ int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, co
     else if (n > 0)
       with_bool(few, [&](auto few16) { probe(std::integral_constant<int, 4>(), few16); });
     hipLaunchKernelGGL((pooled_sum_kernel<4>), grid, block, 0, t->stream, t->view(), rows, d_ids, n, d_off, bags, d_w,
-                       mean, patch_value, d_out, (int)t->dim, t->elems, t->group, take);
+                       mean, patch_value, d_out, (int)t->dim, t->elems, t->group, take, publish);
   } else {
     if (queued)
       hipLaunchKernelGGL((pull_missing_kernel<1, true>), small, missing_block, 0, t->stream, t->view(), t->initk,
@@ -2490,7 +2507,7 @@ int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, co
     else if (n > 0)
       with_bool(few, [&](auto few16) { probe(std::integral_constant<int, 1>(), few16); });
     hipLaunchKernelGGL((pooled_sum_kernel<1>), grid, block, 0, t->stream, t->view(), rows, d_ids, n, d_off, bags, d_w,
-                       mean, patch_value, d_out, (int)t->dim, t->elems, t->group, take);
+                       mean, patch_value, d_out, (int)t->dim, t->elems, t->group, take, publish);
   }
   KRK_HIP(hipGetLastError());
   if (notes) {
@@ -2498,7 +2515,6 @@ int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, co
     t->noted_n = n;
     t->noted_version = t->layout_version;
   }
-  if ((flags & KRK_ASYNC) && sparse_wants_publish(t)) KRK_TRY(sparse_publish(&t, 1, t->stream));
   KRK_TRY(sparse_finish_begin(t, flags));
   KRK_TRY(t->output_back(out, (size_t)bags * t->dim, flags, 3));
   return sparse_finish_end(t, flags);
@@ -3622,12 +3638,16 @@ int32_t krk_group_pull_pooled_parts(krk_group* g, const krk_pooled_part* in, uin
     });
   }
   const dim3 sum_grid((unsigned)sum_blocks);
+  GroupPublish publish{};
+  if (flags & KRK_ASYNC)
+    for (krk_sparse* t : g->tables) publish.on |= sparse_wants_publish(t) ? 1u : 0u;
+  for (int m = 0; publish.on && m < n_tables; ++m) publish.epoch[m] = g->tables[m]->pub_epoch = g->tables[m]->epoch;
   if (g->vec == 4) {
     hipLaunchKernelGGL((group_pooled_sum_kernel<4>), sum_grid, block, 0, g->stream, g->d_descs, pool, rows,
-                       (int)g->dim, g->elems, g->group, take);
+                       (int)g->dim, g->elems, g->group, take, publish);
   } else {
     hipLaunchKernelGGL((group_pooled_sum_kernel<1>), sum_grid, block, 0, g->stream, g->d_descs, pool, rows,
-                       (int)g->dim, g->elems, g->group, take);
+                       (int)g->dim, g->elems, g->group, take, publish);
   }
   KRK_HIP(hipGetLastError());
   if (notes) {
@@ -3635,11 +3655,6 @@ int32_t krk_group_pull_pooled_parts(krk_group* g, const krk_pooled_part* in, uin
     g->noted_offsets.assign(pool.row_start, pool.row_start + n_tables + 1);
     g->noted_versions.clear();
     for (krk_sparse* t : g->tables) g->noted_versions.push_back(t->layout_version);
-  }
-  if (flags & KRK_ASYNC) {
-    bool any = false;
-    for (krk_sparse* t : g->tables) any = any || sparse_wants_publish(t);
-    if (any) KRK_TRY(sparse_publish(g->tables.data(), (int)g->tables.size(), g->stream));
   }
   return group_finish(g, flags);
 }
