@@ -24,6 +24,7 @@
 //                                   request that inserts if so
 #pragma once
 
+#include <type_traits>
 #include <vector>
 
 #include "krk_internal.h"
@@ -362,62 +363,65 @@ __device__ inline ProbeResult probe_insert(const TableView& tv, uint64_t id, boo
   return probe_insert_impl<false>(tv, id, active, gl, group, won, slot, src);
 }
 
+// v of lane R of the four this lane belongs to.
+template <int R>
+__device__ __forceinline__ uint32_t quad_lane(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, R * 0x55, 0xf, 0xf, true);
+}
+// the smallest v of the four
+__device__ __forceinline__ uint32_t quad_min(uint32_t v) {
+  const uint32_t a = (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xf, 0xf, true);   // lanes 1 0 3 2
+  v = a < v ? a : v;
+  const uint32_t b = (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xf, 0xf, true);   // lanes 2 3 0 1
+  return b < v ? b : v;
+}
+
 // The same search for 64 ids of a wavefront at a time, one per lane: every lane hashes its own id once, and
-// then four lanes each read the buckets of sixteen ids, four times over, all of them requested before
-// the first is looked at. With four lanes that all hash the same id a look-up costs 70 to 108 vector
-// instructions per sixteen ids, more than half of the time a large one takes (8.5 million pooled ids
-// 164 us, this way 96-108; four million 75 and 49; a hundred 3.1 and 2.7).
-// hit(lane, row, launch) is called by a lane that found the id of lane `lane`. Returns the lanes whose id
-// was not found (or is the one that equals the empty marker: the caller searches for that one).
-template <typename Hit>
-__device__ __forceinline__ unsigned long long find_many(const TableView& tv, uint64_t id, bool active, Hit hit) {
-  const int lane = wave_lane();
-  const int quad = lane / kBucket, gl = lane & (kBucket - 1);
+// then each four lanes read the buckets of their four ids one after the other, all of them requested before
+// the first is looked at. What the four tell each other passes by data-parallel moves, which cost what an
+// addition does; votes and shuffles of the whole wavefront, for ids sixteen lanes apart, took 228 scalar
+// instructions and twelve trips to LDS for 64 ids (8.5 million pooled ids 98 us, this way 69; with four lanes that
+// all hash the same id 164).
+// Returns the row of the lane's id, or kEmptyRow where it is not there, its creator has not published its row
+// yet, or it equals the empty marker: what the claiming search has to be asked. All lanes of the wavefront.
+__device__ __forceinline__ uint32_t find_own(const TableView& tv, uint64_t id, bool active) {
+  const int gl = wave_lane() & (kBucket - 1);
   const uint32_t nb_mask = (uint32_t)(tv.mask >> 2);   // rows are numbered in 32 bits, so there are fewer buckets
   const uint32_t id_lo = (uint32_t)id, id_hi = (uint32_t)(id >> 32);
   uint32_t b = (uint32_t)mix64(id) & nb_mask;
-  unsigned long long missing = __ballot(active && id == kEmptyKey);
-  unsigned long long open = __ballot(active && id != kEmptyKey);
-  constexpr int kRounds = kWave / (kWave / kBucket);   // of sixteen ids
-  // one bit per lane -> one bit per group of four: whether any of them is set
-  auto quads = [](unsigned long long m) -> unsigned long long {
-    m |= m >> 1;
-    m = (m | m >> 2) & 0x1111111111111111ull;
-    m = (m | m >> 3) & 0x0303030303030303ull;
-    m = (m | m >> 6) & 0x000F000F000F000Full;
-    m = (m | m >> 12) & 0x000000FF000000FFull;
-    return (m | m >> 24) & 0xFFFFull;
-  };
-  for (uint32_t tried = 0; open; ++tried) {
-    if (tried > nb_mask) return missing | open;        // every bucket has been looked at
-    uint4 raw[kRounds];
-#pragma unroll
-    for (int r = 0; r < kRounds; ++r) {
-      const uint32_t part = (uint32_t)(open >> (16 * r)) & 0xFFFFu;   // uniform
-      if (part) {
-        const uint32_t at = (uint32_t)__shfl((int)b, 16 * r + quad);
-        if ((part >> quad) & 1u) raw[r] = *reinterpret_cast<const uint4*>(&tv.slots[(uint64_t)at * kBucket + gl]);
+  uint32_t row = kEmptyRow;
+  bool open = active && id != kEmptyKey;
+  const Slot* mine = tv.slots + gl;
+  for (uint32_t tried = 0;; ++tried) {
+    uint4 raw[kBucket];
+    uint32_t on[kBucket];
+    const auto request = [&](auto r) {
+      on[r.value] = quad_lane<r.value>(open ? 1u : 0u);
+      const uint32_t at = quad_lane<r.value>(b);
+      if (on[r.value]) raw[r.value] = *reinterpret_cast<const uint4*>(mine + (uint64_t)at * kBucket);
+    };
+    const auto look = [&](auto r) {
+      const uint32_t lo = quad_lane<r.value>(id_lo), hi = quad_lane<r.value>(id_hi);
+      const bool match = on[r.value] && raw[r.value].x == lo && raw[r.value].y == hi;
+      const uint32_t found = quad_min(match ? raw[r.value].z : kEmptyRow);
+      // a bucket fills from slot 0 upwards: the last slot says whether it has an empty one
+      const uint32_t last = quad_lane<kBucket - 1>(raw[r.value].x & raw[r.value].y);
+      if (gl == r.value && on[r.value]) {
+        row = found;
+        open = found == kEmptyRow && last != 0xFFFFFFFFu;
       }
-    }
-    unsigned long long next = 0;
-#pragma unroll
-    for (int r = 0; r < kRounds; ++r) {
-      const uint32_t part = (uint32_t)(open >> (16 * r)) & 0xFFFFu;
-      if (part) {
-        const uint32_t lo = (uint32_t)__shfl((int)id_lo, 16 * r + quad), hi = (uint32_t)__shfl((int)id_hi, 16 * r + quad);
-        const bool on = (part >> quad) & 1u;
-        const bool match = on && raw[r].x == lo && raw[r].y == hi;
-        const bool empty = on && (raw[r].x & raw[r].y) == 0xFFFFFFFFu;
-        if (match) hit(16 * r + quad, raw[r].z, raw[r].w);
-        const unsigned long long found = quads(__ballot(match)), ends = quads(__ballot(empty));
-        missing |= (ends & ~found) << (16 * r);
-        next |= (part & ~found & ~ends) << (16 * r);
-      }
-    }
-    open = next;
+    };
+    request(std::integral_constant<int, 0>());
+    request(std::integral_constant<int, 1>());
+    request(std::integral_constant<int, 2>());
+    request(std::integral_constant<int, 3>());
+    look(std::integral_constant<int, 0>());
+    look(std::integral_constant<int, 1>());
+    look(std::integral_constant<int, 2>());
+    look(std::integral_constant<int, 3>());
+    if (!__any(open) || tried >= nb_mask) return row;  // (every bucket has been looked at)
     b = (b + 1u) & nb_mask;
   }
-  return missing;
 }
 
 // One lane looking an id up by itself (no votes): the rare second look of pooled_sum_kernel.

@@ -585,8 +585,9 @@ __device__ __forceinline__ void pooled_probe_body(const TableView& tv, const Ini
   }
   const bool active = p0 + lane < n;
   const uint64_t id = active ? ids[p0 + lane] : 0;
-  const unsigned long long missing =
-      find_many(tv, id, active, [&](int l, uint32_t row, uint32_t) { rows[p0 + l] = row; });
+  const uint32_t row = find_own(tv, id, active);
+  if (row != kEmptyRow) rows[p0 + lane] = row;
+  const unsigned long long missing = __ballot(active && row == kEmptyRow);
   if (missing == 0ull) return;                         // uniform
   // The ids that are not there, moved together: the lane of the k-th of them goes to lane k (the other lanes
   // send theirs behind), so that up to sixteen are one round.
