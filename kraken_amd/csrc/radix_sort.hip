@@ -3,7 +3,7 @@
 // up in position order (worker/emitter.cc:516-531 walks the request in order).
 //
 // A pass takes one digit of up to nine bits and is three launches with no waiting between workgroups:
-//   1. radix_hist_kernel: every workgroup counts the digits of its tile of 4096 keys in LDS and
+//   1. radix_hist_kernel: every workgroup counts the digits of its tile of 3072 keys in LDS and
 //      writes the counts digit-major, hist[digit][tile];
 //   2. radix_scan_kernel: one workgroup per digit turns its row of counts into the number of
 //      equal digits in earlier tiles, and notes the digit's total;
@@ -15,61 +15,86 @@
 //      piece: pair p of the ordered tile goes to begin[digit] + earlier[digit][tile] +
 //      (p - where the digit starts in the tile).
 // Equal digits keep their order in every pass, so the sort is stable.
+//
+// An XCD takes a stretch of consecutive tiles (xcd_tile): neighbouring tiles write neighbouring counts and, for
+// every digit, neighbouring pieces of some 48 bytes, which meet in its L2 and leave as whole lines (the scatter
+// of 8.5 million pairs 36.6 -> 32.4 us a pass; it moves 136 MB, 24 us at the rate of a copy).
 #include "krk_internal.h"
 
 namespace krk {
 
 namespace {
 
-constexpr int kRsBlock = 1024;
-constexpr int kRsItems = 4;
+// 512 lanes of six keys and 16-bit counts: four workgroups fit a compute unit, and their phases (keys on their way,
+// votes, scans, the tile's way through LDS) overlap. 8.5 million pairs by 24 bits, us: 1024 lanes of four 186, 512 of
+// eight 153, of six 140; of twelve or sixteen 163 and 176.
+constexpr int kRsBlock = 512;
+constexpr int kRsItems = 6;
 constexpr int kRsTile = kRsBlock * kRsItems;     // keys a workgroup takes
 constexpr int kRsWaves = kRsBlock / kWave;
 constexpr int kRsMaxBits = 9;
 constexpr int kRsDigits = 1 << kRsMaxBits;
 
-// lanes of this wavefront (bit mask) whose `digit` equals this lane's
+// lanes of this wavefront (bit mask) whose `digit` equals this lane's: four vector instructions a bit, one vote and,
+// for either half of the mask, a bitwise operation of three operands
 template <int BITS>
 __device__ __forceinline__ unsigned long long same_digit(uint32_t digit) {
-  unsigned long long same = ~0ull;
+  uint32_t lo = ~0u, hi = ~0u;
 #pragma unroll
   for (int b = 0; b < BITS; ++b) {
-    const bool bit = (digit >> b) & 1u;
-    const unsigned long long votes = __ballot(bit);
-    same &= bit ? votes : ~votes;
+    const int32_t bit = (int32_t)(digit << (31 - b)) >> 31;   // all ones or none
+    const unsigned long long votes = __ballot(bit != 0);
+    lo &= ~((uint32_t)votes ^ (uint32_t)bit);
+    hi &= ~((uint32_t)(votes >> 32) ^ (uint32_t)bit);
   }
-  return same;
+  return (unsigned long long)lo | ((unsigned long long)hi << 32);
 }
 
 // The lanes that hold the digit of the wavefront's first lane are counted with one LDS add, the others
 // with one each: a digit that many keys share (the hottest row of a skewed request) is likely
 // that one, and adds to one counter are served one after the other. Finding all equal digits by
 // votes, one per bit, kept the vector units busy for longer than the keys take to arrive (8.5
-// million keys, nine bits: 24 us a pass for 34 MB).
-__global__ __launch_bounds__(kRsBlock) void radix_hist_kernel(const uint32_t* __restrict__ keys, int64_t n,
+// million keys, nine bits: 24 us a pass for 34 MB). 1024 lanes with four keys each took 14.4 us, 256
+// with twelve in three loads, and counts that leave through one XCD's L2, take 10.9.
+constexpr int kHistLanes = 256;
+typedef uint32_t keys4_t __attribute__((ext_vector_type(4), aligned(4)));
+__global__ __launch_bounds__(kHistLanes) void radix_hist_kernel(const uint32_t* __restrict__ keys, int64_t n,
                                                               int shift, int bits, int64_t pitch,
                                                               uint32_t* __restrict__ hist) {
+  constexpr int kPer = kRsTile / kHistLanes;
+  static_assert(kPer % 4 == 0, "four keys a load");
   __shared__ uint32_t count[kRsDigits];
   const int t = threadIdx.x;
   const int lane = t & (kWave - 1);
   const uint32_t mask = (1u << bits) - 1u;
-  if (t < kRsDigits) count[t] = 0u;
-  __syncthreads();
-  const int64_t base = (int64_t)blockIdx.x * kRsTile;
-  uint32_t key[kRsItems];
+  const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int64_t base = (int64_t)tile * kRsTile;
+  uint32_t key[kPer];
+  const bool whole = base + kRsTile <= n;
+  if (whole) {
 #pragma unroll
-  for (int i = 0; i < kRsItems; ++i) {
-    const int64_t j = base + i * kRsBlock + t;
-    key[i] = j < n ? keys[j] : 0u;
+    for (int i = 0; i < kPer / 4; ++i) {
+      const keys4_t x = *reinterpret_cast<const keys4_t*>(keys + base + (int64_t)(i * kHistLanes + t) * 4);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) key[4 * i + q] = x[q];
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int64_t j = base + i * kHistLanes + t;
+      key[i] = j < n ? keys[j] : 0u;
+    }
   }
+  for (int d = t; d <= (int)mask; d += kHistLanes) count[d] = 0u;
+  __syncthreads();
 #pragma unroll
-  for (int i = 0; i < kRsItems; ++i) {
-    const bool live = base + i * kRsBlock + t < n;
+  for (int i = 0; i < kPer; ++i) {
+    const bool live = whole || base + i * kHistLanes + t < n;
     const uint32_t digit = (key[i] >> shift) & mask;
     const unsigned long long on = __ballot(live);
     if (on == 0ull) break;                             // uniform: the tile's tail
     const int leader = __ffsll(on) - 1;
-    const uint32_t shared = __shfl(digit, leader);
+    const uint32_t shared = __builtin_amdgcn_readlane(digit, leader);
     const unsigned long long same = __ballot(live && digit == shared);
     if (lane == leader) {
       atomicAdd(&count[digit], (uint32_t)__popcll(same));
@@ -78,10 +103,10 @@ __global__ __launch_bounds__(kRsBlock) void radix_hist_kernel(const uint32_t* __
     }
   }
   __syncthreads();
-  if (t <= (int)mask) {
-    uint32_t* row = hist + (int64_t)t * pitch;
-    row[blockIdx.x] = count[t];
-    if (blockIdx.x == gridDim.x - 1)
+  for (int d = t; d <= (int)mask; d += kHistLanes) {
+    uint32_t* row = hist + (int64_t)d * pitch;
+    row[tile] = count[d];
+    if (tile == gridDim.x - 1)
       for (int64_t c = (int64_t)gridDim.x; c < pitch; ++c) row[c] = 0u;   // at most seven
   }
 }
@@ -137,7 +162,7 @@ __global__ __launch_bounds__(kScanLanes) void radix_scan_kernel(uint32_t* __rest
 }
 
 template <int BITS>
-__global__ __launch_bounds__(kRsBlock) void radix_scatter_kernel(const uint32_t* __restrict__ keys,
+__global__ __launch_bounds__(kRsBlock, BITS == 9 ? 6 : 8) void radix_scatter_kernel(const uint32_t* __restrict__ keys,
                                                                  const uint32_t* __restrict__ vals, int64_t n,
                                                                  int shift, int64_t pitch,
                                                                  const uint32_t* __restrict__ hist,
@@ -148,15 +173,16 @@ __global__ __launch_bounds__(kRsBlock) void radix_scatter_kernel(const uint32_t*
   constexpr uint32_t kMask = kDigits - 1;
   __shared__ uint32_t gbase[kDigits];                  // where this tile's keys of the digit go in the output
   __shared__ uint32_t lstart[kDigits];                 // where they begin in the tile's own digit order
-  __shared__ uint32_t wave_hist[kRsWaves * kDigits];   // [wave][digit]
+  __shared__ alignas(4) uint16_t wave_hist[kRsWaves * kDigits];   // [wave][digit]
   __shared__ uint32_t wave_total[kRsWaves];
   __shared__ uint32_t skey[kRsTile], sval[kRsTile];    // the tile in digit order
   const int t = threadIdx.x;
   const int lane = t & (kWave - 1);
   const int wave = t / kWave;
+  const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
   // element i of lane l in wavefront w is key w * 256 + i * 64 + l of the tile: a wavefront's
   // keys are consecutive, and taking i in ascending order visits them in tile order
-  const int64_t tile_base = (int64_t)blockIdx.x * kRsTile;
+  const int64_t tile_base = (int64_t)tile * kRsTile;
   const int64_t base = tile_base + wave * (kWave * kRsItems) + lane;
   uint32_t key[kRsItems], val[kRsItems], rank[kRsItems];
 #pragma unroll
@@ -165,7 +191,7 @@ __global__ __launch_bounds__(kRsBlock) void radix_scatter_kernel(const uint32_t*
     key[i] = j < n ? keys[j] : 0xFFFFFFFFu;
     val[i] = j < n ? vals[j] : 0u;
   }
-  for (int i = t; i < kRsWaves * kDigits; i += kRsBlock) wave_hist[i] = 0u;
+  for (int i = t; i < kRsWaves * kDigits / 2; i += kRsBlock) reinterpret_cast<uint32_t*>(wave_hist)[i] = 0u;
   // an exclusive scan over the workgroup's first kDigits lanes (one value each), through wave_total
   auto scan_digits = [&](uint32_t v) -> uint32_t {
     const uint32_t incl = wave_inclusive_sum(v);
@@ -180,7 +206,7 @@ __global__ __launch_bounds__(kRsBlock) void radix_scatter_kernel(const uint32_t*
     uint32_t all = 0, earlier = 0;
     if (t < kDigits) {
       all = total[t];
-      earlier = hist[(int64_t)t * pitch + blockIdx.x];
+      earlier = hist[(int64_t)t * pitch + tile];
     }
     const uint32_t offset = scan_digits(all);            // its barrier: wave_hist is clear, too
     if (t < kDigits) gbase[t] = offset + earlier;
@@ -191,9 +217,9 @@ __global__ __launch_bounds__(kRsBlock) void radix_scatter_kernel(const uint32_t*
     const uint32_t digit = (key[i] >> shift) & kMask;
     const unsigned long long same = same_digit<BITS>(digit) & __ballot(live);
     const uint32_t before = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
-    uint32_t* cell = &wave_hist[wave * kDigits + digit];
+    uint16_t* cell = &wave_hist[wave * kDigits + digit];
     const uint32_t old = *cell;                        // read by all lanes of the digit ...
-    if (live && before == 0) *cell = old + (uint32_t)__popcll(same);   // ... then advanced by their first
+    if (live && before == 0) *cell = (uint16_t)(old + (uint32_t)__popcll(same));   // ... then advanced by their first
     rank[i] = old + before;
   }
   __syncthreads();
@@ -204,7 +230,7 @@ __global__ __launch_bounds__(kRsBlock) void radix_scatter_kernel(const uint32_t*
 #pragma unroll
     for (int w = 0; w < kRsWaves; ++w) {
       const uint32_t c = wave_hist[w * kDigits + t];
-      wave_hist[w * kDigits + t] = mine;
+      wave_hist[w * kDigits + t] = (uint16_t)mine;
       mine += c;
     }
   }
@@ -282,7 +308,7 @@ int32_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uin
     const int shift = pass * width;
     const int w = bits - shift < width ? bits - shift : width;
     const int digits = 1 << w;
-    hipLaunchKernelGGL(radix_hist_kernel, dim3((unsigned)tiles), dim3(kRsBlock), 0, stream, src_k, n, shift, w,
+    hipLaunchKernelGGL(radix_hist_kernel, dim3((unsigned)tiles), dim3(kHistLanes), 0, stream, src_k, n, shift, w,
                        pitch, hist);
     hipLaunchKernelGGL(radix_scan_kernel, dim3((unsigned)digits), dim3(kScanLanes), 0, stream, hist, pitch, total);
     switch (w) {

@@ -195,3 +195,19 @@ def test_push_raw_and_pooled(api, dim, noted, shape):
             each = each * w[:, None]
         want = before - np.float32(0.5) * _sums(inv[:bags * 8], each, u.size)
         assert np.array_equal(t.Pull(u)[1], want), mode
+
+
+@pytest.mark.parametrize("n", [342 * 3072 - 1, 342 * 3072, 342 * 3072 + 1, 2**20 + 1 + 3072])
+@pytest.mark.parametrize("unique", [1, 300, 500, 70_000, 2**19 + 3, None])
+def test_sorted_requests_by_tiles_and_digits(api, n, unique):
+    """Requests that are sorted (more than 2^20 ids): a last tile that is one key short, full, or holds one key, and
+    keys of 1, 9, 17, 20 and 21 bits, in one to three passes of seven to nine."""
+    rng = np.random.default_rng(n)
+    inv = np.arange(n) if unique is None else rng.integers(0, unique, size=n)
+    if unique is not None:
+        inv[:unique] = np.arange(unique)                # in order of first occurrence
+    ids = splitmix64(inv.astype(np.uint64))
+    grads = _grid(rng, (n, 1))
+    u, got_inv, sums = api.dedup_sum(ids, grads)
+    assert np.array_equal(got_inv, inv) and np.array_equal(u, ids[:u.size])
+    assert np.array_equal(sums, _sums(inv, grads, u.size))
