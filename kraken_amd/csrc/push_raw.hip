@@ -40,12 +40,17 @@ struct alignas(16) DSlot {   // read in one piece
 // and at most one atomic per workgroup instead of 256, and a workgroup of all-distinct ids pays
 // one LDS atomic per lane rather than a vote per distinct id.
 constexpr int kDedupBlock = 1024;
-constexpr int kDedupLds = 2048;   // entries: at most half full
+// Requests of up to 2^16 ids take workgroups of a quarter of that (BLOCK): 26,624 ids are 26 workgroups of 1024 lanes, on
+// a tenth of the chip, each of which waits for sixteen wavefronts at every barrier.
+constexpr int kDedupMidBlock = 256;
+constexpr int64_t kDedupMid = (int64_t)kDedupMidBlock * kDedupMidBlock;
 
-__global__ __launch_bounds__(kDedupBlock) void dedup_claim_kernel(DSlot* slots, uint64_t mask,
-                                                                  const uint64_t* __restrict__ ids, int64_t n,
-                                                                  uint32_t* __restrict__ slot_of,
-                                                                  uint32_t first_block) {
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void dedup_claim_kernel(DSlot* slots, uint64_t mask,
+                                                            const uint64_t* __restrict__ ids, int64_t n,
+                                                            uint32_t* __restrict__ slot_of, uint32_t first_block) {
+  constexpr int kDedupBlock = BLOCK;
+  constexpr int kDedupLds = 2 * BLOCK;   // entries: at most half full
   __shared__ unsigned long long lkey[kDedupLds + 1];   // the last entry belongs to the all-ones id
   __shared__ uint32_t lmin[kDedupLds + 1];
   __shared__ uint32_t lidx[kDedupLds + 1];
@@ -117,9 +122,14 @@ __global__ __launch_bounds__(kDedupBlock) void dedup_claim_kernel(DSlot* slots, 
 // Flags, a scan of them in three launches and an emit that read the index again took six launches
 // where this takes two: they are bound by the launches up to a few hundred thousand ids (a blocking
 // krk_dedup of 26,624 ids 57 -> 45 us) and by the random reads beyond.
-constexpr int kRankTile = kDedupBlock;
+//
+// CLEAN: the index belongs to the calls of up to 2^16 ids, each of which leaves it as empty as it found it: the
+// first position of an id keeps the slot (kSlotOf), and the emit clears it. A memset ahead of the claims, which
+// is what longer requests take, costs a launch and some 4 us.
+constexpr uint32_t kSlotOf = 0x80000000u;
 
-// Exclusive scan over the 1024 lanes of a workgroup; *all = the sum. Ends behind a barrier.
+// Exclusive scan over the lanes of a workgroup; *all = the sum. Ends behind a barrier.
+template <int kDedupBlock>
 __device__ __forceinline__ uint32_t dedup_block_scan(uint32_t v, uint32_t* wave_total, uint32_t* all) {
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const uint32_t incl = wave_inclusive_sum(v);
@@ -137,16 +147,18 @@ __device__ __forceinline__ uint32_t dedup_block_scan(uint32_t v, uint32_t* wave_
   return before;
 }
 
+template <int kRankTile, bool CLEAN>
 __global__ __launch_bounds__(kRankTile) void dedup_rank_kernel(const DSlot* __restrict__ slots, uint32_t* slot_of,
                                                                int64_t n, uint32_t* __restrict__ rank,
                                                                uint32_t* __restrict__ sums) {
   __shared__ uint32_t wave_total[kRankTile / kWave];
   const int64_t p = (int64_t)blockIdx.x * kRankTile + threadIdx.x;
-  const uint32_t first = p < n ? slots[slot_of[p]].minpos : 0xFFFFFFFFu;
+  const uint32_t slot = p < n ? slot_of[p] : 0u;
+  const uint32_t first = p < n ? slots[slot].minpos : 0xFFFFFFFFu;
   uint32_t all;
-  const uint32_t before = dedup_block_scan(first == (uint32_t)p ? 1u : 0u, wave_total, &all);
+  const uint32_t before = dedup_block_scan<kRankTile>(first == (uint32_t)p ? 1u : 0u, wave_total, &all);
   if (p < n) {
-    slot_of[p] = first;
+    slot_of[p] = CLEAN && first == (uint32_t)p ? kSlotOf | slot : first;
     rank[p] = before;
   }
   if (threadIdx.x == 0) sums[blockIdx.x] = all;
@@ -159,7 +171,7 @@ __global__ __launch_bounds__(kDedupBlock) void dedup_bases_kernel(uint32_t* __re
   for (int64_t at = 0; at < m; at += kDedupBlock) {
     const int64_t j = at + threadIdx.x;
     uint32_t all;
-    const uint32_t before = dedup_block_scan(j < m ? sums[j] : 0u, wave_total, &all);
+    const uint32_t before = dedup_block_scan<kDedupBlock>(j < m ? sums[j] : 0u, wave_total, &all);
     if (j < m) sums[j] = carry + before;
     carry += all;
   }
@@ -168,11 +180,11 @@ __global__ __launch_bounds__(kDedupBlock) void dedup_bases_kernel(uint32_t* __re
 
 // Every position learns its id's index in the unique list from the rank of the id's first position,
 // and the first position also writes the id there. keys / pos (dedup_sum): the index and the position
-// as the pair that is sorted. Up to kEmitScan tiles every workgroup adds the tiles' counts up by
+// as the pair that is sorted. Up to as many tiles as it has lanes every workgroup adds the tiles' counts up by
 // itself (4 KB that all of them read); more of them are a launch of their own (SCANNED).
-constexpr int64_t kEmitScan = kDedupBlock;
-template <bool SCANNED>
-__global__ __launch_bounds__(kDedupBlock) void dedup_emit_kernel(const uint32_t* __restrict__ first_of,
+template <int kDedupBlock, bool SCANNED, bool CLEAN>
+__global__ __launch_bounds__(kDedupBlock) void dedup_emit_kernel(DSlot* __restrict__ slots,
+                                                                 const uint32_t* __restrict__ first_of,
                                                                  const uint32_t* __restrict__ rank,
                                                                  const uint32_t* __restrict__ sums, int64_t tiles,
                                                                  const uint64_t* __restrict__ ids, int64_t n,
@@ -183,14 +195,18 @@ __global__ __launch_bounds__(kDedupBlock) void dedup_emit_kernel(const uint32_t*
                                                                  int32_t* __restrict__ total,
                                                                  int32_t* __restrict__ host_total) {
   __shared__ uint32_t wave_total[kDedupBlock / kWave];
-  __shared__ uint32_t base[kEmitScan];
+  __shared__ uint32_t base[kDedupBlock];
   const int64_t p = (int64_t)blockIdx.x * kDedupBlock + threadIdx.x;
-  const uint32_t first = p < n ? first_of[p] : 0u;
+  uint32_t first = p < n ? first_of[p] : 0u;
+  if (CLEAN && (first & kSlotOf)) {
+    *reinterpret_cast<uint4*>(slots + (first & ~kSlotOf)) = uint4{0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu};
+    first = (uint32_t)p;
+  }
   uint32_t all;
   if (SCANNED) {
     all = sums[tiles];
   } else {
-    base[threadIdx.x] = dedup_block_scan((int64_t)threadIdx.x < tiles ? sums[threadIdx.x] : 0u, wave_total, &all);
+    base[threadIdx.x] = dedup_block_scan<kDedupBlock>((int64_t)threadIdx.x < tiles ? sums[threadIdx.x] : 0u, wave_total, &all);
     __syncthreads();
   }
   if (p >= n) return;
@@ -198,7 +214,7 @@ __global__ __launch_bounds__(kDedupBlock) void dedup_emit_kernel(const uint32_t*
     *total = (int32_t)all;
     if (host_total) *host_total = (int32_t)all;        // the count, where a blocking caller reads it
   }
-  const uint32_t r = (SCANNED ? sums[first / kRankTile] : base[first / kRankTile]) + rank[first];
+  const uint32_t r = (SCANNED ? sums[first / kDedupBlock] : base[first / kDedupBlock]) + rank[first];
   if (inv) inv[p] = (long long)r;
   if (keys) {
     keys[p] = r;
@@ -1608,6 +1624,9 @@ extern "C" {
 // under one lock, and they run on the null stream.
 static std::mutex g_dedup_mu;
 static DeviceBuffer g_dedup_pool;
+// The index of calls of up to 2^16 ids (2 MB), empty between them; not known to be while a call's launches are enqueued.
+static DeviceBuffer g_dedup_index;
+static bool g_dedup_index_empty = false;
 static DeviceBuffer g_dedup_reduce[5];
 
 struct DedupWork {
@@ -1618,6 +1637,7 @@ struct DedupWork {
   uint32_t* sums;   // first occurrences of every tile of positions, and one more
   int32_t* d_total;
   char* extra;   // `extra_bytes` more for the caller (staged host arguments)
+  bool clean = false;   // the index is the one that is left empty
 };
 
 static size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
@@ -1625,12 +1645,19 @@ static size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 static int32_t dedup_layout(int64_t n, size_t extra_bytes, DedupWork* w) {
   uint64_t cap = 1024;
   while (cap < (uint64_t)n * 2) cap <<= 1;
-  const size_t slots_b = (cap + 1) * sizeof(DSlot);
+  w->clean = n > kDedupSmall && n <= kDedupMid;
+  const size_t slots_b = w->clean ? 0 : (cap + 1) * sizeof(DSlot);
   const size_t n4 = round256((size_t)n * 4);
-  const size_t sums_b = round256((size_t)(n / kRankTile + 2) * 4);
+  const size_t sums_b = round256((size_t)(n / kDedupMidBlock + 2) * 4);
   KRK_TRY(g_dedup_pool.reserve(slots_b + 2 * n4 + sums_b + 256 + extra_bytes));
   char* cur = g_dedup_pool.as<char>();
   w->slots = reinterpret_cast<DSlot*>(cur); cur += slots_b;
+  if (w->clean) {
+    constexpr size_t kIndexBytes = (2 * kDedupMid + 1) * sizeof(DSlot);
+    if (g_dedup_index.bytes < kIndexBytes) g_dedup_index_empty = false;
+    KRK_TRY(g_dedup_index.reserve(kIndexBytes));
+    w->slots = g_dedup_index.as<DSlot>();
+  }
   w->cap = cap;
   w->slot_of = reinterpret_cast<uint32_t*>(cur); cur += n4;
   w->rank = reinterpret_cast<uint32_t*>(cur); cur += n4;
@@ -1656,31 +1683,51 @@ static int32_t dedup_layout(int64_t n, size_t extra_bytes, DedupWork* w) {
 constexpr unsigned kDedupHead = 32, kDedupHeadSmall = 8;
 
 static void launch_dedup_claims(const DedupWork& w, const uint64_t* d_ids, int64_t n, hipStream_t s) {
+  if (n <= kDedupMid) {
+    const unsigned blocks = grid_for(n, kDedupMidBlock), ahead = kDedupHeadSmall * (kDedupBlock / kDedupMidBlock);
+    const unsigned head = blocks >= 4 * ahead ? ahead : 0;
+    if (head)
+      hipLaunchKernelGGL((dedup_claim_kernel<kDedupMidBlock>), dim3(head), dim3(kDedupMidBlock), 0, s, w.slots, w.cap - 1,
+                         d_ids, n, w.slot_of, 0u);
+    hipLaunchKernelGGL((dedup_claim_kernel<kDedupMidBlock>), dim3(blocks - head), dim3(kDedupMidBlock), 0, s, w.slots,
+                       w.cap - 1, d_ids, n, w.slot_of, head);
+    return;
+  }
   const unsigned blocks = grid_for(n, kDedupBlock);
   unsigned head = 0;
   if (blocks >= 4 * kDedupHeadSmall) {
     head = blocks >= 4 * kDedupHead ? kDedupHead : kDedupHeadSmall;
-    hipLaunchKernelGGL(dedup_claim_kernel, dim3(head), dim3(kDedupBlock), 0, s, w.slots, w.cap - 1, d_ids, n,
-                       w.slot_of, 0u);
+    hipLaunchKernelGGL((dedup_claim_kernel<kDedupBlock>), dim3(head), dim3(kDedupBlock), 0, s, w.slots, w.cap - 1, d_ids,
+                       n, w.slot_of, 0u);
   }
-  hipLaunchKernelGGL(dedup_claim_kernel, dim3(blocks - head), dim3(kDedupBlock), 0, s, w.slots, w.cap - 1, d_ids,
-                     n, w.slot_of, head);
+  hipLaunchKernelGGL((dedup_claim_kernel<kDedupBlock>), dim3(blocks - head), dim3(kDedupBlock), 0, s, w.slots, w.cap - 1,
+                     d_ids, n, w.slot_of, head);
 }
 
 // What follows the claims: ranks, the unique list, the inverse and (keys, pos) where they are asked for.
 static int32_t launch_dedup_emit(const DedupWork& w, const uint64_t* d_ids, int64_t n, uint64_t* d_uids,
                                  long long* d_inv, uint32_t* keys, uint32_t* pos, int32_t* host_total, hipStream_t s) {
-  const int64_t tiles = (n + kRankTile - 1) / kRankTile;
-  const dim3 grid((unsigned)tiles), block(kRankTile);
-  hipLaunchKernelGGL(dedup_rank_kernel, grid, block, 0, s, w.slots, w.slot_of, n, w.rank, w.sums);
-  if (tiles <= kEmitScan) {
-    hipLaunchKernelGGL((dedup_emit_kernel<false>), grid, block, 0, s, w.slot_of, w.rank, w.sums, tiles, d_ids, n, d_uids,
-                       d_inv, keys, pos, w.d_total, host_total);
-  } else {
-    hipLaunchKernelGGL(dedup_bases_kernel, dim3(1), block, 0, s, w.sums, tiles);
-    hipLaunchKernelGGL((dedup_emit_kernel<true>), grid, block, 0, s, w.slot_of, w.rank, w.sums, tiles, d_ids, n, d_uids,
-                       d_inv, keys, pos, w.d_total, host_total);
-  }
+  const auto launch = [&](auto lanes, auto clean) {
+    constexpr int kLanes = lanes.value;
+    const int64_t tiles = (n + kLanes - 1) / kLanes;
+    const dim3 grid((unsigned)tiles), block(kLanes);
+    const auto emit = [&](auto scanned) {
+      hipLaunchKernelGGL((dedup_emit_kernel<lanes.value, scanned.value, clean.value>), grid, block, 0, s, w.slots, w.slot_of,
+                         w.rank, w.sums, tiles, d_ids, n, d_uids, d_inv, keys, pos, w.d_total, host_total);
+    };
+    hipLaunchKernelGGL((dedup_rank_kernel<lanes.value, clean.value>), grid, block, 0, s, w.slots, w.slot_of, n, w.rank,
+                       w.sums);
+    if (tiles <= kLanes) {
+      emit(std::false_type());
+    } else {
+      hipLaunchKernelGGL(dedup_bases_kernel, dim3(1), dim3(kDedupBlock), 0, s, w.sums, tiles);
+      emit(std::true_type());
+    }
+  };
+  using Mid = std::integral_constant<int, kDedupMidBlock>;
+  if (w.clean) launch(Mid(), std::true_type());
+  else if (n <= kDedupMid) launch(Mid(), std::false_type());
+  else launch(std::integral_constant<int, kDedupBlock>(), std::false_type());
   KRK_HIP(hipGetLastError());
   return KRK_SUCCESS;
 }
@@ -1722,9 +1769,16 @@ static int32_t dedup_core(const DedupWork& w, const uint64_t* d_ids, int64_t n, 
     KRK_HIP(hipGetLastError());
     return KRK_SUCCESS;
   }
-  KRK_HIP(hipMemsetAsync(w.slots, 0xFF, (w.cap + 1) * sizeof(DSlot), s));
+  if (!w.clean) {
+    KRK_HIP(hipMemsetAsync(w.slots, 0xFF, (w.cap + 1) * sizeof(DSlot), s));
+  } else if (!g_dedup_index_empty) {
+    KRK_HIP(hipMemsetAsync(w.slots, 0xFF, (2 * kDedupMid + 1) * sizeof(DSlot), s));
+  }
+  g_dedup_index_empty = g_dedup_index_empty && !w.clean;
   launch_dedup_claims(w, d_ids, n, s);
-  return launch_dedup_emit(w, d_ids, n, d_uids, d_inv, keys, pos, g_dedup_count, s);
+  KRK_TRY(launch_dedup_emit(w, d_ids, n, d_uids, d_inv, keys, pos, g_dedup_count, s));
+  g_dedup_index_empty = g_dedup_index_empty || w.clean;
+  return KRK_SUCCESS;
 }
 
 int32_t krk_dedup(const uint64_t* ids, int64_t n, uint64_t* uids, int64_t* inv, int64_t* n_unique,
@@ -1776,7 +1830,7 @@ constexpr int64_t kNoAllocCap = (int64_t)KRK_DEDUP_NOALLOC_MAX * 2;   // index s
 constexpr size_t kNoAllocSlotsBytes = (((size_t)kNoAllocCap + 1) * sizeof(DSlot) + 255) & ~(size_t)255;
 constexpr size_t kNoAllocN4 = (size_t)KRK_DEDUP_NOALLOC_MAX * 4;
 constexpr size_t kNoAllocSumsBytes = 4096;
-static_assert((KRK_DEDUP_NOALLOC_MAX / kRankTile + 2) * 4 <= kNoAllocSumsBytes, "a count per tile of positions");
+static_assert((KRK_DEDUP_NOALLOC_MAX / kDedupBlock + 2) * 4 <= kNoAllocSumsBytes && (kDedupMid / kDedupMidBlock + 2) * 4 <= kNoAllocSumsBytes, "a count per tile of positions");
 constexpr size_t kNoAllocBytes = kNoAllocSlotsBytes + 2 * kNoAllocN4 + kNoAllocSumsBytes + 256;
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];

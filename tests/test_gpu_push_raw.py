@@ -357,3 +357,24 @@ def test_push_raw_short_path_extremes(api, oracle, dim, shape):
         np.add.at(mass, inv, np.abs(grads).astype(np.float64))
         after = t.Pull(u)[1].astype(np.float64)
         assert (np.abs((before - after) - exact) <= 4e-7 * mass + 2e-7 * np.abs(before) + 1e-30).all()
+
+
+def test_dedups_leave_their_index_empty(api):
+    """Calls of 8193 to 2^16 ids share an index that each of them leaves empty; shorter and longer calls, and calls that
+    stage host arrays, use other memory in between. The all-ones id has a slot of its own at each size."""
+    rng = np.random.default_rng(5)
+    for n in (8193, 2**16, 2**16 + 1, 20_000, 100, 8193, 2**16 - 1, 300_000, 9000, 2**16):
+        ids = splitmix64(rng.integers(0, n // 2, size=n).astype(np.uint64))
+        ids[rng.integers(0, n, size=3)] = np.uint64(0xFFFFFFFFFFFFFFFF)
+        _, first, inv = np.unique(ids, return_index=True, return_inverse=True)
+        order = np.argsort(first)                      # of first occurrence
+        place = np.empty_like(order)
+        place[order] = np.arange(order.size)
+        for _ in range(2):
+            u, got = api.dedup(ids)
+            assert np.array_equal(u, ids[first[order]]) and np.array_equal(got, place[inv])
+        grads = (rng.integers(-64, 65, size=(n, 4)) / 4096.0).astype(np.float32)
+        u, got, sums = api.dedup_sum(ids, grads)
+        assert np.array_equal(u, ids[first[order]]) and np.array_equal(got, place[inv])
+        want = np.stack([np.bincount(got, weights=grads[:, c].astype(np.float64), minlength=u.size) for c in range(4)], 1)
+        assert np.array_equal(sums, want.astype(np.float32))
