@@ -264,6 +264,23 @@ __device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t v) {
 #undef KRK_DPP_ADD
   return v;
 }
+// Narrows the lanes of a wavefront (both halves of a mask) to those whose value has bit b as this lane's has it: four
+// vector instructions, one vote and, for either half, a bitwise operation of three operands. All lanes call it.
+__device__ __forceinline__ void match_bit(uint32_t v, int b, uint32_t& lo, uint32_t& hi) {
+  const int32_t bit = (int32_t)(v << (31 - b)) >> 31;   // all ones or none
+  const unsigned long long votes = __ballot(bit != 0);
+  lo &= ~((uint32_t)votes ^ (uint32_t)bit);
+  hi &= ~((uint32_t)(votes >> 32) ^ (uint32_t)bit);
+}
+// the lanes of `among` whose lowest `bits` bits equal this lane's (at most MAX; bits is uniform)
+template <int MAX>
+__device__ __forceinline__ unsigned long long same_value(uint32_t v, unsigned long long among, int bits = MAX) {
+  uint32_t lo = (uint32_t)among, hi = (uint32_t)(among >> 32);
+#pragma unroll
+  for (int b = 0; b < MAX; ++b)
+    if (b < bits) match_bit(v, b, lo, hi);
+  return (unsigned long long)lo | ((unsigned long long)hi << 32);
+}
 constexpr uint64_t kEmptyKey = 0xFFFFFFFFFFFFFFFFull;
 constexpr uint32_t kEmptyRow = 0xFFFFFFFFu;
 

@@ -166,7 +166,8 @@ __global__ __launch_bounds__(LANES) void scatter_kernel(Input in, const uint32_t
   const uint32_t* __restrict__ keys = NOTED ? in.noted.rows : in.keys;
   // element i of lane l in wavefront w is pair w * 256 + i * 64 + l of the tile: a wavefront's
   // pairs are consecutive, and taking i in ascending order visits them in tile order
-  const int64_t base = (int64_t)blockIdx.x * kTile + wave * (kWave * kItems) + lane;
+  const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);   // neighbours' pieces of a bucket meet in one L2
+  const int64_t base = (int64_t)tile * kTile + wave * (kWave * kItems) + lane;
   uint32_t key[kItems], val[kItems], rank[kItems];
 #pragma unroll
   for (int i = 0; i < kItems; ++i) {
@@ -188,14 +189,14 @@ __global__ __launch_bounds__(LANES) void scatter_kernel(Input in, const uint32_t
           for (int k = 0; k < kPer; ++k) {
             const uint32_t x = hist[c * kBuckets + first + k];
             all[k] += x;
-            if (c < (int)blockIdx.x) earlier[k] += x;
+            if (c < (int)tile) earlier[k] += x;
           }
         }
       } else {
 #pragma unroll
         for (int k = 0; k < kPer; ++k) {
           all[k] = total[first + k];
-          earlier[k] = hist[(int64_t)blockIdx.x * kBuckets + first + k];
+          earlier[k] = hist[(int64_t)tile * kBuckets + first + k];
         }
       }
 #pragma unroll
@@ -245,13 +246,7 @@ __global__ __launch_bounds__(LANES) void scatter_kernel(Input in, const uint32_t
     const bool live = place<NOTED>(in, base + i * kWave, key[i], h);
     key[i] = h;
     const uint32_t bucket = h >> shift;
-    unsigned long long same = __ballot(live);
-#pragma unroll
-    for (int b = 0; b < BITS; ++b) {
-      const bool bit = (bucket >> b) & 1u;
-      const unsigned long long votes = __ballot(bit);
-      same &= bit ? votes : ~votes;
-    }
+    const unsigned long long same = same_value<BITS>(bucket, __ballot(live));
     const uint32_t before = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
     uint32_t* cell = &wave_hist[wave * kBuckets + bucket];
     const uint32_t old = *cell;                        // read by all lanes of the bucket ...

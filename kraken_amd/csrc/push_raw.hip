@@ -960,14 +960,7 @@ struct SortCall {
 
 // lanes of this wavefront (bit mask) whose `digit` equals this lane's
 __device__ __forceinline__ unsigned long long match_digit(uint32_t digit) {
-  unsigned long long same = ~0ull;
-#pragma unroll
-  for (int b = 0; b < kDigitBits; ++b) {
-    const bool bit = (digit >> b) & 1u;
-    const unsigned long long votes = __ballot(bit);
-    same &= bit ? votes : ~votes;
-  }
-  return same;
+  return same_value<kDigitBits>(digit, ~0ull);
 }
 
 // exclusive prefix sum of one value per lane over the workgroup (1024 lanes); total to all

@@ -35,21 +35,6 @@ constexpr int kRsWaves = kRsBlock / kWave;
 constexpr int kRsMaxBits = 9;
 constexpr int kRsDigits = 1 << kRsMaxBits;
 
-// lanes of this wavefront (bit mask) whose `digit` equals this lane's: four vector instructions a bit, one vote and,
-// for either half of the mask, a bitwise operation of three operands
-template <int BITS>
-__device__ __forceinline__ unsigned long long same_digit(uint32_t digit) {
-  uint32_t lo = ~0u, hi = ~0u;
-#pragma unroll
-  for (int b = 0; b < BITS; ++b) {
-    const int32_t bit = (int32_t)(digit << (31 - b)) >> 31;   // all ones or none
-    const unsigned long long votes = __ballot(bit != 0);
-    lo &= ~((uint32_t)votes ^ (uint32_t)bit);
-    hi &= ~((uint32_t)(votes >> 32) ^ (uint32_t)bit);
-  }
-  return (unsigned long long)lo | ((unsigned long long)hi << 32);
-}
-
 // The lanes that hold the digit of the wavefront's first lane are counted with one LDS add, the others
 // with one each: a digit that many keys share (the hottest row of a skewed request) is likely
 // that one, and adds to one counter are served one after the other. Finding all equal digits by
@@ -215,7 +200,7 @@ __global__ __launch_bounds__(kRsBlock, BITS == 9 ? 6 : 8) void radix_scatter_ker
   for (int i = 0; i < kRsItems; ++i) {
     const bool live = base + i * kWave < n;            // the tile's tail holds no keys
     const uint32_t digit = (key[i] >> shift) & kMask;
-    const unsigned long long same = same_digit<BITS>(digit) & __ballot(live);
+    const unsigned long long same = same_value<BITS>(digit, __ballot(live));
     const uint32_t before = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
     uint16_t* cell = &wave_hist[wave * kDigits + digit];
     const uint32_t old = *cell;                        // read by all lanes of the digit ...

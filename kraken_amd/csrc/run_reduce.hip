@@ -144,15 +144,7 @@ __device__ __forceinline__ void sort_list(RunLds& s, int len, int bits, int from
     for (int i = 0; i < kListItems; ++i) {
       if (i < per_lane) {                              // uniform
         const uint32_t digit = ((key[i] & key_mask) >> shift) & (uint32_t)(digits - 1);
-        unsigned long long same = ~0ull;
-#pragma unroll
-        for (int b = 0; b < kRunBits; ++b) {
-          if (b < width) {                             // uniform
-            const bool bit = (digit >> b) & 1u;
-            const unsigned long long votes = __ballot(bit);
-            same &= bit ? votes : ~votes;
-          }
-        }
+        const unsigned long long same = same_value<kRunBits>(digit, ~0ull, width);
         const uint32_t before = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
         uint32_t* cell = &hist[wave * digits + digit];
         const uint32_t old = *cell;                    // read by all lanes of the digit ...
