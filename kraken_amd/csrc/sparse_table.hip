@@ -1547,14 +1547,42 @@ __global__ __launch_bounds__(kBlock) void route_rank_kernel(const uint64_t* __re
 // node_count[k] = ids of node k, read off the scanned per-workgroup counts: where node k + 1's
 // ids begin minus where node k's do (thousands of workgroups adding to the same few counters
 // in memory cost more than the rest of the routing together).
+// SCANNED: block_base holds the counts' prefix sums; otherwise the counts themselves, kRouteCounts of them at most, which
+// every workgroup adds up in LDS (a launch that scans a few hundred counts takes 2.2 us and a gap).
+constexpr int kRouteCounts = 2048;
+template <bool SCANNED>
 __global__ __launch_bounds__(kBlock) void route_scatter_kernel(const uint8_t* __restrict__ rank8, int64_t n,
                                                                const int32_t* __restrict__ block_base, int nodes,
                                                                long long* __restrict__ perm,
                                                                int32_t* __restrict__ node_count) {
-  if (blockIdx.x == 0 && (int)threadIdx.x < nodes) {
-    const int64_t k = threadIdx.x, blocks = gridDim.x;
-    const int32_t end = k + 1 < nodes ? block_base[(k + 1) * blocks] : (int32_t)n;
-    node_count[k] = end - block_base[k * blocks];
+  __shared__ int32_t counts[SCANNED ? 1 : kRouteCounts], base[SCANNED ? 1 : kRouteMaxNodes], scan_lds[kBlock / kWave];
+  static_assert(kRouteMaxNodes == kBlock, "a node a lane");
+  if constexpr (SCANNED) {
+    if (blockIdx.x == 0 && (int)threadIdx.x < nodes) {
+      const int64_t k = threadIdx.x, blocks = gridDim.x;
+      const int32_t end = k + 1 < nodes ? block_base[(k + 1) * blocks] : (int32_t)n;
+      node_count[k] = end - block_base[k * blocks];
+    }
+  } else {
+    const int blocks = (int)gridDim.x, t = threadIdx.x;
+    for (int i = t; i < nodes * blocks; i += kBlock) counts[i] = block_base[i];
+    __syncthreads();
+    int32_t earlier = 0, all = 0;
+    if (t < nodes) {
+      for (int b = 0; b < blocks; ++b) {
+        const int32_t c = counts[t * blocks + b];
+        all += c;
+        earlier += b < (int)blockIdx.x ? c : 0;
+      }
+      if (blockIdx.x == 0) node_count[t] = all;
+    }
+    // where node t begins: an exclusive sum over the lanes
+    const int32_t incl = (int32_t)wave_inclusive_sum((uint32_t)all);
+    if (wave_lane() == kWave - 1) scan_lds[t / kWave] = incl;
+    __syncthreads();
+    int32_t begin = incl - all;
+    for (int w = 0; w < t / kWave; ++w) begin += scan_lds[w];
+    base[t] = begin + earlier;
   }
   __shared__ int32_t wave_count[kBlock / kWave][kRouteMaxNodes];
   for (int i = threadIdx.x; i < (kBlock / kWave) * kRouteMaxNodes; i += kBlock) (&wave_count[0][0])[i] = 0;
@@ -1564,20 +1592,14 @@ __global__ __launch_bounds__(kBlock) void route_scatter_kernel(const uint8_t* __
   const uint32_t k = on ? rank8[p] : 0u;
   const int lane = wave_lane();
   const int wave = threadIdx.x / kWave;
-  unsigned long long same = __ballot(on);
-#pragma unroll
-  for (int b = 0; b < 8; ++b) {
-    const bool bit = (k >> b) & 1u;
-    const unsigned long long votes = __ballot(bit);
-    same &= bit ? votes : ~votes;
-  }
+  const unsigned long long same = same_value<8>(k, __ballot(on));
   const int before = __popcll(same & ((1ull << lane) - 1ull));
   if (on && before == 0) wave_count[wave][k] = __popcll(same);
   __syncthreads();
   if (!on) return;
   int offset = before;
   for (int w = 0; w < wave; ++w) offset += wave_count[w][k];
-  perm[block_base[(int64_t)k * gridDim.x + blockIdx.x] + offset] = p;
+  perm[(SCANNED ? block_base[(int64_t)k * gridDim.x + blockIdx.x] : base[k]) + offset] = p;
 }
 
 // ---- erase -------------------------------------------------------------------
@@ -3111,9 +3133,12 @@ int32_t krk_route_ids(uint64_t table_id, const uint64_t* ring_hash, const uint64
                      (unsigned long long)route_hash64(table_id), d_ring_hash, d_ring_rank, (int)ring_n, d_nodes,
                      (int)m, d_owner, d_rank8, d_bc);
   KRK_HIP(hipGetLastError());
-  KRK_TRY(exclusive_scan_i32(d_bc, d_bc, m * blocks, d_total, d_scan, st));
-  hipLaunchKernelGGL(route_scatter_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, st, d_rank8, n, d_bc, (int)m,
-                     d_perm, d_count);
+  const bool scan = m * blocks > kRouteCounts;
+  if (scan) KRK_TRY(exclusive_scan_i32(d_bc, d_bc, m * blocks, d_total, d_scan, st));
+  with_bool(scan, [&](auto scanned) {
+    hipLaunchKernelGGL((route_scatter_kernel<scanned.value>), dim3((unsigned)blocks), dim3(kBlock), 0, st, d_rank8, n,
+                       d_bc, (int)m, d_perm, d_count);
+  });
   KRK_HIP(hipGetLastError());
   if (host) {
     if (owner) KRK_HIP(hipMemcpy(owner, d_owner, (size_t)n * 8, hipMemcpyDeviceToHost));

@@ -269,3 +269,18 @@ def test_route_ids_scan_sizes(api, oracle, n):
     assert np.array_equal(perm.to_host()[:n], np.argsort(rank, kind="stable"))
     assert counts.tolist() == np.bincount(rank, minlength=7).tolist()
 
+
+
+# a workgroup's 256 ids a count: 2048 counts are added up by the launch that uses them, more are scanned
+@pytest.mark.parametrize("nodes,virtual,n", [(1, 1, 1), (8, 64, 255), (8, 64, 256 * 256), (8, 64, 256 * 256 + 1), (256, 8, 2048),
+                                             (256, 8, 2049), (7, 293, 292 * 256), (7, 293, 292 * 256 + 1), (1, 3, 1000)])
+def test_route_ids_counts(api, oracle, nodes, virtual, n):
+    rng = np.random.default_rng(n + nodes)
+    ring = sorted(zip(rng.integers(0, 1 << 64, nodes * virtual, dtype=np.uint64).tolist(),
+                      rng.permutation(np.repeat(np.arange(nodes) * 3, virtual)).tolist()))
+    ids = splitmix64(rng.integers(0, 1 << 40, size=n, dtype=np.uint64))
+    want = oracle.route_owners(ring, 11, ids)
+    node_ids, counts, owner, perm = api.route_ids(11, ring, api.DeviceArray.from_host(ids))
+    assert np.array_equal(owner.to_host(), want) and np.array_equal(node_ids, np.arange(nodes) * 3)
+    assert np.array_equal(perm.to_host(), np.argsort(want, kind="stable"))
+    assert np.array_equal(counts, np.bincount((want // 3).astype(np.int64), minlength=nodes))
