@@ -13,8 +13,8 @@
 //      offsets by one scan over (bucket, wavefront)), puts the tile into bucket order in LDS and
 //      writes it out from there, so that a bucket's pairs of the tile leave as one piece. Its first
 //      workgroup also writes the plan of the reduction.
-// Bound by latencies: 12 us for 50,000 pairs, 26 us for a million (24 MB), against 38 and 57 us for the
-// three passes of a sort by whole row numbers.
+// Bound by latencies: kernels of 12 us for 50,000 pairs, 22 us for a million (24 MB), against 36 and 53 us for
+// the three passes of a sort by whole row numbers.
 #include "reduce_internal.h"
 
 namespace krk {

@@ -1510,7 +1510,8 @@ static int32_t sort_and_reduce(const ReduceShape& sh, hipStream_t stream, Device
 // pairs and a tiled reduction. Buckets spare the sort's passes and the reduction's carry levels, of
 // which a request of 50,000 ids has eight launches; where a request is many times what the chip
 // holds at once, the tiled reduction's walks use the memory better than workgroups that sort first
-// (8.5 million pooled ids of 32 floats: reduction 468 us against 574, partition and sort 180 and 215).
+// (8.5 million pooled ids of 32 floats: reduction 468 us against 574, partition and sort 180 and
+// 215; the sort has come down to 140 since).
 // noted: single tables whose rows the pull noted; fill is not called then.
 template <typename Fill>
 static int32_t fill_and_reduce(const ReduceShape& sh, hipStream_t stream, DeviceBuffer* scratch, const TableView& tv,
@@ -2030,7 +2031,7 @@ int32_t krk_expand_rows(const float* rows, int64_t n_rows, const int64_t* inv, i
     d_inv = s_inv;
   }
   // the word lies in page-locked memory that the kernel writes to: neither a launch that clears it nor
-  // a copy that fetches it (three launches and two waits, 30 us, for what takes one of each, 18 us)
+  // a copy that fetches it (three launches and two waits, 30 us where one of each took 18)
   *static_cast<volatile int32_t*>(d_err) = 0;
   int64_t blocks = (n * elems + kBlock - 1) / kBlock;
   if (blocks > 256 * 64) blocks = 256 * 64;   // grid-stride beyond that

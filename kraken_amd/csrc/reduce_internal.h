@@ -316,8 +316,8 @@ struct RunHash {
 // Requests of more pairs are sorted (radix_sort.hip). Up to here 1024 buckets of 1024 pairs on average, which a
 // workgroup's LDS holds twice over, and the scatter's 32-bit counts of that many buckets for sixteen
 // wavefronts fill 104 of the 160 KB. Pushes just below the line, us, buckets / sort: 2^20 ids of 16
-// floats, distinct / consecutive / Zipf 1.05 / 1.3, 131 / 126 / 104 / 90 against 164 / 154 / 143 / 139; of 128 floats
-// 618 / 607 / 279 / 185 against 638 / 609 / 324 / 236 (rows of 256 and 512 floats, distinct, 1145 and 2236 against
+// floats, distinct / consecutive / Zipf 1.05 / 1.3, 124 / 121 / 98 / 86 against 163 / 150 / 133 / 132; of 128 floats
+// 617 / 602 / 268 / 185 against 640 / 590 / 297 / 217 (rows of 256 and 512 floats, distinct, 1145 and 2236 against
 // 1043 and 2126, Zipf 1.3 310 and 570 against 355 and 648: the sort leaves the rows in the order they lie in).
 // Above it, with 2048 buckets of 16-bit counts, which cost 3 to 9 % below it: 1.5 million ids of 128
 // floats 882 / 868 / 382 / 242 against 886 / 842 / 435 / 301, 2^21 1208 / 1198 / 508 / 313 against 1200 / 1141 / 562 / 382,
