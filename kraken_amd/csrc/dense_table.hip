@@ -339,14 +339,23 @@ __global__ __launch_bounds__(kDenseBlock) void coo_update_kernel(DenseMember m, 
   }
 }
 
+// End of an API call. Host arrays may have been staged by copies of pageable memory, whose pages the runtime may
+// hold on to until it is asked to synchronise: only calls on device memory wait for a word.
+static int32_t dense_finish(krk_dense* t, uint32_t flags) {
+  if (flags & KRK_ASYNC) return KRK_SUCCESS;
+  if (flags & KRK_DEVICE_PTRS) return wait_stream(t->stream);
+  KRK_HIP(hipStreamSynchronize(t->stream));
+  return KRK_SUCCESS;
+}
+
 constexpr unsigned kCooGrid = 512;
 
 // One Optim::Update with a sparse gradient of nnz > 0 entries (device addresses); entries whose
-// index lies outside [0, n) are skipped. wait: the caller waits for the update anyway, so it can be
+// index lies outside [0, n) are skipped. A blocking call waits for the update anyway, so it is
 // waited for here, and the launches for unordered indices follow only where there are any (three
 // launches that look at a flag and leave: 13 us). *waited: nothing is left to wait for.
 static int32_t dense_apply_coo(krk_dense* t, const krk_optim& o, const long long* d_idx, const float* d_val,
-                               int64_t nnz, float lr, bool wait, bool* waited) {
+                               int64_t nnz, float lr, uint32_t flags, bool* waited) {
   *waited = false;
   if (!t->coo_grad) KRK_HIP(hipMalloc((void**)&t->coo_grad, (size_t)t->n * sizeof(float) + 16));
   if (!coo_tiled(t->n, nnz)) {
@@ -364,8 +373,8 @@ static int32_t dense_apply_coo(krk_dense* t, const krk_optim& o, const long long
                        d_idx, d_val, tiles, lr, k);
   });
   KRK_HIP(hipGetLastError());
-  if (wait) {
-    KRK_TRY(wait_stream(t->stream));
+  if (!(flags & KRK_ASYNC)) {
+    KRK_TRY(dense_finish(t, flags));
     *waited = __atomic_load_n(t->coo_work.host_unordered, __ATOMIC_RELAXED) != tiles.tag;
     if (*waited) return KRK_SUCCESS;
   }
@@ -547,13 +556,6 @@ struct DenseGroupLock {
   DenseGroupLock& operator=(const DenseGroupLock&) = delete;
 };
 
-static int32_t dense_finish(krk_dense* t, uint32_t flags) {
-  if (flags & KRK_ASYNC) return KRK_SUCCESS;
-  if (flags & KRK_DEVICE_PTRS) return wait_stream(t->stream);
-  KRK_HIP(hipStreamSynchronize(t->stream));
-  return KRK_SUCCESS;
-}
-
 }  // namespace krk
 
 using namespace krk;
@@ -672,8 +674,7 @@ int32_t krk_dense_push_coo(krk_dense* t, const krk_optim* o, const int64_t* idx,
   KRK_TRY(t->input(idx, (size_t)nnz, flags, 0, &d_idx));
   KRK_TRY(t->input(val, (size_t)nnz, flags, 1, &d_val));
   bool waited = false;
-  KRK_TRY(dense_apply_coo(t, *o, reinterpret_cast<const long long*>(d_idx), d_val, nnz, lr, !(flags & KRK_ASYNC),
-                          &waited));
+  KRK_TRY(dense_apply_coo(t, *o, reinterpret_cast<const long long*>(d_idx), d_val, nnz, lr, flags, &waited));
   return waited ? KRK_SUCCESS : dense_finish(t, flags);
 }
 
