@@ -143,14 +143,27 @@ struct ObjBase {
   bool bounced[4] = {false, false, false, false};  // output slot lies in `bounce`
   bool direct[4] = {false, false, false, false};   // output slot is the caller's own page-locked buffer
   // The end of a blocking call whose last launch writes `waiting`'s word (sparse_finish_begin): whether it has been
-  // waited for, and whether the call has to synchronise after all (an output lies in memory of the caller's that is
-  // not known to be coherent)
+  // waited for, and whether the call has to synchronise instead: the caller's pageable memory takes part in an
+  // asynchronous copy (the runtime may hold on to its pages until then), or an output lies in memory of the
+  // caller's that is not known to be coherent.
   StreamWait waiting;
-  bool waited = false, incoherent = false;
+  bool waited = false, must_synchronise = false;
   int32_t finish_wait() {
-    if (!waiting.word) KRK_HIP(hipStreamSynchronize(stream));
-    else KRK_TRY(wait_for(&waiting, stream));
+    if (waiting.word && !must_synchronise) {
+      KRK_TRY(wait_for(&waiting, stream));
+    } else {
+      KRK_HIP(hipStreamSynchronize(stream));
+      waiting.close();
+      must_synchronise = false;
+    }
     waited = true;
+    return KRK_SUCCESS;
+  }
+  // An asynchronous copy to or from pageable memory of the caller's.
+  int32_t copy_pages(void* dst, const void* src, size_t bytes, hipMemcpyKind kind) {
+    must_synchronise = true;
+    waited = false;   // also where another output of the call has been waited for
+    KRK_HIP(hipMemcpyAsync(dst, src, bytes, kind, stream));
     return KRK_SUCCESS;
   }
   int32_t open_stream();
@@ -181,8 +194,7 @@ struct ObjBase {
       return KRK_SUCCESS;
     }
     KRK_TRY(stage[slot].reserve(bytes + 16));
-    incoherent = true;   // the runtime may hold on to the caller's pages until it is asked to synchronise
-    KRK_HIP(hipMemcpyAsync(stage[slot].ptr, p, bytes, hipMemcpyHostToDevice, stream));
+    KRK_TRY(copy_pages(stage[slot].ptr, p, bytes, hipMemcpyHostToDevice));
     *dev = stage[slot].as<T>();
     return KRK_SUCCESS;
   }
@@ -197,7 +209,7 @@ struct ObjBase {
     bool coherent = false;
     if (void* d = direct_host_pointer(p, 16, &coherent)) {
       direct[slot] = true;
-      if (!coherent) incoherent = true;
+      if (!coherent) must_synchronise = true;
       *dev = reinterpret_cast<T*>(d);
       return KRK_SUCCESS;
     }
@@ -221,9 +233,7 @@ struct ObjBase {
       std::memcpy(p, bounce[slot].ptr, count * sizeof(T));
       return KRK_SUCCESS;
     }
-    waiting.close();   // the copy lies behind the launch that writes its word
-    KRK_HIP(hipMemcpyAsync(p, stage[slot].ptr, count * sizeof(T), hipMemcpyDeviceToHost, stream));
-    return KRK_SUCCESS;
+    return copy_pages(p, stage[slot].ptr, count * sizeof(T), hipMemcpyDeviceToHost);
   }
 };
 

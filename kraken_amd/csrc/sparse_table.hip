@@ -2088,17 +2088,16 @@ int32_t collect_counters(krk_sparse* t) {
   return KRK_SUCCESS;
 }
 
-// End of an API call: blocking calls wait, refresh the row count and surface device-side errors.
-// the counters of an object's tables, and the word that its call waits for
+// Enqueues what ends a blocking call: the counters of the object's tables, and the word that the call waits for.
 static int32_t enqueue_finish(ObjBase* o, krk_sparse* const* tables, int n) {
-  o->waiting.close();
+  o->waiting.close();                                  // (left open by a call that failed)
   o->waited = false;
-  if (!o->incoherent) o->waiting.open();
-  o->incoherent = false;
+  if (!o->must_synchronise) o->waiting.open();
   const int32_t rc = enqueue_counters(tables, n, o->stream, &o->waiting);
   if (rc != KRK_SUCCESS) o->waiting.close();
   return rc;
 }
+// End of an API call: blocking calls wait, refresh the row count and surface device-side errors.
 int32_t sparse_finish_begin(krk_sparse* t, uint32_t flags) {
   if (flags & KRK_ASYNC) return KRK_SUCCESS;
   return enqueue_finish(t, &t, 1);
@@ -2830,9 +2829,8 @@ static int32_t fetch_impl(krk_sparse* t, const uint64_t* ids, int64_t n, uint8_t
   KRK_HIP(hipGetLastError());
   if (vals) KRK_TRY(t->output_back(vals, cells, flags, 1));
   if (state) KRK_TRY(t->output_back(state, cells, flags, 2));
-  if (host && steps)
-    KRK_HIP(hipMemcpyAsync(steps, d_steps, (size_t)n * sizeof(long long), hipMemcpyDeviceToHost, t->stream));
-  if (host && found) KRK_HIP(hipMemcpyAsync(found, d_found, (size_t)n, hipMemcpyDeviceToHost, t->stream));
+  if (host && steps) KRK_TRY(t->copy_pages(steps, d_steps, (size_t)n * sizeof(long long), hipMemcpyDeviceToHost));
+  if (host && found) KRK_TRY(t->copy_pages(found, d_found, (size_t)n, hipMemcpyDeviceToHost));
   return sparse_finish(t, 0);
 }
 
@@ -2886,7 +2884,7 @@ int32_t krk_sparse_erase(krk_sparse* t, const uint64_t* ids, int64_t n, int64_t*
   }
   if (erased) *erased = 0;
   std::lock_guard<std::mutex> lk(t->mu);
-  KRK_TRY(sparse_finish(t, 0));        // drains the stream and reports what earlier calls left
+  KRK_TRY(sparse_finish(t, 0));        // waits for what was enqueued and reports what earlier calls left
   KRK_TRY(refresh_rows(t));
   const int64_t rows = t->size_ub;
   if (n == 0 || rows == 0) return KRK_SUCCESS;

@@ -29,6 +29,9 @@ struct Runtime {
   std::map<const void*, std::string> kernels;
   std::map<uintptr_t, Block> blocks;
   std::map<hipStream_t, bool> pageable;             // an asynchronous copy of pageable memory since the last wait
+  std::vector<uint32_t*> words;                     // of every launch that tells the host, null where it has none
+  int synchronised = 0;
+  uint32_t rows = 0;                                // what the tables' counters say
   dim3 grid, block;
   size_t shmem = 0;
   hipStream_t stream = nullptr;
@@ -54,6 +57,11 @@ static hipError_t give(void* p) {
   free(p);
   return hipSuccess;
 }
+static void tell(uint32_t* word, uint32_t ticket) {
+  rt().words.push_back(word);
+  if (word) __atomic_store_n(word, ticket, __ATOMIC_RELEASE);
+}
+
 extern "C" {
 hipError_t hipMalloc(void** p, size_t bytes) { return take(p, bytes, false, 0); }
 hipError_t hipFree(void* p) { return give(p); }
@@ -78,6 +86,7 @@ hipError_t hipMemcpyAsync(void* d, const void* s, size_t bytes, hipMemcpyKind, h
 hipError_t hipMemset(void* d, int v, size_t bytes) { std::memset(d, v, bytes); return hipSuccess; }
 hipError_t hipMemsetAsync(void* d, int v, size_t bytes, hipStream_t) { std::memset(d, v, bytes); return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t stream) {
+  rt().synchronised++;
   rt().pageable[stream] = false;
   return hipSuccess;
 }
@@ -132,7 +141,21 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shmem, hip
 hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t) {
   const std::string& name = rt().kernels[f];
   if (name.find("signal_kernel") != std::string::npos) {
-    __atomic_store_n(*static_cast<uint32_t**>(args[0]), *static_cast<uint32_t*>(args[1]), __ATOMIC_RELEASE);
+    tell(*static_cast<uint32_t**>(args[0]), *static_cast<uint32_t*>(args[1]));
+  } else if (name.find("counters_kernel") != std::string::npos) {
+    struct Counters {   // CountersArgs of sparse_table.hip
+      int32_t n;
+      uint32_t* word;
+      uint32_t ticket;
+      const uint32_t* counters[32];
+      uint32_t* host[32];
+    };
+    const Counters& a = *static_cast<const Counters*>(args[0]);
+    for (int i = 0; i < a.n; ++i) {
+      std::memset(a.host[i], 0, 16);
+      a.host[i][0] = rt().rows;
+    }
+    tell(a.word, a.ticket);
   }
   return hipSuccess;
 }
@@ -162,6 +185,14 @@ static void whole(const char* what, int32_t rc) {
   rt().pageable.clear();
 }
 
+static krk_sparse* make_table(int64_t dim) {
+  krk_init init;
+  krk_sparse* t = nullptr;
+  CHECK(krk_init_defaults(KRK_INIT_CONSTANT, &init) == 0);
+  CHECK(krk_sparse_create(dim, &init, 1000, &t) == 0);
+  return t;
+}
+
 // Host arrays of megabytes, which are staged by the runtime's copies, and of kilobytes, which are not.
 static void dense_pages(int64_t cells) {
   krk_optim sgd;
@@ -178,12 +209,95 @@ static void dense_pages(int64_t cells) {
   CHECK(krk_dense_destroy(d) == 0);
 }
 
+static void sparse_pages(int64_t n) {
+  const int64_t dim = 8;
+  krk_optim sgd;
+  CHECK(krk_optim_defaults(KRK_SGD, &sgd) == 0);
+  sgd.has_momentum = 1;
+  sgd.momentum = 0.9f;
+  std::vector<uint64_t> ids(n);
+  std::vector<float> rows(n * dim), state(n * dim);
+  std::vector<int32_t> at(n);
+  std::vector<int64_t> steps(n), offsets(n + 1);
+  std::vector<uint8_t> found(n);
+  std::vector<float> wire(2 * (size_t)krk_wire_rows_bytes(n, dim) / 4 + 16);
+  for (int64_t i = 0; i < n; ++i) ids[i] = 3 * (uint64_t)i + 1, offsets[i + 1] = i + 1;
+
+  void* locked = nullptr;
+  CHECK(krk_host_malloc(&locked, n * 8) == 0);
+  std::memcpy(locked, ids.data(), n * 8);
+
+  krk_sparse* t = make_table(dim);
+  whole("pull", krk_sparse_pull(t, ids.data(), n, rows.data(), 0));
+  whole("push", krk_sparse_push(t, &sgd, ids.data(), n, rows.data(), dim, 0.1f, 0));
+  whole("push_raw", krk_sparse_push_raw(t, &sgd, ids.data(), n, rows.data(), dim, 0.1f, 0));
+  whole("pull_pooled", krk_sparse_pull_pooled(t, ids.data(), n, offsets.data(), n, nullptr, KRK_POOL_SUM, 0.0f,
+                                              rows.data(), 0));
+  whole("pull_wire", krk_sparse_pull_wire(t, ids.data(), n, wire.data()));
+  whole("lookup", krk_sparse_lookup(t, ids.data(), n, at.data(), 0));
+  whole("lookup of page-locked ids", krk_sparse_lookup(t, static_cast<uint64_t*>(locked), n, at.data(), 0));
+  whole("fetch by page-locked ids", krk_sparse_fetch(t, static_cast<uint64_t*>(locked), n, nullptr, rows.data(), 1, nullptr,
+                                                     nullptr, 0));
+  whole("import", krk_sparse_import(t, ids.data(), n, rows.data(), 0));
+  whole("import_state", krk_sparse_import_state(t, ids.data(), n, KRK_ST_MOMENTUM_BUFFER, state.data(), steps.data(), 0));
+  whole("fetch", krk_sparse_fetch(t, ids.data(), n, found.data(), rows.data(), KRK_ST_MOMENTUM_BUFFER, state.data(),
+                                  steps.data(), 0));
+  whole("fetch of what is there", krk_sparse_fetch(t, ids.data(), n, found.data(), nullptr, 1, nullptr, nullptr, 0));
+  int64_t exported = 0;
+  rt().rows = (uint32_t)n;
+  whole("export", krk_sparse_export(t, ids.data(), rows.data(), KRK_ST_MOMENTUM_BUFFER, state.data(), steps.data(), n,
+                                    &exported, 0));
+  CHECK(exported == n);
+  whole("export of ids", krk_sparse_export(t, ids.data(), nullptr, 1, nullptr, nullptr, n, &exported, 0));
+  whole("export of values", krk_sparse_export(t, nullptr, rows.data(), 1, nullptr, nullptr, n, &exported, 0));
+  rt().rows = 0;
+  CHECK(krk_sparse_destroy(t) == 0);
+  CHECK(krk_host_free(locked) == 0);
+
+  krk_sparse* members[2] = {make_table(dim), make_table(dim)};
+  krk_group* g = nullptr;
+  CHECK(krk_group_create(members, 2, &g) == 0);
+  const int64_t parts[3] = {0, n / 3, n};
+  whole("group pull", krk_group_pull(g, ids.data(), parts, rows.data(), 0));
+  whole("group push", krk_group_push(g, &sgd, ids.data(), parts, rows.data(), dim, 0.1f, 0));
+  CHECK(krk_group_destroy(g) == 0);
+  for (krk_sparse* m : members) CHECK(krk_sparse_destroy(m) == 0);
+
+}
+
+// After a call that had to synchronise the next ones wait for their word again.
+static void words_after_pages() {
+  const int64_t n = 50000;
+  std::vector<uint64_t> ids(n);
+  std::vector<float> rows(n * 8);
+  krk_sparse* t = make_table(8);
+  whole("pull", krk_sparse_pull(t, ids.data(), n, rows.data(), 0));
+  rt().words.clear();
+  rt().synchronised = 0;
+  whole("pull", krk_sparse_pull(t, ids.data(), 10, rows.data(), 0));
+  CHECK(rt().synchronised == 0 && rt().words.size() == 1 && rt().words[0] != nullptr);
+  // page-locked memory that is not known to be coherent is read after a synchronise, memory that is is not
+  for (const unsigned flags : {(unsigned)hipHostMallocDefault, (unsigned)hipHostMallocCoherent}) {
+    void* out = nullptr;
+    CHECK(hipHostMalloc(&out, 10 * 8 * 4, flags) == hipSuccess);
+    rt().synchronised = 0;
+    whole("pull", krk_sparse_pull(t, ids.data(), 10, static_cast<float*>(out), 0));
+    CHECK((rt().synchronised != 0) == (flags == hipHostMallocDefault));
+    CHECK(hipHostFree(out) == hipSuccess);
+  }
+  CHECK(krk_sparse_destroy(t) == 0);
+}
+
 int main(int argc, char** argv) {
   const std::string which = argc > 1 ? argv[1] : "";
   CHECK(krk_runtime_init(0) == 0);
   if (which == "dense") {
     dense_pages((int64_t)5 << 20);
     dense_pages(2048);
+  } else if (which == "sparse") {
+    sparse_pages(300000);
+    sparse_pages(512);
+    words_after_pages();
   } else {
     return 2;
   }

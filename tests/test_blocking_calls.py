@@ -23,8 +23,8 @@ def program(tmp_path_factory):
     return exe
 
 
-# dense: a blocking call on pageable arrays synchronises after the copies that staged them
-@pytest.mark.parametrize("which", ["dense"])
+# dense, sparse: a blocking call on pageable arrays synchronises after the copies that staged them
+@pytest.mark.parametrize("which", ["dense", "sparse"])
 def test_blocking_calls(program, which):
     r = subprocess.run([program, which], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
