@@ -128,9 +128,10 @@ int32_t wait_for(StreamWait* w, hipStream_t stream) {
     if (there || ((looks & 63) == 63 && clock::now() > until)) break;
     __builtin_ia32_pause();
   }
+  // the word is given back only once nothing is left that writes it (or the stream has failed)
+  const hipError_t e = there ? hipSuccess : hipStreamSynchronize(stream);
   w->close();
-  if (!there) KRK_HIP(hipStreamSynchronize(stream));
-  return KRK_SUCCESS;
+  return e == hipSuccess ? KRK_SUCCESS : hip_fail(e, "hipStreamSynchronize", __FILE__, __LINE__);
 }
 
 __global__ void signal_kernel(uint32_t* word, uint32_t ticket) { signal_host(word, ticket); }

@@ -2,7 +2,9 @@
 // memory is the heap, copies are made at once, and of the kernels only those run that tell the host that
 // a call has ended. It checks what the library asks of the runtime:
 //   - a call that handed pageable memory of the caller's to an asynchronous copy synchronises with its stream
-//     after it, whatever it waits for besides (the runtime may hold on to those pages until then).
+//     after it, whatever it waits for besides (the runtime may hold on to those pages until then);
+//   - a word that a launch under way will still write belongs to the call that waits for it until that launch has
+//     ended, so that no other call waits on the same word; where all words are taken calls synchronise.
 #ifndef __HIP_PLATFORM_AMD__
 #define __HIP_PLATFORM_AMD__
 #endif
@@ -12,7 +14,9 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <map>
+#include <set>
 #include <string>
 #include <vector>
 
@@ -24,14 +28,21 @@ struct Block {
   bool host;
   unsigned flags;
 };
+struct Late {
+  uint32_t* word;
+  uint32_t ticket;
+};
 // Function-local: the library registers its kernels before this file's own variables are constructed.
 struct Runtime {
   std::map<const void*, std::string> kernels;
   std::map<uintptr_t, Block> blocks;
   std::map<hipStream_t, bool> pageable;             // an asynchronous copy of pageable memory since the last wait
+  std::map<hipStream_t, std::vector<Late>> late;    // words that a stream's launches will write
   std::vector<uint32_t*> words;                     // of every launch that tells the host, null where it has none
+  bool signals_late = false;
   int synchronised = 0;
   uint32_t rows = 0;                                // what the tables' counters say
+  std::function<void()> on_synchronise;
   dim3 grid, block;
   size_t shmem = 0;
   hipStream_t stream = nullptr;
@@ -57,9 +68,11 @@ static hipError_t give(void* p) {
   free(p);
   return hipSuccess;
 }
-static void tell(uint32_t* word, uint32_t ticket) {
+static void tell(hipStream_t stream, uint32_t* word, uint32_t ticket) {
   rt().words.push_back(word);
-  if (word) __atomic_store_n(word, ticket, __ATOMIC_RELEASE);
+  if (!word) return;
+  if (rt().signals_late) rt().late[stream].push_back(Late{word, ticket});
+  else __atomic_store_n(word, ticket, __ATOMIC_RELEASE);
 }
 
 extern "C" {
@@ -87,6 +100,9 @@ hipError_t hipMemset(void* d, int v, size_t bytes) { std::memset(d, v, bytes); r
 hipError_t hipMemsetAsync(void* d, int v, size_t bytes, hipStream_t) { std::memset(d, v, bytes); return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t stream) {
   rt().synchronised++;
+  if (rt().on_synchronise) rt().on_synchronise();
+  for (const Late& l : rt().late[stream]) __atomic_store_n(l.word, l.ticket, __ATOMIC_RELEASE);
+  rt().late[stream].clear();
   rt().pageable[stream] = false;
   return hipSuccess;
 }
@@ -138,10 +154,10 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shmem, hip
   *stream = rt().stream;
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t) {
+hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t stream) {
   const std::string& name = rt().kernels[f];
   if (name.find("signal_kernel") != std::string::npos) {
-    tell(*static_cast<uint32_t**>(args[0]), *static_cast<uint32_t*>(args[1]));
+    tell(stream, *static_cast<uint32_t**>(args[0]), *static_cast<uint32_t*>(args[1]));
   } else if (name.find("counters_kernel") != std::string::npos) {
     struct Counters {   // CountersArgs of sparse_table.hip
       int32_t n;
@@ -155,7 +171,7 @@ hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipSt
       std::memset(a.host[i], 0, 16);
       a.host[i][0] = rt().rows;
     }
-    tell(a.word, a.ticket);
+    tell(stream, a.word, a.ticket);
   }
   return hipSuccess;
 }
@@ -288,6 +304,35 @@ static void words_after_pages() {
   CHECK(krk_sparse_destroy(t) == 0);
 }
 
+// Calls whose launches end late, each begun while the one before it synchronises: 64 words, then none.
+static void late_words() {
+  constexpr int kWords = 64, kCalls = kWords + 2;
+  std::vector<krk_sparse*> tables;
+  for (int i = 0; i < kCalls; ++i) tables.push_back(make_table(8));
+  uint64_t id = 7;
+  std::vector<float> row(8);
+  rt().words.clear();
+  rt().signals_late = true;
+  int depth = 0;
+  rt().on_synchronise = [&]() {
+    if (depth + 1 >= kCalls) return;
+    ++depth;
+    CHECK(krk_sparse_pull(tables[depth], &id, 1, row.data(), 0) == KRK_SUCCESS);
+  };
+  CHECK(krk_sparse_pull(tables[0], &id, 1, row.data(), 0) == KRK_SUCCESS);
+  rt().on_synchronise = nullptr;
+  rt().signals_late = false;
+  CHECK((int)rt().words.size() == kCalls);
+  std::set<uint32_t*> different(rt().words.begin(), rt().words.end());
+  CHECK((int)different.size() == kWords + 1 && different.count(nullptr) == 1);
+  // all of them are free again
+  rt().words.clear();
+  rt().synchronised = 0;
+  for (krk_sparse* t : tables) CHECK(krk_sparse_pull(t, &id, 1, row.data(), 0) == KRK_SUCCESS);
+  CHECK(rt().synchronised == 0);
+  for (krk_sparse* t : tables) CHECK(krk_sparse_destroy(t) == 0);
+}
+
 int main(int argc, char** argv) {
   const std::string which = argc > 1 ? argv[1] : "";
   CHECK(krk_runtime_init(0) == 0);
@@ -298,6 +343,8 @@ int main(int argc, char** argv) {
     sparse_pages(300000);
     sparse_pages(512);
     words_after_pages();
+  } else if (which == "words") {
+    late_words();
   } else {
     return 2;
   }

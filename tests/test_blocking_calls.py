@@ -24,7 +24,8 @@ def program(tmp_path_factory):
 
 
 # dense, sparse: a blocking call on pageable arrays synchronises after the copies that staged them
-@pytest.mark.parametrize("which", ["dense", "sparse"])
+# words: no two calls wait on one word, and the calls that find none synchronise
+@pytest.mark.parametrize("which", ["dense", "sparse", "words"])
 def test_blocking_calls(program, which):
     r = subprocess.run([program, which], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
