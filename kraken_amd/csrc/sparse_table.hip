@@ -632,6 +632,56 @@ struct GroupPublish {
 constexpr int kPoolAhead = 4;
 typedef uint32_t vrows_t __attribute__((ext_vector_type(4), aligned(4)));   // row numbers lie on four bytes
 
+// Which of a request's bags are long the host does not know, and 64 neighbours may hold many times the positions of
+// others (bags in order of length, one field's histories behind other fields' single ids): the launch would
+// wait for their wavefront. So a block of `take` bags that holds more than `limit` positions, and clearly more than its
+// longest bag takes time for anyway, is shared out, as many bags a part as a wavefront has lane groups: the block's own
+// wavefront sums the first part up, those of the first kSpareBlocks workgroups of the launch the others, each one
+// the part-th part of every step-th block.
+// 852k bags of 32 floats, look-up and sum in us, a bag per group / blocks of 64 / shared out: 0 to 20 ids each 171 / 114 /
+// 118, the same in ascending order 142 / 107 / 111; one id each, but a hundred in the last thirteenth 141 / 185 / 108; a
+// long tail (Pareto 1.3, to 3000 ids) 881 / 520 / 528, in ascending order 746 / 3635 / 527 (of 128 floats 827 / 13040 / 600).
+// 512 and 256 workgroups: 124 and 182 for the last thirteenth, 1 to 2 us less where nothing is shared out. Not
+// kept: a wavefront's 64 bags from eight places of the request, which evens them out as well, but whose rows then leave in
+// pieces of a kilobyte (0 to 20 ids each 128, one id each 39 for 33).
+constexpr int kSpareBlocks = 1024;
+struct BagShares {
+  int32_t take;           // bags of a block, a power of two
+  int32_t limit;
+};
+__device__ __forceinline__ bool shared_out(const BagShares& by, int64_t positions, int my_count, int groups) {
+  if (positions <= by.limit) return false;             // uniform
+  int longest = my_count;
+#pragma unroll
+  for (int d = 1; d < kWave; d *= 2) {
+    const int other = __shfl_xor(longest, d);
+    longest = other > longest ? other : longest;
+  }
+  return 2 * positions > (int64_t)3 * groups * longest;
+}
+
+// Blocks are numbered in 32 bits: a launch has fewer than 2^25 of them. positions(block) is asked for a block a lane;
+// sum(block, part) by the whole wavefront, for a block of its own (part 0) or one that may be shared out.
+template <typename Positions, typename Sum>
+__device__ __forceinline__ void share_bags(const BagShares& by, int blocks, int groups, Positions positions, Sum sum) {
+  constexpr int kSpare = kSpareBlocks * (kBlock / kWave);
+  const int wave = (int)blockIdx.x * (kBlock / kWave) + __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+  const bool own = wave >= kSpare;
+  const int parts = __builtin_ctz(by.take) - __builtin_ctz(groups);   // their number's logarithm
+  const int step = kSpare >> parts;
+  const int part = own ? 0 : wave & ((1 << parts) - 1);
+  if (!own && part == 0) return;
+  for (int b0 = own ? wave - kSpare : wave >> parts; b0 < blocks; b0 += kWave * step) {
+    unsigned long long m = 1ull;
+    if (!own) {
+      const int b = b0 + wave_lane() * step;
+      m = __ballot(b < blocks && positions(b) > by.limit);
+    }
+    for (; m; m &= m - 1) sum(__builtin_amdgcn_readfirstlane(b0 + __builtin_ctzll(m) * step), part);
+    if (own) return;
+  }
+}
+
 // A wavefront takes `bags` <= 64 bags, the first of which is `first`; lane i knows where bag i begins and how long it
 // is. Its lane groups work on a bag each, four records at a time, and where there are more bags than groups (MORE)
 // a group whose bag ends takes the next one that nobody has: with a bag per group and wavefront, groups waited for the
@@ -645,15 +695,22 @@ template <int VEC, bool WEIGHTED, bool MORE>
 __device__ __forceinline__ void pooled_sum_wave(const TableView& tv, const uint32_t* __restrict__ rows,
                                                 const uint64_t* __restrict__ ids, int64_t n,
                                                 const long long* __restrict__ offsets, int64_t first, int bags,
-                                                const float* __restrict__ weights, int mean, float patch,
-                                                float* __restrict__ out, int dim, int elems, int shift) {
+                                                const BagShares& by, int part, const float* __restrict__ weights,
+                                                int mean, float patch, float* __restrict__ out, int dim, int elems,
+                                                int shift) {
   const int lane = wave_lane();
   const int gl = lane & ((1 << shift) - 1);
   const int sub = lane >> shift;
-  const bool part = gl < elems;
+  const int groups = kWave >> shift;
+  const bool in_row = gl < elems;
   int my_at = 0, my_count = 0;
+  long long lo = 0, hi = 0;
   if (lane < bags) {
-    long long lo = offsets[first + lane], hi = offsets[first + lane + 1];
+    lo = offsets[first + lane];
+    hi = offsets[first + lane + 1];
+  }
+  const long long positions = MORE ? __shfl(hi, bags - 1) - __shfl(lo, 0) : 0;
+  if (lane < bags) {
     if (lo < 0) lo = 0;
     if (hi > n) hi = n;
     if (hi > lo) {                                     // (a request has fewer than 2^31 positions)
@@ -661,18 +718,26 @@ __device__ __forceinline__ void pooled_sum_wave(const TableView& tv, const uint3
       my_count = (int)(hi - lo);
     }
   }
+  int bag = sub, end = bags;                           // this group's bag; the first one that is not this wavefront's
+  if constexpr (MORE) {
+    const bool shared = shared_out(by, positions, my_count, groups);
+    if (part != 0 && !shared) return;                  // uniform
+    bag = part * groups + sub;
+    if (shared && part * groups + groups < bags) end = part * groups + groups;
+  }
   // jagged_ops.cc:219
   const float my_ratio = mean && my_count > 0 ? (float)(1.0 / (double)(float)my_count) : 1.0f;
-  const float* base = tv.recs + (part ? gl * VEC : 0);
+  const float* base = tv.recs + (in_row ? gl * VEC : 0);
   const uint32_t stride = (uint32_t)tv.stride * (uint32_t)sizeof(float);
   const auto record = [&](uint32_t row) {
     return reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + (uint64_t)row * stride);
   };
   const auto numbers = [&](int at) { return *reinterpret_cast<const KRK_GLOBAL vrows_t*>((uintptr_t)(rows + at)); };
   const unsigned long long groups_below = (1ull << (sub << shift)) - 1ull;   // the lanes of the groups before this one
-  int bag = sub, taken = kWave >> shift;               // this group's bag; how many bags have been taken
-  bool have = bag < bags;
+  int taken = part * groups + groups;                  // the next bag that nobody has
+  bool have = bag < end;
   int at = __shfl(my_at, bag), left = __shfl(my_count, bag);
+  if (!have) left = 0;
   vrows_t next = {0u, 0u, 0u, 0u};
   if (left > 0) next = numbers(at);
   float acc[VEC];
@@ -690,7 +755,7 @@ __device__ __forceinline__ void pooled_sum_wave(const TableView& tv, const uint3
       taken += __popcll(ends);
       const int other_at = __shfl(my_at, another & (kWave - 1));
       const int other_count = __shfl(my_count, another & (kWave - 1));
-      if (have && last && another < bags) {
+      if (have && last && another < end) {
         next_have = true;
         next_bag = another;
         next_at = other_at;
@@ -754,7 +819,7 @@ __device__ __forceinline__ void pooled_sum_wave(const TableView& tv, const uint3
         const float x = mean ? acc[c] * ratio : acc[c];
         acc[c] = left > 0 ? x : patch;                 // (left is 0 here for an empty bag only)
       }
-      if (part) vstore_once<VEC>(out + (first + bag) * (int64_t)dim + gl * VEC, acc);
+      if (in_row) vstore_once<VEC>(out + (first + bag) * (int64_t)dim + gl * VEC, acc);
 #pragma unroll
       for (int c = 0; c < VEC; ++c) acc[c] = -0.0f;
     }
@@ -766,42 +831,52 @@ __device__ __forceinline__ void pooled_sum_wave(const TableView& tv, const uint3
   }
 }
 
-template <int VEC>
+template <int VEC, bool MORE>
 __device__ __forceinline__ void pooled_sum_body(const TableView& tv, const uint32_t* __restrict__ rows,
                                                 const uint64_t* __restrict__ ids, int64_t n,
                                                 const long long* __restrict__ offsets, int64_t first, int64_t bags,
-                                                int take, const float* __restrict__ weights, int mean, float patch,
-                                                float* __restrict__ out, int dim, int elems, int group) {
+                                                const BagShares& by, int part, const float* __restrict__ weights,
+                                                int mean, float patch, float* __restrict__ out, int dim, int elems,
+                                                int group) {
   if (first >= bags) return;                           // the whole wavefront
-  const int here = bags - first < take ? (int)(bags - first) : take;
+  const int here = bags - first < by.take ? (int)(bags - first) : by.take;
   const int shift = __builtin_ctz(group);              // a power of two
-  const auto run = [&](auto weighted, auto more) {
-    pooled_sum_wave<VEC, weighted.value, more.value>(tv, rows, ids, n, offsets, first, here, weights, mean, patch, out,
-                                                     dim, elems, shift);
+  const auto run = [&](auto weighted) {
+    pooled_sum_wave<VEC, weighted.value, MORE>(tv, rows, ids, n, offsets, first, here, by, part, weights, mean,
+                                               patch, out, dim, elems, shift);
   };
-  const std::true_type yes;
-  const std::false_type no;
-  if (take > kWave >> shift) {
-    if (weights) run(yes, yes); else run(no, yes);
-  } else {
-    if (weights) run(yes, no); else run(no, no);
-  }
+  if (weights) run(std::true_type()); else run(std::false_type());
 }
 
-// take: the bags of a wavefront (pooled_take). publish: where the number of the table's rows goes besides, or null
+// positions of the bags [first, first + take), as far as they exist
+__device__ __forceinline__ int64_t bag_positions(const long long* __restrict__ offsets, int64_t bags, int64_t first,
+                                                 int take) {
+  if (first >= bags) return 0;
+  return offsets[bags - first < take ? bags : first + take] - offsets[first];
+}
+
+// by.take: the bags of a wavefront (pooled_take); MORE: they are more than its lane groups, and the launch has
+// kSpareBlocks workgroups in front. publish: where the number of the table's rows goes besides, or null
 // (publish_kernel's work, by a lane of the launch that follows the one that makes rows: 4.4 us and a gap less).
-template <int VEC>
-__global__ __launch_bounds__(kBlock) void pooled_sum_kernel(TableView tv, const uint32_t* __restrict__ rows,
-                                                            const uint64_t* __restrict__ ids,
-                                                            int64_t n, const long long* __restrict__ offsets,
-                                                            int64_t bags, const float* __restrict__ weights,
-                                                            int mean, float patch, float* __restrict__ out,
-                                                            int dim, int elems, int group, int take,
-                                                            unsigned long long* publish) {
+// (96 scalar registers leave eight wavefronts a SIMD; with MORE the compiler takes 103, and those 7 go to spare lanes.)
+template <int VEC, bool MORE>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(96))) void pooled_sum_kernel(
+    TableView tv, const uint32_t* __restrict__ rows, const uint64_t* __restrict__ ids, int64_t n,
+    const long long* __restrict__ offsets, int64_t bags, const float* __restrict__ weights, int mean, float patch,
+    float* __restrict__ out, int dim, int elems, int group, BagShares by, unsigned long long* publish) {
   if (publish && blockIdx.x == 0 && threadIdx.x == 0) publish_rows(publish, tv.counters, tv.epoch);
   // the host only launches this with elems <= group
-  const int64_t first = ((int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave) * take;
-  pooled_sum_body<VEC>(tv, rows, ids, n, offsets, first, bags, take, weights, mean, patch, out, dim, elems, group);
+  const auto sum = [&](int64_t first, int part) {
+    pooled_sum_body<VEC, MORE>(tv, rows, ids, n, offsets, first, bags, by, part, weights, mean, patch, out, dim, elems,
+                               group);
+  };
+  if constexpr (MORE) {
+    share_bags(by, (int)((bags + by.take - 1) >> __builtin_ctz(by.take)), kWave / group,
+               [&](int b) { return bag_positions(offsets, bags, (int64_t)b * by.take, by.take); },
+               [&](int b, int part) { sum((int64_t)b * by.take, part); });
+  } else {
+    sum(((int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave) * by.take, 0);
+  }
 }
 
 template <int OPT, int VEC>
@@ -1206,25 +1281,43 @@ __global__ __launch_bounds__(kBlock) void group_pooled_find_kernel(const TableDe
                    (int)((fill.parity_bits >> t) & 1u));
 }
 
-template <int VEC>
-__global__ __launch_bounds__(kBlock) void group_pooled_sum_kernel(const TableDesc* __restrict__ descs, PooledCall call,
-                                                                  const uint32_t* __restrict__ rows, int dim,
-                                                                  int elems, int group, int take, GroupPublish publish) {
+template <int VEC, bool MORE>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(96))) void group_pooled_sum_kernel(
+    const TableDesc* __restrict__ descs, PooledCall call, const uint32_t* __restrict__ rows, int dim, int elems, int group,
+    BagShares by, GroupPublish publish) {
   if (publish.on && blockIdx.x == 0 && threadIdx.x < call.n_tables) {
     const TableView& tv = descs[threadIdx.x].tv;       // (a table's page-locked words: its count, and `inserted`)
     publish_rows(reinterpret_cast<unsigned long long*>(tv.inserted) - 1, tv.counters, publish.epoch[threadIdx.x]);
   }
-  int m = 0;
-  if (call.even_blocks) {
-    m = (int)(blockIdx.x / call.even_blocks);
+  const auto member = [&](uint32_t block) {
+    if (call.even_blocks) return (int)(block / call.even_blocks);
+    int m = 0;
+    while (m + 1 < call.n_tables && block >= call.block_start[m + 1]) ++m;
+    return m;
+  };
+  const auto sum = [&](int m, int64_t first, int part) {
+    const int64_t a = call.row_start[m];
+    pooled_sum_body<VEC, MORE>(descs[m].tv, rows + a, call.ids[m], call.row_start[m + 1] - a, call.offsets[m], first,
+                               call.bag_start[m + 1] - call.bag_start[m], by, part, call.weights[m],
+                               (int)((call.mean_bits >> m) & 1u), call.patch[m], call.rows[m], dim, elems, group);
+  };
+  // a member's blocks of bags are numbered from its first workgroup's wavefronts on
+  constexpr int kWaves = kBlock / kWave;
+  const auto first_of = [&](int b, int m) { return (int64_t)(b - (int)call.block_start[m] * kWaves) * by.take; };
+  if constexpr (MORE) {
+    share_bags(by, (int)call.block_start[call.n_tables] * kWaves, kWave / group,
+               [&](int b) {
+                 const int m = member((uint32_t)b / kWaves);
+                 return bag_positions(call.offsets[m], call.bag_start[m + 1] - call.bag_start[m], first_of(b, m), by.take);
+               },
+               [&](int b, int part) {
+                 const int m = __builtin_amdgcn_readfirstlane(member((uint32_t)b / kWaves));
+                 sum(m, first_of(b, m), part);
+               });
   } else {
-    while (m + 1 < call.n_tables && blockIdx.x >= call.block_start[m + 1]) ++m;
+    const int m = member(blockIdx.x);
+    sum(m, first_of((int)(blockIdx.x * kWaves + threadIdx.x / kWave), m), 0);
   }
-  const int64_t first = ((int64_t)(blockIdx.x - call.block_start[m]) * (kBlock / kWave) + threadIdx.x / kWave) * take;
-  const int64_t a = call.row_start[m];
-  pooled_sum_body<VEC>(descs[m].tv, rows + a, call.ids[m], call.row_start[m + 1] - a, call.offsets[m], first,
-                       call.bag_start[m + 1] - call.bag_start[m], take, call.weights[m],
-                       (int)((call.mean_bits >> m) & 1u), call.patch[m], call.rows[m], dim, elems, group);
 }
 
 template <int OPT, int VEC>
@@ -2331,11 +2424,20 @@ static bool pooled_few(bool filling, int64_t n, int* left) {
 
 // Bags that a wavefront of a pooled sum takes: as many as it has lane groups while that leaves the chip (8192
 // wavefronts at a time) room, and up to 64 of a larger request, so that the groups' bags even out (see
-// pooled_sum_wave; 852k bags of 32 floats with 8 / 16 / 32 / 64 a wavefront 142 / 123 / 113 / 109 us).
+// pooled_sum_wave, and share_bags for bags that do not; 852k bags of 32 floats with 8 / 16 / 32 / 64 a wavefront
+// 142 / 123 / 113 / 109 us).
 static int pooled_take(int64_t bags, int group) {
   int take = kWave / group;
   while (take < kWave && bags >= (int64_t)8192 * 2 * take) take *= 2;
   return take;
+}
+
+// How the bags of a pooled sum, n positions in `blocks` blocks of `take`, are shared out: see share_bags. A block is
+// shared where it holds more than twice the mean, and not for a record or two of each of its bags.
+static BagShares bag_shares(int64_t n, int64_t blocks, int take) {
+  int64_t limit = 2 * n / blocks;
+  if (limit < kPoolAhead * take) limit = kPoolAhead * take;
+  return BagShares{take, (int32_t)std::min<int64_t>(limit, INT32_MAX)};
 }
 
 // The launches of one pull of n > 0 ids into d_out [n, dim]; the caller holds the table's lock
@@ -2498,8 +2600,11 @@ int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, co
   uint32_t* rows = notes ? notes : t->scratch[5].as<uint32_t>();
   uint32_t* todo = t->scratch[5].as<uint32_t>() + rows_words;
   const int take = pooled_take(bags, t->group);
+  const bool more = take > kWave / t->group;
+  const BagShares by = bag_shares(n, grid_for(bags, take), take);
   // a lane looks up an id of its own, or four lanes one where many are to be inserted
-  const dim3 probe_grid(grid_for(n, few || queued ? kBlock / kBucket : kBlock)), grid(grid_for(bags, take * (kBlock / kWave))), block(kBlock);
+  const dim3 probe_grid(grid_for(n, few || queued ? kBlock / kBucket : kBlock)), block(kBlock);
+  const dim3 grid(grid_for(bags, take * (kBlock / kWave)) + (more ? kSpareBlocks : 0));
   const auto probe = [&](auto vec, auto few) {
     hipLaunchKernelGGL((pooled_probe_kernel<vec.value, few.value>), probe_grid, block, 0, t->stream, t->view(), t->initk,
                        d_ids, n, rows, t->elems);
@@ -2508,6 +2613,12 @@ int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, co
   const int mean = mode == KRK_POOL_MEAN;
   unsigned long long* publish = (flags & KRK_ASYNC) && sparse_wants_publish(t) ? t->host_pub : nullptr;
   if (publish) t->pub_epoch = t->epoch;
+  const auto sum = [&](auto vec) {
+    with_bool(more, [&](auto more) {
+      hipLaunchKernelGGL((pooled_sum_kernel<vec.value, more.value>), grid, block, 0, t->stream, t->view(), rows, d_ids, n,
+                         d_off, bags, d_w, mean, patch_value, d_out, (int)t->dim, t->elems, t->group, by, publish);
+    });
+  };
   int parity = 0;
   if (queued) {
     parity = t->pull_parity;
@@ -2520,16 +2631,14 @@ int32_t krk_sparse_pull_pooled(krk_sparse* t, const uint64_t* ids, int64_t n, co
                          d_ids, nullptr, todo, parity, list_capacity, (int)t->dim, t->elems, t->group, rows);
     else if (n > 0)
       with_bool(few, [&](auto few16) { probe(std::integral_constant<int, 4>(), few16); });
-    hipLaunchKernelGGL((pooled_sum_kernel<4>), grid, block, 0, t->stream, t->view(), rows, d_ids, n, d_off, bags, d_w,
-                       mean, patch_value, d_out, (int)t->dim, t->elems, t->group, take, publish);
+    sum(std::integral_constant<int, 4>());
   } else {
     if (queued)
       hipLaunchKernelGGL((pull_missing_kernel<1, true>), small, missing_block, 0, t->stream, t->view(), t->initk,
                          d_ids, nullptr, todo, parity, list_capacity, (int)t->dim, t->elems, t->group, rows);
     else if (n > 0)
       with_bool(few, [&](auto few16) { probe(std::integral_constant<int, 1>(), few16); });
-    hipLaunchKernelGGL((pooled_sum_kernel<1>), grid, block, 0, t->stream, t->view(), rows, d_ids, n, d_off, bags, d_w,
-                       mean, patch_value, d_out, (int)t->dim, t->elems, t->group, take, publish);
+    sum(std::integral_constant<int, 1>());
   }
   KRK_HIP(hipGetLastError());
   if (notes) {
@@ -3590,6 +3699,10 @@ int32_t krk_group_pull_pooled_parts(krk_group* g, const krk_pooled_part* in, uin
   const int64_t total = pool.row_start[n_tables];
   const int take = pooled_take(pool.bag_start[n_tables], g->group);
   const int64_t sum_blocks = pooled_layout(&pool, take * (kBlock / kWave));
+  int64_t bag_blocks = 0;
+  for (int m = 0; m < n_tables; ++m) bag_blocks += (pool.bag_start[m + 1] - pool.bag_start[m] + take - 1) / take;
+  const BagShares by = bag_shares(total, bag_blocks, take);
+  const bool more = take > kWave / g->group;
   if (sum_blocks < 0) {
     set_error("combined request too large for one launch; split it");
     return KRK_E_CAPACITY;
@@ -3661,17 +3774,21 @@ int32_t krk_group_pull_pooled_parts(krk_group* g, const krk_pooled_part* in, uin
       }
     });
   }
-  const dim3 sum_grid((unsigned)sum_blocks);
+  const dim3 sum_grid((unsigned)(sum_blocks + (more ? kSpareBlocks : 0)));
   GroupPublish publish{};
   if (flags & KRK_ASYNC)
     for (krk_sparse* t : g->tables) publish.on |= sparse_wants_publish(t) ? 1u : 0u;
   for (int m = 0; publish.on && m < n_tables; ++m) publish.epoch[m] = g->tables[m]->pub_epoch = g->tables[m]->epoch;
+  const auto sum = [&](auto vec) {
+    with_bool(more, [&](auto more) {
+      hipLaunchKernelGGL((group_pooled_sum_kernel<vec.value, more.value>), sum_grid, block, 0, g->stream, g->d_descs,
+                         pool, rows, (int)g->dim, g->elems, g->group, by, publish);
+    });
+  };
   if (g->vec == 4) {
-    hipLaunchKernelGGL((group_pooled_sum_kernel<4>), sum_grid, block, 0, g->stream, g->d_descs, pool, rows,
-                       (int)g->dim, g->elems, g->group, take, publish);
+    sum(std::integral_constant<int, 4>());
   } else {
-    hipLaunchKernelGGL((group_pooled_sum_kernel<1>), sum_grid, block, 0, g->stream, g->d_descs, pool, rows,
-                       (int)g->dim, g->elems, g->group, take, publish);
+    sum(std::integral_constant<int, 1>());
   }
   KRK_HIP(hipGetLastError());
   if (notes) {
