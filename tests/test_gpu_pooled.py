@@ -424,6 +424,76 @@ def test_pooled_pulls_of_many_bags(api, dim, groups, per_wavefront):
     assert rc == 0 and np.array_equal(got.to_host(), weighted)
 
 
+def _in_order(rows, off, w, mean, patch):
+    """The bags' sums in position order, in fp32: rows are the positions' (jagged_ops.cc:205-224)."""
+    lengths = np.diff(off)
+    want = np.full((lengths.size, rows.shape[1]), patch, np.float32)
+    for u in range(int(lengths.max(initial=0))):
+        on = np.flatnonzero(lengths > u)
+        row = rows[off[:-1][on] + u]
+        if w is not None:
+            row = row * w[off[:-1][on] + u][:, None]
+        want[on] = row if u == 0 else want[on] + row
+    if mean:
+        some = lengths > 0
+        want[some] *= (1.0 / lengths[some]).astype(np.float32)[:, None]
+    return want
+
+
+# Rows of 128 floats: a wavefront has two lane groups, and takes 4 bags from 32,768 on, 64 from 524,288 on. Of 32 floats
+# eight groups and 16 bags from 131,072 on, of 8 floats 32 and 64 from 524,288 on, of 10 floats four and 8 from 65,536 on.
+@pytest.mark.parametrize("dim,bags", [(128, (32_768,)), (128, (40_000, 0, 7)), (128, (12_000, 11_500, 12_001)),
+                                      (128, (32_766, 1, 1)), (128, (6, 524_300)), (32, (140_000, 3)), (32, (524_289,)),
+                                      (8, (524_290,)), (8, (300_000, 299_000)), (10, (70_000, 9))])
+def test_combined_pooled_pulls_of_many_bags(api, dim, bags):
+    """Members of which a wavefront takes more bags than it has lane groups: one, unequal ones (of no bag, of fewer than
+    a wavefront takes), equal ones, with two stretches of long bags that are shared out among wavefronts; ids that
+    the request itself makes, each at many positions, so that positions read an id's row while another one is
+    making it; then the same request over rows that are there, and the first member's part by itself."""
+    C = api.C
+
+    class Part(C.Structure):
+        _fields_ = [("ids", C.c_void_p), ("n", C.c_int64), ("offsets", C.c_void_p), ("bags", C.c_int64),
+                    ("weights", C.c_void_p), ("rows", C.c_void_p), ("stride", C.c_int64), ("mode", C.c_int32),
+                    ("patch", C.c_float)]
+
+    rng = np.random.default_rng(sum(bags))
+    gi = api.Initializer.create(api.InitializerType.kNormal, {"stddev": "0.01", "seed": "4"})
+    tables = [api.SparseTable(dim, gi, capacity_hint=64) for _ in bags]
+    group = api.TableGroup(tables)
+    made, held = [], []
+    for m, count in enumerate(bags):
+        lengths = rng.choice([0, 1, 2, 4, 5], size=count, p=[.3, .4, .2, .05, .05])
+        lengths[1001:1300] = 40
+        lengths[-101:] = rng.integers(20, 40, lengths[-101:].size)
+        off = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int64)
+        ids = splitmix64(rng.integers(0, 60, size=int(off[-1])).astype(np.uint64))
+        ids[::97] = np.uint64(2**64 - 1)
+        w = rng.standard_normal(ids.size).astype(np.float32) if m % 2 == 0 else None
+        out = api.DeviceArray((max(count, 1), dim), np.float32)
+        d_ids, d_off = api.DeviceArray.from_host(ids), api.DeviceArray.from_host(off)
+        d_w = api.DeviceArray.from_host(w) if w is not None else None
+        held.append((d_ids, d_off, d_w))
+        made.append((ids, off, w, m % 3 == 1, -0.75 - m, out))
+    parts = (Part * len(bags))(*[Part(h[0].ptr, i.size, h[1].ptr, off.size - 1, h[2].ptr if h[2] else None, out.ptr, dim,
+                                      1 if mean else 0, patch)
+                                 for h, (i, off, w, mean, patch, out) in zip(held, made)])
+    for step in range(2):
+        assert api.lib().krk_group_pull_pooled_parts(group.h, parts, api.DEVICE_PTRS) == 0
+        for t, (ids, off, w, mean, patch, out) in zip(tables, made):
+            if off.size == 1:
+                continue
+            u, inv = np.unique(ids, return_inverse=True)
+            rows = t.Pull(u)[1][inv] if u.size else np.zeros((0, dim), np.float32)
+            assert len(t) == u.size
+            want = _in_order(rows, off, w, mean, patch)
+            assert np.array_equal(out.to_host(), want), step
+            if t is tables[0]:
+                rc, got = t.PullPooled(held[0][0], held[0][1], "mean" if mean else "sum", patch_value=patch, weights=held[0][2])
+                assert rc == 0 and np.array_equal(got.to_host(), want), step
+    group.close()
+
+
 def test_pooled_pulls_of_uneven_bags_take_no_longer_in_order(api):
     """Long bags that stand together (bags in order of their length, one field's histories behind the other fields'
     single ids) are shared out among wavefronts. As 64 neighbours of one wavefront this request took seven
