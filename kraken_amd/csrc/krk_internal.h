@@ -119,8 +119,9 @@ struct StreamWait {
   bool open();    // takes a free word; false where there is none: the call then synchronises with the stream
   void close();   // gives it back
 };
-// Waits until the word of an open wait holds its number, and closes it. A stream that takes longer than a millisecond,
-// has failed or is being captured is left to hipStreamSynchronize.
+// Waits until the word of an open wait holds its number, and closes it. A stream that takes longer than five
+// milliseconds, has failed or is being captured is left to hipStreamSynchronize. The core is busy meanwhile, as it is in
+// hipStreamSynchronize; after 50 us other threads may have it between two looks.
 int32_t wait_for(StreamWait* w, hipStream_t stream);
 // The same for a stream whose last launch writes no word: puts a launch behind it that does.
 int32_t wait_stream(hipStream_t stream);

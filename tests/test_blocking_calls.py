@@ -16,7 +16,7 @@ def program(tmp_path_factory):
         from kraken_amd import build
         build.build(verbose=False)
     exe = str(tmp_path_factory.mktemp("host") / "blocking_calls_test")
-    subprocess.check_call(["g++", "-std=c++17", "-O1", "-Wall", "-I" + os.path.join(ROOT, "include"),
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-Wall", "-pthread", "-I" + os.path.join(ROOT, "include"),
                            "-isystem", os.path.join(ROCM, "include"),
                            os.path.join(ROOT, "tests", "host", "blocking_calls_test.cc"), "-o", exe, "-L" + lib_dir,
                            "-lkraken_hip", "-Wl,-rpath," + lib_dir, "-Wl,-rpath," + os.path.join(ROCM, "lib")])
@@ -25,7 +25,8 @@ def program(tmp_path_factory):
 
 # dense, sparse: a blocking call on pageable arrays synchronises after the copies that staged them
 # words: no two calls wait on one word, and the calls that find none synchronise
-@pytest.mark.parametrize("which", ["dense", "sparse", "words"])
+# core: a waiting thread lets the other threads of its core run
+@pytest.mark.parametrize("which", ["dense", "sparse", "words", "core"])
 def test_blocking_calls(program, which):
     r = subprocess.run([program, which], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr

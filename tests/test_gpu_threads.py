@@ -201,8 +201,8 @@ def test_more_blocking_calls_at_once_than_there_are_words_to_wait_on(api):
 
 
 def test_a_blocking_call_behind_work_that_takes_longer_than_its_wait_looks(api):
-    """The host looks at its word for a millisecond and then synchronises: the call returns only once what it
-    enqueued behind some 20 ms of other work has run."""
+    """The host looks at its word for five milliseconds and then synchronises: the call returns only once what it
+    enqueued behind some 13 ms of other work has run."""
     n = 1 << 26
     t = api.DenseTable(np.zeros(n, np.float32))
     g, out = api.DeviceArray.from_host(np.ones(n, np.float32)), api.DeviceArray(n, np.float32)
