@@ -13,7 +13,11 @@
  * gradients, outputs) is a device pointer on the table's GPU. Calls are
  * blocking unless KRK_ASYNC is also set (device pointers only): the work is
  * then only enqueued on the table's stream and a failure is reported by the
- * next blocking call or by the object's *_sync() function.
+ * next blocking call or by the object's *_sync() function. A blocking call returns when its
+ * results are there and its inputs may be changed or freed. The calling thread uses its core while it
+ * waits, and lets other threads have it from 50 us on. The runtime has not been asked to synchronise the
+ * stream by then unless an array was staged from or to pageable memory: programs need not call
+ * hipDeviceSynchronize after it, and it takes some 10 to 30 us if they do.
  *
  * Stream capture: do not record these calls into a HIP graph. Every launch that may insert
  * rows carries a launch number chosen on the host, and a replayed launch would present an old

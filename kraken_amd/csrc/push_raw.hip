@@ -117,7 +117,7 @@ __global__ __launch_bounds__(BLOCK) void dedup_claim_kernel(DSlot* slots, uint64
 
 // The ranks of the first occurrences, in two launches and one random read per position. The first
 // one reads the smallest position of every position's id out of the index, leaves it in place of the
-// slot number, and ranks the first occurrences of its 1024 positions among themselves; their
+// slot number, and ranks the first occurrences of its tile's positions among themselves; their
 // counts go to sums[]. The second one (dedup_emit_kernel) adds what earlier tiles hold.
 // Flags, a scan of them in three launches and an emit that read the index again took six launches
 // where this takes two: they are bound by the launches up to a few hundred thousand ids (a blocking
@@ -125,7 +125,10 @@ __global__ __launch_bounds__(BLOCK) void dedup_claim_kernel(DSlot* slots, uint64
 //
 // CLEAN: the index belongs to the calls of up to 2^16 ids, each of which leaves it as empty as it found it: the
 // first position of an id keeps the slot (kSlotOf), and the emit clears it. A memset ahead of the claims, which
-// is what longer requests take, costs a launch and some 4 us.
+// is what longer requests take, costs a launch and some 4 us; it also leaves the slots in the L2, which an index that
+// was left empty some time ago is not. That costs less: 26,624 ids right behind 512 MB of other writes, dedup 28.8 us
+// with the memset and workgroups of 1024, 22.4 this way (28.1 and 21.5 call after call), dedup + sum 57.5 and 50 to 55
+// (54.6 and 47), 60,000 ids 33.3 and 24.0, 66 and 57 to 62.
 constexpr uint32_t kSlotOf = 0x80000000u;
 
 // Exclusive scan over the lanes of a workgroup; *all = the sum. Ends behind a barrier.

@@ -165,7 +165,7 @@ __global__ __launch_bounds__(kRsBlock, BITS == 9 ? 6 : 8) void radix_scatter_ker
   const int lane = t & (kWave - 1);
   const int wave = t / kWave;
   const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
-  // element i of lane l in wavefront w is key w * 256 + i * 64 + l of the tile: a wavefront's
+  // element i of lane l in wavefront w is key w * (64 * kRsItems) + i * 64 + l of the tile: a wavefront's
   // keys are consecutive, and taking i in ascending order visits them in tile order
   const int64_t tile_base = (int64_t)tile * kRsTile;
   const int64_t base = tile_base + wave * (kWave * kRsItems) + lane;

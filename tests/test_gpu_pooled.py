@@ -391,7 +391,7 @@ def test_pooled_pulls_make_rows(api, n, dim, combined):
         group.close()
 
 
-@pytest.mark.parametrize("dim,groups", [(8, 16), (32, 8), (128, 2), (10, 4)])
+@pytest.mark.parametrize("dim,groups", [(8, 32), (32, 8), (128, 2), (10, 4)])
 @pytest.mark.parametrize("per_wavefront", [1, 2, 32])
 def test_pooled_pulls_of_many_bags(api, dim, groups, per_wavefront):
     """Requests from whose number of bags on a wavefront takes more of them than it has lane groups (twice and up

@@ -172,8 +172,9 @@ def test_group_calls_and_member_calls_from_several_threads(api, oracle):
 
 
 def test_more_blocking_calls_at_once_than_there_are_words_to_wait_on(api):
-    """72 threads, a table each: every call returns after its own work, with its own rows, whichever of
-    the 64 words its wait got, or none."""
+    """72 threads, a table each, more than there are words (64): every call returns after its own work, with its own
+    rows. A word is held for microseconds, so that threads seldom find none here; tests/test_blocking_calls.py takes
+    all of them."""
     n_threads, dim = 72, 8
     tables = [api.SparseTable(dim, api.Initializer.create(api.InitializerType.kConstant, {"value": str(k)}))
               for k in range(n_threads)]
