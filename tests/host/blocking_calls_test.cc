@@ -11,10 +11,6 @@
 #endif
 #include <hip/hip_runtime_api.h>
 
-#include <sched.h>
-#include <time.h>
-
-#include <atomic>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -23,7 +19,6 @@
 #include <map>
 #include <set>
 #include <string>
-#include <thread>
 #include <vector>
 
 #include "kraken_hip.h"
@@ -46,9 +41,7 @@ struct Runtime {
   std::map<hipStream_t, std::vector<Late>> late;    // words that a stream's launches will write
   std::vector<uint32_t*> words;                     // of every launch that tells the host, null where it has none
   bool signals_late = false;
-  bool signals_by_thread = false;
-  std::atomic<uint32_t*> by_thread{nullptr};        // the word that another thread is to write, and its number
-  uint32_t by_thread_ticket = 0;
+  int yields_until_told = 0;                        // > 0: late words are written at the last of so many sched_yields
   int synchronised = 0;
   uint32_t rows = 0;                                // what the tables' counters say
   std::function<void()> on_synchronise;
@@ -80,14 +73,22 @@ static hipError_t give(void* p) {
 static void tell(hipStream_t stream, uint32_t* word, uint32_t ticket) {
   rt().words.push_back(word);
   if (!word) return;
-  if (rt().signals_by_thread) {
-    rt().by_thread_ticket = ticket;
-    rt().by_thread.store(word);
-  } else if (rt().signals_late) rt().late[stream].push_back(Late{word, ticket});
+  if (rt().signals_late) rt().late[stream].push_back(Late{word, ticket});
   else __atomic_store_n(word, ticket, __ATOMIC_RELEASE);
 }
 
+static void write_late() {
+  for (auto& s : rt().late) {
+    for (const Late& l : s.second) __atomic_store_n(l.word, l.ticket, __ATOMIC_RELEASE);
+    s.second.clear();
+  }
+}
+
 extern "C" {
+int sched_yield() {
+  if (rt().yields_until_told > 0 && --rt().yields_until_told == 0) write_late();
+  return 0;
+}
 hipError_t hipMalloc(void** p, size_t bytes) { return take(p, bytes, false, 0); }
 hipError_t hipFree(void* p) { return give(p); }
 hipError_t hipHostMalloc(void** p, size_t bytes, unsigned flags) { return take(p, bytes, true, flags); }
@@ -113,7 +114,6 @@ hipError_t hipMemsetAsync(void* d, int v, size_t bytes, hipStream_t) { std::mems
 hipError_t hipStreamSynchronize(hipStream_t stream) {
   rt().synchronised++;
   if (rt().on_synchronise) rt().on_synchronise();
-  while (rt().by_thread.load()) sched_yield();
   for (const Late& l : rt().late[stream]) __atomic_store_n(l.word, l.ticket, __ATOMIC_RELEASE);
   rt().late[stream].clear();
   rt().pageable[stream] = false;
@@ -346,47 +346,20 @@ static void late_words() {
   for (krk_sparse* t : tables) CHECK(krk_sparse_destroy(t) == 0);
 }
 
-// The word is written by a thread of the same core, after 150 us of its own. It does not sleep in between, so
-// that it runs when the waiting thread lets it, or has used its time slice of some milliseconds up.
+// The word is written once the waiting thread has let others of its core run a few times.
 static void one_core() {
-  cpu_set_t all, one;
-  CHECK(sched_getaffinity(0, sizeof(all), &all) == 0);
-  CPU_ZERO(&one);
-  for (int c = 0; c < CPU_SETSIZE && CPU_COUNT(&one) == 0; ++c)
-    if (CPU_ISSET(c, &all)) CPU_SET(c, &one);
   krk_sparse* t = make_table(8);
   uint64_t id = 7;
   std::vector<float> row(8);
-  CHECK(sched_setaffinity(0, sizeof(one), &one) == 0);   // the thread below inherits it
-  std::atomic<bool> done{false};
-  std::thread device([&]() {
-    const auto cpu_us = []() {
-      timespec now;
-      clock_gettime(CLOCK_THREAD_CPUTIME_ID, &now);
-      return (int64_t)now.tv_sec * 1000000 + now.tv_nsec / 1000;
-    };
-    while (!done) {
-      uint32_t* word = rt().by_thread.load();
-      if (!word) {
-        sched_yield();
-        continue;
-      }
-      const int64_t begun = cpu_us();
-      while (cpu_us() - begun < 150) {}
-      __atomic_store_n(word, rt().by_thread_ticket, __ATOMIC_RELEASE);
-      rt().by_thread.store(nullptr);
-    }
-  });
-  rt().signals_by_thread = true;
+  rt().signals_late = true;
   rt().synchronised = 0;
   constexpr int kCalls = 40;
   for (int i = 0; i < kCalls; ++i) {
+    rt().yields_until_told = 5;
     CHECK(krk_sparse_pull(t, &id, 1, row.data(), 0) == KRK_SUCCESS);
-    while (rt().by_thread.load()) sched_yield();
   }
-  rt().signals_by_thread = false;
-  done = true;
-  device.join();
+  rt().signals_late = false;
+  rt().yields_until_told = 0;
   if (rt().synchronised > kCalls / 4) {
     std::printf("FAILED: %d of %d calls looked for as long as they may\n", rt().synchronised, kCalls);
     ++failures;

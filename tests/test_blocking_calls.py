@@ -16,7 +16,7 @@ def program(tmp_path_factory):
         from kraken_amd import build
         build.build(verbose=False)
     exe = str(tmp_path_factory.mktemp("host") / "blocking_calls_test")
-    subprocess.check_call(["g++", "-std=c++17", "-O1", "-Wall", "-pthread", "-I" + os.path.join(ROOT, "include"),
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-Wall", "-I" + os.path.join(ROOT, "include"),
                            "-isystem", os.path.join(ROCM, "include"),
                            os.path.join(ROOT, "tests", "host", "blocking_calls_test.cc"), "-o", exe, "-L" + lib_dir,
                            "-lkraken_hip", "-Wl,-rpath," + lib_dir, "-Wl,-rpath," + os.path.join(ROCM, "lib")])
