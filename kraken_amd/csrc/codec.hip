@@ -422,61 +422,215 @@ __device__ __forceinline__ void coo_start_tiles(uint32_t* __restrict__ starts, i
 }
 
 // Where each tile's entries begin: the first entry of a tile, and the first one behind the empty
-// tiles before it, name themselves. A wavefront takes 256 entries in two rows of 128, a lane two
+// tiles before it, name themselves. A wavefront takes chunks of 256 entries in two rows of 128, a lane two
 // neighbours of each in one 16-byte load (whole lines an access); the entry before a lane's two is
 // its neighbour's second.
+constexpr int kCooRows = 2;
+constexpr int kCooChunk = kCooRows * 128;
+typedef long long coo_pair __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ void coo_load_chunk(const long long* __restrict__ idx, int64_t base, int64_t nnz, bool vec,
+                                               coo_pair (&cur)[kCooRows]) {
+  const int lane = threadIdx.x & 63;
+  const bool whole = vec && base + kCooChunk <= nnz;   // uniform
+#pragma unroll
+  for (int r = 0; r < kCooRows; ++r) {
+    const int64_t j = base + r * 128 + lane * 2;
+    if (whole) {
+      cur[r] = __builtin_nontemporal_load(reinterpret_cast<const coo_pair*>(idx + j));
+    } else {
+      cur[r][0] = idx[j < nnz ? j : nnz - 1];
+      cur[r][1] = idx[j + 1 < nnz ? j + 1 : nnz - 1];
+    }
+  }
+}
+
+// The starts that a row of 128 entries from entry j of a lane on names; `last`: the entry before the row, then its
+// last one. False where an entry does not ascend or lies outside [0, n).
+__device__ __forceinline__ bool coo_row_starts(const coo_pair& cur, int64_t j, int64_t nnz, int64_t n, long long& last,
+                                               const CooTiles& out) {
+  const int lane = threadIdx.x & 63;
+  long long prev = __shfl_up(cur[1], 1);
+  if (lane == 0) prev = last;
+  last = __shfl(cur[1], 63);
+  // nearly every lane: two more entries of the tile the one before is in
+  const bool quick = j + 2 < nnz && prev >= 0 && prev < cur[0] && cur[0] < cur[1] && cur[1] < n &&
+                     (prev ^ cur[1]) < kCooTile;
+  if (__ballot(!quick) == 0ull) return true;
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const bool mine = !quick && j + i < nnz;
+    const long long c = cur[i];
+    const bool wrong = mine && (c < 0 || c <= prev || c >= n);   // prev may be negative, and wrong, itself
+    bad = bad || wrong;
+    int from = 1, to = 0, tile = 0;
+    if (mine && !wrong) {
+      tile = (int)(c / kCooTile);
+      from = prev < 0 ? 0 : (int)(prev / kCooTile) + 1;
+      to = tile;
+    }
+    coo_start_tiles(out.starts, from, to, (uint32_t)(j + i));
+    const bool end = mine && !wrong && j + i == nnz - 1;
+    if (__ballot(end) != 0ull)
+      coo_start_tiles(out.starts, end ? tile + 1 : 1, end ? (int)out.tiles : 0, (uint32_t)nnz);
+    prev = c;
+  }
+  return __ballot(bad) == 0ull;
+}
+
 __global__ __launch_bounds__(kCodecBlock) void coo_tiles_bounds_kernel(const long long* __restrict__ idx,
                                                                        int64_t nnz, int64_t n, bool vec, CooTiles out) {
-  typedef long long pair __attribute__((ext_vector_type(2)));
-  constexpr int kRows = 2;
-  const int lane = threadIdx.x & 63;
-  const int64_t step = (int64_t)gridDim.x * (kCodecBlock / 64) * (kRows * 128);
-  for (int64_t base = ((int64_t)blockIdx.x * (kCodecBlock / 64) + threadIdx.x / 64) * (kRows * 128); base < nnz;
+  const int64_t step = (int64_t)gridDim.x * (kCodecBlock / 64) * kCooChunk;
+  for (int64_t base = ((int64_t)blockIdx.x * (kCodecBlock / 64) + threadIdx.x / 64) * kCooChunk; base < nnz;
        base += step) {                               // a wavefront's lanes stay together
-    pair cur[kRows];
+    coo_pair cur[kCooRows];
+    coo_load_chunk(idx, base, nnz, vec, cur);
+    long long last = base ? idx[base - 1] : -1;      // the entry before the row
+    bool fine = true;
 #pragma unroll
-    for (int r = 0; r < kRows; ++r) {
-      const int64_t j = base + r * 128 + lane * 2;
-      if (vec && j + 1 < nnz) {
-        cur[r] = __builtin_nontemporal_load(reinterpret_cast<const pair*>(idx + j));
-      } else {
-        cur[r][0] = idx[j < nnz ? j : nnz - 1];
-        cur[r][1] = idx[j + 1 < nnz ? j + 1 : nnz - 1];
+    for (int r = 0; r < kCooRows; ++r)
+      fine &= coo_row_starts(cur[r], base + r * 128 + (threadIdx.x & 63) * 2, nnz, n, last, out);
+    if (!fine) __hip_atomic_store(out.unordered, out.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// The same, and a bit for every element that an entry names, so that who walks the tiles need not read the indices
+// again. A wavefront takes a run of consecutive chunks and carries the words that later entries may share along: every
+// word is written once, by the wavefront that holds the first of the entries behind the word before it, and nothing
+// has to be cleared ahead. Words of tiles without entries are not written. The bits meet in LDS, in a window of up
+// to two tiles' words that moves on by 64 of them, a line of memory; chunks wider than that take several windows.
+// What bounds it is the read of the indices, and next to it instruction issue: nearly every chunk of a gradient that keeps
+// a quarter of its elements is an easy one (no gap of a tile or more, all of it in the window, not the run's last),
+// and those take a third of the general path's 200 vector instructions. 33 million entries among 67 million elements: the general path
+// alone 58 us, with the easy one 55, with lines instead of each chunk's words 52 in runs of 4 (2, 8, 16: 55, 53, 55);
+// without bits 44.6. The update that follows takes 317 us for 365.
+constexpr int kCooRun = 4;                           // chunks of a wavefront
+constexpr int kCooWindow = 128;
+
+__global__ __launch_bounds__(kCodecBlock) void coo_bits_kernel(const long long* __restrict__ idx, int64_t nnz, int64_t n,
+                                                               bool vec, CooTiles out) {
+  static_assert(kCooTile == 64 * 32, "a tile's bits are a word a lane");
+  __shared__ uint32_t wave_words[(kCodecBlock / 64) * kCooWindow];
+  const int lane = threadIdx.x & 63;
+  uint32_t* words = &wave_words[(threadIdx.x >> 6) * kCooWindow];
+  words[lane] = 0u;
+  words[lane + 64] = 0u;
+  const int64_t run = ((int64_t)blockIdx.x * (kCodecBlock / 64) + threadIdx.x / 64) * (kCooRun * kCooChunk);
+  if (run >= nnz) return;
+  const int64_t stop = run + kCooRun * kCooChunk < nnz ? run + kCooRun * kCooChunk : nnz;
+  coo_pair cur[kCooRows], ahead[kCooRows];
+  coo_load_chunk(idx, run, nnz, vec, cur);
+  long long last = run ? idx[run - 1] : -1;          // the entry before the chunk
+  // entries of the run behind this one may lie in this one's last word
+  const long long after = lane < 32 && stop + lane < nnz ? idx[stop + lane] : -1;
+  bool fine = true;
+  const bool small = n <= (int64_t)0xFFFFFFFF;
+  // the first word that is not written yet; words[i]: what is known of word from + i, of at most 64 between two chunks
+  uint32_t from = last < 0 ? 0u : (uint32_t)(last >> 5) + 1u;
+  for (int64_t base = run; base < stop; base += kCooChunk) {
+    if (base + kCooChunk < stop) coo_load_chunk(idx, base + kCooChunk, nnz, vec, ahead);
+    const int64_t j = base + lane * 2;
+    const bool ends = base + kCooChunk >= stop;
+    if (small && !ends && last >= 0) {               // uniform: indices are their low halves, if in range
+      uint32_t prev[kCooRows], most = 0u, high = 0u, before = (uint32_t)last;
+#pragma unroll
+      for (int r = 0; r < kCooRows; ++r) {
+        const uint32_t c0 = (uint32_t)cur[r][0], c1 = (uint32_t)cur[r][1];
+        // the entry before a lane's two: its lower neighbour's second (wave_shr:1), the lowest lane's the row before's last
+        prev[r] = (uint32_t)__builtin_amdgcn_update_dpp((int)before, (int)c1, 0x138, 0xf, 0xf, false);
+        before = (uint32_t)__builtin_amdgcn_readlane((int)c1, 63);
+        high |= (uint32_t)(cur[r][0] >> 32) | (uint32_t)(cur[r][1] >> 32);
+        most = max(most, max(c0 - prev[r] - 1u, c1 - c0 - 1u));
+      }
+      const uint32_t top = before >> 5;
+      const bool easy = __ballot(high != 0u || most >= (uint32_t)kCooTile - 1u) == 0ull && before < (uint32_t)n &&
+                        top - from < (uint32_t)kCooWindow;
+      if (easy) {
+#pragma unroll
+        for (int r = 0; r < kCooRows; ++r) {
+          const uint32_t c0 = (uint32_t)cur[r][0], c1 = (uint32_t)cur[r][1];
+          const uint32_t t = prev[r] >> 11, t0 = c0 >> 11, t1 = c1 >> 11;
+          if (t != t1) {                             // a lane in a tile's length: no gap passes over a whole tile
+            if (t != t0) out.starts[t0] = (uint32_t)(j + r * 128);
+            if (t0 != t1) out.starts[t1] = (uint32_t)(j + r * 128 + 1);
+          }
+          const uint32_t w0 = c0 >> 5, w1 = c1 >> 5, b0 = 1u << (c0 & 31u), b1 = 1u << (c1 & 31u);
+          // (the first chunk's first entries may lie in the word before, which another wavefront writes)
+          if (w0 != w1 && w0 - from < (uint32_t)kCooWindow) atomicOr(&words[w0 - from], b0);
+          if (w1 - from < (uint32_t)kCooWindow) atomicOr(&words[w1 - from], w0 == w1 ? b0 | b1 : b1);
+        }
+        __builtin_amdgcn_wave_barrier();             // one wavefront: its LDS accesses stay in order
+        if (top - from >= 64u) {                     // a line of complete words, and the window moves on by it
+          out.bits[from + lane] = words[lane];
+          words[lane] = words[lane + 64];
+          words[lane + 64] = 0u;
+          from += 64u;
+          __builtin_amdgcn_wave_barrier();
+        }
+        last = (long long)before;
+#pragma unroll
+        for (int r = 0; r < kCooRows; ++r) cur[r] = ahead[r];
+        continue;
       }
     }
-    long long last = base ? idx[base - 1] : -1;      // the entry before the row
-    bool bad = false;
 #pragma unroll
-    for (int r = 0; r < kRows; ++r) {
-      const int64_t j = base + r * 128 + lane * 2;
-      long long prev = __shfl_up(cur[r][1], 1);
-      if (lane == 0) prev = last;
-      last = __shfl(cur[r][1], 63);
-      // nearly every lane: two more entries of the tile the one before is in
-      const bool quick = j + 2 < nnz && prev >= 0 && prev < cur[r][0] && cur[r][0] < cur[r][1] && cur[r][1] < n &&
-                         (prev ^ cur[r][1]) < kCooTile;
-      if (__ballot(!quick) == 0ull) continue;
+    for (int r = 0; r < kCooRows; ++r) fine &= coo_row_starts(cur[r], j + r * 128, nnz, n, last, out);
+    if (!fine) break;                                // the bits will not be looked at
+    const uint32_t top = (uint32_t)(last >> 5);
+    const bool closes = base + kCooChunk >= nnz;     // behind the very last entry: the rest of its tile
+    const uint32_t to = closes ? (top | 63u) + 1u : ends ? top + 1u : top;   // words [from, to) are complete
+    uint32_t w[2 * kCooRows], bit[2 * kCooRows];
+    bool on[2 * kCooRows];
+#pragma unroll
+    for (int r = 0; r < kCooRows; ++r) {
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        const bool mine = !quick && j + i < nnz;
-        const long long c = cur[r][i];
-        const bool wrong = mine && (c < 0 || c <= prev || c >= n);   // prev may be negative, and wrong, itself
-        bad = bad || wrong;
-        int from = 1, to = 0, tile = 0;
-        if (mine && !wrong) {
-          tile = (int)(c / kCooTile);
-          from = prev < 0 ? 0 : (int)(prev / kCooTile) + 1;
-          to = tile;
-        }
-        coo_start_tiles(out.starts, from, to, (uint32_t)(j + i));
-        const bool end = mine && !wrong && j + i == nnz - 1;
-        if (__ballot(end) != 0ull)
-          coo_start_tiles(out.starts, end ? tile + 1 : 1, end ? (int)out.tiles : 0, (uint32_t)nnz);
-        prev = c;
+        const uint32_t c = (uint32_t)cur[r][i];      // (n / 32 words: the low half says which bit, both which word)
+        w[2 * r + i] = (uint32_t)(cur[r][i] >> 5);
+        bit[2 * r + i] = 1u << (c & 31u);
+        on[2 * r + i] = j + r * 128 + i < nnz;
+      }
+      if (on[2 * r + 1] && w[2 * r] == w[2 * r + 1]) {
+        bit[2 * r + 1] |= bit[2 * r];
+        on[2 * r] = false;
       }
     }
-    if (bad) __hip_atomic_store(out.unordered, out.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const bool shares = ends && after > last && (after >> 5) == (long long)top;
+    for (uint32_t at = from;;) {                     // the window: words from `at` to the end of the next tile
+      const uint32_t behind = (at & ~63u) + kCooWindow, wide = behind - at;
+#pragma unroll
+      for (int i = 0; i < 2 * kCooRows; ++i)
+        if (on[i] && w[i] - at < wide) atomicOr(&words[w[i] - at], bit[i]);
+      if (shares && top - at < wide) atomicOr(&words[top - at], 1u << (after & 31));
+      __builtin_amdgcn_wave_barrier();               // one wavefront: its LDS accesses stay in order
+      const uint32_t v0 = words[lane], v1 = words[lane + 64];
+      if ((uint32_t)lane < wide && at + lane < to) out.bits[at + lane] = v0;
+      if ((uint32_t)lane + 64u < wide && at + lane + 64u < to) out.bits[at + lane + 64u] = v1;
+      words[lane] = 0u;
+      words[lane + 64] = 0u;
+      __builtin_amdgcn_wave_barrier();
+      if (to <= behind && top < behind) {
+        if (!ends) {                                 // the open word goes on as the next chunk's first
+          const uint32_t open = (uint32_t)__shfl((int)(top - at < 64u ? v0 : v1), (int)((top - at) & 63u));
+          if (lane == 0) words[0] = open;
+        }
+        break;
+      }
+      uint32_t next = top;                           // the nearest tile that has an entry (or is to be ended)
+#pragma unroll
+      for (int i = 0; i < 2 * kCooRows; ++i)
+        if (on[i] && w[i] >= behind && w[i] < next) next = w[i];
+#pragma unroll
+      for (int d = 32; d > 0; d >>= 1) next = min(next, (uint32_t)__shfl_xor((int)next, d));
+      next &= ~63u;
+      at = (uint32_t)__builtin_amdgcn_readfirstlane((int)(next < behind ? behind : next));
+    }
+    from = from > top ? from : top;
+#pragma unroll
+    for (int r = 0; r < kCooRows; ++r) cur[r] = ahead[r];
   }
+  if (!fine) __hip_atomic_store(out.unordered, out.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // One workgroup per output tile: the tile is put together in LDS (zeros, then the tile's entries,
@@ -521,6 +675,32 @@ __global__ __launch_bounds__(kCodecBlock) void coo_tiles_write_kernel(const long
   }
 }
 
+// The same from the bits: a wavefront's lanes see for themselves which entries are theirs, nothing passes through LDS.
+__global__ __launch_bounds__(kCodecBlock) void coo_bits_write_kernel(const float* __restrict__ val,
+                                                                     float* __restrict__ dense, int64_t n,
+                                                                     CooTiles tiles) {
+  if (coo_unordered(tiles)) return;
+  const int64_t base = (int64_t)blockIdx.x * kCooTile;
+  const uint32_t start = tiles.starts[blockIdx.x];
+  const uint32_t end = tiles.starts[blockIdx.x + 1];
+  const CooTileBits tile(tiles.bits[(size_t)blockIdx.x * (kCooTile / 32) + (threadIdx.x & 63)]);
+  const bool whole = base + kCooTile <= n && (((uintptr_t)dense) & 15) == 0;
+#pragma unroll
+  for (int i = 0; i < kCooTile / 4 / kCodecBlock; ++i) {
+    const int q = i * kCodecBlock + threadIdx.x;
+    float g[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (end > start) tile.quad(q, val, start, end, g);   // uniform
+    const int64_t at = base + 4 * q;
+    if (whole) {
+      __builtin_nontemporal_store((vfloat4){g[0], g[1], g[2], g[3]}, reinterpret_cast<vfloat4*>(dense + at));
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (at + c < n) dense[at + c] = g[c];
+    }
+  }
+}
+
 __global__ __launch_bounds__(kCodecBlock) void coo_zero_if_kernel(float* __restrict__ dense, int64_t n,
                                                                   CooTiles tiles) {
   if (!coo_unordered(tiles)) return;
@@ -543,6 +723,12 @@ __global__ __launch_bounds__(kCodecBlock) void coo_add_kernel(const long long* _
   }
 }
 
+// From an entry in this many elements on an entry's place is kept as a bit: 1/64 of the indices' bytes at an entry an
+// element, an eighth at one in eight, and who walks the tiles reads that. 67 million elements, an entry in 1 / 2 / 4 / 8 / 12 of them,
+// blocking, us, by the indices and by bits: Adam push 560 / 452 / 382 / 356 / 343 and 468 / 404 / 369 / 355 / 349,
+// decode 276 / 163 / 114 / 91 / 82 and 192 / 121 / 91 / 77 / 71.
+constexpr int64_t kCooBitsFrom = 8;
+
 static unsigned stream_grid(int64_t n) {
   int64_t blocks = (n + kCodecBlock - 1) / kCodecBlock;
   if (blocks > 256 * 8) blocks = 256 * 8;
@@ -558,6 +744,12 @@ int32_t coo_find_tiles(CooWork* work, const long long* d_idx, int64_t nnz, int64
   out->unordered = work->buffer.as<uint32_t>();
   out->starts = out->unordered + 1;
   out->tiles = (uint32_t)tiles;
+  bool with_bits = nnz * kCooBitsFrom >= n;
+  if (with_bits && work->bits.reserve((size_t)tiles * (kCooTile / 8)) != KRK_SUCCESS) {
+    (void)hipGetLastError();                         // no failure of a later launch
+    with_bits = false;                               // the indices are read again, then
+  }
+  out->bits = with_bits ? work->bits.as<uint32_t>() : nullptr;
   if (!work->host_unordered) {
     KRK_HIP(hipHostMalloc((void**)&work->host_unordered, 64, hipHostMallocCoherent));
     *work->host_unordered = 0u;
@@ -571,8 +763,13 @@ int32_t coo_find_tiles(CooWork* work, const long long* d_idx, int64_t nnz, int64
   }
   out->tag = ++work->calls;
   const bool vec = ((uintptr_t)d_idx & 15) == 0;
-  hipLaunchKernelGGL(coo_tiles_bounds_kernel, dim3(stream_grid((nnz + 3) / 4)), dim3(kCodecBlock), 0, stream, d_idx,
-                     nnz, n, vec, *out);
+  const dim3 block(kCodecBlock);
+  if (with_bits) {
+    constexpr int64_t per = (int64_t)(kCodecBlock / 64) * kCooRun * kCooChunk;
+    hipLaunchKernelGGL(coo_bits_kernel, dim3((unsigned)((nnz + per - 1) / per)), block, 0, stream, d_idx, nnz, n, vec, *out);
+  } else {
+    hipLaunchKernelGGL(coo_tiles_bounds_kernel, dim3(stream_grid((nnz + 3) / 4)), block, 0, stream, d_idx, nnz, n, vec, *out);
+  }
   KRK_HIP(hipGetLastError());
   return KRK_SUCCESS;
 }
@@ -604,7 +801,11 @@ int32_t coo_densify(CooWork* work, const long long* d_idx, const float* d_val, i
   }
   CooTiles tiles;
   KRK_TRY(coo_find_tiles(work, d_idx, nnz, n, &tiles, stream));
-  hipLaunchKernelGGL(coo_tiles_write_kernel, dim3(tiles.tiles), block, 0, stream, d_idx, d_val, d_dense, n, tiles);
+  if (tiles.bits) {
+    hipLaunchKernelGGL(coo_bits_write_kernel, dim3(tiles.tiles), block, 0, stream, d_val, d_dense, n, tiles);
+  } else {
+    hipLaunchKernelGGL(coo_tiles_write_kernel, dim3(tiles.tiles), block, 0, stream, d_idx, d_val, d_dense, n, tiles);
+  }
   KRK_HIP(hipGetLastError());
   return coo_scatter_if_unordered(tiles, d_idx, d_val, nnz, d_dense, n, stream);
 }

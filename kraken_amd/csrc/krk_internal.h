@@ -543,7 +543,7 @@ __device__ __forceinline__ void optim_element(const OptimK& k, float lr, float g
 // dense[0, n) = 0, then dense[idx[j]] += val[j]. Large tensors whose indices ascend strictly and
 // lie in range (what ToCoo produces) are taken tile by tile: one launch over the indices finds
 // where each tile's entries begin (coo_find_tiles), and whoever walks the tiles puts one together
-// in LDS. Any other input is zeroed and scattered into; which of the two it is is decided on the
+// in LDS, or, where there are many entries, from a bit an element that the first launch leaves. Any other input is zeroed and scattered into; which of the two it is is decided on the
 // device, and the launches of the other way look at the flag and leave.
 constexpr int kCooTile = 2048;                   // floats of one tile: 8 KB of LDS
 constexpr int64_t kCooTiledFrom = 1 << 22;       // smaller tensors: zero + scatter, two launches are quicker
@@ -553,16 +553,42 @@ struct CooTiles {
   uint32_t tag;
   uint32_t tiles;
   uint32_t* host_unordered;   // page-locked copy of the flag, raised by who walks the tiles
+  uint32_t* bits;         // null, or a bit an element, 64 words a tile: whether an entry names it
 };
 __device__ __forceinline__ bool coo_unordered(const CooTiles& t) { return *t.unordered == t.tag; }
 struct CooWork {          // work space of one caller, kept between calls
-  DeviceBuffer buffer;
+  DeviceBuffer buffer, bits;
   uint32_t calls = 0;
   uint32_t* host_unordered = nullptr;
   void release() {
     buffer.release();
+    bits.release();
     if (host_unordered) (void)hipHostFree(host_unordered);
     host_unordered = nullptr;
+  }
+};
+// Which of a tile's elements have an entry, and how many entries of the tile lie before each of its 64 words: a lane
+// holds the word of its number. All lanes of a wavefront.
+struct CooTileBits {
+  uint32_t word, before;
+  __device__ __forceinline__ explicit CooTileBits(uint32_t w) : word(w) {
+    const uint32_t own = (uint32_t)__popc(w);
+    before = wave_inclusive_sum(own) - own;
+  }
+  // The gradient of the four elements of quad q of the tile, whose entries are [start, end) (end > start, or all bits are
+  // clear): the values of those that have an entry, zero for the others.
+  __device__ __forceinline__ void quad(int q, const float* __restrict__ val, uint32_t start, uint32_t end, float (&g)[4]) const {
+    const uint32_t w = (uint32_t)__shfl((int)word, q >> 3);
+    const int shift = (q & 7) * 4;
+    const uint32_t mine = (w >> shift) & 15u;
+    uint32_t at = start + (uint32_t)__shfl((int)before, q >> 3) + (uint32_t)__popc(w & ((1u << shift) - 1u));
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      // (read whether the element has an entry or not: four loads that wait for one another in no way)
+      const float v = val[min(at, end - 1u)];
+      g[c] = (mine >> c) & 1u ? v : 0.0f;
+      at += (mine >> c) & 1u;
+    }
   }
 };
 inline bool coo_tiled(int64_t n, int64_t nnz) { return n >= kCooTiledFrom && nnz < ((int64_t)1 << 31); }

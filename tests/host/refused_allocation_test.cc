@@ -1,6 +1,7 @@
 // A push of up to 2^20 ids takes work space for the sums of rows that many positions share, and is sorted
 // where that cannot be had. This program stands between the library and hipMalloc and refuses what
-// is larger than a limit: the push has the same result, and the next one, with the room, too.
+// is larger than a limit: the push has the same result, and the next one, with the room, too. A decode of
+// many entries keeps a bit an element, and reads the indices twice where it has no room for them.
 #include <dlfcn.h>
 
 #include <cstddef>
@@ -70,6 +71,27 @@ int main() {
     for (int64_t i = 0; i < rows * dim; ++i) CHECK(got[i] == before[i] - (float)(0.5 * sums[i] * pass));
   }
   CHECK(krk_sparse_destroy(t) == 0);
+
+  const int64_t len = (int64_t)1 << 23, nnz = len / 2;   // a megabyte of bits, 16 KB of everything else
+  std::vector<int64_t> idx(nnz);
+  std::vector<float> val(nnz), dense(len), want(len, 0.0f);
+  for (int64_t j = 0; j < nnz; ++j) {
+    idx[j] = 2 * j + (j * 7 % 5 == 0);
+    val[j] = want[idx[j]] = (float)(j % 1000 + 1);
+  }
+  void *d_idx = nullptr, *d_val = nullptr, *d_dense = nullptr;
+  CHECK(krk_malloc(&d_idx, nnz * 8) == 0 && krk_malloc(&d_val, nnz * 4) == 0 && krk_malloc(&d_dense, len * 4) == 0);
+  CHECK(krk_memcpy_h2d(d_idx, idx.data(), nnz * 8) == 0 && krk_memcpy_h2d(d_val, val.data(), nnz * 4) == 0);
+  for (int pass = 1; pass <= 2; ++pass) {
+    limit = pass == 2 ? SIZE_MAX : (size_t)512 << 10;
+    refused = 0;
+    CHECK(krk_coo_to_dense(static_cast<int64_t*>(d_idx), static_cast<float*>(d_val), nnz, static_cast<float*>(d_dense),
+                           len, KRK_DEVICE_PTRS) == 0);
+    CHECK(refused == (pass == 2 ? 0 : 1));
+    limit = SIZE_MAX;
+    CHECK(krk_memcpy_d2h(dense.data(), d_dense, len * 4) == 0);
+    CHECK(dense == want);
+  }
   std::printf("refused allocation ok\n");
   return 0;
 }

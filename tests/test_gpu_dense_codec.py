@@ -278,6 +278,62 @@ def test_coo_gaps_of_every_length(api, oracle):
         assert np.array_equal(api.coo_to_dense(idx, val, n), want), entries[:4]
 
 
+def _many_entries(case, n):
+    """Ascending indices, an entry in eight elements or more."""
+    rng = np.random.default_rng(7)
+    if case == "front":                  # one long run of entries and nothing behind it
+        return np.arange(n // 6)
+    if case == "back":
+        return np.arange(n - n // 6, n)
+    if case == "tiles":                  # every third tile full, the first and the last of the others' elements too
+        i = np.arange(n)
+        t, at = i // 2048, i % 2048
+        return i[(t % 3 == 0) | ((t % 3 == 1) & ((at == 0) | (at == 2047)))]
+    if case == "gaps":                   # stretches of a few words with gaps of 1 to 200 words between them
+        size, gap = rng.integers(1, 40, n // 32) * 32 + rng.integers(0, 32, n // 32), rng.integers(1, 200, n // 32) * 32
+        at = np.cumsum(size + gap) - size
+        i = np.concatenate([np.arange(a, a + s) for a, s in zip(at[at < n], size)])
+        return i[i < n]
+    keep = rng.random(n) < dict(half=0.5, fifth=0.2, all=2.0)[case]
+    return np.flatnonzero(keep)
+
+
+@pytest.mark.parametrize("n", [1 << 22, (1 << 22) + 2047])
+@pytest.mark.parametrize("case", ["front", "back", "tiles", "gaps", "half", "fifth", "all"])
+def test_coo_many_entries(api, oracle, case, n):
+    """Tensors with an entry in eight elements or more: decode and push, every element exact. Then with the number of
+    entries next to where a wavefront's chunks and runs of chunks end, and with one pair out of order, one
+    index twice and one outside, where two wavefronts meet."""
+    full = _many_entries(case, n).astype(np.int64)
+    assert full.size * 8 >= n
+    t = api.DenseTable(np.zeros(n, np.float32))
+    opt = api.Optim.create(api.OptimType.kSGD)
+    w = np.zeros(n, np.float32)
+
+    def check(idx):
+        nonlocal w
+        val = (np.arange(idx.size) % 61 - 30).astype(np.float32)
+        inside = (idx >= 0) & (idx < n)
+        want = np.zeros(n, np.float32)
+        np.add.at(want, idx[inside], val[inside])
+        assert np.array_equal(api.coo_to_dense(idx, val, n), want)
+        assert t.PushCoo(opt, idx, val, 0.5) == 0
+        w = w - np.float32(0.5) * want
+        assert np.array_equal(t.Pull()[1], w)
+
+    check(full)
+    for cut in (1, 31, 32, 255, 256, 257, 1023, 1024, 1025):
+        check(full[full.size % 1024 + 1024 - cut:] if case == "back" else full[:full.size - full.size % 1024 - 1024 + cut])
+    at = full.size // 2 // 1024 * 1024
+    swapped, twice, outside = full.copy(), full.copy(), full.copy()
+    swapped[[at - 1, at]] = swapped[[at, at - 1]]
+    twice[at] = twice[at - 1]
+    outside[-1] = n
+    for idx in (swapped, twice, outside):
+        check(idx)
+    check(full)
+
+
 def test_dense_push_coo_large(api, oracle):
     n = (1 << 22) + 77
     rng = np.random.default_rng(4)
