@@ -48,16 +48,16 @@ struct Quad {
 };
 typedef float vfloat4 __attribute__((ext_vector_type(4)));   // what the non-temporal builtins accept
 
+__device__ __forceinline__ Quad whole_quad(const float* __restrict__ p, int64_t j) {
+  const vfloat4 x = __builtin_nontemporal_load(reinterpret_cast<const vfloat4*>(p + j));
+  return Quad{{x[0], x[1], x[2], x[3]}};
+}
 // four consecutive elements from j on; elements at or behind n read as zero
 __device__ __forceinline__ Quad load_quad(const float* __restrict__ p, int64_t j, int64_t n, bool vec) {
+  if (vec && j + 3 < n) return whole_quad(p, j);
   Quad q;
-  if (vec && j + 3 < n) {
-    const vfloat4 x = __builtin_nontemporal_load(reinterpret_cast<const vfloat4*>(p + j));
-    q.v[0] = x[0]; q.v[1] = x[1]; q.v[2] = x[2]; q.v[3] = x[3];
-  } else {
 #pragma unroll
-    for (int c = 0; c < 4; ++c) q.v[c] = j + c < n ? p[j + c] : 0.0f;
-  }
+  for (int c = 0; c < 4; ++c) q.v[c] = j + c < n ? p[j + c] : 0.0f;
   return q;
 }
 
@@ -206,17 +206,37 @@ __global__ __launch_bounds__(kCodecBlock) void emit_count_kernel(const float* __
   }
 }
 
-// One tile of `ROWS` rows of 256 elements per wavefront: the kept (index, value) pairs in input order
+// A lane's elements of a tile of `ROWS` rows of 256 elements per wavefront.
+template <int BLOCK, int ROWS>
+__device__ __forceinline__ void load_tile(const float* __restrict__ g, const float* __restrict__ e, int64_t n,
+                                          int64_t tile, bool vec, Quad (&a)[ROWS], Quad (&b)[ROWS]) {
+  constexpr int64_t kTile = BLOCK / 64 * 256 * ROWS;
+  const int64_t base = tile * kTile + (threadIdx.x >> 6) * (256 * ROWS) + (threadIdx.x & 63) * 4;
+  if (vec && (tile + 1) * kTile <= n) {            // uniform
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      a[r] = whole_quad(g, base + r * 256);
+      b[r] = whole_quad(e, base + r * 256);
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      a[r] = load_quad(g, base + r * 256, n, vec);
+      b[r] = load_quad(e, base + r * 256, n, true);
+    }
+  }
+}
+
+// One tile, of which a and b are what load_tile loaded: the kept (index, value) pairs in input order
 // and the new residual. announce(kept) is called once the tile's count is known, by every thread;
 // resolve() yields where the tile's pairs go, to every thread, and is asked for last, when everything
 // that does not depend on it is done. A tile's pairs are first gathered in LDS in output order
 // and then written out by consecutive lanes, so that the index and value arrays are written in whole
 // lines (a lane writing its own few kept elements leaves partly written lines behind).
-template <int BLOCK, int ROWS, typename Announce, typename Resolve>
-__device__ __forceinline__ void emit_tile(const float* __restrict__ g, const float* __restrict__ e, int64_t n,
-                                          int64_t tile, bool vec, uint32_t tau_bits, long long* __restrict__ idx,
-                                          float* __restrict__ val, float* __restrict__ e_next, Announce announce,
-                                          Resolve resolve) {
+template <int BLOCK, int ROWS, typename Announce, typename Ahead, typename Resolve>
+__device__ __forceinline__ void emit_tile(const Quad (&a)[ROWS], const Quad (&b)[ROWS], int64_t n, int64_t tile,
+                                          uint32_t tau_bits, long long* __restrict__ idx, float* __restrict__ val,
+                                          float* __restrict__ e_next, Announce announce, Ahead ahead, Resolve resolve) {
   constexpr int kWaveElems = 256 * ROWS;
   constexpr int kWaves = BLOCK / 64;
   constexpr int kTile = kWaves * kWaveElems;
@@ -232,21 +252,14 @@ __device__ __forceinline__ void emit_tile(const float* __restrict__ g, const flo
   Quad f[ROWS];
   unsigned long long masks[ROWS][4];
   int wave_total = 0;
-  {
-    Quad a[ROWS], b[ROWS];
+  const bool whole = (tile + 1) * kTile <= n;      // uniform
 #pragma unroll
-    for (int r = 0; r < ROWS; ++r) {
-      a[r] = load_quad(g, base + r * 256, n, vec);
-      b[r] = load_quad(e, base + r * 256, n, true);
-    }
+  for (int r = 0; r < ROWS; ++r) {
 #pragma unroll
-    for (int r = 0; r < ROWS; ++r) {
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        f[r].v[k] = a[r].v[k] + b[r].v[k];
-        masks[r][k] = __ballot(base + r * 256 + k < n && abs_bits(f[r].v[k]) >= tau_bits);
-        wave_total += __popcll(masks[r][k]);
-      }
+    for (int k = 0; k < 4; ++k) {
+      f[r].v[k] = a[r].v[k] + b[r].v[k];
+      masks[r][k] = __ballot((whole || base + r * 256 + k < n) && abs_bits(f[r].v[k]) >= tau_bits);
+      wave_total += __popcll(masks[r][k]);
     }
   }
   if (lane == 0) wave_sum[wave] = wave_total;
@@ -258,6 +271,7 @@ __device__ __forceinline__ void emit_tile(const float* __restrict__ g, const flo
     count += wave_sum[w];
   }
   announce(count);
+  ahead();
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
     const int64_t j = base + r * 256;
@@ -280,7 +294,7 @@ __device__ __forceinline__ void emit_tile(const float* __restrict__ g, const flo
       }
       rest[k] = keep ? 0.0f : f[r].v[k];           // t/math.cc:1098-1123 : |x| < th keeps x
     }
-    if (j + 3 < n) {
+    if (whole || j + 3 < n) {
       const vfloat4 out = {rest[0], rest[1], rest[2], rest[3]};
       __builtin_nontemporal_store(out, reinterpret_cast<vfloat4*>(e_next + j));
     } else {
@@ -306,12 +320,15 @@ __global__ __launch_bounds__(kCodecBlock) void emit_write_kernel(
     const uint32_t* __restrict__ sel, const int32_t* __restrict__ tile_offsets, long long* __restrict__ idx,
     float* __restrict__ val, float* __restrict__ e_next) {
   const uint32_t tau_bits = sel[2];
-  for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x)
-    emit_tile<kCodecBlock, kCodecRows>(g, e, n, tile, vec, tau_bits, idx, val, e_next, [](int) {},
-                          [&](int) -> int64_t {
-                            __syncthreads();
-                            return tile_offsets[tile];
-                          });
+  for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    Quad a[kCodecRows], b[kCodecRows];
+    load_tile<kCodecBlock>(g, e, n, tile, vec, a, b);
+    emit_tile<kCodecBlock>(a, b, n, tile, tau_bits, idx, val, e_next, [](int) {}, [] {},
+                           [&](int) -> int64_t {
+                             __syncthreads();
+                             return tile_offsets[tile];
+                           });
+  }
 }
 
 // The whole emit step in one pass: gradient and residual are read once (a count pass ahead of the
@@ -324,12 +341,22 @@ __global__ __launch_bounds__(kCodecBlock) void emit_write_kernel(
 // workgroup that already runs, and it announces its count before it waits for anything: every wait
 // ends. An announcement carries the number of the call, so the array is never cleared; the last
 // workgroup to leave puts the counter back to zero.
-// Tiles of 8192: the counter serves one workgroup after the other, some 15 ns each, which is what
-// smaller tiles wait for (67 million elements: 427 us in tiles of 2048, 297 us in tiles of 4096).
+// A workgroup takes its next tile's number, and asks for its elements, ahead of writing the one it has: a tile
+// that is held but not announced is waited for by later tiles only, and its workgroup waits for earlier ones, so the lowest such
+// tile's turn always comes.
+// What bounds it is the rate of a copy: 67 million elements, of which 33 million are kept, 1.27 GB, 217 us (5.8 TB/s). 243 us with each
+// tile's loads behind the tile before it, two workgroups a compute unit, 8192 elements a tile; with the loads ahead, tiles
+// of 8192 / 16,384 elements and 192, 256, 320, 384 workgroups 255, 222, 250, 248 / 230, 217, 216, 217: the fewer tiles are on
+// their way, the less far a tile has to look back. The counter serves one workgroup after the other, some 15 ns each,
+// which is what smaller tiles wait for (573 and 331 us in tiles of 2048 and 4096); tensors that give
+// few workgroups a tile are better off with them. A blocking step, us, as before / in tiles of 4096 / 8192 / 16,384: 300,000
+// elements 15.6 / 14.2 / 16.2 / 19.2, a million 17.6 / 19.1 / 17.4 / 19.9, 4 million 31.9 / 31.6 / 29.2 / 32.6,
+// 16 million 74 / 89 / 67 / 70, 33 million 132 / 170 / 119 / 119, 67 million 252 / 331 / 229 / 224.
+constexpr int64_t kSingleShort = (int64_t)1 << 19;
+constexpr int64_t kSingleLong = (int64_t)1 << 25;
 constexpr int kSingleBlock = 512;
-constexpr int kSingleRows = 4;
-constexpr int kSingleTile = (kSingleBlock / 64) * 256 * kSingleRows;
-constexpr int kSingleGrid = 512;
+constexpr int single_tile(int rows) { return (kSingleBlock / 64) * 256 * rows; }
+constexpr int kSingleGrid = 256;
 constexpr uint32_t kTileCount = 1u, kTileTotal = 2u;   // what the low word is: the tile's own count, or all up to it
 constexpr uint32_t kMaxEmitCalls = 1u << 30;
 
@@ -338,6 +365,7 @@ __device__ __forceinline__ void tell(unsigned long long* state, uint32_t call, u
                      __HIP_MEMORY_SCOPE_AGENT);
 }
 
+template <int ROWS>
 __global__ __launch_bounds__(kSingleBlock) void emit_single_kernel(
     const float* __restrict__ g, const float* __restrict__ e, int64_t n, uint32_t tiles, bool vec,
     uint32_t* __restrict__ sel, unsigned long long* tile_state, uint32_t* tickets, uint32_t call,
@@ -346,15 +374,24 @@ __global__ __launch_bounds__(kSingleBlock) void emit_single_kernel(
   __shared__ uint32_t s_tile, s_before;
   const uint32_t tau_bits = sel[2];
   const int lane = threadIdx.x & 63;
-  for (;;) {
-    if (threadIdx.x == 0) s_tile = atomicAdd(&tickets[0], 1u);
-    __syncthreads();
-    const uint32_t tile = s_tile;
-    if (tile >= tiles) break;                      // the whole workgroup
-    emit_tile<kSingleBlock, kSingleRows>(
-        g, e, n, tile, vec, tau_bits, idx, val, e_next,
+  const bool once = tiles <= gridDim.x;            // a tile a workgroup: the counter is spared the second round
+  if (threadIdx.x == 0) s_tile = atomicAdd(&tickets[0], 1u);
+  __syncthreads();
+  uint32_t tile = s_tile;
+  __syncthreads();
+  Quad a[ROWS], b[ROWS];
+  if (tile < tiles) load_tile<kSingleBlock>(g, e, n, tile, vec, a, b);
+  while (tile < tiles) {                           // the whole workgroup
+    if (threadIdx.x == 0) s_tile = once ? tiles : atomicAdd(&tickets[0], 1u);
+    uint32_t next = tiles;
+    emit_tile<kSingleBlock>(
+        a, b, n, tile, tau_bits, idx, val, e_next,
         [&](int count) {
           if (threadIdx.x == 0) tell(&tile_state[tile], call, tile == 0 ? kTileTotal : kTileCount, (uint32_t)count);
+        },
+        [&] {
+          next = s_tile;                           // (a barrier behind its store)
+          if (next < tiles) load_tile<kSingleBlock>(g, e, n, next, vec, a, b);
         },
         [&](int count) -> int64_t {
           if (threadIdx.x < 64) {
@@ -394,6 +431,7 @@ __global__ __launch_bounds__(kSingleBlock) void emit_single_kernel(
           __syncthreads();
           return s_before;
         });
+    tile = next;
   }
   if (threadIdx.x == 0 && atomicAdd(&tickets[1], 1u) == gridDim.x - 1) {
     __hip_atomic_store(&tickets[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -837,7 +875,7 @@ int32_t krk_dct_create(int64_t n, krk_dct** out) {
     if (e == hipSuccess) e = hipMalloc((void**)&s->tile_counts, (size_t)s->tiles * sizeof(int32_t));
     if (e == hipSuccess) e = hipMalloc((void**)&s->tile_offsets, (size_t)s->tiles * sizeof(int32_t));
     if (e == hipSuccess) e = hipMalloc(&s->scan_tmp, scan_scratch_bytes(s->tiles));
-    const size_t state_b = (size_t)((n + kSingleTile - 1) / kSingleTile + 1) * sizeof(unsigned long long);
+    const size_t state_b = (size_t)((n + single_tile(2) - 1) / single_tile(2) + 1) * sizeof(unsigned long long);
     if (e == hipSuccess) e = hipMalloc((void**)&s->tile_state, state_b);
     if (e == hipSuccess) e = hipMalloc((void**)&s->tickets, 64);
     if (e == hipSuccess) e = hipMemsetAsync(s->tile_state, 0, state_b, s->stream);
@@ -917,16 +955,21 @@ int32_t krk_dct_compress(krk_dct* s, const float* grad, uint64_t life_span, floa
   // Room for every element and device buffers: nothing can overflow and nothing is staged, so one
   // pass emits and the count comes with it.
   if ((flags & KRK_DEVICE_PTRS) && capacity >= n) {
-    const int64_t tiles = (n + kSingleTile - 1) / kSingleTile;
+    const int rows = n <= kSingleShort ? 2 : n <= kSingleLong ? 4 : 8;
+    const int64_t tiles = (n + single_tile(rows) - 1) / single_tile(rows);
     if (++s->emit_calls == kMaxEmitCalls) {
       KRK_HIP(hipMemsetAsync(s->tile_state, 0, (size_t)tiles * sizeof(unsigned long long), s->stream));
       s->emit_calls = 1;
     }
     uint32_t* d_host_sel = nullptr;
     KRK_HIP(hipHostGetDevicePointer((void**)&d_host_sel, s->host_sel, 0));
-    hipLaunchKernelGGL(emit_single_kernel, dim3((unsigned)(tiles < kSingleGrid ? tiles : kSingleGrid)),
-                       dim3(kSingleBlock), 0, s->stream, d_g, s->e, n, (uint32_t)tiles, vec, s->sel, s->tile_state,
-                       s->tickets, s->emit_calls, reinterpret_cast<long long*>(idx), val, s->e_next, d_host_sel);
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles < kSingleGrid ? tiles : kSingleGrid)), dim3(kSingleBlock), 0, s->stream, d_g, s->e, n, (uint32_t)tiles, vec, s->sel, s->tile_state,
+                         s->tickets, s->emit_calls, reinterpret_cast<long long*>(idx), val, s->e_next, d_host_sel);
+    };
+    if (rows == 8) launch(emit_single_kernel<8>);
+    else if (rows == 4) launch(emit_single_kernel<4>);
+    else launch(emit_single_kernel<2>);
     KRK_HIP(hipGetLastError());
     KRK_TRY(wait_stream(s->stream));
     *nnz = (int64_t)s->host_sel[3];

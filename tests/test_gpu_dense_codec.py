@@ -174,6 +174,28 @@ def test_codec_single_pass_emit(api, oracle, n, eta):
     bag.close()
 
 
+@pytest.mark.parametrize("n", [4095, 4096, 4097, 1 << 19, (1 << 19) + 1, 8192 * 256, 8192 * 256 + 1, 16384 * 2048 + 1])
+def test_codec_single_pass_tile_sizes(api, n):
+    """Where the tiles' size changes (2^19 and 2^25 elements), at their edges, and with as many tiles as workgroups and
+    one more: the pairs, in order, and the residual, against numpy with the threshold that the codec found."""
+    rng = np.random.default_rng(n)
+    bag = api.DenseBag(n)
+    e = np.zeros(n, np.float32)
+    for step in range(2):
+        g = rng.standard_normal(n, dtype=np.float32)
+        d_idx, d_val, nnz = bag.MaybeToCoo(2, 0.75, api.DeviceArray.from_host(g))
+        f = g + e
+        a = np.abs(f)
+        if step == 0:                                # the k-th largest of k = n / 4
+            assert bag.tau == np.partition(a, n - int(n * 0.25))[n - int(n * 0.25)]
+        idx = np.flatnonzero(a >= bag.tau)
+        assert nnz == idx.size
+        assert np.array_equal(d_idx.to_host()[:nnz], idx) and np.array_equal(d_val.to_host()[:nnz], f[idx])
+        e = np.where(a < bag.tau, f, np.float32(0))
+        assert np.array_equal(bag.residual, e)
+    bag.close()
+
+
 @pytest.mark.parametrize("case", ["sgd_mom", "adam_amsgrad", "rmsprop_all"])
 @pytest.mark.parametrize("n", [(1 << 22), (1 << 22) + 2049])
 def test_dense_push_coo_tiles(api, oracle, case, n):
