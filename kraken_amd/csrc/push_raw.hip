@@ -1451,7 +1451,7 @@ template <typename Fill>
 static int32_t sort_and_reduce(const ReduceShape& sh, hipStream_t stream, DeviceBuffer* scratch,
                                const TableView& tv, int opt, int64_t n, uint32_t miss_key, int bits,
                                const float* d_vals, const ApplyArgs& args, const PooledSrc& ps,
-                               const GroupSrc* gs, const GroupPooledSrc* gps, Fill fill) {
+                               const GroupSrc* gs, const GroupPooledSrc* gps, const NotedBags& noted_bags, Fill fill) {
   const int tile0 = kLevel0Tile;
   const int per_block = kBlock / sh.group;
   const int64_t groups0 = ((n + tile0 - 1) / tile0 + per_block - 1) / per_block;   // workgroups of level 0
@@ -1468,9 +1468,14 @@ static int32_t sort_and_reduce(const ReduceShape& sh, hipStream_t stream, Device
   uint32_t* skeys = nullptr;
   uint32_t* spos = nullptr;
 
-  fill(keys, pos);
-  KRK_HIP(hipGetLastError());
-  KRK_TRY(radix_sort_pairs(keys, pos, pos + n, pos + 2 * n, n, bits, scratch[1].ptr, stream, &skeys, &spos));
+  if (noted_bags.offsets) {
+    KRK_TRY(radix_sort_noted_bags(noted_bags, tv, miss_key, keys, pos, pos + n, pos + 2 * n, n, bits, scratch[1].ptr,
+                                  stream, &skeys, &spos));
+  } else {
+    fill(keys, pos);
+    KRK_HIP(hipGetLastError());
+    KRK_TRY(radix_sort_pairs(keys, pos, pos + n, pos + 2 * n, n, bits, scratch[1].ptr, stream, &skeys, &spos));
+  }
 
   // level 0 reads value rows through the sorted payloads; later levels read the carry list
   uint32_t* ckeys[2] = {scratch[2].as<uint32_t>(), scratch[2].as<uint32_t>() + carry_entries};
@@ -1515,12 +1520,14 @@ static int32_t sort_and_reduce(const ReduceShape& sh, hipStream_t stream, Device
 // holds at once, the tiled reduction's walks use the memory better than workgroups that sort first
 // (8.5 million pooled ids of 32 floats: reduction 468 us against 574, partition and sort 180 and
 // 215; the sort has come down to 140 since).
-// noted: single tables whose rows the pull noted; fill is not called then.
+// noted: single tables whose rows the pull noted; fill is not called then. noted_bags: the same for pooled
+// pushes that are sorted.
 template <typename Fill>
 static int32_t fill_and_reduce(const ReduceShape& sh, hipStream_t stream, DeviceBuffer* scratch, const TableView& tv,
                                int opt, int64_t n, uint32_t miss_key, int bits, const float* d_vals,
                                const ApplyArgs& args, const PooledSrc& ps, const GroupSrc* gs,
-                               const GroupPooledSrc* gps, const NotedRows& noted, Fill fill) {
+                               const GroupPooledSrc* gps, const NotedRows& noted, const NotedBags& noted_bags,
+                               Fill fill) {
   // (buckets take a quarter of the gradients' size as work space, which the sort does not need)
   bool buckets = n <= kRunsMax;
   if (buckets && reserve_runs(sh, scratch, n) != KRK_SUCCESS) {
@@ -1528,7 +1535,7 @@ static int32_t fill_and_reduce(const ReduceShape& sh, hipStream_t stream, Device
     buckets = false;
   }
   if (!buckets)
-    return sort_and_reduce(sh, stream, scratch, tv, opt, n, miss_key, bits, d_vals, args, ps, gs, gps, fill);
+    return sort_and_reduce(sh, stream, scratch, tv, opt, n, miss_key, bits, d_vals, args, ps, gs, gps, noted_bags, fill);
   uint32_t* keys = scratch[0].as<uint32_t>();
   if (!noted.rows) {
     fill(keys, keys + n);
@@ -1579,12 +1586,12 @@ static SortCall table_sort_call(const krk_sparse* t, int64_t n) {
 // pooled pushes). The caller holds the table's lock and has made the optimizer's columns exist.
 template <typename Fill>
 static int32_t push_sorted(krk_sparse* t, const krk_optim* o, int64_t n, const float* d_g, float lr,
-                           const PooledSrc& ps, const NotedRows& noted, Fill fill) {
+                           const PooledSrc& ps, const NotedRows& noted, const NotedBags& noted_bags, Fill fill) {
   uint32_t miss_key;
   const int bits = key_bits(t, &miss_key);
   const ReduceShape sh{t->dim, t->vec, t->elems, t->group};
   return fill_and_reduce(sh, t->stream, t->scratch, t->view(), o->type, n, miss_key, bits, d_g,
-                         table_apply_args(t, o, lr), ps, nullptr, nullptr, noted,
+                         table_apply_args(t, o, lr), ps, nullptr, nullptr, noted, noted_bags,
                          [&](uint32_t* keys, uint32_t* pos) { fill(keys, pos, miss_key); });
 }
 
@@ -1987,7 +1994,7 @@ int32_t krk_dedup_sum(const uint64_t* ids, int64_t n, const float* grads, int64_
                       PooledSrc{}, nullptr, nullptr));
   } else {
     KRK_TRY(fill_and_reduce(sh, s, g_dedup_reduce, tv, kOptStore, n, miss_key, bits, d_g, args, PooledSrc{}, nullptr,
-                            nullptr, NotedRows{}, [](uint32_t*, uint32_t*) {}));
+                            nullptr, NotedRows{}, NotedBags{}, [](uint32_t*, uint32_t*) {}));
   }
   KRK_TRY(dedup_read_count(s, &u));
   *n_unique = u;
@@ -2123,7 +2130,7 @@ int32_t krk_sparse_push_raw(krk_sparse* t, const krk_optim* o, const uint64_t* i
     return sparse_finish(t, flags);
   }
   const uint32_t* notes = noted_rows(t, ids, n, flags);
-  KRK_TRY(push_sorted(t, o, n, d_g, lr, PooledSrc{}, NotedRows{notes, d_ids},
+  KRK_TRY(push_sorted(t, o, n, d_g, lr, PooledSrc{}, NotedRows{notes, d_ids}, NotedBags{},
                       [&](uint32_t* keys, uint32_t* pos, uint32_t miss_key) {
                         if (notes) {
                           hipLaunchKernelGGL(noted_keys_kernel, dim3(grid_for(n, kBlock)), dim3(kBlock), 0, t->stream,
@@ -2262,7 +2269,7 @@ static int32_t group_push_raw_enqueue(krk_group* g, const krk_optim* o, const in
   }
   const uint32_t* notes = noted_rows(g, parts.ids, offsets, flags);
   return fill_and_reduce(sh, g->stream, g->scratch, TableView{}, o->type, total, miss_key, gk.bits, nullptr, args,
-                         PooledSrc{}, &gs, &src, NotedRows{}, [&](uint32_t* keys, uint32_t* pos) {
+                         PooledSrc{}, &gs, &src, NotedRows{}, NotedBags{}, [&](uint32_t* keys, uint32_t* pos) {
                            if (notes) {
                              hipLaunchKernelGGL(group_noted_keys_kernel, dim3(grid_for(total, kBlock)), dim3(kBlock), 0,
                                                 g->stream, g->d_descs, call, parts, total, row_bits, miss_key, notes,
@@ -2275,10 +2282,10 @@ static int32_t group_push_raw_enqueue(krk_group* g, const krk_optim* o, const in
                          });
 }
 
-// A pooled push on one table, which `call` describes as its only member (device addresses). The caller
-// holds the table's lock and has made the optimizer's columns exist.
+// A pooled push on one table, which `call` describes as its only member (device addresses; device_offsets: and
+// the offsets are device memory). The caller holds the table's lock and has made the optimizer's columns exist.
 static int32_t push_pooled_enqueue(krk_sparse* t, const krk_optim* o, PooledCall& call, const uint32_t* notes,
-                                   float lr) {
+                                   bool device_offsets, float lr) {
   const int64_t n = call.row_start[1], bags = call.bag_start[1];
   const bool weighted = call.weights[0] != nullptr;
   const int64_t blocks = pooled_layout(&call, kBlock / kBagLanes);
@@ -2337,7 +2344,10 @@ static int32_t push_pooled_enqueue(krk_sparse* t, const krk_optim* o, PooledCall
     KRK_HIP(hipGetLastError());
     return KRK_SUCCESS;
   }
-  return push_sorted(t, o, n, call.rows[0], lr, src, NotedRows{}, fill);
+  // (tiles search the offsets for their bags: not across PCIe)
+  const NotedBags noted{notes, call.ids[0], notes && device_offsets ? call.offsets[0] : nullptr, bags, words,
+                        weighted ? bag_of : nullptr};
+  return push_sorted(t, o, n, call.rows[0], lr, src, NotedRows{}, noted, fill);
 }
 
 extern "C" {
@@ -2466,7 +2476,7 @@ int32_t krk_sparse_push_pooled(krk_sparse* t, const krk_optim* o, const uint64_t
   call.rows[0] = const_cast<float*>(d_g);
   call.stride[0] = (uint32_t)t->dim;
   call.mean_bits = mode == KRK_POOL_MEAN ? 1u : 0u;
-  KRK_TRY(push_pooled_enqueue(t, o, call, noted_rows(t, ids, n, flags), lr));
+  KRK_TRY(push_pooled_enqueue(t, o, call, noted_rows(t, ids, n, flags), (flags & KRK_DEVICE_PTRS) != 0, lr));
   return sparse_finish(t, flags);
 }
 
@@ -2578,6 +2588,6 @@ int32_t krk_group_push_pooled_parts(krk_group* g, const krk_optim* o, const krk_
     return group_finish(g, flags);
   }
   KRK_TRY(fill_and_reduce(sh, g->stream, g->scratch, TableView{}, o->type, total, gk.miss_key, gk.bits, nullptr, args,
-                          PooledSrc{}, &gs, &src, NotedRows{}, fill));
+                          PooledSrc{}, &gs, &src, NotedRows{}, NotedBags{}, fill));
   return group_finish(g, flags);
 }

@@ -19,7 +19,7 @@
 // An XCD takes a stretch of consecutive tiles (xcd_tile): neighbouring tiles write neighbouring counts and, for
 // every digit, neighbouring pieces of some 48 bytes, which meet in its L2 and leave as whole lines (the scatter
 // of 8.5 million pairs 36.6 -> 32.4 us a pass; it moves 136 MB, 24 us at the rate of a copy).
-#include "krk_internal.h"
+#include "reduce_internal.h"
 
 namespace krk {
 
@@ -35,6 +35,149 @@ constexpr int kRsWaves = kRsBlock / kWave;
 constexpr int kRsMaxBits = 9;
 constexpr int kRsDigits = 1 << kRsMaxBits;
 
+// ---- a pooled push's pairs, from the pull's notes and the bags' offsets ----
+// The first pass puts them together as it reads them: its histogram takes the notes, the scan's launch
+// finds the bags in which tiles begin, and the scatter works every position's bag out. A launch that wrote the pairs
+// out in advance (a lane group a bag, as for requests short enough for buckets) moved 117 MB for 8.5 million positions,
+// 32 us; without it the first histogram takes 15.5 us for 11 (the notes come from further away than pairs just
+// written) and the first scatter 38 for 30: a pooled step of 952 us 936. Requests of up to 2^20
+// positions keep that launch: in the partition's launches the same cost what it saved.
+
+// The bag that the offsets step over p with, offsets[bag] <= p < offsets[bag + 1]: searched by a whole
+// wavefront, 64 offsets a step. offsets[0] <= p < offsets[bags], which every step keeps true of what is left,
+// also where offsets in between descend (they are not checked).
+__device__ __forceinline__ int64_t bag_at(const long long* __restrict__ offsets, int64_t bags, long long p) {
+  const int lane = threadIdx.x & (kWave - 1);
+  int64_t lo = 0, hi = bags;
+  while (hi - lo > 1) {
+    const int64_t step = (hi - lo + kWave - 1) / kWave;
+    const int64_t at = lo + (lane + 1) * step;
+    const unsigned long long before = __ballot(at < hi && offsets[at] <= p);
+    const int64_t steps = kWave - __clzll((long long)before);   // the last lane whose offset is not above p; none: 0
+    lo += steps * step;
+    hi = lo + step < hi ? lo + step : hi;
+  }
+  return lo;
+}
+
+// The bags in which the tiles of `tile` positions begin, starts[0..tiles], a wavefront each: work for a launch
+// ahead of the one that needs them, whose workgroups waited 5 us for them with a search of their own
+// (8.5 million positions, three rounds of workgroups: 43 us in place of 30).
+__device__ __forceinline__ void find_tile_starts(const NotedBags& in, int64_t wave, int64_t tiles, int tile,
+                                                 uint32_t* __restrict__ starts) {
+  if (wave > tiles) return;
+  const long long first = in.offsets[0], past = in.offsets[in.bags];
+  long long p = wave * tile;
+  if (p < first) p = first;
+  if (p >= past) p = past - 1;
+  const int64_t b = first < past ? bag_at(in.offsets, in.bags, p) : 0;   // (no position lies in a bag)
+  if ((threadIdx.x & (kWave - 1)) == 0) starts[wave] = (uint32_t)b;
+}
+
+// The words of a tile's positions, element i of a lane being position wave * (64 * ITEMS) + i * 64 + lane
+// of the tile: the lanes leave every bag's word where it begins (mark), and a position takes the nearest one at
+// or before it (word), which votes find inside a wavefront's stretch, and a note per wavefront before that. Positions of
+// no bag get kNoBag. Whatever the offsets hold, a position of the tile between the first and the last offset
+// finds a word, that of the tile's first such position if no other. All lanes call all three in turn, with a
+// barrier between mark and word; word_at (a word a position) and notes are LDS, free again after the next barrier.
+template <int ITEMS, int LANES>
+struct TileWords {
+  static constexpr int kTile = LANES * ITEMS, kWaves = LANES / kWave;
+  // A tile of more bags, nearly all of them empty, has its positions search for theirs: a batch may end in a
+  // million empty bags, which the lanes of one workgroup would walk for milliseconds.
+  static constexpr int64_t kWalked = 16 * LANES;
+  const NotedBags& in;
+  int64_t base, b, b0, b1;
+  long long lo, hi, begin, end;
+  int at[ITEMS];
+
+  // (requests the first bags' ends; what the caller can request without waiting comes before it)
+  __device__ __forceinline__ TileWords(const NotedBags& bags, const uint32_t* __restrict__ starts, int64_t tile,
+                                       int64_t n)
+      : in(bags), base(tile * kTile), begin(0), end(0) {
+    b0 = starts[tile];
+    b1 = starts[tile + 1];
+    b1 = b1 < b0 ? b0 : b1;                            // (offsets that descend)
+    b = b0 + threadIdx.x;
+    if (b <= b1) {
+      begin = in.offsets[b];
+      end = in.offsets[b + 1];
+    }
+    const int64_t end_of_tile = base + kTile < n ? base + kTile : n;
+    const long long first = in.offsets[0], past = in.offsets[in.bags];
+    lo = first > base ? first : base;
+    hi = past < end_of_tile ? past : end_of_tile;
+  }
+
+  __device__ __forceinline__ void mark(uint32_t* word_at, int* notes) {
+    const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) word_at[i * LANES + t] = kNoBag;
+    __syncthreads();
+    if (lo < hi && b1 - b0 > kWalked) {
+      for (long long p = lo + t; p < hi; p += LANES) {
+        int64_t in_bag = b0, behind = b1 + 1;          // offsets[in_bag] <= p < offsets[behind]
+        while (behind - in_bag > 1) {
+          const int64_t middle = (in_bag + behind) / 2;
+          if (in.offsets[middle] <= p) in_bag = middle; else behind = middle;
+        }
+        word_at[p - base] = in.words.pack((uint32_t)in_bag, in.offsets[in_bag + 1] - in.offsets[in_bag]);
+      }
+    } else if (lo < hi) {
+      while (b <= b1) {
+        const long long p = (b == b0 ? lo : begin) - base;
+        if (b == b0 || (end > begin && p > lo - base && p < hi - base)) word_at[p] = in.words.pack((uint32_t)b, end - begin);
+        b += LANES;
+        if (b <= b1) {
+          begin = in.offsets[b];
+          end = in.offsets[b + 1];
+        }
+      }
+    }
+    __syncthreads();
+    int nearest = -1;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      const int from = wave * (kWave * ITEMS) + i * kWave;
+      const unsigned long long marked = __ballot(word_at[from + lane] != kNoBag);
+      const unsigned long long here = marked & (~0ull >> (kWave - 1 - lane));
+      at[i] = here ? from + kWave - 1 - __clzll((long long)here) : nearest;
+      if (marked) nearest = from + kWave - 1 - __clzll((long long)marked);
+    }
+    if (lane == 0) notes[wave] = nearest;
+  }
+
+  __device__ __forceinline__ void word(const uint32_t* word_at, const int* notes, uint32_t (&out)[ITEMS]) const {
+    const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
+    int earlier = -1;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const int m = notes[w];
+      if (w < wave && m >= 0) earlier = m;
+    }
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      const int64_t j = base + wave * (kWave * ITEMS) + i * kWave + lane;
+      const int from = at[i] >= 0 ? at[i] : earlier;
+      out[i] = j >= lo && j < hi && from >= 0 ? word_at[from] : kNoBag;
+    }
+  }
+};
+
+struct NotedInput {
+  NotedBags bags;
+  TableView tv;
+  uint32_t miss_key;
+  uint32_t* starts;              // the bags in which tiles begin
+};
+__device__ __forceinline__ uint32_t noted_key(const NotedInput& in, uint32_t row, int64_t j) {
+  return krk::noted_key(in.tv, row, in.bags.ids + j, 0u, in.miss_key);
+}
+
+struct NoWords {                 // pairs that are there
+  __device__ __forceinline__ NoWords(const NotedBags&, const uint32_t*, int64_t, int64_t) {}
+};
+
 // The lanes that hold the digit of the wavefront's first lane are counted with one LDS add, the others
 // with one each: a digit that many keys share (the hottest row of a skewed request) is likely
 // that one, and adds to one counter are served one after the other. Finding all equal digits by
@@ -43,9 +186,11 @@ constexpr int kRsDigits = 1 << kRsMaxBits;
 // with twelve in three loads, and counts that leave through one XCD's L2, take 10.9.
 constexpr int kHistLanes = 256;
 typedef uint32_t keys4_t __attribute__((ext_vector_type(4), aligned(4)));
+
+template <bool BAGS>
 __global__ __launch_bounds__(kHistLanes) void radix_hist_kernel(const uint32_t* __restrict__ keys, int64_t n,
                                                               int shift, int bits, int64_t pitch,
-                                                              uint32_t* __restrict__ hist) {
+                                                              uint32_t* __restrict__ hist, NotedInput in) {
   constexpr int kPer = kRsTile / kHistLanes;
   static_assert(kPer % 4 == 0, "four keys a load");
   __shared__ uint32_t count[kRsDigits];
@@ -71,6 +216,19 @@ __global__ __launch_bounds__(kHistLanes) void radix_hist_kernel(const uint32_t* 
     }
   }
   for (int d = t; d <= (int)mask; d += kHistLanes) count[d] = 0u;
+  if constexpr (BAGS) {
+    const long long first = in.bags.offsets[0], past = in.bags.offsets[in.bags.bags];
+    bool plain = whole && base >= first && base + kRsTile <= past;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) plain = plain && key[i] != kEmptyRow;
+    if (!plain) {
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+        const int64_t j = whole ? base + (int64_t)(i / 4 * kHistLanes + t) * 4 + i % 4 : base + i * kHistLanes + t;
+        if (j < n) key[i] = j >= first && j < past ? noted_key(in, key[i], j) : in.miss_key;
+      }
+    }
+  }
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < kPer; ++i) {
@@ -103,7 +261,13 @@ __global__ __launch_bounds__(kHistLanes) void radix_hist_kernel(const uint32_t* 
 constexpr int kScanLanes = 256;
 constexpr int kScanPer = 8;
 __global__ __launch_bounds__(kScanLanes) void radix_scan_kernel(uint32_t* __restrict__ hist, int64_t pitch,
-                                                                uint32_t* __restrict__ total) {
+                                                                uint32_t* __restrict__ total, int digits, int64_t tiles,
+                                                                NotedBags bags, uint32_t* __restrict__ starts) {
+  if (blockIdx.x >= (uint32_t)digits) {
+    find_tile_starts(bags, (int64_t)(blockIdx.x - digits) * (kScanLanes / kWave) + threadIdx.x / kWave, tiles, kRsTile,
+                     starts);
+    return;
+  }
   __shared__ uint32_t wave_total[kScanLanes / kWave];
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
@@ -146,14 +310,14 @@ __global__ __launch_bounds__(kScanLanes) void radix_scan_kernel(uint32_t* __rest
   if (threadIdx.x == 0) total[blockIdx.x] = carry;
 }
 
-template <int BITS>
+template <int BITS, bool BAGS>
 __global__ __launch_bounds__(kRsBlock, BITS == 9 ? 6 : 8) void radix_scatter_kernel(const uint32_t* __restrict__ keys,
                                                                  const uint32_t* __restrict__ vals, int64_t n,
                                                                  int shift, int64_t pitch,
                                                                  const uint32_t* __restrict__ hist,
                                                                  const uint32_t* __restrict__ total,
                                                                  uint32_t* __restrict__ keys_out,
-                                                                 uint32_t* __restrict__ vals_out) {
+                                                                 uint32_t* __restrict__ vals_out, NotedInput in) {
   constexpr int kDigits = 1 << BITS;
   constexpr uint32_t kMask = kDigits - 1;
   __shared__ uint32_t gbase[kDigits];                  // where this tile's keys of the digit go in the output
@@ -174,8 +338,15 @@ __global__ __launch_bounds__(kRsBlock, BITS == 9 ? 6 : 8) void radix_scatter_ker
   for (int i = 0; i < kRsItems; ++i) {
     const int64_t j = base + i * kWave;
     key[i] = j < n ? keys[j] : 0xFFFFFFFFu;
-    val[i] = j < n ? vals[j] : 0u;
+    val[i] = !BAGS && j < n ? vals[j] : 0u;
   }
+  uint32_t all = 0, earlier = 0;
+  if (t < kDigits) {
+    all = total[t];
+    earlier = hist[(int64_t)t * pitch + tile];
+  }
+  std::conditional_t<BAGS, TileWords<kRsItems, kRsBlock>, NoWords> words(in.bags, in.starts, tile, n);
+  __shared__ int notes[kRsWaves];
   for (int i = t; i < kRsWaves * kDigits / 2; i += kRsBlock) reinterpret_cast<uint32_t*>(wave_hist)[i] = 0u;
   // an exclusive scan over the workgroup's first kDigits lanes (one value each), through wave_total
   auto scan_digits = [&](uint32_t v) -> uint32_t {
@@ -188,13 +359,22 @@ __global__ __launch_bounds__(kRsBlock, BITS == 9 ? 6 : 8) void radix_scatter_ker
   };
   // where each digit's output begins (scan of the totals), plus what earlier tiles hold of it
   {
-    uint32_t all = 0, earlier = 0;
-    if (t < kDigits) {
-      all = total[t];
-      earlier = hist[(int64_t)t * pitch + tile];
-    }
+    if constexpr (BAGS) words.mark(skey, notes);
     const uint32_t offset = scan_digits(all);            // its barrier: wave_hist is clear, too
     if (t < kDigits) gbase[t] = offset + earlier;
+  }
+  if constexpr (BAGS) {
+    words.word(skey, notes, val);
+#pragma unroll
+    for (int i = 0; i < kRsItems; ++i) {
+      const int64_t j = base + i * kWave;
+      if (j >= n) continue;
+      key[i] = val[i] != kNoBag ? noted_key(in, key[i], j) : in.miss_key;
+      if (in.bags.bag_of) {
+        in.bags.bag_of[j] = val[i];
+        val[i] = (uint32_t)j;
+      }
+    }
   }
 #pragma unroll
   for (int i = 0; i < kRsItems; ++i) {
@@ -255,9 +435,13 @@ __global__ __launch_bounds__(kRsBlock, BITS == 9 ? 6 : 8) void radix_scatter_ker
 template <int BITS>
 void launch_scatter(const uint32_t* keys, const uint32_t* vals, int64_t n, int shift, int64_t tiles, int64_t pitch,
                     const uint32_t* hist, const uint32_t* total, uint32_t* keys_out, uint32_t* vals_out,
-                    hipStream_t stream) {
-  hipLaunchKernelGGL((radix_scatter_kernel<BITS>), dim3((unsigned)tiles), dim3(kRsBlock), 0, stream, keys, vals, n,
-                     shift, pitch, hist, total, keys_out, vals_out);
+                    hipStream_t stream, const NotedInput* in) {
+  if (in)
+    hipLaunchKernelGGL((radix_scatter_kernel<BITS, true>), dim3((unsigned)tiles), dim3(kRsBlock), 0, stream, keys, vals,
+                       n, shift, pitch, hist, total, keys_out, vals_out, *in);
+  else
+    hipLaunchKernelGGL((radix_scatter_kernel<BITS, false>), dim3((unsigned)tiles), dim3(kRsBlock), 0, stream, keys, vals,
+                       n, shift, pitch, hist, total, keys_out, vals_out, NotedInput{});
 }
 
 // counts between two digits' rows of the histogram
@@ -267,12 +451,13 @@ int64_t hist_pitch(int64_t tiles) { return (tiles + kScanPer - 1) / kScanPer * k
 
 size_t radix_sort_work_bytes(int64_t n) {
   const int64_t tiles = (n + kRsTile - 1) / kRsTile;
-  return (size_t)(hist_pitch(tiles) + 1) * kRsDigits * sizeof(uint32_t);
+  // the tiles' counts, the digits' totals, and the bags in which tiles begin
+  return ((size_t)(hist_pitch(tiles) + 1) * kRsDigits + (size_t)tiles + 1) * sizeof(uint32_t);
 }
 
-int32_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt, int64_t n,
-                         int bits, void* work, hipStream_t stream, uint32_t** keys_sorted,
-                         uint32_t** vals_sorted) {
+static int32_t sort_pairs(const NotedInput* in, uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt,
+                          int64_t n, int bits, void* work, hipStream_t stream, uint32_t** keys_sorted,
+                          uint32_t** vals_sorted) {
   if (bits < 1) bits = 1;
   if (bits > 32) bits = 32;
   const int64_t tiles = (n + kRsTile - 1) / kRsTile;
@@ -293,19 +478,28 @@ int32_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uin
     const int shift = pass * width;
     const int w = bits - shift < width ? bits - shift : width;
     const int digits = 1 << w;
-    hipLaunchKernelGGL(radix_hist_kernel, dim3((unsigned)tiles), dim3(kHistLanes), 0, stream, src_k, n, shift, w,
-                       pitch, hist);
-    hipLaunchKernelGGL(radix_scan_kernel, dim3((unsigned)digits), dim3(kScanLanes), 0, stream, hist, pitch, total);
+    const NotedInput* from = pass == 0 ? in : nullptr;
+    const uint32_t* read_k = from ? from->bags.rows : src_k;
+    if (from)
+      hipLaunchKernelGGL(radix_hist_kernel<true>, dim3((unsigned)tiles), dim3(kHistLanes), 0, stream, read_k, n, shift, w,
+                         pitch, hist, *from);
+    else
+      hipLaunchKernelGGL(radix_hist_kernel<false>, dim3((unsigned)tiles), dim3(kHistLanes), 0, stream, read_k, n, shift,
+                         w, pitch, hist, NotedInput{});
+    // (one wavefront for each tile's first bag, and one more)
+    const int64_t finders = from ? (tiles + 1 + kScanLanes / kWave - 1) / (kScanLanes / kWave) : 0;
+    hipLaunchKernelGGL(radix_scan_kernel, dim3((unsigned)(digits + finders)), dim3(kScanLanes), 0, stream, hist, pitch,
+                       total, digits, tiles, from ? from->bags : NotedBags{}, from ? from->starts : nullptr);
     switch (w) {
-      case 1: launch_scatter<1>(src_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream); break;
-      case 2: launch_scatter<2>(src_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream); break;
-      case 3: launch_scatter<3>(src_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream); break;
-      case 4: launch_scatter<4>(src_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream); break;
-      case 5: launch_scatter<5>(src_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream); break;
-      case 6: launch_scatter<6>(src_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream); break;
-      case 7: launch_scatter<7>(src_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream); break;
-      case 8: launch_scatter<8>(src_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream); break;
-      default: launch_scatter<9>(src_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream); break;
+      case 1: launch_scatter<1>(read_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream, from); break;
+      case 2: launch_scatter<2>(read_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream, from); break;
+      case 3: launch_scatter<3>(read_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream, from); break;
+      case 4: launch_scatter<4>(read_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream, from); break;
+      case 5: launch_scatter<5>(read_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream, from); break;
+      case 6: launch_scatter<6>(read_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream, from); break;
+      case 7: launch_scatter<7>(read_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream, from); break;
+      case 8: launch_scatter<8>(read_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream, from); break;
+      default: launch_scatter<9>(read_k, src_v, n, shift, tiles, pitch, hist, total, dst_k, dst_v, stream, from); break;
     }
     KRK_HIP(hipGetLastError());
     uint32_t* tk = src_k;
@@ -318,6 +512,21 @@ int32_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uin
   *keys_sorted = src_k;
   *vals_sorted = src_v;
   return KRK_SUCCESS;
+}
+
+int32_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt, int64_t n,
+                         int bits, void* work, hipStream_t stream, uint32_t** keys_sorted,
+                         uint32_t** vals_sorted) {
+  return sort_pairs(nullptr, keys, vals, keys_alt, vals_alt, n, bits, work, stream, keys_sorted, vals_sorted);
+}
+
+int32_t radix_sort_noted_bags(const NotedBags& bags, const TableView& tv, uint32_t miss_key, uint32_t* keys,
+                              uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt, int64_t n, int bits, void* work,
+                              hipStream_t stream, uint32_t** keys_sorted, uint32_t** vals_sorted) {
+  const int64_t tiles = (n + kRsTile - 1) / kRsTile;
+  uint32_t* starts = reinterpret_cast<uint32_t*>(work) + (hist_pitch(tiles) + 1) * kRsDigits;
+  const NotedInput in{bags, tv, miss_key, starts};
+  return sort_pairs(&in, keys, vals, keys_alt, vals_alt, n, bits, work, stream, keys_sorted, vals_sorted);
 }
 
 }  // namespace krk

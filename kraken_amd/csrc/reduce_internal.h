@@ -288,6 +288,22 @@ __device__ __forceinline__ uint32_t noted_key(const TableView& tv, uint32_t row,
   return member_key | row;
 }
 
+// The positions of a single table's pooled push whose rows the pull noted, in place of keys and payloads.
+struct NotedBags {
+  const uint32_t* rows;
+  const uint64_t* ids;
+  const long long* offsets;      // null: the pairs come from somewhere else
+  int64_t bags;
+  BagWord words;
+  uint32_t* bag_of;              // null: a payload is a bag's word. Otherwise it is the position, and the word goes here
+};
+
+// radix_sort_pairs (krk_internal.h) of the pairs that these positions are; its first pass puts them together
+// (radix_sort.hip). The first two arrays may be written as the others are.
+int32_t radix_sort_noted_bags(const NotedBags& bags, const TableView& tv, uint32_t miss_key, uint32_t* keys,
+                              uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt, int64_t n, int bits, void* work,
+                              hipStream_t stream, uint32_t** keys_sorted, uint32_t** vals_sorted);
+
 // ---- partition.hip -----------------------------------------------------------------------------
 // Which workgroup of the reduction takes what: the pairs of a bucket lie side by side, and a bucket
 // of more than `whole` pairs is cut into chunks of `chunk`.

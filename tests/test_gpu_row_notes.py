@@ -352,3 +352,99 @@ def test_long_pushes_with_notes_equal_those_without(api, n):
     _same_tables(api, a, b, [api.StateType.kStateSum])
     a.close()
     b.close()
+
+
+TILE = 3072   # positions a workgroup of the sort takes
+
+
+def _bags(kind, n, rng):
+    if kind == "plain":
+        return np.concatenate([[0], np.sort(rng.integers(0, n + 1, n // 9)), [n]])
+    if kind == "tiles":                                # bags that begin and end where tiles do, a long one, and single ids
+        return np.concatenate([[0], np.arange(1, 200), np.arange(TILE, 9 * TILE, TILE) - 1, np.arange(40, 50) * TILE, [n - 1, n]])
+    if kind == "outside":                              # positions before the first bag and behind the last
+        return np.concatenate([[TILE + 5], np.sort(rng.integers(TILE + 5, n - 2 * TILE, n // 20)), [n - 2 * TILE - 7]])
+    if kind == "one":
+        return np.array([0, n])
+    if kind == "none":                                 # no position in any bag
+        return np.array([77, 77, 77])
+    # many empty bags side by side, in the middle and at the end
+    return np.concatenate([[0, 5], np.full(20_000, 2 * TILE + 100), np.sort(rng.integers(2 * TILE + 100, n + 1, 5000)), np.full(300_000, n)])
+
+
+@pytest.mark.parametrize("n", [1 + (1 << 20), 342 * TILE, 342 * TILE + 1])
+@pytest.mark.parametrize("kind", ["plain", "tiles", "outside", "one", "none", "empties"])
+@pytest.mark.parametrize("mode,weighted", [("sum", False), ("mean", False), ("sum", True)])
+def test_sorted_pooled_pushes_with_notes_equal_those_without(api, n, kind, mode, weighted):
+    """Pooled pushes of more than 2^20 positions: with notes the sort takes its pairs from them and from the
+    offsets. New ids (notes that were taken too early among them) and resident ones. Gradients, weights and
+    lengths where a mean is taken are powers of two, or one bag's: sums do not depend on the order of equal rows."""
+    dim = 4
+    rng = np.random.default_rng(n + len(kind))
+    off = _bags(kind, n, rng).astype(np.int64)
+    if mode == "mean":
+        off = off[0] + (off - off[0]) // 4 * 4 if kind != "one" else off
+        lengths = np.diff(off)
+        grads = (rng.integers(-8, 9, size=(off.size - 1, dim)) / 16.0 * np.maximum(lengths, 1)[:, None]).astype(np.float32)
+        grads = np.where(lengths[:, None] < 4096, grads, 0).astype(np.float32)
+    else:
+        grads = (rng.integers(-8, 9, size=(off.size - 1, dim)) / 16.0).astype(np.float32)
+    d_off, d_g = api.DeviceArray.from_host(off), api.DeviceArray.from_host(grads)
+    d_w = api.DeviceArray.from_host(2.0 ** rng.integers(-1, 2, n).astype(np.float32)) if weighted else None
+    o = api.Optim.create(api.OptimType.kSGD)
+    a, b = api.SparseTable(dim, _init(api)), api.SparseTable(dim, _init(api))
+    lib, C = api.lib(), api.C
+    p = lambda x: C.c_void_p(x.ptr) if x is not None else None
+    outs = [api.DeviceArray((off.size - 1, dim), np.float32) for _ in range(2)]
+    pool = {"sum": 0, "mean": 1}[mode]
+    for step in range(2):
+        d_ids = api.DeviceArray.from_host(zipf_ids(rng, 1.1, 300_000, n) + np.uint64(step * 20000))
+        for t, out, note, pulled in ((a, outs[0], api.NOTE_ROWS, api.IDS_AS_PULLED), (b, outs[1], 0, 0)):
+            assert lib.krk_sparse_pull_pooled(t.h, p(d_ids), n, p(d_off), off.size - 1, p(d_w), pool, 0.0, p(out),
+                                              api.DEVICE_PTRS | note) == 0
+            assert lib.krk_sparse_push_pooled(t.h, C.byref(o.raw), p(d_ids), n, p(d_off), off.size - 1, p(d_w), pool,
+                                              p(d_g), dim, 0.5, api.DEVICE_PTRS | pulled) == 0
+    ea, eb = a.export(), b.export()
+    oa, ob = np.argsort(ea[0]), np.argsort(eb[0])
+    assert np.array_equal(ea[0][oa], eb[0][ob])
+    if mode == "sum":
+        assert np.array_equal(ea[1][oa], eb[1][ob])
+    else:
+        # a ratio is rounded once and a run's sum once an addend, in whatever order (of runs, which rows' numbers
+        # decide): 4000 addends of one row below 2^4 in magnitude, each off by 2^-24 of the sum so far
+        np.testing.assert_allclose(ea[1][oa], eb[1][ob], rtol=1e-5, atol=1e-3)
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+def test_sorted_pooled_push_of_offsets_that_descend(api, weighted):
+    """As test_offsets_that_descend_stay_inside_the_request, for a push that is sorted: a position between
+    the first and the last offset takes part, the others do not."""
+    C, dim, n = api.C, 4, (1 << 20) + 500
+    t = api.SparseTable(dim, api.Initializer.create(api.InitializerType.kConstant, {"value": "1"}))
+    sgd = api.Optim.create(api.OptimType.kSGD)
+    ids = np.arange(1, n + 1, dtype=np.uint64)
+    d_ids = api.DeviceArray.from_host(ids)
+    d_w = api.DeviceArray.from_host(np.full(n, 0.5, np.float32)) if weighted else None
+    p = lambda x: C.c_void_p(x.ptr) if x is not None else None
+    for off in ([5, 2, 8, 8, 20, 11, n - 10], [n - 10, 30, 5], [0, n + 7, -3, n], [-(1 << 40), 7, 1 << 40], [n + 100, 3, 9, n + 200],
+                [0] + [900_000, 100] * 20_000 + [n]):
+        off = np.array(off, np.int64)
+        d_off = api.DeviceArray.from_host(off)
+        d_g = api.DeviceArray.from_host(np.ones((off.size - 1, dim), np.float32))
+        out = api.DeviceArray((off.size - 1, dim), np.float32)
+        assert t.Pull(d_ids)[0] == 0                   # (the pooled pull need not see every position)
+        before = t.Pull(ids)[1]
+        if off.size < 100:
+            assert api.lib().krk_sparse_pull_pooled(t.h, p(d_ids), n, p(d_off), off.size - 1, p(d_w), 0, 0.0, p(out),
+                                                    api.DEVICE_PTRS | api.NOTE_ROWS) == 0
+        else:                                          # (twenty thousand bags of most positions would take long to add up)
+            assert t.Pull(d_ids, note_rows=True)[0] == 0
+        assert api.lib().krk_sparse_push_pooled(t.h, C.byref(sgd.raw), p(d_ids), n, p(d_off), off.size - 1, p(d_w), 0, p(d_g),
+                                                dim, 0.5, api.DEVICE_PTRS | api.IDS_AS_PULLED) == 0
+        at = np.arange(n)
+        moved = (at >= off[0]) & (at < off[-1])
+        want = before - np.float32(0.25 if weighted else 0.5) * moved[:, None].astype(np.float32)
+        assert np.array_equal(t.Pull(ids)[1], want), off[:3]
+    t.close()
