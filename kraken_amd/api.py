@@ -214,11 +214,17 @@ def _check(rc, what):
 
 
 def _ptr(a):
+    """An array's address as an argument of the library's functions (all of which declare c_void_p): of a
+    numpy array something that keeps the array alive as well. A call passes two to eight of them, and
+    numpy's own way to the address costs it 2 to 3 us each; a writable C-contiguous array says it as a buffer."""
     if a is None:
         return None
     if isinstance(a, DeviceArray):
-        return C.c_void_p(a.ptr)
-    return a.ctypes.data_as(C.c_void_p)
+        return a.ptr
+    try:
+        return C.byref(C.c_char.from_buffer(a))
+    except (TypeError, ValueError, BufferError):     # read-only, strided or empty
+        return a.ctypes.data_as(C.c_void_p)
 
 
 class DeviceArray:
@@ -338,12 +344,17 @@ class Initializer:
 
 
 def _flags(*arrays, extra=0):
-    dev = [isinstance(a, DeviceArray) for a in arrays if a is not None]
-    if dev and all(dev):
-        return DEVICE_PTRS | extra
-    if any(dev):
+    dev = host = False
+    for a in arrays:
+        if isinstance(a, DeviceArray):
+            dev = True
+        elif a is not None:
+            host = True
+    if not dev:
+        return extra
+    if host:
         raise ValueError("mix of host and device arrays in one call")
-    return extra
+    return DEVICE_PTRS | extra
 
 
 def _take_handle(obj):

@@ -101,3 +101,39 @@ def test_no_gpu_fails_loudly(api):
         api.DenseBag(1024)
     with pytest.raises(api.KrakenHipError):
         api.dedup(np.arange(4, dtype=np.uint64))
+
+
+@pytest.mark.parametrize("form", ["plain", "view", "read_only", "strided", "fortran", "empty", "records", "dates", "scalar"])
+def test_an_array_argument_is_its_address(api, form):
+    """Whichever way api._ptr gets at an array's address: it is numpy's, and the argument keeps the array."""
+    import gc
+    import weakref
+    make = {"plain": lambda: np.arange(12, dtype=np.uint64), "view": lambda: np.zeros((5, 6), np.float32)[2:],
+            "read_only": lambda: np.frombuffer(b"abcdefgh", np.uint8), "strided": lambda: np.zeros((4, 6), np.float32)[:, 1::2],
+            "fortran": lambda: np.zeros((4, 6), np.float32, order="F"), "empty": lambda: np.zeros((0, 4), np.float32),
+            "records": lambda: np.zeros(3, [("rank", "<u8"), ("dim", "u1")]), "dates": lambda: np.zeros(3, "datetime64[s]"),
+            "scalar": lambda: np.zeros((), np.float32)}[form]
+    a = make()
+    arg = api._ptr(a)
+    assert form == "empty" or C.cast(arg, C.c_void_p).value == a.ctypes.data
+    alive = weakref.ref(a)
+    del a
+    gc.collect()
+    assert alive() is not None
+    del arg
+    gc.collect()
+    assert alive() is None
+    assert api._ptr(None) is None
+
+
+def test_arrays_of_two_kinds_in_one_call(api):
+    """Device arrays in a call say so in its flags, and are not mixed with host arrays."""
+    dev = api.DeviceArray.__new__(api.DeviceArray)
+    dev.ptr = None
+    host = np.zeros(3, np.float32)
+    assert api._flags() == 0 and api._flags(None, extra=api.ASYNC) == api.ASYNC
+    assert api._flags(host, None) == 0
+    assert api._flags(dev, None, dev, extra=api.ASYNC) == api.DEVICE_PTRS | api.ASYNC
+    for arrays in ((dev, host), (host, dev), (None, host, dev)):
+        with pytest.raises(ValueError):
+            api._flags(*arrays)
