@@ -764,8 +764,12 @@ __global__ __launch_bounds__(kCodecBlock) void coo_add_kernel(const long long* _
 // From an entry in this many elements on an entry's place is kept as a bit: 1/64 of the indices' bytes at an entry an
 // element, an eighth at one in eight, and who walks the tiles reads that. 67 million elements, an entry in 1 / 2 / 4 / 8 / 12 of them,
 // blocking, us, by the indices and by bits: Adam push 560 / 452 / 382 / 356 / 343 and 468 / 404 / 369 / 355 / 349,
-// decode 276 / 163 / 114 / 91 / 82 and 192 / 121 / 91 / 77 / 71.
+// decode 276 / 163 / 114 / 91 / 82 and 192 / 121 / 91 / 77 / 71. In small tensors the indices lie in the caches when
+// they are read again, and the bits' launch is the longer one: an Adam push of 20,000 / 300,000 / 2 million / 4 million elements, an entry in
+// four, 18.1 / 17.3 / 23.7 / 34.0 us by bits and 15.1 / 15.2 / 21.7 / 34.5 by the indices; four in five 17.9 / 16.9 / 24.7 / 36.7
+// and 15.4 / 15.5 / 24.6 / 39.9.
 constexpr int64_t kCooBitsFrom = 8;
+constexpr int64_t kCooBitsLarge = (int64_t)3 << 20;
 
 static unsigned stream_grid(int64_t n) {
   int64_t blocks = (n + kCodecBlock - 1) / kCodecBlock;
@@ -777,26 +781,25 @@ static unsigned stream_grid(int64_t n) {
 int32_t coo_find_tiles(CooWork* work, const long long* d_idx, int64_t nnz, int64_t n, CooTiles* out,
                        hipStream_t stream) {
   const int64_t tiles = (n + kCooTile - 1) / kCooTile;
-  const size_t before = work->buffer.bytes;
-  KRK_TRY(work->buffer.reserve((size_t)(tiles + 2) * sizeof(uint32_t)));
-  out->unordered = work->buffer.as<uint32_t>();
-  out->starts = out->unordered + 1;
+  uint32_t* room = work->lent;
+  bool fresh = work->calls == 0 || work->calls == 0xFFFFFFFFu;   // a fresh buffer holds no tag, and 0 is none
+  if (!room) {
+    const size_t before = work->buffer.bytes;
+    KRK_TRY(work->buffer.reserve(coo_tile_words(n) * sizeof(uint32_t)));
+    room = work->buffer.as<uint32_t>();
+    fresh = fresh || work->buffer.bytes != before;
+  }
+  out->unordered = room;
+  out->starts = room + 1;
   out->tiles = (uint32_t)tiles;
-  bool with_bits = nnz * kCooBitsFrom >= n;
+  bool with_bits = n >= kCooBitsLarge && nnz * kCooBitsFrom >= n;
   if (with_bits && work->bits.reserve((size_t)tiles * (kCooTile / 8)) != KRK_SUCCESS) {
     (void)hipGetLastError();                         // no failure of a later launch
     with_bits = false;                               // the indices are read again, then
   }
   out->bits = with_bits ? work->bits.as<uint32_t>() : nullptr;
-  if (!work->host_unordered) {
-    KRK_HIP(hipHostMalloc((void**)&work->host_unordered, 64, hipHostMallocCoherent));
-    *work->host_unordered = 0u;
-  }
-  KRK_HIP(hipHostGetDevicePointer((void**)&out->host_unordered, work->host_unordered, 0));
-  // a fresh buffer holds no tag, and one that says 0 is never handed out
-  if (work->buffer.bytes != before || work->calls == 0xFFFFFFFFu) {
+  if (fresh) {
     KRK_HIP(hipMemsetAsync(out->unordered, 0, sizeof(uint32_t), stream));
-    *work->host_unordered = 0u;
     work->calls = 0;
   }
   out->tag = ++work->calls;

@@ -120,12 +120,14 @@ struct StreamWait {
   ~StreamWait() { close(); }
   static void prepare();   // the memory of the words, with the runtime
   bool open();    // takes a free word; false where there is none: the call then synchronises with the stream
+  uint32_t* told() const { return word + 1; }
   void close();   // gives it back
 };
 // Waits until the word of an open wait holds its number, and closes it. A stream that takes longer than five
 // milliseconds, has failed or is being captured is left to hipStreamSynchronize. The core is busy meanwhile, as it is in
-// hipStreamSynchronize; after 50 us other threads may have it between two looks.
-int32_t wait_for(StreamWait* w, hipStream_t stream);
+// hipStreamSynchronize; after 50 us other threads may have it between two looks. told: what lies behind the word
+// in its cache line (StreamWait::told), as the launch that wrote the word left it.
+int32_t wait_for(StreamWait* w, hipStream_t stream, uint32_t* told = nullptr);
 // The same for a stream whose last launch writes no word: puts a launch behind it that does.
 int32_t wait_stream(hipStream_t stream);
 // Called by the one wavefront of that launch.
@@ -546,27 +548,27 @@ __device__ __forceinline__ void optim_element(const OptimK& k, float lr, float g
 // in LDS, or, where there are many entries, from a bit an element that the first launch leaves. Any other input is zeroed and scattered into; which of the two it is is decided on the
 // device, and the launches of the other way look at the flag and leave.
 constexpr int kCooTile = 2048;                   // floats of one tile: 8 KB of LDS
-constexpr int64_t kCooTiledFrom = 1 << 22;       // smaller tensors: zero + scatter, two launches are quicker
+// Smaller tensors: zero + scatter, two launches are quicker than two and those of the other way, unless the call
+// waits and learns which of the ways it was (dense_apply_coo).
+constexpr int64_t kCooTiledFrom = 1 << 22;
 struct CooTiles {
   uint32_t* starts;       // [tiles + 1]: tile t owns entries [starts[t], starts[t + 1])
   uint32_t* unordered;    // == tag: the indices do not ascend strictly or leave [0, n)
   uint32_t tag;
   uint32_t tiles;
-  uint32_t* host_unordered;   // page-locked copy of the flag, raised by who walks the tiles
   uint32_t* bits;         // null, or a bit an element, 64 words a tile: whether an entry names it
 };
 __device__ __forceinline__ bool coo_unordered(const CooTiles& t) { return *t.unordered == t.tag; }
 struct CooWork {          // work space of one caller, kept between calls
   DeviceBuffer buffer, bits;
+  uint32_t* lent = nullptr;   // room for coo_tile_words of the caller's tensor behind something else of the caller's
   uint32_t calls = 0;
-  uint32_t* host_unordered = nullptr;
   void release() {
     buffer.release();
     bits.release();
-    if (host_unordered) (void)hipHostFree(host_unordered);
-    host_unordered = nullptr;
   }
 };
+inline size_t coo_tile_words(int64_t n) { return (size_t)((n + kCooTile - 1) / kCooTile) + 2; }
 // Which of a tile's elements have an entry, and how many entries of the tile lie before each of its 64 words: a lane
 // holds the word of its number. All lanes of a wavefront.
 struct CooTileBits {

@@ -131,7 +131,7 @@ void StreamWait::close() {
 constexpr std::chrono::microseconds kLookAlone(50);
 constexpr std::chrono::microseconds kLookAtAll(5000);
 
-int32_t wait_for(StreamWait* w, hipStream_t stream) {
+int32_t wait_for(StreamWait* w, hipStream_t stream, uint32_t* told) {
   using clock = std::chrono::steady_clock;
   const clock::time_point begun = clock::now();
   bool there = false, yield = false;
@@ -147,6 +147,7 @@ int32_t wait_for(StreamWait* w, hipStream_t stream) {
   }
   // the word is given back only once nothing is left that writes it (or the stream has failed)
   const hipError_t e = there ? hipSuccess : hipStreamSynchronize(stream);
+  if (told) *told = __atomic_load_n(w->told(), __ATOMIC_RELAXED);
   w->close();
   return e == hipSuccess ? KRK_SUCCESS : hip_fail(e, "hipStreamSynchronize", __FILE__, __LINE__);
 }

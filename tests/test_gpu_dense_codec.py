@@ -466,3 +466,51 @@ def test_dense_group_members_and_columns(api, oracle, members):
                     assert_close(t.state(st), ws if ws is not None else np.zeros(n, np.float32), "%s state %d" % (name, st))
         grp.close()
         own = members - 2 if members > 1 else 0
+
+
+@pytest.mark.parametrize("n", [1, 3, 255, 2047, 2048, 2049, 4096, 300_001, (1 << 22) - 1])
+@pytest.mark.parametrize("type_", [3, 1])
+def test_sparse_pushes_to_small_tables(api, n, type_):
+    """Blocking pushes go tile by tile whatever the table's size, and after one whose indices do not ascend by
+    fill and scatter for a while: the sequence against a table that takes every gradient dense. Host and device arrays,
+    from device memory that is not on 16 bytes too; values are dyadic, so a sum does not depend on its order."""
+    C, rng = api.C, np.random.default_rng(n)
+    w0 = (rng.integers(-64, 65, n) / 64.0).astype(np.float32)
+    t, r = api.DenseTable(w0), api.DenseTable(w0)
+    opt = api.Optim.create(type_)
+
+    def push(idx, how):
+        idx = np.asarray(idx, np.int64)
+        val = (rng.integers(-32, 33, idx.size) / 32.0).astype(np.float32)
+        inside = (idx >= 0) & (idx < n)
+        dense = np.zeros(n, np.float32)
+        np.add.at(dense, idx[inside], val[inside])
+        if how == "host":
+            assert t.PushCoo(opt, idx, val, 0.25) == 0
+        else:
+            skip = int(how == "shifted")
+            d_idx = api.DeviceArray.from_host(np.concatenate([np.zeros(skip, np.int64), idx]))
+            d_val = api.DeviceArray.from_host(val)
+            flags = api.DEVICE_PTRS | (api.ASYNC if how == "async" else 0)
+            assert api.lib().krk_dense_push_coo(t.h, C.byref(opt.raw), C.c_void_p(d_idx.ptr + 8 * skip),
+                                                C.c_void_p(d_val.ptr), idx.size, 0.25, flags) == 0
+            t.sync()
+        assert r.Push(opt, dense, 0.25) == 0
+        assert np.array_equal(t.Pull()[1], r.Pull()[1]), (idx[:4], how)
+
+    some = np.sort(rng.choice(n, max(1, n // 3), replace=False))
+    for how in ("device", "host", "shifted", "async"):
+        push(some, how)
+        push([n - 1], how)
+        push(np.arange(n) if n < 5000 else some[:77], how)
+    mixed = rng.permutation(np.concatenate([some, some[:1]]))      # an index twice
+    for idx in (mixed, np.array([-5, 0]), np.array([n, n + 1]), np.array([0, n])):
+        push(idx, "device")
+        push(some, "async")
+        for _ in range(260 if n in (3, 2049) else 2):               # past the pushes that do not look for tiles
+            push(some, "device")
+        push(idx, "host")
+        push(some, "host")
+    push(np.repeat(some, 4)[: n + 2], "device")                    # more entries than elements, where there is room
+    t.close()
+    r.close()
