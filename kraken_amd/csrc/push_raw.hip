@@ -536,6 +536,72 @@ __host__ __device__ inline size_t segreduce_lds_words(int per_block, int group, 
 constexpr int kFromCarry = 0;    // partial sums of the level before
 constexpr int kFromRows = 1;     // level 0: gradient rows
 constexpr int kFromBags = 2;     // level 0 of a pooled push: bags' gradient rows, scaled as they are read
+
+// A span that lies inside one run, which goes on in a neighbour: the sum of its entries, as segreduce_kernel adds
+// them up (a tile by a lane group, the tiles' sums in order), to carry slot `slot`; behind it zeros, if the run goes on on
+// both sides. Skewed requests are such spans for the most part (three in five of 8.5 million Zipf 1.1 ids), and what they
+// cost by the general way was neither the rows' bytes nor their lines but waiting: four rows requested at a time where
+// no record needs the registers, a look at every entry's key, and a lane group that adds 64 partial sums up, the zeros
+// among them, asking for each once it has the one before. Eight rows at a time, and 32 sums requested ahead of the
+// additions: the reduction of 8.5 million pooled ids of 32 floats under Adam 405 -> 346 us; forward, backward and
+// forward, us: that 941 -> 874, 2.4 million of 8 floats 250 -> 239, 3 million weighted of 16 320 -> 303, 1.3 million of 64
+// 291 -> 281, 1.6 million of 32 209 -> 193.
+template <int VEC, bool POOLED>
+__device__ __forceinline__ void reduce_one_run(const KRK_GLOBAL float* const* lds_src, const float* lds_r,
+                                               const float* lds_w, float* part_val, int tile, int per_block, int dim,
+                                               int elems, int group, int64_t slot, bool zeros,
+                                               float* __restrict__ vals_out) {
+  constexpr int kAtOnce = 8;
+  const int lt = threadIdx.x / group, gl = threadIdx.x & (group - 1), lane_floats = group * VEC;
+  for (int e0 = 0; e0 < elems; e0 += group) {
+    const int e = e0 + gl;
+    const bool lane_on = e < elems;
+    float acc[VEC] = {};
+    for (int j0 = 0; j0 < tile; j0 += kAtOnce) {
+      float v[kAtOnce][VEC] = {};
+#pragma unroll
+      for (int u = 0; u < kAtOnce; ++u) {
+        if (!lane_on) continue;
+        const KRK_GLOBAL float* src = lds_src[lt * tile + j0 + u] + e * VEC;
+        if constexpr (POOLED) gload<VEC>((const float*)src, v[u]); else gload_once<VEC>(src, v[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < kAtOnce; ++u) {
+        const int j = lt * tile + j0 + u;
+        if constexpr (POOLED) {
+          const float r = lds_r[j];
+#pragma unroll
+          for (int c = 0; c < VEC; ++c) v[u][c] = v[u][c] * r;
+          if (lds_w) {
+            const float w = lds_w[j];
+#pragma unroll
+            for (int c = 0; c < VEC; ++c) v[u][c] = v[u][c] * w;
+          }
+        }
+#pragma unroll
+        for (int c = 0; c < VEC; ++c) acc[c] = j0 + u == 0 ? v[u][c] : acc[c] + v[u][c];
+      }
+    }
+    vstore<VEC>(part_val + lt * lane_floats + gl * VEC, acc);
+    __syncthreads();
+    if (lt == 0) {
+#pragma unroll 8
+      for (int k = 1; k < per_block; ++k) {
+        float next[VEC];
+        vload<VEC>(part_val + k * lane_floats + gl * VEC, next);
+#pragma unroll
+        for (int c = 0; c < VEC; ++c) acc[c] = acc[c] + next[c];
+      }
+      if (lane_on) {
+        vstore<VEC>(vals_out + slot * dim + e * VEC, acc);
+        const float zero[VEC] = {};
+        if (zeros) vstore<VEC>(vals_out + (slot + 1) * dim + e * VEC, zero);
+      }
+    }
+    if (e0 + group < elems) __syncthreads();               // the next chunk reuses the sums
+  }
+}
+
 template <int OPT, int VEC, int FROM, bool GROUPED>
 __global__ __launch_bounds__(kBlock) void segreduce_kernel(
     TableView tv, const uint32_t* __restrict__ keys, const uint32_t* __restrict__ pos,
@@ -599,6 +665,17 @@ __global__ __launch_bounds__(kBlock) void segreduce_kernel(
   }
   if (threadIdx.x < 2) out_key[threadIdx.x] = kNoRow;
   __syncthreads();
+
+  if constexpr (LEVEL0) {
+    const uint32_t key = lds_keys[1];
+    const bool enters = lds_keys[0] == key, leaves = lds_keys[span + 1] == key;
+    if (key < empty_from && lds_keys[span] == key && (enters || leaves)) {   // uniform
+      reduce_one_run<VEC, POOLED>(lds_src, lds_r, weighted ? lds_w : nullptr, part_val, tile, per_block, dim, elems,
+                                  group, 2 * (int64_t)blockIdx.x + (enters ? 0 : 1), enters && leaves, vals_out);
+      if (threadIdx.x < 2) keys_out[2 * (int64_t)blockIdx.x + threadIdx.x] = (threadIdx.x ? leaves : enters) ? key : kNoRow;
+      return;
+    }
+  }
 
   const int lt = threadIdx.x / group;                       // this lane group's tile in the workgroup
   const int gl = threadIdx.x & (group - 1);

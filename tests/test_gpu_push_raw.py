@@ -359,6 +359,56 @@ def test_push_raw_short_path_extremes(api, oracle, dim, shape):
         assert (np.abs((before - after) - exact) <= 4e-7 * mass + 2e-7 * np.abs(before) + 1e-30).all()
 
 
+# pairs of the rows in the order of their numbers: spans (16 pairs a lane group, 64 to 1024 of them by the row's width)
+# that one row fills exactly, enters, leaves or passes through, and spans of many rows
+RUNS_OF_SPANS = [1024, 1024, 2048, 1025, 1023, 1, 63, 960, 3000, 72, 512, 1536, 7, 250_000, 17, 90_001, 1022, 1, 1, 1]
+
+
+def _span_ids(rng, t, salt):
+    """Ids of t whose sorted pairs are runs of RUNS_OF_SPANS, short runs and one run of the rest, shuffled."""
+    ids = splitmix64(np.arange(4000, dtype=np.uint64) + np.uint64(salt))
+    t.Pull(ids)
+    ids = ids[np.argsort(t.lookup(ids))]
+    counts = np.concatenate([RUNS_OF_SPANS, rng.integers(1, 60, ids.size - len(RUNS_OF_SPANS) - 1)])
+    counts = np.append(counts, (1 << 20) + 5 - counts.sum())
+    assert counts[-1] > 100_000
+    return rng.permutation(np.repeat(ids, counts))
+
+
+@pytest.mark.parametrize("dim,source", [(4, "rows"), (5, "rows"), (32, "rows"), (100, "rows"), (8, "members"), (16, "bags"),
+                                        (16, "weighted"), (64, "bags"), (64, "weighted"), (70, "bags"), (260, "weighted")])
+def test_sorted_pushes_whose_runs_fill_spans(api, oracle, dim, source):
+    """Pushes of more than 2^20 pairs, whose reduction takes spans inside one row's run by a way of their own. Dyadic
+    gradients and weights and plain SGD: exact whatever the order of additions."""
+    rng = np.random.default_rng(dim)
+    tables = [api.SparseTable(dim, api.Initializer.create(api.InitializerType.kConstant, {"value": "1"}))
+              for _ in range(2 if source == "members" else 1)]
+    sgd = api.Optim.create(api.OptimType.kSGD)
+    parts = [_span_ids(rng, t, 10_000 * k) for k, t in enumerate(tables)]
+    ids = np.concatenate(parts)
+    if source in ("rows", "members"):
+        grads = _dyadic_grads(rng, (ids.size, dim))
+        if source == "rows":
+            assert tables[0].PushRaw(sgd, ids, grads, 0.5) == 0
+        else:
+            group = api.TableGroup(tables)
+            assert group.CombinePushRaw(sgd, ids, group._offsets([p.size for p in parts]), grads, 0.5) == 0
+            group.close()
+    else:
+        offsets = np.concatenate([[0], np.sort(rng.integers(0, ids.size, ids.size // 30)), [ids.size]]).astype(np.int64)
+        bags = _dyadic_grads(rng, (offsets.size - 1, dim))
+        weights = 2.0 ** rng.integers(-1, 2, ids.size).astype(np.float32) if source == "weighted" else None
+        assert tables[0].PushPooled(sgd, ids, offsets, bags, 0.5, weights=weights) == 0
+        grads = np.repeat(bags, np.diff(offsets), axis=0)
+        if weights is not None:
+            grads *= weights[:, None]
+    for k, t in enumerate(tables):
+        mine = slice(k * parts[0].size, k * parts[0].size + parts[k].size)
+        u, gs = oracle.dedup_sum(parts[k], grads[mine])
+        assert np.array_equal(t.Pull(u)[1], np.float32(1.0) - np.float32(0.5) * gs)
+        t.close()
+
+
 def test_dedups_leave_their_index_empty(api):
     """Calls of 8193 to 2^16 ids share an index that each of them leaves empty; shorter and longer calls, and calls that
     stage host arrays, use other memory in between. The all-ones id has a slot of its own at each size."""
