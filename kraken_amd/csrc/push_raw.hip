@@ -542,7 +542,7 @@ constexpr int kFromBags = 2;     // level 0 of a pooled push: bags' gradient row
 // both sides. Skewed requests are such spans for the most part (three in five of 8.5 million Zipf 1.1 ids), and what they
 // cost by the general way was neither the rows' bytes nor their lines but waiting: four rows requested at a time where
 // no record needs the registers, a look at every entry's key, and a lane group that adds 64 partial sums up, the zeros
-// among them, asking for each once it has the one before. Eight rows at a time, and 32 sums requested ahead of the
+// among them, asking for each once it has the one before. Eight rows at a time (sixteen: the same), and 32 sums requested ahead of the
 // additions: the reduction of 8.5 million pooled ids of 32 floats under Adam 405 -> 346 us; forward, backward and
 // forward, us: that 941 -> 874, 2.4 million of 8 floats 250 -> 239, 3 million weighted of 16 320 -> 303, 1.3 million of 64
 // 291 -> 281, 1.6 million of 32 209 -> 193.
@@ -1596,7 +1596,7 @@ static int32_t sort_and_reduce(const ReduceShape& sh, hipStream_t stream, Device
 // which a request of 50,000 ids has eight launches; where a request is many times what the chip
 // holds at once, the tiled reduction's walks use the memory better than workgroups that sort first
 // (8.5 million pooled ids of 32 floats: reduction 468 us against 574, partition and sort 180 and
-// 215; the sort has come down to 140 since).
+// 215; the reduction has come down to 346 and the sort to 140 since).
 // noted: single tables whose rows the pull noted; fill is not called then. noted_bags: the same for pooled
 // pushes that are sorted.
 template <typename Fill>
