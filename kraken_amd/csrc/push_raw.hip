@@ -539,13 +539,13 @@ constexpr int kFromBags = 2;     // level 0 of a pooled push: bags' gradient row
 
 // A span that lies inside one run, which goes on in a neighbour: the sum of its entries, as segreduce_kernel adds
 // them up (a tile by a lane group, the tiles' sums in order), to carry slot `slot`; behind it zeros, if the run goes on on
-// both sides. Skewed requests are such spans for the most part (three in five of 8.5 million Zipf 1.1 ids), and what they
-// cost by the general way was neither the rows' bytes nor their lines but waiting: four rows requested at a time where
-// no record needs the registers, a look at every entry's key, and a lane group that adds 64 partial sums up, the zeros
-// among them, asking for each once it has the one before. Eight rows at a time (sixteen: the same), and 32 sums requested ahead of the
-// additions: the reduction of 8.5 million pooled ids of 32 floats under Adam 405 -> 346 us; forward, backward and
+// both sides. Skewed requests are such spans for the most part (three in five of 8.5 million Zipf 1.1 ids), and by the
+// general way they waited rather than moved bytes: four rows requested at a time where no record needs the
+// registers, and a look at every entry's key between them. Eight rows at a time (sixteen: the same): the reduction of 8.5 million
+// pooled ids of 32 floats under Adam 405 -> 346 us, 4.7 -> 5.5 TB/s of its misses and writes; forward, backward and
 // forward, us: that 941 -> 874, 2.4 million of 8 floats 250 -> 239, 3 million weighted of 16 320 -> 303, 1.3 million of 64
-// 291 -> 281, 1.6 million of 32 209 -> 193.
+// 291 -> 281, 1.6 million of 32 209 -> 193. (Partial sums requested four or eight ahead of adding them up gain nothing
+// in the general way.)
 template <int VEC, bool POOLED>
 __device__ __forceinline__ void reduce_one_run(const KRK_GLOBAL float* const* lds_src, const float* lds_r,
                                                const float* lds_w, float* part_val, int tile, int per_block, int dim,
