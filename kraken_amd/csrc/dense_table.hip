@@ -435,10 +435,12 @@ constexpr int kCooPlainPushes = 256;
 // launches that look at a flag and leave: 13 us). So a blocking call goes tile by tile whatever the size: of
 // 300 / 20,000 / 300,000 / 2 million elements, an entry in four, Adam, 17.5 / 18.0 / 18.8 / 30.5 us by fill, scatter
 // and update, 15.1 / 17.1 / 17.2 / 23.6 in tiles. Indices that do not ascend cost it a look at them (20 to 100 us), so
-// after such a push a small table takes the fill and scatter for the next ones. *waited:
-// nothing is left to wait for.
+// after such a push a small table takes the fill and scatter for the next ones. Indices that the kernels read in host
+// memory cross PCIe twice in tiles and once in the scatter (page-locked, 300,000 / 2 million elements, an entry in four,
+// 51 / 227 us and 37 / 132; pageable 64 and 52 for 300,000), so a small table's tiles are for indices in device
+// memory, the caller's or staged there (in_device). *waited: nothing is left to wait for.
 static int32_t dense_apply_coo(krk_dense* t, const krk_optim& o, const long long* d_idx, const float* d_val,
-                               int64_t nnz, float lr, uint32_t flags, bool* waited) {
+                               int64_t nnz, bool in_device, float lr, uint32_t flags, bool* waited) {
   *waited = false;
   if (!t->coo_grad) {
     // (one allocation: a table's first sparse push pays for it)
@@ -448,7 +450,7 @@ static int32_t dense_apply_coo(krk_dense* t, const krk_optim& o, const long long
   }
   const bool small = t->n < kCooTiledFrom;
   bool tiled = coo_tiled(t->n, nnz);
-  if (small && !(flags & KRK_ASYNC) && nnz <= t->n) {   // (more entries than elements do not ascend)
+  if (small && in_device && !(flags & KRK_ASYNC) && nnz <= t->n) {   // (more entries than elements do not ascend)
     tiled = t->coo_plain == 0;
     if (!tiled) --t->coo_plain;
   }
@@ -779,7 +781,8 @@ int32_t krk_dense_push_coo(krk_dense* t, const krk_optim* o, const int64_t* idx,
   KRK_TRY(t->input(idx, (size_t)nnz, flags, 0, &d_idx));
   KRK_TRY(t->input(val, (size_t)nnz, flags, 1, &d_val));
   bool waited = false;
-  KRK_TRY(dense_apply_coo(t, *o, reinterpret_cast<const long long*>(d_idx), d_val, nnz, lr, flags, &waited));
+  const bool in_device = (flags & KRK_DEVICE_PTRS) || (const void*)d_idx == t->stage[0].ptr;
+  KRK_TRY(dense_apply_coo(t, *o, reinterpret_cast<const long long*>(d_idx), d_val, nnz, in_device, lr, flags, &waited));
   return waited ? KRK_SUCCESS : dense_finish(t, flags);
 }
 

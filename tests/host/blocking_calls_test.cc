@@ -5,12 +5,15 @@
 //     after it, whatever it waits for besides (the runtime may hold on to those pages until then);
 //   - a word that a launch under way will still write belongs to the call that waits for it until that launch has
 //     ended, so that no other call waits on the same word; where all words are taken calls synchronise;
-//   - a thread that waits lets others of its core run, on whom the end of its work may depend.
+//   - a thread that waits lets others of its core run, on whom the end of its work may depend;
+//   - a sparse gradient of a small dense table whose indices the kernels read in host memory is scattered, which
+//     reads them once.
 #ifndef __HIP_PLATFORM_AMD__
 #define __HIP_PLATFORM_AMD__
 #endif
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -43,6 +46,7 @@ struct Runtime {
   bool signals_late = false;
   int yields_until_told = 0;                        // > 0: late words are written at the last of so many sched_yields
   int synchronised = 0;
+  std::vector<std::string> launched;                // names, mangled
   uint32_t rows = 0;                                // what the tables' counters say
   std::function<void()> on_synchronise;
   dim3 grid, block;
@@ -169,6 +173,7 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shmem, hip
 }
 hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t stream) {
   const std::string& name = rt().kernels[f];
+  rt().launched.push_back(name);
   if (name.find("signal_kernel") != std::string::npos) {
     tell(stream, *static_cast<uint32_t**>(args[0]), *static_cast<uint32_t*>(args[1]));
   } else if (name.find("counters_kernel") != std::string::npos) {
@@ -367,6 +372,41 @@ static void one_core() {
   CHECK(krk_sparse_destroy(t) == 0);
 }
 
+// How many of the launches since the last look were of kernels of this name.
+static int launches(const char* name) {
+  int n = 0;
+  for (const std::string& l : rt().launched) n += l.find(name) != std::string::npos;
+  return n;
+}
+
+// Sparse gradients of tables below 2^22 elements: page-locked arrays of any size and pageable ones that pass through
+// page-locked buffers (up to 1 MB) are filled and scattered, each of many pushes.
+static void sparse_gradients_in_host_memory() {
+  krk_optim sgd;
+  CHECK(krk_optim_defaults(KRK_SGD, &sgd) == 0);
+  for (const int64_t cells : {(int64_t)300, (int64_t)300000, ((int64_t)1 << 22) - 1}) {
+    for (const bool locked : {true, false}) {
+      const int64_t nnz = locked ? cells / 2 : std::min<int64_t>(cells / 2, 1 << 17);
+      std::vector<float> vals(cells);
+      std::vector<int64_t> index(nnz);
+      for (int64_t i = 0; i < nnz; ++i) index[i] = i;
+      void *l_index = nullptr, *l_vals = nullptr;
+      CHECK(krk_host_malloc(&l_index, nnz * 8) == 0 && krk_host_malloc(&l_vals, nnz * 4) == 0);
+      std::memcpy(l_index, index.data(), nnz * 8);
+      krk_dense* d = nullptr;
+      CHECK(krk_dense_create(vals.data(), cells, 0, &d) == 0);
+      rt().launched.clear();
+      for (int push = 0; push < 3; ++push)
+        whole("push_coo", krk_dense_push_coo(d, &sgd, locked ? static_cast<int64_t*>(l_index) : index.data(),
+                                             locked ? static_cast<float*>(l_vals) : vals.data(), nnz, 0.1f, 0));
+      CHECK(launches("coo_add_kernel") == 3 && launches("dense_update_kernel") == 3);
+      CHECK(launches("coo_tiles_bounds_kernel") == 0 && launches("coo_bits_kernel") == 0);
+      CHECK(krk_dense_destroy(d) == 0);
+      CHECK(krk_host_free(l_index) == 0 && krk_host_free(l_vals) == 0);
+    }
+  }
+}
+
 int main(int argc, char** argv) {
   const std::string which = argc > 1 ? argv[1] : "";
   CHECK(krk_runtime_init(0) == 0);
@@ -381,6 +421,8 @@ int main(int argc, char** argv) {
     late_words();
   } else if (which == "core") {
     one_core();
+  } else if (which == "host_gradients") {
+    sparse_gradients_in_host_memory();
   } else {
     return 2;
   }

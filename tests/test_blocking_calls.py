@@ -26,7 +26,8 @@ def program(tmp_path_factory):
 # dense, sparse: a blocking call on pageable arrays synchronises after the copies that staged them
 # words: no two calls wait on one word, and the calls that find none synchronise
 # core: a waiting thread lets the other threads of its core run
-@pytest.mark.parametrize("which", ["dense", "sparse", "words", "core"])
+# host_gradients: sparse gradients in host memory of small dense tables are read once
+@pytest.mark.parametrize("which", ["dense", "sparse", "words", "core", "host_gradients"])
 def test_blocking_calls(program, which):
     r = subprocess.run([program, which], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr

@@ -473,7 +473,8 @@ def test_dense_group_members_and_columns(api, oracle, members):
 def test_sparse_pushes_to_small_tables(api, n, type_):
     """Blocking pushes go tile by tile whatever the table's size, and after one whose indices do not ascend by
     fill and scatter for a while: the sequence against a table that takes every gradient dense. Host and device arrays,
-    from device memory that is not on 16 bytes too; values are dyadic, so a sum does not depend on its order."""
+    page-locked ones and device memory that is not on 16 bytes too; values are dyadic, so a sum does not depend on its
+    order."""
     C, rng = api.C, np.random.default_rng(n)
     w0 = (rng.integers(-64, 65, n) / 64.0).astype(np.float32)
     t, r = api.DenseTable(w0), api.DenseTable(w0)
@@ -487,6 +488,13 @@ def test_sparse_pushes_to_small_tables(api, n, type_):
         np.add.at(dense, idx[inside], val[inside])
         if how == "host":
             assert t.PushCoo(opt, idx, val, 0.25) == 0
+        elif how == "pinned":
+            p = C.c_void_p()
+            assert api.lib().krk_host_malloc(C.byref(p), max(1, 12 * idx.size)) == 0
+            C.memmove(p, idx.ctypes.data, idx.nbytes)
+            C.memmove(p.value + idx.nbytes, val.ctypes.data, val.nbytes)
+            assert api.lib().krk_dense_push_coo(t.h, C.byref(opt.raw), p, p.value + idx.nbytes, idx.size, 0.25, 0) == 0
+            assert api.lib().krk_host_free(p) == 0
         else:
             skip = int(how == "shifted")
             d_idx = api.DeviceArray.from_host(np.concatenate([np.zeros(skip, np.int64), idx]))
@@ -499,7 +507,7 @@ def test_sparse_pushes_to_small_tables(api, n, type_):
         assert np.array_equal(t.Pull()[1], r.Pull()[1]), (idx[:4], how)
 
     some = np.sort(rng.choice(n, max(1, n // 3), replace=False))
-    for how in ("device", "host", "shifted", "async"):
+    for how in ("device", "host", "pinned", "shifted", "async"):
         push(some, how)
         push([n - 1], how)
         push(np.arange(n) if n < 5000 else some[:77], how)
@@ -511,6 +519,7 @@ def test_sparse_pushes_to_small_tables(api, n, type_):
             push(some, "device")
         push(idx, "host")
         push(some, "host")
+        push(idx, "pinned")
     push(np.repeat(some, 4)[: n + 2], "device")                    # more entries than elements, where there is room
     t.close()
     r.close()
