@@ -459,6 +459,12 @@ __device__ __forceinline__ void coo_start_tiles(uint32_t* __restrict__ starts, i
   }
 }
 
+// Says that the indices are unordered. Stores to one word are served one after the other, some 30 ns each, and where
+// the entries come in no order everyone has one: whoever finds the word written spares its own.
+__device__ __forceinline__ void coo_raise(const CooTiles& out) {
+  if (!coo_unordered(out)) __hip_atomic_store(out.unordered, out.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Where each tile's entries begin: the first entry of a tile, and the first one behind the empty
 // tiles before it, name themselves. A wavefront takes chunks of 256 entries in two rows of 128, a lane two
 // neighbours of each in one 16-byte load (whole lines an access); the entry before a lane's two is
@@ -495,26 +501,33 @@ __device__ __forceinline__ bool coo_row_starts(const coo_pair& cur, int64_t j, i
   const bool quick = j + 2 < nnz && prev >= 0 && prev < cur[0] && cur[0] < cur[1] && cur[1] < n &&
                      (prev ^ cur[1]) < kCooTile;
   if (__ballot(!quick) == 0ull) return true;
+  // A row that holds a wrong entry names no starts, which nobody will look at: where the entries come in no order,
+  // every second one would write those of hundreds of tiles (half a million shuffled entries of 2 million
+  // elements: 119 us with those, 9 without).
   bool bad = false;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const long long c = cur[i], before = i ? cur[0] : prev;
+    bad = bad || (!quick && j + i < nnz && (c < 0 || c <= before || c >= n));   // before may be negative, and wrong, itself
+  }
+  if (__ballot(bad) != 0ull) return false;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const bool mine = !quick && j + i < nnz;
     const long long c = cur[i];
-    const bool wrong = mine && (c < 0 || c <= prev || c >= n);   // prev may be negative, and wrong, itself
-    bad = bad || wrong;
     int from = 1, to = 0, tile = 0;
-    if (mine && !wrong) {
+    if (mine) {
       tile = (int)(c / kCooTile);
       from = prev < 0 ? 0 : (int)(prev / kCooTile) + 1;
       to = tile;
     }
     coo_start_tiles(out.starts, from, to, (uint32_t)(j + i));
-    const bool end = mine && !wrong && j + i == nnz - 1;
+    const bool end = mine && j + i == nnz - 1;
     if (__ballot(end) != 0ull)
       coo_start_tiles(out.starts, end ? tile + 1 : 1, end ? (int)out.tiles : 0, (uint32_t)nnz);
     prev = c;
   }
-  return __ballot(bad) == 0ull;
+  return true;
 }
 
 __global__ __launch_bounds__(kCodecBlock) void coo_tiles_bounds_kernel(const long long* __restrict__ idx,
@@ -529,7 +542,7 @@ __global__ __launch_bounds__(kCodecBlock) void coo_tiles_bounds_kernel(const lon
 #pragma unroll
     for (int r = 0; r < kCooRows; ++r)
       fine &= coo_row_starts(cur[r], base + r * 128 + (threadIdx.x & 63) * 2, nnz, n, last, out);
-    if (!fine) __hip_atomic_store(out.unordered, out.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!fine) coo_raise(out);
   }
 }
 
@@ -668,7 +681,7 @@ __global__ __launch_bounds__(kCodecBlock) void coo_bits_kernel(const long long* 
 #pragma unroll
     for (int r = 0; r < kCooRows; ++r) cur[r] = ahead[r];
   }
-  if (!fine) __hip_atomic_store(out.unordered, out.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (!fine) coo_raise(out);
 }
 
 // One workgroup per output tile: the tile is put together in LDS (zeros, then the tile's entries,
@@ -747,14 +760,20 @@ __global__ __launch_bounds__(kCodecBlock) void coo_zero_if_kernel(float* __restr
 }
 
 // dense[idx[j]] += val[j]; repeated indices add up (t/math.cc:1043), indices outside [0, n) are
-// skipped. IF: only where the tiles were found to be unordered.
-template <bool IF>
+// skipped. kAddIf: only where the tiles were found to be unordered. kAddLook: and says whether tiles would be.
+constexpr int kAddAll = 0, kAddIf = 1, kAddLook = 2;
+template <int WHAT>
 __global__ __launch_bounds__(kCodecBlock) void coo_add_kernel(const long long* __restrict__ idx,
                                                               const float* __restrict__ val, int64_t nnz,
                                                               float* __restrict__ dense, int64_t n, CooTiles tiles) {
-  if (IF && !coo_unordered(tiles)) return;
-  const int64_t step = (int64_t)gridDim.x * kCodecBlock;
-  for (int64_t j = (int64_t)blockIdx.x * kCodecBlock + threadIdx.x; j < nnz; j += step) {
+  if (WHAT == kAddIf && !coo_unordered(tiles)) return;
+  const int64_t step = (int64_t)gridDim.x * kCodecBlock, first = (int64_t)blockIdx.x * kCodecBlock + threadIdx.x;
+  if (WHAT == kAddLook) {              // (ahead of the additions: behind them all workgroups would raise the flag at once)
+    bool wrong = false;
+    for (int64_t j = first; j < nnz; j += step) wrong = wrong || idx[j] < 0 || idx[j] >= n || (j > 0 && idx[j - 1] >= idx[j]);
+    if (__syncthreads_or(wrong) && threadIdx.x == 0) coo_raise(tiles);
+  }
+  for (int64_t j = first; j < nnz; j += step) {
     const long long i = idx[j];
     if (i < 0 || i >= n) continue;
     unsafeAtomicAdd(&dense[i], val[j]);   // hardware fp32 add, no CAS loop
@@ -778,9 +797,7 @@ static unsigned stream_grid(int64_t n) {
   return (unsigned)blocks;
 }
 
-int32_t coo_find_tiles(CooWork* work, const long long* d_idx, int64_t nnz, int64_t n, CooTiles* out,
-                       hipStream_t stream) {
-  const int64_t tiles = (n + kCooTile - 1) / kCooTile;
+int32_t coo_new_tag(CooWork* work, int64_t n, CooTiles* out, hipStream_t stream) {
   uint32_t* room = work->lent;
   bool fresh = work->calls == 0 || work->calls == 0xFFFFFFFFu;   // a fresh buffer holds no tag, and 0 is none
   if (!room) {
@@ -791,18 +808,25 @@ int32_t coo_find_tiles(CooWork* work, const long long* d_idx, int64_t nnz, int64
   }
   out->unordered = room;
   out->starts = room + 1;
-  out->tiles = (uint32_t)tiles;
-  bool with_bits = n >= kCooBitsLarge && nnz * kCooBitsFrom >= n;
-  if (with_bits && work->bits.reserve((size_t)tiles * (kCooTile / 8)) != KRK_SUCCESS) {
-    (void)hipGetLastError();                         // no failure of a later launch
-    with_bits = false;                               // the indices are read again, then
-  }
-  out->bits = with_bits ? work->bits.as<uint32_t>() : nullptr;
+  out->tiles = (uint32_t)((n + kCooTile - 1) / kCooTile);
+  out->bits = nullptr;
   if (fresh) {
     KRK_HIP(hipMemsetAsync(out->unordered, 0, sizeof(uint32_t), stream));
     work->calls = 0;
   }
   out->tag = ++work->calls;
+  return KRK_SUCCESS;
+}
+
+int32_t coo_find_tiles(CooWork* work, const long long* d_idx, int64_t nnz, int64_t n, CooTiles* out,
+                       hipStream_t stream) {
+  KRK_TRY(coo_new_tag(work, n, out, stream));
+  bool with_bits = n >= kCooBitsLarge && nnz * kCooBitsFrom >= n;
+  if (with_bits && work->bits.reserve((size_t)out->tiles * (kCooTile / 8)) != KRK_SUCCESS) {
+    (void)hipGetLastError();                         // no failure of a later launch
+    with_bits = false;                               // the indices are read again, then
+  }
+  if (with_bits) out->bits = work->bits.as<uint32_t>();
   const bool vec = ((uintptr_t)d_idx & 15) == 0;
   const dim3 block(kCodecBlock);
   if (with_bits) {
@@ -823,20 +847,22 @@ int32_t coo_scatter_if_unordered(const CooTiles& tiles, const long long* d_idx, 
                                  float* d_dense, int64_t n, hipStream_t stream) {
   const dim3 block(kCodecBlock);
   hipLaunchKernelGGL(coo_zero_if_kernel, rare_grid(n), block, 0, stream, d_dense, n, tiles);
-  hipLaunchKernelGGL(coo_add_kernel<true>, rare_grid(nnz), block, 0, stream, d_idx, d_val, nnz, d_dense, n, tiles);
+  hipLaunchKernelGGL(coo_add_kernel<kAddIf>, rare_grid(nnz), block, 0, stream, d_idx, d_val, nnz, d_dense, n, tiles);
   KRK_HIP(hipGetLastError());
   return KRK_SUCCESS;
 }
 
 int32_t coo_densify(CooWork* work, const long long* d_idx, const float* d_val, int64_t nnz, float* d_dense, int64_t n,
-                    hipStream_t stream) {
+                    hipStream_t stream, const CooTiles* look) {
   if (n <= 0) return KRK_SUCCESS;
   const dim3 block(kCodecBlock);
   if (!coo_tiled(n, nnz) || nnz == 0) {
     KRK_HIP(hipMemsetAsync(d_dense, 0, (size_t)n * sizeof(float), stream));   // t/math.cc:1066 dense.Zero()
-    if (nnz)
-      hipLaunchKernelGGL(coo_add_kernel<false>, dim3((unsigned)((nnz + kCodecBlock - 1) / kCodecBlock)), block, 0,
-                         stream, d_idx, d_val, nnz, d_dense, n, CooTiles{});
+    const dim3 grid((unsigned)((nnz + kCodecBlock - 1) / kCodecBlock));
+    if (nnz && look)
+      hipLaunchKernelGGL(coo_add_kernel<kAddLook>, grid, block, 0, stream, d_idx, d_val, nnz, d_dense, n, *look);
+    else if (nnz)
+      hipLaunchKernelGGL(coo_add_kernel<kAddAll>, grid, block, 0, stream, d_idx, d_val, nnz, d_dense, n, CooTiles{});
     KRK_HIP(hipGetLastError());
     return KRK_SUCCESS;
   }

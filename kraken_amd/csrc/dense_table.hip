@@ -18,7 +18,8 @@ struct krk_dense : krk::ObjBase {
   float* state[KRK_ST_COUNT] = {};   // created on first use, zero filled
   float* coo_grad = nullptr;         // densified COO gradient
   krk::CooWork coo_work;             // work space of the tiled densify
-  int coo_plain = 0;                 // blocking sparse pushes that will not look for tiles (kCooPlainPushes)
+  bool coo_ascends = false;          // small tables: the last blocking sparse push that was looked at had ascending indices
+  int coo_plain = 0;                 // and how many will be scattered without a look (kCooPlainPushes)
   int64_t steps = 0;                 // Adam's kSteps (one counter for the whole tensor)
   bool sgd_started = false;          // momentum buffer exists (first update copies the gradient)
   hipStream_t own_stream = nullptr;  // the stream created with the table (a group lends its own)
@@ -420,22 +421,43 @@ static int32_t dense_finish(krk_dense* t, uint32_t flags) {
 
 constexpr unsigned kCooGrid = 512;
 
-// The last launch of a push that waits: the word, and behind it whether the tiles were no help.
+// The last launch of a push that waits: the word, and behind it whether the indices were found to be unordered.
 __global__ void signal_unordered_kernel(uint32_t* word, uint32_t ticket, CooTiles tiles) {
   word[1] = coo_unordered(tiles) ? 1u : 0u;
   signal_host(word, ticket);
 }
 
-// A small tensor's pushes that are zeroed and scattered into after one whose indices did not ascend.
+// Waits for what a push enqueued. *unordered: what its launches found out; *waited: false, and neither is known, where
+// there was no word to be had.
+static int32_t dense_finish_coo(krk_dense* t, const CooTiles& tiles, uint32_t flags, bool* unordered, bool* waited) {
+  StreamWait end;
+  *waited = false;
+  if (!end.open()) return KRK_SUCCESS;
+  hipLaunchKernelGGL(signal_unordered_kernel, dim3(1), dim3(1), 0, t->stream, end.word, end.ticket, tiles);
+  KRK_HIP(hipGetLastError());
+  // (host arrays may have been staged by copies of pageable memory: see dense_finish)
+  if (!(flags & KRK_DEVICE_PTRS)) KRK_HIP(hipStreamSynchronize(t->stream));
+  uint32_t told = 0;
+  KRK_TRY(wait_for(&end, t->stream, &told));
+  *unordered = told != 0;
+  *waited = true;
+  return KRK_SUCCESS;
+}
+
+// A small tensor's pushes that are zeroed and scattered into, with no look at their order, after one whose indices did
+// not ascend.
 constexpr int kCooPlainPushes = 256;
 
 // One Optim::Update with a sparse gradient of nnz > 0 entries (device addresses); entries whose
 // index lies outside [0, n) are skipped. A blocking call waits for the update anyway, so it is
 // waited for here, and the launches for unordered indices follow only where there are any (three
-// launches that look at a flag and leave: 13 us). So a blocking call goes tile by tile whatever the size: of
-// 300 / 20,000 / 300,000 / 2 million elements, an entry in four, Adam, 17.5 / 18.0 / 18.8 / 30.5 us by fill, scatter
-// and update, 15.1 / 17.1 / 17.2 / 23.6 in tiles. Indices that do not ascend cost it a look at them (20 to 100 us), so
-// after such a push a small table takes the fill and scatter for the next ones. Indices that the kernels read in host
+// launches that look at a flag and leave: 13 us). So blocking calls go tile by tile whatever the size, once a
+// push has been seen to ascend: 300 / 20,000 / 300,000 / 2 million elements, an entry in four, Adam, device
+// arrays, 15.1 / 16.2 / 17.0 / 30.0 us by fill, scatter and update, 12.9 / 15.8 / 15.7 / 22.4 in tiles. A push that
+// goes tile by tile and whose indices do not ascend is scattered after all, behind a second wait (shuffled, 36 / 63 us for
+// 300,000 / 2 million elements, 19 / 48 where it is scattered at once), so the push before it decides: a small table's first
+// one is scattered, and the scatter looks at the order in passing (28 us for 27 of 2 million elements); after one that does
+// not ascend the next ones are scattered as they are. Indices that the kernels read in host
 // memory cross PCIe twice in tiles and once in the scatter (page-locked, 300,000 / 2 million elements, an entry in four,
 // 51 / 227 us and 37 / 132; pageable 64 and 52 for 300,000), so a small table's tiles are for indices in device
 // memory, the caller's or staged there (in_device). *waited: nothing is left to wait for.
@@ -448,20 +470,29 @@ static int32_t dense_apply_coo(krk_dense* t, const krk_optim& o, const long long
     KRK_HIP(hipMalloc((void**)&t->coo_grad, grad + coo_tile_words(t->n) * sizeof(uint32_t)));
     t->coo_work.lent = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(t->coo_grad) + grad);
   }
-  const bool small = t->n < kCooTiledFrom;
-  bool tiled = coo_tiled(t->n, nnz);
-  if (small && in_device && !(flags & KRK_ASYNC) && nnz <= t->n) {   // (more entries than elements do not ascend)
-    tiled = t->coo_plain == 0;
-    if (!tiled) --t->coo_plain;
+  const bool small = t->n < kCooTiledFrom, waits = !(flags & KRK_ASYNC);
+  bool tiled = coo_tiled(t->n, nnz), look = false, unordered = false;
+  if (small && in_device && waits && nnz <= t->n) {   // (more entries than elements do not ascend)
+    tiled = t->coo_ascends;
+    look = !tiled && t->coo_plain == 0;
+    if (t->coo_plain) --t->coo_plain;
   }
+  CooTiles tiles;
   if (!tiled) {
-    KRK_TRY(coo_densify(&t->coo_work, d_idx, d_val, nnz, t->coo_grad, t->n, t->stream));
-    return dense_apply(t, o, t->coo_grad, lr);
+    if (look) KRK_TRY(coo_new_tag(&t->coo_work, t->n, &tiles, t->stream));
+    KRK_TRY(coo_densify(&t->coo_work, d_idx, d_val, nnz, t->coo_grad, t->n, t->stream, look ? &tiles : nullptr));
+    KRK_TRY(dense_apply(t, o, t->coo_grad, lr));
+    if (!look) return KRK_SUCCESS;
+    KRK_TRY(dense_finish_coo(t, tiles, flags, &unordered, waited));
+    if (*waited) {
+      t->coo_ascends = !unordered;
+      t->coo_plain = unordered ? kCooPlainPushes : 0;
+    }
+    return KRK_SUCCESS;
   }
   DenseMember m;
   KRK_TRY(dense_member(t, o, &m));
   const OptimK k = make_optim_k(o);
-  CooTiles tiles;
   KRK_TRY(coo_find_tiles(&t->coo_work, d_idx, nnz, t->n, &tiles, t->stream));
   const dim3 block(kDenseBlock);
   with_optim(o.type, [&](auto opt) {
@@ -473,17 +504,14 @@ static int32_t dense_apply_coo(krk_dense* t, const krk_optim& o, const long long
     }
   });
   KRK_HIP(hipGetLastError());
-  StreamWait end;
-  if (!(flags & KRK_ASYNC) && end.open()) {
-    hipLaunchKernelGGL(signal_unordered_kernel, dim3(1), dim3(1), 0, t->stream, end.word, end.ticket, tiles);
-    KRK_HIP(hipGetLastError());
-    uint32_t unordered = 0;
-    // (host arrays may have been staged by copies of pageable memory: see dense_finish)
-    if (!(flags & KRK_DEVICE_PTRS)) KRK_HIP(hipStreamSynchronize(t->stream));
-    KRK_TRY(wait_for(&end, t->stream, &unordered));
-    *waited = !unordered;
-    if (*waited) return KRK_SUCCESS;
-    if (small) t->coo_plain = kCooPlainPushes;
+  if (waits) {
+    KRK_TRY(dense_finish_coo(t, tiles, flags, &unordered, waited));
+    if (*waited && !unordered) return KRK_SUCCESS;
+    if (*waited && small) {
+      t->coo_ascends = false;
+      t->coo_plain = kCooPlainPushes;
+    }
+    *waited = false;
   }
   KRK_TRY(coo_scatter_if_unordered(tiles, d_idx, d_val, nnz, t->coo_grad, t->n, t->stream));
   with_optim(o.type, [&](auto opt) {

@@ -549,7 +549,7 @@ __device__ __forceinline__ void optim_element(const OptimK& k, float lr, float g
 // device, and the launches of the other way look at the flag and leave.
 constexpr int kCooTile = 2048;                   // floats of one tile: 8 KB of LDS
 // Smaller tensors: zero + scatter, two launches are quicker than two and those of the other way, unless the call
-// waits and learns which of the ways it was (dense_apply_coo).
+// waits and learns which of the ways it was, and calls before it let it expect that (dense_apply_coo).
 constexpr int64_t kCooTiledFrom = 1 << 22;
 struct CooTiles {
   uint32_t* starts;       // [tiles + 1]: tile t owns entries [starts[t], starts[t + 1])
@@ -594,13 +594,16 @@ struct CooTileBits {
   }
 };
 inline bool coo_tiled(int64_t n, int64_t nnz) { return n >= kCooTiledFrom && nnz < ((int64_t)1 << 31); }
+// A flag of a new call, lowered: out without starts and bits.
+int32_t coo_new_tag(CooWork* work, int64_t n, CooTiles* out, hipStream_t stream);
 int32_t coo_find_tiles(CooWork* work, const long long* d_idx, int64_t nnz, int64_t n, CooTiles* out,
                        hipStream_t stream);
 // What is left to do where the indices are unordered, and nothing otherwise: dense = the entries' sums.
 int32_t coo_scatter_if_unordered(const CooTiles& tiles, const long long* d_idx, const float* d_val, int64_t nnz,
                                  float* d_dense, int64_t n, hipStream_t stream);
+// look (smaller tensors): raised if the indices are not such as could be taken tile by tile.
 int32_t coo_densify(CooWork* work, const long long* d_idx, const float* d_val, int64_t nnz, float* d_dense, int64_t n,
-                    hipStream_t stream);
+                    hipStream_t stream, const CooTiles* look = nullptr);
 
 // Stable radix sort of n (key, payload) pairs by the low `bits` bits of the key (radix_sort.hip).
 // keys / vals are overwritten; keys_alt / vals_alt hold n entries each; work holds

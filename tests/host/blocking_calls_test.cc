@@ -7,7 +7,9 @@
 //     ended, so that no other call waits on the same word; where all words are taken calls synchronise;
 //   - a thread that waits lets others of its core run, on whom the end of its work may depend;
 //   - a sparse gradient of a small dense table whose indices the kernels read in host memory is scattered, which
-//     reads them once.
+//     reads them once;
+//   - sparse gradients of a small dense table go tile by tile from the push on that follows one whose indices were
+//     seen to ascend, and are scattered for a while after one whose indices do not.
 #ifndef __HIP_PLATFORM_AMD__
 #define __HIP_PLATFORM_AMD__
 #endif
@@ -47,6 +49,7 @@ struct Runtime {
   int yields_until_told = 0;                        // > 0: late words are written at the last of so many sched_yields
   int synchronised = 0;
   std::vector<std::string> launched;                // names, mangled
+  bool unordered = false;                           // what launches find out about a sparse gradient's indices
   uint32_t rows = 0;                                // what the tables' counters say
   std::function<void()> on_synchronise;
   dim3 grid, block;
@@ -174,7 +177,11 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shmem, hip
 hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t stream) {
   const std::string& name = rt().kernels[f];
   rt().launched.push_back(name);
-  if (name.find("signal_kernel") != std::string::npos) {
+  if (name.find("signal_unordered_kernel") != std::string::npos) {
+    uint32_t* word = *static_cast<uint32_t**>(args[0]);
+    word[1] = rt().unordered ? 1u : 0u;
+    tell(stream, word, *static_cast<uint32_t*>(args[1]));
+  } else if (name.find("signal_kernel") != std::string::npos) {
     tell(stream, *static_cast<uint32_t**>(args[0]), *static_cast<uint32_t*>(args[1]));
   } else if (name.find("counters_kernel") != std::string::npos) {
     struct Counters {   // CountersArgs of sparse_table.hip
@@ -407,6 +414,42 @@ static void sparse_gradients_in_host_memory() {
   }
 }
 
+// How many of n pushes of a gradient in device memory went tile by tile, and how many were scattered.
+struct Ways {
+  int tiles, scattered;
+  bool operator==(const Ways& o) const { return tiles == o.tiles && scattered == o.scattered; }
+};
+static Ways push_in_device_memory(krk_dense* d, bool unordered, int n, int64_t nnz = 100) {
+  static void *index = nullptr, *vals = nullptr;
+  if (!index) CHECK(krk_malloc(&index, 8 * 100000) == 0 && krk_malloc(&vals, 4 * 100000) == 0);
+  krk_optim sgd;
+  CHECK(krk_optim_defaults(KRK_SGD, &sgd) == 0);
+  rt().launched.clear();
+  rt().unordered = unordered;
+  for (int push = 0; push < n; ++push)
+    whole("push_coo", krk_dense_push_coo(d, &sgd, static_cast<int64_t*>(index), static_cast<float*>(vals), nnz, 0.1f,
+                                         KRK_DEVICE_PTRS));
+  CHECK(launches("coo_tiles_bounds_kernel") == launches("coo_update_kernel"));
+  return Ways{launches("coo_tiles_bounds_kernel"), launches("coo_add_kernel")};
+}
+
+static void order_of_sparse_gradients() {
+  std::vector<float> vals(50000);
+  krk_dense* d = nullptr;
+  CHECK(krk_dense_create(vals.data(), (int64_t)vals.size(), 0, &d) == 0);
+  CHECK((push_in_device_memory(d, true, 258) == Ways{0, 258}));   // never a look at the tiles
+  CHECK((push_in_device_memory(d, false, 257) == Ways{0, 257}));  // some of them spared, then one that is looked at
+  CHECK((push_in_device_memory(d, false, 300) == Ways{300, 0}));
+  CHECK((push_in_device_memory(d, false, 1, 60000) == Ways{0, 1}));   // more entries than elements
+  CHECK((push_in_device_memory(d, false, 3) == Ways{3, 0}));
+  CHECK((push_in_device_memory(d, true, 1) == Ways{1, 1}));       // seen too late
+  CHECK((push_in_device_memory(d, true, 300) == Ways{0, 300}));
+  CHECK(krk_dense_destroy(d) == 0);
+  CHECK(krk_dense_create(vals.data(), (int64_t)vals.size(), 0, &d) == 0);
+  CHECK((push_in_device_memory(d, false, 5) == Ways{4, 1}));
+  CHECK(krk_dense_destroy(d) == 0);
+}
+
 int main(int argc, char** argv) {
   const std::string which = argc > 1 ? argv[1] : "";
   CHECK(krk_runtime_init(0) == 0);
@@ -423,6 +466,8 @@ int main(int argc, char** argv) {
     one_core();
   } else if (which == "host_gradients") {
     sparse_gradients_in_host_memory();
+  } else if (which == "gradients_order") {
+    order_of_sparse_gradients();
   } else {
     return 2;
   }
