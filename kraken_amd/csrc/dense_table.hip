@@ -421,9 +421,11 @@ static int32_t dense_finish(krk_dense* t, uint32_t flags) {
 
 constexpr unsigned kCooGrid = 512;
 
-// The last launch of a push that waits: the word, and behind it whether the indices were found to be unordered.
+// The last launch of a push that waits: the word, and behind it the word's number if the indices were not found to be
+// unordered. (Not a plain yes: that may be one that an earlier call's launch, which failed in between and gave its word
+// back, has written meanwhile. What is no yes to this call is taken for a no, which is right for ordered ones too.)
 __global__ void signal_unordered_kernel(uint32_t* word, uint32_t ticket, CooTiles tiles) {
-  word[1] = coo_unordered(tiles) ? 1u : 0u;
+  word[1] = coo_unordered(tiles) ? 0u : ticket;
   signal_host(word, ticket);
 }
 
@@ -439,7 +441,7 @@ static int32_t dense_finish_coo(krk_dense* t, const CooTiles& tiles, uint32_t fl
   if (!(flags & KRK_DEVICE_PTRS)) KRK_HIP(hipStreamSynchronize(t->stream));
   uint32_t told = 0;
   KRK_TRY(wait_for(&end, t->stream, &told));
-  *unordered = told != 0;
+  *unordered = told != end.ticket;
   *waited = true;
   return KRK_SUCCESS;
 }

@@ -9,7 +9,8 @@
 //   - a sparse gradient of a small dense table whose indices the kernels read in host memory is scattered, which
 //     reads them once;
 //   - sparse gradients of a small dense table go tile by tile from the push on that follows one whose indices were
-//     seen to ascend, and are scattered for a while after one whose indices do not.
+//     seen to ascend, and are scattered for a while after one whose indices do not;
+//   - what a launch says behind its word is believed by the call that waits on the word only if it is that call's.
 #ifndef __HIP_PLATFORM_AMD__
 #define __HIP_PLATFORM_AMD__
 #endif
@@ -49,6 +50,9 @@ struct Runtime {
   int yields_until_told = 0;                        // > 0: late words are written at the last of so many sched_yields
   int synchronised = 0;
   std::vector<std::string> launched;                // names, mangled
+  int fail_after = 0;                               // > 0: that many launches from here an error is reported
+  uint32_t* old_word = nullptr;                     // a word that a launch of a failed call writes over the next one's
+  uint32_t old_ticket = 0;
   bool unordered = false;                           // what launches find out about a sparse gradient's indices
   uint32_t rows = 0;                                // what the tables' counters say
   std::function<void()> on_synchronise;
@@ -149,7 +153,7 @@ hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int) {
   return hipSuccess;
 }
 const char* hipGetErrorString(hipError_t) { return "no such thing here"; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() { return rt().fail_after > 0 && --rt().fail_after == 0 ? hipErrorUnknown : hipSuccess; }
 hipError_t hipPeekAtLastError() { return hipSuccess; }
 hipError_t hipMemGetInfo(size_t* f, size_t* t) { *f = *t = (size_t)1 << 33; return hipSuccess; }
 hipError_t hipGetSymbolAddress(void** p, const void*) { return take(p, (size_t)64 << 20, false, 0); }
@@ -179,8 +183,19 @@ hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipSt
   rt().launched.push_back(name);
   if (name.find("signal_unordered_kernel") != std::string::npos) {
     uint32_t* word = *static_cast<uint32_t**>(args[0]);
-    word[1] = rt().unordered ? 1u : 0u;
-    tell(stream, word, *static_cast<uint32_t*>(args[1]));
+    const uint32_t ticket = *static_cast<uint32_t*>(args[1]);
+    if (rt().fail_after > 0) {                        // a launch of a call that will fail: it ends during the next one
+      rt().old_word = word;
+      rt().old_ticket = ticket;
+    } else {
+      word[1] = rt().unordered ? 0u : ticket;
+      tell(stream, word, ticket);
+      if (rt().old_word) {
+        if (rt().old_word != word) std::abort();
+        word[1] = word[0] = rt().old_ticket;          // (that push's indices ascended)
+        rt().old_word = nullptr;
+      }
+    }
   } else if (name.find("signal_kernel") != std::string::npos) {
     tell(stream, *static_cast<uint32_t**>(args[0]), *static_cast<uint32_t*>(args[1]));
   } else if (name.find("counters_kernel") != std::string::npos) {
@@ -450,6 +465,27 @@ static void order_of_sparse_gradients() {
   CHECK(krk_dense_destroy(d) == 0);
 }
 
+// A push that fails behind its last launch, and one of a shuffled gradient that gets the same word: the launch of the
+// first ends behind that of the second.
+static void word_of_a_failed_push() {
+  const int64_t cells = (int64_t)1 << 22;
+  std::vector<float> vals(cells);
+  krk_dense* d[2] = {};
+  for (krk_dense*& t : d) CHECK(krk_dense_create(vals.data(), cells, 0, &t) == 0);
+  CHECK((push_in_device_memory(d[1], false, 1) == Ways{1, 0}));
+  void *index = nullptr, *values = nullptr;
+  CHECK(krk_malloc(&index, 800) == 0 && krk_malloc(&values, 400) == 0);
+  krk_optim sgd;
+  CHECK(krk_optim_defaults(KRK_SGD, &sgd) == 0);
+  rt().fail_after = 3;                              // behind the launches of the tiles, the update and the word
+  CHECK(krk_dense_push_coo(d[0], &sgd, static_cast<int64_t*>(index), static_cast<float*>(values), 100, 0.1f,
+                           KRK_DEVICE_PTRS) != KRK_SUCCESS);
+  CHECK(rt().fail_after == 0 && rt().old_word != nullptr);
+  CHECK((push_in_device_memory(d[1], true, 1) == Ways{1, 1}));
+  CHECK(rt().old_word == nullptr);
+  for (krk_dense* t : d) CHECK(krk_dense_destroy(t) == 0);
+}
+
 int main(int argc, char** argv) {
   const std::string which = argc > 1 ? argv[1] : "";
   CHECK(krk_runtime_init(0) == 0);
@@ -468,6 +504,8 @@ int main(int argc, char** argv) {
     sparse_gradients_in_host_memory();
   } else if (which == "gradients_order") {
     order_of_sparse_gradients();
+  } else if (which == "old_words") {
+    word_of_a_failed_push();
   } else {
     return 2;
   }
