@@ -810,6 +810,7 @@ int32_t coo_new_tag(CooWork* work, int64_t n, CooTiles* out, hipStream_t stream)
   out->starts = room + 1;
   out->tiles = (uint32_t)((n + kCooTile - 1) / kCooTile);
   out->bits = nullptr;
+  out->told = nullptr;
   if (fresh) {
     KRK_HIP(hipMemsetAsync(out->unordered, 0, sizeof(uint32_t), stream));
     work->calls = 0;

@@ -266,11 +266,17 @@ static int32_t dense_apply(krk_dense* t, const krk_optim& o, const float* d_grad
 // The tile's parameters and moments do not depend on the entries: they are requested first.
 constexpr int kCooPer = kCooTile / 4 / kDenseBlock;   // 16-byte pieces of a tile a lane updates
 
+__device__ __forceinline__ bool tiles_no_help(const CooTiles& tiles) {
+  const bool unordered = coo_unordered(tiles);
+  if (tiles.told && blockIdx.x == 0 && threadIdx.x == 0) *tiles.told = unordered ? 0u : tiles.ticket;
+  return unordered;
+}
+
 template <int OPT>
 __global__ __launch_bounds__(kDenseBlock) void coo_update_kernel(DenseMember m, const long long* __restrict__ idx,
                                                                  const float* __restrict__ val, CooTiles tiles,
                                                                  float lr, OptimK k) {
-  if (coo_unordered(tiles)) return;              // the launches that follow do the work
+  if (tiles_no_help(tiles)) return;              // the launches that follow do the work
   __shared__ __align__(16) float grad[kCooTile];
   const dfloat4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
   for (uint32_t tile = blockIdx.x; tile < tiles.tiles; tile += gridDim.x) {
@@ -345,7 +351,7 @@ __global__ __launch_bounds__(kDenseBlock) void coo_update_kernel(DenseMember m, 
 template <int OPT>
 __global__ __launch_bounds__(kDenseBlock) void coo_bits_update_kernel(DenseMember m, const float* __restrict__ val,
                                                                       CooTiles tiles, float lr, OptimK k) {
-  if (coo_unordered(tiles)) return;              // the launches that follow do the work
+  if (tiles_no_help(tiles)) return;              // the launches that follow do the work
   const dfloat4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
   const int lane = threadIdx.x & 63;
   uint32_t start = tiles.starts[blockIdx.x], end = tiles.starts[blockIdx.x + 1];   // (no workgroup without a tile)
@@ -421,27 +427,32 @@ static int32_t dense_finish(krk_dense* t, uint32_t flags) {
 
 constexpr unsigned kCooGrid = 512;
 
-// The last launch of a push that waits: the word, and behind it the word's number if the indices were not found to be
-// unordered. (Not a plain yes: that may be one that an earlier call's launch, which failed in between and gave its word
-// back, has written meanwhile. What is no yes to this call is taken for a no, which is right for ordered ones too.)
+// Whether a push's indices were not found to be unordered, as its launches tell the host behind a word: by the word's
+// number. (Not by a plain yes: that may be one that an earlier call's launch, which failed in between and gave its
+// word back, has written meanwhile. What is no yes to this call is taken for a no, which is right for ordered ones too.)
+// The last launch of a push of device arrays that waits writes both.
 __global__ void signal_unordered_kernel(uint32_t* word, uint32_t ticket, CooTiles tiles) {
   word[1] = coo_unordered(tiles) ? 0u : ticket;
   signal_host(word, ticket);
 }
 
-// Waits for what a push enqueued. *unordered: what its launches found out; *waited: false, and neither is known, where
-// there was no word to be had.
-static int32_t dense_finish_coo(krk_dense* t, const CooTiles& tiles, uint32_t flags, bool* unordered, bool* waited) {
-  StreamWait end;
+// Waits for what a push enqueued. *unordered: what its launches found out. end is not open where there was no word to be
+// had: neither is known then.
+static int32_t dense_finish_coo(krk_dense* t, StreamWait* end, const CooTiles& tiles, uint32_t flags, bool* unordered,
+                                bool* waited) {
   *waited = false;
-  if (!end.open()) return KRK_SUCCESS;
-  hipLaunchKernelGGL(signal_unordered_kernel, dim3(1), dim3(1), 0, t->stream, end.word, end.ticket, tiles);
-  KRK_HIP(hipGetLastError());
-  // (host arrays may have been staged by copies of pageable memory: see dense_finish)
-  if (!(flags & KRK_DEVICE_PTRS)) KRK_HIP(hipStreamSynchronize(t->stream));
+  if (!end->word) return KRK_SUCCESS;
   uint32_t told = 0;
-  KRK_TRY(wait_for(&end, t->stream, &told));
-  *unordered = told != end.ticket;
+  if (flags & KRK_DEVICE_PTRS) {
+    hipLaunchKernelGGL(signal_unordered_kernel, dim3(1), dim3(1), 0, t->stream, end->word, end->ticket, tiles);
+    KRK_HIP(hipGetLastError());
+    KRK_TRY(wait_for(end, t->stream, &told));
+  } else {
+    KRK_HIP(hipStreamSynchronize(t->stream));   // (see dense_finish)
+    told = __atomic_load_n(end->told(), __ATOMIC_RELAXED);
+    end->close();
+  }
+  *unordered = told != end->ticket;
   *waited = true;
   return KRK_SUCCESS;
 }
@@ -459,12 +470,17 @@ constexpr int kCooPlainPushes = 256;
 // goes tile by tile and whose indices do not ascend is scattered after all, behind a second wait (shuffled, 36 / 63 us for
 // 300,000 / 2 million elements, 19 / 48 where it is scattered at once), so the push before it decides: a small table's first
 // one is scattered, and the scatter looks at the order in passing (28 us for 27 of 2 million elements); after one that does
-// not ascend the next ones are scattered as they are. Indices that the kernels read in host
-// memory cross PCIe twice in tiles and once in the scatter (page-locked, 300,000 / 2 million elements, an entry in four,
-// 51 / 227 us and 37 / 132; pageable 64 and 52 for 300,000), so a small table's tiles are for indices in device
-// memory, the caller's or staged there (in_device). *waited: nothing is left to wait for.
+// not ascend the next ones are scattered as they are.
+// That is for device arrays. Indices that the kernels read in host memory cross PCIe twice in tiles and once in the
+// scatter (page-locked, 300,000 / 2 million elements, an entry in four, 51 / 227 us and 37 / 132; pageable 64 and 52
+// for 300,000). And from eight commands on between two synchronises the runtime gives back pinned pages and freed
+// memory in a way that slows the copies and allocations which follow: a new table's first push of 2 million elements
+// from pageable arrays takes 250 us with seven (two copies, Adam's columns, fill, scatter, update) and with nine mostly
+// 3000, as does creating the next table. So a push of host arrays enqueues no launch
+// that it can do without: a small one is always scattered, and of a large one the update itself says whether
+// the tiles were of help. *waited: nothing is left to wait for.
 static int32_t dense_apply_coo(krk_dense* t, const krk_optim& o, const long long* d_idx, const float* d_val,
-                               int64_t nnz, bool in_device, float lr, uint32_t flags, bool* waited) {
+                               int64_t nnz, float lr, uint32_t flags, bool* waited) {
   *waited = false;
   if (!t->coo_grad) {
     // (one allocation: a table's first sparse push pays for it)
@@ -474,18 +490,19 @@ static int32_t dense_apply_coo(krk_dense* t, const krk_optim& o, const long long
   }
   const bool small = t->n < kCooTiledFrom, waits = !(flags & KRK_ASYNC);
   bool tiled = coo_tiled(t->n, nnz), look = false, unordered = false;
-  if (small && in_device && waits && nnz <= t->n) {   // (more entries than elements do not ascend)
+  if (small && (flags & KRK_DEVICE_PTRS) && waits && nnz <= t->n) {   // (more entries than elements do not ascend)
     tiled = t->coo_ascends;
     look = !tiled && t->coo_plain == 0;
     if (t->coo_plain) --t->coo_plain;
   }
   CooTiles tiles;
+  StreamWait end;
   if (!tiled) {
     if (look) KRK_TRY(coo_new_tag(&t->coo_work, t->n, &tiles, t->stream));
     KRK_TRY(coo_densify(&t->coo_work, d_idx, d_val, nnz, t->coo_grad, t->n, t->stream, look ? &tiles : nullptr));
     KRK_TRY(dense_apply(t, o, t->coo_grad, lr));
-    if (!look) return KRK_SUCCESS;
-    KRK_TRY(dense_finish_coo(t, tiles, flags, &unordered, waited));
+    if (!look || !end.open()) return KRK_SUCCESS;
+    KRK_TRY(dense_finish_coo(t, &end, tiles, flags, &unordered, waited));
     if (*waited) {
       t->coo_ascends = !unordered;
       t->coo_plain = unordered ? kCooPlainPushes : 0;
@@ -496,6 +513,10 @@ static int32_t dense_apply_coo(krk_dense* t, const krk_optim& o, const long long
   KRK_TRY(dense_member(t, o, &m));
   const OptimK k = make_optim_k(o);
   KRK_TRY(coo_find_tiles(&t->coo_work, d_idx, nnz, t->n, &tiles, t->stream));
+  if (waits && end.open() && !(flags & KRK_DEVICE_PTRS)) {
+    tiles.told = end.told();
+    tiles.ticket = end.ticket;
+  }
   const dim3 block(kDenseBlock);
   with_optim(o.type, [&](auto opt) {
     const dim3 grid(std::min(tiles.tiles, kCooGrid));
@@ -507,7 +528,7 @@ static int32_t dense_apply_coo(krk_dense* t, const krk_optim& o, const long long
   });
   KRK_HIP(hipGetLastError());
   if (waits) {
-    KRK_TRY(dense_finish_coo(t, tiles, flags, &unordered, waited));
+    KRK_TRY(dense_finish_coo(t, &end, tiles, flags, &unordered, waited));
     if (*waited && !unordered) return KRK_SUCCESS;
     if (*waited && small) {
       t->coo_ascends = false;
@@ -811,8 +832,7 @@ int32_t krk_dense_push_coo(krk_dense* t, const krk_optim* o, const int64_t* idx,
   KRK_TRY(t->input(idx, (size_t)nnz, flags, 0, &d_idx));
   KRK_TRY(t->input(val, (size_t)nnz, flags, 1, &d_val));
   bool waited = false;
-  const bool in_device = (flags & KRK_DEVICE_PTRS) || (const void*)d_idx == t->stage[0].ptr;
-  KRK_TRY(dense_apply_coo(t, *o, reinterpret_cast<const long long*>(d_idx), d_val, nnz, in_device, lr, flags, &waited));
+  KRK_TRY(dense_apply_coo(t, *o, reinterpret_cast<const long long*>(d_idx), d_val, nnz, lr, flags, &waited));
   return waited ? KRK_SUCCESS : dense_finish(t, flags);
 }
 

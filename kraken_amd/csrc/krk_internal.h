@@ -557,6 +557,8 @@ struct CooTiles {
   uint32_t tag;
   uint32_t tiles;
   uint32_t* bits;         // null, or a bit an element, 64 words a tile: whether an entry names it
+  uint32_t* told;         // null, or page-locked: who walks the tiles puts `ticket` there, 0 if they are no help
+  uint32_t ticket;
 };
 __device__ __forceinline__ bool coo_unordered(const CooTiles& t) { return *t.unordered == t.tag; }
 struct CooWork {          // work space of one caller, kept between calls

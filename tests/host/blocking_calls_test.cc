@@ -6,10 +6,10 @@
 //   - a word that a launch under way will still write belongs to the call that waits for it until that launch has
 //     ended, so that no other call waits on the same word; where all words are taken calls synchronise;
 //   - a thread that waits lets others of its core run, on whom the end of its work may depend;
-//   - a sparse gradient of a small dense table whose indices the kernels read in host memory is scattered, which
-//     reads them once;
+//   - a sparse gradient in host memory of a small dense table is scattered, which reads its indices once;
 //   - sparse gradients of a small dense table go tile by tile from the push on that follows one whose indices were
 //     seen to ascend, and are scattered for a while after one whose indices do not;
+//   - a table's first sparse gradient in pageable memory takes at most seven of the runtime's commands;
 //   - what a launch says behind its word is believed by the call that waits on the word only if it is that call's.
 #ifndef __HIP_PLATFORM_AMD__
 #define __HIP_PLATFORM_AMD__
@@ -49,6 +49,7 @@ struct Runtime {
   bool signals_late = false;
   int yields_until_told = 0;                        // > 0: late words are written at the last of so many sched_yields
   int synchronised = 0;
+  int commands = 0;                                 // asynchronous copies and fills, and launches
   std::vector<std::string> launched;                // names, mangled
   int fail_after = 0;                               // > 0: that many launches from here an error is reported
   uint32_t* old_word = nullptr;                     // a word that a launch of a failed call writes over the next one's
@@ -116,12 +117,17 @@ hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
 }
 hipError_t hipMemcpy(void* d, const void* s, size_t bytes, hipMemcpyKind) { std::memcpy(d, s, bytes); return hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t bytes, hipMemcpyKind, hipStream_t stream) {
+  rt().commands++;
   if (!block_of(d) || !block_of(s)) rt().pageable[stream] = true;
   std::memcpy(d, s, bytes);
   return hipSuccess;
 }
 hipError_t hipMemset(void* d, int v, size_t bytes) { std::memset(d, v, bytes); return hipSuccess; }
-hipError_t hipMemsetAsync(void* d, int v, size_t bytes, hipStream_t) { std::memset(d, v, bytes); return hipSuccess; }
+hipError_t hipMemsetAsync(void* d, int v, size_t bytes, hipStream_t) {
+  rt().commands++;
+  std::memset(d, v, bytes);
+  return hipSuccess;
+}
 hipError_t hipStreamSynchronize(hipStream_t stream) {
   rt().synchronised++;
   if (rt().on_synchronise) rt().on_synchronise();
@@ -181,6 +187,7 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shmem, hip
 hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t stream) {
   const std::string& name = rt().kernels[f];
   rt().launched.push_back(name);
+  rt().commands++;
   if (name.find("signal_unordered_kernel") != std::string::npos) {
     uint32_t* word = *static_cast<uint32_t**>(args[0]);
     const uint32_t ticket = *static_cast<uint32_t*>(args[1]);
@@ -196,6 +203,15 @@ hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipSt
         rt().old_word = nullptr;
       }
     }
+  } else if (name.find("coo_update_kernel") != std::string::npos || name.find("coo_bits_update_kernel") != std::string::npos) {
+    struct Tiles {   // CooTiles of krk_internal.h
+      void *starts, *unordered;
+      uint32_t tag, tiles;
+      void* bits;
+      uint32_t *told, ticket;
+    };
+    const Tiles& a = *static_cast<const Tiles*>(args[name.find("coo_bits") != std::string::npos ? 2 : 3]);
+    if (a.told) *a.told = rt().unordered ? 0u : a.ticket;
   } else if (name.find("signal_kernel") != std::string::npos) {
     tell(stream, *static_cast<uint32_t**>(args[0]), *static_cast<uint32_t*>(args[1]));
   } else if (name.find("counters_kernel") != std::string::npos) {
@@ -429,6 +445,28 @@ static void sparse_gradients_in_host_memory() {
   }
 }
 
+// Sparse gradients in pageable memory that is staged by copies. unordered: large ones are scattered behind the tiles.
+static void first_sparse_gradient() {
+  krk_optim adam;
+  CHECK(krk_optim_defaults(KRK_ADAM, &adam) == 0);
+  for (const int64_t cells : {(int64_t)2000000, (int64_t)5000000}) {
+    std::vector<float> vals(cells);
+    std::vector<int64_t> index(cells / 2);
+    for (int64_t i = 0; i < cells / 2; ++i) index[i] = i;
+    for (const bool unordered : {false, true}) {
+      rt().unordered = unordered;
+      krk_dense* d = nullptr;
+      CHECK(krk_dense_create(vals.data(), cells, 0, &d) == 0);
+      rt().launched.clear();
+      rt().commands = 0;
+      whole("push_coo", krk_dense_push_coo(d, &adam, index.data(), vals.data(), cells / 2, 0.1f, 0));
+      CHECK(rt().commands <= (unordered && cells > 4200000 ? 10 : 7));
+      CHECK(launches("coo_add_kernel") == (cells < 4200000 || unordered));
+      CHECK(krk_dense_destroy(d) == 0);
+    }
+  }
+}
+
 // How many of n pushes of a gradient in device memory went tile by tile, and how many were scattered.
 struct Ways {
   int tiles, scattered;
@@ -506,6 +544,8 @@ int main(int argc, char** argv) {
     order_of_sparse_gradients();
   } else if (which == "old_words") {
     word_of_a_failed_push();
+  } else if (which == "first_gradient") {
+    first_sparse_gradient();
   } else {
     return 2;
   }

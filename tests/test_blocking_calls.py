@@ -28,8 +28,10 @@ def program(tmp_path_factory):
 # core: a waiting thread lets the other threads of its core run
 # host_gradients: sparse gradients in host memory of small dense tables are read once
 # gradients_order: which of them go tile by tile
+# first_gradient: a table's first one in pageable memory takes few commands
 # old_words: a launch of a call that failed says something over the next call's word
-@pytest.mark.parametrize("which", ["dense", "sparse", "words", "core", "host_gradients", "gradients_order", "old_words"])
+@pytest.mark.parametrize("which", ["dense", "sparse", "words", "core", "host_gradients", "gradients_order",
+                                   "first_gradient", "old_words"])
 def test_blocking_calls(program, which):
     r = subprocess.run([program, which], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
