@@ -567,6 +567,7 @@ __global__ __launch_bounds__(kCodecBlock) void coo_bits_kernel(const long long* 
   uint32_t* words = &wave_words[(threadIdx.x >> 6) * kCooWindow];
   words[lane] = 0u;
   words[lane + 64] = 0u;
+  wave_lds_order();
   const int64_t run = ((int64_t)blockIdx.x * (kCodecBlock / 64) + threadIdx.x / 64) * (kCooRun * kCooChunk);
   if (run >= nnz) return;
   const int64_t stop = run + kCooRun * kCooChunk < nnz ? run + kCooRun * kCooChunk : nnz;
@@ -611,13 +612,13 @@ __global__ __launch_bounds__(kCodecBlock) void coo_bits_kernel(const long long* 
           if (w0 != w1 && w0 - from < (uint32_t)kCooWindow) atomicOr(&words[w0 - from], b0);
           if (w1 - from < (uint32_t)kCooWindow) atomicOr(&words[w1 - from], w0 == w1 ? b0 | b1 : b1);
         }
-        __builtin_amdgcn_wave_barrier();             // one wavefront: its LDS accesses stay in order
+        wave_lds_order();
         if (top - from >= 64u) {                     // a line of complete words, and the window moves on by it
           out.bits[from + lane] = words[lane];
           words[lane] = words[lane + 64];
           words[lane + 64] = 0u;
           from += 64u;
-          __builtin_amdgcn_wave_barrier();
+          wave_lds_order();
         }
         last = (long long)before;
 #pragma unroll
@@ -654,17 +655,18 @@ __global__ __launch_bounds__(kCodecBlock) void coo_bits_kernel(const long long* 
       for (int i = 0; i < 2 * kCooRows; ++i)
         if (on[i] && w[i] - at < wide) atomicOr(&words[w[i] - at], bit[i]);
       if (shares && top - at < wide) atomicOr(&words[top - at], 1u << (after & 31));
-      __builtin_amdgcn_wave_barrier();               // one wavefront: its LDS accesses stay in order
+      wave_lds_order();
       const uint32_t v0 = words[lane], v1 = words[lane + 64];
       if ((uint32_t)lane < wide && at + lane < to) out.bits[at + lane] = v0;
       if ((uint32_t)lane + 64u < wide && at + lane + 64u < to) out.bits[at + lane + 64u] = v1;
       words[lane] = 0u;
       words[lane + 64] = 0u;
-      __builtin_amdgcn_wave_barrier();
+      wave_lds_order();
       if (to <= behind && top < behind) {
         if (!ends) {                                 // the open word goes on as the next chunk's first
           const uint32_t open = (uint32_t)__shfl((int)(top - at < 64u ? v0 : v1), (int)((top - at) & 63u));
           if (lane == 0) words[0] = open;
+          wave_lds_order();
         }
         break;
       }

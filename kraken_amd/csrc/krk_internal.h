@@ -280,6 +280,14 @@ __device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t v) {
 #undef KRK_DPP_ADD
   return v;
 }
+// Between LDS accesses of one wavefront's lanes and those of its other lanes to the same words. The hardware keeps
+// one wavefront's LDS accesses in the order they are issued in; this keeps the compiler from issuing them in
+// another one, which the barrier alone, no access to memory to it, need not. No instruction of its own.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 // Narrows the lanes of a wavefront (both halves of a mask) to those whose value has bit b as this lane's has it: four
 // vector instructions, one vote and, for either half, a bitwise operation of three operands. All lanes call it.
 __device__ __forceinline__ void match_bit(uint32_t v, int b, uint32_t& lo, uint32_t& hi) {

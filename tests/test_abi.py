@@ -137,3 +137,16 @@ def test_arrays_of_two_kinds_in_one_call(api):
     for arrays in ((dev, host), (host, dev), (None, host, dev)):
         with pytest.raises(ValueError):
             api._flags(*arrays)
+
+
+def test_lanes_meet_in_lds_in_order():
+    """Where lanes of a wavefront pass words to each other through LDS without a workgroup's barrier, fences stand around
+    the wavefront's barrier, which is no access to memory to the compiler: krk_internal.h's wave_lds_order."""
+    import glob
+    csrc = os.path.join(ROOT, "kraken_amd", "csrc")
+    uses = [(os.path.basename(p), line.strip()) for p in sorted(glob.glob(os.path.join(csrc, "*")))
+            for line in open(p) if "amdgcn_wave_barrier" in line]
+    assert uses == [("krk_internal.h", "__builtin_amdgcn_wave_barrier();")]
+    inline = open(os.path.join(csrc, "krk_internal.h")).read().split("void wave_lds_order() {")[1].split("}")[0].split()
+    assert inline == ['__builtin_amdgcn_fence(__ATOMIC_RELEASE,', '"wavefront");', "__builtin_amdgcn_wave_barrier();",
+                      '__builtin_amdgcn_fence(__ATOMIC_ACQUIRE,', '"wavefront");']
