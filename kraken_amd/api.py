@@ -221,10 +221,12 @@ def _ptr(a):
         return None
     if isinstance(a, DeviceArray):
         return a.ptr
-    try:
-        return C.byref(C.c_char.from_buffer(a))
-    except (TypeError, ValueError, BufferError):     # read-only, strided or empty
-        return a.ctypes.data_as(C.c_void_p)
+    if isinstance(a, np.ndarray):                    # (whatever else says it is a buffer is refused below)
+        try:
+            return C.byref(C.c_char.from_buffer(a))
+        except (TypeError, ValueError, BufferError):     # read-only, strided or empty
+            pass
+    return a.ctypes.data_as(C.c_void_p)
 
 
 class DeviceArray:

@@ -126,6 +126,14 @@ def test_an_array_argument_is_its_address(api, form):
     assert api._ptr(None) is None
 
 
+@pytest.mark.parametrize("make", [lambda: bytearray(64), lambda: memoryview(bytearray(64)), lambda: (C.c_float * 16)(),
+                                  lambda: __import__("array").array("f", [0.0] * 16), lambda: [0.0] * 16, lambda: b"0" * 64])
+def test_what_is_no_array_is_refused(api, make):
+    """Buffers of other kinds carry neither shape nor type: an `out` of the wrong length would be written past its end."""
+    with pytest.raises(AttributeError):
+        api._ptr(make())
+
+
 def test_arrays_of_two_kinds_in_one_call(api):
     """Device arrays in a call say so in its flags, and are not mixed with host arrays."""
     dev = api.DeviceArray.__new__(api.DeviceArray)
