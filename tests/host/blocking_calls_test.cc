@@ -10,6 +10,7 @@
 //   - sparse gradients of a small dense table go tile by tile from the push on that follows one whose indices were
 //     seen to ascend, and are scattered for a while after one whose indices do not;
 //   - a table's first sparse gradient in pageable memory takes at most seven of the runtime's commands;
+//   - a decode gives large work space back;
 //   - what a launch says behind its word is believed by the call that waits on the word only if it is that call's.
 #ifndef __HIP_PLATFORM_AMD__
 #define __HIP_PLATFORM_AMD__
@@ -524,6 +525,25 @@ static void word_of_a_failed_push() {
   for (krk_dense* t : d) CHECK(krk_dense_destroy(t) == 0);
 }
 
+// A decode belongs to no object: what it keeps on the device afterwards is bounded.
+static void work_space_of_decodes() {
+  void* place = nullptr;                            // (no kernel runs: an address is enough)
+  CHECK(krk_malloc(&place, 4096) == 0);
+  const auto held = []() {
+    size_t bytes = 0;
+    for (const auto& b : rt().blocks) bytes += b.second.bytes;
+    return bytes;
+  };
+  const size_t before = held();
+  for (const int64_t n : {(int64_t)1 << 23, (int64_t)1 << 31, (int64_t)5 << 30, (int64_t)1 << 23}) {
+    CHECK(krk_coo_to_dense(static_cast<int64_t*>(place), static_cast<float*>(place), n / 8, static_cast<float*>(place), n,
+                           KRK_DEVICE_PTRS) == KRK_SUCCESS);
+    CHECK(launches("coo_bits_write_kernel") == 1);
+    rt().launched.clear();
+    CHECK(held() - before <= ((size_t)256 << 20) + ((size_t)16 << 20));
+  }
+}
+
 int main(int argc, char** argv) {
   const std::string which = argc > 1 ? argv[1] : "";
   CHECK(krk_runtime_init(0) == 0);
@@ -546,6 +566,8 @@ int main(int argc, char** argv) {
     word_of_a_failed_push();
   } else if (which == "first_gradient") {
     first_sparse_gradient();
+  } else if (which == "decodes") {
+    work_space_of_decodes();
   } else {
     return 2;
   }

@@ -29,9 +29,10 @@ def program(tmp_path_factory):
 # host_gradients: sparse gradients in host memory of small dense tables are read once
 # gradients_order: which of them go tile by tile
 # first_gradient: a table's first one in pageable memory takes few commands
+# decodes: what a decode keeps on the device is bounded
 # old_words: a launch of a call that failed says something over the next call's word
 @pytest.mark.parametrize("which", ["dense", "sparse", "words", "core", "host_gradients", "gradients_order",
-                                   "first_gradient", "old_words"])
+                                   "first_gradient", "decodes", "old_words"])
 def test_blocking_calls(program, which):
     r = subprocess.run([program, which], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
