@@ -331,27 +331,28 @@ __global__ __launch_bounds__(kCodecBlock) void emit_write_kernel(
   }
 }
 
-// The whole emit step in one pass: gradient and residual are read once (a count pass ahead of the
-// write pass read them twice: 536 MB more for 67 million elements, 95 of 333 us with the scan). Where
-// a tile's pairs go is the number of pairs in the tiles before it, which the workgroups tell one
-// another: tile_state[t] holds what tile t keeps as soon as that is known, and what tiles 0..t keep
-// together once that is. A tile looks back over its predecessors, 64 at a time, as far as the nearest
-// whose total is known.
-// Tiles are handed out by a counter in ascending order, so every predecessor of a tile is held by a
-// workgroup that already runs, and it announces its count before it waits for anything: every wait
-// ends. An announcement carries the number of the call, so the array is never cleared; the last
-// workgroup to leave puts the counter back to zero.
-// A workgroup takes its next tile's number, and asks for its elements, ahead of writing the one it has: a tile
-// that is held but not announced is waited for by later tiles only, and its workgroup waits for earlier ones, so the lowest such
-// tile's turn always comes.
-// What bounds it is the rate of a copy: 67 million elements, of which 33 million are kept, 1.27 GB, 217 us (5.8 TB/s). 243 us with each
-// tile's loads behind the tile before it, two workgroups a compute unit, 8192 elements a tile; with the loads ahead, tiles
-// of 8192 / 16,384 elements and 192, 256, 320, 384 workgroups 255, 222, 250, 248 / 230, 217, 216, 217: the fewer tiles are on
-// their way, the less far a tile has to look back. The counter serves one workgroup after the other, some 15 ns each,
-// which is what smaller tiles wait for (573 and 331 us in tiles of 2048 and 4096); tensors that give
-// few workgroups a tile are better off with them. A blocking step, us, as before / in tiles of 4096 / 8192 / 16,384: 300,000
-// elements 15.6 / 14.2 / 16.2 / 19.2, a million 17.6 / 19.1 / 17.4 / 19.9, 4 million 31.9 / 31.6 / 29.2 / 32.6,
-// 16 million 74 / 89 / 67 / 70, 33 million 132 / 170 / 119 / 119, 67 million 252 / 331 / 229 / 224.
+// The whole emit step in one pass: gradient and residual are read once (a count pass ahead of the write pass read
+// them twice: 536 MB more for 67 million elements, 95 of 333 us with the scan). Where a tile's pairs go is the number
+// of pairs in the tiles before it, which the workgroups tell one another: tile_state[t] holds what tile t keeps as
+// soon as that is known, and what tiles 0..t keep together once that is. A tile looks back over its predecessors, 64
+// at a time, as far as the nearest whose total is known. Tiles are handed out by a counter in ascending order, so
+// every predecessor of a tile is held by a workgroup that already runs, and it announces its count before it waits
+// for anything: every wait ends. An announcement carries the number of the call, so the array is never cleared; the
+// last workgroup to leave puts the counter back to zero.
+// A workgroup takes its next tile's number, and asks for its elements, ahead of writing the one it has: a tile that
+// is held but not announced is waited for by later tiles only, and its workgroup waits for earlier ones, so the
+// lowest such tile's turn always comes.
+// What bounds it is the rate of a copy: 67 million elements, of which 33 million are kept, 1.27 GB, 217 us (5.8
+// TB/s). 243 us with each tile's loads behind the tile before it, two workgroups a compute unit, 8192 elements a
+// tile; with the loads ahead, tiles of 8192 / 16,384 elements and 192, 256, 320, 384 workgroups 255, 222, 250, 248 /
+// 230, 217, 216, 217: the fewer tiles are on their way, the less far a tile has to look back. The counter serves one
+// workgroup after the other, some 15 ns each, which is what smaller tiles wait for (573 and 331 us in tiles of 2048
+// and 4096); tensors that give few workgroups a tile are better off with them. A blocking step, us, as before / in
+// tiles of 4096 / 8192 / 16,384: 300,000 elements 15.6 / 14.2 / 16.2 / 19.2, a million 17.6 / 19.1 / 17.4 / 19.9, 4
+// million 31.9 / 31.6 / 29.2 / 32.6, 16 million 74 / 89 / 67 / 70, 33 million 132 / 170 / 119 / 119, 67 million 252 /
+// 331 / 229 / 224. Above: compress, push and pull of 33 / 40 / 50 / 67 / 100 / 134 / 200 million elements in tiles of
+// 8192 380 / 446 / 547 / 722 / 1073 / 1432 / 2139 us, of 16,384 373 / 442 / 547 / 710 / 1062 / 1422 / 2146: one in a
+// hundred or nothing.
 constexpr int64_t kSingleShort = (int64_t)1 << 19;
 constexpr int64_t kSingleLong = (int64_t)1 << 25;
 constexpr int kSingleBlock = 512;
@@ -547,15 +548,15 @@ __global__ __launch_bounds__(kCodecBlock) void coo_tiles_bounds_kernel(const lon
 }
 
 // The same, and a bit for every element that an entry names, so that who walks the tiles need not read the indices
-// again. A wavefront takes a run of consecutive chunks and carries the words that later entries may share along: every
-// word is written once, by the wavefront that holds the first of the entries behind the word before it, and nothing
-// has to be cleared ahead. Words of tiles without entries are not written. The bits meet in LDS, in a window of up
-// to two tiles' words that moves on by 64 of them, a line of memory; chunks wider than that take several windows.
-// What bounds it is the read of the indices, and next to it instruction issue: nearly every chunk of a gradient that keeps
-// a quarter of its elements is an easy one (no gap of a tile or more, all of it in the window, not the run's last),
-// and those take a third of the general path's 200 vector instructions. 33 million entries among 67 million elements: the general path
-// alone 58 us, with the easy one 55, with lines instead of each chunk's words 52 in runs of 4 (2, 8, 16: 55, 53, 55);
-// without bits 44.6. The update that follows takes 317 us for 365.
+// again. A wavefront takes a run of consecutive chunks and carries the words that later entries may share along:
+// every word is written once, by the wavefront that holds the first of the entries behind the word before it, and
+// nothing has to be cleared ahead. Words of tiles without entries are not written. The bits meet in LDS, in a window
+// of up to two tiles' words that moves on by 64 of them, a line of memory; chunks wider than that take several
+// windows. What bounds it is the read of the indices, and next to it instruction issue: nearly every chunk of a
+// gradient that keeps a quarter of its elements is an easy one (no gap of a tile or more, all of it in the window,
+// not the run's last), and those take a third of the general path's 200 vector instructions. 33 million entries among
+// 67 million elements: the general path alone 58 us, with the easy one 55, with lines instead of each chunk's words
+// 52 in runs of 4 (2, 8, 16: 55, 53, 55); without bits 44.6. The update that follows takes 317 us for 365.
 constexpr int kCooRun = 4;                           // chunks of a wavefront
 constexpr int kCooWindow = 128;
 
@@ -772,7 +773,10 @@ __global__ __launch_bounds__(kCodecBlock) void coo_add_kernel(const long long* _
   const int64_t step = (int64_t)gridDim.x * kCodecBlock, first = (int64_t)blockIdx.x * kCodecBlock + threadIdx.x;
   if (WHAT == kAddLook) {              // (ahead of the additions: behind them all workgroups would raise the flag at once)
     bool wrong = false;
-    for (int64_t j = first; j < nnz; j += step) wrong = wrong || idx[j] < 0 || idx[j] >= n || (j > 0 && idx[j - 1] >= idx[j]);
+    for (int64_t j = first; j < nnz; j += step) {
+      const long long i = idx[j];
+      wrong = wrong || i < 0 || i >= n || (j > 0 && idx[j - 1] >= i);
+    }
     if (__syncthreads_or(wrong) && threadIdx.x == 0) coo_raise(tiles);
   }
   for (int64_t j = first; j < nnz; j += step) {
@@ -783,12 +787,15 @@ __global__ __launch_bounds__(kCodecBlock) void coo_add_kernel(const long long* _
 }
 
 // From an entry in this many elements on an entry's place is kept as a bit: 1/64 of the indices' bytes at an entry an
-// element, an eighth at one in eight, and who walks the tiles reads that. 67 million elements, an entry in 1 / 2 / 4 / 8 / 12 of them,
-// blocking, us, by the indices and by bits: Adam push 560 / 452 / 382 / 356 / 343 and 468 / 404 / 369 / 355 / 349,
-// decode 276 / 163 / 114 / 91 / 82 and 192 / 121 / 91 / 77 / 71. In small tensors the indices lie in the caches when
-// they are read again, and the bits' launch is the longer one: an Adam push of 20,000 / 300,000 / 2 million / 4 million elements, an entry in
-// four, 18.1 / 17.3 / 23.7 / 34.0 us by bits and 15.1 / 15.2 / 21.7 / 34.5 by the indices; four in five 17.9 / 16.9 / 24.7 / 36.7
-// and 15.4 / 15.5 / 24.6 / 39.9.
+// element, an eighth at one in eight, and who walks the tiles reads that. 67 million elements, an entry in 1 / 2 / 4
+// / 8 / 12 of them, blocking, us, by the indices and by bits: Adam push 560 / 452 / 382 / 356 / 343 and 468 / 404 /
+// 369 / 355 / 349, decode 276 / 163 / 114 / 91 / 82 and 192 / 121 / 91 / 77 / 71. In small tensors the indices lie in
+// the caches when they are read again, and the bits' launch is the longer one: an Adam push of 20,000 / 300,000 / 2
+// million / 4 million elements, an entry in four, 18.1 / 17.3 / 23.7 / 34.0 us by bits and 15.1 / 15.2 / 21.7 / 34.5
+// by the indices; four in five 17.9 / 16.9 / 24.7 / 36.7 and 15.4 / 15.5 / 24.6 / 39.9. Around the line, 2.5 / 3 /
+// 3.5 / 4 / 5 million elements: an entry in eight 27.9 / 31.4 / 34.1 / 36.3 / 39.9 by bits and 25.2 / 29.4 / 33.6 /
+// 35.6 / 40.0, in four 27.4 / 31.2 / 33.2 / 35.7 / 40.2 and 25.8 / 30.2 / 33.9 / 35.9 / 40.6, four in five 29.1 /
+// 32.6 / 35.0 / 38.0 / 42.5 and 31.0 / 34.9 / 40.2 / 42.0 / 48.4.
 constexpr int64_t kCooBitsFrom = 8;
 constexpr int64_t kCooBitsLarge = (int64_t)3 << 20;
 
@@ -834,9 +841,11 @@ int32_t coo_find_tiles(CooWork* work, const long long* d_idx, int64_t nnz, int64
   const dim3 block(kCodecBlock);
   if (with_bits) {
     constexpr int64_t per = (int64_t)(kCodecBlock / 64) * kCooRun * kCooChunk;
-    hipLaunchKernelGGL(coo_bits_kernel, dim3((unsigned)((nnz + per - 1) / per)), block, 0, stream, d_idx, nnz, n, vec, *out);
+    hipLaunchKernelGGL(coo_bits_kernel, dim3((unsigned)((nnz + per - 1) / per)), block, 0, stream, d_idx, nnz, n, vec,
+                       *out);
   } else {
-    hipLaunchKernelGGL(coo_tiles_bounds_kernel, dim3(stream_grid((nnz + 3) / 4)), block, 0, stream, d_idx, nnz, n, vec, *out);
+    hipLaunchKernelGGL(coo_tiles_bounds_kernel, dim3(stream_grid((nnz + 3) / 4)), block, 0, stream, d_idx, nnz, n, vec,
+                       *out);
   }
   KRK_HIP(hipGetLastError());
   return KRK_SUCCESS;
@@ -999,8 +1008,9 @@ int32_t krk_dct_compress(krk_dct* s, const float* grad, uint64_t life_span, floa
     uint32_t* d_host_sel = nullptr;
     KRK_HIP(hipHostGetDevicePointer((void**)&d_host_sel, s->host_sel, 0));
     auto launch = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles < kSingleGrid ? tiles : kSingleGrid)), dim3(kSingleBlock), 0, s->stream, d_g, s->e, n, (uint32_t)tiles, vec, s->sel, s->tile_state,
-                         s->tickets, s->emit_calls, reinterpret_cast<long long*>(idx), val, s->e_next, d_host_sel);
+      hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles < kSingleGrid ? tiles : kSingleGrid)), dim3(kSingleBlock), 0,
+                         s->stream, d_g, s->e, n, (uint32_t)tiles, vec, s->sel, s->tile_state, s->tickets,
+                         s->emit_calls, reinterpret_cast<long long*>(idx), val, s->e_next, d_host_sel);
     };
     if (rows == 8) launch(emit_single_kernel<8>);
     else if (rows == 4) launch(emit_single_kernel<4>);

@@ -469,7 +469,7 @@ constexpr int kCooPlainPushes = 256;
 // arrays, 15.1 / 16.2 / 17.0 / 30.0 us by fill, scatter and update, 12.9 / 15.8 / 15.7 / 22.4 in tiles. A push that
 // goes tile by tile and whose indices do not ascend is scattered after all, behind a second wait (shuffled, 36 / 63 us for
 // 300,000 / 2 million elements, 19 / 48 where it is scattered at once), so the push before it decides: a small table's first
-// one is scattered, and the scatter looks at the order in passing (28 us for 27 of 2 million elements); after one that does
+// one is scattered, and the scatter looks at the order in passing (28 to 31 us for 27 of 2 million elements); after one that does
 // not ascend the next ones are scattered as they are.
 // That is for device arrays. Indices that the kernels read in host memory cross PCIe twice in tiles and once in the
 // scatter (page-locked, 300,000 / 2 million elements, an entry in four, 51 / 227 us and 37 / 132; pageable 64 and 52

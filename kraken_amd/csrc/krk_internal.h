@@ -547,13 +547,11 @@ __device__ __forceinline__ void optim_element(const OptimK& k, float lr, float g
   }
 }
 
-// ---- device-wide exclusive scan of int32 (three plain launches, no spinning) ----
-// out[i] = sum(in[0..i)), total written to *total_out (device). in/out may alias.
-// CooTensorImpl::ToDense (t/coo_tensor_impl.cc:250-260, t/math.cc:1006-1096) on the device:
-// dense[0, n) = 0, then dense[idx[j]] += val[j]. Large tensors whose indices ascend strictly and
-// lie in range (what ToCoo produces) are taken tile by tile: one launch over the indices finds
-// where each tile's entries begin (coo_find_tiles), and whoever walks the tiles puts one together
-// in LDS, or, where there are many entries, from a bit an element that the first launch leaves. Any other input is zeroed and scattered into; which of the two it is is decided on the
+// CooTensorImpl::ToDense (t/coo_tensor_impl.cc:250-260, t/math.cc:1006-1096) on the device: dense[0, n) = 0, then
+// dense[idx[j]] += val[j]. Large tensors whose indices ascend strictly and lie in range (what ToCoo produces) are
+// taken tile by tile: one launch over the indices finds where each tile's entries begin (coo_find_tiles), and
+// whoever walks the tiles puts one together in LDS, or, where there are many entries, from a bit an element that
+// the first launch leaves. Any other input is zeroed and scattered into; which of the two it is is decided on the
 // device, and the launches of the other way look at the flag and leave.
 constexpr int kCooTile = 2048;                   // floats of one tile: 8 KB of LDS
 // Smaller tensors: zero + scatter, two launches are quicker than two and those of the other way, unless the call
@@ -589,7 +587,8 @@ struct CooTileBits {
   }
   // The gradient of the four elements of quad q of the tile, whose entries are [start, end) (end > start, or all bits are
   // clear): the values of those that have an entry, zero for the others.
-  __device__ __forceinline__ void quad(int q, const float* __restrict__ val, uint32_t start, uint32_t end, float (&g)[4]) const {
+  __device__ __forceinline__ void quad(int q, const float* __restrict__ val, uint32_t start, uint32_t end,
+                                       float (&g)[4]) const {
     const uint32_t w = (uint32_t)__shfl((int)word, q >> 3);
     const int shift = (q & 7) * 4;
     const uint32_t mine = (w >> shift) & 15u;
@@ -624,7 +623,9 @@ int32_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uin
                          int bits, void* work, hipStream_t stream, uint32_t** keys_sorted,
                          uint32_t** vals_sorted);
 
-// scratch must hold scan_scratch_bytes(n).
+// ---- device-wide exclusive scan of int32 (three plain launches, no spinning) ----
+// out[i] = sum(in[0..i)), total written to *total_out (device). in/out may alias. scratch must hold
+// scan_scratch_bytes(n).
 size_t scan_scratch_bytes(int64_t n);
 int32_t exclusive_scan_i32(const int32_t* in, int32_t* out, int64_t n, int32_t* total_out,
                            void* scratch, hipStream_t stream);

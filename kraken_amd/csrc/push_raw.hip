@@ -538,14 +538,15 @@ constexpr int kFromRows = 1;     // level 0: gradient rows
 constexpr int kFromBags = 2;     // level 0 of a pooled push: bags' gradient rows, scaled as they are read
 
 // A span that lies inside one run, which goes on in a neighbour: the sum of its entries, as segreduce_kernel adds
-// them up (a tile by a lane group, the tiles' sums in order), to carry slot `slot`; behind it zeros, if the run goes on on
-// both sides. Skewed requests are such spans for the most part (three in five of 8.5 million Zipf 1.1 ids), and by the
-// general way they waited rather than moved bytes: four rows requested at a time where no record needs the
-// registers, and a look at every entry's key between them. Eight rows at a time (sixteen: the same): the reduction of 8.5 million
-// pooled ids of 32 floats under Adam 405 -> 346 us, 4.7 -> 5.5 TB/s of its misses and writes; forward, backward and
-// forward, us: that 941 -> 874, 2.4 million of 8 floats 250 -> 239, 3 million weighted of 16 320 -> 303, 1.3 million of 64
-// 291 -> 281, 1.6 million of 32 209 -> 193. (Partial sums requested four or eight ahead of adding them up gain nothing
-// in the general way.)
+// them up (a tile by a lane group, the tiles' sums in order), to carry slot `slot`; behind it zeros, if the run goes
+// on on both sides. Skewed requests are such spans for the most part (three in five of 8.5 million Zipf 1.1 ids), and
+// by the general way they waited rather than moved bytes: four rows requested at a time where no record needs the
+// registers, and a look at every entry's key between them. Eight rows at a time (sixteen: the same): the reduction of
+// 8.5 million pooled ids of 32 floats under Adam 405 -> 346 us, 4.7 -> 5.5 TB/s of its misses and writes. Forward,
+// backward and forward of a layer under Adam over 4 million rows, Zipf 1.1, without / with it in turn, us: that 938 /
+// 872; in mean bags of up to twenty ids 2.4 million of 8 floats 269 / 257, 1.6 million of 32 273 / 263, 1.3 million
+// of 64 325 / 312; 3 million weighted ones of 16 412 / 404; 1.5 million ids without bags of 32 309 / 300. (Partial
+// sums requested four or eight ahead of adding them up gain nothing in the general way.)
 template <int VEC, bool POOLED>
 __device__ __forceinline__ void reduce_one_run(const KRK_GLOBAL float* const* lds_src, const float* lds_r,
                                                const float* lds_w, float* part_val, int tile, int per_block, int dim,

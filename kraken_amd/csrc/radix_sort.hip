@@ -40,7 +40,8 @@ constexpr int kRsDigits = 1 << kRsMaxBits;
 // finds the bags in which tiles begin, and the scatter works every position's bag out. A launch that wrote the pairs
 // out in advance (a lane group a bag, as for requests short enough for buckets) moved 117 MB for 8.5 million positions,
 // 32 us; without it the first histogram takes 15.5 us for 11 (the notes come from further away than pairs just
-// written) and the first scatter 38 for 30: a pooled step of 952 us 936. Requests of up to 2^20
+// written) and the first scatter 38 for 30: a pooled step of 891 us 872, of 2.4 million positions 264 and 257, of 1.3
+// million 320 and 312 (rows of 32, 8 and 64 floats). Requests of up to 2^20
 // positions keep that launch: in the partition's launches the same cost what it saved.
 
 // The bag that the offsets step over p with, offsets[bag] <= p < offsets[bag + 1]: searched by a whole

@@ -337,9 +337,10 @@ struct RunHash {
 // 1043 and 2126, Zipf 1.3 310 and 570 against 355 and 648: the sort leaves the rows in the order they lie in).
 // Above it, with 2048 buckets of 16-bit counts, which cost 3 to 9 % below it: 1.5 million ids of 128
 // floats 882 / 868 / 382 / 242 against 886 / 842 / 435 / 301, 2^21 1208 / 1198 / 508 / 313 against 1200 / 1141 / 562 / 382,
-// i.e. skewed requests gain a tenth to a fifth and consecutive rows lose a twentieth. (The sort's side of all this is from before
-// spans of one row had a way of their own; with that, forward, backward and forward by buckets / by the sort: 2^20 ids of 128 floats,
-// Zipf 1.3, 360 / 401, a million of 16, Zipf 1.05, 139 / 180, 950,000 pooled of 32, Zipf 1.1, 158 / 193.)
+// i.e. skewed requests gain a tenth to a fifth and consecutive rows lose a twentieth. (The sort's side of all this is
+// from before spans of one row had a way of their own; with that, forward, backward and forward by buckets / by the
+// sort: 2^20 ids of 128 floats, Zipf 1.3, 360 / 401, a million of 16, Zipf 1.05, 139 / 180, 950,000 pooled of 32,
+// Zipf 1.1, 158 / 193.)
 constexpr int64_t kRunsMax = (int64_t)1 << 20;
 // Bytes of the partition's work space.
 size_t partition_work_bytes(int64_t n, int bucket_bits);
