@@ -798,6 +798,12 @@ __global__ __launch_bounds__(kCodecBlock) void coo_add_kernel(const long long* _
 // 32.6 / 35.0 / 38.0 / 42.5 and 31.0 / 34.9 / 40.2 / 42.0 / 48.4.
 constexpr int64_t kCooBitsFrom = 8;
 constexpr int64_t kCooBitsLarge = (int64_t)3 << 20;
+// A decode is two short launches, of which the bits make the first one 3 us longer whatever the tensor's size: what they
+// spare has to be more entries than that. By the indices / by bits, us: an entry in eight of 4.2 / 8 / 12 / 16 / 24 million
+// elements 23.3 / 27.2 / 31.5 / 35.5 / 43.3 and 26.6 / 28.8 / 31.6 / 34.6 / 40.6, in four of 4.2 / 6 / 8 / 12 million 24.4 /
+// 27.4 / 29.7 / 35.4 and 26.1 / 27.6 / 28.9 / 32.1, in two of 4.2 / 6 million 27.1 / 30.9 and 26.1 / 28.4; 512 elements in a
+// row of each 4096, of 8 / 12 / 16 / 24 million, 28.1 / 32.3 / 36.3 / 44.3 and 30.2 / 33.7 / 36.5 / 43.8.
+constexpr int64_t kCooBitsDecode = (int64_t)7 << 18;
 
 static unsigned stream_grid(int64_t n) {
   int64_t blocks = (n + kCodecBlock - 1) / kCodecBlock;
@@ -828,10 +834,10 @@ int32_t coo_new_tag(CooWork* work, int64_t n, CooTiles* out, hipStream_t stream)
   return KRK_SUCCESS;
 }
 
-int32_t coo_find_tiles(CooWork* work, const long long* d_idx, int64_t nnz, int64_t n, CooTiles* out,
+int32_t coo_find_tiles(CooWork* work, const long long* d_idx, int64_t nnz, int64_t n, bool update, CooTiles* out,
                        hipStream_t stream) {
   KRK_TRY(coo_new_tag(work, n, out, stream));
-  bool with_bits = n >= kCooBitsLarge && nnz * kCooBitsFrom >= n;
+  bool with_bits = nnz * kCooBitsFrom >= n && (update ? n >= kCooBitsLarge : nnz >= kCooBitsDecode);
   if (with_bits && work->bits.reserve((size_t)out->tiles * (kCooTile / 8)) != KRK_SUCCESS) {
     (void)hipGetLastError();                         // no failure of a later launch
     with_bits = false;                               // the indices are read again, then
@@ -879,7 +885,7 @@ int32_t coo_densify(CooWork* work, const long long* d_idx, const float* d_val, i
     return KRK_SUCCESS;
   }
   CooTiles tiles;
-  KRK_TRY(coo_find_tiles(work, d_idx, nnz, n, &tiles, stream));
+  KRK_TRY(coo_find_tiles(work, d_idx, nnz, n, false, &tiles, stream));
   if (tiles.bits) {
     hipLaunchKernelGGL(coo_bits_write_kernel, dim3(tiles.tiles), block, 0, stream, d_val, d_dense, n, tiles);
   } else {

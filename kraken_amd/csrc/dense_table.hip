@@ -512,7 +512,7 @@ static int32_t dense_apply_coo(krk_dense* t, const krk_optim& o, const long long
   DenseMember m;
   KRK_TRY(dense_member(t, o, &m));
   const OptimK k = make_optim_k(o);
-  KRK_TRY(coo_find_tiles(&t->coo_work, d_idx, nnz, t->n, &tiles, t->stream));
+  KRK_TRY(coo_find_tiles(&t->coo_work, d_idx, nnz, t->n, true, &tiles, t->stream));
   if (waits && end.open() && !(flags & KRK_DEVICE_PTRS)) {
     tiles.told = end.told();
     tiles.ticket = end.ticket;

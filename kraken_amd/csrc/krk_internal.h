@@ -605,7 +605,8 @@ struct CooTileBits {
 inline bool coo_tiled(int64_t n, int64_t nnz) { return n >= kCooTiledFrom && nnz < ((int64_t)1 << 31); }
 // A flag of a new call, lowered: out without starts and bits.
 int32_t coo_new_tag(CooWork* work, int64_t n, CooTiles* out, hipStream_t stream);
-int32_t coo_find_tiles(CooWork* work, const long long* d_idx, int64_t nnz, int64_t n, CooTiles* out,
+// update: for an optimizer's update, which has more to wait for than a decode (bits pay earlier).
+int32_t coo_find_tiles(CooWork* work, const long long* d_idx, int64_t nnz, int64_t n, bool update, CooTiles* out,
                        hipStream_t stream);
 // What is left to do where the indices are unordered, and nothing otherwise: dense = the entries' sums.
 int32_t coo_scatter_if_unordered(const CooTiles& tiles, const long long* d_idx, const float* d_val, int64_t nnz,

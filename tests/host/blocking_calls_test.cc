@@ -525,7 +525,8 @@ static void word_of_a_failed_push() {
   for (krk_dense* t : d) CHECK(krk_dense_destroy(t) == 0);
 }
 
-// A decode belongs to no object: what it keeps on the device afterwards is bounded.
+// Decodes of few entries read the indices twice, whatever the tensor's size. A decode belongs to no object: what it
+// keeps on the device afterwards is bounded.
 static void work_space_of_decodes() {
   void* place = nullptr;                            // (no kernel runs: an address is enough)
   CHECK(krk_malloc(&place, 4096) == 0);
@@ -535,10 +536,16 @@ static void work_space_of_decodes() {
     return bytes;
   };
   const size_t before = held();
+  for (const int64_t n : {(int64_t)1 << 22, (int64_t)12 << 20, (int64_t)1 << 26}) {
+    CHECK(krk_coo_to_dense(static_cast<int64_t*>(place), static_cast<float*>(place), (int64_t)3 << 19,
+                           static_cast<float*>(place), n, KRK_DEVICE_PTRS) == KRK_SUCCESS);
+    CHECK(launches("coo_bits_kernel") == 0 && launches("coo_tiles_write_kernel") == 1);
+    rt().launched.clear();
+  }
   for (const int64_t n : {(int64_t)1 << 23, (int64_t)1 << 31, (int64_t)5 << 30, (int64_t)1 << 23}) {
-    CHECK(krk_coo_to_dense(static_cast<int64_t*>(place), static_cast<float*>(place), n / 8, static_cast<float*>(place), n,
+    CHECK(krk_coo_to_dense(static_cast<int64_t*>(place), static_cast<float*>(place), n / 4, static_cast<float*>(place), n,
                            KRK_DEVICE_PTRS) == KRK_SUCCESS);
-    CHECK(launches("coo_bits_write_kernel") == 1);
+    CHECK(launches("coo_bits_write_kernel") == 1 && launches("coo_tiles_write_kernel") == 0);
     rt().launched.clear();
     CHECK(held() - before <= ((size_t)256 << 20) + ((size_t)16 << 20));
   }

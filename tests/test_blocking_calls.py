@@ -29,7 +29,7 @@ def program(tmp_path_factory):
 # host_gradients: sparse gradients in host memory of small dense tables are read once
 # gradients_order: which of them go tile by tile
 # first_gradient: a table's first one in pageable memory takes few commands
-# decodes: what a decode keeps on the device is bounded
+# decodes: which of them leave bits of the elements, and what one keeps on the device is bounded
 # old_words: a launch of a call that failed says something over the next call's word
 @pytest.mark.parametrize("which", ["dense", "sparse", "words", "core", "host_gradients", "gradients_order",
                                    "first_gradient", "decodes", "old_words"])

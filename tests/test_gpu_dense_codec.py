@@ -356,6 +356,20 @@ def test_coo_many_entries(api, oracle, case, n):
     check(full)
 
 
+@pytest.mark.parametrize("case", ["front", "back", "tiles", "gaps", "fifth"])
+def test_coo_decode_of_millions_of_entries(api, case):
+    """Decodes leave a bit an element from 7 * 2^18 entries on: just below that and just above, and all of them."""
+    n = 14_000_001                                     # (an entry in eight elements is less than that)
+    full = _many_entries(case, n).astype(np.int64)
+    assert n < 8 * ((7 << 18) - 1) and full.size > (7 << 18) + 1
+    for count in ((7 << 18) - 1, 7 << 18, (7 << 18) + 1, full.size):
+        idx = full[:count]
+        val = (np.arange(count) % 61 - 30).astype(np.float32)
+        want = np.zeros(n, np.float32)
+        want[idx] = val
+        assert np.array_equal(api.coo_to_dense(idx, val, n), want)
+
+
 def test_dense_push_coo_large(api, oracle):
     n = (1 << 22) + 77
     rng = np.random.default_rng(4)
