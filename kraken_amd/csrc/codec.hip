@@ -12,6 +12,7 @@
 // one pass (emit_single_kernel); where the count decides whether anything may be written at all it is
 // a count pass, a scan of the per-tile counts and a write pass that recomputes f.
 #include <algorithm>
+#include <atomic>
 #include <new>
 
 #include "krk_internal.h"
@@ -812,31 +813,28 @@ static unsigned stream_grid(int64_t n) {
   return (unsigned)blocks;
 }
 
-int32_t coo_new_tag(CooWork* work, int64_t n, CooTiles* out, hipStream_t stream) {
+// Every call of the process has another tag, so nothing lowers the flag, in new memory neither: what happens to be
+// there is some other call's, or, should it be this one's, says 'unordered', which is slow and right for any indices.
+static std::atomic<uint32_t> g_coo_tag{0};
+
+int32_t coo_new_tag(CooWork* work, int64_t n, CooTiles* out) {
   uint32_t* room = work->lent;
-  bool fresh = work->calls == 0 || work->calls == 0xFFFFFFFFu;   // a fresh buffer holds no tag, and 0 is none
   if (!room) {
-    const size_t before = work->buffer.bytes;
     KRK_TRY(work->buffer.reserve(coo_tile_words(n) * sizeof(uint32_t)));
     room = work->buffer.as<uint32_t>();
-    fresh = fresh || work->buffer.bytes != before;
   }
   out->unordered = room;
   out->starts = room + 1;
   out->tiles = (uint32_t)((n + kCooTile - 1) / kCooTile);
   out->bits = nullptr;
   out->told = nullptr;
-  if (fresh) {
-    KRK_HIP(hipMemsetAsync(out->unordered, 0, sizeof(uint32_t), stream));
-    work->calls = 0;
-  }
-  out->tag = ++work->calls;
+  out->tag = g_coo_tag.fetch_add(1, std::memory_order_relaxed) + 1;
   return KRK_SUCCESS;
 }
 
 int32_t coo_find_tiles(CooWork* work, const long long* d_idx, int64_t nnz, int64_t n, bool update, CooTiles* out,
                        hipStream_t stream) {
-  KRK_TRY(coo_new_tag(work, n, out, stream));
+  KRK_TRY(coo_new_tag(work, n, out));
   bool with_bits = nnz * kCooBitsFrom >= n && (update ? n >= kCooBitsLarge : nnz >= kCooBitsDecode);
   if (with_bits && work->bits.reserve((size_t)out->tiles * (kCooTile / 8)) != KRK_SUCCESS) {
     (void)hipGetLastError();                         // no failure of a later launch

@@ -498,7 +498,7 @@ static int32_t dense_apply_coo(krk_dense* t, const krk_optim& o, const long long
   CooTiles tiles;
   StreamWait end;
   if (!tiled) {
-    if (look) KRK_TRY(coo_new_tag(&t->coo_work, t->n, &tiles, t->stream));
+    if (look) KRK_TRY(coo_new_tag(&t->coo_work, t->n, &tiles));
     KRK_TRY(coo_densify(&t->coo_work, d_idx, d_val, nnz, t->coo_grad, t->n, t->stream, look ? &tiles : nullptr));
     KRK_TRY(dense_apply(t, o, t->coo_grad, lr));
     if (!look || !end.open()) return KRK_SUCCESS;

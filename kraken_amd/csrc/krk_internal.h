@@ -570,7 +570,6 @@ __device__ __forceinline__ bool coo_unordered(const CooTiles& t) { return *t.uno
 struct CooWork {          // work space of one caller, kept between calls
   DeviceBuffer buffer, bits;
   uint32_t* lent = nullptr;   // room for coo_tile_words of the caller's tensor behind something else of the caller's
-  uint32_t calls = 0;
   void release() {
     buffer.release();
     bits.release();
@@ -603,8 +602,8 @@ struct CooTileBits {
   }
 };
 inline bool coo_tiled(int64_t n, int64_t nnz) { return n >= kCooTiledFrom && nnz < ((int64_t)1 << 31); }
-// A flag of a new call, lowered: out without starts and bits.
-int32_t coo_new_tag(CooWork* work, int64_t n, CooTiles* out, hipStream_t stream);
+// A call's tag, which its flag is not raised to yet: out without starts and bits.
+int32_t coo_new_tag(CooWork* work, int64_t n, CooTiles* out);
 // update: for an optimizer's update, which has more to wait for than a decode (bits pay earlier).
 int32_t coo_find_tiles(CooWork* work, const long long* d_idx, int64_t nnz, int64_t n, bool update, CooTiles* out,
                        hipStream_t stream);

@@ -491,7 +491,10 @@ static void order_of_sparse_gradients() {
   std::vector<float> vals(50000);
   krk_dense* d = nullptr;
   CHECK(krk_dense_create(vals.data(), (int64_t)vals.size(), 0, &d) == 0);
-  CHECK((push_in_device_memory(d, true, 258) == Ways{0, 258}));   // never a look at the tiles
+  rt().commands = 0;
+  CHECK((push_in_device_memory(d, true, 1) == Ways{0, 1}));
+  CHECK(rt().commands == 4);                        // fill, scatter, update, word
+  CHECK((push_in_device_memory(d, true, 257) == Ways{0, 257}));   // never a look at the tiles
   CHECK((push_in_device_memory(d, false, 257) == Ways{0, 257}));  // some of them spared, then one that is looked at
   CHECK((push_in_device_memory(d, false, 300) == Ways{300, 0}));
   CHECK((push_in_device_memory(d, false, 1, 60000) == Ways{0, 1}));   // more entries than elements
